@@ -599,7 +599,7 @@ def gemm(a, w, out, choices=None) -> None:
         return
     if a.dtype == F32:
         _check(out, "out", F32)
-        call("as_gemm_f32", _ptr(a), _ptr(rows), _ptr(out), M, N, K, _stream())
+        call("as_gemm_f32", _ptr(a), _ptr(rows), _ptr(out), M, N, K, 0, _stream())
         return
     if out.dtype not in (BF16, F32):
         raise KernelError(f"gemm: unsupported output dtype {out.dtype}")

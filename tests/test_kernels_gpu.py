@@ -289,6 +289,27 @@ def test_gemm_fp32_rows_do_not_depend_on_the_batch(ops):
         assert torch.equal(one[0], full[i])
 
 
+@pytest.mark.parametrize("M,N,K,shift", [(1, 33, 4, 0), (15, 17, 256, 0), (16, 16, 260, 0), (17, 31, 512, 0), (33, 65, 516, 0), (63, 47, 1028, 0),
+                                         (65, 130, 2052, 0), (20, 40, 257, 0), (5, 50, 64, 1), (40, 70, 1000, 1)])  # fmt: skip
+def test_gemm_fp32_tiles_agree(ops, M, N, K, shift):
+    """Every tile of the 32-bit product gives the same bits (the order of a sum depends on K alone), whole and odd widths,
+    aligned and shifted matrices.  Bound: chains of at most K / 16 + 31 terms and 6 additions (of K terms up to 256
+    columns), each rounding 2^-24 of the sums of absolute values."""
+    from atomserve_amd.kernels.lib import call
+
+    torch.manual_seed(60)
+    a = torch.randn(M * K + shift, device=DEV)[shift:].view(M, K)
+    w = torch.randn(N * K + shift, device=DEV)[shift:].view(N, K)
+    outs = []
+    for form in range(6):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        call("as_gemm_f32", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, form, torch.cuda.current_stream().cuda_stream)
+        outs.append(out)
+    assert all(torch.equal(outs[0], o) for o in outs)
+    bound = (a.abs().double() @ w.abs().double().T) * (K / 16 + 37 if K > 256 else K) * 2.0**-24
+    assert bool(((outs[0].double() - a.double() @ w.double().T).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 96, 64), (8, 1000, 96), (64, 4096, 1024), (300, 257, 192), (5, 2000, 4096),
                                    (16, 4096, 4096), (12, 8200, 4096), (9, 16000, 2048), (3, 40, 200), (16, 24, 8),
                                    (4, 1040, 5120), (7, 520, 6144), (2, 100, 2560), (11, 4100, 3072), (8, 512, 12288),
