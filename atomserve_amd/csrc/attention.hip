@@ -1424,6 +1424,195 @@ extern "C" int as_attn_single_query(const void* q, const void* k_pages, const vo
   return AS_BAD_DTYPE;
 }
 
+// ---- fp32 through the matrix cores -------------------------------------------------------
+//
+// attn_f32: the attention of 32-bit heads, 16 queries of one kv head to a workgroup as the columns of 16 x 16 tiles:
+// the G heads of one token (decode: items), or of 16 / G neighbouring tokens of a prompt (tiles), so that every key and value
+// is read once for all of them.  The four waves take the steps of 16 keys in turn, each with maxima, sums and
+// outputs of its own, which meet in LDS at the end.  Per step, all products by v_mfma_f32_16x16x4_f32 (32-bit products and sums):
+//   S[key][query] = K[key][:] . Q[query][:]     keys straight from the page, 16 bytes a lane
+//   O^T[d][query] += V^T[d][key] P[key][query]  values straight from the transposed page; P is what the lane holds
+// The next step's keys are asked for when this step's have met the queries, its values when these have been added up.
+// Bound by the 64 matrix instructions of a step (heads of 128): 0.9 us a wave, and by launch and merge for short
+// contexts.  16 heads of 128 on 8 kv heads, in a captured step: 4 requests of 600 tokens 12.2 us, of 2,000 tokens 18.4 (45.2 and 54.4
+// on the general kernel, which reads each value of a transposed page alone); a prompt of 333 tokens 24 (147: a workgroup to
+// every token read all keys before it).
+template <int DT>
+__global__ __launch_bounds__(256) void attn_f32_kernel(
+    const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
+    const int* __restrict__ tiles, const int* __restrict__ items, const int* __restrict__ positions,
+    const int* __restrict__ tok_row, const int* __restrict__ block_tables, int table_width, float* __restrict__ out,
+    float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int bs,
+    float scale, Sight sight, int subs, int part_size, int P) {
+  constexpr int D = 16 * DT, LD = D + 4;
+  extern __shared__ float smem[];  // [4][16] m, [4][16] l, [4][16][LD] outputs
+  const int G = H / KV, kvh = blockIdx.y, part = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  int t0, count, row, pos0;
+  const int item = blockIdx.x;
+  if (tiles) {
+    const int per = 16 / G;  // tokens of a workgroup
+    const int* tile = tiles + (size_t)(item / subs) * 4;
+    const int at = item % subs * per;
+    count = min(per, tile[1] - at);
+    if (count <= 0) return;
+    t0 = tile[0] + at;
+    row = tile[2];
+    pos0 = tile[3] + at;
+  } else {
+    t0 = items ? items[item] : item;
+    count = 1;
+    row = tok_row ? tok_row[t0] : t0;
+    pos0 = positions[t0];
+  }
+  const int tok = lr / G, head = kvh * G + lr % G;
+  const bool valid = tok < count;
+  const int pos = valid ? pos0 + tok : -1;
+  const int first = valid ? first_in_window(sight, pos + 1) : 0;       // this column's first visible key
+  const int start = first_in_window(sight, pos0 + 1) & ~15;             // the workgroup's, in whole steps
+  const int k0 = start + part * part_size, k1 = P == 1 ? pos0 + count : min(pos0 + count, k0 + part_size);
+  if (k0 >= k1) {  // an empty partition (items only): mark it so for the reduce
+    if (tid < G) {
+      const size_t o = ((size_t)item * H + kvh * G + tid) * P + part;
+      part_m[o] = NEG_INF;
+      part_l[o] = 0.f;
+    }
+    for (int x = tid; x < G * D; x += 256) part_acc[(((size_t)item * H + kvh * G + x / D) * P + part) * D + x % D] = 0.f;
+    return;
+  }
+  const int steps = (k1 - k0 + 15) >> 4;
+  const int* table = block_tables + (size_t)row * table_width;
+
+  f32x4_t qf[DT], kf[DT], vf[DT], o[DT];
+  const float* qrow = q + ((size_t)(t0 + (valid ? tok : 0)) * H + (valid ? head : kvh * G)) * D;
+#pragma unroll
+  for (int i = 0; i < DT; ++i) {
+    qf[i] = *reinterpret_cast<const f32x4_t*>(qrow + (i >> 1) * 32 + lg * 8 + (i & 1) * 4) * scale;
+    o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  auto page_of = [&](int step) {  // the 16 keys' place: page and offset, as an offset into one head's pages
+    const int key = k0 + min(step, steps - 1) * 16;
+    return ((size_t)table[key / bs] * KV + kvh) * bs * D;
+  };
+  auto load_keys = [&](size_t base, int step) {
+    const float* p = k_pages + base + (size_t)((k0 + min(step, steps - 1) * 16) % bs + lr) * D + lg * 8;
+#pragma unroll
+    for (int i = 0; i < DT; ++i) kf[i] = *reinterpret_cast<const f32x4_t*>(p + (i >> 1) * 32 + (i & 1) * 4);
+  };
+  auto load_values = [&](size_t base, int step) {
+    const float* p = v_pages + base + (size_t)lr * bs + (k0 + min(step, steps - 1) * 16) % bs + lg * 4;
+#pragma unroll
+    for (int i = 0; i < DT; ++i) vf[i] = *reinterpret_cast<const f32x4_t*>(p + (size_t)i * 16 * bs);
+  };
+  float m = NEG_INF, l = 0.f;
+  size_t base = page_of(wave), next = page_of(wave + 4);
+  if (wave < steps) {
+    load_keys(base, wave);
+    load_values(base, wave);
+  }
+  for (int step = wave; step < steps; step += 4) {
+    f32x4_t s0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+    for (int i = 0; i < DT; i += 2)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][x], qf[i][x], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i + 1][x], qf[i + 1][x], s1, 0, 0, 0);
+      }
+    load_keys(next, step + 4);
+    f32x4_t s = s0 + s1;
+    const int key = k0 + step * 16 + lg * 4;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (sight.cap > 0.f) s[r] = sight.cap * tanhf(s[r] / sight.cap);
+      if (key + r > pos || key + r < first || key + r >= k1) s[r] = NEG_INF;
+    }
+    const float top = fmaxf(m, quad_rows_max(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+    const float at = top == NEG_INF ? 0.f : top;  // nothing seen yet: every weight is e^-inf = 0
+    if (__any(top > m)) {
+      const float keep = expf(m - at);
+      l *= keep;
+#pragma unroll
+      for (int i = 0; i < DT; ++i) o[i] *= keep;
+      m = top;
+    }
+    float p[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[r] = expf(s[r] - at);
+    l += (p[0] + p[1]) + (p[2] + p[3]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < DT; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[i][r], p[r], o[i], 0, 0, 0);
+    load_values(next, step + 4);
+    next = page_of(step + 8);
+  }
+  l = quad_rows_sum(l);
+  float* sm = smem;
+  float* sl = smem + 64;
+  float* so = smem + 128;
+  if (lg == 0) { sm[wave * 16 + lr] = m; sl[wave * 16 + lr] = l; }
+#pragma unroll
+  for (int i = 0; i < DT; ++i) *reinterpret_cast<f32x4_t*>(so + (size_t)(wave * 16 + lr) * LD + i * 16 + lg * 4) = o[i];
+  __syncthreads();
+  for (int x = tid; x < count * G * D; x += 256) {
+    const int c = x / D, d = x % D;
+    float top = fmaxf(fmaxf(sm[c], sm[16 + c]), fmaxf(sm[32 + c], sm[48 + c])), num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float e = sm[w * 16 + c] == NEG_INF ? 0.f : expf(sm[w * 16 + c] - top);
+      num += so[(size_t)(w * 16 + c) * LD + d] * e;
+      den += sl[w * 16 + c] * e;
+    }
+    const int h = kvh * G + c % G;
+    if (P == 1) {
+      if (sight.sink) {
+        const float sk = sink_score(1, sight.sinks, h), most = fmaxf(top, sk), e = expf(top - most);
+        num *= e;
+        den = den * e + expf(sk - most);
+      }
+      out[((size_t)(t0 + c / G) * H + h) * D + d] = num / den;
+    } else {
+      const size_t place = ((size_t)item * H + h) * P + part;
+      part_acc[place * D + d] = num;
+      if (d == 0) { part_m[place] = top; part_l[place] = den; }
+    }
+  }
+}
+
+// Which shapes it takes: heads of 64 or 128, at most 16 query heads to a kv head, pages of whole steps of 16 keys, no
+// kept first keys (a second stretch of keys; the general kernel walks them).
+extern "C" int as_attn_f32(const float* q, const float* k_pages, const float* v_pages, const int* tiles, int num_tiles,
+                           int most, const int* items, int num_items, const int* positions, const int* tok_row,
+                           const int* block_tables, int table_width, float* out, float* part_m, float* part_l,
+                           float* part_acc, int H, int KV, int D, int bs, float scale, int window, int keep, int chunk,
+                           float cap, int sink, const float* sinks, int wide, int part_size, int P, hipStream_t stream) {
+  const Sight sight{window, keep, chunk, cap, sink, sinks, wide};
+  const int blocks_of = tiles ? num_tiles : num_items;
+  if (blocks_of <= 0) return AS_OK;
+  if (H <= 0 || KV <= 0 || KV > 65535 || H % KV || H / KV > 16 || (D != 64 && D != 128) || bs <= 0 || bs % 16 || table_width <= 0 ||
+      part_size <= 0 || part_size % 16 || P <= 0 || P > 65535 || !sight_ok(sight) || keep || wide)
+    return AS_BAD_SHAPE;
+  if ((tiles && (P != 1 || most <= 0)) || (P > 1 && (!part_m || !part_l || !part_acc))) return AS_BAD_SHAPE;
+  const int per = tiles ? 16 / (H / KV) : 1, subs = tiles ? (most + per - 1) / per : 1;
+  if ((long)blocks_of * subs > 0x7fffffffL) return AS_BAD_SHAPE;
+  const dim3 grid(blocks_of * subs, KV, P);
+  const size_t lds = (128 + 4 * 16 * (D + 4)) * sizeof(float);
+  if (D == 64)
+    attn_f32_kernel<4><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width,
+                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P);
+  else
+    attn_f32_kernel<8><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width,
+                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P);
+  if (P > 1) {
+    const int rc = launch_status();
+    if (rc != AS_OK) return rc;
+    attn_reduce_kernel<float><<<dim3(num_items, H), D, 0, stream>>>(items, part_m, part_l, part_acc, out, H, D, P, sight.sink, sight.sinks, 0);
+  }
+  return launch_status();
+}
+
 // ---- the same without scratch buffers from the caller ----------------------------------
 //
 // The partial results of a split context live in an array of the library's own; see no_alloc.h.

@@ -270,7 +270,13 @@ def attn_single_query(q, k_pages, v_pages, items, positions, tok_row, block_tabl
              _ptr(tok_row), _ptr(block_tables), block_tables.shape[1], _ptr(out), _ptr(part_m), _ptr(part_l),
              _ptr(part_acc), H, KV * share, D, bs, float(scale), *sight, part_size, P, share, _stream())  # fmt: skip
         return
-    part_size, P, part_m, part_l, part_acc = _partitions(N, H, KV, D, max_context, window or chunk, mfma, part_size, q.device, sight[1])
+    matrix32 = not force_generic and attn_f32_supported(q.dtype, H, KV, D, bs, sight[1]) and (part_size is None or part_size % 32 == 0)
+    part_size, P, part_m, part_l, part_acc = _partitions(N, H, KV, D, max_context, window or chunk, mfma or matrix32, part_size, q.device, sight[1])
+    if matrix32:
+        call("as_attn_f32", _ptr(q), _ptr(k_pages), _ptr(v_pages), 0, 0, 0, _ptr(items), N, _ptr(positions), _ptr(tok_row),
+             _ptr(block_tables), block_tables.shape[1], _ptr(out), _ptr(part_m), _ptr(part_l), _ptr(part_acc), H, KV, D, bs,
+             float(scale), *sight, part_size, P, _stream())  # fmt: skip
+        return
     if mfma:
         call("as_attn_decode_mfma", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(items), N, _ptr(positions),
              _ptr(tok_row), _ptr(block_tables), block_tables.shape[1], _ptr(out), _ptr(part_m), _ptr(part_l),
@@ -279,6 +285,33 @@ def attn_single_query(q, k_pages, v_pages, items, positions, tok_row, block_tabl
     call("as_attn_single_query", _ptr(q), _ptr(k_pages), _ptr(v_pages), _DT[q.dtype], _ptr(items), N,
          _ptr(positions), _ptr(tok_row), _ptr(block_tables), block_tables.shape[1], _ptr(out), _ptr(part_m),
          _ptr(part_l), _ptr(part_acc), H, KV, D, bs, float(scale), *sight, part_size, P, _stream())  # fmt: skip
+
+
+def attn_f32_supported(dtype, num_heads: int, num_kv_heads: int, head_dim: int, block_size: int, keep_first: int = 0) -> bool:
+    """Whether 32-bit heads run on the matrix cores (`attn_f32`, products and sums in 32 bits): heads of 64 or 128, at most 16 of
+    them to a kv head, whole steps of 16 keys to a page, no kept first keys; the rest runs on the general kernel."""
+    return (dtype == F32 and head_dim in (64, 128) and num_heads % num_kv_heads == 0 and num_heads // num_kv_heads <= 16
+            and block_size % 16 == 0 and keep_first == 0)  # fmt: skip
+
+
+def attn_prefill_f32(q, k_pages, v_pages, tiles, block_tables, out, scale, window, max_context, softcap=0.0, sink=False, chunk=0) -> None:
+    """`attn_prefill` for the 32-bit heads that `attn_f32_supported` names (tiles of up to PREFILL_TILE_QUERIES tokens)."""
+    _check(q, "q", F32, (None, None, None))
+    T, H, D = q.shape
+    sight = _sight(window, 0, chunk, softcap, sink, q, out)
+    _check(k_pages, "k_pages", F32, (None, None, None, D))
+    _, KV, bs, _ = k_pages.shape
+    _check(v_pages, "v_pages", F32, (k_pages.shape[0], KV, D, bs))
+    _check(tiles, "tiles", I32, (None, 4))
+    _check(block_tables, "block_tables", I32, (None, None))
+    if tiles.shape[0] == 0:
+        return
+    if not attn_f32_supported(q.dtype, H, KV, D, bs):
+        raise KernelError(f"prefill attention: unsupported heads {H}/{KV}, head width {D} or page size {bs}")
+    if max_context > block_tables.shape[1] * bs:
+        raise KernelError("attention: block tables are shorter than the longest context")
+    call("as_attn_f32", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(tiles), tiles.shape[0], PREFILL_TILE_QUERIES, 0, 0, 0, 0,
+         _ptr(block_tables), block_tables.shape[1], _ptr(out), 0, 0, 0, H, KV, D, bs, float(scale), *sight, 16, 1, _stream())  # fmt: skip
 
 
 DECODE_MFMA_MAX_LDS = 64 << 10  # what a workgroup may ask for without raising the kernel's limit

@@ -903,6 +903,40 @@ def test_attention_serves_only_the_listed_tokens(ops):
     assert bool((out[[0, 2, 3]] == 9.0).all())
 
 
+@pytest.mark.parametrize("H,KV,D,bs,how", [(16, 8, 128, 16, {}), (10, 2, 128, 32, {"window": 40}), (16, 1, 64, 16, {"window": 1}),
+                                           (3, 3, 64, 48, {"chunk": 23}), (21, 3, 128, 16, {"softcap": 0.5, "sink": True}),
+                                           (8, 2, 64, 16, {"window": 100, "sink": True})])  # fmt: skip
+def test_attention_in_32_bits_on_the_matrix_cores(ops, H, KV, D, bs, how):
+    """Single queries (whole contexts and partitions) and prompt tiles of 32-bit heads against the general kernel, which the
+    plain one checks: group sizes that do and do not divide a tile of 16 queries, contexts and portions around a step of 16
+    keys, windows, chunks, caps and sinks.  Tolerance: scores of at most 30 carry 128 roundings of 2^-24 each way, weights
+    and outputs (values of at most 5) as many again: 1e-4."""
+    torch.manual_seed(61)
+    rows = [(0, 1), (0, 15), (0, 16), (0, 17), (15, 9), (16, 65), (130, 33), (511, 12)]  # (start, new tokens)
+    lens = [a + n for a, n in rows]
+    _, k_pages, v_pages, tables, _ = paged_case(F32, H, KV, D, bs, lens, seed=5, k_scale=2.0 / math.sqrt(D / 16))
+    T = sum(n for _, n in rows)
+    q = torch.randn(T, H, D, device=DEV)
+    how = dict(how)
+    window = how.pop("window", 0)
+    positions, tok_row, tiles, flat = [], [], [], 0
+    for r, (start, n) in enumerate(rows):
+        positions += list(range(start, start + n))
+        tok_row += [r] * n
+        tiles += [[flat + q0, min(64, n - q0), r, start + q0] for q0 in range(0, n, 64)]
+        flat += n
+    single = (q, k_pages, v_pages, i32(list(range(T))), i32(positions), i32(tok_row), tables)
+    ref = torch.zeros(T, H, D, device=DEV)
+    ops.attn_single_query(*single, ref, D**-0.5, window, max(lens), force_generic=True, **how)
+    for part in (None, 32, 128, 2048):
+        out = torch.full((T, H, D), float("nan"), device=DEV)
+        ops.attn_single_query(*single, out, D**-0.5, window, max(lens), part, **how)
+        assert torch.allclose(out, ref, atol=1e-4), (part, (out - ref).abs().max())
+    out = torch.full((T, H, D), float("nan"), device=DEV)
+    ops.attn_prefill_f32(q, k_pages, v_pages, i32(tiles[::-1]), tables, out, D**-0.5, window, max(lens), **how)
+    assert torch.allclose(out, ref, atol=1e-4), (out - ref).abs().max()
+
+
 @pytest.mark.parametrize("H,KV,D,bs,window", [(32, 8, 128, 16, 0), (6, 2, 32, 16, 0), (8, 8, 64, 32, 0), (4, 1, 96, 16, 0),
                                                (16, 2, 128, 16, 0), (4, 2, 64, 16, 40), (4, 2, 64, 16, 1), (4, 2, 256, 16, 0),
                                                (2, 1, 224, 32, 0), (10, 2, 160, 16, 70)])  # fmt: skip
