@@ -295,7 +295,7 @@ __global__ __launch_bounds__(64) void delta_scan_kernel(const float* __restrict_
                                                         const int* __restrict__ row_first,
                                                         const int* __restrict__ row_len,
                                                         const int* __restrict__ row_start,
-                                                        const int* __restrict__ row_slots, int writes,
+                                                        const int* __restrict__ row_slots, int writes, int most,
                                                         float* __restrict__ out) {
   constexpr int NV = MODE == 1 ? 3 : 2;  // vectors of a token that go through LDS: key, query (, decays)
   extern __shared__ __attribute__((aligned(16))) float lds[];  // [DELTA_TB][NV][dimp], dimp = SL * RPL
@@ -307,6 +307,7 @@ __global__ __launch_bounds__(64) void delta_scan_kernel(const float* __restrict_
   const bool live = j < vdim;
   const int g = h / (H / G);
   const int first = row_first[r], len = row_len[r], slot = row_slots[r];
+  if (most > 0 && len > most) return;  // the chunked form's
   const int i0 = slice * RPL;
   float S[RPL];
   float N[MODE == 2 ? RPL : 1];
@@ -471,7 +472,7 @@ template <int MODE>
 static int launch_delta_scan(const float* qkv, int C, int G, int dim, int H, int vdim, const float* beta,
                              const float* decay, const float* chan, float* state, float* norm_state, float* max_state,
                              const int* row_first, const int* row_len, const int* row_start, const int* row_slots,
-                             int writes, float* out, int num_rows, int force_slices, hipStream_t stream) {
+                             int writes, float* out, int num_rows, int force_slices, hipStream_t stream, int most = 0) {
   if (num_rows <= 0) return AS_OK;
   if (G <= 0 || H <= 0 || H % G || dim <= 0 || vdim <= 0 || C < 2 * G * dim + H * vdim || H > 65535)
     return AS_BAD_SHAPE;
@@ -499,7 +500,7 @@ static int launch_delta_scan(const float* qkv, int C, int G, int dim, int H, int
 #define LAUNCH(R, SLV)                                                                                            \
   delta_scan_kernel<R, SLV, MODE><<<grid, 64, lds, stream>>>(qkv, C, G, dim, H, vdim, beta, decay, chan, state,   \
                                                              norm_state, max_state, row_first, row_len, row_start, \
-                                                             row_slots, writes, out)
+                                                             row_slots, writes, most, out)
 #define LAUNCH_SL(R)              \
   do {                            \
     if (slices == 1) LAUNCH(R, 1);      \
@@ -517,12 +518,398 @@ static int launch_delta_scan(const float* qkv, int C, int G, int dim, int H, int
   return launch_status();
 }
 
+// most > 0: rows of more tokens are left out (`as_delta_chunks` takes them).
 extern "C" int as_delta_scan(const float* qkv, int C, int G, int dim, int H, int vdim, const float* beta,
                              const float* decay, float* state, const int* row_first, const int* row_len,
                              const int* row_start, const int* row_slots, int writes, float* out, int num_rows,
-                             int force_slices, hipStream_t stream) {
+                             int force_slices, int most, hipStream_t stream) {
   return launch_delta_scan<0>(qkv, C, G, dim, H, vdim, beta, decay, nullptr, state, nullptr, nullptr, row_first, row_len,
-                              row_start, row_slots, writes, out, num_rows, force_slices, stream);
+                              row_start, row_slots, writes, out, num_rows, force_slices, stream, most);
+}
+
+// The rule in chunks of 64 tokens (long rows).  With D[t, j] = g_{j+1} .. g_t, P_t = g_1 .. g_t within the chunk and S the state
+// before it, the updates of a chunk solve a triangular system:
+//   u_t = beta_t (v_t - P_t S^T k_t - sum_{j<t} D[t, j] (k_t . k_j) u_j),  so  U = (I + A)^-1 diag(beta) (V - P K S)
+// with A[t, j] = beta_t D[t, j] k_t . k_j below the diagonal;
+//   o_t = P_t S^T q_t + sum_{j<=t} D[t, j] (q_t . k_j) u_j,   S <- P_64 S + sum_j D[64, j] k_j u_j^T.
+// delta_pairs (a workgroup a chunk and head, all side by side) makes (I + A)^-1 diag(beta) and D (Q K^T); delta_chunks (a
+// workgroup a row, head and 16 columns of the state) walks the chunks.  All of it in 32 bits: products by
+// v_mfma_f32_16x16x4_f32, the decays by multiplication in the order of the scan (no logarithms, so none is lost to a
+// strong decay before a weak one).  A token whose key, query, value, beta or decay is not finite ends its chunk: the tokens before
+// it are computed without it, its own outputs and all that follow are NaN.
+// Bound by the chain of a chunk (128 matrix instructions of a workgroup's last wave, which take 1.9 us, and three barriers: 4.1 us a
+// chunk) and by the fill of the GPU (rows x heads x column groups workgroups).  One prompt of 1,500 tokens, 16 heads of 128 x 128:
+// 26 + 99 us; token by token (0.4 us a token, the scan above) 618.  The triangle inverted by one wave, a column to a lane from the top down, took
+// the first kernel 33 us.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+#define DC 64                            // tokens of a chunk
+#define DC_SCRATCH (2 * DC * DC + 3 * DC)  // floats per chunk and head: the inverse, the pairs, P, D[64, :], the first bad token
+
+__device__ __forceinline__ int delta_chunks_of(int len, int most) { return len > most ? (len + DC - 1) / DC : 0; }
+__device__ __forceinline__ bool finite4(floatx4 v) {
+  const float s = (v[0] - v[0]) + (v[1] - v[1]) + (v[2] - v[2]) + (v[3] - v[3]);  // 0, or NaN if one is not finite
+  return s == 0.f;
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void delta_pairs_kernel(const float* __restrict__ qkv, int C, int G, int H, int vdim,
+                                                          const float* __restrict__ beta, const float* __restrict__ decay,
+                                                          const int* __restrict__ row_first, const int* __restrict__ row_len,
+                                                          int num_rows, int most, float* __restrict__ scratch) {
+  constexpr int dim = 16 * DT, LA = DC + 4, LDD = DC + 1;
+  __shared__ __attribute__((aligned(16))) float A[DC * LA];
+  __shared__ float D[DC * LDD];
+  __shared__ __attribute__((aligned(16))) float sg[DC], sb[DC];
+  __shared__ floatx4 inv[4][4][64];
+  __shared__ __attribute__((aligned(16))) float rows[4][16 * 20];
+  __shared__ int s_bad;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4, h = blockIdx.y, g = h / (H / G);
+  int chunk = blockIdx.x, r = 0;
+  for (; r < num_rows; ++r) {
+    const int n = delta_chunks_of(row_len[r], most);
+    if (chunk < n) break;
+    chunk -= n;
+  }
+  if (r == num_rows) return;
+  const int first = row_first[r] + chunk * DC, n = min(DC, row_len[r] - chunk * DC);
+  float* mine = scratch + ((size_t)blockIdx.x * H + h) * DC_SCRATCH;
+  const int q_col = g * dim, k_col = (G + g) * dim, v_col = 2 * G * dim + h * vdim;
+  if (tid == 0) s_bad = DC;
+  __syncthreads();
+  auto row_of = [&](int tile, int col) { return qkv + (size_t)(first + min(tile * 16 + lr, n - 1)) * C + col + lg * 4; };
+  floatx4 q[DT], kk[4][DT];  // this wave's 16 queries, and the keys of every token up to its own: all asked for at once
+  {
+    const float* qp = row_of(wave, q_col);
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {
+      if (j <= wave) {
+        const float* kp = row_of(j, k_col);
+#pragma unroll
+        for (int i = 0; i < DT; ++i) kk[j][i] = *reinterpret_cast<const floatx4*>(kp + i * 16);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < DT; ++i) q[i] = *reinterpret_cast<const floatx4*>(qp + i * 16);
+    if (tid < DC) {
+      const size_t at = (size_t)(first + min(tid, n - 1)) * H + h;
+      const float bt = beta[at], gt = decay[at];
+      if (tid < n && !finite4(floatx4{bt, gt, 0.f, 0.f})) atomicMin(&s_bad, tid);
+      sg[tid] = tid < n ? gt : 1.f;
+      sb[tid] = tid < n ? bt : 0.f;
+    }
+    const int quads = vdim / 4, pieces = n * quads;
+    for (int x0 = tid; x0 < pieces; x0 += 256 * 8) {  // the values are only looked at here
+      floatx4 v[8];
+#pragma unroll
+      for (int y = 0; y < 8; ++y) {
+        const int x = min(x0 + y * 256, pieces - 1);
+        v[y] = *reinterpret_cast<const floatx4*>(qkv + (size_t)(first + x / quads) * C + v_col + x % quads * 4);
+      }
+#pragma unroll
+      for (int y = 0; y < 8; ++y)
+        if (!finite4(v[y])) atomicMin(&s_bad, min(x0 + y * 256, pieces - 1) / quads);
+    }
+    bool good = true;
+#pragma unroll
+    for (int i = 0; i < DT; ++i) {
+      good = good && finite4(q[i]);
+      if (wave == 0) good = good && finite4(kk[0][i]);
+      if (wave == 1) good = good && finite4(kk[1][i]);
+      if (wave == 2) good = good && finite4(kk[2][i]);
+      if (wave == 3) good = good && finite4(kk[3][i]);
+    }
+    if (!good && wave * 16 + lr < n) atomicMin(&s_bad, wave * 16 + lr);
+  }
+  __syncthreads();
+  const int bad = s_bad;  // tokens from here on count as none
+  if (bad < DC) {
+    if (tid < DC && tid >= bad) { sg[tid] = 1.f; sb[tid] = 0.f; }
+#pragma unroll
+    for (int i = 0; i < DT; ++i) {
+      if (wave * 16 + lr >= bad) q[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j * 16 + lr >= bad) kk[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    __syncthreads();
+  }
+  {  // column `lane` of D: this wave keeps its 16 rows
+    float cur = 0.f;
+    for (int t4 = 0; t4 < DC; t4 += 16) {
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) {
+        const floatx4 gg = *reinterpret_cast<const floatx4*>(sg + t4 + i);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          cur = t4 + i + x == lane ? 1.f : cur * gg[x];  // 0 above the diagonal
+          if (t4 >> 4 == wave) D[(t4 + i + x) * LDD + lane] = cur;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  floatx4 own[DT];  // the keys of this wave's own tokens
+#pragma unroll
+  for (int i = 0; i < DT; ++i) own[i] = wave == 0 ? kk[0][i] : wave == 1 ? kk[1][i] : wave == 2 ? kk[2][i] : kk[3][i];
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) {
+    if (jt <= wave) {
+      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(own[i][x], kk[jt][i][x], acc, 0, 0, 0);
+      const int j = jt * 16 + lr;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int t = wave * 16 + lg * 4 + x;
+        A[t * LA + j] = j < t ? sb[t] * D[t * LDD + j] * acc[x] : 0.f;
+      }
+    }
+  }
+  // The inverse in blocks of 16: a wave inverts its block on the diagonal, column by column from the top down, then the
+  // blocks below, one diagonal after the other: T_ij = -T_ii sum_k A_ik T_kj.  A block lies as a product leaves it (lane:
+  // column lr, rows 4 lg + x), which is how the next product takes it as its right operand.
+  floatx4 diag, left;  // T_ww as a right and as a left operand
+  {
+    const float* block = A + (wave * 16) * LA + wave * 16;
+    float x[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float v = t == lr ? 1.f : 0.f;
+#pragma unroll
+      for (int i = 0; i < t; i += 4) {
+        const floatx4 row = *reinterpret_cast<const floatx4*>(block + t * LA + i);
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+          if (i + y < t) v = fmaf(-row[y], x[i + y], v);
+      }
+      x[t] = v;
+    }
+#pragma unroll
+    for (int y = 0; y < 4; ++y) diag[y] = lg == 0 ? x[y] : lg == 1 ? x[4 + y] : lg == 2 ? x[8 + y] : x[12 + y];
+    if (lg == 0) {
+#pragma unroll
+      for (int t = 0; t < 16; ++t) rows[wave][t * 20 + lr] = x[t];
+    }
+    inv[wave][wave][lane] = diag;
+  }
+  __syncthreads();
+  left = *reinterpret_cast<const floatx4*>(rows[wave] + lr * 20 + lg * 4);
+#pragma unroll
+  for (int d = 1; d < 4; ++d) {
+    if (wave >= d) {
+      const int j = wave - d;
+      floatx4 m = floatx4{0.f, 0.f, 0.f, 0.f}, t = m;
+      for (int k = j; k < wave; ++k) {
+        const floatx4 l = *reinterpret_cast<const floatx4*>(A + (wave * 16 + lr) * LA + k * 16 + lg * 4), r = inv[k][j][lane];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) m = __builtin_amdgcn_mfma_f32_16x16x4f32(l[x], r[x], m, 0, 0, 0);
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) t = __builtin_amdgcn_mfma_f32_16x16x4f32(-left[x], m[x], t, 0, 0, 0);
+      inv[wave][j][lane] = t;
+    }
+    __syncthreads();
+  }
+  for (int j = 0; j <= wave; ++j) {
+    const floatx4 t = inv[wave][j][lane];
+    const float bj = sb[j * 16 + lr];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) mine[(wave * 16 + lg * 4 + x) * DC + j * 16 + lr] = t[x] * bj;
+  }
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) {  // queries and keys
+    if (jt <= wave) {
+      floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i][x], kk[jt][i][x], acc, 0, 0, 0);
+      const int j = jt * 16 + lr;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int t = wave * 16 + lg * 4 + x;
+        mine[DC * DC + t * DC + j] = j <= t ? D[t * LDD + j] * acc[x] : 0.f;
+      }
+    }
+  }
+  if (wave == 0) {
+    mine[2 * DC * DC + lane] = D[lane * LDD] * sg[0];
+    mine[2 * DC * DC + DC + lane] = D[(DC - 1) * LDD + lane];
+    if (lane == 0) reinterpret_cast<int*>(mine)[2 * DC * DC + 2 * DC] = bad;
+  }
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restrict__ qkv, int C, int G, int H, int vdim,
+                                                           float* __restrict__ state, const int* __restrict__ row_first,
+                                                           const int* __restrict__ row_len, const int* __restrict__ row_start,
+                                                           const int* __restrict__ row_slots, int writes, int most,
+                                                           const float* __restrict__ scratch, int per_xcd, int total,
+                                                           float* __restrict__ out) {
+  constexpr int dim = 16 * DT, LK = dim + 4;
+  __shared__ __attribute__((aligned(16))) float keys[DC * LK];
+  __shared__ floatx4 sy[4 * 64], su[4 * 64], se[4 * 64], ss[DT * 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  // a head's column groups side by side on one XCD (workgroups are dealt to the eight in turn): they read the same
+  const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (item >= total) return;
+  const int groups = vdim / 16, c0 = item % groups * 16, h = item / groups % H, r = item / groups / H, g = h / (H / G);
+  const int len = row_len[r], chunks = delta_chunks_of(len, most);
+  if (chunks == 0) return;
+  int before = 0;
+  for (int i = 0; i < r; ++i) before += delta_chunks_of(row_len[i], most);
+  const int first = row_first[r], slot = row_slots[r];
+  const bool carried = row_start[r] > 0 && slot >= 0;
+  float* kept = state + ((size_t)(slot < 0 ? 0 : slot) * H + h) * dim * vdim + c0 + lr;
+  const int q_col = g * dim, k_col = (G + g) * dim, v_col = 2 * G * dim + h * vdim + c0 + lr;
+
+  // S: tile i holds rows 16 i + 4 lg + x of column c0 + lr, the layout of a product's result, which is also what a product
+  // takes as its right operand when the left one brings its four columns 16 i + 4 lg + x the same way
+  floatx4 S[DT], kf[DT], qf[DT], tf[4], pf[4], vv, P, E;
+#pragma unroll
+  for (int i = 0; i < DT; ++i) {
+#pragma unroll
+    for (int x = 0; x < 4; ++x) S[i][x] = carried ? kept[(size_t)(16 * i + 4 * lg + x) * vdim] : 0.f;
+    if (wave == 0) ss[i * 64 + lane] = S[i];
+  }
+  int bad = DC;
+  float last_P = 1.f;
+  auto token = [&](int n, int t) { return qkv + (size_t)(first + min(n * DC + t, len - 1)) * C; };
+  auto load_rows = [&](int n) {
+    const float* p = token(n, wave * 16 + lr) + lg * 4;
+#pragma unroll
+    for (int i = 0; i < DT; ++i) kf[i] = *reinterpret_cast<const floatx4*>(p + k_col + i * 16);
+#pragma unroll
+    for (int i = 0; i < DT; ++i) qf[i] = *reinterpret_cast<const floatx4*>(p + q_col + i * 16);
+  };
+  auto load_rest = [&](int n) {
+    const float* mine = scratch + ((size_t)(before + n) * H + h) * DC_SCRATCH;
+    const float* p = mine + (wave * 16 + lr) * DC + lg * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j <= wave) {
+        tf[j] = *reinterpret_cast<const floatx4*>(p + j * 16);
+        pf[j] = *reinterpret_cast<const floatx4*>(p + DC * DC + j * 16);
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 4; ++x) vv[x] = token(n, wave * 16 + lg * 4 + x)[v_col];
+    P = *reinterpret_cast<const floatx4*>(mine + 2 * DC * DC + wave * 16 + lg * 4);
+    E = *reinterpret_cast<const floatx4*>(mine + 2 * DC * DC + DC + wave * 16 + lg * 4);
+    last_P = mine[2 * DC * DC + DC - 1];
+    bad = reinterpret_cast<const int*>(mine)[2 * DC * DC + 2 * DC];
+  };
+  load_rows(0);
+  load_rest(0);
+  for (int n = 0; n < chunks; ++n) {
+    const int limit = bad;
+    if (limit < DC && wave * 16 + lr >= limit) {
+#pragma unroll
+      for (int i = 0; i < DT; ++i) kf[i] = qf[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < DT; ++i) *reinterpret_cast<floatx4*>(keys + (wave * 16 + lr) * LK + i * 16 + lg * 4) = kf[i];
+    floatx4 xk = floatx4{0.f, 0.f, 0.f, 0.f}, xq = xk;
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        xk = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][x], S[i][x], xk, 0, 0, 0);
+        xq = __builtin_amdgcn_mfma_f32_16x16x4f32(qf[i][x], S[i][x], xq, 0, 0, 0);
+      }
+    const int ahead = min(n + 1, chunks - 1);
+    load_rows(ahead);
+    floatx4 y = vv - P * xk;
+    if (limit < DC) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        if (wave * 16 + lg * 4 + x >= limit) y[x] = 0.f;
+    }
+    sy[wave * 64 + lane] = y;
+    __syncthreads();
+    floatx4 u = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j <= wave) {
+        const floatx4 yj = sy[j * 64 + lane];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) u = __builtin_amdgcn_mfma_f32_16x16x4f32(tf[j][x], yj[x], u, 0, 0, 0);
+      }
+    }
+    su[wave * 64 + lane] = u;
+    se[wave * 64 + lane] = u * E;
+    __syncthreads();
+    floatx4 o = P * xq;
+    // the state first (the next chunk waits for it), then the outputs
+    floatx4 next[DT / 4];
+#pragma unroll
+    for (int m = 0; m < DT / 4; ++m) {
+      const int i = wave * (DT / 4) + m;
+      next[m] = ss[i * 64 + lane] * last_P;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const floatx4 uj = se[j * 64 + lane];
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          next[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(keys[(j * 16 + lg * 4 + x) * LK + i * 16 + lr], uj[x], next[m], 0, 0, 0);
+      }
+      if (limit < DC) next[m] = floatx4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+      ss[i * 64 + lane] = next[m];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j <= wave) {
+        const floatx4 uj = su[j * 64 + lane];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) o = __builtin_amdgcn_mfma_f32_16x16x4f32(pf[j][x], uj[x], o, 0, 0, 0);
+      }
+    }
+    load_rest(ahead);  // before the stores: who waits for it does not wait for them
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const int t = wave * 16 + lg * 4 + x;
+      if (n * DC + t < len) out[((size_t)(first + n * DC + t) * H + h) * vdim + c0 + lr] = t < limit ? o[x] : __builtin_nanf("");
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < DT; ++i) S[i] = ss[i * 64 + lane];
+  }
+  if (writes && slot >= 0 && wave == 0) {
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+      for (int x = 0; x < 4; ++x) kept[(size_t)(16 * i + 4 * lg + x) * vdim] = S[i][x];
+  }
+}
+
+// Rows of more than `most` tokens.  Heads of 64 or 128 keys, values in whole tiles of 16, every key, query and value on 16
+// bytes.  scratch: most_chunks x H x (2 x 64 x 64 + 3 x 64) floats, most_chunks at least the chunks of 64 tokens that these rows have.
+extern "C" int as_delta_chunks(const float* qkv, int C, int G, int dim, int H, int vdim, const float* beta, const float* decay,
+                               float* state, const int* row_first, const int* row_len, const int* row_start,
+                               const int* row_slots, int writes, float* out, int num_rows, int most, float* scratch,
+                               int most_chunks, hipStream_t stream) {
+  if (num_rows <= 0 || most_chunks <= 0) return AS_OK;
+  if (G <= 0 || H <= 0 || H % G || H > 65535 || (dim != 64 && dim != 128) || vdim <= 0 || vdim % 16 || C % 4 || most < 0 ||
+      C < 2 * G * dim + H * vdim || ((uintptr_t)qkv & 15) || ((uintptr_t)scratch & 15) || !scratch)
+    return AS_BAD_SHAPE;
+  const long total = (long)num_rows * H * (vdim / 16);
+  if (total > 0x3fffffff) return AS_BAD_SHAPE;
+  const int per_xcd = (int)((total + 7) / 8);
+#define LAUNCH(DT)                                                                                                             \
+  do {                                                                                                                         \
+    delta_pairs_kernel<DT><<<dim3(most_chunks, H), 256, 0, stream>>>(qkv, C, G, H, vdim, beta, decay, row_first, row_len,      \
+                                                                     num_rows, most, scratch);                                 \
+    delta_chunks_kernel<DT><<<per_xcd * 8, 256, 0, stream>>>(qkv, C, G, H, vdim, state, row_first, row_len, row_start,         \
+                                                             row_slots, writes, most, scratch, per_xcd, (int)total, out);      \
+  } while (0)
+  if (dim == 64) LAUNCH(4);
+  else LAUNCH(8);
+#undef LAUNCH
+  return launch_status();
 }
 
 // The same rule with a decay per head and key channel: chan [T, H, dim].

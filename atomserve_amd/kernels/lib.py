@@ -40,7 +40,8 @@ SIGNATURES = {
     "as_sigmoid_gate_heads": ("elementwise", [P, I, I, I, I, P, I, I, I, F, P, I, I, I, P]),
     "as_short_conv": ("recurrent", [P, I, I, I, I, P, P, P, I, I, I, P, P, P, P, P, P, P, I, I, I, P]),
     "as_delta_prepare": ("recurrent", [P, I, I, I, I, P, I, I, I, I, P, P, I, P, P, I, P]),
-    "as_delta_scan": ("recurrent", [P, I, I, I, I, I, P, P, P, P, P, P, P, I, P, I, I, P]),
+    "as_delta_scan": ("recurrent", [P, I, I, I, I, I, P, P, P, P, P, P, P, I, P, I, I, I, P]),
+    "as_delta_chunks": ("recurrent", [P, I, I, I, I, I, P, P, P, P, P, P, P, I, P, I, I, P, I, P]),
     "as_delta_finish": ("recurrent", [P, I, I, P, I, I, F, P, I, I, I, I, F, P, I, I, I, P]),
     "as_delta_scan_channels": ("recurrent", [P, I, I, I, I, I, P, P, P, P, P, P, P, I, P, I, I, P]),
     "as_delta_prepare_channels": ("recurrent", [P, I, I, I, I, P, I, I, I, P, I, I, P, P, P, P, I, P]),

@@ -1633,12 +1633,23 @@ def delta_prepare(qkv, num_kv_heads, dim, num_heads, proj, b_off, a_off, a_log, 
          _ptr(dt_bias), _DT[w_dtype], _ptr(beta), _ptr(decay), T, _stream())  # fmt: skip
 
 
-def delta_scan(qkv, num_kv_heads, dim, num_heads, vdim, beta, decay, state, step_rows, out, writes=True, slices=0) -> None:
+# Rows of more tokens than this take the delta rule in chunks of 64 (csrc/recurrent.hip, delta_chunks), shorter ones token by
+# token: the chunks' two kernels take 35 us for one chunk of 8 to 32 heads of 128 and 4 us for every further one, the scan 0.4 us
+# a token (16 heads: 64 tokens 31 against 35 us, 100 tokens 46 and 37, 2,048 tokens 855 and 163; eight rows of 64 46 and 56, of 128
+# 81 and 72).
+DELTA_SCAN_MOST = 79
+DELTA_CHUNK = 64
+DELTA_CHUNK_SCRATCH = 2 * DELTA_CHUNK * DELTA_CHUNK + 3 * DELTA_CHUNK  # floats per chunk and head
+
+
+def delta_scan(qkv, num_kv_heads, dim, num_heads, vdim, beta, decay, state, step_rows, out, writes=True, slices=0, longest=0) -> None:
     """The gated delta rule over each row's tokens, per head h (keys and queries of head h // (H / G)):
     S <- decay S; u = beta (v - S^T k); S <- S + k u^T; out = S^T q.  state fp32 [slots, H, dim, vdim]; a row
     that starts at position 0 starts from zero.  qkv as `delta_prepare` left it; out fp32 [T, H, vdim].
     slices: into how many lanes a column of the state is cut (1, 2, 4, 8, 16); 0: chosen so that the step's rows,
-    heads and column groups fill the GPU (the results differ by the order of the sums only)."""
+    heads and column groups fill the GPU (the results differ by the order of the sums only).
+    longest: the most tokens that a row brings, if the caller knows it: long rows then run in chunks (heads of 64 or 128
+    keys, values in multiples of 16), the short ones of the step beside them as they are."""
     _check(qkv, "qkv", F32, (None, None))
     T, C = qkv.shape
     G, H = num_kv_heads, num_heads
@@ -1650,8 +1661,16 @@ def delta_scan(qkv, num_kv_heads, dim, num_heads, vdim, beta, decay, state, step
     _check(out, "out", F32, (T, H, vdim))
     R = _check_rows((None, *step_rows[1:]), 0)
     _, row_first, row_len, row_start, row_slots = step_rows
-    call("as_delta_scan", _ptr(qkv), C, G, dim, H, vdim, _ptr(beta), _ptr(decay), _ptr(state), _ptr(row_first),
-         _ptr(row_len), _ptr(row_start), _ptr(row_slots), int(bool(writes)), _ptr(out), R, int(slices), _stream())  # fmt: skip
+    chunked = (longest > DELTA_SCAN_MOST and slices == 0 and dim in (64, 128) and vdim % 16 == 0 and C % 4 == 0
+               and qkv.data_ptr() % 16 == 0)  # fmt: skip
+    args = (_ptr(qkv), C, G, dim, H, vdim, _ptr(beta), _ptr(decay), _ptr(state), _ptr(row_first), _ptr(row_len), _ptr(row_start),
+            _ptr(row_slots), int(bool(writes)), _ptr(out), R)  # fmt: skip
+    if not chunked or R > 1:
+        call("as_delta_scan", *args, int(slices), DELTA_SCAN_MOST if chunked else 0, _stream())
+    if chunked:
+        chunks = T // DELTA_CHUNK + min(R, T // (DELTA_SCAN_MOST + 1))  # at least as many as the long rows have
+        scratch = torch.empty((chunks, H, DELTA_CHUNK_SCRATCH), dtype=F32, device=qkv.device)
+        call("as_delta_chunks", *args, DELTA_SCAN_MOST, _ptr(scratch), chunks, _stream())
 
 
 def delta_finish(o, weight, eps, proj, g_off, act, gate="silu", scale: float = 1.0, out_off: int = 0) -> None:

@@ -90,7 +90,8 @@ class DeltaRule(Mixer):
         decay = torch.empty((T, H), dtype=torch.float32, device=dev)
         ops.delta_prepare(qkv, G, s.key_dim, H, proj, self.beta_off, self.step_off, self.a_log, self.dt_bias, beta, decay)
         o = torch.empty((T, H, s.value_dim), dtype=torch.float32, device=dev)
-        ops.delta_scan(qkv, G, s.key_dim, H, s.value_dim, beta, decay, state.state, rows, o, writes=state.writes)
+        ops.delta_scan(qkv, G, s.key_dim, H, s.value_dim, beta, decay, state.state, rows, o, writes=state.writes,
+                       longest=step.longest_row)  # fmt: skip
         act = torch.empty((T, H * s.value_dim), dtype=env.dtype, device=dev)
         ops.delta_finish(o, self.out_norm_weight, s.out_norm_eps, proj, self.gate_off, act)
         y = torch.empty((T, s.hidden_size), dtype=env.dtype, device=dev)

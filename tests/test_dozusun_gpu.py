@@ -298,6 +298,64 @@ def test_delta_scan_however_the_state_is_cut_over_lanes(dim, vdim):
     assert tried >= 4
 
 
+@pytest.mark.parametrize("dim,vdim,G,H", [(128, 128, 1, 2), (64, 48, 2, 2), (128, 16, 1, 3)])
+def test_delta_rule_in_chunks(dim, vdim, G, H):
+    """Rows around the chunk of 64 tokens and around the length from which chunks are taken, short rows beside them, states that
+    are carried or not, decays from 1 down to 0 in any order: the chunked form is no further from the recurrence in 64 bits
+    than twice the scan (the same sums of 32-bit terms in another order), and a token that is not finite leaves the tokens
+    before it and the other rows untouched."""
+    from atomserve_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(dim + vdim)
+    lens, starts, slots = [80, 128, 79, 1, 129, 200, 127, 300], [0, 5, 0, 9, 0, 64, 3, 0], [2, 0, 1, 7, 3, 4, -1, 6]
+    T, C = sum(lens), 2 * G * dim + H * vdim
+    qkv = torch.randn(T, C, generator=gen)
+    for x in qkv[:, : 2 * G * dim].split(dim, 1):
+        x /= x.norm(dim=1, keepdim=True)
+    beta, decay = torch.rand(T, H, generator=gen), torch.rand(T, H, generator=gen) ** 0.05
+    strong = torch.rand(T, H, generator=gen)
+    decay[strong < 0.02] = 1e-30
+    decay[strong < 0.005] = 0.0
+    decay[strong > 0.9] = 1.0
+    decay[-300:, 0] = 0.999  # a row that hardly forgets
+    state0 = torch.randn(8, H, dim, vdim, generator=gen)
+    q, k = (qkv[:, i * G * dim : (i + 1) * G * dim].view(T, G, dim).repeat_interleave(H // G, 1).double() for i in (0, 1))
+    v, want, at, final = qkv[:, 2 * G * dim :].view(T, H, vdim).double(), torch.zeros(T, H, vdim, dtype=torch.float64), 0, state0.double().clone()
+    for n, start, slot in zip(lens, starts, slots):
+        S = final[slot].clone() if start > 0 and slot >= 0 else torch.zeros(H, dim, vdim, dtype=torch.float64)
+        for t in range(at, at + n):
+            S = decay[t].double()[:, None, None] * S
+            u = beta[t].double()[:, None] * (v[t] - torch.einsum("hdv,hd->hv", S, k[t]))
+            S = S + torch.einsum("hd,hv->hdv", k[t], u)
+            want[t] = torch.einsum("hdv,hd->hv", S, q[t])
+        if slot >= 0:
+            final[slot] = S
+        at += n
+    firsts = [sum(lens[:i]) for i in range(len(lens))]
+    rows = (None,) + tuple(torch.tensor(x, dtype=torch.int32, device=DEV) for x in (firsts, lens, starts, slots))
+
+    def run(values, **how):
+        state, out = state0.clone().to(DEV), torch.full((T, H, vdim), 7.0, device=DEV)
+        ops.delta_scan(values.to(DEV), G, dim, H, vdim, beta.to(DEV), decay.to(DEV), state, rows, out, **how)
+        return out.cpu(), state.cpu()
+
+    (scan, scan_state), (out, state) = run(qkv), run(qkv, longest=max(lens))
+    far = lambda x, ref: float((x.double() - ref).norm() / ref.norm())  # noqa: E731
+    assert far(out, want) <= 2 * far(scan, want) and far(state, final) <= 2 * far(scan_state, final), (
+        f"{far(out, want):.2e} against {far(scan, want):.2e}, states {far(state, final):.2e} against {far(scan_state, final):.2e}")  # fmt: skip
+    assert (out.double() - want).abs().max() <= 2e-5 * float(want.abs().max())
+    kept, kept_state = run(qkv, longest=max(lens), writes=False)
+    assert torch.equal(kept, out) and torch.equal(kept_state, state0)
+    broken = qkv.clone()
+    place = firsts[5] + 70
+    broken[place, 2 * G * dim + 3] = float("inf")  # a value of the first head
+    got, got_state = run(broken, longest=max(lens))
+    rest = torch.ones(T, dtype=torch.bool)
+    rest[place : firsts[6]] = False
+    assert torch.allclose(got[rest], out[rest], atol=2e-5 * float(want.abs().max())) and torch.equal(got[:, 1:], out[:, 1:])
+    assert bool(got[place : firsts[6], 0, 3].isnan().all()) and bool(got_state[4, 0, :, 3].isnan().any()) and torch.equal(got_state[3], state[3])
+
+
 def test_delta_rule_keeps_a_far_token():
     """With a decay near one and a query that asks for one early token's key, the output hundreds of tokens later
     is that token's value: a state that was lost or restarted on the way shows as a difference of the output's size."""
