@@ -7,6 +7,7 @@ library cannot be built or loaded raises.
 """
 
 import ctypes
+import threading
 from ctypes import c_double, c_float, c_int, c_longlong, c_size_t, c_void_p
 
 import torch  # noqa: F401  (loads libamdhip64 first)
@@ -136,14 +137,67 @@ def entry(name: str):
     return fn
 
 
+class _Watch(threading.local):
+    """What this thread writes down: the calls of entry points and the tensors whose addresses they were given."""
+
+    calls = None
+    held = None
+    spoiled = False  # something ran that is not a call of an entry point, or not the call that the next time would make
+
+
+watch = _Watch()
+
+
 def call(name: str, *args) -> None:
-    status = entry(name)(*args)
+    fn = entry(name)
+    status = fn(*args)
     if status != 0:
         raise KernelError(f"{name}: {STATUS.get(status, status)}")
+    if watch.calls is not None:
+        watch.calls.append((name, fn, args))
+
+
+class Launches:
+    """The launches that a piece of code makes (`with Launches() as made:`), to be made again with other
+    addresses: `made.aim(sources)`, then `made.again(targets)` for as many lists of targets as there are: wherever a
+    call was given sources[i], it is given targets[i].  The tensors that the calls read and wrote are held as long as this
+    object lives, so that nobody else is given their memory between two repetitions."""
+
+    def __enter__(self):
+        if watch.calls is not None:
+            raise KernelError("launches are written down by one list at a time")
+        self.calls, self.held = [], []
+        watch.calls, watch.held, watch.spoiled = self.calls, self.held, False
+        return self
+
+    def __exit__(self, *error):
+        self.whole = not watch.spoiled
+        watch.calls = watch.held = None
+        return False
+
+    def aim(self, sources: list) -> None:
+        self.sources = sources
+        place = {address: i for i, address in enumerate(sources) if address}
+        self.patched = [(name, fn, list(args), [(at, place[v]) for at, v in enumerate(args) if type(v) is int and v in place])
+                        for name, fn, args in self.calls]  # fmt: skip
+
+    def fits(self, targets: list) -> bool:
+        """Whether `targets` can stand for the sources: as many, none where there was none, one address for one address."""
+        known = {}
+        return len(targets) == len(self.sources) and all(
+            bool(a) == bool(b) and (not a or known.setdefault(a, b) == b) for a, b in zip(self.sources, targets))  # fmt: skip
+
+    def again(self, targets: list) -> None:
+        for name, fn, args, patches in self.patched:
+            for at, i in patches:
+                args[at] = targets[i]
+            status = fn(*args)
+            if status != 0:
+                raise KernelError(f"{name}: {STATUS.get(status, status)}")
 
 
 def loaded_libraries() -> list:
     return sorted(_libs)
 
 
-__all__ = ["KernelError", "call", "entry", "loaded_libraries", "c_double"]
+__all__ = ["KernelError", "Launches", "call", "entry", "loaded_libraries", "c_double"]

@@ -6,6 +6,8 @@ the one hard-wired instance of this loop)."""
 import torch
 
 from atomserve_amd.kernels import ops
+from atomserve_amd.kernels.lib import Launches
+from atomserve_amd.models import repeats
 from atomserve_amd.parts.base import BuildEnv, GatedDelta, WeightDecl, build
 from atomserve_amd.parts.plan import ModelPlan
 
@@ -31,6 +33,7 @@ class DecoderModel:
                 raise ValueError(f"run list names layer {r.layer}, the plan has {len(self.blocks)}")
         self.embed_weight = None
         self.head_weight = None
+        self.stretches = repeats.stretches(plan, self.blocks)  # which layers are like the ones before them
 
     @property
     def capturable(self) -> bool:
@@ -146,19 +149,35 @@ class DecoderModel:
         elif p.reentry:
             x0 = x if p.run[0].reenter else x.clone()
         delta = None
-        for i, r in enumerate(p.run):
-            if r.reenter:
+        first, period, count = self.stretches or (len(p.run), 0, 0)
+        i = 0
+        while i < len(p.run):
+            if i == first and repeats.may_run_again(self, step, first, period):
+                before = delta
+                with Launches() as made:
+                    for k in range(period):
+                        delta = self._run(first + k, x, delta, step)
+                done, delta = repeats.run_again(self, made, step, before, delta, first, period, count)
+                i += period + done
+                continue
+            if p.run[i].reenter:
                 x, delta = self._reenter(x, delta, x0), None
-            # the norm that the run after this one starts with: this run's last product may add
-            # into x and leave that norm pending instead of handing over a delta
-            follows = self.blocks[p.run[i + 1].layer].first_norm() if i + 1 < len(p.run) else None
-            block = self.blocks[r.layer]
-            extra = {}
-            kept = block.cache_request()
-            if kept:
-                extra["own"] = {name: step.cache_view((self.layer_cache_id(i), name), True) for name in kept}
-            delta = block.forward(x, delta, step, step.cache_view(p.cache_id(i), r.writes), next_norm=follows, **extra)
+            delta = self._run(i, x, delta, step)
+            i += 1
         return self._head(x, delta, step, logits)
+
+    def _run(self, i: int, x, delta, step):
+        """Run `i` of the plan over the stream x and the pending output of the run before; returns its own."""
+        p, r = self.plan, self.plan.run[i]
+        # the norm that the run after this one starts with: this run's last product may add
+        # into x and leave that norm pending instead of handing over a delta
+        follows = self.blocks[p.run[i + 1].layer].first_norm() if i + 1 < len(p.run) else None
+        block = self.blocks[r.layer]
+        extra = {}
+        kept = block.cache_request()
+        if kept:
+            extra["own"] = {name: step.cache_view((self.layer_cache_id(i), name), True) for name in kept}
+        return block.forward(x, delta, step, step.cache_view(p.cache_id(i), r.writes), next_norm=follows, **extra)
 
     def _reenter(self, x, delta, x0):
         """The stream after the pending output `delta` has been added, beside x0, through the re-entry matrix:

@@ -55,6 +55,10 @@ class Attention(Mixer):
             )
         self.q_norm_weight = self.k_norm_weight = None
 
+    def repeats(self, step) -> bool:
+        # the rotation's table is made once a step, by the first layer that wants it
+        return type(self) is Attention and (self.position is None or self.position.made(step))
+
     def weight_decls(self) -> dict:
         s = self.spec
         decls = {

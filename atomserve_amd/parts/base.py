@@ -72,6 +72,13 @@ class Part:
         self.spec = spec
         self.env = env
 
+    def repeats(self, step: Any) -> bool:
+        """Whether what `forward` launches in this step is what any other part of an equal spec launches, with that
+        part's tensors (attributes that are tensors or `ops.Streamed`) and caches in place of this one's: every
+        launch goes through `kernels.lib.call`, and nothing is taken from, or left to, another layer's part.  A part says
+        so itself, for its own class only (a class derived from it may do more)."""
+        return False
+
     def weight_decls(self) -> dict:
         return {}
 
@@ -237,6 +244,10 @@ class Position(Part):
 
     def prepare(self, step: Any) -> Any:
         raise NotImplementedError
+
+    def made(self, step: Any) -> bool:
+        """Whether `prepare` launches nothing more in this step."""
+        return False
 
 
 class Arrangement:

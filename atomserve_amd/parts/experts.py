@@ -23,6 +23,10 @@ class TableExperts(FeedForward):
         if not 1 <= spec.top <= spec.num_experts <= ops.MOE_MAX_EXPERTS:
             raise ValueError(f"{spec.top} of {spec.num_experts} experts (at most {ops.MOE_MAX_EXPERTS}) cannot be chosen")
 
+    def repeats(self, step) -> bool:
+        # a table that an earlier layer has sorted the step by is not sorted by again
+        return type(self) is TableExperts and ("table_experts", self.table.data_ptr()) not in step.shared
+
     def weight_decls(self) -> dict:
         s = self.spec
         return {

@@ -20,6 +20,9 @@ class GatedMLP(FeedForward):
         if spec.activation == "clamped_swish" and not spec.limit > 0:
             raise ValueError("the activation with limits needs a positive limit")
 
+    def repeats(self, step) -> bool:
+        return type(self) is GatedMLP
+
     def weight_decls(self) -> dict:
         s = self.spec
         return {

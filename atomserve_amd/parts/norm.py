@@ -43,6 +43,9 @@ class RMSNorm(Norm):
     takes_gated_delta = True
     takes_normed_delta = True
 
+    def repeats(self, step) -> bool:
+        return type(self) is RMSNorm
+
     def weight_decls(self) -> dict:
         return {"weight": WeightDecl(() if self.spec.one_gain else (self.spec.size,), role="vector")}
 

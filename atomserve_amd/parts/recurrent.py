@@ -46,6 +46,9 @@ class DeltaRule(Mixer):
         self.gate_off, self.beta_off, self.step_off = self.channels, self.channels + v, self.channels + v + s.num_heads
         self.in_rows = self.step_off + s.num_heads
 
+    def repeats(self, step) -> bool:
+        return type(self) is DeltaRule
+
     def weight_decls(self) -> dict:
         s = self.spec
         return {
@@ -135,6 +138,9 @@ class SideBySide(Mixer):
         self.x_off = self.y_off + r.width
         self.in_rows = self.x_off + r.width
         self.out_cols = H * a.value_dim + r.width
+
+    def repeats(self, step) -> bool:
+        return type(self) is SideBySide
 
     def weight_decls(self) -> dict:
         s, a, r = self.spec, self.spec.left, self.spec.right

@@ -37,6 +37,9 @@ class RotaryHalf(Position):
             step.shared[key] = table
         return table
 
+    def made(self, step) -> bool:
+        return type(self) is RotaryHalf and ("rope_half", self.spec.rotary_dim, self.spec.theta) in step.shared
+
 
 register("position", "rope_half", RotaryHalf)
 
