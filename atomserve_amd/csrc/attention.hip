@@ -412,26 +412,34 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     const int* __restrict__ items, const int* __restrict__ positions, const int* __restrict__ tok_row,
     const int* __restrict__ block_tables, int table_width, bf16* __restrict__ out, float* __restrict__ part_m,
     float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int bs, float scale, Sight sight,
-    int part_size, int P, int cus, int share, FreshQKV fresh) {
+    int part_size, int P, int N, int cus, int share, FreshQKV fresh) {
   // share > 1: every `share` consecutive kv heads named here are one head of the pages (a group of more query heads
   // than a workgroup takes, cut into several); the pages then hold KV / share heads.
   constexpr int D = DC * 32, DT = DC * 2;  // DT: tiles of 16 output coordinates
   extern __shared__ float smem[];          // [4][16] m, [4][16] l, [4][D][G] acc
   __shared__ __align__(16) bf16 fresh_kv[2][256];  // FRESH: the new token's key and value
   const int G = H / KV;
-  int item = blockIdx.x, kvh = blockIdx.y;
-  const int part = blockIdx.z;
-  if (P == 1) {
+  int item = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
+  if (P > 1 && N > 8) {
+    // Partitions of many tokens: workgroups are dealt to the XCDs in turn, and with the tokens changing fastest an XCD had every
+    // eighth context, so that the one with the longest worked alone at the end.  With the kv heads changing fastest each has its
+    // share of every context: 13 requests of 300 to 7,000 keys in a step of 16 rows 67 -> 47 us, 20 of 200 to 3,000 in one of
+    // 32 60 -> 41 (equal contexts: within 2 per cent).  Up to eight tokens an XCD has one, and its keys' pages to itself: left so.
+    const int s = blockIdx.x + N * (blockIdx.y + KV * blockIdx.z), rest = s / KV;
+    part = rest / N;
+    item = rest - part * N;
+    kvh = (s - rest * KV + item) % KV;
+  } else if (P == 1) {
     // Whole contexts, one workgroup each, of unequal length: two workgroups share a compute unit, and
     // the first two rounds of `cus` workgroups are placed at once, the second on top of the first.
     // Work is taken eight items at a time, their kv heads one after the other (so neighbours in this
     // order read different pages at the same time), with the second round backwards: with `items`
     // sorted longest first a compute unit's first two are a long and a short one, and what follows
     // goes to whichever compute unit is free, longest first.
-    int s = blockIdx.x + gridDim.x * blockIdx.y;
-    const int total = gridDim.x * gridDim.y;
+    int s = blockIdx.x + N * blockIdx.y;
+    const int total = N * KV;
     if (s >= cus && s < 2 * cus) s = cus + (min(2 * cus, total) - 1 - s);
-    const int N = gridDim.x, first = s / (8 * KV) * 8, r = s % (8 * KV), here = min(8, N - first);
+    const int first = s / (8 * KV) * 8, r = s % (8 * KV), here = min(8, N - first);
     item = first + r % here;
     kvh = r / here;
   }
@@ -1267,7 +1275,7 @@ static int launch_decode_mfma(const void* q, const void* k_pages, const void* v_
   attn_decode_mfma_kernel<DCV, FRESHV, SEEV><<<grid, 256, shmem, stream>>>(                               \
       (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, items, positions, tok_row, block_tables, \
       table_width, (bf16*)out, part_m, part_l, part_acc, H, KV, bs, scale, sight, part_size, P,           \
-      compute_units(), share, FRESHV ? *fresh : none)
+      num_items, compute_units(), share, FRESHV ? *fresh : none)
 #define LAUNCH(DCV, FRESHV) LAUNCH3(DCV, FRESHV, 0)
 #define LAUNCH_PLAIN(DCV)                          \
   if (see == 2) LAUNCH3(DCV, 0, 2);                \
@@ -1443,14 +1451,16 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
     const int* __restrict__ tiles, const int* __restrict__ items, const int* __restrict__ positions,
     const int* __restrict__ tok_row, const int* __restrict__ block_tables, int table_width, float* __restrict__ out,
     float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int bs,
-    float scale, Sight sight, int subs, int part_size, int P) {
+    float scale, Sight sight, int subs, int part_size, int P, int N) {
   constexpr int D = 16 * DT, LD = D + 4;
   extern __shared__ float smem[];  // [4][16] m, [4][16] l, [4][16][LD] outputs
-  const int G = H / KV, kvh = blockIdx.y, part = blockIdx.z;
+  const int G = H / KV;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   int t0, count, row, pos0;
-  const int item = blockIdx.x;
+  // the kv heads change fastest: workgroups are dealt to the XCDs in turn, and every XCD has its share of every context
+  const int place = blockIdx.x + N * (blockIdx.y + KV * blockIdx.z), rest = place / KV;
+  const int part = rest / N, item = rest - part * N, kvh = (place - rest * KV + item) % KV;
   if (tiles) {
     const int per = 16 / G;  // tokens of a workgroup
     const int* tile = tiles + (size_t)(item / subs) * 4;
@@ -1574,9 +1584,9 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
       }
       out[((size_t)(t0 + c / G) * H + h) * D + d] = num / den;
     } else {
-      const size_t place = ((size_t)item * H + h) * P + part;
-      part_acc[place * D + d] = num;
-      if (d == 0) { part_m[place] = top; part_l[place] = den; }
+      const size_t o = ((size_t)item * H + h) * P + part;
+      part_acc[o * D + d] = num;
+      if (d == 0) { part_m[o] = top; part_l[o] = den; }
     }
   }
 }
@@ -1601,10 +1611,10 @@ extern "C" int as_attn_f32(const float* q, const float* k_pages, const float* v_
   const size_t lds = (128 + 4 * 16 * (D + 4)) * sizeof(float);
   if (D == 64)
     attn_f32_kernel<4><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width,
-                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P);
+                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P, blocks_of * subs);
   else
     attn_f32_kernel<8><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width,
-                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P);
+                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P, blocks_of * subs);
   if (P > 1) {
     const int rc = launch_status();
     if (rc != AS_OK) return rc;
