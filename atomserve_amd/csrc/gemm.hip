@@ -1014,7 +1014,9 @@ static int launch_tile(const void* a, const void* w, const void* wt, void* out, 
   else if (!gated && out_dtype == DT_BF16 && tiled && NS <= 4) {  // narrow tiles: what a plain product of few columns takes
     if constexpr (NS <= 4) TILE_GO(false, false, bf16, true);
   } else if (!gated && out_dtype == DT_BF16) TILE_GO(false, false, bf16, false);
-  else if (!gated && out_dtype == DT_F32) TILE_GO(false, false, float, false);
+  else if (!gated && out_dtype == DT_F32 && tiled && NS != 6) {  // the head
+    if constexpr (NS != 6) TILE_GO(false, false, float, true);
+  } else if (!gated && out_dtype == DT_F32) TILE_GO(false, false, float, false);
   else return AS_BAD_DTYPE;
 #undef TILE_GO
   return launch_status();

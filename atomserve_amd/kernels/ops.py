@@ -642,6 +642,10 @@ def gemm(a, w, out, choices=None) -> None:
         raise KernelError(f"gemm: unsupported output dtype {out.dtype}")
     if _few_rows(M, K, N, w=w if out.dtype == BF16 else None):  # fp32 results (the head): no tile product to prefer
         call("as_gemm_bf16_skinny", _ptr(a), _ptr(rows), _wave_ptr(w), _ptr(out), _DT[out.dtype], M, N, K, 0, _stream())
+        return
+    strips = _wide_tile_strips(M, N, K) if out.dtype == F32 and _wave_ptr(w) else 0
+    if strips:
+        call("as_gemm_bf16_tile", _ptr(a), _ptr(rows), _wave_ptr(w), _ptr(out), 0, _DT[F32], M, N, K, 0, 0, strips, _stream())
     else:
         (choices or SHARED).gemm(a, w, out, M, N, K)
 
@@ -889,6 +893,21 @@ def _tile_preferred(rows: int, k: int, n: int, w) -> bool:
     above 16 rows or a model wide enough (the narrower of k and n is the stream's width in all four
     products of a layer)."""
     return bool(_wave_ptr(w)) and _tile_rows(rows, k, BF16) and (rows > SKINNY_MAX_ROWS or min(k, n) >= TILE_FROM_9_MIN_WIDTH)
+
+
+WIDE_TILE_MAX_ROWS = 96
+
+
+def _wide_tile_strips(rows: int, n: int, k: int) -> int:
+    """Strips of 16 weight rows per workgroup of the tile kernel for a product with 32-bit results and outputs enough to
+    fill the GPU several times (the head), 0 where the library's product runs: 17 to 96 rows and K in whole chunks.  151,936
+    outputs at 33 to 64 rows: K = 1,024 68 us against 83 for the library's best of 16 and 89 for its first, which a step of an
+    untuned row count takes; K = 4,096 243 against 251 and 276; at 128 rows its best is the faster one (287 against 297).  Few rows
+    want narrow tiles (17 rows, K = 2,048: 2 strips 99 us, 4 strips 114; 64 rows 144, 134 and 8 strips 128)."""
+    if not SKINNY_MAX_ROWS < rows <= WIDE_TILE_MAX_ROWS or k % TILE_CHUNK or n % 16 or n * k * 2 > 0xF0000000:
+        return 0
+    strips = 2 if rows <= 24 else 4 if rows <= 32 or (k <= 1024 and rows <= 64) else 8
+    return strips if n >= 16 * strips * compute_units() else 0
 
 
 def _gated_tile_strips(rows: int, outputs: int) -> int:

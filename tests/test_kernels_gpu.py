@@ -328,6 +328,18 @@ def test_gemm_bf16(ops, M, N, K):
     assert torch.allclose(out32, ref, atol=math.sqrt(K) * 2.0**-8, rtol=2.0**-7)
 
 
+@pytest.mark.parametrize("M", [16, 17, 24, 25, 32, 33, 64, 65, 96, 97])
+@pytest.mark.parametrize("N,K", [(32768, 256), (32768, 1280), (32768 + 16, 512), (16384, 1024)])
+def test_head_product_of_many_rows(ops, M, N, K):
+    """Products with 32-bit results at every tile width and beyond the rows that the tiles take, weights with their copy: sums of
+    K terms in 32 bits of exact products, 2^-24 sqrt(K) of their sizes against the plain product."""
+    torch.manual_seed(62)
+    a, w = torch.randn(M, K, device=DEV).to(BF16), (torch.randn(N, K, device=DEV) / math.sqrt(K)).to(BF16)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.gemm(a, ops.Streamed(w), out)
+    assert (out.double() - a.double() @ w.double().T).abs().max() <= 16 * math.sqrt(K) * 2.0**-24
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 96, 64), (8, 1000, 96), (5, 1030, 4096), (16, 12288, 4096), (9, 700, 2048),
                                    (3, 40, 200), (16, 24, 8), (4, 520, 5120), (7, 264, 6144), (8, 128, 12288),
                                    (40, 300, 512), (32, 1030, 2048), (17, 264, 2048), (29, 128, 4096),
