@@ -406,42 +406,43 @@ __device__ __forceinline__ void load_gains8(const bf16* w, float* g) {
 
 // D / 32; FRESH 0: finished queries, 1: qkv with bf16 gains, 2: with fp32 gains; SEE 0: a window at most (nothing of the rest of
 // `sight` is read), 1: kept first tokens, chunks, a sink and fp32 outputs too, 2: also capped scores
-template <int DC, int FRESH, int SEE>
+template <int DC, int FRESH, int SEE, bool TURNED = false>
 __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ items, const int* __restrict__ positions, const int* __restrict__ tok_row,
     const int* __restrict__ block_tables, int table_width, bf16* __restrict__ out, float* __restrict__ part_m,
     float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int bs, float scale, Sight sight,
-    int part_size, int P, int N, int cus, int share, FreshQKV fresh) {
+    int part_size, int P, int cus, int share, FreshQKV fresh) {
   // share > 1: every `share` consecutive kv heads named here are one head of the pages (a group of more query heads
   // than a workgroup takes, cut into several); the pages then hold KV / share heads.
   constexpr int D = DC * 32, DT = DC * 2;  // DT: tiles of 16 output coordinates
   extern __shared__ float smem[];          // [4][16] m, [4][16] l, [4][D][G] acc
   __shared__ __align__(16) bf16 fresh_kv[2][256];  // FRESH: the new token's key and value
   const int G = H / KV;
-  int item = blockIdx.x, kvh = blockIdx.y, part = blockIdx.z;
-  if (P > 1 && N > 8) {
-    // Partitions of many tokens: workgroups are dealt to the XCDs in turn, and with the tokens changing fastest an XCD had every
-    // eighth context, so that the one with the longest worked alone at the end.  With the kv heads changing fastest each has its
-    // share of every context: 13 requests of 300 to 7,000 keys in a step of 16 rows 67 -> 47 us, 20 of 200 to 3,000 in one of
-    // 32 60 -> 41 (equal contexts: within 2 per cent).  Up to eight tokens an XCD has one, and its keys' pages to itself: left so.
-    const int s = blockIdx.x + N * (blockIdx.y + KV * blockIdx.z), rest = s / KV;
-    part = rest / N;
-    item = rest - part * N;
-    kvh = (s - rest * KV + item) % KV;
-  } else if (P == 1) {
+  int item = blockIdx.x, kvh = blockIdx.y;
+  const int part = blockIdx.z;
+  if (!TURNED && P == 1) {
     // Whole contexts, one workgroup each, of unequal length: two workgroups share a compute unit, and
     // the first two rounds of `cus` workgroups are placed at once, the second on top of the first.
     // Work is taken eight items at a time, their kv heads one after the other (so neighbours in this
     // order read different pages at the same time), with the second round backwards: with `items`
     // sorted longest first a compute unit's first two are a long and a short one, and what follows
     // goes to whichever compute unit is free, longest first.
-    int s = blockIdx.x + N * blockIdx.y;
-    const int total = N * KV;
+    int s = blockIdx.x + gridDim.x * blockIdx.y;
+    const int total = gridDim.x * gridDim.y;
     if (s >= cus && s < 2 * cus) s = cus + (min(2 * cus, total) - 1 - s);
-    const int first = s / (8 * KV) * 8, r = s % (8 * KV), here = min(8, N - first);
+    const int N = gridDim.x, first = s / (8 * KV) * 8, r = s % (8 * KV), here = min(8, N - first);
     item = first + r % here;
     kvh = r / here;
+  }
+  if constexpr (TURNED) {
+    // Partitions of many tokens come as a turned grid: workgroups are dealt to the XCDs in turn, and with the tokens changing
+    // fastest an XCD had every eighth context, so that the one with the longest worked alone at the end.  With the kv heads
+    // changing fastest each has its share of every context: 13 requests of 300 to 7,000 keys in a step of 16 rows 67 -> 46 us, 20
+    // of 200 to 3,000 in one of 32 60 -> 41 (equal contexts: within 2 per cent).  Up to eight tokens an XCD has one, and its keys'
+    // pages to itself: left so.  (An instance of its own: the same branch at run time costs whole contexts 3 to 5 per cent.)
+    item = blockIdx.y;
+    kvh = blockIdx.x;
   }
   const int t = items ? items[item] : item;  // null: every token, in order
   const int pos = positions[t];
@@ -1266,21 +1267,24 @@ static int launch_decode_mfma(const void* q, const void* k_pages, const void* v_
   if (D % 32 || D > 256 || G > 16 || bs % 16 || part_size % 32) return AS_BAD_SHAPE;
   if (fresh && D % 64) return AS_BAD_SHAPE;
   if (share < 1 || KV % share || (fresh && share != 1)) return AS_BAD_SHAPE;
-  dim3 grid(num_items, KV, P);
+  const bool turned = P > 1 && num_items > 8 && num_items <= 65535 && needed_sight(sight) == 0;
+  const dim3 grid = turned ? dim3(KV, num_items, P) : dim3(num_items, KV, P);
   const size_t shmem = sizeof(float) * (size_t)(128 + 4 * D * G);
   if (shmem + 1024 > (64u << 10)) return AS_BAD_SHAPE;  // wide heads in large groups: the general kernel's
   const FreshQKV none = {};
   const int see = needed_sight(sight);
-#define LAUNCH3(DCV, FRESHV, SEEV)                                                                        \
-  attn_decode_mfma_kernel<DCV, FRESHV, SEEV><<<grid, 256, shmem, stream>>>(                               \
+#define LAUNCH4(DCV, FRESHV, SEEV, TURNEDV)                                                               \
+  attn_decode_mfma_kernel<DCV, FRESHV, SEEV, TURNEDV><<<grid, 256, shmem, stream>>>(                      \
       (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, items, positions, tok_row, block_tables, \
       table_width, (bf16*)out, part_m, part_l, part_acc, H, KV, bs, scale, sight, part_size, P,           \
-      num_items, compute_units(), share, FRESHV ? *fresh : none)
-#define LAUNCH(DCV, FRESHV) LAUNCH3(DCV, FRESHV, 0)
+      compute_units(), share, FRESHV ? *fresh : none)
+#define LAUNCH(DCV, FRESHV)                       \
+  if (turned) LAUNCH4(DCV, FRESHV, 0, true);      \
+  else LAUNCH4(DCV, FRESHV, 0, false)
 #define LAUNCH_PLAIN(DCV)                          \
-  if (see == 2) LAUNCH3(DCV, 0, 2);                \
-  else if (see == 1) LAUNCH3(DCV, 0, 1);           \
-  else LAUNCH3(DCV, 0, 0)
+  if (see == 2) LAUNCH4(DCV, 0, 2, false);         \
+  else if (see == 1) LAUNCH4(DCV, 0, 1, false);    \
+  else LAUNCH(DCV, 0)
 #define LAUNCH_FRESH(FRESHV)            \
   switch (D / 64) {                     \
     case 1: LAUNCH(2, FRESHV); break;   \
@@ -1307,7 +1311,7 @@ static int launch_decode_mfma(const void* q, const void* k_pages, const void* v_
 #undef LAUNCH_FRESH
 #undef LAUNCH_PLAIN
 #undef LAUNCH
-#undef LAUNCH3
+#undef LAUNCH4
   if (hipGetLastError() != hipSuccess) return AS_LAUNCH_FAILED;
   if (P > 1) {
     attn_reduce_kernel<bf16><<<dim3(num_items, H), D <= 64 ? 64 : (D <= 128 ? 128 : 256), 0, stream>>>(

@@ -821,6 +821,25 @@ def test_whole_contexts_in_a_given_order(ops, N, KV):
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("N,KV", [(9, 8), (13, 3), (33, 1)])
+def test_partitions_of_more_than_eight_tokens(ops, N, KV):
+    """Above eight tokens the kv heads of partitioned contexts change fastest in the grid: each token's result has the bits that it
+    has in a call of eight, whatever the order of the tokens."""
+    H, D, bs = 2 * KV, 64, 16
+    torch.manual_seed(N)
+    lens = torch.randint(1, 700, (N,)).tolist()
+    q, k_pages, v_pages, tables, positions = paged_case(BF16, H, KV, D, bs, lens, seed=N, k_scale=3.0 / math.sqrt(D / 16))
+    rows, scale = i32(list(range(N))), D**-0.5
+    want = torch.full((N, H, D), float("nan"), dtype=BF16, device=DEV)
+    for first in range(0, N, 8):
+        ops.attn_single_query(q, k_pages, v_pages, rows[first : first + 8], positions, rows, tables, want, scale, 0, max(lens), 128)
+    assert not torch.isnan(want.float()).any()
+    for order in (None, torch.randperm(N).to(torch.int32).to(DEV)):
+        out = torch.full((N, H, D), float("nan"), dtype=BF16, device=DEV)
+        ops.attn_single_query(q, k_pages, v_pages, order, positions, rows, tables, out, scale, 0, max(lens), 128)
+        assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("H,KV,D,bs,gain,window", [
     (32, 8, 128, 16, BF16, 0), (6, 2, 64, 32, F32, 0), (14, 2, 192, 16, BF16, 40), (5, 5, 256, 16, BF16, 0),
     (16, 1, 128, 48, F32, 0), (8, 2, 128, 16, BF16, 1),
