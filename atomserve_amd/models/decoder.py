@@ -153,11 +153,14 @@ class DecoderModel:
         i = 0
         while i < len(p.run):
             if i == first and repeats.may_run_again(self, step, first, period):
-                before = delta
+                before, known = delta, set(step.shared)
                 with Launches() as made:
                     for k in range(period):
                         delta = self._run(first + k, x, delta, step)
                 done, delta = repeats.run_again(self, made, step, before, delta, first, period, count)
+                if done:  # what the stretch has left for the step's later runs lies where its repetitions have written theirs
+                    for key in step.shared.keys() - known:
+                        del step.shared[key]
                 i += period + done
                 continue
             if p.run[i].reenter:

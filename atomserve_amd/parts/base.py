@@ -75,8 +75,9 @@ class Part:
     def repeats(self, step: Any) -> bool:
         """Whether what `forward` launches in this step is what any other part of an equal spec launches, with that
         part's tensors (attributes that are tensors or `ops.Streamed`) and caches in place of this one's: every
-        launch goes through `kernels.lib.call`, and nothing is taken from, or left to, another layer's part.  A part says
-        so itself, for its own class only (a class derived from it may do more)."""
+        launch goes through `kernels.lib.call`, and nothing is taken from another layer's part.  What it leaves in
+        `step.shared` is the repetitions' to overwrite, and is dropped once they are made.  A part says so itself, for its own
+        class only (a class derived from it may do more)."""
         return False
 
     def weight_decls(self) -> dict:

@@ -1,0 +1,159 @@
+"""Layers launched from the list of a layer like them against the same layers run one by one, without a GPU: real models, plans
+and wrappers over entry points that compute nothing.  What a call would write is taken to be a name made of the entry point, its
+numbers and what it reads, so that two ways of launching a step agree on the names in the logits and in the caches exactly
+where every kernel reads the same things in the same width."""
+
+import functools
+import glob
+import hashlib
+import os
+import re
+
+import pytest
+import torch
+
+from atomserve_amd.cache.manager import CacheManager
+from atomserve_amd.config.registry import architecture_for
+from atomserve_amd.engine.batch import Row
+from atomserve_amd.engine.runner import ModelRunner
+from atomserve_amd.kernels import build, lib, ops
+from atomserve_amd.models.decoder import DecoderModel
+from atomserve_amd.weights import random_checkpoint
+from atomserve_amd.weights.loader import DictSource, bind_checkpoint
+
+
+def _signatures() -> dict:
+    """entry point -> per argument (its name, None for a number, else whether it is only read)."""
+    found = {}
+    for path in glob.glob(os.path.join(build.CSRC, "*.hip")):
+        with open(path) as f:
+            for name, args in re.findall(r'extern "C" int (as_\w+)\(([^)]*)\)', f.read()):
+                found[name] = [(a.split()[-1].lstrip("*"), ("const" in a) if "*" in a else None) for a in args.split(",") if a.strip()]
+    return found
+
+
+SIGNATURES = _signatures()
+# what a kernel changes in place, by the argument's name; an `out` is written whole unless a second kernel fills its other rows
+IN_PLACE = {"x", "state", "history", "k_pages", "v_pages"}
+IN_PLACE_OF = {"as_delta_prepare": {"qkv"}, "as_delta_chunks": {"out"}}
+
+
+class Names:
+    """Stands for the GPU: what lies at which address, as names."""
+
+    def __init__(self):
+        self.at, self.calls = {}, 0
+
+    def call(self, entry, *args):
+        if entry == "as_blas_plan":
+            return 1
+        read, written, numbers = [], [], []
+        self.calls += 1
+        for i, ((name, const), value) in enumerate(zip(SIGNATURES[entry], args, strict=True)):
+            if const is None:
+                numbers.append((name, value))
+            elif name in ("stream", "workspace"):
+                pass
+            elif not value:
+                read.append((name, None))
+            else:
+                if const or name in IN_PLACE or name in IN_PLACE_OF.get(entry, ()):
+                    read.append((name, self.at.get(value, "?")))
+                if not const:
+                    written.append((name, value))
+        made = hashlib.sha256(repr((entry, numbers, read)).encode()).hexdigest()
+        for name, address in written:
+            self.at[address] = (made, name)
+        return 0
+
+
+@pytest.fixture
+def gpu(monkeypatch):
+    """A GPU of names: `ops` takes tensors in host memory for its own, and no two tensors of a step share an address."""
+    names, kept, real = Names(), [], torch.empty
+
+    def check(t, name, dtype=None, shape=None):
+        assert isinstance(t, torch.Tensor) and t.is_contiguous(), name
+        assert dtype is None or t.dtype is dtype or (isinstance(dtype, tuple) and t.dtype in dtype), name
+        assert shape is None or (len(shape) == t.dim() and all(s in (None, d) for s, d in zip(shape, t.shape))), name
+
+    def empty(*args, **how):
+        kept.append(real(*args, **how))
+        return kept[-1]
+
+    entry = lambda name: functools.partial(names.call, name)  # noqa: E731
+    monkeypatch.setattr(lib, "entry", entry)
+    monkeypatch.setattr(ops, "entry", entry)
+    monkeypatch.setattr(ops, "_check", check)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_compute_units", 256)
+    monkeypatch.setattr(ops, "_library_workspace", lambda device: kept[0])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch, "empty", empty)
+    torch.empty(1)
+    return names
+
+
+def steps(gpu, raw, weights, dtype, listed, change=None):
+    """What a prompt, a portion beside it and short rows leave in the logits, the pages and the states, and the number of calls."""
+    arch = architecture_for(raw)
+    config = arch.parse_config(raw)
+    model = DecoderModel(arch.build_plan(config), dtype, "cpu")
+    bind_checkpoint(model, arch, config, DictSource(weights))
+    model.env.products.fix()
+    if change is not None:
+        change(model)
+    if not listed:
+        model.stretches = None
+    runner = ModelRunner(model, CacheManager(model.cache_requests(), 16, 64, 8))
+    gpu.at.clear()
+    for i, block in enumerate(model.blocks):
+        for part, p in block.parts().items():
+            for attr, v in vars(p).items():
+                for at, t in ((attr, v),) if isinstance(v, torch.Tensor) else ((attr, v.rows),) if isinstance(v, ops.Streamed) else ():
+                    gpu.at.setdefault(t.data_ptr(), ("weight", i, part, at.removesuffix("_weight"), t.dtype))
+    cached = []
+    for ident, (kind, _, _) in runner.manager.group_of_cache.items():
+        for t in runner.pools.pages(ident)[1:] if kind == "paged" else runner.pools.state_of(ident)[1:]:
+            cached.append(t.data_ptr())
+            gpu.at[cached[-1]] = ("cache", ident, len(cached))
+    held, out, calls, kept = {}, [], [], set(gpu.at)
+    for step in ([("a", 40)], [("a", 1), ("b", 90)], [("a", 3), ("c", 5)]):
+        rows = []
+        for rid, n in step:
+            cache, at = held.get(rid) or (runner.manager.new_request(), 0)
+            assert runner.manager.reserve(cache, at, n)
+            rows.append(Row(list(range(n)), at, cache.tables, [n - 1], cache.state_slot))
+            held[rid] = (cache, at + n)
+        gpu.at = {address: name for address, name in gpu.at.items() if address in kept}  # of the step before nothing else is left
+        before = gpu.calls
+        out.append(gpu.at[runner.step(rows).data_ptr()])
+        calls.append(gpu.calls - before)
+    return out, [gpu.at[address] for address in cached], calls
+
+
+def qwen3(layers):
+    return {"architectures": ["Qwen3ForCausalLM"], "vocab_size": 300, "hidden_size": 128, "intermediate_size": 256,
+            "num_hidden_layers": layers, "num_attention_heads": 4, "num_key_value_heads": 2, "head_dim": 64, "rms_norm_eps": 1e-6,
+            "rope_theta": 1e4, "tie_word_embeddings": False, "max_position_embeddings": 4096}  # fmt: skip
+
+
+def table_experts(layers, times):
+    delta = {"heads": 2, "kv_heads": 1, "dim": 64, "vdim": 64, "conv": 3}
+    moe = {"kind": "moe", "expert": {"ff": 64}, "router": {"experts": 4, "top": 2}}
+    raw = {"architecture": "Dozusun", "vocab": 300, "width": 128, "norm": {"eps": 1e-6},
+           "layers": [{"type": "delta", "mixer": delta, "mlp": moe}] * layers}  # fmt: skip
+    return raw if times == 1 else dict(raw, loop={"start": 0, "stop": layers, "times": times})
+
+
+def checkpoint(raw, dtype):
+    arch = architecture_for(raw)
+    return random_checkpoint(arch, arch.parse_config(raw), seed=3, dtype=dtype, device="cpu", std=0.05)
+
+
+@pytest.mark.parametrize("layers,times", [(4, 1), (2, 2), (3, 2), (2, 3), (3, 3), (5, 2)])
+def test_looped_layers_choose_experts_by_their_own_tables(gpu, layers, times):
+    """A layer that comes round again after its stretch has been repeated finds no other layer's routes under its table."""
+    raw = table_experts(layers, times)
+    weights = checkpoint(raw, torch.float32)
+    assert steps(gpu, raw, weights, torch.float32, True)[:2] == steps(gpu, raw, weights, torch.float32, False)[:2]

@@ -33,7 +33,9 @@ def dozusun(kinds):
 
 CASES = {"qwen3-6": (qwen3(6), (1, 1, 3)), "qwen3-3": (qwen3(3), None), "qwen3-5": (qwen3(5, 512), (1, 1, 2)),
          "dozusun-pairs": (dozusun("pdpdpdpd"), (1, 2, 2)), "dozusun-alone": (dozusun("nnnn"), (1, 1, 2)),
-         "dozusun-mixed": (dozusun("pddnpd"), (1, 1, 1))}  # fmt: skip
+         "dozusun-mixed": (dozusun("pddnpd"), (1, 1, 1)),
+         "dozusun-looped": (dict(dozusun("ddd"), loop={"start": 0, "stop": 3, "times": 2}), (1, 1, 2)),
+         "dozusun-looped-twice": (dict(dozusun("ddd"), loop={"start": 0, "stop": 3, "times": 3}), (1, 2, 2))}  # fmt: skip
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
