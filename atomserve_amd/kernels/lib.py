@@ -160,7 +160,8 @@ def call(name: str, *args) -> None:
 class Launches:
     """The launches that a piece of code makes (`with Launches() as made:`), to be made again with other
     addresses: `made.aim(sources)`, then `made.again(targets)` for as many lists of targets as there are: wherever a
-    call was given sources[i], it is given targets[i].  The tensors that the calls read and wrote are held as long as this
+    call was given sources[i], it is given targets[i].  All else in the calls stays: who makes them again answers for it that
+    what lies at targets[i] has the type, the shape and the layout of what lies at sources[i].  The tensors that the calls read and wrote are held as long as this
     object lives, so that nobody else is given their memory between two repetitions."""
 
     def __enter__(self):
@@ -176,16 +177,17 @@ class Launches:
         return False
 
     def aim(self, sources: list) -> None:
-        self.sources = sources
         place = {address: i for i, address in enumerate(sources) if address}
         self.patched = [(name, fn, list(args), [(at, place[v]) for at, v in enumerate(args) if type(v) is int and v in place])
                         for name, fn, args in self.calls]  # fmt: skip
+        met = {i for *_, patches in self.patched for _, i in patches}
+        # sources with the address of one that the calls were given: which of them it was is not known
+        self.same = [(i, place[a]) for i, a in enumerate(sources) if a and place[a] in met and place[a] != i]
+        self.met = sorted(met.union(i for i, _ in self.same))
 
     def fits(self, targets: list) -> bool:
-        """Whether `targets` can stand for the sources: as many, none where there was none, one address for one address."""
-        known = {}
-        return len(targets) == len(self.sources) and all(
-            bool(a) == bool(b) and (not a or known.setdefault(a, b) == b) for a, b in zip(self.sources, targets))  # fmt: skip
+        """Whether `targets` (of use: those at the places `met`) can stand for the sources: one address for one address."""
+        return all(targets[i] == targets[j] for i, j in self.same)
 
     def again(self, targets: list) -> None:
         for name, fn, args, patches in self.patched:

@@ -61,44 +61,102 @@ def stretches(plan, blocks) -> tuple:
     return best
 
 
-def _view_addresses(view, into: list) -> None:
-    """The addresses of a cache view's tensors, or of a dict of views, in an order that equal kinds share."""
+def _view_parts(view, into: list) -> None:
+    """What a cache view or a dict of views holds, in an order that equal kinds share: tensors, and numbers as they are."""
     if isinstance(view, dict):
         for name in sorted(view):
-            _view_addresses(view[name], into)
+            _view_parts(view[name], into)
     elif view is not None:
-        for name in type(view).__slots__:
-            found = getattr(view, name)
-            if isinstance(found, torch.Tensor):
-                into.append(found.data_ptr())
+        into.extend([getattr(view, name) for name in type(view).__slots__])
 
 
-def _own_names(model, first: int, period: int) -> list:
-    """For each run of the stretch that starts at run `first` the (part, attribute, has a copy) that are a layer's own
-    tensors: all of its parts' attributes that are tensors or `ops.Streamed`."""
-    return [[(name, attr, isinstance(v, ops.Streamed)) for name, part in model.blocks[model.plan.run[first + k].layer].parts().items()
-             for attr, v in sorted(vars(part).items()) if isinstance(v, (torch.Tensor, ops.Streamed))] for k in range(period)]  # fmt: skip
+class _Own:
+    """What belongs to a stretch and takes the place of the written-down one's: its layers' tensors (all of their parts'
+    attributes that are tensors or `ops.Streamed`, a matrix and its copy), its caches and the gains of the norms that follow its
+    layers (which their last products may prepare).
 
+    Beside its address a launch carries types, shapes and layouts that the wrappers have checked for the written-down stretch
+    alone, and gains may be stored in 32 bits in one layer and in 16 in another (a checkpoint says so tensor by tensor): every
+    tensor that the launches read has to be of the same kind in every stretch, and what one stretch does without, all do."""
 
-def _own_addresses(model, step, names: list, start: int) -> list:
-    """The addresses that belong to the stretch that starts at run `start`: its layers' tensors, its caches and the gains of
-    the norms that follow its layers (which their last products may prepare)."""
-    plan, found = model.plan, []
-    for k, wanted in enumerate(names):
-        i = start + k
-        parts = model.blocks[plan.run[i].layer].parts()
-        for name, attr, streamed in wanted:
-            v = getattr(parts[name], attr)
-            if streamed:
-                found.append(v.rows.data_ptr())
-                found.append(0 if v.wave is None else v.wave.data_ptr())
+    def __init__(self, model, step, first: int, period: int):
+        self.model, self.step, self.tensors = model, step, []
+        self.layers = []  # per layer: its class, and its parts' attributes as (part, class, [(attribute, whether it has a copy)])
+        for k in range(period):
+            block, names = model.blocks[model.plan.run[first + k].layer], []
+            for name, part in block.parts().items():
+                wanted = [(attr, isinstance(v, ops.Streamed)) for attr, v in vars(part).items()
+                          if v is None or isinstance(v, (torch.Tensor, ops.Streamed))]  # fmt: skip
+                names.append((name, type(part), wanted))
+            self.layers.append((type(block), names))
+        self.tensors = self.of(first)
+
+    def of(self, start: int):
+        """Tensors, numbers of the caches and None, of the stretch that starts at run `start`; None where a layer is of another
+        class, something stands in place of its methods, or a plain tensor for a matrix with a copy or the other way round."""
+        model, plan, found = self.model, self.model.plan, []
+        for i, (kind, names) in enumerate(self.layers, start):
+            block = model.blocks[plan.run[i].layer]
+            if type(block) is not kind or "forward" in vars(block):
+                return None
+            parts = block.parts()
+            for name, kind, wanted in names:
+                have = vars(parts[name])
+                if type(parts[name]) is not kind or "forward" in have:
+                    return None
+                for attr, streamed in wanted:
+                    v = have.get(attr)
+                    if streamed:
+                        if type(v) is not ops.Streamed:
+                            return None
+                        found.append(v.rows)
+                        found.append(v.wave)
+                    else:
+                        found.append(v)
+            _view_parts(self.step.cache_view(plan.cache_id(i), True), found)
+            after = model.blocks[plan.run[i + 1].layer].first_norm() if i + 1 < len(plan.run) else None
+            if after is not None:
+                found.extend([v for _, v in sorted(vars(after).items()) if isinstance(v, torch.Tensor)])
+        return found
+
+    def addresses(self) -> list:
+        return [v.data_ptr() if isinstance(v, torch.Tensor) else 0 for v in self.tensors]
+
+    def read(self, places: list) -> None:
+        """The places whose tensors the launches read."""
+        at, self.met, self.alike = {}, [], []
+        for i in places:
+            v = self.tensors[i]
+            if at.setdefault(id(v), i) == i:
+                self.met.append((i, v.dtype, v.shape, v.is_contiguous()))
             else:
-                found.append(v.data_ptr())
-        _view_addresses(step.cache_view(plan.cache_id(i), True), found)
-        after = model.blocks[plan.run[i + 1].layer].first_norm() if i + 1 < len(plan.run) else None
-        if after is not None:
-            found.extend(v.data_ptr() for _, v in sorted(vars(after).items()) if isinstance(v, torch.Tensor))
-    return found
+                self.alike.append((i, at[id(v)]))  # one tensor under two names
+        places = set(places)
+        self.plain = [(i, v) for i, v in enumerate(self.tensors) if not isinstance(v, torch.Tensor)]
+        self.unread = [i for i, v in enumerate(self.tensors) if isinstance(v, torch.Tensor) and i not in places]
+
+    def targets(self, start: int):
+        """The addresses of the stretch that starts at run `start` where the launches read them, or None if it is of another kind."""
+        own = self.of(start)
+        if own is None or len(own) != len(self.tensors):
+            return None
+        found = [0] * len(own)
+        for i, dtype, shape, contiguous in self.met:
+            v = own[i]
+            if v is None or v.dtype is not dtype or v.shape != shape or v.is_contiguous() != contiguous:
+                return None
+            found[i] = v.data_ptr()
+        for i, j in self.alike:
+            if own[i] is not own[j]:
+                return None
+            found[i] = found[j]
+        for i, v in self.plain:
+            if own[i] is not v and (isinstance(own[i], torch.Tensor) or own[i] != v):
+                return None
+        for i in self.unread:
+            if own[i] is None:
+                return None
+        return found
 
 
 def _left(delta):
@@ -123,15 +181,15 @@ def run_again(model, made: Launches, step, before, after, first: int, period: in
         return 0, after
     turns = [[t.data_ptr() for t in taken], [t.data_ptr() for t in given]]
 
-    names = _own_names(model, first, period)
-    made.aim(_own_addresses(model, step, names, first) + turns[0] + turns[1])
+    own = _Own(model, step, first, period)
+    made.aim(own.addresses() + turns[0] + turns[1])
+    own.read([i for i in made.met if i < len(own.tensors)])
     done = 0
     for _ in range(count):
-        start = first + done + period
-        blocks = [model.blocks[model.plan.run[start + k].layer] for k in range(period)]
-        if not all(_plain(b) for b in blocks):
+        targets = own.targets(first + done + period)
+        if targets is None:
             break
-        targets = _own_addresses(model, step, names, start) + turns[1] + turns[0]
+        targets += turns[1] + turns[0]
         if not made.fits(targets):
             break
         made.again(targets)

@@ -88,6 +88,7 @@ def gpu(monkeypatch):
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     monkeypatch.setattr(ops, "_compute_units", 256)
     monkeypatch.setattr(ops, "_library_workspace", lambda device: kept[0])
+    monkeypatch.setattr(ops.Streamed, "possible", staticmethod(lambda w: w.dtype == torch.bfloat16 and w.shape[0] % 16 == 0 and w.shape[1] % 64 == 0))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(torch, "empty", empty)
     torch.empty(1)
@@ -110,8 +111,9 @@ def steps(gpu, raw, weights, dtype, listed, change=None):
     for i, block in enumerate(model.blocks):
         for part, p in block.parts().items():
             for attr, v in vars(p).items():
-                for at, t in ((attr, v),) if isinstance(v, torch.Tensor) else ((attr, v.rows),) if isinstance(v, ops.Streamed) else ():
-                    gpu.at.setdefault(t.data_ptr(), ("weight", i, part, at.removesuffix("_weight"), t.dtype))
+                for kind, t in (("rows", v),) if isinstance(v, torch.Tensor) else (("rows", v.rows), ("wave", v.wave)) if isinstance(v, ops.Streamed) else ():
+                    if t is not None:
+                        gpu.at.setdefault(t.data_ptr(), ("weight", i, part, attr.removesuffix("_weight"), kind, t.dtype))
     cached = []
     for ident, (kind, _, _) in runner.manager.group_of_cache.items():
         for t in runner.pools.pages(ident)[1:] if kind == "paged" else runner.pools.state_of(ident)[1:]:
@@ -157,3 +159,72 @@ def test_looped_layers_choose_experts_by_their_own_tables(gpu, layers, times):
     raw = table_experts(layers, times)
     weights = checkpoint(raw, torch.float32)
     assert steps(gpu, raw, weights, torch.float32, True)[:2] == steps(gpu, raw, weights, torch.float32, False)[:2]
+
+
+QK, NORMS = ("self_attn.q_norm", "self_attn.k_norm"), ("input_layernorm", "post_attention_layernorm")
+WIDER = {"two layers' norms": (NORMS, (3, 4)), "the last layer's norms": (NORMS, (5,)), "one layer's q and k gains": (QK, (2,)),
+         "all q and k gains but one layer's": (QK, (0, 1, 3, 4, 5)), "every second layer's gains": (QK + NORMS, (0, 2, 4)),
+         "the first layer's gains": (QK + NORMS, (0,)), "the written-down layer's gains": (QK + NORMS, (1,))}  # fmt: skip
+
+
+@pytest.mark.parametrize("which", sorted(WIDER))
+def test_gains_are_read_in_the_width_they_are_stored_in(gpu, which):
+    """A 16-bit model whose checkpoint keeps the gains of some layers in 32 bits: every layer's are read in their own width."""
+    raw = qwen3(6)
+    weights = checkpoint(raw, torch.bfloat16)
+    names, layers = WIDER[which]
+    for i in layers:
+        for name in names:
+            weights[f"model.layers.{i}.{name}.weight"] = weights[f"model.layers.{i}.{name}.weight"].float()
+    assert steps(gpu, raw, weights, torch.bfloat16, True) == steps(gpu, raw, weights, torch.bfloat16, False)
+
+
+def _without_copy(model):
+    model.blocks[3].ffn.down.wave = None
+
+
+def _plain_matrix(model):
+    model.blocks[4].mixer.o = model.blocks[4].mixer.o_weight
+
+
+def _wider_gain(model):
+    model.blocks[5].ffn_norm.weight = model.blocks[5].ffn_norm.weight.float()
+
+
+def _another_shape(model):  # what the wrappers refuse for the layer alone
+    model.blocks[4].mixer_norm.weight = torch.ones(64, dtype=torch.bfloat16)
+
+
+def _another_layout(model):
+    model.blocks[4].mixer_norm.weight = torch.ones(256, dtype=torch.bfloat16)[::2]
+
+
+@pytest.mark.parametrize("change", [_without_copy, _plain_matrix, _wider_gain])
+def test_layers_that_were_changed_run_themselves(gpu, change):
+    """A matrix without its copy, a plain tensor in a matrix's place, a gain of another width: what a layer alone would launch."""
+    raw = qwen3(6)
+    weights = checkpoint(raw, torch.bfloat16)
+    assert steps(gpu, raw, weights, torch.bfloat16, True, change) == steps(gpu, raw, weights, torch.bfloat16, False, change)
+
+
+@pytest.mark.parametrize("change", [_another_shape, _another_layout])
+@pytest.mark.parametrize("listed", [True, False])
+def test_what_the_wrappers_refuse_stays_refused(gpu, change, listed):
+    raw = qwen3(6)
+    with pytest.raises(AssertionError, match="weight"):
+        steps(gpu, raw, checkpoint(raw, torch.bfloat16), torch.bfloat16, listed, change)
+
+
+def test_a_list_is_made_again_only_for_what_it_fits(gpu):
+    """Layers of equal sizes are launched from the list: as many calls, and the wrappers' checks run for the first layers alone."""
+    raw, checked = qwen3(6), []
+    weights = checkpoint(raw, torch.bfloat16)
+    real = ops._check
+    ops._check = lambda t, name, dtype=None, shape=None: (checked.append(name), real(t, name, dtype, shape))
+    try:
+        listed = steps(gpu, raw, weights, torch.bfloat16, True)
+        few = len(checked)
+        alone = steps(gpu, raw, weights, torch.bfloat16, False)
+    finally:
+        ops._check = real
+    assert listed == alone and few < 0.7 * (len(checked) - few)

@@ -38,13 +38,33 @@ CASES = {"qwen3-6": (qwen3(6), (1, 1, 3)), "qwen3-3": (qwen3(3), None), "qwen3-5
          "dozusun-looped-twice": (dict(dozusun("ddd"), loop={"start": 0, "stop": 3, "times": 3}), (1, 2, 2))}  # fmt: skip
 
 
+# whose gains are stored in the other width: (names, layers)
+WIDER = {"two layers' norms": (("input_layernorm", "post_attention_layernorm"), (3, 4)), "one layer's q and k gains": (("self_attn.q_norm", "self_attn.k_norm"), (2,)),
+         "all q and k gains but one layer's": (("self_attn.q_norm", "self_attn.k_norm"), (0, 1, 3, 4, 5))}  # fmt: skip
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_layers_from_a_list_are_the_layers(name, dtype):
-    raw, covered = CASES[name]
+    check_layers(*CASES[name], dtype)
+
+
+@pytest.mark.parametrize("which", sorted(WIDER))
+def test_layers_with_gains_of_other_widths_are_the_layers(which):
+    def change(weights):
+        names, layers = WIDER[which]
+        for name in [f"model.layers.{i}.{n}.weight" for i in layers for n in names]:
+            weights[name] = weights[name].float()
+
+    check_layers(*CASES["qwen3-6"], torch.bfloat16, change)
+
+
+def check_layers(raw, covered, dtype, change=None):
     arch = architecture_for(raw)
     config = arch.parse_config(raw)
     weights = random_checkpoint(arch, config, seed=3, dtype=dtype, device="cuda:0", std=0.05)
+    if change is not None:
+        change(weights)
 
     def steps(listed: bool):
         model = DecoderModel(arch.build_plan(config), dtype, "cuda:0")
