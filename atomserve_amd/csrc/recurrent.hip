@@ -535,15 +535,18 @@ extern "C" int as_delta_scan(const float* qkv, int C, int G, int dim, int H, int
 // delta_pairs (a workgroup a chunk and head, all side by side) makes (I + A)^-1 diag(beta) and D (Q K^T); delta_chunks (a
 // workgroup a row, head and 16 columns of the state) walks the chunks.  All of it in 32 bits: products by
 // v_mfma_f32_16x16x4_f32, the decays by multiplication in the order of the scan (no logarithms, so none is lost to a
-// strong decay before a weak one).  A token whose key, query, value, beta or decay is not finite ends its chunk: the tokens before
-// it are computed without it, its own outputs and all that follow are NaN.
+// strong decay before a weak one).  A chunk whose updates u are not all finite (a number that is not came in, or one grew beyond
+// 32 bits), or that has a query that is not, is walked token by token by one wave instead, as the scan does, from the state before
+// it: 0 times such a number is NaN, and in the matrix form it would reach the tokens before it, where the scan keeps a query's
+// to its own token and a value's to its column of the state.
 // Bound by the chain of a chunk (128 matrix instructions of a workgroup's last wave, which take 1.9 us, and three barriers: 4.1 us a
 // chunk) and by the fill of the GPU (rows x heads x column groups workgroups).  One prompt of 1,500 tokens, 16 heads of 128 x 128:
-// 26 + 99 us; token by token (0.4 us a token, the scan above) 618.  The triangle inverted by one wave, a column to a lane from the top down, took
-// the first kernel 33 us.
+// 25 + 98 us; token by token (0.4 us a token, the scan above) 619; with every chunk walked by token (its values NaN from the first
+// on) 1,360.  The triangle inverted by one wave, a column to a lane from the top down, took the first kernel 33 us.  The state
+// before a chunk stays in LDS for that walk: kept in registers, heads of 128 exceed what two workgroups on a compute unit leave.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 #define DC 64                            // tokens of a chunk
-#define DC_SCRATCH (2 * DC * DC + 3 * DC)  // floats per chunk and head: the inverse, the pairs, P, D[64, :], the first bad token
+#define DC_SCRATCH (2 * DC * DC + 3 * DC)  // floats per chunk and head: the inverse, the pairs, P, D[64, :], whether a query is not finite
 
 __device__ __forceinline__ int delta_chunks_of(int len, int most) { return len > most ? (len + DC - 1) / DC : 0; }
 __device__ __forceinline__ bool finite4(floatx4 v) {
@@ -562,7 +565,6 @@ __global__ __launch_bounds__(256) void delta_pairs_kernel(const float* __restric
   __shared__ __attribute__((aligned(16))) float sg[DC], sb[DC];
   __shared__ floatx4 inv[4][4][64];
   __shared__ __attribute__((aligned(16))) float rows[4][16 * 20];
-  __shared__ int s_bad;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4, h = blockIdx.y, g = h / (H / G);
   int chunk = blockIdx.x, r = 0;
@@ -575,8 +577,6 @@ __global__ __launch_bounds__(256) void delta_pairs_kernel(const float* __restric
   const int first = row_first[r] + chunk * DC, n = min(DC, row_len[r] - chunk * DC);
   float* mine = scratch + ((size_t)blockIdx.x * H + h) * DC_SCRATCH;
   const int q_col = g * dim, k_col = (G + g) * dim, v_col = 2 * G * dim + h * vdim;
-  if (tid == 0) s_bad = DC;
-  __syncthreads();
   auto row_of = [&](int tile, int col) { return qkv + (size_t)(first + min(tile * 16 + lr, n - 1)) * C + col + lg * 4; };
   floatx4 q[DT], kk[4][DT];  // this wave's 16 queries, and the keys of every token up to its own: all asked for at once
   {
@@ -593,47 +593,14 @@ __global__ __launch_bounds__(256) void delta_pairs_kernel(const float* __restric
     for (int i = 0; i < DT; ++i) q[i] = *reinterpret_cast<const floatx4*>(qp + i * 16);
     if (tid < DC) {
       const size_t at = (size_t)(first + min(tid, n - 1)) * H + h;
-      const float bt = beta[at], gt = decay[at];
-      if (tid < n && !finite4(floatx4{bt, gt, 0.f, 0.f})) atomicMin(&s_bad, tid);
-      sg[tid] = tid < n ? gt : 1.f;
-      sb[tid] = tid < n ? bt : 0.f;
+      sg[tid] = tid < n ? decay[at] : 1.f;
+      sb[tid] = tid < n ? beta[at] : 0.f;
     }
-    const int quads = vdim / 4, pieces = n * quads;
-    for (int x0 = tid; x0 < pieces; x0 += 256 * 8) {  // the values are only looked at here
-      floatx4 v[8];
-#pragma unroll
-      for (int y = 0; y < 8; ++y) {
-        const int x = min(x0 + y * 256, pieces - 1);
-        v[y] = *reinterpret_cast<const floatx4*>(qkv + (size_t)(first + x / quads) * C + v_col + x % quads * 4);
-      }
-#pragma unroll
-      for (int y = 0; y < 8; ++y)
-        if (!finite4(v[y])) atomicMin(&s_bad, min(x0 + y * 256, pieces - 1) / quads);
-    }
-    bool good = true;
-#pragma unroll
-    for (int i = 0; i < DT; ++i) {
-      good = good && finite4(q[i]);
-      if (wave == 0) good = good && finite4(kk[0][i]);
-      if (wave == 1) good = good && finite4(kk[1][i]);
-      if (wave == 2) good = good && finite4(kk[2][i]);
-      if (wave == 3) good = good && finite4(kk[3][i]);
-    }
-    if (!good && wave * 16 + lr < n) atomicMin(&s_bad, wave * 16 + lr);
   }
-  __syncthreads();
-  const int bad = s_bad;  // tokens from here on count as none
-  if (bad < DC) {
-    if (tid < DC && tid >= bad) { sg[tid] = 1.f; sb[tid] = 0.f; }
+  bool finite = true;
 #pragma unroll
-    for (int i = 0; i < DT; ++i) {
-      if (wave * 16 + lr >= bad) q[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (j * 16 + lr >= bad) kk[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-    __syncthreads();
-  }
+  for (int i = 0; i < DT; ++i) finite = finite && finite4(q[i]);
+  const int by_token = __syncthreads_or(!finite);
   {  // column `lane` of D: this wave keeps its 16 rows
     float cur = 0.f;
     for (int t4 = 0; t4 < DC; t4 += 16) {
@@ -738,12 +705,13 @@ __global__ __launch_bounds__(256) void delta_pairs_kernel(const float* __restric
   if (wave == 0) {
     mine[2 * DC * DC + lane] = D[lane * LDD] * sg[0];
     mine[2 * DC * DC + DC + lane] = D[(DC - 1) * LDD + lane];
-    if (lane == 0) reinterpret_cast<int*>(mine)[2 * DC * DC + 2 * DC] = bad;
+    if (lane == 0) reinterpret_cast<int*>(mine)[2 * DC * DC + 2 * DC] = by_token;
   }
 }
 
 template <int DT>
 __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restrict__ qkv, int C, int G, int H, int vdim,
+                                                           const float* __restrict__ beta, const float* __restrict__ decay,
                                                            float* __restrict__ state, const int* __restrict__ row_first,
                                                            const int* __restrict__ row_len, const int* __restrict__ row_start,
                                                            const int* __restrict__ row_slots, int writes, int most,
@@ -751,7 +719,7 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
                                                            float* __restrict__ out) {
   constexpr int dim = 16 * DT, LK = dim + 4;
   __shared__ __attribute__((aligned(16))) float keys[DC * LK];
-  __shared__ floatx4 sy[4 * 64], su[4 * 64], se[4 * 64], ss[DT * 64];
+  __shared__ floatx4 sy[4 * 64], su[4 * 64], se[4 * 64], ss[2][DT * 64];  // ss: the states before and after a chunk
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   // a head's column groups side by side on one XCD (workgroups are dealt to the eight in turn): they read the same
@@ -774,9 +742,9 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
   for (int i = 0; i < DT; ++i) {
 #pragma unroll
     for (int x = 0; x < 4; ++x) S[i][x] = carried ? kept[(size_t)(16 * i + 4 * lg + x) * vdim] : 0.f;
-    if (wave == 0) ss[i * 64 + lane] = S[i];
+    if (wave == 0) ss[0][i * 64 + lane] = S[i];
   }
-  int bad = DC;
+  int by_token = 0;
   float last_P = 1.f;
   auto token = [&](int n, int t) { return qkv + (size_t)(first + min(n * DC + t, len - 1)) * C; };
   auto load_rows = [&](int n) {
@@ -801,16 +769,12 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
     P = *reinterpret_cast<const floatx4*>(mine + 2 * DC * DC + wave * 16 + lg * 4);
     E = *reinterpret_cast<const floatx4*>(mine + 2 * DC * DC + DC + wave * 16 + lg * 4);
     last_P = mine[2 * DC * DC + DC - 1];
-    bad = reinterpret_cast<const int*>(mine)[2 * DC * DC + 2 * DC];
+    by_token = reinterpret_cast<const int*>(mine)[2 * DC * DC + 2 * DC];
   };
   load_rows(0);
   load_rest(0);
   for (int n = 0; n < chunks; ++n) {
-    const int limit = bad;
-    if (limit < DC && wave * 16 + lr >= limit) {
-#pragma unroll
-      for (int i = 0; i < DT; ++i) kf[i] = qf[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
+    floatx4 *const old = ss[n & 1], *const now = ss[(n + 1) & 1];
 #pragma unroll
     for (int i = 0; i < DT; ++i) *reinterpret_cast<floatx4*>(keys + (wave * 16 + lr) * LK + i * 16 + lg * 4) = kf[i];
     floatx4 xk = floatx4{0.f, 0.f, 0.f, 0.f}, xq = xk;
@@ -823,12 +787,7 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
       }
     const int ahead = min(n + 1, chunks - 1);
     load_rows(ahead);
-    floatx4 y = vv - P * xk;
-    if (limit < DC) {
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-        if (wave * 16 + lg * 4 + x >= limit) y[x] = 0.f;
-    }
+    const floatx4 y = vv - P * xk;
     sy[wave * 64 + lane] = y;
     __syncthreads();
     floatx4 u = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -846,20 +805,22 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
     floatx4 o = P * xq;
     // the state first (the next chunk waits for it), then the outputs
     floatx4 next[DT / 4];
+    bool finite = true;
 #pragma unroll
     for (int m = 0; m < DT / 4; ++m) {
       const int i = wave * (DT / 4) + m;
-      next[m] = ss[i * 64 + lane] * last_P;
+      next[m] = old[i * 64 + lane] * last_P;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const floatx4 uj = se[j * 64 + lane];
+        if (m == 0) finite = finite && finite4(uj);
 #pragma unroll
         for (int x = 0; x < 4; ++x)
           next[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(keys[(j * 16 + lg * 4 + x) * LK + i * 16 + lr], uj[x], next[m], 0, 0, 0);
       }
-      if (limit < DC) next[m] = floatx4{__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
-      ss[i * 64 + lane] = next[m];
+      now[i * 64 + lane] = next[m];
     }
+    const bool lost = by_token || __any(!finite);  // the same in all four waves: each has looked at every update
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       if (j <= wave) {
@@ -872,11 +833,51 @@ __global__ __launch_bounds__(256) void delta_chunks_kernel(const float* __restri
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
       const int t = wave * 16 + lg * 4 + x;
-      if (n * DC + t < len) out[((size_t)(first + n * DC + t) * H + h) * vdim + c0 + lr] = t < limit ? o[x] : __builtin_nanf("");
+      if (!lost && n * DC + t < len) out[((size_t)(first + n * DC + t) * H + h) * vdim + c0 + lr] = o[x];
     }
     __syncthreads();
+    if (lost) {
+      if (wave == 0) {
 #pragma unroll
-    for (int i = 0; i < DT; ++i) S[i] = ss[i * 64 + lane];
+        for (int i = 0; i < DT; ++i) S[i] = old[i * 64 + lane];
+        for (int t = 0; t < min(DC, len - n * DC); ++t) {
+          const size_t at = (size_t)(first + n * DC + t) * H + h;
+          const float* row = qkv + (size_t)(first + n * DC + t) * C;
+          const float g_now = decay[at], b_now = beta[at], v_now = row[v_col];
+          float p = 0.f, r = 0.f, kq = 0.f;
+#pragma unroll
+          for (int i = 0; i < DT; ++i) {
+            const floatx4 k = *reinterpret_cast<const floatx4*>(keys + t * LK + i * 16 + lg * 4);
+            const floatx4 q = *reinterpret_cast<const floatx4*>(row + q_col + i * 16 + lg * 4);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              p = fmaf(S[i][x], k[x], p);
+              r = fmaf(S[i][x], q[x], r);
+              kq = fmaf(k[x], q[x], kq);
+            }
+          }
+          p += __shfl_xor(p, 16, WAVE);
+          r += __shfl_xor(r, 16, WAVE);
+          kq += __shfl_xor(kq, 16, WAVE);
+          p += __shfl_xor(p, 32, WAVE);
+          r += __shfl_xor(r, 32, WAVE);
+          kq += __shfl_xor(kq, 32, WAVE);
+          const float u_now = b_now * (v_now - g_now * p);
+#pragma unroll
+          for (int i = 0; i < DT; ++i) {
+            const floatx4 k = *reinterpret_cast<const floatx4*>(keys + t * LK + i * 16 + lg * 4);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) S[i][x] = fmaf(k[x], u_now, g_now * S[i][x]);
+          }
+          if (lg == 0) out[at * vdim + c0 + lr] = fmaf(g_now, r, u_now * kq);
+        }
+#pragma unroll
+        for (int i = 0; i < DT; ++i) now[i * 64 + lane] = S[i];
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < DT; ++i) S[i] = now[i * 64 + lane];
   }
   if (writes && slot >= 0 && wave == 0) {
 #pragma unroll
@@ -903,7 +904,7 @@ extern "C" int as_delta_chunks(const float* qkv, int C, int G, int dim, int H, i
   do {                                                                                                                         \
     delta_pairs_kernel<DT><<<dim3(most_chunks, H), 256, 0, stream>>>(qkv, C, G, H, vdim, beta, decay, row_first, row_len,      \
                                                                      num_rows, most, scratch);                                 \
-    delta_chunks_kernel<DT><<<per_xcd * 8, 256, 0, stream>>>(qkv, C, G, H, vdim, state, row_first, row_len, row_start,         \
+    delta_chunks_kernel<DT><<<per_xcd * 8, 256, 0, stream>>>(qkv, C, G, H, vdim, beta, decay, state, row_first, row_len, row_start,         \
                                                              row_slots, writes, most, scratch, per_xcd, (int)total, out);      \
   } while (0)
   if (dim == 64) LAUNCH(4);

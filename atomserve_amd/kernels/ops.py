@@ -1659,9 +1659,9 @@ def delta_prepare(qkv, num_kv_heads, dim, num_heads, proj, b_off, a_off, a_log, 
 
 
 # Rows of more tokens than this take the delta rule in chunks of 64 (csrc/recurrent.hip, delta_chunks), shorter ones token by
-# token: the chunks' two kernels take 35 us for one chunk of 8 to 32 heads of 128 and 4 us for every further one, the scan 0.4 us
-# a token (16 heads: 64 tokens 31 against 35 us, 100 tokens 46 and 37, 2,048 tokens 855 and 163; eight rows of 64 46 and 56, of 128
-# 81 and 72).
+# token: the chunks' two kernels take 25 us for one chunk of 8 to 16 heads of 128 and 4 us for every further one, the scan 0.4 us
+# a token (16 heads: 64 tokens 31 against 26 us, 100 tokens 46 and 30, 2,048 tokens 855 and 153; eight rows of 64 46 and 46, of 128
+# 83 and 67).  The line lies above one chunk: a step's many rows of up to 64 tokens are the scan's (30 rows of 60 116 and 127).
 DELTA_SCAN_MOST = 79
 DELTA_CHUNK = 64
 DELTA_CHUNK_SCRATCH = 2 * DELTA_CHUNK * DELTA_CHUNK + 3 * DELTA_CHUNK  # floats per chunk and head

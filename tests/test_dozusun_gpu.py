@@ -4,6 +4,8 @@ batches with pages and state slots used again, and through the engine's schedule
 weights are made here; where random weights would hide a fault (a window's edge, a far token in a state)
 the inputs are made so that it shows."""
 
+import math
+
 import pytest
 import torch
 
@@ -302,8 +304,8 @@ def test_delta_scan_however_the_state_is_cut_over_lanes(dim, vdim):
 def test_delta_rule_in_chunks(dim, vdim, G, H):
     """Rows around the chunk of 64 tokens and around the length from which chunks are taken, short rows beside them, states that
     are carried or not, decays from 1 down to 0 in any order: the chunked form is no further from the recurrence in 64 bits
-    than twice the scan (the same sums of 32-bit terms in another order), and a token that is not finite leaves the tokens
-    before it and the other rows untouched."""
+    than twice the scan (the same sums of 32-bit terms in another order), and a number that is not finite reaches what it
+    reaches in the scan: a query's its own token, a value's its column of the state from its token on."""
     from atomserve_amd.kernels import ops
 
     gen = torch.Generator().manual_seed(dim + vdim)
@@ -334,7 +336,7 @@ def test_delta_rule_in_chunks(dim, vdim, G, H):
     firsts = [sum(lens[:i]) for i in range(len(lens))]
     rows = (None,) + tuple(torch.tensor(x, dtype=torch.int32, device=DEV) for x in (firsts, lens, starts, slots))
 
-    def run(values, **how):
+    def run(values, beta=beta, decay=decay, **how):
         state, out = state0.clone().to(DEV), torch.full((T, H, vdim), 7.0, device=DEV)
         ops.delta_scan(values.to(DEV), G, dim, H, vdim, beta.to(DEV), decay.to(DEV), state, rows, out, **how)
         return out.cpu(), state.cpu()
@@ -346,14 +348,26 @@ def test_delta_rule_in_chunks(dim, vdim, G, H):
     assert (out.double() - want).abs().max() <= 2e-5 * float(want.abs().max())
     kept, kept_state = run(qkv, longest=max(lens), writes=False)
     assert torch.equal(kept, out) and torch.equal(kept_state, state0)
-    broken = qkv.clone()
-    place = firsts[5] + 70
-    broken[place, 2 * G * dim + 3] = float("inf")  # a value of the first head
-    got, got_state = run(broken, longest=max(lens))
-    rest = torch.ones(T, dtype=torch.bool)
-    rest[place : firsts[6]] = False
-    assert torch.allclose(got[rest], out[rest], atol=2e-5 * float(want.abs().max())) and torch.equal(got[:, 1:], out[:, 1:])
-    assert bool(got[place : firsts[6], 0, 3].isnan().all()) and bool(got_state[4, 0, :, 3].isnan().any()) and torch.equal(got_state[3], state[3])
+    # a number that is not finite, of the first head (or the keys and queries it shares): what the scan makes of it, wherever it lies in a chunk
+    whole = 2e-5 * float(want.abs().max())
+    for at, which, number in ((70, "v", math.inf), (0, "v", math.nan), (199, "v", -math.inf), (70, "q", math.nan), (127, "q", math.inf),
+                              (64, "k", math.nan), (63, "k", math.inf), (100, "beta", math.nan), (100, "decay", math.inf), (3, "decay", math.nan)):  # fmt: skip
+        place, bad, given = firsts[5] + at, qkv.clone(), {"beta": beta.clone(), "decay": decay.clone()}
+        if which in given:
+            given[which][place, 0] = number
+        else:
+            bad[place, {"q": 1, "k": G * dim + 1, "v": 2 * G * dim + 3}[which]] = number
+        (ref, ref_state), (got, got_state) = run(bad, **given), run(bad, longest=max(lens), **given)
+        for x, y, tol in ((got, ref, whole), (got_state, ref_state, 2e-5 * float(final.abs().max()))):
+            assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x == math.inf, y == math.inf) and torch.equal(x == -math.inf, y == -math.inf), (at, which)
+            good = y.isfinite()
+            assert (x[good] - y[good]).abs().max() <= tol, (at, which)
+        untouched = {"q": [place], "v": range(place, firsts[6])}.get(which, range(place, firsts[6]))
+        others = torch.ones(T, dtype=torch.bool)
+        others[list(untouched)] = False
+        assert got[others].isfinite().all() and (which != "q" or got_state.isfinite().all())
+        if which == "v":
+            assert got[:, 0, :3].isfinite().all() and got[:, 0, 4:].isfinite().all() and got[:, 1:].isfinite().all()
 
 
 def test_delta_rule_keeps_a_far_token():
