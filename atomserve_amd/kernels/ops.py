@@ -232,7 +232,7 @@ def attn_single_query(q, k_pages, v_pages, items, positions, tok_row, block_tabl
     """Attention of single query tokens over the paged cache.  bfloat16 with head widths in steps
     of 32 and pages of a multiple of 16 tokens runs on the matrix cores (a group of more than 16 query
     heads, or of wide heads that overfill a workgroup's LDS, as several equal groups that read the same kv
-    head); everything else (and all of fp32) on the general kernel.
+    head), and so do the fp32 heads that `attn_f32_supported` names, in 32 bits; everything else on the general kernel.
 
     q, out [T, H, D] (out fp32 for bfloat16 heads: the results unrounded); items [N] int32: the tokens (rows of q) to process, None for all of them in
     order; positions, tok_row [T] int32 (tok_row None: token t belongs to row t, a decode step);
@@ -296,6 +296,32 @@ def attn_f32_supported(dtype, num_heads: int, num_kv_heads: int, head_dim: int, 
     them to a kv head, whole steps of 16 keys to a page, no kept first keys; the rest runs on the general kernel."""
     return (dtype == F32 and head_dim in (64, 128) and num_heads % num_kv_heads == 0 and num_heads // num_kv_heads <= 16
             and block_size % 16 == 0 and keep_first == 0)  # fmt: skip
+
+
+# What 32-bit attention costs (microseconds, fitted to the kernel's times for portions of 9 to 512 tokens behind 0 to 30,000 keys, 4 to
+# 16 heads on 1 to 8 kv heads), by head width: (a prompt tile's launch and merge, 64 keys of one, a single query's launch,
+# a microsecond of `_partition_cost`).
+F32_ATTENTION_COSTS = {64: (5.2, 1.07, 4.0, 1.2), 128: (7.8, 1.65, 4.5, 2.2)}
+
+
+def attn_tiles_preferred(tokens: int, short: int, H: int, KV: int, D: int, max_context: int, window: int) -> bool:
+    """Whether a step of 32-bit heads runs its long rows as prompt tiles (`attn_prefill_f32`, the `short` tokens of short rows
+    beside them as single queries) or all of its tokens as single queries.  A tile reads its keys once for all of its queries,
+    but walks all of them in one workgroup; single queries' keys are cut into partitions.  16 heads of 128 on 8 kv heads,
+    tiles against single queries: 9 tokens alone 9.3 and 6.6 us, 64 10.5 and 8.8; 9 behind 2,000 keys 61 and 35, 33 61 and 81;
+    9 behind 8,000 209 and 97, 64 213 and 350; 9 behind 30,000 760 and 315."""
+    base, step, one, by = F32_ATTENTION_COSTS[D]
+    span = _seen_keys(max_context, window, 0, True)
+
+    def single(n: int) -> float:
+        groups = n * KV
+        if groups >= attn_fill_groups():
+            return one + by * (_partition_cost(groups, span, _up32(span)) - 4.0)
+        return one + by * (min(_partition_cost(groups, span, part) for part in MFMA_PARTITIONS) - 4.0)
+
+    workgroups = (tokens - short) * H / 16  # two share a compute unit, and 512 take 1.76 times as long as 256
+    tiles = (base + step * max(1.0, span / 64)) * max(1.0, workgroups / (1.13 * compute_units()))
+    return tiles + (single(short) if short else 0.0) <= single(tokens)
 
 
 def attn_prefill_f32(q, k_pages, v_pages, tiles, block_tables, out, scale, window, max_context, softcap=0.0, sink=False, chunk=0) -> None:

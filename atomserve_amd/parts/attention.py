@@ -144,18 +144,20 @@ def attend(q, out, step, cache, scale: float, window: int, split, wide: bool = F
         ops.wide_attend(q, cache.k_pages, cache.v_pages, step.positions, None if step.decode_only else step.tok_row,
                         cache.block_tables, out, scale, step.max_context, window, **sight)  # fmt: skip
         return
-    # Shapes that no prefill kernel takes: every token is a single query.
+    # Shapes that no prefill kernel takes, and 32-bit portions that it would walk for longer: every token is a single query.
     # Otherwise short rows are single queries and long rows go through the prefill kernel.
     if step.decode_only:  # token t is row t: the kernels need no maps from one to the other
         ops.attn_single_query(q, cache.k_pages, cache.v_pages, step.all_tokens, step.positions, None,
                               cache.block_tables, out, scale, window, step.max_context, **sight)  # fmt: skip
         return
-    f32 = ops.attn_f32_supported(q.dtype, q.shape[1], cache.k_pages.shape[1], q.shape[2], cache.block_size, sight.get("keep_first", 0) if window else 0)
-    if not f32 and not ops.attn_prefill_supported(q.dtype, q.shape[2], cache.block_size):
+    rows, (T, H, D), KV = step.split(split), q.shape, cache.k_pages.shape[1]
+    f32 = ops.attn_f32_supported(q.dtype, H, KV, D, cache.block_size, sight.get("keep_first", 0) if window else 0)
+    if f32 and rows.num_long_tiles:
+        f32 = ops.attn_tiles_preferred(T, rows.num_short_tokens, H, KV, D, step.max_context, window or sight.get("chunk", 0))
+    if not f32 and not ops.attn_prefill_supported(q.dtype, D, cache.block_size):
         ops.attn_single_query(q, cache.k_pages, cache.v_pages, step.all_tokens, step.positions, step.tok_row,
                               cache.block_tables, out, scale, window, step.max_context, **sight)  # fmt: skip
         return
-    rows = step.split(split)
     if rows.num_short_tokens:
         ops.attn_single_query(q, cache.k_pages, cache.v_pages, rows.short_tokens, step.positions, step.tok_row,
                               cache.block_tables, out, scale, window, rows.max_short_context, **sight)  # fmt: skip

@@ -90,3 +90,33 @@ def test_how_rows_of_a_state_space_are_cut_into_segments():
     assert choose(512, 2048, 64) == 256 and choose(511, 2048, 64) == 0 and choose(256, 2048, 64) == 0
     assert choose(2048, 2048, 8) == 64 and choose(200, 200, 1) == 64 and choose(100, 100, 1) == 0 and choose(0, 5, 1) == 0
     assert choose(8192, 8192, 4096) == 0  # a row's own workgroups fill it
+
+
+def test_which_32_bit_portions_run_as_prompt_tiles():
+    """A tile reads its keys once for all of its queries, a single query's keys are cut into partitions: short portions behind
+    long prefixes are single queries (as tiles they took longer than on the general kernel), prompts are tiles."""
+    tiles = lambda tokens, context, H=16, KV=8, D=128, window=0, short=0: ops.attn_tiles_preferred(  # noqa: E731
+        tokens, short, H, KV, D, context, window)
+    assert [tiles(n, 8000 + n) for n in (9, 16, 64, 128, 512)] == [False, False, True, True, True]
+    assert [tiles(n, n) for n in (9, 37, 64, 333, 512)] == [False, False, False, True, True]
+    assert not tiles(9, 30009) and not tiles(9, 2009) and tiles(33, 2033)
+    assert [tiles(n, 8000 + n, 4, 2, 64) for n in (9, 64, 128, 512)] == [False, False, False, True]
+    assert not tiles(9, 8009, window=512) and tiles(128, 8128, window=512) and tiles(520, 8000, short=8)
+
+
+@pytest.mark.parametrize("tokens,start,how", [(9, 8000, "single"), (9, 0, "single"), (128, 8000, "tiles"), (333, 0, "tiles"), (5, 100, "short")])
+def test_the_route_of_a_32_bit_portion(monkeypatch, tokens, start, how):
+    from types import SimpleNamespace
+
+    from atomserve_amd.parts.attention import attend
+
+    made = []
+    monkeypatch.setattr(ops, "attn_single_query", lambda q, k, v, items, *args, **kw: made.append(("single", items)))
+    monkeypatch.setattr(ops, "attn_prefill_f32", lambda q, k, v, tiles, *args, **kw: made.append(("tiles", tiles)))
+    pages = torch.empty(1, 8, 16, 128)
+    cache = SimpleNamespace(k_pages=pages, v_pages=pages.view(1, 8, 128, 16), block_tables=None, block_size=16)
+    rows = SimpleNamespace(num_short_tokens=tokens if tokens <= 8 else 0, num_long_tiles=0 if tokens <= 8 else -(-tokens // 64),
+                           short_tokens="short", long_tiles="long", max_short_context=start + tokens)  # fmt: skip
+    step = SimpleNamespace(decode_only=False, all_tokens="all", positions=None, tok_row=None, max_context=start + tokens, split=lambda key: rows)
+    attend(torch.empty(tokens, 16, 128), None, step, cache, 1.0, 0, (8, 64))
+    assert made == [{"single": ("single", "all"), "tiles": ("tiles", "long"), "short": ("single", "short")}[how]]
