@@ -670,7 +670,7 @@ def gemm(a, w, out, choices=None) -> None:
         call("as_gemm_bf16_skinny", _ptr(a), _ptr(rows), _wave_ptr(w), _ptr(out), _DT[out.dtype], M, N, K, 0, _stream())
         return
     strips = _wide_tile_strips(M, N, K) if out.dtype == F32 and _wave_ptr(w) else 0
-    if strips:
+    if strips and M <= WIDE_TILE_ALWAYS_ROWS and a.data_ptr() % 16 == 0:
         call("as_gemm_bf16_tile", _ptr(a), _ptr(rows), _wave_ptr(w), _ptr(out), 0, _DT[F32], M, N, K, 0, 0, strips, _stream())
     else:
         (choices or SHARED).gemm(a, w, out, M, N, K)
@@ -697,8 +697,8 @@ _workspace = {}  # device index -> the library's scratch memory, one for the pro
 # Beside the library's candidates a trial may time this package's plain tile product (9 to 128 rows, K in
 # chunks of 256, bf16 out, weights with a copy in wave order) with tiles of 2 and of 4 strips: for qkv
 # of Qwen3-8B sizes it takes 12.7 / 14.8 / 16.3 us at 32 / 48 / 64 rows against the library's best 14.7 /
-# 17.3 / 17.6; for the 4,096 columns of o the library wins at 32 to 64 rows.  Such a candidate's number
-# is OWN_CANDIDATE + its strips.
+# 17.3 / 17.6; for the 4,096 columns of o the library wins at 32 to 64 rows.  With 32-bit results (the head) the tile
+# product of 65 to 96 rows is such a candidate too (`_wide_tile_strips`).  Such a candidate's number is OWN_CANDIDATE + its strips.
 OWN_CANDIDATE = 1000
 
 
@@ -723,6 +723,9 @@ def _torch_gemm(a, w, out) -> None:
 
 def _own_candidates(M, N, K, dtype, w) -> list:
     """w: the weights, to see whether they have a copy in wave order; None: taken for granted."""
+    if dtype == F32 and (w is None or _wave_ptr(w)):
+        strips = _wide_tile_strips(M, N, K)
+        return [OWN_CANDIDATE + strips] if strips else []
     if dtype != BF16 or not _tile_rows(M, K, BF16, TILE_SPLIT_MAX_ROWS) or N % 16:
         return []
     if w is not None and not _wave_ptr(w):
@@ -732,9 +735,9 @@ def _own_candidates(M, N, K, dtype, w) -> list:
 
 def _library_call(a, w, out, M, N, K, candidate) -> None:
     if candidate >= OWN_CANDIDATE:
-        if not _wave_ptr(w) or out.dtype != BF16:
-            raise KernelError("the tile product was chosen for weights with a copy in wave order and bf16 results")
-        call("as_gemm_bf16_tile", _ptr(a), _ptr(_rows(w)), _wave_ptr(w), _ptr(out), 0, _DT[BF16], M, N, K, 0, 0,
+        if not _wave_ptr(w) or (out.dtype == F32 and a.data_ptr() % 16):
+            raise KernelError("the tile product was chosen for weights with a copy in wave order and rows that start on 16 bytes")
+        call("as_gemm_bf16_tile", _ptr(a), _ptr(_rows(w)), _wave_ptr(w), _ptr(out), 0, _DT[out.dtype], M, N, K, 0, 0,
              candidate - OWN_CANDIDATE, _stream())  # fmt: skip
         return
     call("as_blas_gemm", _ptr(a), _ptr(_rows(w)), _ptr(out), _DT[out.dtype], M, N, K, candidate,
@@ -815,8 +818,8 @@ class ProductChoices:
                 choice = self.choice[key] = _fastest_of(self.trials.pop(key))
         if choice < 0:
             return _torch_gemm(a, w, out)
-        if choice >= OWN_CANDIDATE and not _wave_ptr(w):
-            choice = 0  # chosen on weights that had a copy in wave order; these have none
+        if choice >= OWN_CANDIDATE and (not _wave_ptr(w) or (out.dtype == F32 and a.data_ptr() % 16)):
+            choice = 0  # chosen on weights that had a copy in wave order, or on aligned rows; these have none, or are not
         _library_call(a, w, out, M, N, K, choice)
 
     def _choice_of_tuned_rows(self, M, N, K, dtype):
@@ -922,14 +925,21 @@ def _tile_preferred(rows: int, k: int, n: int, w) -> bool:
 
 
 WIDE_TILE_MAX_ROWS = 96
+WIDE_TILE_ALWAYS_ROWS = 64  # above: one more candidate beside the library's in the timed trials
 
 
 def _wide_tile_strips(rows: int, n: int, k: int) -> int:
     """Strips of 16 weight rows per workgroup of the tile kernel for a product with 32-bit results and outputs enough to
-    fill the GPU several times (the head), 0 where the library's product runs: 17 to 96 rows and K in whole chunks.  151,936
-    outputs at 33 to 64 rows: K = 1,024 68 us against 83 for the library's best of 16 and 89 for its first, which a step of an
-    untuned row count takes; K = 4,096 243 against 251 and 276; at 128 rows its best is the faster one (287 against 297).  Few rows
-    want narrow tiles (17 rows, K = 2,048: 2 strips 99 us, 4 strips 114; 64 rows 144, 134 and 8 strips 128)."""
+    fill the GPU several times (the head), 0 where only the library's product runs: 17 to 96 rows and K in whole chunks.
+    151,936 outputs, the tile kernel against the library's best of 16 and its first (which a step of an untuned row count takes):
+    K            33 rows            64 rows            80 rows            96 rows
+    1,024     60   80   80       69   79   85       89   82   87       90   86   88
+    2,048    120  141  156      128  153  159      142  156  158      144  161  171
+    2,560    143  156  175      160  167  184      177  170  176      182  180  196
+    4,096    231  240  255      243  252  269      258  266  273      269  276  278
+    5,120    270  294  294      294  293  313      321  305  317      329  328  331
+    so up to 64 rows it runs, above them it is tried; at 128 rows and K = 4,096 the library's best takes 287 against 297.
+    Few rows want narrow tiles (17 rows, K = 2,048: 2 strips 99 us, 4 strips 114; 64 rows 144, 134 and 8 strips 128)."""
     if not SKINNY_MAX_ROWS < rows <= WIDE_TILE_MAX_ROWS or k % TILE_CHUNK or n % 16 or n * k * 2 > 0xF0000000:
         return 0
     strips = 2 if rows <= 24 else 4 if rows <= 32 or (k <= 1024 and rows <= 64) else 8

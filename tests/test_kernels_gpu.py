@@ -332,12 +332,48 @@ def test_gemm_bf16(ops, M, N, K):
 @pytest.mark.parametrize("N,K", [(32768, 256), (32768, 1280), (32768 + 16, 512), (16384, 1024)])
 def test_head_product_of_many_rows(ops, M, N, K):
     """Products with 32-bit results at every tile width and beyond the rows that the tiles take, weights with their copy: sums of
-    K terms in 32 bits of exact products, 2^-24 sqrt(K) of their sizes against the plain product."""
+    K terms in 32 bits of exact products, 2^-24 sqrt(K) of their sizes against the plain product.  17 to 64 rows run on the tile
+    kernel (up to 32 of a narrow K on the few-rows one), 65 to 96 may (a trial finds out), and rows that do not start on 16 bytes go to the library."""
+    from atomserve_amd.kernels.lib import Launches, call
+
     torch.manual_seed(62)
     a, w = torch.randn(M, K, device=DEV).to(BF16), (torch.randn(N, K, device=DEV) / math.sqrt(K)).to(BF16)
-    out = torch.full((M, N), float("nan"), device=DEV)
-    ops.gemm(a, ops.Streamed(w), out)
-    assert (out.double() - a.double() @ w.double().T).abs().max() <= 16 * math.sqrt(K) * 2.0**-24
+    w, ref, good = ops.Streamed(w), a.double() @ w.double().T, 16 * math.sqrt(K) * 2.0**-24
+
+    def routes(a):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        with Launches() as made:
+            ops.gemm(a, w, out, ops.ProductChoices(fixed=True))
+        assert (out.double() - ref).abs().max() <= good
+        return [name for name, _, _ in made.calls]
+
+    few = ops._few_rows(M, K, N)
+    assert M <= 32 if few else M > 16
+    assert routes(a) == ["as_gemm_bf16_skinny" if few else "as_gemm_bf16_tile" if M <= 64 else "as_blas_gemm"]
+    shifted = torch.empty(M * K + 1, dtype=BF16, device=DEV)[1:].view(M, K)
+    shifted.copy_(a)
+    if not few:
+        assert routes(shifted) == ["as_blas_gemm"]
+    own, most = ops._own_candidates(M, N, K, F32, w), N // (256 * 128)  # 8 strips of 16 rows for every compute unit
+    assert own == ([ops.OWN_CANDIDATE + 8] if 65 <= M <= 96 and most else own if M <= 64 else [])
+    assert ops._own_candidates(M, N, K, F32, ops.Streamed(w.rows, copy=False)) == []
+    for strips in (2, 4, 8) if M > 16 else ():
+        out = torch.full((M, N - 16), float("nan"), device=DEV)  # the last workgroup's strips are not whole
+        call("as_gemm_bf16_tile", a.data_ptr(), w.rows.data_ptr(), w.wave.data_ptr(), out.data_ptr(), 0, 0, M, N - 16, K, 0, 0, strips,
+             torch.cuda.current_stream().cuda_stream)  # fmt: skip
+        assert (out.double() - ref[:, : N - 16]).abs().max() <= good
+    for candidate in own if M > 64 else ():
+        choices = ops.ProductChoices()
+        choices.tune_rows(M)
+        out = torch.full((M, N), float("nan"), device=DEV)
+        choices.gemm(a, w, out, M, N, K)
+        assert choices.trials[(M, N, K, F32)]["ids"][-1] == candidate
+        choices.trials.clear()
+        choices.choice[(M, N, K, F32)] = candidate
+        for x, weights in ((a, w), (shifted, w), (a, w.rows)):
+            out.fill_(float("nan"))
+            choices.gemm(x, weights, out, M, N, K)
+            assert (out.double() - ref).abs().max() <= good
 
 
 @pytest.mark.parametrize("M,I,K", [(1, 96, 64), (8, 1000, 96), (5, 1030, 4096), (16, 12288, 4096), (9, 700, 2048),
