@@ -638,6 +638,11 @@ __global__ __launch_bounds__(256) void delta_pairs_kernel(const float* __restric
   // The inverse in blocks of 16: a wave inverts its block on the diagonal, column by column from the top down, then the
   // blocks below, one diagonal after the other: T_ij = -T_ii sum_k A_ik T_kj.  A block lies as a product leaves it (lane:
   // column lr, rows 4 lg + x), which is how the next product takes it as its right operand.
+  // A wave reads what its own lanes have written: LDS answers a wave in order, and the fences keep the compiler from
+  // moving the reads before the writes (a lane's own addresses differ, so nothing else would).
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   floatx4 diag, left;  // T_ww as a right and as a left operand
   {
     const float* block = A + (wave * 16) * LA + wave * 16;
