@@ -1445,6 +1445,8 @@ extern "C" int as_attn_single_query(const void* q, const void* k_pages, const vo
 //   S[key][query] = K[key][:] . Q[query][:]     keys straight from the page, 16 bytes a lane
 //   O^T[d][query] += V^T[d][key] P[key][query]  values straight from the transposed page; P is what the lane holds
 // The next step's keys are asked for when this step's have met the queries, its values when these have been added up.
+// Values of places that none of the workgroup's queries sees count as 0 whatever lies there (0.1 us); of keys that only some of
+// a tile's queries see they are finite, as every kernel that stores values makes them.
 // Bound by the 64 matrix instructions of a step (heads of 128): 0.9 us a wave, and by launch and merge for short
 // contexts.  16 heads of 128 on 8 kv heads, in a captured step: 4 requests of 600 tokens 12.2 us, of 2,000 tokens 18.4 (45.2 and 54.4
 // on the general kernel, which reads each value of a transposed page alone); a prompt of 333 tokens 24 (147: a workgroup to
@@ -1484,7 +1486,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   const bool valid = tok < count;
   const int pos = valid ? pos0 + tok : -1;
   const int first = valid ? first_in_window(sight, pos + 1) : 0;       // this column's first visible key
-  const int start = first_in_window(sight, pos0 + 1) & ~15;             // the workgroup's, in whole steps
+  const int seen = first_in_window(sight, pos0 + 1), start = seen & ~15;  // the workgroup's first, and that in whole steps
   const int k0 = start + part * part_size, k1 = P == 1 ? pos0 + count : min(pos0 + count, k0 + part_size);
   if (k0 >= k1) {  // an empty partition (items only): mark it so for the reduce
     if (tid < G) {
@@ -1555,6 +1557,14 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
 #pragma unroll
     for (int r = 0; r < 4; ++r) p[r] = expf(s[r] - at);
     l += (p[0] + p[1]) + (p[2] + p[3]);
+    if (__builtin_expect(k0 + step * 16 < seen || k0 + step * 16 + 16 > k1, 0)) {  // whatever lies where no key is seen: a weight of 0 is not enough
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (key + r < seen || key + r >= k1) {
+#pragma unroll
+          for (int i = 0; i < DT; ++i) vf[i][r] = 0.f;
+        }
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll

@@ -1004,6 +1004,43 @@ def test_attention_in_32_bits_on_the_matrix_cores(ops, H, KV, D, bs, how):
     assert torch.allclose(out, ref, atol=1e-4), (out - ref).abs().max()
 
 
+@pytest.mark.parametrize("D,bs,how", [(128, 16, {}), (64, 48, {"window": 21}), (128, 32, {"chunk": 40})])
+def test_32_bit_attention_reads_nothing_into_places_without_keys(ops, D, bs, how):
+    """Places of a page behind a context's end and in front of its window may hold anything, also what is not finite: the
+    results, of single queries and of prompt tiles, are those over clean pages, bit for bit."""
+    H, KV, lens, n = 4, 2, [1, 15, 17, 40, 130, 531], 12
+    how = dict(how)
+    window, chunk = how.pop("window", 0), how.get("chunk", 0)
+    _, k_pages, v_pages, tables, _ = paged_case(F32, H, KV, D, bs, lens, seed=3, k_scale=0.5)
+    q = torch.randn(n * len(lens), H, D, device=DEV, generator=torch.Generator(DEV).manual_seed(4))
+
+    def run(k_pages, v_pages, news, part=None):
+        tiles, positions, flat = [], [], 0
+        for r, new in enumerate(news):
+            tiles.append([flat, new, r, lens[r] - new])
+            positions += list(range(lens[r] - new, lens[r]))
+            flat += new
+        out = torch.full((flat, H, D), float("nan"), device=DEV)
+        if max(news) == 1:
+            ops.attn_single_query(q[:flat], k_pages, v_pages, None, i32(positions), None, tables, out, D**-0.5, window, max(lens), part, **how)
+        else:
+            ops.attn_prefill_f32(q[:flat], k_pages, v_pages, i32(tiles), tables, out, D**-0.5, window, max(lens), **how)
+        return out
+
+    for news, part in (([1] * len(lens), None), ([1] * len(lens), 64), ([min(n, m) for m in lens], None)):
+        want, dirty = run(k_pages, v_pages, news, part), [k_pages.clone(), v_pages.clone()]
+        held = torch.zeros(k_pages.shape[0], bs, dtype=torch.bool)
+        for r, (new, length) in enumerate(zip(news, lens)):
+            first = length - new  # the first query's position
+            seen = max(0, first - window + 1) if window else first // chunk * chunk if chunk else 0
+            for key in range(seen, length):
+                held[int(tables[r, key // bs]), key % bs] = True
+        for bad in (float("nan"), float("inf")):
+            dirty[0].masked_fill_(~held.to(DEV)[:, None, :, None], bad)
+            dirty[1].masked_fill_(~held.to(DEV)[:, None, None, :], bad)
+            assert want.isfinite().all() and torch.equal(run(*dirty, news, part), want)
+
+
 @pytest.mark.parametrize("H,KV,D,bs,window", [(32, 8, 128, 16, 0), (6, 2, 32, 16, 0), (8, 8, 64, 32, 0), (4, 1, 96, 16, 0),
                                                (16, 2, 128, 16, 0), (4, 2, 64, 16, 40), (4, 2, 64, 16, 1), (4, 2, 256, 16, 0),
                                                (2, 1, 224, 32, 0), (10, 2, 160, 16, 70)])  # fmt: skip
