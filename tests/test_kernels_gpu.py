@@ -289,25 +289,47 @@ def test_gemm_fp32_rows_do_not_depend_on_the_batch(ops):
         assert torch.equal(one[0], full[i])
 
 
-@pytest.mark.parametrize("M,N,K,shift", [(1, 33, 4, 0), (15, 17, 256, 0), (16, 16, 260, 0), (17, 31, 512, 0), (33, 65, 516, 0), (63, 47, 1028, 0),
-                                         (65, 130, 2052, 0), (20, 40, 257, 0), (5, 50, 64, 1), (40, 70, 1000, 1)])  # fmt: skip
+@pytest.mark.parametrize("M,N,K,shift", [(1, 33, 260, 0), (15, 17, 272, 0), (16, 16, 257, 0), (17, 31, 512, 0), (33, 65, 516, 0), (63, 47, 1028, 0),
+                                         (65, 130, 2052, 0), (20, 40, 259, 0), (66, 129, 1030, 0), (5, 50, 288, 1), (40, 70, 1000, 1),
+                                         (64, 64, 1024, 2), (18, 33, 513, 3)])  # fmt: skip
 def test_gemm_fp32_tiles_agree(ops, M, N, K, shift):
-    """Every tile of the 32-bit product gives the same bits (the order of a sum depends on K alone), whole and odd widths,
-    aligned and shifted matrices.  Bound: chains of at most K / 16 + 31 terms and 6 additions (of K terms up to 256
-    columns), each rounding 2^-24 of the sums of absolute values."""
+    """Every tile of the 32-bit product of more than 256 columns gives the same bits, and a row alone those that it has among others (the
+    order of a sum depends on K alone): whole and odd widths, aligned and shifted matrices.  Bound: slices of at most K / 16 + 32 columns
+    and 6 additions, each rounding 2^-24 of the sums of absolute values."""
     from atomserve_amd.kernels.lib import call
 
     torch.manual_seed(60)
     a = torch.randn(M * K + shift, device=DEV)[shift:].view(M, K)
     w = torch.randn(N * K + shift, device=DEV)[shift:].view(N, K)
-    outs = []
-    for form in range(6):
-        out = torch.full((M, N), float("nan"), device=DEV)
-        call("as_gemm_f32", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, form, torch.cuda.current_stream().cuda_stream)
-        outs.append(out)
+
+    def product(a, form):
+        out = torch.full((a.shape[0], N), float("nan"), device=DEV)
+        call("as_gemm_f32", a.data_ptr(), w.data_ptr(), out.data_ptr(), a.shape[0], N, K, form, torch.cuda.current_stream().cuda_stream)
+        return out
+
+    outs = [product(a, form) for form in range(6)]
     assert all(torch.equal(outs[0], o) for o in outs)
-    bound = (a.abs().double() @ w.abs().double().T) * (K / 16 + 37 if K > 256 else K) * 2.0**-24
+    for i in {0, M // 2, M - 1}:
+        assert torch.equal(product(a[i : i + 1], 0)[0], outs[0][i])
+    bound = (a.abs().double() @ w.abs().double().T) * (K / 16 + 38) * 2.0**-24
     assert bool(((outs[0].double() - a.double() @ w.double().T).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("M,N,K,shift", [(1, 33, 4, 0), (15, 17, 256, 0), (64, 64, 16, 0), (65, 63, 255, 0), (63, 130, 33, 0), (129, 65, 200, 3),
+                                         (5, 50, 64, 1)])  # fmt: skip
+def test_gemm_fp32_of_narrow_rows(ops, M, N, K, shift):
+    """Up to 256 columns every output is one chain of multiply-adds in the order of the columns: K roundings of 2^-24 of the sums of
+    absolute values, and a row alone has the bits that it has among others."""
+    torch.manual_seed(61)
+    a = torch.randn(M * K + shift, device=DEV)[shift:].view(M, K)
+    w = torch.randn(N * K + shift, device=DEV)[shift:].view(N, K)
+    out, one = torch.full((M, N), float("nan"), device=DEV), torch.full((1, N), float("nan"), device=DEV)
+    ops.gemm(a, w, out)
+    bound = (a.abs().double() @ w.abs().double().T) * K * 2.0**-24
+    assert bool(((out.double() - a.double() @ w.double().T).abs() <= bound).all())
+    for i in {0, M // 2, M - 1}:
+        ops.gemm(a[i : i + 1], w, one)
+        assert torch.equal(one[0], out[i])
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 96, 64), (8, 1000, 96), (64, 4096, 1024), (300, 257, 192), (5, 2000, 4096),
