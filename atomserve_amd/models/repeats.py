@@ -81,21 +81,28 @@ class _Own:
 
     def __init__(self, model, step, first: int, period: int):
         self.model, self.step, self.tensors = model, step, []
-        self.layers = []  # per layer: its class, and its parts' attributes as (part, class, [(attribute, whether it has a copy)])
+        # per layer: its class, its parts' attributes as (part, class, [(attribute, whether it has a copy)]) and those of the norm that follows
+        self.layers = []
         for k in range(period):
             block, names = model.blocks[model.plan.run[first + k].layer], []
             for name, part in block.parts().items():
                 wanted = [(attr, isinstance(v, ops.Streamed)) for attr, v in vars(part).items()
                           if v is None or isinstance(v, (torch.Tensor, ops.Streamed))]  # fmt: skip
                 names.append((name, type(part), wanted))
-            self.layers.append((type(block), names))
+            after = self.norm_after(first + k)
+            self.layers.append((type(block), names, [attr for attr, v in vars(after).items() if v is None or isinstance(v, torch.Tensor)]
+                                if after is not None else []))  # fmt: skip
         self.tensors = self.of(first)
+
+    def norm_after(self, i: int):
+        run = self.model.plan.run
+        return self.model.blocks[run[i + 1].layer].first_norm() if i + 1 < len(run) else None
 
     def of(self, start: int):
         """Tensors, numbers of the caches and None, of the stretch that starts at run `start`; None where a layer is of another
         class, something stands in place of its methods, or a plain tensor for a matrix with a copy or the other way round."""
         model, plan, found = self.model, self.model.plan, []
-        for i, (kind, names) in enumerate(self.layers, start):
+        for i, (kind, names, gains) in enumerate(self.layers, start):
             block = model.blocks[plan.run[i].layer]
             if type(block) is not kind or "forward" in vars(block):
                 return None
@@ -114,9 +121,9 @@ class _Own:
                     else:
                         found.append(v)
             _view_parts(self.step.cache_view(plan.cache_id(i), True), found)
-            after = model.blocks[plan.run[i + 1].layer].first_norm() if i + 1 < len(plan.run) else None
-            if after is not None:
-                found.extend([v for _, v in sorted(vars(after).items()) if isinstance(v, torch.Tensor)])
+            if gains:
+                have = vars(self.norm_after(i))
+                found.extend([have.get(attr) for attr in gains])
         return found
 
     def addresses(self) -> list:
@@ -128,7 +135,7 @@ class _Own:
         for i in places:
             v = self.tensors[i]
             if at.setdefault(id(v), i) == i:
-                self.met.append((i, v.dtype, v.shape, v.is_contiguous()))
+                self.met.append((i, v, v.data_ptr(), v.dtype, v.shape, v.is_contiguous()))
             else:
                 self.alike.append((i, at[id(v)]))  # one tensor under two names
         places = set(places)
@@ -141,11 +148,13 @@ class _Own:
         if own is None or len(own) != len(self.tensors):
             return None
         found = [0] * len(own)
-        for i, dtype, shape, contiguous in self.met:
+        for i, source, address, dtype, shape, contiguous in self.met:
             v = own[i]
-            if v is None or v.dtype is not dtype or v.shape != shape or v.is_contiguous() != contiguous:
-                return None
-            found[i] = v.data_ptr()
+            if v is not source:  # what all layers of a step share is itself
+                if v is None or v.dtype is not dtype or v.shape != shape or v.is_contiguous() != contiguous:
+                    return None
+                address = v.data_ptr()
+            found[i] = address
         for i, j in self.alike:
             if own[i] is not own[j]:
                 return None
