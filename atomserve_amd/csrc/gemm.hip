@@ -1,11 +1,5 @@
-// Matrix products out[M, N] = a[M, K] @ w[N, K]^T (weights keep the checkpoint's
+// Matrix products of bf16 matrices, out[M, N] = a[M, K] @ w[N, K]^T (weights keep the checkpoint's
 // [out, in] layout).
-//
-// gemm_f32: genuine fp32 multiply-add on the matrix cores' fp32 instruction (products and sums in 32 bits, no mode
-// of reduced precision).  The order of every output's sum depends on K alone, so a row's result does not depend on
-// which other rows share the launch, nor on the tile that the launch chose: K is cut into 16 slices of whole steps of
-// 16 columns (an even number), each slice is one chain, four neighbouring slices are added up in order, then the four
-// sums of four.  Up to F32_NARROW columns the sum is one chain over k = 0..K-1 in order.
 // Plain reference: reference atomserve/quant.py:89-91 (F.linear).
 #include "common.h"
 
@@ -16,247 +10,6 @@ template <typename OutT> __device__ __forceinline__ void store4(OutT* p, floatx4
 template <> __device__ __forceinline__ void store4<float>(float* p, floatx4 v, int valid) {
   if (valid == 4 && (((uintptr_t)p) & 15) == 0) { *reinterpret_cast<floatx4*>(p) = v; return; }
   for (int i = 0; i < valid; ++i) p[i] = v[i];
-}
-
-// A workgroup makes a tile of 16 MT rows of `a` by 16 NT rows of `w`; its waves share the tile and take the slices of
-// K (16 waves one each, 4 waves four neighbouring ones each), so that no wave needs what another has loaded: operands
-// go straight from memory into the operands of v_mfma_f32_16x16x4_f32, 16 bytes a lane (four columns: the k order
-// within a step is the same permutation for both operands), DEPTH steps ahead.  The waves' sums meet in LDS.
-// `w` is the left operand: a lane's 4 results are 4 consecutive outputs of one row of `a`.
-// Few rows: bound by reading w (4 rows of 1,024 against 151,936 outputs: 119 us, 5.2 TB/s); a tile of two strips reads
-// the rows of `a` half as often as one of one, and two steps share a line of 128 bytes whose halves are asked for
-// together (150 us when they are asked for a step apart).  Many rows: bound by the matrix cores (157 TFLOP/s): 512 rows of 2,048 against
-// 12,288 outputs take 250 us (103 TFLOP/s), 333 of 1,024 against 4,096 50 us.  A kernel of fp32 multiply-adds through LDS, 64 x 64
-// outputs a workgroup, took 124 us on average for the products of 4 rows at a width of 1,024 and 129 for 333.
-// VEC: rows start on 16 bytes (K % 4 == 0 and both matrices do).
-#define F32_SLICES 16
-template <int MT, int NT, int WAVES, int DEPTH, bool VEC>
-__global__ __launch_bounds__(WAVES * 64, MT * NT == 16 ? 2 : 1) void gemm_f32_kernel(const float* __restrict__ a, const float* __restrict__ w,
-                                                              float* __restrict__ out, int M, int N, int K, int tiles_m,
-                                                              int tiles, int per_xcd) {
-  constexpr int T = MT * NT;
-  extern __shared__ floatx4 red[];  // [4][T][64]
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lr = lane & 15, lg = lane >> 4;
-  // Workgroups are dealt to the 8 XCDs in turn; each XCD takes a run of tiles with the tiles of the same rows of `w`
-  // side by side, so that its L2 reads its share of the weights once.
-  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (tile >= tiles) return;
-  const int n0 = tile / tiles_m * (16 * NT), m0 = tile % tiles_m * (16 * MT);
-  const int steps = (K + 31) / 32 * 2;  // two steps share 32 columns: a lane's pieces of the two are neighbours
-  const int per = (steps + 2 * F32_SLICES - 1) / (2 * F32_SLICES) * 2;  // steps of a slice
-  constexpr int SLICES = F32_SLICES / WAVES;              // of a wave
-  const int st0 = min(steps, wave * SLICES * per), st1 = min(steps, st0 + SLICES * per);
-
-  const float* wrow[NT];
-  const float* arow[MT];
-#pragma unroll
-  for (int i = 0; i < NT; ++i) wrow[i] = w + (size_t)min(n0 + i * 16 + lr, N - 1) * K;
-#pragma unroll
-  for (int i = 0; i < MT; ++i) arow[i] = a + (size_t)min(m0 + i * 16 + lr, M - 1) * K;
-
-  auto fetch = [&](const float* row, int k) -> floatx4 {  // columns k .. k+3 (VEC: what lies beyond K is cleared before its use)
-    if constexpr (VEC) {
-      return *reinterpret_cast<const floatx4*>(row + (k < K ? k : 0));
-    } else {
-      floatx4 v;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = k + i < K ? row[k + i] : 0.f;
-      return v;
-    }
-  };
-  auto column = [&](int step) { return (step >> 1) * 32 + lg * 8 + (step & 1) * 4; };
-  floatx4 wv[DEPTH][NT], av[DEPTH][MT], acc[NT][MT], sum[NT][MT];
-#pragma unroll
-  for (int i = 0; i < NT; ++i)
-#pragma unroll
-    for (int j = 0; j < MT; ++j) { acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f}; sum[i][j] = acc[i][j]; }
-#pragma unroll
-  for (int u = 0; u < DEPTH; ++u) {
-    const int k = column(min(st0 + u, steps - 1));
-#pragma unroll
-    for (int i = 0; i < NT; ++i) wv[u][i] = fetch(wrow[i], k);
-#pragma unroll
-    for (int j = 0; j < MT; ++j) av[u][j] = fetch(arow[j], k);
-  }
-  int left = per;  // steps until the slice ends
-  for (int st = st0; st < st1; st += DEPTH) {
-#pragma unroll
-    for (int u = 0; u < DEPTH; ++u) {
-      if (st + u < st1) {
-        if (VEC && (K & 31) && st + u >= steps - 2 && column(st + u) >= K) {
-#pragma unroll
-          for (int i = 0; i < NT; ++i) wv[u][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int j = 0; j < MT; ++j) av[u][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-#pragma unroll
-        for (int x = 0; x < 4; ++x)
-#pragma unroll
-          for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int j = 0; j < MT; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][i][x], av[u][j][x], acc[i][j], 0, 0, 0);
-        if (u & 1) {  // both steps of the pair that follows: one after the other, so that a line is fetched once
-#pragma unroll
-          for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int v = 0; v < 2; ++v) wv[u - 1 + v][i] = fetch(wrow[i], column(min(st + u - 1 + v + DEPTH, steps - 1)));
-#pragma unroll
-          for (int j = 0; j < MT; ++j)
-#pragma unroll
-            for (int v = 0; v < 2; ++v) av[u - 1 + v][j] = fetch(arow[j], column(min(st + u - 1 + v + DEPTH, steps - 1)));
-        }
-        if (SLICES > 1 && --left == 0) {
-          left = per;
-#pragma unroll
-          for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int j = 0; j < MT; ++j) { sum[i][j] += acc[i][j]; acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f}; }
-        }
-      }
-    }
-  }
-  if constexpr (SLICES > 1) {
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-      for (int j = 0; j < MT; ++j) red[(wave * T + i * MT + j) * 64 + lane] = sum[i][j] + acc[i][j];  // acc: a slice that K's end cut short
-  } else {  // four waves add into one place, one after the other
-#pragma unroll
-    for (int turn = 0; turn < 4; ++turn) {
-      if ((wave & 3) == turn) {
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-          for (int j = 0; j < MT; ++j) {
-            floatx4* place = red + ((wave >> 2) * T + i * MT + j) * 64 + lane;
-            *place = turn == 0 ? acc[i][j] : *place + acc[i][j];
-          }
-      }
-      if (turn < 3) __syncthreads();
-    }
-  }
-  __syncthreads();
-  for (int x = threadIdx.x; x < T * 64; x += WAVES * 64) {
-    const floatx4 v = ((red[x] + red[x + T * 64]) + red[x + 2 * T * 64]) + red[x + 3 * T * 64];
-    const int l = x & 63, t = x >> 6;
-    const int n = n0 + t / MT * 16 + (l >> 4) * 4, m = m0 + t % MT * 16 + (l & 15);
-    if (m < M && n < N) store4(out + (size_t)m * N + n, v, min(4, N - n));
-  }
-}
-
-// K <= F32_NARROW (toy widths, ranks of two-step projections): there is little to stream and nothing to cut, and the sum
-// stays one chain: a workgroup makes 64 x 64 outputs through LDS, a thread 4 x 4 of them, by fp32 multiply-adds.  333 rows of 192
-// against 4,096 outputs: 16.4 us; the same chain on the matrix cores, a wave to 16 x 32 outputs straight from memory,
-// gives the same bits in 50 us (2,048 rows of 64 against 2,048: 14.3 and 45.8).
-#define F32_NARROW 256
-#define BM 64
-#define BN 64
-#define BK 16
-__global__ __launch_bounds__(256) void gemm_f32_narrow_kernel(const float* __restrict__ a, const float* __restrict__ w,
-                                                       float* __restrict__ out, int M, int N, int K) {
-  __shared__ float as[BK][BM + 4];
-  __shared__ float ws[BK][BN + 4];
-  const int tid = threadIdx.x;
-  const int tx = tid & 15, ty = tid >> 4;  // 16 x 16 threads, 4 x 4 outputs each
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int lr = tid >> 2, lk = (tid & 3) * 4;  // this thread loads 4 consecutive k of row lr
-  float acc[4][4] = {};
-  const bool vec = (K & 3) == 0;
-  for (int kb = 0; kb < K; kb += BK) {
-    float av[4] = {0.f, 0.f, 0.f, 0.f}, wv[4] = {0.f, 0.f, 0.f, 0.f};
-    const int k = kb + lk;
-    if (m0 + lr < M) {
-      const float* p = a + (size_t)(m0 + lr) * K + k;
-      if (vec && k + 3 < K) { const float4 r = *reinterpret_cast<const float4*>(p); av[0] = r.x; av[1] = r.y; av[2] = r.z; av[3] = r.w; }
-      else { for (int i = 0; i < 4; ++i) if (k + i < K) av[i] = p[i]; }
-    }
-    if (n0 + lr < N) {
-      const float* p = w + (size_t)(n0 + lr) * K + k;
-      if (vec && k + 3 < K) { const float4 r = *reinterpret_cast<const float4*>(p); wv[0] = r.x; wv[1] = r.y; wv[2] = r.z; wv[3] = r.w; }
-      else { for (int i = 0; i < 4; ++i) if (k + i < K) wv[i] = p[i]; }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { as[lk + i][lr] = av[i]; ws[lk + i][lr] = wv[i]; }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < BK; ++kk) {
-      float ar[4], wr[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { ar[i] = as[kk][ty * 4 + i]; wr[i] = ws[kk][tx * 4 + i]; }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jn = 0; jn < 4; ++jn) acc[i][jn] = fmaf(ar[i], wr[jn], acc[i][jn]);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int jn = 0; jn < 4; ++jn) {
-      const int n = n0 + tx * 4 + jn;
-      if (n < N) out[(size_t)m * N + n] = acc[i][jn];
-    }
-  }
-}
-
-// The tile: what a round of workgroups (one to a compute unit) takes per 1,024 of K, measured for N = 1,024 to 12,288 and
-// K = 1,024 to 6,144 at 1 to 512 rows (within 15 per cent of the best tile there): small tiles where the larger ones
-// would leave compute units idle, large ones where operands would be read over and over (N = 1,024, K = 2,048: 4 rows 10.6
-// us with the first and 41 with the last; N = 12,288 at 512 rows 1,000 and 257).  The results are the same bit for bit.
-struct F32Tile { int mt, nt; float round_us, alone_us; };  // alone: the tiles of one round, with room to spare
-static const F32Tile f32_tiles[] = {{1, 1, 5.5f, 2.8f}, {1, 2, 5.8f, 5.8f}, {2, 2, 8.f, 8.f}, {4, 2, 13.f, 13.f}, {4, 4, 21.5f, 21.5f}};
-
-// form: 0: chosen here; else 1 + the index of a tile (tests).
-extern "C" int as_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
-  if (M <= 0) return AS_OK;
-  if (N <= 0 || K <= 0 || form < 0 || form > 5) return AS_BAD_SHAPE;
-  const auto tiles_of = [&](const F32Tile& t, long* across) {
-    *across = ((long)M + 16 * t.mt - 1) / (16 * t.mt);
-    return *across * (((long)N + 16 * t.nt - 1) / (16 * t.nt));
-  };
-  if (K <= F32_NARROW) {
-    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-    if (grid.y > 65535) return AS_BAD_SHAPE;
-    gemm_f32_narrow_kernel<<<grid, 256, 0, stream>>>(a, w, out, M, N, K);
-    return launch_status();
-  }
-  long tiles_m = 0, tiles = 0;
-  if (form == 0) {
-    float best = 0.f;
-    for (int i = 0; i < 5; ++i) {
-      const long rounds = (tiles_of(f32_tiles[i], &tiles_m) + compute_units() - 1) / compute_units();
-      const float cost = 5.f + (float)K / 1024.f * (rounds == 1 ? f32_tiles[i].alone_us : f32_tiles[i].round_us * (float)rounds);
-      if (form == 0 || cost < best) { best = cost; form = i + 1; }
-    }
-  }
-  tiles = tiles_of(f32_tiles[form - 1], &tiles_m);
-  if (tiles > 0x3fffffff) return AS_BAD_SHAPE;
-  const int per_xcd = (int)((tiles + 7) / 8);
-  const bool vec = (K & 3) == 0 && (((uintptr_t)a | (uintptr_t)w) & 15) == 0;
-#define LAUNCH(MTV, NTV, WV, DV)                                                                                       \
-  do {                                                                                                                 \
-    const size_t lds = (size_t)4 * MTV * NTV * 64 * sizeof(floatx4);                                                   \
-    if (vec)                                                                                                           \
-      gemm_f32_kernel<MTV, NTV, WV, DV, true><<<per_xcd * 8, WV * 64, lds, stream>>>(a, w, out, M, N, K, (int)tiles_m, \
-                                                                                     (int)tiles, per_xcd);             \
-    else                                                                                                               \
-      gemm_f32_kernel<MTV, NTV, WV, 2, false><<<per_xcd * 8, WV * 64, lds, stream>>>(a, w, out, M, N, K, (int)tiles_m, \
-                                                                                     (int)tiles, per_xcd);             \
-  } while (0)
-  switch (form) {
-    case 1: LAUNCH(1, 1, 16, 4); break;
-    case 2: LAUNCH(1, 2, 4, 4); break;
-    case 3: LAUNCH(2, 2, 4, 4); break;
-    case 4: LAUNCH(4, 2, 4, 4); break;
-    default: LAUNCH(4, 4, 4, 2); break;
-  }
-#undef LAUNCH
-  return launch_status();
 }
 
 // ---- bf16, few rows (decode): weights stream once from HBM through the matrix cores ----

@@ -1,0 +1,640 @@
+// Matrix products of 32-bit matrices: out[M, N] = a[M, K] @ w[N, K]^T (weights keep the checkpoint's [out, in] layout).
+//
+// A float is the sum of three bf16 values: its nearest one, the nearest one of what is left, and the rest, which fits
+// (8 + 8 + 8 bits).  A product of two floats is then nine products of bf16 values, of which the matrix cores, sixteen times
+// faster on bf16 than on fp32, compute the six largest; the three left out are below 2^-24 of the product and of either sign.
+// Sums are fp32.  The largest of the six has a chain of sums of its own: small products that are added to a large sum are cut
+// off downwards, and that error has one sign.  Against 64 bits (K = 1,024 / 2,048 / 3,072, normal values) the error is 0.76e-7 /
+// 0.87e-7 / 0.98e-7 of the result (in one chain 1.15e-7 / 1.7e-7 / 2.1e-7), with the cores' fp32 instruction in the same order
+// 1.55e-7 / 2.1e-7 / 2.6e-7; heavy tails, outliers and one sign alike: at most 0.9 of that instruction's error.
+// Numbers below 2^-110 keep an absolute error of 2^-134 instead.  Values that are not finite (or that round to infinity in bf16)
+// would become NaN in the parts: a result that is not finite is computed again with the fp32 instruction.
+//
+// The order of every output's sum depends on K alone, so a row's result does not depend on which other rows share the launch,
+// nor on the kernel or the tile that the launch chose: K is cut into 16 slices of whole steps of 32 columns, each slice is one
+// pair of chains (the largest products; the other five of a step in one order), four neighbouring slices are added up in order, then the four sums of four.
+// Up to F32_NARROW columns the sum is one chain of fp32 multiply-adds over k = 0..K-1 in order.
+// Plain reference: reference atomserve/quant.py:89-91 (F.linear).
+#include "common.h"
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx8 __attribute__((ext_vector_type(8)));
+typedef bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+#define F32_SLICES 16
+#define F32_GROUPS 4  // of neighbouring slices
+#define F32_NARROW 256
+
+struct Parts { bf16x8 h, m, l; };  // eight floats as h + m + l
+
+__device__ __forceinline__ floatx8 widen(bf16x8 v) {
+  const uintx4 u = __builtin_bit_cast(uintx4, v);
+  floatx8 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    r[2 * i] = __uint_as_float(u[i] << 16);
+    r[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
+  }
+  return r;
+}
+
+__device__ __forceinline__ Parts parts(floatx4 p, floatx4 q) {
+  floatx8 x = __builtin_shufflevector(p, q, 0, 1, 2, 3, 4, 5, 6, 7);
+  Parts s;
+  s.h = __builtin_convertvector(x, bf16x8);  // to nearest
+  x -= widen(s.h);
+  s.m = __builtin_convertvector(x, bf16x8);
+  x -= widen(s.m);
+  s.l = __builtin_convertvector(x, bf16x8);
+  return s;
+}
+
+// Which parts of w and of a the six products of a step take, the smallest first; the largest (x = 5) has a chain of its own
+__device__ __forceinline__ bf16x8 part(const Parts& s, int i) { return i == 0 ? s.h : i == 1 ? s.m : s.l; }
+constexpr int PART_W[6] = {2, 0, 1, 1, 0, 0}, PART_A[6] = {0, 2, 1, 0, 1, 0};
+
+__device__ __forceinline__ bool finite(floatx4 v) {
+  bool ok = true;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) ok = ok && (__float_as_uint(v[r]) & 0x7f800000u) != 0x7f800000u;
+  return ok;
+}
+
+__device__ __forceinline__ void store4(float* p, floatx4 v, int valid) {
+  if (valid == 4 && (((uintptr_t)p) & 15) == 0) { *reinterpret_cast<floatx4*>(p) = v; return; }
+  for (int i = 0; i < valid; ++i) p[i] = v[i];
+}
+
+// Columns k .. k+3 of a row, those from K on as zeros.  VEC: rows start on 16 bytes and K % 4 == 0.
+template <bool VEC> __device__ __forceinline__ floatx4 fetch(const float* row, int k, int K) {
+  if constexpr (VEC) {
+    const floatx4 v = *reinterpret_cast<const floatx4*>(row + (k < K ? k : 0));
+    return k < K ? v : floatx4{0.f, 0.f, 0.f, 0.f};
+  } else {
+    floatx4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = k + i < K ? row[k + i] : 0.f;
+    return v;
+  }
+}
+
+// `v`, where it is not finite, again by the fp32 instruction over the steps st0 .. st1 - 1: 16 rows of w (this lane's `wrow`)
+// by 16 of a.  All lanes of a wave call it together; seldom taken, so it waits for every step's loads.
+template <bool VEC> __device__ __forceinline__ floatx4 again_f32(floatx4 v, const float* wrow, const float* arow, int K, int st0, int st1) {
+  const int lg = (threadIdx.x & 63) >> 4;
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int st = st0; st < st1; ++st)
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int k = st * 32 + lg * 8 + half * 4;
+      const floatx4 wv = fetch<VEC>(wrow, k, K), av = fetch<VEC>(arow, k, K);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[x], av[x], acc, 0, 0, 0);
+    }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v[r] = (__float_as_uint(v[r]) & 0x7f800000u) == 0x7f800000u ? acc[r] : v[r];
+  return v;
+}
+
+// What a product carries along when the residual sum and the RMSNorm around it are folded into the products of a decode step
+// (a pre-norm layer: x += part(norm(x))), as the few-rows products of bf16 do:
+//   producer (LINK): the sum goes on top of the stream x = out[M, N]; scaled[M, N] = x * gain, the input of the next product
+//     without its 1/rms factor; ssq_out[M, strips] = the sums of x^2 per 16 columns.
+//   consumer (ssq_in): 1/rms of each row comes from the row's sums of squares and multiplies the product's sums.
+struct LinkF32 {
+  const float* ssq_in;
+  int strips_in;
+  float eps;
+  const float* gain;
+  float* scaled;
+  float* ssq_out;
+};
+
+enum { PLAIN, GATED, LINK };
+
+__device__ __forceinline__ floatx4 silu_times(floatx4 g, floatx4 u) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) u[r] *= g[r] / (1.0f + expf(-g[r]));
+  return u;
+}
+
+template <int LANES> __device__ __forceinline__ bf16x8 rotated(bf16x8 v) {  // within 16 lanes: lane i takes lane (i + LANES) % 16
+  if constexpr (LANES == 0) return v;
+  uintx4 u = __builtin_bit_cast(uintx4, v);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) u[i] = __builtin_amdgcn_update_dpp(0, (int)u[i], 0x120 + 16 - LANES, 0xf, 0xf, false);
+  return __builtin_bit_cast(bf16x8, u);
+}
+
+// Operands straight from memory: a workgroup makes a tile of 16 MT rows of `a` by 16 NT rows of `w`; its waves share the tile
+// and take the slices of K (16 waves one each, 8 two, 4 four neighbouring ones), so that no wave needs what another has loaded: 32
+// bytes a lane and step, DEPTH steps ahead.  The waves' sums meet in LDS.  `w` is the left operand: a lane's 4 results are
+// 4 consecutive outputs of one row of `a`.
+// SHARE: with at most 16 / SHARE rows the 16 lanes of a row group hold SHARE steps' rows side by side, which are taken apart
+// once for all of them and turned into place by a rotation of the lanes: the vector unit, which takes the floats apart (44
+// instructions for 8 columns of 16 rows), is what a product of few rows is made of beside reading w.
+// GATED: NT = 2, gate rows and the up rows of the same outputs (w has 2 N rows); LINK: MT = NT = 1; ssq_in: MT = 1.
+// VEC: rows start on 16 bytes (K % 4 == 0 and both matrices do).
+template <int MT, int NT, int WAVES, int DEPTH, int SHARE, bool VEC, int MODE>
+__global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_rows_kernel(const float* __restrict__ a,
+                                                                                       const float* __restrict__ w, float* __restrict__ out,
+                                                                                       int M, int N, int K, int tiles_m, int tiles,
+                                                                                       int per_xcd, LinkF32 link) {
+  static_assert(DEPTH % SHARE == 0 && (SHARE == 1 || MT == 1), "whole groups of steps, one row tile");
+  static_assert(MODE != GATED || NT == 2, "a gate strip and its up strip");
+  static_assert(MODE != LINK || (NT == 1 && MT == 1), "one strip of the stream");
+  constexpr int T = MT * NT, SLICES = F32_SLICES / WAVES;  // slices of a wave
+  constexpr int ENTRIES = SLICES == 4 ? 4 : F32_SLICES;    // sums that meet in LDS: of groups or of slices
+  constexpr int ROWS = 16 / SHARE;
+  extern __shared__ floatx4 red[];  // [ENTRIES][T][64]
+  __shared__ float inv_rms[16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  // Workgroups are dealt to the 8 XCDs in turn; each XCD takes a run of tiles with the tiles of the same rows of `w`
+  // side by side, so that its L2 reads its share of the weights once.
+  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (tile >= tiles) return;
+  constexpr int ACROSS = MODE == GATED ? 16 : 16 * NT;
+  const int n0 = tile / tiles_m * ACROSS, m0 = tile % tiles_m * (16 * MT);
+  const int steps = (K + 31) / 32, per = (steps + F32_SLICES - 1) / F32_SLICES;
+  const int st0 = min(steps, wave * SLICES * per), st1 = min(steps, st0 + SLICES * per);
+
+  auto weight = [&](int i) {  // this lane's row of strip i
+    return w + (MODE == GATED ? (size_t)min(n0 + lr, N - 1) + (size_t)i * N : (size_t)min(n0 + i * 16 + lr, N - 1)) * K;
+  };
+  const float* wrow[NT];
+  const float* arow[MT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) wrow[i] = weight(i);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) arow[i] = a + (size_t)min(m0 + i * 16 + lr % ROWS, M - 1) * K;
+
+  floatx4 wv[DEPTH][NT][2], av[DEPTH / SHARE][MT][2], acc[NT][MT], low[NT][MT], sum[SLICES == 4 ? NT : 1][MT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) { acc[i][j] = low[i][j] = floatx4{0.f, 0.f, 0.f, 0.f}; if (SLICES == 4) sum[i][j] = acc[i][j]; }
+  auto load = [&](int u, int st) {  // a step's columns of w, and, for the first of SHARE steps, of a
+    const int k = min(st, steps - 1) * 32 + lg * 8;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int half = 0; half < 2; ++half) wv[u][i][half] = fetch<VEC>(wrow[i], k + 4 * half, K);
+    if (u % SHARE == 0) {
+      const int ka = SHARE == 1 ? k : min(st + lr / ROWS, steps - 1) * 32 + lg * 8;
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) av[u / SHARE][j][half] = fetch<VEC>(arow[j], ka + 4 * half, K);
+    }
+  };
+  auto slice_done = [&](int slice) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        if constexpr (SLICES == 4) sum[i][j] += acc[i][j] + low[i][j];
+        else red[(slice * T + i * MT + j) * 64 + lane] = acc[i][j] + low[i][j];
+        acc[i][j] = low[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u) load(u, st0 + u);
+  if (link.ssq_in != nullptr && wave < M && wave < 16) {  // 1 / rms of the rows, a wave a row; published by the barrier below
+    for (int row = wave; row < M && row < 16; row += WAVES) {
+      float ss = 0.f;
+      for (int j = lane; j < link.strips_in; j += 64) ss += link.ssq_in[(size_t)row * link.strips_in + j];
+      ss = wave_sum(ss);
+      if (lane == 0) inv_rms[row] = 1.0f / sqrtf(ss / (float)K + link.eps);
+    }
+  }
+  int left = per, slice = wave * SLICES;  // steps until the slice ends
+  Parts shared[MT];
+  for (int st = st0; st < st1; st += DEPTH) {
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) {
+      if (st + u < st1) {
+        Parts as[MT], ws[NT];
+        if (u % SHARE == 0) {
+#pragma unroll
+          for (int j = 0; j < MT; ++j) shared[j] = parts(av[u / SHARE][j][0], av[u / SHARE][j][1]);
+        }
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+          switch (u % SHARE * ROWS) {  // known when compiled
+            case 0: as[j] = shared[j]; break;
+            case 4: as[j] = Parts{rotated<4>(shared[j].h), rotated<4>(shared[j].m), rotated<4>(shared[j].l)}; break;
+            case 8: as[j] = Parts{rotated<8>(shared[j].h), rotated<8>(shared[j].m), rotated<8>(shared[j].l)}; break;
+            default: as[j] = Parts{rotated<12>(shared[j].h), rotated<12>(shared[j].m), rotated<12>(shared[j].l)}; break;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NT; ++i) ws[i] = parts(wv[u][i][0], wv[u][i][1]);
+        load(u, st + u + DEPTH);
+#pragma unroll
+        for (int x = 0; x < 6; ++x)
+#pragma unroll
+          for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+              floatx4& to = x == 5 ? acc[i][j] : low[i][j];
+              to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part(ws[i], PART_W[x]), part(as[j], PART_A[x]), to, 0, 0, 0);
+            }
+        if (--left == 0) {
+          left = per;
+          slice_done(slice++);
+        }
+      }
+    }
+  }
+  if constexpr (SLICES == 4) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) red[(wave * T + i * MT + j) * 64 + lane] = sum[i][j] + (acc[i][j] + low[i][j]);  // a slice that K's end cut short
+  } else {
+    for (; slice < (wave + 1) * SLICES; ++slice) slice_done(slice);  // one that K's end cut short, and empty ones
+  }
+  __syncthreads();
+  auto total = [&](int t) {
+    floatx4 v;
+#pragma unroll
+    for (int g = 0; g < F32_GROUPS; ++g) {
+      floatx4 s;
+      if constexpr (ENTRIES == F32_GROUPS) {
+        s = red[(g * T + t) * 64 + lane];
+      } else {
+        s = red[(4 * g * T + t) * 64 + lane];
+#pragma unroll
+        for (int x = 1; x < 4; ++x) s += red[((4 * g + x) * T + t) * 64 + lane];
+      }
+      v = g == 0 ? s : v + s;
+    }
+    const int m = m0 + t % MT * 16 + lr;
+    const bool mine = m < M && n0 + (MODE == GATED ? 0 : t / MT * 16) + lg * 4 < N;
+    if (__any(mine && !finite(v))) v = again_f32<VEC>(v, weight(t / MT), a + (size_t)min(m, M - 1) * K, K, 0, steps);
+    return v;
+  };
+  for (int t = wave; t < (MODE == GATED ? MT : T); t += WAVES) {
+    const int n = n0 + t / MT * 16 + lg * 4, m = m0 + t % MT * 16 + lr;
+    floatx4 v = total(t);
+    if (link.ssq_in != nullptr) v *= inv_rms[lr];  // MT = 1: rows 0 .. 15 are the launch's
+    if constexpr (MODE == GATED) {
+      floatx4 up = total(MT + t);
+      if (link.ssq_in != nullptr) up *= inv_rms[lr];
+      v = silu_times(v, up);
+    }
+    if constexpr (MODE == LINK) {
+      float ss = 0.f;
+      if (m < M && n < N) {  // N % 4 == 0
+        float* xp = out + (size_t)m * N + n;
+        v += *reinterpret_cast<floatx4*>(xp);
+        *reinterpret_cast<floatx4*>(xp) = v;
+        *reinterpret_cast<floatx4*>(link.scaled + (size_t)m * N + n) = v * *reinterpret_cast<const floatx4*>(link.gain + n);
+        ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+      }
+      ss += __shfl_xor(ss, 16, 64);  // the four lanes that hold the strip's 16 columns of row m
+      ss += __shfl_xor(ss, 32, 64);
+      if (lane < 16 && m < M) link.ssq_out[(size_t)m * ((N + 15) / 16) + n0 / 16] = ss;
+    } else if (m < M && n < N) {
+      store4(out + (size_t)m * N + n, v, min(4, N - n));
+    }
+  }
+}
+
+// Operands through LDS, for many rows: 8 waves (WM x WN) make a tile of BM = 16 WM MTW rows of `a` by BN = 16 WN NTW rows of
+// `w` in steps of 32 columns.  Every float is taken apart once a workgroup, on its way from registers (loaded two steps ahead) into
+// LDS, where the parts of the next step are written while those of this one are multiplied: one barrier a step.
+// A place holds 16 bytes, 8 columns of a row; place (row, column block c) of a part is row * 4 + (c ^ f(row / 4 % 4)), f =
+// 0, 2, 3, 1: the hardware reads 16-byte operands in the lane groups {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31} and the
+// same above 32, which so touch every bank once.
+// GATED: half of a tile's rows of w are gate rows, half the up rows of the same outputs.
+// SPLIT: blockIdx.y names a group of four slices, whose sums go to out[group][m][n] for whoever adds the groups up in order.
+// VEC only: rows start on 16 bytes and K % 4 == 0.
+template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT>
+__global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                             float* __restrict__ out, int M, int N, int K, int tiles_m, int tiles,
+                                                             int per_xcd) {
+  constexpr int THREADS = 512, AHEAD = 2;
+  constexpr int BM = 16 * WM * MTW, BN = 16 * WN * NTW, ROWS = BM + BN;
+  constexpr int PIECES = ROWS * 4 / THREADS;  // of 8 columns a thread and step
+  constexpr int PLANE = ROWS * 4;
+  static_assert(WM * WN == 8 && ROWS * 4 % THREADS == 0 && (!IS_GATED || NTW == 2) && !(IS_GATED && SPLIT), "");
+  extern __shared__ bf16x8 lds[];  // [2][3][PLANE]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (tile >= tiles) return;
+  const int n0 = tile / tiles_m * (IS_GATED ? BN / 2 : BN), m0 = tile % tiles_m * BM;
+  const int wm = wave % WM, wn = wave / WM;
+  const int all = (K + 31) / 32, per = (all + F32_SLICES - 1) / F32_SLICES;
+  const int st0 = SPLIT ? min(all, (int)blockIdx.y * 4 * per) : 0, st1 = SPLIT ? min(all, st0 + 4 * per) : all;
+  if (SPLIT) out += (size_t)blockIdx.y * M * N;
+  // row r of the tile's rows of w
+  auto weight = [&](int r) -> const float* {
+    const int n = IS_GATED ? n0 + (r >> 5) * 16 + (r & 15) : n0 + r;
+    return w + (size_t)(min(n, N - 1) + (IS_GATED && (r & 16) ? N : 0)) * K;
+  };
+  const float* src[PIECES];
+  int dst[PIECES];
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) {
+    const int x = threadIdx.x + p * THREADS, r = x >> 2, c = x & 3;
+    src[p] = r < BM ? a + (size_t)min(m0 + r, M - 1) * K : weight(r - BM);
+    dst[p] = r * 4 + (c ^ (0x78 >> (r >> 1 & 6) & 3));
+  }
+  floatx4 ahead[AHEAD][PIECES][2];
+  auto load = [&](int u, int st) {
+    const int at = min(st, all - 1), k = at * 32 + (threadIdx.x & 3) * 8;
+    if (at * 32 + 32 <= K) {
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) ahead[u][p][half] = *reinterpret_cast<const floatx4*>(src[p] + k + 4 * half);
+    } else {
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p)
+#pragma unroll
+        for (int half = 0; half < 2; ++half) ahead[u][p][half] = fetch<true>(src[p], k + 4 * half, K);
+    }
+  };
+  auto place = [&](int u, int buf) {
+    bf16x8* base = lds + buf * 3 * PLANE;
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      const Parts s = parts(ahead[u][p][0], ahead[u][p][1]);
+      base[dst[p]] = s.h;
+      base[PLANE + dst[p]] = s.m;
+      base[2 * PLANE + dst[p]] = s.l;
+    }
+  };
+  floatx4 acc[NTW][MTW], low[NTW][MTW], group[NTW][MTW], total[NTW][MTW];
+#pragma unroll
+  for (int i = 0; i < NTW; ++i)
+#pragma unroll
+    for (int j = 0; j < MTW; ++j) acc[i][j] = low[i][j] = group[i][j] = total[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) load(u, st0 + u);
+  place(0, 0);
+  load(0, st0 + AHEAD);
+  int left = per, slice = 0;
+  const int ra = (wm * MTW * 16 + lr) * 4 + (lg ^ (0x78 >> (lr >> 1 & 6) & 3));
+  const int rw = (BM + wn * NTW * 16 + lr) * 4 + (lg ^ (0x78 >> (lr >> 1 & 6) & 3));
+  auto step = [&](int st, int u, int buf) {  // u: where st + 1 waits in registers; buf: where st lies in LDS
+    __syncthreads();
+    const bf16x8* base = lds + buf * 3 * PLANE;
+    bf16x8 av[MTW][3], wv[NTW][3];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+#pragma unroll
+      for (int j = 0; j < MTW; ++j) av[j][x] = base[x * PLANE + ra + j * 64];
+#pragma unroll
+      for (int i = 0; i < NTW; ++i) wv[i][x] = base[x * PLANE + rw + i * 64];
+    }
+    place(u, buf ^ 1);
+    load(u, st + 1 + AHEAD);
+#pragma unroll
+    for (int x = 0; x < 6; ++x)
+#pragma unroll
+      for (int i = 0; i < NTW; ++i)
+#pragma unroll
+        for (int j = 0; j < MTW; ++j) {
+          floatx4& to = x == 5 ? acc[i][j] : low[i][j];
+          to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i][PART_W[x]], av[j][PART_A[x]], to, 0, 0, 0);
+        }
+    if (--left == 0) {
+      left = per;
+      ++slice;
+#pragma unroll
+      for (int i = 0; i < NTW; ++i)
+#pragma unroll
+        for (int j = 0; j < MTW; ++j) {
+          group[i][j] += acc[i][j] + low[i][j];
+          acc[i][j] = low[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+          if (!SPLIT && (slice & 3) == 0) {
+            total[i][j] += group[i][j];
+            group[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+          }
+        }
+    }
+  };
+  int st = st0;
+  for (; st + 2 <= st1; st += 2) {
+    step(st, 1, 0);
+    step(st + 1, 0, 1);
+  }
+  if (st < st1) step(st, 1, 0);
+#pragma unroll
+  for (int j = 0; j < MTW; ++j) {
+    const int m = m0 + (wm * MTW + j) * 16 + lr;
+    floatx4 v[NTW];
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) {
+      v[i] = total[i][j] + (group[i][j] + (acc[i][j] + low[i][j]));
+      const int r = (wn * NTW + i) * 16;
+      const bool mine = m < M && (IS_GATED ? n0 + wn * 16 : n0 + r) + lg * 4 < N;
+      if (__any(mine && !finite(v[i]))) v[i] = again_f32<true>(v[i], weight(r + lr), a + (size_t)min(m, M - 1) * K, K, st0, st1);
+    }
+    if constexpr (IS_GATED) {
+      const int n = n0 + wn * 16 + lg * 4;
+      if (m < M && n < N) store4(out + (size_t)m * N + n, silu_times(v[0], v[1]), min(4, N - n));
+    } else {
+#pragma unroll
+      for (int i = 0; i < NTW; ++i) {
+        const int n = n0 + (wn * NTW + i) * 16 + lg * 4;
+        if (m < M && n < N) store4(out + (size_t)m * N + n, v[i], min(4, N - n));
+      }
+    }
+  }
+}
+
+// K <= F32_NARROW (toy widths, ranks of two-step projections): there is little to stream and nothing to cut, and the sum
+// stays one chain: a workgroup makes 64 x 64 outputs through LDS, a thread 4 x 4 of them, by fp32 multiply-adds.  333 rows of 192
+// against 4,096 outputs: 16.4 us; the same chain on the matrix cores, a wave to 16 x 32 outputs straight from memory,
+// gives the same bits in 50 us (2,048 rows of 64 against 2,048: 14.3 and 45.8).
+#define BM 64
+#define BN 64
+#define BK 16
+__global__ __launch_bounds__(256) void gemm_f32_narrow_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                       float* __restrict__ out, int M, int N, int K) {
+  __shared__ float as[BK][BM + 4];
+  __shared__ float ws[BK][BN + 4];
+  const int tid = threadIdx.x;
+  const int tx = tid & 15, ty = tid >> 4;  // 16 x 16 threads, 4 x 4 outputs each
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int lr = tid >> 2, lk = (tid & 3) * 4;  // this thread loads 4 consecutive k of row lr
+  float acc[4][4] = {};
+  const bool vec = (K & 3) == 0;
+  for (int kb = 0; kb < K; kb += BK) {
+    float av[4] = {0.f, 0.f, 0.f, 0.f}, wv[4] = {0.f, 0.f, 0.f, 0.f};
+    const int k = kb + lk;
+    if (m0 + lr < M) {
+      const float* p = a + (size_t)(m0 + lr) * K + k;
+      if (vec && k + 3 < K) { const float4 r = *reinterpret_cast<const float4*>(p); av[0] = r.x; av[1] = r.y; av[2] = r.z; av[3] = r.w; }
+      else { for (int i = 0; i < 4; ++i) if (k + i < K) av[i] = p[i]; }
+    }
+    if (n0 + lr < N) {
+      const float* p = w + (size_t)(n0 + lr) * K + k;
+      if (vec && k + 3 < K) { const float4 r = *reinterpret_cast<const float4*>(p); wv[0] = r.x; wv[1] = r.y; wv[2] = r.z; wv[3] = r.w; }
+      else { for (int i = 0; i < 4; ++i) if (k + i < K) wv[i] = p[i]; }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { as[lk + i][lr] = av[i]; ws[lk + i][lr] = wv[i]; }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < BK; ++kk) {
+      float ar[4], wr[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) { ar[i] = as[kk][ty * 4 + i]; wr[i] = ws[kk][tx * 4 + i]; }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int jn = 0; jn < 4; ++jn) acc[i][jn] = fmaf(ar[i], wr[jn], acc[i][jn]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int m = m0 + ty * 4 + i;
+    if (m >= M) continue;
+#pragma unroll
+    for (int jn = 0; jn < 4; ++jn) {
+      const int n = n0 + tx * 4 + jn;
+      if (n < N) out[(size_t)m * N + n] = acc[i][jn];
+    }
+  }
+}
+
+static long f32_tiles(int M, int N, int rows, int columns) {
+  return (((long)M + rows - 1) / rows) * (((long)N + columns - 1) / columns);
+}
+static bool aligned16(const void* a, const void* b) { return ((((uintptr_t)a) | ((uintptr_t)b)) & 15) == 0; }
+
+template <int MT, int NT, int WAVES, int DEPTH, int SHARE, int MODE>
+static int launch_rows(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
+  constexpr size_t lds = (size_t)(WAVES == 4 ? F32_GROUPS : F32_SLICES) * MT * NT * 64 * sizeof(floatx4);
+  static_assert(lds + 64 <= 65536, "what a launch may ask for without an attribute");
+  const long tiles = f32_tiles(M, N, 16 * MT, MODE == GATED ? 16 : 16 * NT);
+  if (tiles > 0x3fffffff) return AS_BAD_SHAPE;
+  const int per_xcd = (int)((tiles + 7) / 8), tiles_m = (M + 16 * MT - 1) / (16 * MT);
+  if ((K & 3) == 0 && aligned16(a, w))
+    gemm_f32_rows_kernel<MT, NT, WAVES, DEPTH, SHARE, true, MODE><<<per_xcd * 8, WAVES * 64, lds, stream>>>(a, w, out, M, N, K, tiles_m,
+                                                                                                         (int)tiles, per_xcd, link);
+  else
+    gemm_f32_rows_kernel<MT, NT, WAVES, SHARE, SHARE, false, MODE><<<per_xcd * 8, WAVES * 64, lds, stream>>>(a, w, out, M, N, K, tiles_m,
+                                                                                                         (int)tiles, per_xcd, link);
+  return launch_status();
+}
+
+// One row tile: as many steps side by side as its rows leave lanes for.
+template <int NT, int WAVES, int DEPTH, int MODE>
+static int launch_few(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
+  if (M <= 4) return launch_rows<1, NT, WAVES, 4, 4, MODE>(a, w, out, M, N, K, link, stream);
+  if (M <= 8) return launch_rows<1, NT, WAVES, DEPTH, 2, MODE>(a, w, out, M, N, K, link, stream);
+  return launch_rows<1, NT, WAVES, DEPTH, 1, MODE>(a, w, out, M, N, K, link, stream);
+}
+
+template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT>
+static int launch_tile(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+  constexpr int TM = 16 * WM * MTW, TN = 16 * WN * NTW;
+  constexpr int lds = 2 * 3 * (TM + TN) * 64;
+  if ((K & 3) != 0 || !aligned16(a, w)) return AS_BAD_SHAPE;
+  const long tiles = f32_tiles(M, N, TM, IS_GATED ? TN / 2 : TN);
+  if (tiles > 0x3fffffff) return AS_BAD_SHAPE;
+  const auto kernel = gemm_f32_tile_kernel<WM, WN, MTW, NTW, IS_GATED, SPLIT>;
+  if (lds > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+    return AS_LAUNCH_FAILED;
+  const int per_xcd = (int)((tiles + 7) / 8), tiles_m = (M + TM - 1) / TM;
+  kernel<<<dim3(per_xcd * 8, SPLIT ? F32_GROUPS : 1), 512, lds, stream>>>(a, w, out, M, N, K, tiles_m, (int)tiles, per_xcd);
+  return launch_status();
+}
+
+// Which kernel: the tile of rows of a by rows of w, and what a workgroup on every compute unit takes per 1,024 of K
+// beside the 4.5 us of a launch: the first round, every round.  Measured for N = 1,024 to 12,288 and K = 1,024 to 6,144 at 1 to 512 rows:
+// small tiles where the larger ones would leave compute units idle, large ones where operands would be read over and over
+// (N = 4,096, K = 1,024: 4 rows 8.3 us with the first and 53 with the last; N = 12,288, K = 2,048 at 512 rows 624 and 197,
+// with the fp32 instruction from memory 272).  The results are the same bit for bit.
+struct F32Tile { int rows, columns; float alone_us, round_us; };
+static const F32Tile f32_forms[] = {{16, 16, 3.4f, 4.5f},   {16, 16, 4.5f, 3.6f},   {16, 32, 6.2f, 5.6f},    {32, 16, 5.5f, 7.4f},
+                                    {32, 32, 7.8f, 9.f},    {64, 32, 12.f, 13.f},   {64, 64, 18.f, 14.5f},   {128, 128, 48.f, 48.f}};
+#define F32_FORMS 8
+#define F32_TILE_FORMS 6  // the first through LDS
+
+static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
+  const long rounds = (f32_tiles(M, N, t.rows, t.columns) * split + compute_units() - 1) / compute_units();
+  const float crowd = t.rows == 16 && t.columns == 16 && M > 8 ? 1.2f : 1.f;  // nothing of a's parts is shared
+  return 4.5f + (float)K / 1024.f / (float)split * crowd * (t.alone_us + t.round_us * (float)(rounds - 1));
+}
+
+// form: 0: chosen here; else 1 + the index of a kernel (tests).
+template <int MODE> static int gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
+  const bool vec = (K & 3) == 0 && aligned16(a, w);
+  if (form == 0) {
+    float best = 0.f;
+    for (int i = MODE == GATED ? 2 : 0; i < F32_FORMS; ++i) {
+      if ((MODE == GATED && i == 3) || (i >= F32_TILE_FORMS && !vec)) continue;
+      const float cost = f32_cost(f32_forms[i], M, MODE == GATED ? 2 * N : N, K, 1);
+      if (form == 0 || cost < best) { best = cost; form = i + 1; }
+    }
+  }
+  const LinkF32 link{};
+  if constexpr (MODE == GATED) {
+    switch (form) {
+      case 3:
+        if (f32_tiles(M, N, 16, 16) <= compute_units()) return launch_rows<1, 2, 8, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
+        return launch_rows<1, 2, 4, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
+      case 5: return launch_rows<2, 2, 4, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
+      case 6: return launch_rows<4, 2, 4, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
+      case 7: return launch_tile<4, 2, 1, 2, true, false>(a, w, out, M, N, K, stream);
+      case 8: return launch_tile<2, 4, 4, 2, true, false>(a, w, out, M, N, K, stream);
+    }
+  } else {
+    switch (form) {
+      case 1:
+        if (M <= 16) return launch_few<1, 8, 4, PLAIN>(a, w, out, M, N, K, link, stream);
+        return launch_rows<1, 1, 8, 4, 1, PLAIN>(a, w, out, M, N, K, link, stream);
+      case 2:
+        if (M <= 16) return launch_few<1, 4, 4, PLAIN>(a, w, out, M, N, K, link, stream);
+        return launch_rows<1, 1, 4, 4, 1, PLAIN>(a, w, out, M, N, K, link, stream);
+      case 3: return launch_rows<1, 2, 4, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
+      case 4: return launch_rows<2, 1, 8, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
+      case 5: return launch_rows<2, 2, 4, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
+      case 6: return launch_rows<4, 2, 4, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
+      case 7: return launch_tile<4, 2, 1, 2, false, false>(a, w, out, M, N, K, stream);
+      case 8: return launch_tile<2, 4, 4, 2, false, false>(a, w, out, M, N, K, stream);
+    }
+  }
+  return AS_BAD_SHAPE;
+}
+
+extern "C" int as_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
+  if (M <= 0) return AS_OK;
+  if (N <= 0 || K <= 0 || form < 0 || form > F32_FORMS) return AS_BAD_SHAPE;
+  if (K <= F32_NARROW) {
+    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
+    if (grid.y > 65535) return AS_BAD_SHAPE;
+    gemm_f32_narrow_kernel<<<grid, 256, 0, stream>>>(a, w, out, M, N, K);
+    return launch_status();
+  }
+  return gemm_f32<PLAIN>(a, w, out, M, N, K, form, stream);
+}
+
+// out[M, N] = silu(a @ w[:N]^T) * (a @ w[N:]^T) for w[2 N, K].  K > F32_NARROW; the activation on the sums that the plain product
+// stores: the same bits as the two kernels.
+extern "C" int as_gemm_f32_gated(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
+  if (M <= 0) return AS_OK;
+  if (N <= 0 || N > 0x3fffffff || K <= F32_NARROW || form < 0 || form > F32_FORMS) return AS_BAD_SHAPE;
+  return gemm_f32<GATED>(a, w, out, M, N, K, form, stream);
+}
+
+// sums[4][M, N]: the product's sums over the four quarters of K's slices; added up in order they are the product, bit for bit.  For
+// products of too few outputs to fill the GPU: N = 1,024, K = 2,048 at 333 rows 17.8 us, whole 28.7.  K > F32_NARROW, K % 4 == 0,
+// N % 4 == 0, rows that start on 16 bytes.
+extern "C" int as_gemm_f32_split(const float* a, const float* w, float* sums, int M, int N, int K, int form, hipStream_t stream) {
+  if (M <= 0) return AS_OK;
+  if (N <= 0 || (N & 3) || K <= F32_NARROW || form < 0 || form > 2) return AS_BAD_SHAPE;
+  if (form == 0) form = f32_cost(f32_forms[6], M, N, K, F32_GROUPS) <= f32_cost(f32_forms[7], M, N, K, F32_GROUPS) ? 1 : 2;
+  if (form == 1) return launch_tile<4, 2, 1, 2, false, true>(a, w, sums, M, N, K, stream);
+  return launch_tile<2, 4, 4, 2, false, true>(a, w, sums, M, N, K, stream);
+}

@@ -988,6 +988,40 @@ def gemm_split(a, w, plan=None):
     return sums
 
 
+F32_NARROW = 256  # up to here a 32-bit sum is one chain, which nothing cuts
+F32_GROUPS = 4  # what a 32-bit sum's order comes in above that, whatever kernel runs
+
+
+def gemm_f32_split_preferred(rows: int, n: int, k: int, w) -> bool:
+    """Whether a 32-bit product of more than 16 rows, whose sums are wanted in parts, is cut into the four groups of its
+    order: while its tiles of 64 x 64 outputs are no more than the compute units (512 rows, K = 2,048: N = 2,048 30 us against
+    42 whole; N = 4,096 60 against 61, which the longer reading of whoever adds the parts up outweighs)."""
+    return (rows > SKINNY_MAX_ROWS and k > F32_NARROW and k % 4 == 0 and n % 4 == 0 and _rows(w).data_ptr() % 16 == 0
+            and -(-rows // 64) * -(-n // 64) <= compute_units())  # fmt: skip
+
+
+def gemm_f32_split(a, w):
+    """The partial sums [4, M, N] of the 32-bit a[M, K] @ w[N, K]^T: added up in order they are `gemm`'s result."""
+    _check(a, "a", F32, (None, None))
+    M, K = a.shape
+    rows = _rows(w)
+    _check(rows, "w", F32, (None, K))
+    N = rows.shape[0]
+    sums = torch.empty((F32_GROUPS, M, N), dtype=F32, device=a.device)
+    call("as_gemm_f32_split", _ptr(a), _ptr(rows), _ptr(sums), M, N, K, 0, _stream())
+    return sums
+
+
+def gemm_split_sums(a, w):
+    """a @ w^T as partial sums for whoever adds them up, or None where the product is better made whole (or has no such kernel)."""
+    M, K = a.shape
+    N = _rows(w).shape[0]
+    if a.dtype == F32:
+        return gemm_f32_split(a, w) if gemm_f32_split_preferred(M, N, K, w) and a.data_ptr() % 16 == 0 else None
+    plan = gemm_split_plan(M, N, K, a.dtype)
+    return None if plan is None else gemm_split(a, w, plan)
+
+
 GATED_MAX_K = 6144  # the widest input the fused product-and-activation kernel keeps in registers
 
 
@@ -1003,7 +1037,8 @@ def _gated_two_tiles(rows: int, k: int, w) -> bool:
 def gemm_silu_mul(a, w, out, choices=None) -> None:
     """out[M, I] = silu(a @ w[:I]^T) * (a @ w[I:]^T) for w[2 I, K]: the gate and up products and
     the activation.  bf16 with few rows: one kernel, the products rounded to bf16 before the
-    activation exactly as the two-kernel path does; otherwise the product, then the activation."""
+    activation exactly as the two-kernel path does; fp32 of more than 256 columns: one kernel, the same bits as
+    two (333 rows, 1,024 -> 6,144: 51 us, 51 and 5 for two); otherwise the product, then the activation."""
     _check(a, "a", (F32, BF16), (None, None))
     M, K = a.shape
     _check(out, "out", a.dtype, (M, None))
@@ -1011,6 +1046,9 @@ def gemm_silu_mul(a, w, out, choices=None) -> None:
     rows = _rows(w)
     _check(rows, "w", a.dtype, (2 * inter, K))
     if M == 0:
+        return
+    if a.dtype == F32 and K > F32_NARROW:
+        call("as_gemm_f32_gated", _ptr(a), _ptr(rows), _ptr(out), M, inter, K, 0, _stream())
         return
     if a.dtype == BF16 and (_few_rows(M, K, inter, GATED_MAX_K, w=w) or _gated_two_tiles(M, K, w)):
         call("as_gemm_bf16_gated", _ptr(a), _ptr(rows), _wave_ptr(w), _ptr(out), M, inter, K, _stream())

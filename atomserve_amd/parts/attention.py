@@ -124,9 +124,9 @@ class Attention(Mixer):
             if link is not None:
                 return link
             if next_norm.takes_split_sums:
-                plan = ops.gemm_split_plan(T, s.hidden_size, out.view(T, H * D).shape[1], env.dtype)
-                if plan is not None:
-                    return SplitSums(ops.gemm_split(out.view(T, H * D), self.o, plan))
+                sums = ops.gemm_split_sums(out.view(T, H * D), self.o)
+                if sums is not None:
+                    return SplitSums(sums)
         y = torch.empty((T, s.hidden_size), dtype=env.dtype, device=device)
         ops.gemm(out.view(T, H * D), self.o, y, env.products)
         return y

@@ -53,9 +53,9 @@ class GatedMLP(FeedForward):
             if link is not None:
                 return link
             if next_norm.takes_split_sums:
-                plan = ops.gemm_split_plan(T, s.hidden_size, act.shape[1], env.dtype)
-                if plan is not None:
-                    return SplitSums(ops.gemm_split(act, self.down, plan))
+                sums = ops.gemm_split_sums(act, self.down)
+                if sums is not None:
+                    return SplitSums(sums)
         y = torch.empty((T, s.hidden_size), dtype=env.dtype, device=device)
         ops.gemm(act, self.down, y, env.products)
         return y

@@ -1375,3 +1375,64 @@ def test_products_of_9_to_128_rows_in_tiles(ops, M, N, K):
         x3 = x.clone()
         ops.rmsnorm(x3, gain, 1e-5, sel, rows=rows, update_x=False, split_sums=sums)
         assert torch.equal(x3, x) and close_bf16(sel, out2[[M - 1, 0, 3]].double())
+
+
+def f32_product(name, a, w, out, form):
+    from atomserve_amd.kernels.lib import call
+
+    N = out.shape[-1]
+    call(name, a.data_ptr(), w.data_ptr(), out.data_ptr(), a.shape[0], N, a.shape[1], form, torch.cuda.current_stream().cuda_stream)
+    return out
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 32, 260), (4, 48, 1028), (5, 16, 512), (8, 80, 2080), (9, 36, 300), (16, 64, 3072), (17, 68, 1024),
+                                   (63, 128, 288), (65, 132, 1000), (129, 260, 2052), (200, 64, 544)])  # fmt: skip
+def test_gemm_f32_gated_and_split_are_the_plain_product(ops, M, N, K):
+    """Every kernel of the 32-bit product, whole, with the gated activation after it (the same bits as the activation's kernel) and
+    in four partial sums that a reader adds up in order: the same bits.  Bound: the six products of a step and the sums of a slice
+    and of the slices each round to 2^-24 of the sums of absolute values, three products of parts below 2^-24 are left out."""
+    torch.manual_seed(62)
+    a, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    blank = lambda *shape: torch.full(shape, float("nan"), device=DEV)  # noqa: E731
+    want = f32_product("as_gemm_f32", a, w, blank(M, N), 0)
+    for form in range(1, 9):
+        assert torch.equal(f32_product("as_gemm_f32", a, w, blank(M, N), form), want)
+    bound = (a.abs().double() @ w.abs().double().T) * (6 * (K / 512 + 1) + 22) * 2.0**-24
+    assert bool(((want.double() - a.double() @ w.double().T).abs() <= bound).all())
+    act = blank(M, N // 2)
+    ops.silu_mul(want, act)
+    for form in (0, 3, 5, 6, 7, 8):
+        assert torch.equal(f32_product("as_gemm_f32_gated", a, w, blank(M, N // 2), form), act)
+    for form in range(3):
+        s = f32_product("as_gemm_f32_split", a, w, blank(4, M, N), form)
+        assert torch.equal(((s[0] + s[1]) + s[2]) + s[3], want)
+
+
+@pytest.mark.parametrize("M,shift", [(3, 0), (16, 0), (70, 0), (6, 1)])
+def test_gemm_f32_numbers_that_are_not_finite(ops, M, shift):
+    """Infinities, NaN, numbers that round to infinity in 16 bits and tiny ones go where plain 32-bit arithmetic takes them, from every
+    kernel; the outputs that meet none keep the bits that they have without them."""
+    torch.manual_seed(63)
+    N, K = 70, 288
+    a, w = torch.randn(M * K + shift, device=DEV)[shift:].view(M, K), torch.randn(N * K + shift, device=DEV)[shift:].view(N, K)
+    clean = f32_product("as_gemm_f32", a, w, torch.empty(M, N, device=DEV), 0)
+    a[1, 5], a[2, 40] = float("inf"), float("nan")
+    a[0] = 0.0
+    a[0, 7], a[0, 8] = 3.4e38, 1e-38
+    w[3, 9], w[4, 5] = -float("inf"), 0.0
+    w[:, 7:9] = torch.rand(N, 2, device=DEV) * 0.5  # 3.4e38 times them is finite
+    ref = a.cpu() @ w.cpu().T
+    kind = lambda t: (torch.isnan(t), torch.isposinf(t), torch.isneginf(t))  # noqa: E731
+    for form in range(7 if shift else 9):  # the last two read rows that start on 16 bytes
+        out = f32_product("as_gemm_f32", a, w, torch.empty(M, N, device=DEV), form).cpu()
+        assert all(torch.equal(x, y) for x, y in zip(kind(out), kind(ref)))
+        ok = torch.isfinite(ref)
+        assert bool((out[0][ok[0]] - ref[0][ok[0]]).abs().le(1e-6 * ref[0][ok[0]].abs()).all())  # one product each, and its neighbour far below
+    if M > 3:
+        w2 = w.clone()
+        w2[:, 7:9] = torch.randn(N, 2, device=DEV)
+        after = f32_product("as_gemm_f32", a[3:], w2, torch.empty(M - 3, N, device=DEV), 0)
+        base = f32_product("as_gemm_f32", a[3:], torch.where(torch.isinf(w2), torch.zeros_like(w2), w2), torch.empty(M - 3, N, device=DEV), 0)
+        keep = [n for n in range(N) if n != 3]
+        assert torch.equal(after[:, keep], base[:, keep]) and bool(torch.isinf(after[:, 3]).all())
+    assert bool(torch.isfinite(clean).all())
