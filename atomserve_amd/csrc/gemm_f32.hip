@@ -291,7 +291,10 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
         float* xp = out + (size_t)m * N + n;
         v += *reinterpret_cast<floatx4*>(xp);
         *reinterpret_cast<floatx4*>(xp) = v;
-        *reinterpret_cast<floatx4*>(link.scaled + (size_t)m * N + n) = v * *reinterpret_cast<const floatx4*>(link.gain + n);
+        floatx4 g;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) g[r] = link.gain[n + r];
+        *reinterpret_cast<floatx4*>(link.scaled + (size_t)m * N + n) = v * g;
         ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
       }
       ss += __shfl_xor(ss, 16, 64);  // the four lanes that hold the strip's 16 columns of row m
@@ -559,7 +562,8 @@ struct F32Tile { int rows, columns; float alone_us, round_us; };
 static const F32Tile f32_forms[] = {{16, 16, 3.4f, 4.5f},   {16, 16, 4.5f, 3.6f},   {16, 32, 6.2f, 5.6f},    {32, 16, 5.5f, 7.4f},
                                     {32, 32, 7.8f, 9.f},    {64, 32, 12.f, 13.f},   {64, 64, 18.f, 14.5f},   {128, 128, 48.f, 48.f}};
 #define F32_FORMS 8
-#define F32_TILE_FORMS 6  // the first through LDS
+#define F32_TILE_FORMS 6    // the first through LDS
+#define F32_ONE_ROW_TILE 3  // so many of one row tile
 
 static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
   const long rounds = (f32_tiles(M, N, t.rows, t.columns) * split + compute_units() - 1) / compute_units();
@@ -568,17 +572,17 @@ static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
 }
 
 // form: 0: chosen here; else 1 + the index of a kernel (tests).
-template <int MODE> static int gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
+template <int MODE> static int gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, const LinkF32& link,
+                                        hipStream_t stream) {
   const bool vec = (K & 3) == 0 && aligned16(a, w);
   if (form == 0) {
     float best = 0.f;
-    for (int i = MODE == GATED ? 2 : 0; i < F32_FORMS; ++i) {
+    for (int i = MODE == GATED ? 2 : 0; i < (link.ssq_in ? F32_ONE_ROW_TILE : F32_FORMS); ++i) {
       if ((MODE == GATED && i == 3) || (i >= F32_TILE_FORMS && !vec)) continue;
       const float cost = f32_cost(f32_forms[i], M, MODE == GATED ? 2 * N : N, K, 1);
       if (form == 0 || cost < best) { best = cost; form = i + 1; }
     }
   }
-  const LinkF32 link{};
   if constexpr (MODE == GATED) {
     switch (form) {
       case 3:
@@ -617,7 +621,7 @@ extern "C" int as_gemm_f32(const float* a, const float* w, float* out, int M, in
     gemm_f32_narrow_kernel<<<grid, 256, 0, stream>>>(a, w, out, M, N, K);
     return launch_status();
   }
-  return gemm_f32<PLAIN>(a, w, out, M, N, K, form, stream);
+  return gemm_f32<PLAIN>(a, w, out, M, N, K, form, LinkF32{}, stream);
 }
 
 // out[M, N] = silu(a @ w[:N]^T) * (a @ w[N:]^T) for w[2 N, K].  K > F32_NARROW; the activation on the sums that the plain product
@@ -625,15 +629,44 @@ extern "C" int as_gemm_f32(const float* a, const float* w, float* out, int M, in
 extern "C" int as_gemm_f32_gated(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
   if (M <= 0) return AS_OK;
   if (N <= 0 || N > 0x3fffffff || K <= F32_NARROW || form < 0 || form > F32_FORMS) return AS_BAD_SHAPE;
-  return gemm_f32<GATED>(a, w, out, M, N, K, form, stream);
+  return gemm_f32<GATED>(a, w, out, M, N, K, form, LinkF32{}, stream);
+}
+
+// The producer of a LinkF32: x[M, N] += a @ w^T; scaled[M, N] = x * gain; ssq[M, ceil(N / 16)] = sums of x^2 per 16 columns.
+// M <= 16, K > F32_NARROW, N % 4 == 0, x and scaled on 16 bytes.
+extern "C" int as_gemm_f32_link(const float* a, const float* w, float* x, const float* gain, float* scaled, float* ssq, int M, int N, int K,
+                                hipStream_t stream) {
+  if (M <= 0) return AS_OK;
+  if (M > 16 || N <= 0 || (N & 3) || K <= F32_NARROW || !gain || !scaled || !ssq || !aligned16(x, scaled)) return AS_BAD_SHAPE;
+  const LinkF32 link{nullptr, 0, 0.f, gain, scaled, ssq};
+  return launch_few<1, 8, 4, LINK>(a, w, x, M, N, K, link, stream);
+}
+
+// The consumer of a LinkF32: out[M, N] = (scaled @ w^T) / rms(x) with rms from ssq[M, strips_in] (strips_in = ceil(K / 16)) and eps;
+// gated: silu of the first half of w's 2 N rows times the second half, both scaled first.  M <= 16, K > F32_NARROW.
+extern "C" int as_gemm_f32_scaled(const float* scaled, const float* ssq, int strips_in, float eps, const float* w, float* out, int M, int N,
+                                  int K, int gated, hipStream_t stream) {
+  if (M <= 0) return AS_OK;
+  if (M > 16 || N <= 0 || N > 0x3fffffff || K <= F32_NARROW || !ssq || strips_in != (K + 15) / 16) return AS_BAD_SHAPE;
+  const LinkF32 link{ssq, strips_in, eps, nullptr, nullptr, nullptr};
+  return gated ? gemm_f32<GATED>(scaled, w, out, M, N, K, 0, link, stream) : gemm_f32<PLAIN>(scaled, w, out, M, N, K, 0, link, stream);
 }
 
 // sums[4][M, N]: the product's sums over the four quarters of K's slices; added up in order they are the product, bit for bit.  For
-// products of too few outputs to fill the GPU: N = 1,024, K = 2,048 at 333 rows 17.8 us, whole 28.7.  K > F32_NARROW, K % 4 == 0,
-// N % 4 == 0, rows that start on 16 bytes.
+// products of too few outputs to fill the GPU: N = 1,024, K = 2,048 at 333 rows 17.7 us, whole 28.5.  K > F32_NARROW, K % 4 == 0,
+// N % 4 == 0.  Rows that do not start on 16 bytes: the product is made whole, three of the sums are zeros.
+__global__ __launch_bounds__(256) void zeros_kernel(float* __restrict__ out, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) out[i] = 0.f;
+}
+
 extern "C" int as_gemm_f32_split(const float* a, const float* w, float* sums, int M, int N, int K, int form, hipStream_t stream) {
   if (M <= 0) return AS_OK;
-  if (N <= 0 || (N & 3) || K <= F32_NARROW || form < 0 || form > 2) return AS_BAD_SHAPE;
+  if (N <= 0 || (N & 3) || K <= F32_NARROW || (K & 3) || form < 0 || form > 2) return AS_BAD_SHAPE;
+  if (!aligned16(a, w)) {
+    zeros_kernel<<<compute_units() * 4, 256, 0, stream>>>(sums + (size_t)M * N, (size_t)(F32_GROUPS - 1) * M * N);
+    const int rc = launch_status();
+    return rc != AS_OK ? rc : gemm_f32<PLAIN>(a, w, sums, M, N, K, 0, LinkF32{}, stream);
+  }
   if (form == 0) form = f32_cost(f32_forms[6], M, N, K, F32_GROUPS) <= f32_cost(f32_forms[7], M, N, K, F32_GROUPS) ? 1 : 2;
   if (form == 1) return launch_tile<4, 2, 1, 2, false, true>(a, w, sums, M, N, K, stream);
   return launch_tile<2, 4, 4, 2, false, true>(a, w, sums, M, N, K, stream);

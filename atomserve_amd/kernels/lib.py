@@ -83,6 +83,8 @@ SIGNATURES = {
     "as_attn_f32": ("attention", [P, P, P, P, I, I, P, I, P, P, P, I, P, P, P, P, I, I, I, I, F, I, I, I, F, I, P, I, I, I, P]),
     "as_gemm_f32": ("gemm_f32", [P, P, P, I, I, I, I, P]),
     "as_gemm_f32_gated": ("gemm_f32", [P, P, P, I, I, I, I, P]),
+    "as_gemm_f32_link": ("gemm_f32", [P, P, P, P, P, P, I, I, I, P]),
+    "as_gemm_f32_scaled": ("gemm_f32", [P, P, I, F, P, P, I, I, I, I, P]),
     "as_gemm_f32_split": ("gemm_f32", [P, P, P, I, I, I, I, P]),
     "as_gemm_bf16_skinny": ("gemm", [P, P, P, P, I, I, I, I, I, P]),
     "as_gemm_bf16_gated": ("gemm", [P, P, P, P, I, I, I, P]),

@@ -59,7 +59,8 @@ class RMSNorm(Norm):
 
     def absorb(self, a, w, x):
         M, N = x.shape
-        if not ops.gemm_link_supported(M, N, a.shape[1], self.env.dtype, w):
+        if not (ops.gemm_f32_link_supported(M, N, a.shape[1], x) if self.env.dtype == torch.float32
+                else ops.gemm_link_supported(M, N, a.shape[1], self.env.dtype, w)):  # fmt: skip
             return None
         scaled = torch.empty((M, N), dtype=self.env.dtype, device=x.device)
         ssq = torch.empty((M, -(-N // 16)), dtype=torch.float32, device=x.device)

@@ -1403,8 +1403,9 @@ def test_gemm_f32_gated_and_split_are_the_plain_product(ops, M, N, K):
     ops.silu_mul(want, act)
     for form in (0, 3, 5, 6, 7, 8):
         assert torch.equal(f32_product("as_gemm_f32_gated", a, w, blank(M, N // 2), form), act)
-    for form in range(3):
-        s = f32_product("as_gemm_f32_split", a, w, blank(4, M, N), form)
+    shifted = torch.empty(N * K + 1, device=DEV)[1:].view(N, K).copy_(w)
+    for form, rows in ((0, w), (1, w), (2, w), (0, shifted)):
+        s = f32_product("as_gemm_f32_split", a, rows, blank(4, M, N), form)
         assert torch.equal(((s[0] + s[1]) + s[2]) + s[3], want)
 
 
@@ -1436,3 +1437,38 @@ def test_gemm_f32_numbers_that_are_not_finite(ops, M, shift):
         keep = [n for n in range(N) if n != 3]
         assert torch.equal(after[:, keep], base[:, keep]) and bool(torch.isinf(after[:, 3]).all())
     assert bool(torch.isfinite(clean).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 260, 1024), (4, 1024, 2048), (5, 272, 300), (8, 1024, 3072), (9, 516, 288), (16, 2048, 6144)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gemm_link_and_scaled_f32(ops, M, N, K, shift):
+    """The residual sum and the norm folded into 32-bit products: x has the bits of the plain product on top, the sums of squares
+    are those of x within their rounding (16 columns), and the product of what is left, times 1 / rms, is that of the normed rows:
+    bounds from the sums of absolute values, two more roundings (x * gain, 1 / rms) of 2^-24 and the root's own."""
+    torch.manual_seed(64)
+    eps, L = 1e-6, 96
+    a, w = torch.randn(M, K, device=DEV), torch.randn(N * K + shift, device=DEV)[shift:].view(N, K) * 0.05
+    gain = torch.randn(N + 1, device=DEV)[shift : shift + N] * 0.1 + 1
+    x = torch.randn(M, N, device=DEV)
+    prod = torch.empty(M, N, device=DEV)
+    ops.gemm(a, w, prod)
+    want = x + prod
+    scaled, ssq = torch.empty(M, N, device=DEV), torch.empty(M, -(-N // 16), device=DEV)
+    assert ops.gemm_f32_link_supported(M, N, K, x)
+    ops.gemm_link(a, w, x, gain, scaled, ssq)
+    assert torch.equal(x, want) and torch.equal(scaled, x * gain)
+    squares = torch.nn.functional.pad(x.double().square(), (0, -N % 16)).view(M, -1, 16).sum(2)
+    assert bool(((ssq.double() - squares).abs() <= squares * 8 * 2.0**-24).all())
+    inv = 1 / (x.double().square().mean(1, keepdim=True) + eps).sqrt()
+    for gated in (False, True):
+        w2 = torch.randn((2 * L if gated else L) * N + shift, device=DEV)[shift:].view(-1, N) * 0.05
+        out = torch.full((M, L), float("nan"), device=DEV)
+        ops.gemm_scaled(scaled, ssq, eps, w2, out, gated=gated)
+        rows = x.double() * gain.double() * inv
+        ref, bound = rows @ w2.double().T, (rows.abs() @ w2.double().abs().T) * (6 * (N / 512 + 1) + 40) * 2.0**-24
+        if gated:
+            g, u = ref[:, :L], ref[:, L:]
+            ref = g * torch.sigmoid(g) * u
+            bound = 1.1 * bound[:, :L] * u.abs() + (g.abs() + bound[:, :L]) * bound[:, L:] + 8 * 2.0**-24 * ref.abs() + 1e-12
+        assert bool(((out.double() - ref).abs() <= bound).all())
+    assert not ops.gemm_f32_link_supported(17, N, K) and not ops.gemm_f32_link_supported(M, 256, K)
