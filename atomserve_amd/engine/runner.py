@@ -101,6 +101,10 @@ class DecodeGraphs:
     kernel is this package's; above, the matrix products are the library's, which replay
     correctly (checked against eager steps in the tests, several replays with eager work between).
 
+    The first context bucket of few rows comes in two forms: one for contexts of up to `SHORT_CONTEXT` tokens, whose
+    attention walks them whole, beside the one that cuts them into partitions which another kernel merges (one request
+    of 100 tokens at Qwen3-0.6B sizes: 936 us a step with the merge, 837 without; at 400 tokens both take as long).
+
     A step is captured on rows that pad only (they store nothing and use the state slot that belongs
     to nobody), so capturing, and the runs that warm it up, touch no request's cache or state; the
     real rows are packed into the captured buffer afterwards.  A model whose mixers keep a state of
@@ -109,16 +113,17 @@ class DecodeGraphs:
     All captured steps draw their intermediate tensors from one memory pool and write their logits
     into one buffer [largest bucket, vocab] (they never run at the same time; a step's logits are
     read, by the sampling kernels or a copy, before the next step of the same stream overwrites
-    them); at most `MAX_GRAPHS` are kept, the one replayed longest ago goes first.  `bytes_held`
+    them); at most `MAX_GRAPHS` buckets are kept, the one replayed longest ago goes first.  `bytes_held`
     is the memory the captures took from the device."""
 
     ROW_BUCKETS = (1, 2, 4, 8, 16, 32, 48, 64, 96, 128, 192, 256)
     CONTEXT_STEP = 1024
+    SHORT_CONTEXT, SHORT_ROWS = 256, 32  # with more rows the requests themselves fill the GPU and no context is cut
     MAX_GRAPHS = 64
 
     def __init__(self, runner):
         self.runner = runner
-        self.graphs = OrderedDict()  # (rows, context) -> (graph, its batch, its logits), least recently used first
+        self.graphs = OrderedDict()  # (rows, context) -> {longest context: (graph, its batch, its logits)}, least recently used first
         self.pool = None
         self.filler_tables = [[0] for _ in runner.manager.paged_groups]  # one object: a filler row is recognised
         self.logits = None  # [most_rows, vocab] fp32, shared by all captured steps
@@ -148,24 +153,27 @@ class DecodeGraphs:
         n = _bucket(len(rows), self.ROW_BUCKETS)
         longest = max(row.start + 1 for row in rows)
         context = -(-longest // self.CONTEXT_STEP) * self.CONTEXT_STEP
-        width = -(-context // bs)
+        bound = next(b for b in self._bounds(n, context) if longest <= b)
+        width = -(-bound // bs)
         # every row of the captured step yields logits; rows that want none are dropped after the replay
         padded = [row if row.want else Row(row.tokens, row.start, row.tables, [0], row.state_slot) for row in rows]
         padded += [self.filler() for _ in range(n - len(rows))]
         key = (n, context)
-        entry = self.graphs.get(key)
-        if entry is None:
+        forms = self.graphs.get(key)
+        if forms is None:
             while len(self.graphs) >= self.MAX_GRAPHS:
                 self.graphs.popitem(last=False)
-            entry = self.graphs[key] = self._capture(n, width, context)
-            fresh = True
+            forms = self.graphs[key] = {}
         else:
             self.graphs.move_to_end(key)
-            fresh = False
+        entry = forms.get(bound)
+        fresh = entry is None
+        if fresh:
+            entry = forms[bound] = self._capture(n, width, bound)
         if fresh or not entry[1].advance(padded):
             # other requests than last time, or a window moved: pack anew into the captured buffer
-            batch = r.prepare(padded, table_width=width, max_context=context, into=entry[1])
-            entry = self.graphs[key] = (entry[0], batch, entry[2])
+            batch = r.prepare(padded, table_width=width, max_context=bound, into=entry[1])
+            entry = forms[bound] = (entry[0], batch, entry[2])
         if tokens_from is not None:
             entry[1].token_ids[: len(rows)].copy_(tokens_from)
         graph, batch, logits = entry
@@ -177,6 +185,10 @@ class DecodeGraphs:
             return logits[: len(rows)]
         return logits[torch.tensor(wanted, dtype=torch.long, device=logits.device)] if wanted else logits[:0]
 
+
+    def _bounds(self, n: int, context: int) -> tuple:
+        """The longest contexts of the forms in which the bucket (n rows, contexts up to `context`) is captured."""
+        return (self.SHORT_CONTEXT, context) if context == self.CONTEXT_STEP and n <= self.SHORT_ROWS else (context,)
 
     def _capture(self, n: int, width: int, context: int):
         """Captures the decode step of `n` rows and contexts up to `context`, on padding rows."""
@@ -233,7 +245,7 @@ class DecodeGraphs:
         """Captures the decode step of every row bucket up to the one that holds `max_rows`, with rows that
         store nothing: a server does this once at its start instead of pausing (for tens of milliseconds)
         when a bucket is first met.  For every context bucket up to `max_context` if all of them fit among
-        the graphs that are kept, else for the first one only.  Returns how many graphs were captured."""
+        the graphs that are kept, else for the first one only.  Returns how many buckets were captured."""
         if not self.eligible([self.filler()]):
             return 0
         before = len(self.graphs)
@@ -245,8 +257,10 @@ class DecodeGraphs:
         bs = self.runner.manager.block_size
         for context in contexts:
             for n in row_buckets:
-                if (n, context) not in self.graphs:
-                    self.graphs[(n, context)] = self._capture(n, -(-context // bs), context)
+                forms = self.graphs.setdefault((n, context), {})
+                for bound in self._bounds(n, context):
+                    if bound not in forms:
+                        forms[bound] = self._capture(n, -(-bound // bs), bound)
         return len(self.graphs) - before
 
 

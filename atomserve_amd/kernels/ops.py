@@ -373,6 +373,11 @@ def attn_fill_groups() -> int:
 MFMA_PARTITIONS = (128, 256, 512, 1024, 2048)  # keys per workgroup of the matrix-core decode kernel
 
 
+# Microseconds of the merge's kernel beside what `_partition_cost` counts; whole contexts have none (16 heads on 8 kv heads, 1 request:
+# 100 keys 7.5 us whole and 10.9 in partitions of 128 with the merge, 256 keys 9.5 and 10.8, 400 keys 12.7 and 10.2).
+MERGE_LAUNCH = 4.1
+
+
 def _partition_cost(groups: int, span: int, part: int) -> float:
     """Microseconds, roughly, of the decode attention and its merge when `groups` (token, kv head) pairs
     cut `span` keys into partitions of `part`: a workgroup costs 4 us and 25 ns a key, two of them run
@@ -412,7 +417,7 @@ def _partitions(N, H, KV, D, max_context, window, mfma, part_size, device, keep_
             if groups >= attn_fill_groups():
                 part_size = -(-span // 32) * 32  # enough workgroups without partitions: no merge
             else:
-                part_size = min(MFMA_PARTITIONS, key=lambda part: _partition_cost(groups, span, part))
+                part_size = min(MFMA_PARTITIONS, key=lambda part: _partition_cost(groups, span, part) + (MERGE_LAUNCH if part < span else 0.0))
         else:
             groups, part_size = N * KV * max(1, (G + 7) // 8), 256
             while part_size < span and groups * math.ceil(span / part_size) > 2048:
@@ -1083,7 +1088,7 @@ def gemm_link_supported(rows: int, n_out: int, k: int, dtype, w=None) -> bool:
 def gemm_f32_link_supported(rows: int, n_out: int, k: int, x=None) -> bool:
     """Whether `gemm_link` and, for its result, `gemm_scaled` exist in 32 bits: one row tile, both products' sums in the
     order that is cut (their kernels; n_out is the width of the stream, which is the next product's input).  x: the stream, if known.
-    Four decode steps of 4 requests at Qwen3-0.6B sizes: 7,824 us without, 6,550 with (the norm's kernel takes 4.4 us)."""
+    Four decode steps of 4 requests at Qwen3-0.6B sizes: 7,824 us without, 7,258 with (the norm's kernel takes 4.4 us)."""
     return (0 < rows <= SKINNY_MAX_ROWS and k > F32_NARROW and n_out > F32_NARROW and n_out % 4 == 0
             and (x is None or x.data_ptr() % 16 == 0))  # fmt: skip
 

@@ -69,6 +69,18 @@ def test_how_single_queries_contexts_are_partitioned():
         ops._partitions(8, 32, 8, 128, 2048, 0, True, 100, "cpu")
 
 
+def test_short_contexts_are_walked_whole():
+    """Up to 256 keys a workgroup of a (token, kv head) pair is faster than partitions and their merge, whoever asks; the captured
+    step of few rows has a form for them."""
+    from atomserve_amd.engine.runner import DecodeGraphs
+
+    for rows in (1, 8, 32):
+        assert ops._partitions(rows, 16, 8, 128, 256, 0, True, None, "cpu")[1] == 1
+        assert ops._partitions(rows, 16, 8, 128, 512, 0, True, None, "cpu")[1] > 1
+    bounds = lambda n, context: DecodeGraphs._bounds(DecodeGraphs, n, context)  # noqa: E731
+    assert bounds(1, 1024) == bounds(32, 1024) == (256, 1024) and bounds(48, 1024) == (1024,) and bounds(1, 2048) == (2048,)
+
+
 def test_how_products_of_17_to_128_rows_are_tiled():
     """Tiles of 64 weight rows, K cut into as many ranges of whole chunks as fill the compute units; the gated
     product's tile width by what the longest path loads."""
