@@ -9,7 +9,9 @@
 // again); a portion of a prompt goes on from what the portion before left.  State tables are fp32
 // [slots, ...]; a row's state is written back only when `writes`.
 #include "common.h"
+#include "float_parts.h"
 #include "rows.h"
+#include <type_traits>
 
 #define CONV_MAX_TAPS 8
 
@@ -1161,6 +1163,129 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(const float* __restric
   }
 }
 
+// The same on the matrix cores, for parts of whole steps of 32 inputs: u and 32-bit weights as three bf16 parts each (six products
+// of a pair), bf16 weights as they are (three).  A workgroup takes 64 tokens by 64 outputs of both gates of one part and a
+// wave 16 of the outputs; every value is taken apart once a workgroup, on its way into LDS, and the next step's are loaded
+// while this one's are multiplied.  Three workgroups fit a compute unit (37 KB of LDS): they fill one another's waits, for a
+// workgroup's few steps (eight of a part of 256) end before a deep pipeline would have paid.  An output's sum is one pair of
+// chains over the steps in order, so it does not depend on what shares the launch.  A sum that is not finite is computed
+// again by multiply-adds (an infinity has no parts).  What bounds it: the
+// exponentials and divisions of the way out, about as much as the products and the taking apart.  1,500 tokens of 8 parts of
+// 256: 79 -> 38 us (bf16 weights 27), 2,048 of 16: 179 -> 99 (65), 20 of 8: 43 -> 14; the error of a against 64 bits 1.3e-7
+// -> 0.66e-7.
+// Places of 16 bytes (8 inputs of a row) in LDS as in the 32-bit products: row * 4 + (c ^ f(row / 4 % 4)), f = 0, 2, 3, 1.
+#define GATE_ROWS (GATE_TT + 2 * GATE_TO)
+__device__ __forceinline__ int gate_place(int row, int c) { return row * 4 + (c ^ (0x78 >> (row >> 1 & 6) & 3)); }
+
+template <typename W> __device__ float plain_dot(const float* u, const W* w, int n) {
+  float s = 0.f;
+  for (int k = 0; k < n; ++k) s = fmaf(to_f32(w[k]), u[k], s);
+  return s;
+}
+
+template <typename W>
+__global__ __launch_bounds__(256, 3) void rglru_gates_mfma_kernel(const float* __restrict__ u, int width, int bw,
+                                                               const W* __restrict__ ra, const W* __restrict__ ra_b,
+                                                               const W* __restrict__ ri, const W* __restrict__ ri_b,
+                                                               const W* __restrict__ lam, float c,
+                                                               float* __restrict__ a_out, float* __restrict__ x_out,
+                                                               int num_tokens) {
+  constexpr bool PARTED = sizeof(W) == 4;
+  __shared__ bf16x8 lds[3][GATE_ROWS * 4];
+  const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, lr = lane & 15, lg = lane >> 4;
+  const int b = blockIdx.y, t0 = blockIdx.x * GATE_TT, o0 = blockIdx.z * GATE_TO;
+  const int row = threadIdx.x >> 2, piece = threadIdx.x & 3;  // this thread brings 8 inputs of a token and of two outputs
+  const float* src_u = u + (size_t)min(t0 + row, num_tokens - 1) * width + b * bw + piece * 8;
+  const size_t at_w = ((size_t)b * bw + min(o0 + row, bw - 1)) * bw + piece * 8;
+  const W* src_w[2] = {ra + at_w, ri + at_w};
+  floatx4 au[2], aw[2][2];
+  bf16x8 whole[2];
+  auto load = [&](int k) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) au[h] = *reinterpret_cast<const floatx4*>(src_u + k + 4 * h);
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      if constexpr (PARTED) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) aw[g][h] = *reinterpret_cast<const floatx4*>(src_w[g] + k + 4 * h);
+      } else {
+        whole[g] = *reinterpret_cast<const bf16x8*>(src_w[g] + k);
+      }
+    }
+  };
+  auto place = [&](int to, const Parts& s) {
+    lds[0][to] = s.h;
+    lds[1][to] = s.m;
+    lds[2][to] = s.l;
+  };
+  floatx4 acc[2][4], low[2][4];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[g][j] = low[g][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  load(0);
+  for (int k = 0; k < bw; k += 32) {
+    __syncthreads();  // the step before has been read
+    place(gate_place(row, piece), parts(au[0], au[1]));
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int to = gate_place(GATE_TT + g * GATE_TO + row, piece);
+      if constexpr (PARTED) place(to, parts(aw[g][0], aw[g][1]));
+      else lds[0][to] = whole[g];
+    }
+    __syncthreads();
+    if (k + 32 < bw) load(k + 32);
+    Parts ws[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int from = gate_place(GATE_TT + g * GATE_TO + wave * 16 + lr, lg);
+      ws[g].h = lds[0][from];
+      if constexpr (PARTED) { ws[g].m = lds[1][from]; ws[g].l = lds[2][from]; }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int from = gate_place(j * 16 + lr, lg);
+      const Parts us = {lds[0][from], lds[1][from], lds[2][from]};
+#pragma unroll
+      for (int x = 0; x < 6; ++x) {
+        if (!PARTED && PART_W[x] != 0) continue;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          floatx4& to = x == 5 ? acc[g][j] : low[g][j];
+          to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part(ws[g], PART_W[x]), part(us, PART_A[x]), to, 0, 0, 0);
+        }
+      }
+    }
+  }
+  // a lane holds outputs o .. o+3 of token t0 + 16 j + lr
+  const int o = o0 + wave * 16 + 4 * lg, ch = b * bw + o;
+  if (o >= bw) return;  // bw is a multiple of 4
+  float rb[4], ib[4], sp[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) { rb[i] = to_f32(ra_b[ch + i]); ib[i] = to_f32(ri_b[ch + i]); sp[i] = softplusf_(to_f32(lam[ch + i])); }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int t = t0 + j * 16 + lr;
+    if (t >= num_tokens) continue;
+    floatx4 r = acc[0][j] + low[0][j], g = acc[1][j] + low[1][j], av, xv;
+    if (!finite(r) || !finite(g)) {
+      for (int i = 0; i < 4; ++i) {
+        r[i] = plain_dot(u + (size_t)t * width + b * bw, ra + (size_t)(ch + i) * bw, bw);
+        g[i] = plain_dot(u + (size_t)t * width + b * bw, ri + (size_t)(ch + i) * bw, bw);
+      }
+    }
+    const floatx4 uu = *reinterpret_cast<const floatx4*>(u + (size_t)t * width + ch);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float log_a = -c * sigmoidf_(r[i] + rb[i]) * sp[i];
+      av[i] = expf(log_a);
+      xv[i] = sqrtf(-expm1f(2.0f * log_a)) * sigmoidf_(g[i] + ib[i]) * uu[i];
+    }
+    *reinterpret_cast<floatx4*>(a_out + (size_t)t * width + ch) = av;
+    *reinterpret_cast<floatx4*>(x_out + (size_t)t * width + ch) = xv;
+  }
+}
+
 // The same for a few tokens (a decode step): the two matrices are streamed once.  Sixteen lanes share an
 // output channel (a wave four channels): each takes four inputs in sixteen (16-byte loads, a row of the
 // matrix read in whole lines), and their sums meet through DPP moves within the sixteen; eight tokens at a
@@ -1244,6 +1369,16 @@ extern "C" int as_rglru_gates(const float* u, int width, int blocks, const void*
   }
   dim3 grid((num_tokens + GATE_TT - 1) / GATE_TT, blocks, (bw + GATE_TO - 1) / GATE_TO);
   if (grid.z > 65535) return AS_BAD_SHAPE;
+  const uintptr_t starts = (uintptr_t)u | (uintptr_t)ra | (uintptr_t)ri | (uintptr_t)a_out | (uintptr_t)x_out;
+  if (bw % 32 == 0 && (starts & 15) == 0 && (w_dtype == DT_F32 || w_dtype == DT_BF16)) {  // whole steps of 16-byte pieces
+    if (w_dtype == DT_F32)
+      rglru_gates_mfma_kernel<float><<<grid, 256, 0, stream>>>(u, width, bw, (const float*)ra, (const float*)ra_b, (const float*)ri,
+                                                              (const float*)ri_b, (const float*)lam, c, a_out, x_out, num_tokens);
+    else
+      rglru_gates_mfma_kernel<bf16><<<grid, 256, 0, stream>>>(u, width, bw, (const bf16*)ra, (const bf16*)ra_b, (const bf16*)ri,
+                                                             (const bf16*)ri_b, (const bf16*)lam, c, a_out, x_out, num_tokens);
+    return launch_status();
+  }
   if (w_dtype == DT_F32)
     rglru_gates_kernel<float><<<grid, 256, 0, stream>>>(u, width, bw, (const float*)ra, (const float*)ra_b,
                                                         (const float*)ri, (const float*)ri_b, (const float*)lam, c,
@@ -1258,63 +1393,151 @@ extern "C" int as_rglru_gates(const float* u, int width, int blocks, const void*
 
 // The scan: S = a S + x per channel, from zero at the start of a sequence; what leaves is
 // scale * S * gelu_tanh(y + y_bias) with y from proj [T, ld] at y_off, into out [T, ld_out] at out_off.
-// A workgroup owns 64 channels of a row and cuts the row's tokens into SCAN_SEGS equal stretches, a wave
-// each: every wave first runs its stretch from zero (keeping the product of its decays and what it ends
-// with), the stretches' ends are chained in LDS in order, and every wave runs its stretch again from its
-// true start, now writing.  The chain of dependent steps is a row's length / 8 instead of its length.
-#define SCAN_SEGS 16
+// A workgroup owns 16 channels of a row and takes its tokens 1,024 at a time, a thread up to 16 neighbouring ones of one channel
+// (a shorter row's are dealt evenly to the 64 threads of a channel): it loads them all at once, composes them from the identity (the product of the decays and what the stretch ends with), the
+// stretches are chained (four of a wave by lane moves, the waves' through LDS), and the thread runs its tokens again, out of
+// its registers, from their true start.  Every input is read once, and the chain of dependent steps is 16 + 2 + 16 a thousand
+// tokens.  Neighbouring workgroups of an XCD take neighbouring channels, so that a 128-byte line of two workgroups'
+// channels enters one L2.  1,500 tokens of 2,048 channels 56 -> 18 us (45 MB: 2.5 TB/s; half of the compute units hold a
+// workgroup), 2,048 of 4,096 80 -> 28, 300 of 1,024 11.1 -> 5.7; with 16 waves' sixteenths of the row, every input read twice.
+
+// Channel c of a row, token by token: rows of one token (a decode step), whose single step gives the same values either way.
 template <typename T, typename W>
-__global__ __launch_bounds__(64 * SCAN_SEGS) void rglru_scan_kernel(
-    const float* __restrict__ a, const float* __restrict__ x, int width, const T* __restrict__ proj, int ld, int y_off,
-    const W* __restrict__ y_bias, float scale, float* __restrict__ state, const int* __restrict__ row_first,
-    const int* __restrict__ row_len, const int* __restrict__ row_start, const int* __restrict__ row_slots, int writes,
-    T* __restrict__ out, int ld_out, int out_off) {
-  __shared__ float seg_a[SCAN_SEGS][WAVE], seg_b[SCAN_SEGS][WAVE];
-  const int lane = threadIdx.x & (WAVE - 1), seg = threadIdx.x / WAVE;
-  const int r = blockIdx.y, c = blockIdx.x * WAVE + lane;
-  const bool live = c < width;
-  const int first = row_first[r], len = row_len[r], slot = row_slots[r];
-  const int per = (len + SCAN_SEGS - 1) / SCAN_SEGS;
-  const int lo = min(len, seg * per), hi = min(len, lo + per);
-  float A = 1.f, B = 0.f;
-  if (live) {
-#pragma unroll 4
-    for (int j = lo; j < hi; ++j) {
-      const size_t t = (size_t)first + j;
-      const float av = a[t * width + c];
-      B = fmaf(av, B, x[t * width + c]);
-      A *= av;
-    }
-  }
-  seg_a[seg][lane] = A;
-  seg_b[seg][lane] = B;
-  __syncthreads();
-  if (!live) return;
-  float* mine = state + (size_t)(slot < 0 ? 0 : slot) * width + c;
-  float S = (row_start[r] > 0 && slot >= 0) ? *mine : 0.f;
-  for (int s = 0; s < seg; ++s) S = fmaf(seg_a[s][lane], S, seg_b[s][lane]);
+__device__ __forceinline__ void rglru_step(const float* __restrict__ a, const float* __restrict__ x, int width, const T* __restrict__ proj,
+                                           int ld, int y_off, const W* __restrict__ y_bias, float scale, float* __restrict__ state, int first,
+                                           int len, int start, int slot, int writes, T* __restrict__ out, int ld_out, int out_off, int c) {
+  float* held = state + (size_t)(slot < 0 ? 0 : slot) * width + c;
+  float S = (start > 0 && slot >= 0) ? *held : 0.f;
   const float yb = y_bias ? to_f32(y_bias[c]) : 0.f;
-#pragma unroll 4
-  for (int j = lo; j < hi; ++j) {
+  for (int j = 0; j < len; ++j) {
     const size_t t = (size_t)first + j;
     S = fmaf(a[t * width + c], S, x[t * width + c]);
     out[t * ld_out + out_off + c] = from_f32<T>(scale * S * gelu_tanhf_(to_f32(proj[t * ld + y_off + c]) + yb));
   }
-  if (writes && slot >= 0 && seg == SCAN_SEGS - 1) *mine = S;  // the last stretch ends where the row ends
+  if (writes && slot >= 0) *held = S;
 }
 
+#define SCAN_TOKENS 16   // a thread's
+#define SCAN_CHANNELS 16
+#define SCAN_WAVES 16
+template <typename T, typename W>
+__global__ __launch_bounds__(64 * SCAN_WAVES) void rglru_scan_kernel(
+    const float* __restrict__ a, const float* __restrict__ x, int width, const T* __restrict__ proj, int ld, int y_off,
+    const W* __restrict__ y_bias, float scale, float* __restrict__ state, const int* __restrict__ row_first,
+    const int* __restrict__ row_len, const int* __restrict__ row_start, const int* __restrict__ row_slots, int writes,
+    T* __restrict__ out, int ld_out, int out_off, int tiles, int per_xcd) {
+  __shared__ float ends[2][2][SCAN_WAVES][SCAN_CHANNELS];  // [round % 2][decays, ends]
+  const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+  const int ch = lane & (SCAN_CHANNELS - 1), sub = lane / SCAN_CHANNELS;  // four stretches a wave
+  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (tile >= tiles) return;
+  const int r = blockIdx.y, len = row_len[r];
+  if (len <= 1) {  // a decoding row beside a portion: a thread a channel, so that most of the row's workgroups end here
+    const int one = tile * WAVE * SCAN_WAVES + threadIdx.x;
+    if (one < width)
+      rglru_step(a, x, width, proj, ld, y_off, y_bias, scale, state, row_first[r], len, row_start[r], row_slots[r], writes, out, ld_out, out_off, one);
+    return;
+  }
+  const int mine = tile * SCAN_CHANNELS + ch, c = min(mine, width - 1);
+  const int first = row_first[r], slot = row_slots[r];
+  float* held = state + (size_t)(slot < 0 ? 0 : slot) * width + c;
+  float S = (row_start[r] > 0 && slot >= 0) ? *held : 0.f;  // the state where the round begins
+  const float yb = y_bias ? to_f32(y_bias[c]) : 0.f;
+  const int per = min(SCAN_TOKENS, (len + 4 * SCAN_WAVES - 1) / (4 * SCAN_WAVES));
+  // a thread's tokens in a straight line, as many as the row's length asks for (tests between them would make every load wait)
+  auto walk = [&](auto most) {
+    constexpr int N = decltype(most)::value;
+    int buf = 0;
+    for (int base = 0; base < len; base += SCAN_TOKENS * 4 * SCAN_WAVES, buf ^= 1) {
+      const int lo = base + (wave * 4 + sub) * per, mine_n = min(per, len - lo);  // tokens of this stretch, if any
+      float av[N], xv[N], yv[N];
+      if (mine_n > 0) {  // places beyond the row repeat its last token and count as the identity
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const size_t t = (size_t)first + lo + min(i, mine_n - 1);
+          av[i] = a[t * width + c];
+          xv[i] = x[t * width + c];
+          yv[i] = to_f32(proj[t * ld + y_off + c]);
+        }
+      }
+      float A = 1.f, B = 0.f;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        if (i < mine_n) {
+          B = fmaf(av[i], B, xv[i]);
+          A *= av[i];
+        }
+      }
+#pragma unroll
+      for (int off = SCAN_CHANNELS; off < WAVE; off *= 2) {  // with the stretches before it in the wave
+        const float Ab = __shfl_up(A, off, WAVE), Bb = __shfl_up(B, off, WAVE);
+        if (lane >= off) {
+          B = fmaf(A, Bb, B);
+          A *= Ab;
+        }
+      }
+      if (sub == 3) {
+        ends[buf][0][wave][ch] = A;
+        ends[buf][1][wave][ch] = B;
+      }
+      float Ae = __shfl_up(A, SCAN_CHANNELS, WAVE), Be = __shfl_up(B, SCAN_CHANNELS, WAVE);
+      if (sub == 0) { Ae = 1.f; Be = 0.f; }
+      __syncthreads();  // the next round writes the other half; the one after it comes behind the next round's barrier
+      float s = S;
+#pragma unroll
+      for (int w = 0; w < SCAN_WAVES; ++w) {
+        if (w == wave) s = S;
+        S = fmaf(ends[buf][0][w][ch], S, ends[buf][1][w][ch]);
+      }
+      s = fmaf(Ae, s, Be);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        if (i < mine_n) {
+          s = fmaf(av[i], s, xv[i]);
+          if (mine < width)
+            out[((size_t)first + lo + i) * ld_out + out_off + c] = from_f32<T>(scale * s * gelu_tanhf_(yv[i] + yb));
+        }
+      }
+    }
+  };
+  if (per > 8) walk(std::integral_constant<int, 16>{});
+  else if (per > 4) walk(std::integral_constant<int, 8>{});
+  else if (per > 2) walk(std::integral_constant<int, 4>{});
+  else walk(std::integral_constant<int, 2>{});
+  if (writes && slot >= 0 && threadIdx.x < SCAN_CHANNELS && mine < width) *held = S;
+}
+
+template <typename T, typename W>
+__global__ __launch_bounds__(WAVE) void rglru_step_kernel(
+    const float* __restrict__ a, const float* __restrict__ x, int width, const T* __restrict__ proj, int ld, int y_off,
+    const W* __restrict__ y_bias, float scale, float* __restrict__ state, const int* __restrict__ row_first,
+    const int* __restrict__ row_len, const int* __restrict__ row_start, const int* __restrict__ row_slots, int writes,
+    T* __restrict__ out, int ld_out, int out_off) {
+  const int r = blockIdx.y, c = blockIdx.x * WAVE + threadIdx.x;
+  if (c < width)
+    rglru_step(a, x, width, proj, ld, y_off, y_bias, scale, state, row_first[r], row_len[r], row_start[r], row_slots[r], writes, out,
+               ld_out, out_off, c);
+}
+
+// num_tokens: of the whole step; as many as rows: every row has one.
 extern "C" int as_rglru_scan(const float* a, const float* x, int width, const void* proj, int dtype, int ld, int y_off,
                              const void* y_bias, int w_dtype, float scale, float* state, const int* row_first,
                              const int* row_len, const int* row_start, const int* row_slots, int writes, void* out,
-                             int ld_out, int out_off, int num_rows, hipStream_t stream) {
+                             int ld_out, int out_off, int num_rows, int num_tokens, hipStream_t stream) {
   if (num_rows <= 0) return AS_OK;
   if (width <= 0 || num_rows > 65535 || ld < y_off + width || ld_out < out_off + width) return AS_BAD_SHAPE;
-  const int threads = WAVE * SCAN_SEGS;
-  dim3 grid((width + WAVE - 1) / WAVE, num_rows);
-#define LAUNCH(T, W)                                                                                              \
-  rglru_scan_kernel<T, W><<<grid, threads, 0, stream>>>(a, x, width, (const T*)proj, ld, y_off, (const W*)y_bias, \
-                                                        scale, state, row_first, row_len, row_start, row_slots,  \
-                                                        writes, (T*)out, ld_out, out_off)
+  const int tiles = (width + SCAN_CHANNELS - 1) / SCAN_CHANNELS, per_xcd = (tiles + 7) / 8;
+#define LAUNCH(T, W)                                                                                                     \
+  do {                                                                                                                   \
+    if (num_tokens == num_rows)                                                                                          \
+      rglru_step_kernel<T, W><<<dim3((width + WAVE - 1) / WAVE, num_rows), WAVE, 0, stream>>>(                           \
+          a, x, width, (const T*)proj, ld, y_off, (const W*)y_bias, scale, state, row_first, row_len, row_start,         \
+          row_slots, writes, (T*)out, ld_out, out_off);                                                                  \
+    else                                                                                                                 \
+      rglru_scan_kernel<T, W><<<dim3(per_xcd * 8, num_rows), WAVE * SCAN_WAVES, 0, stream>>>(                            \
+          a, x, width, (const T*)proj, ld, y_off, (const W*)y_bias, scale, state, row_first, row_len, row_start,         \
+          row_slots, writes, (T*)out, ld_out, out_off, tiles, per_xcd);                                                  \
+  } while (0)
   if (dtype == DT_F32 && w_dtype == DT_F32) LAUNCH(float, float);
   else if (dtype == DT_BF16 && w_dtype == DT_BF16) LAUNCH(bf16, bf16);
   else if (dtype == DT_BF16 && w_dtype == DT_F32) LAUNCH(bf16, float);

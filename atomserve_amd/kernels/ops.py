@@ -1936,7 +1936,7 @@ def rglru_scan(a, x, proj, y_off, y_bias, scale, state, step_rows, out, out_off,
     _, row_first, row_len, row_start, row_slots = step_rows
     call("as_rglru_scan", _ptr(a), _ptr(x), width, _ptr(proj), _DT[proj.dtype], proj.shape[1], y_off, _ptr(y_bias),
          _DT[w_dtype], float(scale), _ptr(state), _ptr(row_first), _ptr(row_len), _ptr(row_start), _ptr(row_slots),
-         int(bool(writes)), _ptr(out), out.shape[1], out_off, R, _stream())  # fmt: skip
+         int(bool(writes)), _ptr(out), out.shape[1], out_off, R, T, _stream())  # fmt: skip
 
 
 # ---- experts ------------------------------------------------------------------------------------------

@@ -633,3 +633,79 @@ def test_the_command_line_generates_from_a_folder(tmp_path, capsys):
     assert code == 0
     lines = [json.loads(line) for line in capsys.readouterr().out.splitlines() if line.startswith("{")]
     assert lines[-1]["output_ids"] == plain.greedy(raw, weights, prompt, 5)
+
+
+# ---- the gated linear recurrence's kernels alone ---------------------------------------------------------
+
+
+@pytest.mark.parametrize("tokens, blocks, bw, dtype", [(17, 3, 32, "float32"), (64, 2, 64, "float32"), (65, 1, 96, "bfloat16"),
+                                                       (130, 2, 160, "bfloat16"), (333, 4, 256, "float32"), (40, 2, 36, "float32")])  # fmt: skip
+def test_gates_of_a_linear_recurrence(tokens, blocks, bw, dtype):
+    """Parts of whole steps of 32 inputs (the matrix cores), edges of token and output tiles, and one that is none.  An infinity
+    and a NaN reach the outputs of their token and part alone."""
+    from atomserve_amd.kernels import ops
+
+    gen = torch.Generator().manual_seed(tokens)
+    width, W = blocks * bw, DTYPES[dtype]
+    u = torch.randn(tokens, width, generator=gen)
+    u[3, 1], u[tokens - 1, width - 1] = float("inf"), float("nan")
+    ra, ri = (torch.randn(blocks, bw, bw, generator=gen).mul(0.1).to(W) for _ in range(2))
+    ra_b, ri_b, lam = (torch.randn(width, generator=gen).to(W) for _ in range(3))
+    a, x = torch.empty(tokens, width, device=DEV), torch.empty(tokens, width, device=DEV)
+    ops.rglru_gates(u.to(DEV), *(t.to(DEV) for t in (ra, ra_b, ri, ri_b, lam)), 8.0, a, x)
+    ub = u.double().view(tokens, blocks, bw)
+    r, i = (torch.sigmoid(torch.stack([ub[:, b] @ w[b].double().T for b in range(blocks)], 1).reshape(tokens, width) + v.double())
+            for w, v in ((ra, ra_b), (ri, ri_b)))  # fmt: skip
+    log_a = -8.0 * r * torch.nn.functional.softplus(lam.double())
+    for got, want in ((a, log_a.exp()), (x, torch.sqrt(-torch.expm1(2 * log_a)) * i * u.double())):
+        got = got.cpu().double()
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        fine = want.isfinite()
+        # sums of up to 256 products of 0.1 rms: 17 roundings of 2^-24 of at most 40 in all; a gate moves by a quarter of that, log_a
+        # by up to 8 * 3 times a gate, and exp(log_a) by at most 1 / e of its relative change
+        assert (got - want)[fine].abs().max() <= 2e-5 * max(1.0, want[fine].abs().max())
+
+
+@pytest.mark.parametrize("width", [16, 100, 2048])
+@pytest.mark.parametrize("dtype, bias", [("float32", "float32"), ("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("bfloat16", None)])
+def test_scan_of_a_linear_recurrence(width, dtype, bias):
+    """Rows around a thread's 16 tokens, a wave's 64 and a round's 1,024, from zero and from a state; a row of one token gives the
+    same bits alone (the step kernel) as beside the others."""
+    from atomserve_amd.kernels import ops
+
+    lens = [1, 15, 16, 17, 64, 65, 1023, 1024, 1025, 2100, 1]
+    starts = [7, 0, 5, 0, 9, 0, 3, 0, 4, 8, 0]
+    gen, T, T_dtype = torch.Generator().manual_seed(width), sum(lens), DTYPES[dtype]
+    a = torch.rand(T, width, generator=gen) * 0.2 + 0.8
+    x = torch.randn(T, width, generator=gen)
+    proj = torch.randn(T, width + 24, generator=gen).to(T_dtype)
+    yb = None if bias is None else torch.randn(width, generator=gen).to(DTYPES[bias])
+    state = torch.randn(len(lens) + 1, width, generator=gen)
+    first = [sum(lens[:i]) for i in range(len(lens))]
+
+    def run(rows):
+        meta = [torch.tensor([v[i] for i in rows], dtype=torch.int32, device=DEV) for v in (lens, starts, list(range(len(lens))))]
+        own_first = torch.tensor([sum(lens[j] for j in rows[:n]) for n in range(len(rows))], dtype=torch.int32, device=DEV)
+        take = torch.cat([torch.arange(first[i], first[i] + lens[i]) for i in rows])
+        st, out = state.to(DEV), torch.zeros(len(take), width + 8, dtype=T_dtype, device=DEV)
+        ops.rglru_scan(a[take].to(DEV), x[take].to(DEV), proj[take].to(DEV), 24, None if yb is None else yb.to(DEV), 0.5, st,
+                       (None, own_first, meta[0], meta[1], meta[2]), out, 8)  # fmt: skip
+        return out.cpu(), st.cpu()
+
+    out, st = run(list(range(len(lens))))
+    one, st_one = run([0, 10])
+    assert torch.equal(one, out[[0, T - 1]]) and torch.equal(st_one[[0, 10]], st[[0, 10]]) and torch.equal(st[-1], state[-1])
+    assert out[:, :8].abs().max() == 0
+    for i, n in enumerate(lens):
+        s = state[i].double() if starts[i] > 0 else torch.zeros(width, dtype=torch.float64)
+        want = torch.empty(n, width, dtype=torch.float64)
+        for t in range(n):
+            s = a[first[i] + t].double() * s + x[first[i] + t].double()
+            want[t] = s
+        # 1 / (1 - a) is 10 on average: some tens of roundings of 2^-24 of values of a few
+        assert (st[i].double() - s).abs().max() <= 5e-6 * max(1.0, s.abs().max())
+        z = proj[first[i] : first[i] + n, 24:].double() + (0 if yb is None else yb.double())
+        gelu = 0.5 * z * (1 + torch.tanh(math.sqrt(2 / math.pi) * (z + 0.044715 * z**3)))
+        want = 0.5 * want * gelu
+        tol = 1e-5 if dtype == "float32" else 2.0**-8
+        assert ((out[first[i] : first[i] + n, 8:].double() - want).abs() <= tol * want.abs() + 1e-5).all()
