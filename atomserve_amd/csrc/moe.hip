@@ -3,7 +3,7 @@
 // Which experts a token uses is decided on the GPU (a table indexed by the token id here), so a step
 // never waits for the host and can be replayed as a graph.  A (token, chosen expert) is a "pair":
 // pair p = token * top + choice.  `moe_route` sorts the pairs by expert and cuts every expert's run
-// into tiles of up to 64; the two grouped products then take one workgroup per (tile, 64 outputs): the first
+// into tiles of up to 128; the two grouped products then take one workgroup per (tile or half of it, strip of outputs): the first
 // applies act(gate) * up on the way out, the second writes every pair's output where the pair stands
 // (so the outputs of a token's experts lie side by side), and `moe_combine` adds them up with their
 // weights.  A pair's result does not depend on what else is in the step: every output is a dot product
@@ -11,7 +11,8 @@
 #include "common.h"
 #include <type_traits>
 
-#define MOE_TILE 64      // pairs of one expert that a workgroup takes (four column tiles of 16)
+#define MOE_TILE 128     // pairs of one expert that a tile holds at most (eight column tiles of 16); a route has tiles of 64 or 128
+#define MOE_HALF 64      // four column tiles
 #define MOE_KC 128       // inputs per round: the tile's activations of a round meet in LDS
 #define MOE_STRIP 64     // outputs that a workgroup takes: four waves of 16
 #define MOE_MAX_EXPERTS 1024
@@ -22,7 +23,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));  // 16 bytes as 
 
 // ---- routing ------------------------------------------------------------------------------------
 // table [vocab, top] int32: the experts of every token id.  order [P]: the pairs sorted by expert;
-// tiles [max_tiles, 3]: (expert, first place in `order`, count <= 64); counts[0] = number of tiles.
+// tiles [max_tiles, 3]: (expert, first place in `order`, count <= `size`, 64 or 128); counts[0] = number of tiles.
 // One workgroup; the order of pairs within an expert is whatever the atomics make it, which no
 // result depends on.
 // With token_ids null, `table` is [P]: the expert of every pair as a router's kernel left it.  identity > 0: the numbers
@@ -45,7 +46,7 @@ __global__ __launch_bounds__(1024) void moe_route_table_kernel(const int* __rest
                                                                const int* __restrict__ table, int vocab, int top,
                                                                int experts, int num_tokens, int* __restrict__ order,
                                                                int* __restrict__ tiles, int* __restrict__ counts,
-                                                               int max_tiles, int identity) {
+                                                               int max_tiles, int identity, int size) {
   __shared__ int hist[MOE_MAX_EXPERTS];
   __shared__ int cursor[MOE_MAX_EXPERTS];
   const int P = num_tokens * top;
@@ -60,10 +61,10 @@ __global__ __launch_bounds__(1024) void moe_route_table_kernel(const int* __rest
     int at = 0, n = 0;
     for (int e = 0; e < experts; ++e) {
       cursor[e] = at;
-      for (int s = 0; s < hist[e] && n < max_tiles; s += MOE_TILE, ++n) {
+      for (int s = 0; s < hist[e] && n < max_tiles; s += size, ++n) {
         tiles[3 * n] = e;
         tiles[3 * n + 1] = at + s;
-        tiles[3 * n + 2] = min(MOE_TILE, hist[e] - s);
+        tiles[3 * n + 2] = min(size, hist[e] - s);
       }
       at += hist[e];
     }
@@ -259,12 +260,13 @@ extern "C" int as_moe_route_scores(const void* h, const void* router, const floa
 
 extern "C" int as_moe_route_table(const int* token_ids, const int* table, int vocab, int top, int experts,
                                   int num_tokens, int* order, int* tiles, int* counts, int max_tiles, int identity,
-                                  hipStream_t stream) {
+                                  int size, hipStream_t stream) {
   if (num_tokens <= 0) return AS_OK;
   if (top <= 0 || experts <= 0 || experts > MOE_MAX_EXPERTS || (token_ids && vocab <= 0)) return AS_BAD_SHAPE;
-  if (max_tiles < (num_tokens * top + MOE_TILE - 1) / MOE_TILE + experts) return AS_BAD_SHAPE;
+  if (size != MOE_HALF && size != MOE_TILE) return AS_BAD_SHAPE;
+  if (max_tiles < (num_tokens * top + size - 1) / size + experts) return AS_BAD_SHAPE;
   moe_route_table_kernel<<<1, 1024, 0, stream>>>(token_ids, table, vocab, top, experts, num_tokens, order, tiles,
-                                                 counts, max_tiles, identity);
+                                                 counts, max_tiles, identity, size);
   return launch_status();
 }
 
@@ -309,17 +311,18 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(const bf16* __restri
                                                             float limit) {
   constexpr int WROWS = GATED ? 2 * MOE_STRIP : MOE_STRIP;  // weight rows of a round: the strip's, then their up rows
   constexpr int WLOADS = WROWS * (MOE_KC / 8) / 256;        // 16-byte pieces of them per thread
-  __shared__ __attribute__((aligned(16))) bf16 acts[MOE_TILE][MOE_KC + 8];
+  __shared__ __attribute__((aligned(16))) bf16 acts[MOE_HALF][MOE_KC + 8];
   __shared__ __attribute__((aligned(16))) bf16 wts[WROWS][MOE_KC + 8];
-  __shared__ int pair_of[MOE_TILE];
-  const int tile = blockIdx.y;
+  __shared__ int pair_of[MOE_HALF];
+  const int tile = blockIdx.y, skip = blockIdx.z * MOE_HALF;  // a tile of 128 in halves
   if (tile >= counts[0]) return;
-  const int e = tiles[3 * tile], at = tiles[3 * tile + 1], cnt = tiles[3 * tile + 2];
+  const int e = tiles[3 * tile], at = tiles[3 * tile + 1] + skip, cnt = min(tiles[3 * tile + 2] - skip, MOE_HALF);
+  if (cnt <= 0) return;
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
   const int lr = lane & 15, lg = lane >> 4;
   const int nb = blockIdx.x * MOE_STRIP, n0 = nb + wave * 16;
   const int col_tiles = (cnt + 15) >> 4;
-  if (threadIdx.x < MOE_TILE) pair_of[threadIdx.x] = threadIdx.x < cnt ? order[at + threadIdx.x] : -1;
+  if (threadIdx.x < MOE_HALF) pair_of[threadIdx.x] = threadIdx.x < cnt ? order[at + threadIdx.x] : -1;
   __syncthreads();
   const int NW = GATED ? 2 * N : N;
   const bf16* wbase = w + (size_t)e * NW * K;
@@ -419,6 +422,173 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(const bf16* __restri
   }
 }
 
+// The same where K comes in whole blocks of 128 columns and outputs in strips of 16 (and everything on 16 bytes): the weights go
+// straight from memory into registers, for no wave needs another's rows; only the tile's activations, which all waves multiply
+// with, meet in LDS (a chunk in use and the one before, through registers one chunk ahead).  A wave owns two strips of 16 weight
+// rows (GATED: a gate strip and its up strip; few pairs of a product without a gate: one).  A lane takes 32 neighbouring
+// bytes of its row, the two halves of a step of 64 columns (the columns of a step permuted alike for both operands), so that a
+// wave's two loads use whole lines.  Weights' loads go through a buffer descriptor of the expert's matrix: those for chunks past
+// the last are sent beyond its end, where they move nothing, and the number of loads in flight is the same everywhere.
+// Workgroups start at different blocks of columns and wrap round, so that they do not all ask for the same memory channels.
+// WIDE: tiles of 128 pairs by 8 waves.  What bounds a prompt's product is what the compute units load, weights and
+//   activations together, most of it from L2: the larger the tile, the less (1,500 tokens of 2 of 16 experts, width 2,048, gate
+//   and up of 1,536: 950 MB in tiles of 64 x 128, 550 in tiles of 128 x 256).  An XCD takes a run of neighbouring (strip,
+//   tile) places, so that the tiles of one expert read a strip from one L2.
+// else: tiles of 64 by 4 waves, weights two chunks of 128 ahead: few pairs, for which the weights are streamed.
+// Both add up an output's products in one order, which depends on the output and its expert alone.
+// Two of 16 experts, both products of a layer, us before (every operand through LDS, tiles of 64 x 64) and now: width 4,096, 8 tokens
+// 155 and 144, 32 255 and 207 (6.0 and 5.5 TB/s of weights), 512 313 and 272, 2,048 752 and 544 (600 TFLOP/s); width 2,048,
+// 1,500 tokens 183 and 126; width 1,024, 300 tokens 32 and 27.
+enum { MOE_PLAIN, MOE_GATED, MOE_RELU2 };
+
+template <int MODE, typename OutT, bool WIDE>
+__global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 4 : 2) void moe_gemm_stream_kernel(
+    const bf16* __restrict__ a, int a_div, const bf16* __restrict__ w, int N, int K, const int* __restrict__ order,
+    const int* __restrict__ tiles, const int* __restrict__ counts, OutT* __restrict__ out, float limit, int strips) {
+  constexpr bool GATED = MODE == MOE_GATED;
+  constexpr int WAVES = WIDE ? 8 : 4, S = GATED || WIDE ? 2 : 1;  // waves, strips of weight rows a wave
+  constexpr int ACROSS = WAVES * 16 * (GATED ? 1 : S);             // outputs a workgroup
+  constexpr int KC = WIDE ? 64 : 128, STEPS = KC / 64, PIECES = KC / 8;
+  constexpr int MOST = WIDE ? MOE_TILE : MOE_TILE / 2, PASS = WAVES * 64 / PIECES;  // pairs; rows the threads bring at once
+  constexpr unsigned BEYOND = 0xfffffff0u;
+  __shared__ u32x4 lds[2][MOST * PIECES];
+  int tile, strip;
+  if constexpr (WIDE) {
+    const int live = counts[0], total = live * strips, per_xcd = (total + 7) >> 3;
+    const int place = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || place >= total) return;
+    strip = place / live;
+    tile = place - strip * live;
+  } else {
+    strip = blockIdx.x;
+    tile = blockIdx.y;
+    if (tile >= counts[0]) return;
+  }
+  const int e = tiles[3 * tile], at = tiles[3 * tile + 1], cnt = min(tiles[3 * tile + 2], MOST);
+  const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int n0 = strip * ACROSS + wave * (GATED ? 16 : 16 * S);
+  const int nchunks = K / KC, turn = (int)((strip * ACROSS / (GATED ? 128 : 256) * 5u + (unsigned)e * 3u) % (unsigned)(K / 128)) * (128 / KC);
+  const unsigned NW = GATED ? 2 * N : N;
+  const __amdgpu_buffer_rsrc_t w_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(w) + (size_t)e * NW * K, 0,
+                                                                        (int)(NW * (unsigned)K * 2u), 0x00020000);
+  unsigned w_off[S];  // this lane's first byte of its row of either strip (rows beyond N repeat the last one)
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const unsigned row = GATED ? (unsigned)min(n0 + lr, N - 1) + s * (unsigned)N : (unsigned)min(n0 + s * 16 + lr, N - 1);
+    w_off[s] = (row * (unsigned)K + lg * 16) * 2u;
+  }
+  auto where = [&](int j) { const int c = j + turn; return c >= nchunks ? c - nchunks : c; };
+  // LDS place (16 bytes) of block c (8 columns) of pair row r: the hardware reads 16-byte operands in the lane groups
+  // {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31} and the same above 32, which so touch every bank once
+  auto place_of = [](int r, int c) { return PIECES == 16 ? r * 16 + (c ^ (r & 15)) : r * 8 + (c ^ (0x32765410 >> ((r & 14) * 2) & 7)); };
+
+  auto run = [&](auto count) {
+    constexpr int CT = decltype(count)::value, TIMES = (CT * 16 + PASS - 1) / PASS;
+    constexpr int AHEAD = WIDE ? 1 : 2;  // chunks of weights in flight
+    const int piece = threadIdx.x % PIECES, prow = threadIdx.x / PIECES;  // this thread brings 16 bytes of rows prow + PASS i
+    int pair[TIMES];
+    const bf16* arow[TIMES];
+#pragma unroll
+    for (int i = 0; i < TIMES; ++i) pair[i] = order[at + min(prow + PASS * i, cnt - 1)];
+    u32x4 wa[STEPS][S][2], wb[STEPS][S][2], wc[AHEAD == 2 ? STEPS : 1][S][2], held[TIMES];
+    auto fetch = [&](u32x4 (&into)[STEPS][S][2], int j) {
+      const unsigned col = (unsigned)where(j) * (KC * 2u);
+#pragma unroll
+      for (int t = 0; t < STEPS; ++t)
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            into[t][s][h] = __builtin_amdgcn_raw_buffer_load_b128(w_buf, j < nchunks ? w_off[s] + col + t * 128u + h * 16u : BEYOND, 0, 0);
+    };
+    auto request = [&](int j) {  // past the last: the last again
+      const int k = where(min(j, nchunks - 1)) * KC;
+#pragma unroll
+      for (int i = 0; i < TIMES; ++i) held[i] = *reinterpret_cast<const u32x4*>(arow[i] + k);
+    };
+    floatx4 acc[S][CT];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int i = 0; i < CT; ++i) acc[s][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // One chunk: its activations go to LDS, whose half everyone left before the barrier of the chunk before; what comes next is
+    // requested; a bare barrier (a fence would wait for every load in flight); the products.
+    auto chunk = [&](int j, u32x4 (&now)[STEPS][S][2], u32x4 (&later)[STEPS][S][2]) {
+#pragma unroll
+      for (int i = 0; i < TIMES; ++i) lds[j & 1][place_of(prow + PASS * i, piece)] = held[i];
+      request(j + 1);
+      fetch(later, j + AHEAD);
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes have landed
+      __builtin_amdgcn_s_barrier();
+#pragma unroll
+      for (int t = 0; t < STEPS; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < CT; ++i) {
+            const bf16x8 av = __builtin_bit_cast(bf16x8, lds[j & 1][place_of(i * 16 + lr, t * 8 + lg * 2 + h)]);
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+              acc[s][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, now[t][s][h]), av, acc[s][i], 0, 0, 0);
+            if (WIDE && CT > 4 && i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four operands read ahead are what 128 registers hold
+          }
+    };
+    fetch(wa, 0);
+    if constexpr (AHEAD == 2) fetch(wb, 1);
+    __builtin_amdgcn_sched_barrier(0);  // the first weights are asked for before the pairs' numbers are waited for
+#pragma unroll
+    for (int i = 0; i < TIMES; ++i) arow[i] = a + (size_t)(pair[i] / a_div) * K + piece * 8;
+    request(0);
+    if constexpr (AHEAD == 2) {
+      const int rounds = nchunks / 3;
+      for (int it = 0; it < rounds; ++it) {  // three chunks: the roles of the weights' registers come round
+        chunk(3 * it, wa, wc);
+        chunk(3 * it + 1, wb, wa);
+        chunk(3 * it + 2, wc, wb);
+      }
+      if (nchunks - 3 * rounds >= 1) chunk(3 * rounds, wa, wc);
+      if (nchunks - 3 * rounds == 2) chunk(3 * rounds + 1, wb, wa);
+    } else {
+      for (int j = 0; j + 2 <= nchunks; j += 2) {
+        chunk(j, wa, wb);
+        chunk(j + 1, wb, wa);
+      }
+      if (nchunks & 1) chunk(nchunks - 1, wa, wb);
+    }
+    // a lane holds outputs n .. n+3 of either strip for the pair in column lr of each column tile
+#pragma unroll
+    for (int i = 0; i < CT; ++i) {
+      if (i * 16 + lr >= cnt) continue;
+      OutT* to = out + (size_t)order[at + i * 16 + lr] * N;
+#pragma unroll
+      for (int s = 0; s < (GATED ? 1 : S); ++s) {
+        const int n = n0 + s * 16 + 4 * lg;
+        if (n >= N) continue;  // N % 4 == 0
+        __attribute__((aligned(16))) OutT v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float z = acc[s][i][r];
+          if (GATED) z = gate_times_up(to_f32((bf16)z), to_f32((bf16)acc[S - 1][i][r]), limit);  // the two products rounded as if stored
+          if (MODE == MOE_RELU2) { z = fmaxf(to_f32((bf16)z), 0.f); z *= z; }
+          v[r] = from_f32<OutT>(z);
+        }
+        if constexpr (sizeof(OutT) == 4) *reinterpret_cast<float4*>(to + n) = *reinterpret_cast<const float4*>(v);
+        else *reinterpret_cast<uint2*>(to + n) = *reinterpret_cast<const uint2*>(v);
+      }
+    }
+  };
+  const int col_tiles = (cnt + 15) >> 4;
+  if constexpr (WIDE) {
+    if (col_tiles > 6) return run(std::integral_constant<int, 8>{});
+    if (col_tiles > 4) return run(std::integral_constant<int, 6>{});
+  }
+  if (col_tiles == 4) run(std::integral_constant<int, 4>{});
+  else if (col_tiles == 3) run(std::integral_constant<int, 3>{});
+  else if (col_tiles == 2) run(std::integral_constant<int, 2>{});
+  else run(std::integral_constant<int, 1>{});
+}
+
 // fp32: plain multiply-add, every output one chain over k in order.  A thread owns an output and, of every
 // sixteen of the tile's pairs in turn, four.
 template <bool GATED, bool RELU2 = false>
@@ -471,11 +641,12 @@ __global__ __launch_bounds__(256) void moe_gemm_f32_kernel(const float* __restri
 // are still to be added up); the fp32 product writes fp32.
 // gated: 0: the product; 1: act(gate) * up (limit 0: silu(gate) * up; > 0: the gated activation with limits);
 // 2: relu(product)^2 (an expert without a gate).
+// size: of the route's tiles, 64 or 128.
 extern "C" int as_moe_gemm(const void* a, int dtype, int a_div, const void* w, int N, int K, int gated, const int* order,
                            const int* tiles, const int* counts, int max_tiles, void* out, int out_dtype, float limit,
-                           hipStream_t stream) {
+                           int size, hipStream_t stream) {
   if (max_tiles <= 0) return AS_OK;
-  if (N <= 0 || K <= 0 || a_div <= 0 || max_tiles > 65535) return AS_BAD_SHAPE;
+  if (N <= 0 || K <= 0 || a_div <= 0 || max_tiles > 65535 || (size != MOE_HALF && size != MOE_TILE)) return AS_BAD_SHAPE;
   dim3 grid((N + MOE_STRIP - 1) / MOE_STRIP, max_tiles);
   if (dtype == DT_F32) {
     if (out_dtype != DT_F32) return AS_BAD_DTYPE;
@@ -485,6 +656,29 @@ extern "C" int as_moe_gemm(const void* a, int dtype, int a_div, const void* w, i
     return launch_status();
   }
   if (dtype != DT_BF16) return AS_BAD_DTYPE;
+  const unsigned long long expert_bytes = (unsigned long long)(gated == 1 ? 2 : 1) * N * K * 2ull;  // 32-bit offsets within an expert
+  if (K % 128 == 0 && N % 16 == 0 && (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) == 0 && expert_bytes <= 0xf0000000ull &&
+      (gated ? out_dtype == DT_BF16 : out_dtype == DT_BF16 || out_dtype == DT_F32)) {
+    const bool wide = size == MOE_TILE;
+    const int across = (gated == 1 ? 64 : wide ? 128 : 64) * (wide ? 2 : 1), strips = (N + across - 1) / across;
+    if (wide && (long long)strips * max_tiles > 0x3ffffff8ll) return AS_BAD_SHAPE;
+#define STREAM(MODE, T)                                                                                                      \
+  do {                                                                                                                       \
+    if (wide)                                                                                                                \
+      moe_gemm_stream_kernel<MODE, T, true><<<(strips * max_tiles + 7) / 8 * 8, 512, 0, stream>>>(                           \
+          (const bf16*)a, a_div, (const bf16*)w, N, K, order, tiles, counts, (T*)out, limit, strips);                        \
+    else                                                                                                                     \
+      moe_gemm_stream_kernel<MODE, T, false><<<dim3(strips, max_tiles), 256, 0, stream>>>(                                      \
+          (const bf16*)a, a_div, (const bf16*)w, N, K, order, tiles, counts, (T*)out, limit, strips);                        \
+  } while (0)
+    if (gated == 1) STREAM(MOE_GATED, bf16);
+    else if (gated) STREAM(MOE_RELU2, bf16);
+    else if (out_dtype == DT_BF16) STREAM(MOE_PLAIN, bf16);
+    else STREAM(MOE_PLAIN, float);
+#undef STREAM
+    return launch_status();
+  }
+  grid.z = size / MOE_HALF;
   if (gated == 2) {
     if (out_dtype != DT_BF16) return AS_BAD_DTYPE;
     moe_gemm_bf16_kernel<false, bf16, true><<<grid, 256, 0, stream>>>((const bf16*)a, a_div, (const bf16*)w, N, K, order, tiles, counts, (bf16*)out, limit);

@@ -1941,18 +1941,25 @@ def rglru_scan(a, x, proj, y_off, y_bias, scale, state, step_rows, out, out_off,
 
 # ---- experts ------------------------------------------------------------------------------------------
 
-MOE_TILE = 64  # pairs of one expert that a workgroup of the grouped products takes
+MOE_TILES = (64, 128)  # pairs of one expert that a tile of the grouped products holds: of few pairs, of many
+# Large tiles read every weight once where small ones read it for every 64 pairs, and make a quarter of the workgroups: from this many
+# pairs an expert on where all experts' first matrices have MOE_WIDE_ROWS rows (16 experts, gate and up of 1,536 at width 2,048, both
+# products: 400 tokens of two experts 79 us in small tiles and 77 in large ones, 600 109 and 86, 1,500 191 and 127), later where they have
+# fewer (gate and up of 768 at width 1,024: 1,000 tokens 46 and 53, 1,500 64 and 50)
+MOE_MANY, MOE_MANY_NARROW, MOE_WIDE_ROWS = 56, 160, 49152
 MOE_MAX_EXPERTS = 1024
 
 
 class ExpertRoute:
     """Where a step's (token, chosen expert) pairs stand once sorted by expert: what the grouped products read."""
 
-    __slots__ = ("order", "tiles", "counts", "max_tiles", "top", "num_tokens", "pair_weight", "pair_expert")
+    __slots__ = ("order", "tiles", "counts", "max_tiles", "top", "num_tokens", "pair_weight", "pair_expert", "tile")
 
-    def __init__(self, num_tokens: int, top: int, experts: int, device):
+    def __init__(self, num_tokens: int, top: int, experts: int, device, weight_rows: int = 0, tile: int = None):
         pairs = num_tokens * top
-        self.max_tiles = -(-pairs // MOE_TILE) + experts
+        many = MOE_MANY if weight_rows == 0 or weight_rows >= MOE_WIDE_ROWS else MOE_MANY_NARROW
+        self.tile = MOE_TILES[pairs >= many * experts] if tile is None else tile
+        self.max_tiles = -(-pairs // self.tile) + experts
         self.order = torch.empty(max(pairs, 1), dtype=I32, device=device)
         self.tiles = torch.empty((self.max_tiles, 3), dtype=I32, device=device)
         self.counts = torch.empty(1, dtype=I32, device=device)
@@ -1961,31 +1968,33 @@ class ExpertRoute:
         self.pair_expert = None  # int32 [pairs]: each pair's expert, where a router says
 
 
-def moe_route_table(token_ids, table, experts: int) -> ExpertRoute:
-    """Routes by a table [vocab, top] int32 that names every token id's experts."""
+def moe_route_table(token_ids, table, experts: int, weight_rows: int = 0, tile: int = None) -> ExpertRoute:
+    """Routes by a table [vocab, top] int32 that names every token id's experts.  weight_rows (here and below): of all experts'
+    first matrices, where known, and tile (64 or 128, for tests): how the pairs are cut into tiles, which decides speed alone."""
     _check(token_ids, "token_ids", I32, (None,))
     _check(table, "table", I32, (None, None))
     vocab, top = table.shape
     if not 1 <= experts <= MOE_MAX_EXPERTS:
         raise KernelError(f"routing sorts up to {MOE_MAX_EXPERTS} experts, not {experts}")
-    route = ExpertRoute(token_ids.shape[0], top, experts, token_ids.device)
+    route = ExpertRoute(token_ids.shape[0], top, experts, token_ids.device, weight_rows, tile)
     call("as_moe_route_table", _ptr(token_ids), _ptr(table), vocab, top, experts, token_ids.shape[0], _ptr(route.order),
-         _ptr(route.tiles), _ptr(route.counts), route.max_tiles, 0, _stream())  # fmt: skip
+         _ptr(route.tiles), _ptr(route.counts), route.max_tiles, 0, route.tile, _stream())  # fmt: skip
     return route
 
 
-def moe_route_sigmoid(h, router, top: int) -> ExpertRoute:
+def moe_route_sigmoid(h, router, top: int, weight_rows: int = 0) -> ExpertRoute:
     """Routes by a router's scores: z = router h in fp32, s = sigmoid(z), a token's `top` experts those with the
     largest s, weighing s / (their sum + 1e-20).  h [T, K], router [experts, K] of one dtype.  The route carries
     `pair_weight` fp32 [T * top] for `moe_combine`."""
-    return moe_route_scores(h, router, top, "sigmoid")
+    return moe_route_scores(h, router, top, "sigmoid", weight_rows=weight_rows)
 
 
 ROUTER_SCORES = {"sigmoid": 0, "softmax_of_chosen": 1, "softmax": 2}
 
 
 def moe_route_scores(h, router, top: int, score: str, bias=None, groups: int = 1, keep_groups: int = 1,
-                     weight_scale: float = 1.0, correction=None, identity: int = 0) -> ExpertRoute:  # fmt: skip
+                     weight_scale: float = 1.0, correction=None, identity: int = 0,
+                     weight_rows: int = 0) -> ExpertRoute:  # fmt: skip
     """Routes by a router's logits z = router h + bias in fp32 (bias fp32 [experts] or None).  score "sigmoid": the
     `top` largest sigmoid(z), weighing s / (their sum + 1e-20); "softmax_of_chosen": the `top` largest z, weighing the
     softmax over those z alone; "softmax": s = softmax(z) over all experts, the `top` largest among the experts of the
@@ -2013,14 +2022,14 @@ def moe_route_scores(h, router, top: int, score: str, bias=None, groups: int = 1
         raise KernelError("groups of experts and a scale of the weights belong to the score 'softmax'")
     if groups < 1 or experts % groups or not 1 <= keep_groups <= groups or keep_groups * (experts // groups) < top:
         raise KernelError(f"{experts} experts in {groups} groups of which {keep_groups} are kept do not give {top} to choose")
-    route = ExpertRoute(T, top, experts - identity, h.device)
+    route = ExpertRoute(T, top, experts - identity, h.device, weight_rows)
     pair_expert = route.pair_expert = torch.empty(max(T * top, 1), dtype=I32, device=h.device)
     route.pair_weight = torch.empty(max(T * top, 1), dtype=F32, device=h.device)
     call("as_moe_route_scores", _ptr(h), _ptr(router), _ptr(bias), ROUTER_SCORES[score], _ptr(correction), int(groups),
          int(keep_groups), float(weight_scale), _DT[h.dtype], K, experts, top, T,
          _ptr(pair_expert), _ptr(route.pair_weight), _stream())  # fmt: skip
     call("as_moe_route_table", 0, _ptr(pair_expert), 0, top, experts - identity, T, _ptr(route.order), _ptr(route.tiles),
-         _ptr(route.counts), route.max_tiles, int(identity), _stream())  # fmt: skip
+         _ptr(route.counts), route.max_tiles, int(identity), route.tile, _stream())  # fmt: skip
     return route
 
 
@@ -2047,7 +2056,8 @@ def moe_gemm(a, w, route: ExpertRoute, out, gated: bool, per_token: bool, activa
         raise KernelError("moe_gemm: the activated product's result has the inputs' dtype")
     call("as_moe_gemm", _ptr(a), _DT[a.dtype], route.top if per_token else 1, _ptr(w), N, K,
          2 if activation else int(bool(gated)),
-         _ptr(route.order), _ptr(route.tiles), _ptr(route.counts), route.max_tiles, _ptr(out), _DT[out.dtype], float(limit), _stream())  # fmt: skip
+         _ptr(route.order), _ptr(route.tiles), _ptr(route.counts), route.max_tiles, _ptr(out), _DT[out.dtype], float(limit),
+         route.tile, _stream())  # fmt: skip
 
 
 def moe_combine(pair_out, top: int, weight: float, out, pair_weight=None, add=None, same=None, pair_expert=None, experts: int = 0) -> None:

@@ -709,3 +709,46 @@ def test_scan_of_a_linear_recurrence(width, dtype, bias):
         want = 0.5 * want * gelu
         tol = 1e-5 if dtype == "float32" else 2.0**-8
         assert ((out[first[i] : first[i] + n, 8:].double() - want).abs() <= tol * want.abs() + 1e-5).all()
+
+
+@pytest.mark.parametrize("N, K", [(16, 128), (80, 384), (272, 256), (48, 1536)])
+@pytest.mark.parametrize("mode", ["gated", "limited", "relu2", "plain", "plain32"])
+def test_experts_products_in_tiles(N, K, mode):
+    """Runs of pairs around the column tiles, the half tiles and the tiles of 128, an expert without pairs: the kernel of tiles of 64
+    and the one of tiles of 128 against 64 bits, and against each other bit for bit."""
+    from atomserve_amd.kernels import ops
+
+    counts = [1, 16, 17, 0, 64, 65, 96, 97, 128, 129, 260]
+    experts = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)]).int()
+    gen = torch.Generator().manual_seed(N + K)
+    experts = experts[torch.randperm(len(experts), generator=gen)]
+    T, E, gated = len(experts), len(counts), mode in ("gated", "limited")
+    a = torch.randn(T, K, generator=gen).bfloat16()
+    w = torch.randn(E, 2 * N if gated else N, K, generator=gen).mul(K**-0.5).bfloat16()
+    outs = []
+    for tile in (64, 128):
+        route = ops.moe_route_table(torch.arange(T, dtype=torch.int32, device=DEV), experts[:, None].contiguous().to(DEV), E, tile=tile)
+        out = torch.full((T, N), float("nan"), dtype=torch.float32 if mode == "plain32" else torch.bfloat16, device=DEV)
+        ops.moe_gemm(a.to(DEV), w.to(DEV), route, out, gated, per_token=tile == 64, activation="relu2" if mode == "relu2" else None,
+                     limit=1.5 if mode == "limited" else 0.0)  # fmt: skip
+        outs.append(out.cpu())
+    assert torch.equal(outs[0], outs[1])
+    z = torch.stack([w[int(e)].double() @ a[t].double() for t, e in enumerate(experts)])
+    if gated:  # the two products are rounded to bfloat16 first
+        g, u = z[:, :N], z[:, N:]
+        want = torch.nn.functional.silu(g) * u
+        if mode == "limited":
+            g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+            want = g * torch.sigmoid(1.702 * g) * (u + 1)
+    else:
+        want = z.clamp(min=0) ** 2 if mode == "relu2" else z
+    # the result's rounding, 2^-8 of it; before that a square of a rounded product, twice 2^-8, or a gated pair: 2^-8 of either's
+    # part, which |d silu| <= 1.1 (1.8 with limits: slope 1.1 and alpha 1.702) and the other factor, up to max |z| + 1, carry on
+    u8 = 2.0**-8
+    if mode == "plain32":
+        bound = 1e-5 * z.abs().max()
+    elif gated:
+        bound = u8 * want.abs() + u8 * 1.1 * 2 * z.abs().max() * (z.abs().max() + 1) * 0.25
+    else:
+        bound = (3 if mode == "relu2" else 1) * u8 * want.abs() + 1e-5
+    assert ((outs[0].double() - want).abs() <= bound).all()
