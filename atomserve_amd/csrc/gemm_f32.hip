@@ -61,7 +61,7 @@ template <bool VEC> __device__ __forceinline__ floatx4 again_f32(floatx4 v, cons
 // What a product carries along when the residual sum and the RMSNorm around it are folded into the products of a decode step
 // (a pre-norm layer: x += part(norm(x))), as the few-rows products of bf16 do:
 //   producer (LINK): the sum goes on top of the stream x = out[M, N]; scaled[M, N] = x * gain, the input of the next product
-//     without its 1/rms factor; ssq_out[M, strips] = the sums of x^2 per 16 columns.
+//     without its 1/rms factor; ssq_out[M, N / 4] = the sums of x^2 per 4 columns (whatever kernel makes them).
 //   consumer (ssq_in): 1/rms of each row comes from the row's sums of squares and multiplies the product's sums.
 struct LinkF32 {
   const float* ssq_in;
@@ -247,7 +247,6 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
       v = silu_times(v, up);
     }
     if constexpr (MODE == LINK) {
-      float ss = 0.f;
       if (m < M && n < N) {  // N % 4 == 0
         float* xp = out + (size_t)m * N + n;
         v += *reinterpret_cast<floatx4*>(xp);
@@ -256,14 +255,100 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
 #pragma unroll
         for (int r = 0; r < 4; ++r) g[r] = link.gain[n + r];
         *reinterpret_cast<floatx4*>(link.scaled + (size_t)m * N + n) = v * g;
-        ss = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+        link.ssq_out[((size_t)m * N + n) / 4] = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
       }
-      ss += __shfl_xor(ss, 16, 64);  // the four lanes that hold the strip's 16 columns of row m
-      ss += __shfl_xor(ss, 32, 64);
-      if (lane < 16 && m < M) link.ssq_out[(size_t)m * ((N + 15) / 16) + n0 / 16] = ss;
     } else if (m < M && n < N) {
       store4(out + (size_t)m * N + n, v, min(4, N - n));
     }
+  }
+}
+
+// Up to 8 rows where strips of 16 rows of w are too few to occupy the compute units: a workgroup makes 16 / SIDE outputs, and the
+// 16 rows of a wave's matrix operands are 16 / SIDE rows of w (of a) in SIDE neighbouring slices of K side by side, so that a slice's
+// sums stand on the diagonal of the product's SIDE x SIDE blocks (the other blocks mean nothing and are dropped).  Each slice
+// is one pair of chains in the order of the others: the same bits.  16 / SIDE waves, DEPTH steps of both operands in flight:
+// 4 rows, K = 3,072, N = 1,024 (12.6 MB) 13.0 -> 7.4 us, which 64 strips of 16 rows of w had bound, a quarter of the compute
+// units with 64 KB each in flight.
+template <int SIDE, int DEPTH, bool VEC, int MODE>
+__global__ __launch_bounds__(16 / SIDE * 64) void gemm_f32_side_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                    float* __restrict__ out, int M, int N, int K, LinkF32 link) {
+  static_assert(MODE != GATED && (SIDE == 2 || SIDE == 4), "");
+  constexpr int R = 16 / SIDE, WAVES = F32_SLICES / SIDE;  // rows of either operand; waves
+  __shared__ floatx4 red[F32_SLICES][R / 4][R];             // [slice][outputs / 4][row of a]
+  __shared__ float inv_rms[16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int n0 = blockIdx.x * R;
+  const int steps = (K + 31) / 32, per = (steps + F32_SLICES - 1) / F32_SLICES;
+  const int first = (wave * SIDE + lr / R) * per;  // this lane's slice
+  const float* wrow = w + (size_t)min(n0 + lr % R, N - 1) * K;
+  const float* arow = a + (size_t)min(lr % R, M - 1) * K;
+  floatx4 wv[DEPTH][2], av[DEPTH][2], acc = {0.f, 0.f, 0.f, 0.f}, low = acc;
+  auto load = [&](int u, int st) {  // columns from K on count as zeros; steps past the slice are loaded and not used
+    const int k = (first + st) * 32 + lg * 8;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      wv[u][half] = fetch<VEC>(wrow, k + 4 * half, K);
+      av[u][half] = fetch<VEC>(arow, k + 4 * half, K);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < DEPTH; ++u) load(u, min(u, per - 1));
+  if (link.ssq_in != nullptr) {  // 1 / rms of the rows, a wave a row; published by the barrier below
+    for (int row = wave; row < M; row += WAVES) {
+      float ss = 0.f;
+      for (int j = lane; j < link.strips_in; j += 64) ss += link.ssq_in[(size_t)row * link.strips_in + j];
+      ss = wave_sum(ss);
+      if (lane == 0) inv_rms[row] = 1.0f / sqrtf(ss / (float)K + link.eps);
+    }
+  }
+  for (int st = 0; st < per; st += DEPTH) {
+#pragma unroll
+    for (int u = 0; u < DEPTH; ++u) {
+      if (st + u < per) {
+        const Parts ws = parts(wv[u][0], wv[u][1]), as = parts(av[u][0], av[u][1]);
+        if (st + u + DEPTH < per) load(u, st + u + DEPTH);
+#pragma unroll
+        for (int x = 0; x < 6; ++x) {
+          floatx4& to = x == 5 ? acc : low;
+          to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(part(ws, PART_W[x]), part(as, PART_A[x]), to, 0, 0, 0);
+        }
+      }
+    }
+  }
+  // a lane holds rows 4 lg .. 4 lg + 3 of w's side by side in column lr of a's: outputs 4 lg % R of slice 4 lg / R by row lr % R of slice lr / R
+  if (4 * lg / R == lr / R) red[wave * SIDE + lr / R][lg % (R / 4)][lr % R] = acc + low;
+  __syncthreads();
+  if (wave) return;
+  const int n = n0 + 4 * lg, m = lr;  // this lane's outputs n .. n+3 of row m
+  const bool mine = m < M && 4 * lg < R && n < N;
+  floatx4 v = {0.f, 0.f, 0.f, 0.f};
+  if (m < R && 4 * lg < R) {
+#pragma unroll
+    for (int g = 0; g < F32_GROUPS; ++g) {
+      floatx4 s = red[4 * g][lg][m];
+#pragma unroll
+      for (int x = 1; x < 4; ++x) s += red[4 * g + x][lg][m];
+      v = g == 0 ? s : v + s;
+    }
+  }
+  if (__any(mine && !finite(v))) {
+    const floatx4 f = again_f32<VEC>(v, w + (size_t)min(n0 + lr, N - 1) * K, a + (size_t)min(m, M - 1) * K, K, 0, steps);
+    if (mine) v = f;
+  }
+  if (!mine) return;
+  if (link.ssq_in != nullptr) v *= inv_rms[m];
+  float* to = out + (size_t)m * N + n;
+  if constexpr (MODE == LINK) {  // N % 4 == 0
+    v += *reinterpret_cast<floatx4*>(to);
+    *reinterpret_cast<floatx4*>(to) = v;
+    floatx4 g;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) g[r] = link.gain[n + r];
+    *reinterpret_cast<floatx4*>(link.scaled + (size_t)m * N + n) = v * g;
+    link.ssq_out[((size_t)m * N + n) / 4] = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+  } else {
+    store4(to, v, min(4, N - n));
   }
 }
 
@@ -499,6 +584,28 @@ static int launch_few(const float* a, const float* w, float* out, int M, int N, 
   return launch_rows<1, NT, WAVES, DEPTH, 1, MODE>(a, w, out, M, N, K, link, stream);
 }
 
+template <int MODE> static int launch_side(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
+  const bool vec = (K & 3) == 0 && aligned16(a, w);
+#define SIDE_GO(SIDE)                                                                                                            \
+  do {                                                                                                                           \
+    const int blocks = (N + 16 / SIDE - 1) / (16 / SIDE);                                                                        \
+    if (vec) gemm_f32_side_kernel<SIDE, 6, true, MODE><<<blocks, 16 / SIDE * 64, 0, stream>>>(a, w, out, M, N, K, link);         \
+    else gemm_f32_side_kernel<SIDE, 2, false, MODE><<<blocks, 16 / SIDE * 64, 0, stream>>>(a, w, out, M, N, K, link);            \
+  } while (0)
+  if (M <= 4) SIDE_GO(4);
+  else SIDE_GO(2);
+#undef SIDE_GO
+  return launch_status();
+}
+
+// Whether a product of few rows goes side by side: while strips of 16 outputs are at most half of the compute units, and, with two
+// slices side by side, K is long enough for the second operand's loads to pay.  us, the best of the others and side by side:
+// N, K            1 row        4 rows       8 rows           N, K            1 row        4 rows       8 rows
+// 1,024, 1,024    6.4  5.3     7.1  6.3     8.0  8.9         2,048, 2,048    9.6  7.9    10.2  9.6    11.3  9.8
+// 1,024, 2,048    9.3  6.0    10.0  6.9    11.1  9.5         2,048, 6,144   23.1 18.8    23.7 20.8    26.3 20.5
+// 1,024, 3,072   12.0  6.6    13.0  7.4    14.4 10.0         3,072, 1,024    6.9  8.8     7.4 11.6     8.3 16.0
+static bool side_by_side(int M, int N, int K) { return N <= 8 * compute_units() && (M <= 4 || (M <= 8 && K >= 2048)); }
+
 template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT>
 static int launch_tile(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
   constexpr int TM = 16 * WM * MTW, TN = 16 * WN * NTW;
@@ -532,10 +639,13 @@ static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
   return 4.5f + (float)K / 1024.f / (float)split * crowd * (t.alone_us + t.round_us * (float)(rounds - 1));
 }
 
-// form: 0: chosen here; else 1 + the index of a kernel (tests).
+// form: 0: chosen here; else 1 + the index of a kernel, or after them the one of slices side by side (tests).
 template <int MODE> static int gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, const LinkF32& link,
                                         hipStream_t stream) {
   const bool vec = (K & 3) == 0 && aligned16(a, w);
+  if constexpr (MODE == PLAIN) {
+    if (form == F32_FORMS + 1 ? M <= 8 : form == 0 && side_by_side(M, N, K)) return launch_side<PLAIN>(a, w, out, M, N, K, link, stream);
+  }
   if (form == 0) {
     float best = 0.f;
     for (int i = MODE == GATED ? 2 : 0; i < (link.ssq_in ? F32_ONE_ROW_TILE : F32_FORMS); ++i) {
@@ -575,7 +685,7 @@ template <int MODE> static int gemm_f32(const float* a, const float* w, float* o
 
 extern "C" int as_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
   if (M <= 0) return AS_OK;
-  if (N <= 0 || K <= 0 || form < 0 || form > F32_FORMS) return AS_BAD_SHAPE;
+  if (N <= 0 || K <= 0 || form < 0 || form > F32_FORMS + 1) return AS_BAD_SHAPE;
   if (K <= F32_NARROW) {
     const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
     if (grid.y > 65535) return AS_BAD_SHAPE;
@@ -593,22 +703,23 @@ extern "C" int as_gemm_f32_gated(const float* a, const float* w, float* out, int
   return gemm_f32<GATED>(a, w, out, M, N, K, form, LinkF32{}, stream);
 }
 
-// The producer of a LinkF32: x[M, N] += a @ w^T; scaled[M, N] = x * gain; ssq[M, ceil(N / 16)] = sums of x^2 per 16 columns.
+// The producer of a LinkF32: x[M, N] += a @ w^T; scaled[M, N] = x * gain; ssq[M, N / 4] = sums of x^2 per 4 columns.
 // M <= 16, K > F32_NARROW, N % 4 == 0, x and scaled on 16 bytes.
 extern "C" int as_gemm_f32_link(const float* a, const float* w, float* x, const float* gain, float* scaled, float* ssq, int M, int N, int K,
                                 hipStream_t stream) {
   if (M <= 0) return AS_OK;
   if (M > 16 || N <= 0 || (N & 3) || K <= F32_NARROW || !gain || !scaled || !ssq || !aligned16(x, scaled)) return AS_BAD_SHAPE;
   const LinkF32 link{nullptr, 0, 0.f, gain, scaled, ssq};
+  if (side_by_side(M, N, K)) return launch_side<LINK>(a, w, x, M, N, K, link, stream);
   return launch_few<1, 8, 4, LINK>(a, w, x, M, N, K, link, stream);
 }
 
-// The consumer of a LinkF32: out[M, N] = (scaled @ w^T) / rms(x) with rms from ssq[M, strips_in] (strips_in = ceil(K / 16)) and eps;
+// The consumer of a LinkF32: out[M, N] = (scaled @ w^T) / rms(x) with rms from ssq[M, strips_in] (strips_in = K / 4) and eps;
 // gated: silu of the first half of w's 2 N rows times the second half, both scaled first.  M <= 16, K > F32_NARROW.
 extern "C" int as_gemm_f32_scaled(const float* scaled, const float* ssq, int strips_in, float eps, const float* w, float* out, int M, int N,
                                   int K, int gated, hipStream_t stream) {
   if (M <= 0) return AS_OK;
-  if (M > 16 || N <= 0 || N > 0x3fffffff || K <= F32_NARROW || !ssq || strips_in != (K + 15) / 16) return AS_BAD_SHAPE;
+  if (M > 16 || N <= 0 || N > 0x3fffffff || K <= F32_NARROW || (K & 3) || !ssq || strips_in != K / 4) return AS_BAD_SHAPE;
   const LinkF32 link{ssq, strips_in, eps, nullptr, nullptr, nullptr};
   return gated ? gemm_f32<GATED>(scaled, w, out, M, N, K, 0, link, stream) : gemm_f32<PLAIN>(scaled, w, out, M, N, K, 0, link, stream);
 }

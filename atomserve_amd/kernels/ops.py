@@ -1093,11 +1093,16 @@ def gemm_f32_link_supported(rows: int, n_out: int, k: int, x=None) -> bool:
             and (x is None or x.data_ptr() % 16 == 0))  # fmt: skip
 
 
+def link_strips(n: int, dtype) -> int:
+    """Sums of squares that a row of n columns carries from a `gemm_link` to a `gemm_scaled`."""
+    return -(-n // (4 if dtype == F32 else 16))
+
+
 def gemm_link(a, w, x, gain, scaled, ssq) -> None:
     """The last product of a part of a pre-norm layer with the residual sum and the first half of
     the next RMSNorm: x[M, N] (fp32) += bf16(a @ w^T); scaled[M, N] = bf16(x * gain), the next
     product's input without its 1/rms factor; ssq[M, ceil(N / 16)] = sums of x^2 per 16 columns.
-    a, w, scaled bf16, or all fp32 and nothing rounded; gain fp32 [N]."""
+    a, w, scaled bf16, or all fp32 and nothing rounded (ssq then [M, N / 4], per 4 columns); gain fp32 [N]."""
     _check(a, "a", (F32, BF16), (None, None))
     M, K = a.shape
     rows = _rows(w)
@@ -1108,7 +1113,7 @@ def gemm_link(a, w, x, gain, scaled, ssq) -> None:
     _check(x, "x", F32, (M, N))
     _check(gain, "gain", F32, (N,))
     _check(scaled, "scaled", a.dtype, (M, N))
-    _check(ssq, "ssq", F32, (M, -(-N // 16)))
+    _check(ssq, "ssq", F32, (M, link_strips(N, a.dtype)))
     if a.dtype == F32:
         call("as_gemm_f32_link", _ptr(a), _ptr(rows), _ptr(x), _ptr(gain), _ptr(scaled), _ptr(ssq), M, N, K, _stream())
         return
@@ -1122,7 +1127,7 @@ def gemm_scaled(scaled, ssq, eps, w, out, gated=False) -> None:
     second half, both scaled and rounded to bf16 first).  scaled [M, K], w, out bf16, or all fp32."""
     _check(scaled, "scaled", (F32, BF16), (None, None))
     M, K = scaled.shape
-    _check(ssq, "ssq", F32, (M, -(-K // 16)))
+    _check(ssq, "ssq", F32, (M, link_strips(K, scaled.dtype)))
     _check(out, "out", scaled.dtype, (M, None))
     N = out.shape[1]
     rows = _rows(w)

@@ -63,7 +63,7 @@ class RMSNorm(Norm):
                 else ops.gemm_link_supported(M, N, a.shape[1], self.env.dtype, w)):  # fmt: skip
             return None
         scaled = torch.empty((M, N), dtype=self.env.dtype, device=x.device)
-        ssq = torch.empty((M, -(-N // 16)), dtype=torch.float32, device=x.device)
+        ssq = torch.empty((M, ops.link_strips(N, self.env.dtype)), dtype=torch.float32, device=x.device)
         ops.gemm_link(a, w, x, self.gain_f32, scaled, ssq)
         return PendingRMSNorm(self, x, scaled, ssq)
 

@@ -1439,11 +1439,30 @@ def test_gemm_f32_numbers_that_are_not_finite(ops, M, shift):
     assert bool(torch.isfinite(clean).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 4, 257), (2, 19, 300), (4, 1024, 3072), (5, 9, 544), (8, 132, 6144), (7, 2050, 1000)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gemm_f32_slices_side_by_side(ops, M, N, K, shift):
+    """Up to 8 rows with several slices of K side by side in a matrix operand: the bits of the other kernels, at widths that leave
+    slices short or empty, values that are not finite included (a NaN next to them in the operand reaches no other output)."""
+    torch.manual_seed(M + N)
+    a = torch.randn(M * K + shift, device=DEV)[shift:].view(M, K)
+    w = torch.randn(N * K + shift, device=DEV)[shift:].view(N, K) * 0.05
+    for spoil in (False, True):
+        if spoil:
+            a[0, 1], w[N - 1, K - 1], w[N // 2, 5] = float("inf"), float("nan"), float("-inf")
+        want = f32_product("as_gemm_f32", a, w, torch.full((M, N), 7.0, device=DEV), 1)
+        got = f32_product("as_gemm_f32", a, w, torch.full((M, N), 7.0, device=DEV), 9)
+        assert torch.equal(got.nan_to_num(3.0), want.nan_to_num(3.0)) and torch.equal(got.isnan(), want.isnan())
+        if not spoil:
+            ref, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+            assert bool(((got.double() - ref).abs() <= size * (K / 512 + 16) * 2.0**-24).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 260, 1024), (4, 1024, 2048), (5, 272, 300), (8, 1024, 3072), (9, 516, 288), (16, 2048, 6144)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_gemm_link_and_scaled_f32(ops, M, N, K, shift):
     """The residual sum and the norm folded into 32-bit products: x has the bits of the plain product on top, the sums of squares
-    are those of x within their rounding (16 columns), and the product of what is left, times 1 / rms, is that of the normed rows:
+    are those of x within their rounding (4 columns), and the product of what is left, times 1 / rms, is that of the normed rows:
     bounds from the sums of absolute values, two more roundings (x * gain, 1 / rms) of 2^-24 and the root's own."""
     torch.manual_seed(64)
     eps, L = 1e-6, 96
@@ -1453,11 +1472,11 @@ def test_gemm_link_and_scaled_f32(ops, M, N, K, shift):
     prod = torch.empty(M, N, device=DEV)
     ops.gemm(a, w, prod)
     want = x + prod
-    scaled, ssq = torch.empty(M, N, device=DEV), torch.empty(M, -(-N // 16), device=DEV)
+    scaled, ssq = torch.empty(M, N, device=DEV), torch.empty(M, ops.link_strips(N, F32), device=DEV)
     assert ops.gemm_f32_link_supported(M, N, K, x)
     ops.gemm_link(a, w, x, gain, scaled, ssq)
     assert torch.equal(x, want) and torch.equal(scaled, x * gain)
-    squares = torch.nn.functional.pad(x.double().square(), (0, -N % 16)).view(M, -1, 16).sum(2)
+    squares = x.double().square().view(M, -1, 4).sum(2)
     assert bool(((ssq.double() - squares).abs() <= squares * 8 * 2.0**-24).all())
     inv = 1 / (x.double().square().mean(1, keepdim=True) + eps).sqrt()
     for gated in (False, True):
