@@ -48,7 +48,8 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 
 // Sum over a block of up to 1024 threads; every thread gets the result.  `red` is a
-// __shared__ float[17].  The order of additions is fixed, so the result is reproducible.
+// __shared__ float[17].  The order of additions is fixed, so the result is reproducible.  Every thread adds the waves' sums
+// up itself: one thread doing it for all costs another barrier.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
   const int nw = (blockDim.x + WAVE - 1) / WAVE;
@@ -56,13 +57,9 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   __syncthreads();  // protects `red` against a previous use
   if (lane == 0) red[wid] = v;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float s = 0.f;
-    for (int i = 0; i < nw; ++i) s += red[i];
-    red[16] = s;
-  }
-  __syncthreads();
-  return red[16];
+  float s = 0.f;
+  for (int i = 0; i < nw; ++i) s += red[i];
+  return s;
 }
 
 static inline int launch_status() {

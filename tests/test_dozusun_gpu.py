@@ -583,6 +583,36 @@ def test_one_sum_two_norms(dtype):
         assert (picked.float().cpu() - want1[[T - 1, 0]]).abs().max() <= tol * float(want1.abs().max())
 
 
+@pytest.mark.parametrize("n, rows", [(6, 3), (36, 3), (2048, 600), (4096, 5), (4100, 2), (8192, 3), (12292, 2), (16388, 2)])
+@pytest.mark.parametrize("dtype, gains", [("float32", "float32"), ("bfloat16", "bfloat16"), ("bfloat16", "float32")])
+def test_one_sum_two_norms_of_any_width(n, rows, dtype, gains):
+    """Rows in one, two and four pieces of 16 bytes a thread, wider ones and ones that do not come in such pieces; with and without
+    each pending output, a second norm, a selection of rows and the write back."""
+    from atomserve_amd.kernels import ops
+
+    gen, T = torch.Generator().manual_seed(n), DTYPES[dtype]
+    x = torch.randn(rows + 1, n, generator=gen)
+    d1, d2 = (torch.randn(rows + 1, n, generator=gen).to(T) for _ in range(2))
+    w1, w2 = (torch.randn(n, generator=gen).to(DTYPES[gains]) for _ in range(2))
+    pick = torch.randperm(rows + 1, generator=gen)[:rows]
+    for a, b, second, some, update in ((1, 1, 1, 0, 1), (1, 0, 1, 1, 0), (0, 1, 0, 0, 1), (0, 0, 1, 1, 1), (1, 1, 0, 1, 1)):
+        xs, sel = x.to(DEV), pick if some else torch.arange(rows + 1)
+        out = [torch.empty(len(sel), n, dtype=T, device=DEV) for _ in range(1 + second)]
+        ops.rmsnorm_multi(xs, w1.to(DEV), w2.to(DEV) if second else None, 1e-6, out[0], out[1] if second else None,
+                          delta1=d1.to(DEV) if a else None, delta2=d2.to(DEV) if b else None,
+                          rows=sel.int().to(DEV) if some else None, update_x=bool(update))  # fmt: skip
+        v = x.double() + a * d1.double() + b * d2.double()
+        want = x.clone()
+        if (a or b) and update:
+            want[sel] = v[sel].float()
+        assert (xs.cpu() - want).abs().max() <= 2.0**-22 * v.abs().max()  # two sums in 32 bits
+        normed = v[sel] / (v[sel].square().mean(-1, keepdim=True) + 1e-6).sqrt()
+        for o, w in zip(out, (w1, w2)):
+            ref = normed * w.double()
+            tol = 2e-6 if dtype == "float32" else 2.0**-8
+            assert ((o.cpu().double() - ref).abs() <= tol * ref.abs() + 1e-5).all()
+
+
 def test_short_convolution_and_its_history():
     """Taps of 1 to 5 over rows of every length from a history that another request left: the first tokens of a
     sequence see zeros, a row of one token sees the last taps - 1 inputs of the rows before."""
