@@ -652,6 +652,11 @@ def _few_rows(rows: int, k: int, n: int, max_k=None, w=None) -> bool:
             and strips * rows * k * 2 <= SKINNY_TWO_MAX_ACT_BYTES)  # fmt: skip
 
 
+def few_rows_product(a, w) -> bool:
+    """Whether `gemm` of these bf16 matrices with bf16 results goes through the few-rows kernels."""
+    return a.dtype == BF16 and _few_rows(a.shape[0], a.shape[1], _rows(w).shape[0], w=w)
+
+
 def gemm(a, w, out, choices=None) -> None:
     """out[M, N] = a[M, K] @ w[N, K]^T.  fp32: own kernel (true fp32).  bf16: own kernel for few
     rows, the library's matrix product otherwise; `out` may be bf16 or (few rows) fp32.
@@ -806,6 +811,8 @@ class ProductChoices:
                     choice = self.choice[key] = -1  # the library offers nothing for this shape through this door
                 elif self.fixed or (count == 1 and not _own_candidates(M, N, K, out.dtype, w)):
                     choice = self.choice[key] = 0  # the library's first candidate, which is what torch.mm runs
+                elif _plain_tile_strips(M, N, K, out.dtype) and _own_candidates(M, N, K, out.dtype, w):
+                    choice = self.choice[key] = OWN_CANDIDATE + _plain_tile_strips(M, N, K, out.dtype)
                 elif M not in self.tuned_rows:
                     choice = self._choice_of_tuned_rows(M, N, K, out.dtype)  # a prompt of any length: what its bucket settled on
                     if choice is None:
@@ -884,8 +891,9 @@ def _trial_run(trial, a, w, out, M, N, K) -> None:
 
 
 def _fastest_of(trial) -> int:
-    """The candidate whose runs took least on average, among the runs that were timed and have
-    finished and leaving out each candidate's first (which loads the kernel); 0 if none."""
+    """The candidate whose shortest run took least, among the runs that were timed and have finished and leaving out each
+    candidate's first (which loads the kernel); 0 if none.  (A run is lengthened by whatever the host does between its two
+    events, never shortened: on averages qkv of 16 rows at Qwen3-4B sizes went to 12.5 us instead of 9.3 in one process of three.)"""
     times = {}
     for candidate, start, end in trial["runs"]:
         if start is not None and end.query():
@@ -893,9 +901,8 @@ def _fastest_of(trial) -> int:
     best, best_time = 0, float("inf")
     for candidate, took in times.items():
         rest = took[1:] or took
-        mean = sum(rest) / len(rest)
-        if mean < best_time:
-            best, best_time = candidate, mean
+        if min(rest) < best_time:
+            best, best_time = candidate, min(rest)
     return best
 
 
@@ -949,6 +956,29 @@ def _wide_tile_strips(rows: int, n: int, k: int) -> int:
         return 0
     strips = 2 if rows <= 24 else 4 if rows <= 32 or (k <= 1024 and rows <= 64) else 8
     return strips if n >= 16 * strips * compute_units() else 0
+
+
+PLAIN_TILE_MAX_ROWS = 64
+
+
+def _plain_tile_strips(rows: int, n: int, k: int, dtype) -> int:
+    """Strips of 16 weight rows per workgroup of the tile kernel for a plain bf16 product that takes it without trials, 0 where trials
+    decide.  A trial times candidates on whatever the memory-side cache holds and beside the launches' own time: for qkv of 64 rows
+    at Qwen3-8B sizes two processes of five settled on the library's kernel (four steps 6,480 us instead of 6,320).  Weights read
+    from memory, replayed, us of the tile kernel with 2 and with 4 strips and of the library's best of 16:
+    N, K             16 rows            32 rows            48 rows            64 rows            96 rows
+    4,096, 1,024    4.4  5.2  6.3     4.8  6.1  6.4     5.4  6.6  8.0     6.1  7.3  8.2     7.4  8.9  9.0
+    4,096, 2,048    6.4  8.3  7.0     7.0  9.6  8.7     8.0 10.8 12.0     8.9 11.6  9.9    11.0 14.1 12.6
+    6,144, 2,560    9.3 12.5 11.1     9.2 12.3 11.6    10.6 13.7 13.3    11.8 15.1 13.8    14.6 17.8 16.0
+    6,144, 4,096   13.7 17.9 14.0    13.7 17.5 15.2    15.3 19.5 17.6    17.0 21.4 18.1    20.9 25.6 20.6
+    7,168, 5,120   16.1 23.1 18.6    18.8 25.8 21.0    18.9 25.0 22.5    20.6 26.8 23.3    25.6 32.1 26.7
+    10,240, 5,120  24.7 23.0 26.7    28.6 27.0 30.9    32.9 26.8 30.1    36.4 28.9 30.1    46.3 33.8 35.1
+    2,560, 9,728   21.4 30.1 18.1    24.2 35.4 20.5    28.2 40.0 20.8    31.8 44.1 25.4    40.1 53.5 25.5
+    so up to 64 rows it runs where K is short enough for a workgroup to walk whole and there are strips for half of the compute
+    units, with tiles of 2 strips while one round of workgroups holds them."""
+    if dtype != BF16 or not SKINNY_MAX_ROWS < rows <= PLAIN_TILE_MAX_ROWS or k > 5120 or n < 16 * compute_units():
+        return 0
+    return 2 if n <= 32 * compute_units() else 4
 
 
 def _gated_tile_strips(rows: int, outputs: int) -> int:

@@ -9,6 +9,8 @@ from atomserve_amd.kernels import ops
 from atomserve_amd.kernels.lib import Launches
 from atomserve_amd.models import repeats
 from atomserve_amd.parts.base import BuildEnv, GatedDelta, WeightDecl, build
+from atomserve_amd.parts.block import PreNormBlock
+from atomserve_amd.parts.norm import LastNorm
 from atomserve_amd.parts.plan import ModelPlan
 
 
@@ -174,8 +176,11 @@ class DecoderModel:
         p, r = self.plan, self.plan.run[i]
         # the norm that the run after this one starts with: this run's last product may add
         # into x and leave that norm pending instead of handing over a delta
-        follows = self.blocks[p.run[i + 1].layer].first_norm() if i + 1 < len(p.run) else None
         block = self.blocks[r.layer]
+        if i + 1 < len(p.run):
+            follows = self.blocks[p.run[i + 1].layer].first_norm()
+        else:
+            follows = LastNorm(self.final_norm) if isinstance(block, PreNormBlock) else None
         extra = {}
         kept = block.cache_request()
         if kept:

@@ -115,6 +115,21 @@ class RMSNorm(Norm):
 register("norm", "rmsnorm", RMSNorm)
 
 
+class LastNorm:
+    """The norm before the head, as the last layer's part sees it: it selects rows, so nothing is left pending in a product for
+    it, but where the tile kernel makes the product whole sums in parts spare it a long walk over K (four steps of 64 requests at
+    Qwen3-8B sizes 6,303 -> 6,252 us, of 13 at -4B sizes 3,915 -> 3,875: a product of 34 us, of 16, and the norm after it)."""
+
+    takes_split_sums = False
+
+    def __init__(self, norm):
+        self.norm = norm
+
+    def absorb(self, a, w, x):
+        self.takes_split_sums = self.norm.takes_split_sums and not ops.few_rows_product(a, w)
+        return None
+
+
 class LayerNorm(Norm):
     """(x - mean) / sqrt(mean((x - mean)^2) + eps) * gain: a row's mean comes off before it is divided by what is then its
     root mean square; no bias.  fp32 until the one rounding at the end."""

@@ -94,6 +94,16 @@ def test_how_products_of_17_to_128_rows_are_tiled():
     assert [ops._gated_tile_strips(*case) for case in ((64, 12288), (64, 3072), (128, 25600))] == [6, 2, 8]
 
 
+def test_which_plain_products_take_the_tile_kernel_without_trials(monkeypatch):
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    strips = ops._plain_tile_strips
+    for rows in (17, 48, 64):
+        assert [strips(rows, n, k, ops.BF16) for n, k in ((4096, 1024), (6144, 4096), (8192, 5120), (8208, 5120), (10240, 5120))] == [2, 2, 2, 4, 4]
+        assert [strips(rows, n, k, ops.BF16) for n, k in ((4080, 1024), (4096, 8192), (2560, 9728))] == [0, 0, 0]
+        assert strips(rows, 6144, 4096, ops.F32) == 0
+    assert strips(16, 6144, 4096, ops.BF16) == strips(65, 6144, 4096, ops.BF16) == 0
+
+
 def test_how_rows_of_a_state_space_are_cut_into_segments():
     """One long row fills the GPU in segments, whatever short rows stand beside it; many rows of its length stay whole."""
     choose = ops._state_space_segments

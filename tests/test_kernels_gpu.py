@@ -545,6 +545,29 @@ def test_the_tile_product_is_a_candidate_beside_the_librarys(ops, M, N, K):
             assert close_bf16(out, ref, scale=1.0)
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 256), (37, 6144, 1024), (64, 10256, 512)])
+def test_a_tile_product_that_runs_without_trials(ops, M, N, K):
+    """Rows of 17 to 64, wide outputs: the rule's tile kernel, at tuned row counts and others, unless choices are fixed or the weights
+    have no copy in wave order."""
+    torch.manual_seed(6)
+    a = torch.randn(M, K, device=DEV).to(BF16)
+    bare = (torch.randn(N, K, device=DEV) / math.sqrt(K)).to(BF16)
+    w, ref, strips = ops.Streamed(bare), pk.gemm(a, bare), ops._plain_tile_strips(M, N, K, BF16)
+    assert strips == (2 if N <= 8192 else 4)
+    for tuned, fixed in ((False, False), (True, False), (False, True)):
+        choices = ops.ProductChoices(fixed=fixed)
+        if tuned:
+            choices.tune_rows(M)
+        out = torch.full((M, N), float("nan"), dtype=BF16, device=DEV)
+        choices.gemm(a, w, out, M, N, K)
+        assert close_bf16(out, ref, scale=1.0) and not choices.trials
+        assert choices.chosen() == {(M, N, K, BF16): 0 if fixed else ops.OWN_CANDIDATE + strips}
+    choices = ops.ProductChoices()
+    out.fill_(float("nan"))
+    choices.gemm(a, bare, out, M, N, K)
+    assert close_bf16(out, ref, scale=1.0) and all(c < ops.OWN_CANDIDATE for c in choices.chosen().values())
+
+
 def test_library_candidates_replay_from_a_graph(ops):
     """Each candidate captured once and replayed with other inputs and a workspace full of noise,
     with eager work and synchronisations between the replays: every replay gives what the eager
