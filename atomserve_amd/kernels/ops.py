@@ -1977,12 +1977,43 @@ def rglru_scan(a, x, proj, y_off, y_bias, scale, state, step_rows, out, out_off,
 # ---- experts ------------------------------------------------------------------------------------------
 
 MOE_TILES = (64, 128)  # pairs of one expert that a tile of the grouped products holds: of few pairs, of many
-# Large tiles read every weight once where small ones read it for every 64 pairs, and make a quarter of the workgroups: from this many
-# pairs an expert on where all experts' first matrices have MOE_WIDE_ROWS rows (16 experts, gate and up of 1,536 at width 2,048, both
-# products: 400 tokens of two experts 79 us in small tiles and 77 in large ones, 600 109 and 86, 1,500 191 and 127), later where they have
-# fewer (gate and up of 768 at width 1,024: 1,000 tokens 46 and 53, 1,500 64 and 50)
-MOE_MANY, MOE_MANY_NARROW, MOE_WIDE_ROWS = 56, 160, 49152
 MOE_MAX_EXPERTS = 1024
+
+
+# Pairs an expert from which on tiles of 128 are the faster ones, and the values of all experts' first matrices (gate and up,
+# both in bf16) that the first of the two lines needs (`moe_tile`).
+MOE_MANY, MOE_MANY_SMALL, MOE_LARGE_WEIGHTS = 56, 128, 60 << 20
+
+
+def _moe_streamed(w, gated: bool) -> bool:
+    """Whether the grouped product with w [experts, N_w, K] runs on the kernel that takes its weights straight into registers
+    (`as_moe_gemm`: K in whole blocks of 128, outputs in strips of 16, 16-byte rows, 32-bit offsets within an expert)."""
+    rows, K = w.shape[1], w.shape[2]
+    return (w.dtype == BF16 and K % 128 == 0 and rows % (32 if gated else 16) == 0 and w.data_ptr() % 16 == 0
+            and rows * K * 2 <= 0xF0000000)  # fmt: skip
+
+
+def moe_tile(pairs: int, first, second, gated: bool) -> int:
+    """Pairs a tile of a route whose grouped products read `first` [experts, N_w, K] and then `second`; decides speed alone.
+    Only the kernel that streams weights gains from tiles of 128, which read every weight once where tiles of 64 read it for every 64
+    pairs, and make a quarter of the workgroups: the LDS kernel takes such a tile as two halves, half of whose workgroups then find
+    nothing (32 experts of 2,880 at width 2,880, four a token, 1,500 tokens: 892 us in tiles of 64, 973 of 128), and the 32-bit kernel walks
+    it in one workgroup (16 experts of 768 at width 1,024, 1,000 tokens of two: 3,944 and 5,852).  Both products of a layer, us in tiles of
+    64 / of 128, by pairs an expert (16 experts, two a token; gate and up, their values in millions):
+                          38        62        75        100       125       162
+    width 1,024,  25 M    27/41     41/44     40/46     41/53     45/53     55/50
+    2,048,        50 M    44/59     51/66     70/67     77/76     79/77     99/74
+    1,024 of 1,536, 50 M  44/57     53/60     64/64     66/72     81/93     86/84
+    2,048,        67 M    51/65     72/70     76/74     78/82     101/83    120/77
+    2,048,       101 M    79/79     97/89     107/96    113/100   134/137   161/127
+    4,096,       101 M    80/100    130/107   136/111   142/122   150/138   187/140
+    4,096,       403 M    257/269   345/289   388/287   405/320   468/392   595/482
+    Up to 64 pairs an expert both read every weight once and small tiles fill more compute units; from 65 to 128 small tiles read it
+    twice, which larger matrices feel; above that three times."""
+    if not (_moe_streamed(first, gated) and _moe_streamed(second, False)):
+        return MOE_TILES[0]
+    many = MOE_MANY if first.numel() >= MOE_LARGE_WEIGHTS else MOE_MANY_SMALL
+    return MOE_TILES[pairs >= many * first.shape[0]]
 
 
 class ExpertRoute:
@@ -1990,10 +2021,8 @@ class ExpertRoute:
 
     __slots__ = ("order", "tiles", "counts", "max_tiles", "top", "num_tokens", "pair_weight", "pair_expert", "tile")
 
-    def __init__(self, num_tokens: int, top: int, experts: int, device, weight_rows: int = 0, tile: int = None):
-        pairs = num_tokens * top
-        many = MOE_MANY if weight_rows == 0 or weight_rows >= MOE_WIDE_ROWS else MOE_MANY_NARROW
-        self.tile = MOE_TILES[pairs >= many * experts] if tile is None else tile
+    def __init__(self, num_tokens: int, top: int, experts: int, device, tile: int = MOE_TILES[0]):
+        pairs, self.tile = num_tokens * top, tile
         self.max_tiles = -(-pairs // self.tile) + experts
         self.order = torch.empty(max(pairs, 1), dtype=I32, device=device)
         self.tiles = torch.empty((self.max_tiles, 3), dtype=I32, device=device)
@@ -2003,25 +2032,24 @@ class ExpertRoute:
         self.pair_expert = None  # int32 [pairs]: each pair's expert, where a router says
 
 
-def moe_route_table(token_ids, table, experts: int, weight_rows: int = 0, tile: int = None) -> ExpertRoute:
-    """Routes by a table [vocab, top] int32 that names every token id's experts.  weight_rows (here and below): of all experts'
-    first matrices, where known, and tile (64 or 128, for tests): how the pairs are cut into tiles, which decides speed alone."""
+def moe_route_table(token_ids, table, experts: int, tile: int = MOE_TILES[0]) -> ExpertRoute:
+    """Routes by a table [vocab, top] int32 that names every token id's experts.  tile (here and below): see `moe_tile`."""
     _check(token_ids, "token_ids", I32, (None,))
     _check(table, "table", I32, (None, None))
     vocab, top = table.shape
     if not 1 <= experts <= MOE_MAX_EXPERTS:
         raise KernelError(f"routing sorts up to {MOE_MAX_EXPERTS} experts, not {experts}")
-    route = ExpertRoute(token_ids.shape[0], top, experts, token_ids.device, weight_rows, tile)
+    route = ExpertRoute(token_ids.shape[0], top, experts, token_ids.device, tile)
     call("as_moe_route_table", _ptr(token_ids), _ptr(table), vocab, top, experts, token_ids.shape[0], _ptr(route.order),
          _ptr(route.tiles), _ptr(route.counts), route.max_tiles, 0, route.tile, _stream())  # fmt: skip
     return route
 
 
-def moe_route_sigmoid(h, router, top: int, weight_rows: int = 0) -> ExpertRoute:
+def moe_route_sigmoid(h, router, top: int, tile: int = MOE_TILES[0]) -> ExpertRoute:
     """Routes by a router's scores: z = router h in fp32, s = sigmoid(z), a token's `top` experts those with the
     largest s, weighing s / (their sum + 1e-20).  h [T, K], router [experts, K] of one dtype.  The route carries
     `pair_weight` fp32 [T * top] for `moe_combine`."""
-    return moe_route_scores(h, router, top, "sigmoid", weight_rows=weight_rows)
+    return moe_route_scores(h, router, top, "sigmoid", tile=tile)
 
 
 ROUTER_SCORES = {"sigmoid": 0, "softmax_of_chosen": 1, "softmax": 2}
@@ -2029,7 +2057,7 @@ ROUTER_SCORES = {"sigmoid": 0, "softmax_of_chosen": 1, "softmax": 2}
 
 def moe_route_scores(h, router, top: int, score: str, bias=None, groups: int = 1, keep_groups: int = 1,
                      weight_scale: float = 1.0, correction=None, identity: int = 0,
-                     weight_rows: int = 0) -> ExpertRoute:  # fmt: skip
+                     tile: int = MOE_TILES[0]) -> ExpertRoute:  # fmt: skip
     """Routes by a router's logits z = router h + bias in fp32 (bias fp32 [experts] or None).  score "sigmoid": the
     `top` largest sigmoid(z), weighing s / (their sum + 1e-20); "softmax_of_chosen": the `top` largest z, weighing the
     softmax over those z alone; "softmax": s = softmax(z) over all experts, the `top` largest among the experts of the
@@ -2057,7 +2085,7 @@ def moe_route_scores(h, router, top: int, score: str, bias=None, groups: int = 1
         raise KernelError("groups of experts and a scale of the weights belong to the score 'softmax'")
     if groups < 1 or experts % groups or not 1 <= keep_groups <= groups or keep_groups * (experts // groups) < top:
         raise KernelError(f"{experts} experts in {groups} groups of which {keep_groups} are kept do not give {top} to choose")
-    route = ExpertRoute(T, top, experts - identity, h.device, weight_rows)
+    route = ExpertRoute(T, top, experts - identity, h.device, tile)
     pair_expert = route.pair_expert = torch.empty(max(T * top, 1), dtype=I32, device=h.device)
     route.pair_weight = torch.empty(max(T * top, 1), dtype=F32, device=h.device)
     call("as_moe_route_scores", _ptr(h), _ptr(router), _ptr(bias), ROUTER_SCORES[score], _ptr(correction), int(groups),

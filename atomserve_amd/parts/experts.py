@@ -47,8 +47,8 @@ class TableExperts(FeedForward):
         key = ("table_experts", self.table.data_ptr())
         found = step.shared.get(key)
         if found is None:
-            found = step.shared[key] = ops.moe_route_table(step.token_ids, self.table, self.spec.num_experts,
-                                                                self.gate_up_weight.shape[0] * self.gate_up_weight.shape[1])  # fmt: skip
+            tile = ops.moe_tile(step.token_ids.shape[0] * self.spec.top, self.gate_up_weight, self.down_weight, gated=True)
+            found = step.shared[key] = ops.moe_route_table(step.token_ids, self.table, self.spec.num_experts, tile)
         return found
 
     def forward(self, h, step):
@@ -121,8 +121,8 @@ class RoutedExperts(FeedForward):
     def forward(self, h, step):
         s, env = self.spec, self.env
         T, dev = h.shape[0], h.device
-        route = ops.moe_route_sigmoid(h, self.router_weight, s.top, self.up_weight.shape[0] * self.up_weight.shape[1])
         pairs = T * s.top
+        route = ops.moe_route_sigmoid(h, self.router_weight, s.top, ops.moe_tile(pairs, self.up_weight, self.down_weight, gated=False))
         act = torch.empty((pairs, s.intermediate_size), dtype=env.dtype, device=dev)
         ops.moe_gemm(h, self.up_weight, route, act, gated=False, per_token=True, activation=s.activation)
         each = torch.empty((pairs, s.hidden_size), dtype=torch.float32, device=dev)
@@ -214,10 +214,10 @@ class GatedRoutedExperts(FeedForward):
         s, env = self.spec, self.env
         T, dev = h.shape[0], h.device
         clamped = s.activation == "clamped_swish"
+        pairs = T * s.top
         route = ops.moe_route_scores(h, self.router_weight, s.top, s.score, self.router_bias, s.groups, s.keep_groups,
                                      s.weight_scale, self.correction, s.identity,
-                                     self.gate_up_weight.shape[0] * self.gate_up_weight.shape[1])  # fmt: skip
-        pairs = T * s.top
+                                     ops.moe_tile(pairs, self.gate_up_weight, self.down_weight, gated=True))  # fmt: skip
         act = torch.empty((pairs, s.intermediate_size), dtype=env.dtype, device=dev)
         ops.moe_gemm(h, self.gate_up_weight, route, act, gated=True, per_token=True, limit=s.limit if clamped else 0.0)
         each = torch.empty((pairs, s.hidden_size), dtype=torch.float32, device=dev)

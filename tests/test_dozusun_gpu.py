@@ -782,3 +782,41 @@ def test_experts_products_in_tiles(N, K, mode):
     else:
         bound = (3 if mode == "relu2" else 1) * u8 * want.abs() + 1e-5
     assert ((outs[0].double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("N, K", [(24, 72), (80, 136), (130, 256)])
+@pytest.mark.parametrize("mode", ["gated", "relu2", "plain"])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_experts_products_that_stream_no_weights(N, K, mode, dtype):
+    """Sizes in no whole blocks and 32 bits, in tiles of 64 and of 128: a tile's halves, runs that end in the first or the second
+    of them, an expert without pairs; against 64 bits and bit for bit against each other."""
+    from atomserve_amd.kernels import ops
+
+    counts = [1, 63, 64, 65, 0, 96, 127, 128, 129, 192, 193, 260]
+    experts = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)]).int()
+    gen, D = torch.Generator().manual_seed(N + K), DTYPES[dtype]
+    experts = experts[torch.randperm(len(experts), generator=gen)]
+    T, E, gated = len(experts), len(counts), mode == "gated"
+    a = torch.randn(T, K, generator=gen).to(D)
+    w = torch.randn(E, 2 * N if gated else N, K, generator=gen).mul(K**-0.5).to(D)
+    outs = []
+    for tile in (64, 128):
+        route = ops.moe_route_table(torch.arange(T, dtype=torch.int32, device=DEV), experts[:, None].contiguous().to(DEV), E, tile)
+        out = torch.full((T, N), float("nan"), dtype=D, device=DEV)
+        ops.moe_gemm(a.to(DEV), w.to(DEV), route, out, gated, per_token=True, activation="relu2" if mode == "relu2" else None)
+        outs.append(out.cpu())
+    assert torch.equal(outs[0], outs[1])
+    z = torch.stack([w[int(e)].double() @ a[t].double() for t, e in enumerate(experts)])
+    want = torch.nn.functional.silu(z[:, :N]) * z[:, N:] if gated else z.clamp(min=0) ** 2 if mode == "relu2" else z
+    # one rounding of the result; before it, of a product that is squared (twice its own) or of a gated pair, whose parts the other
+    # factor, up to max |z| + 1, and |d silu| <= 1.1 carry on; in 32 bits a chain of K multiply-adds of values of at most 5 max |z|
+    unit = 2.0**-8 if dtype == "bfloat16" else K * 2.0**-24
+    m = z.abs().max()
+    bound = unit * want.abs() + 1e-5
+    if gated:
+        bound = unit * want.abs() + unit * 1.1 * 2 * m * (m + 1) * 0.25
+    elif mode == "relu2":
+        bound = 3 * unit * want.abs() + 1e-5 if dtype == "bfloat16" else 2 * unit * m * m
+    elif dtype == "float32":
+        bound = unit * m
+    assert ((outs[0].double() - want).abs() <= bound).all()

@@ -94,6 +94,32 @@ def test_how_products_of_17_to_128_rows_are_tiled():
     assert [ops._gated_tile_strips(*case) for case in ((64, 12288), (64, 3072), (128, 25600))] == [6, 2, 8]
 
 
+def test_tiles_of_experts_pairs():
+    """Tiles of 128 pairs belong to the kernel that streams weights alone, both products of a layer on it, and there to enough pairs."""
+    weights = lambda rows, k, experts=16, dtype=ops.BF16: torch.empty(experts, rows, k, dtype=dtype, device="meta")  # noqa: E731
+
+    class At:  # weights that start where they are told to
+        def __init__(self, w, at):
+            self.shape, self.dtype, self.at, self.numel = w.shape, w.dtype, at, w.numel
+
+        def data_ptr(self):
+            return self.at
+
+    def tile(pairs, first, second, gated=True, at=(0, 0)):
+        return ops.moe_tile(pairs, At(first, at[0]), At(second, at[1]), gated)
+
+    first, second = weights(3072, 2048), weights(2048, 1536)
+    assert [tile(16 * n, first, second) for n in (1, 55, 56, 300)] == [64, 64, 128, 128]
+    small = weights(1536, 1024), weights(1024, 768)
+    assert [tile(16 * n, *small) for n in (56, 127, 128, 300)] == [64, 64, 128, 128]
+    assert tile(16 * 300, weights(3072, 2048, dtype=ops.F32), weights(2048, 1536, dtype=ops.F32)) == 64
+    for rows, k, out in ((5760, 2880, 2880), (2000, 1024, 1024), (2048, 1000, 1024), (2048, 1024, 1000), (3080, 2048, 2048)):
+        assert tile(16 * 300, weights(rows, k), weights(out, rows // 2)) == 64
+    assert tile(16 * 300, first, second, at=(8, 0)) == tile(16 * 300, first, second, at=(0, 8)) == 64
+    assert tile(16 * 300, weights(4096, 4096), weights(4096, 4096), gated=False) == 128
+    assert tile(300, weights(1 << 18, 8192, 1), weights(8192, 1 << 17, 1)) == 64  # an expert beyond 32-bit offsets
+
+
 def test_which_plain_products_take_the_tile_kernel_without_trials(monkeypatch):
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     strips = ops._plain_tile_strips
