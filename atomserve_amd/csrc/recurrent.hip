@@ -11,6 +11,8 @@
 #include "common.h"
 #include "float_parts.h"
 #include "rows.h"
+#include <algorithm>
+#include <climits>
 #include <type_traits>
 
 #define CONV_MAX_TAPS 8
@@ -1393,61 +1395,105 @@ extern "C" int as_rglru_gates(const float* u, int width, int blocks, const void*
 
 // The scan: S = a S + x per channel, from zero at the start of a sequence; what leaves is
 // scale * S * gelu_tanh(y + y_bias) with y from proj [T, ld] at y_off, into out [T, ld_out] at out_off.
-// A workgroup owns 16 channels of a row and takes its tokens 1,024 at a time, a thread up to 16 neighbouring ones of one channel
-// (a shorter row's are dealt evenly to the 64 threads of a channel): it loads them all at once, composes them from the identity (the product of the decays and what the stretch ends with), the
-// stretches are chained (four of a wave by lane moves, the waves' through LDS), and the thread runs its tokens again, out of
-// its registers, from their true start.  Every input is read once, and the chain of dependent steps is 16 + 2 + 16 a thousand
-// tokens.  Neighbouring workgroups of an XCD take neighbouring channels, so that a 128-byte line of two workgroups'
-// channels enters one L2.  1,500 tokens of 2,048 channels 56 -> 18 us (45 MB: 2.5 TB/s; half of the compute units hold a
-// workgroup), 2,048 of 4,096 80 -> 28, 300 of 1,024 11.1 -> 5.7; with 16 waves' sixteenths of the row, every input read twice.
+// Three ways to walk a row:
+// a row of one token (a decode step): a thread a channel.
+// middle: a workgroup 64 channels, its 16 waves a sixteenth of the tokens each: every wave composes its stretch from the identity (the
+//   product of the decays and what the stretch ends with), the stretches are chained in LDS in order, and every wave runs its
+//   stretch again from its true start, now writing.  Every input is read twice.
+// long: a workgroup 16 channels, 1,024 tokens at a time, a thread up to 16 neighbouring ones of one channel: it loads them all at once,
+//   composes them, the stretches are chained (four of a wave by lane moves, the waves' through LDS), and the thread runs its
+//   tokens again, out of its registers.  Every input is read once and the chain of dependent steps is 16 + 2 + 16 a thousand tokens, but it
+//   takes four times the workgroups, of which a compute unit holds one and of the middle way's two: only while the step's rows of more
+//   than SCAN_LONG tokens fit two rounds of them (every other row stays with the middle way), in a kernel of its own.
+// The rows of a way are dealt to lines of workgroups by their place among them, so that no row costs workgroups that find
+// nothing to do.  Neighbouring workgroups of an XCD take neighbouring channels, so that a 128-byte line of two workgroups'
+// channels enters one L2.
+// us: every row the middle way, one workgroup of 64 channels a row / every row the long way, workgroups of every row / now.  4,096 channels:
+// 255 rows of one token beside one of 512 79 120 19, 200 beside one of two 38 93 5.8, 128 rows of 4 26 228 26, 64 of 16 27 118 26, 16 of 128 26 45 26,
+// 4 of 250 15 19 15, one of 2,048 81 27 26; 2,048 channels: one of 1,500 55 18 17 (45 MB: 2.6 TB/s; half of the compute units hold a
+// workgroup), 8 of one beside 512 17 8.6 8.1; 1,024 channels: one of 300 11.3 5.8 6.1, 4 of 250 10.2 5.5 5.7.
+template <typename T, typename W> struct Scan {
+  const float *a, *x;
+  const T* proj;
+  const W* y_bias;
+  float* state;
+  const int *row_first, *row_len, *row_start, *row_slots;
+  T* out;
+  int width, ld, y_off, ld_out, out_off, writes, num_rows;
+  float scale;
+};
 
-// Channel c of a row, token by token: rows of one token (a decode step), whose single step gives the same values either way.
-template <typename T, typename W>
-__device__ __forceinline__ void rglru_step(const float* __restrict__ a, const float* __restrict__ x, int width, const T* __restrict__ proj,
-                                           int ld, int y_off, const W* __restrict__ y_bias, float scale, float* __restrict__ state, int first,
-                                           int len, int start, int slot, int writes, T* __restrict__ out, int ld_out, int out_off, int c) {
-  float* held = state + (size_t)(slot < 0 ? 0 : slot) * width + c;
-  float S = (start > 0 && slot >= 0) ? *held : 0.f;
-  const float yb = y_bias ? to_f32(y_bias[c]) : 0.f;
-  for (int j = 0; j < len; ++j) {
-    const size_t t = (size_t)first + j;
-    S = fmaf(a[t * width + c], S, x[t * width + c]);
-    out[t * ld_out + out_off + c] = from_f32<T>(scale * S * gelu_tanhf_(to_f32(proj[t * ld + y_off + c]) + yb));
-  }
-  if (writes && slot >= 0) *held = S;
+struct ScanRow { int first, len, start, slot; };
+template <typename T, typename W> __device__ __forceinline__ ScanRow scan_row(const Scan<T, W>& p, int r) {
+  return {p.row_first[r], p.row_len[r], p.row_start[r], p.row_slots[r]};
 }
 
-#define SCAN_TOKENS 16   // a thread's
+// Channel c of a row, token by token.
+template <typename T, typename W>
+__device__ __forceinline__ void rglru_step(const Scan<T, W>& p, const ScanRow& row, int c) {
+  const int first = row.first, len = row.len, slot = row.slot;
+  float* held = p.state + (size_t)(slot < 0 ? 0 : slot) * p.width + c;
+  float S = (row.start > 0 && slot >= 0) ? *held : 0.f;
+  const float yb = p.y_bias ? to_f32(p.y_bias[c]) : 0.f;
+  for (int j = 0; j < len; ++j) {
+    const size_t t = (size_t)first + j;
+    S = fmaf(p.a[t * p.width + c], S, p.x[t * p.width + c]);
+    p.out[t * p.ld_out + p.out_off + c] = from_f32<T>(p.scale * S * gelu_tanhf_(to_f32(p.proj[t * p.ld + p.y_off + c]) + yb));
+  }
+  if (p.writes && slot >= 0) *held = S;
+}
+
+#define SCAN_TOKENS 16   // a thread's, the long way
 #define SCAN_CHANNELS 16
 #define SCAN_WAVES 16
+#define SCAN_THREADS (WAVE * SCAN_WAVES)
+#define SCAN_LONG 64     // more tokens than this may go the long way
+#define SCAN_ONLY 32     // so may a row that is the step's only one
+
 template <typename T, typename W>
-__global__ __launch_bounds__(64 * SCAN_WAVES) void rglru_scan_kernel(
-    const float* __restrict__ a, const float* __restrict__ x, int width, const T* __restrict__ proj, int ld, int y_off,
-    const W* __restrict__ y_bias, float scale, float* __restrict__ state, const int* __restrict__ row_first,
-    const int* __restrict__ row_len, const int* __restrict__ row_start, const int* __restrict__ row_slots, int writes,
-    T* __restrict__ out, int ld_out, int out_off, int tiles, int per_xcd) {
-  __shared__ float ends[2][2][SCAN_WAVES][SCAN_CHANNELS];  // [round % 2][decays, ends]
+__device__ __forceinline__ void rglru_middle(const Scan<T, W>& p, float (&ends)[2][SCAN_WAVES][WAVE], const ScanRow& row, int group) {
+  const int lane = threadIdx.x & (WAVE - 1), seg = threadIdx.x / WAVE;
+  const int first = row.first, len = row.len, slot = row.slot, c = min(group * WAVE + lane, p.width - 1);
+  const int per = (len + SCAN_WAVES - 1) / SCAN_WAVES, lo = min(len, seg * per), hi = min(len, lo + per);
+  float A = 1.f, B = 0.f;
+#pragma unroll 4
+  for (int j = lo; j < hi; ++j) {
+    const size_t t = (size_t)first + j;
+    const float av = p.a[t * p.width + c];
+    B = fmaf(av, B, p.x[t * p.width + c]);
+    A *= av;
+  }
+  float* held = p.state + (size_t)(slot < 0 ? 0 : slot) * p.width + c;
+  float S = (row.start > 0 && slot >= 0) ? *held : 0.f;
+  const float yb = p.y_bias ? to_f32(p.y_bias[c]) : 0.f;
+  ends[0][seg][lane] = A;
+  ends[1][seg][lane] = B;
+  __syncthreads();
+  for (int s = 0; s < seg; ++s) S = fmaf(ends[0][s][lane], S, ends[1][s][lane]);
+  if (group * WAVE + lane >= p.width) return;
+#pragma unroll 4
+  for (int j = lo; j < hi; ++j) {
+    const size_t t = (size_t)first + j;
+    S = fmaf(p.a[t * p.width + c], S, p.x[t * p.width + c]);
+    p.out[t * p.ld_out + p.out_off + c] = from_f32<T>(p.scale * S * gelu_tanhf_(to_f32(p.proj[t * p.ld + p.y_off + c]) + yb));
+  }
+  if (p.writes && slot >= 0 && seg == SCAN_WAVES - 1) *held = S;  // the last stretch ends where the row ends
+}
+
+// `buf`: the half of `ends` whose turn it is, from round to round and from row to row
+template <typename T, typename W>
+__device__ __forceinline__ void rglru_long(const Scan<T, W>& p, float (&ends)[2][2][SCAN_WAVES][SCAN_CHANNELS], int& buf, const ScanRow& row, int tile) {
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
   const int ch = lane & (SCAN_CHANNELS - 1), sub = lane / SCAN_CHANNELS;  // four stretches a wave
-  const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (tile >= tiles) return;
-  const int r = blockIdx.y, len = row_len[r];
-  if (len <= 1) {  // a decoding row beside a portion: a thread a channel, so that most of the row's workgroups end here
-    const int one = tile * WAVE * SCAN_WAVES + threadIdx.x;
-    if (one < width)
-      rglru_step(a, x, width, proj, ld, y_off, y_bias, scale, state, row_first[r], len, row_start[r], row_slots[r], writes, out, ld_out, out_off, one);
-    return;
-  }
-  const int mine = tile * SCAN_CHANNELS + ch, c = min(mine, width - 1);
-  const int first = row_first[r], slot = row_slots[r];
-  float* held = state + (size_t)(slot < 0 ? 0 : slot) * width + c;
-  float S = (row_start[r] > 0 && slot >= 0) ? *held : 0.f;  // the state where the round begins
-  const float yb = y_bias ? to_f32(y_bias[c]) : 0.f;
+  const int mine = tile * SCAN_CHANNELS + ch, c = min(mine, p.width - 1);
+  const int first = row.first, len = row.len, slot = row.slot;
+  float* held = p.state + (size_t)(slot < 0 ? 0 : slot) * p.width + c;
+  float S = (row.start > 0 && slot >= 0) ? *held : 0.f;  // the state where the round begins
+  const float yb = p.y_bias ? to_f32(p.y_bias[c]) : 0.f;
   const int per = min(SCAN_TOKENS, (len + 4 * SCAN_WAVES - 1) / (4 * SCAN_WAVES));
   // a thread's tokens in a straight line, as many as the row's length asks for (tests between them would make every load wait)
   auto walk = [&](auto most) {
     constexpr int N = decltype(most)::value;
-    int buf = 0;
     for (int base = 0; base < len; base += SCAN_TOKENS * 4 * SCAN_WAVES, buf ^= 1) {
       const int lo = base + (wave * 4 + sub) * per, mine_n = min(per, len - lo);  // tokens of this stretch, if any
       float av[N], xv[N], yv[N];
@@ -1455,9 +1501,9 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void rglru_scan_kernel(
 #pragma unroll
         for (int i = 0; i < N; ++i) {
           const size_t t = (size_t)first + lo + min(i, mine_n - 1);
-          av[i] = a[t * width + c];
-          xv[i] = x[t * width + c];
-          yv[i] = to_f32(proj[t * ld + y_off + c]);
+          av[i] = p.a[t * p.width + c];
+          xv[i] = p.x[t * p.width + c];
+          yv[i] = to_f32(p.proj[t * p.ld + p.y_off + c]);
         }
       }
       float A = 1.f, B = 0.f;
@@ -1494,54 +1540,132 @@ __global__ __launch_bounds__(64 * SCAN_WAVES) void rglru_scan_kernel(
       for (int i = 0; i < N; ++i) {
         if (i < mine_n) {
           s = fmaf(av[i], s, xv[i]);
-          if (mine < width)
-            out[((size_t)first + lo + i) * ld_out + out_off + c] = from_f32<T>(scale * s * gelu_tanhf_(yv[i] + yb));
+          if (mine < p.width)
+            p.out[((size_t)first + lo + i) * p.ld_out + p.out_off + c] = from_f32<T>(p.scale * s * gelu_tanhf_(yv[i] + yb));
         }
       }
     }
   };
   if (per > 8) walk(std::integral_constant<int, 16>{});
   else if (per > 4) walk(std::integral_constant<int, 8>{});
-  else if (per > 2) walk(std::integral_constant<int, 4>{});
-  else walk(std::integral_constant<int, 2>{});
-  if (writes && slot >= 0 && threadIdx.x < SCAN_CHANNELS && mine < width) *held = S;
+  else walk(std::integral_constant<int, 4>{});
+  if (p.writes && slot >= 0 && threadIdx.x < SCAN_CHANNELS && mine < p.width) *held = S;
 }
 
+// f(row) for the rows of low < length <= high in the places line, line + lines, ... among them; the whole workgroup together.  A
+// lane to a row: 16 waves that count one by one take longer than the rows.
+template <typename T, typename W, typename F>
+__device__ __forceinline__ void scan_rows(const Scan<T, W>& p, int low, int high, int line, int lines, F f) {
+  const int lane = threadIdx.x & (WAVE - 1);
+  for (int base = 0, before = 0; base < p.num_rows; base += WAVE) {
+    const ScanRow row = scan_row(p, min(base + lane, p.num_rows - 1));
+    const bool one = base + lane < p.num_rows && row.len > low && row.len <= high;
+    const unsigned long long found = __ballot(one);
+    const int place = before + __popcll(found & ((1ull << lane) - 1));
+    before += __popcll(found);
+    for (; line < before; line += lines) {
+      const int l = __ffsll((unsigned long long)__ballot(one && place == line)) - 1;
+      f(ScanRow{__builtin_amdgcn_readlane(row.first, l), __builtin_amdgcn_readlane(row.len, l), __builtin_amdgcn_readlane(row.start, l),
+                __builtin_amdgcn_readlane(row.slot, l)});
+    }
+  }
+}
+
+// Workgroup `at` of those that take rows of one token, a thousand channels each
+template <typename T, typename W> __device__ __forceinline__ void scan_ones(const Scan<T, W>& p, int at) {
+  const int chunks = (p.width + SCAN_THREADS - 1) / SCAN_THREADS, r = at / chunks, c = at % chunks * SCAN_THREADS + (int)threadIdx.x;
+  if (r >= p.num_rows) return;
+  const ScanRow row = scan_row(p, r);
+  if (c < p.width && row.len <= 1) rglru_step(p, row, c);
+}
+
+#define SCAN_PARAMS                                                                                                                     \
+  const float *__restrict__ a, const float *__restrict__ x, int width, const T *__restrict__ proj, int ld, int y_off,                   \
+      const W *__restrict__ y_bias, float scale, float *__restrict__ state, const int *__restrict__ row_first,                          \
+      const int *__restrict__ row_len, const int *__restrict__ row_start, const int *__restrict__ row_slots, int writes,                \
+      T *__restrict__ out, int ld_out, int out_off, int num_rows
+#define SCAN_STRUCT                                                                                                                     \
+  const Scan<T, W> p = {a, x, proj, y_bias, state, row_first, row_len, row_start, row_slots, out, width, ld, y_off, ld_out, out_off,     \
+                        writes, num_rows, scale}
+
+// blockIdx.y < lines: long rows; beyond: rows of one token
 template <typename T, typename W>
-__global__ __launch_bounds__(WAVE) void rglru_step_kernel(
-    const float* __restrict__ a, const float* __restrict__ x, int width, const T* __restrict__ proj, int ld, int y_off,
-    const W* __restrict__ y_bias, float scale, float* __restrict__ state, const int* __restrict__ row_first,
-    const int* __restrict__ row_len, const int* __restrict__ row_start, const int* __restrict__ row_slots, int writes,
-    T* __restrict__ out, int ld_out, int out_off) {
-  const int r = blockIdx.y, c = blockIdx.x * WAVE + threadIdx.x;
-  if (c < width)
-    rglru_step(a, x, width, proj, ld, y_off, y_bias, scale, state, row_first[r], row_len[r], row_start[r], row_slots[r], writes, out,
-               ld_out, out_off, c);
+__global__ __launch_bounds__(SCAN_THREADS) void rglru_long_kernel(SCAN_PARAMS, int lines, int per_xcd) {
+  SCAN_STRUCT;
+  __shared__ float ends[2][2][SCAN_WAVES][SCAN_CHANNELS];  // [round % 2][decays, ends]
+  if ((int)blockIdx.y >= lines) return scan_ones(p, ((int)blockIdx.y - lines) * per_xcd * 8 + (int)blockIdx.x);
+  const int tile = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if (tile * SCAN_CHANNELS >= width) return;
+  int buf = 0;
+  if (lines == num_rows) rglru_long(p, ends, buf, scan_row(p, blockIdx.y), tile);  // all of them
+  else scan_rows(p, SCAN_LONG, INT_MAX, blockIdx.y, lines, [&](const ScanRow& row) { rglru_long(p, ends, buf, row, tile); });
 }
 
-// num_tokens: of the whole step; as many as rows: every row has one.
+// BY_ROW: row blockIdx.y, whatever its length.  Else `lines` times the groups of 64 channels workgroups: rows of 2 to `high` tokens; the
+// others: rows of one token
+template <typename T, typename W, bool BY_ROW>
+__global__ __launch_bounds__(SCAN_THREADS, 8) void rglru_scan_kernel(SCAN_PARAMS, int lines, int groups, int high) {
+  SCAN_STRUCT;
+  __shared__ float ends[2][SCAN_WAVES][WAVE];
+  if constexpr (BY_ROW) {
+    rglru_middle(p, ends, scan_row(p, blockIdx.y), blockIdx.x);
+  } else {
+    if ((int)blockIdx.x >= lines * groups) return scan_ones(p, (int)blockIdx.x - lines * groups);
+    const int line = (int)blockIdx.x / groups, group = (int)blockIdx.x % groups;
+    scan_rows(p, 1, high, line, lines, [&](const ScanRow& row) {
+      __syncthreads();  // the row before has been read
+      rglru_middle(p, ends, row, group);
+    });
+  }
+}
+
+template <typename T, typename W> __global__ __launch_bounds__(WAVE) void rglru_step_kernel(SCAN_PARAMS) {
+  SCAN_STRUCT;
+  const int c = blockIdx.x * WAVE + threadIdx.x;
+  if (c < width) rglru_step(p, scan_row(p, blockIdx.y), c);
+}
+
+// num_tokens: of the whole step; as many as rows: every row has one.  several, many: rows of more than one token, of more than SCAN_LONG
+// (< 0: not known), by which workgroups are dealt out.
 extern "C" int as_rglru_scan(const float* a, const float* x, int width, const void* proj, int dtype, int ld, int y_off,
                              const void* y_bias, int w_dtype, float scale, float* state, const int* row_first,
                              const int* row_len, const int* row_start, const int* row_slots, int writes, void* out,
-                             int ld_out, int out_off, int num_rows, int num_tokens, hipStream_t stream) {
+                             int ld_out, int out_off, int num_rows, int num_tokens, int several, int many, hipStream_t stream) {
   if (num_rows <= 0) return AS_OK;
   if (width <= 0 || num_rows > 65535 || ld < y_off + width || ld_out < out_off + width) return AS_BAD_SHAPE;
-  const int tiles = (width + SCAN_CHANNELS - 1) / SCAN_CHANNELS, per_xcd = (tiles + 7) / 8;
+  const int tiles = (width + SCAN_CHANNELS - 1) / SCAN_CHANNELS, per_xcd = (tiles + 7) / 8, all = per_xcd * 8;
+  const int groups = (width + WAVE - 1) / WAVE, chunks = (width + SCAN_THREADS - 1) / SCAN_THREADS, cus = compute_units();
+  const bool only = num_rows == 1, known = several >= 0 && many >= 0;
+  if (!known) several = num_rows, many = 0;
+  // two rounds of workgroups of either way at most; a line a row where few rows or none have one token
+  const bool long_way = only ? num_tokens > SCAN_ONLY : many > 0 && many <= std::max(1, 2 * cus / tiles);
+  const bool by_row = !long_way && (only || (known && several == num_rows) || (long)num_rows * groups <= 2 * cus);
+  const int longs = only ? 1 : many, middle = only ? 0 : several - (long_way ? many : 0);
+  const int lines = by_row ? 0 : std::min(middle, std::max(1, 4 * cus / groups));
+  const long ones = by_row || only || (known && several == num_rows) ? 0 : (long)num_rows * chunks;
+  const long blocks = (long)lines * groups + (long_way ? 0 : ones);
+  if (blocks > 0x3fffff) return AS_BAD_SHAPE;
+#define ARGS(T, W)                                                                                                       \
+  a, x, width, (const T*)proj, ld, y_off, (const W*)y_bias, scale, state, row_first, row_len, row_start, row_slots, writes, \
+      (T*)out, ld_out, out_off, num_rows
 #define LAUNCH(T, W)                                                                                                     \
   do {                                                                                                                   \
-    if (num_tokens == num_rows)                                                                                          \
-      rglru_step_kernel<T, W><<<dim3((width + WAVE - 1) / WAVE, num_rows), WAVE, 0, stream>>>(                           \
-          a, x, width, (const T*)proj, ld, y_off, (const W*)y_bias, scale, state, row_first, row_len, row_start,         \
-          row_slots, writes, (T*)out, ld_out, out_off);                                                                  \
-    else                                                                                                                 \
-      rglru_scan_kernel<T, W><<<dim3(per_xcd * 8, num_rows), WAVE * SCAN_WAVES, 0, stream>>>(                            \
-          a, x, width, (const T*)proj, ld, y_off, (const W*)y_bias, scale, state, row_first, row_len, row_start,         \
-          row_slots, writes, (T*)out, ld_out, out_off, tiles, per_xcd);                                                  \
+    if (num_tokens == num_rows) {                                                                                        \
+      rglru_step_kernel<T, W><<<dim3(groups, num_rows), WAVE, 0, stream>>>(ARGS(T, W));                                  \
+      break;                                                                                                             \
+    }                                                                                                                    \
+    if (long_way)                                                                                                        \
+      rglru_long_kernel<T, W><<<dim3(all, longs + (int)((ones + all - 1) / all)), SCAN_THREADS, 0, stream>>>(ARGS(T, W), longs, per_xcd); \
+    if (by_row)                                                                                                          \
+      rglru_scan_kernel<T, W, true><<<dim3(groups, num_rows), SCAN_THREADS, 0, stream>>>(ARGS(T, W), 0, groups, 0);       \
+    else if (blocks > 0)                                                                                                 \
+      rglru_scan_kernel<T, W, false><<<(int)blocks, SCAN_THREADS, 0, stream>>>(ARGS(T, W), lines, groups, long_way ? SCAN_LONG : INT_MAX); \
   } while (0)
   if (dtype == DT_F32 && w_dtype == DT_F32) LAUNCH(float, float);
   else if (dtype == DT_BF16 && w_dtype == DT_BF16) LAUNCH(bf16, bf16);
   else if (dtype == DT_BF16 && w_dtype == DT_F32) LAUNCH(bf16, float);
   else return AS_BAD_DTYPE;
+#undef ARGS
 #undef LAUNCH
   return launch_status();
 }

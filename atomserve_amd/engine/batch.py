@@ -89,7 +89,7 @@ class StepBatch:
     split((short, tile)): the rows sorted as a mixer asks (`RowSplit`), one for every distinct answer of
     the model's mixers (`row_splits`), so that mixers with different kernels share a step;
     row_first, row_len, row_start, row_slots [R] int32 (for mixers with per-request state); longest_row: the
-    most tokens that a row brings (known on the host)
+    most tokens that a row brings; row_kinds: how many rows bring more than one, and more than 64 (known on the host)
     """
 
     def __init__(self, rows, block_size: int, num_paged_groups: int, vocab_size: int, device, pools=None,
@@ -276,6 +276,7 @@ class StepBatch:
 
         self.num_tokens, self.num_rows = T, R
         self.longest_row = max(len(row.tokens) for row in rows)
+        self.row_kinds = (0, 0) if T == R else (sum(n > 1 for n in row_len), sum(n > 64 for n in row_len))
         self.decode_only = all(len(row.tokens) == 1 for row in rows)  # token t is row t
         self.token_ids, self.positions, self.tok_row = parts["token_ids"], parts["positions"], parts["tok_row"]
         self.logits_rows, self.num_logits = parts["logits_rows"], len(want)

@@ -1953,9 +1953,10 @@ def rglru_gates(u, ra, ra_bias, ri, ri_bias, lam, c, a_out, x_out) -> None:
          _DT[ra.dtype], float(c), _ptr(a_out), _ptr(x_out), T, _stream())  # fmt: skip
 
 
-def rglru_scan(a, x, proj, y_off, y_bias, scale, state, step_rows, out, out_off, writes=True) -> None:
+def rglru_scan(a, x, proj, y_off, y_bias, scale, state, step_rows, out, out_off, writes=True, row_kinds=None) -> None:
     """S = a S + x per channel over each row's tokens (state fp32 [slots, width]; from zero at position 0);
-    out[t, out_off + c] = scale * S * gelu_tanh(proj[t, y_off + c] + y_bias[c])."""
+    out[t, out_off + c] = scale * S * gelu_tanh(proj[t, y_off + c] + y_bias[c]).  row_kinds: how many rows bring more than one token and
+    how many more than 64, where known (`StepBatch.row_kinds`): how the work is dealt out."""
     _check(a, "a", F32, (None, None))
     T, width = a.shape
     _check(x, "x", F32, (T, width))
@@ -1971,7 +1972,7 @@ def rglru_scan(a, x, proj, y_off, y_bias, scale, state, step_rows, out, out_off,
     _, row_first, row_len, row_start, row_slots = step_rows
     call("as_rglru_scan", _ptr(a), _ptr(x), width, _ptr(proj), _DT[proj.dtype], proj.shape[1], y_off, _ptr(y_bias),
          _DT[w_dtype], float(scale), _ptr(state), _ptr(row_first), _ptr(row_len), _ptr(row_start), _ptr(row_slots),
-         int(bool(writes)), _ptr(out), out.shape[1], out_off, R, T, _stream())  # fmt: skip
+         int(bool(writes)), _ptr(out), out.shape[1], out_off, R, T, *(row_kinds or (-1, -1)), _stream())  # fmt: skip
 
 
 # ---- experts ------------------------------------------------------------------------------------------

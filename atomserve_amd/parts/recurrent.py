@@ -218,7 +218,7 @@ class SideBySide(Mixer):
         ops.rglru_gates(u, self.gate_a_weight, self.gate_a_bias, self.gate_i_weight, self.gate_i_bias, self.lam,
                         r.decay_scale, decay, fresh)  # fmt: skip
         ops.rglru_scan(decay, fresh, proj, self.y_off, self.y_bias, s.right_scale, state.state, rows, act,
-                       H * a.value_dim, writes=state.writes)  # fmt: skip
+                       H * a.value_dim, writes=state.writes, row_kinds=step.row_kinds)  # fmt: skip
         y = torch.empty((T, s.hidden_size), dtype=env.dtype, device=dev)
         ops.gemm(act, self.out, y, env.products)
         return y

@@ -741,6 +741,51 @@ def test_scan_of_a_linear_recurrence(width, dtype, bias):
         assert ((out[first[i] : first[i] + n, 8:].double() - want).abs() <= tol * want.abs() + 1e-5).all()
 
 
+@pytest.mark.parametrize("width, lens", [
+    (2048, [1] * 40 + [70] + [1] * 3 + [512]),  # long rows and ones
+    (2048, [1] * 20 + [2, 37, 64, 65] + [1] * 5),  # one long row, middle ones and ones
+    (2048, [1] * 30 + [100] * 5 + [3]),  # more long rows than fit two rounds
+    (2048, [9] * 18 + [65]), (1024, [9] * 18),  # no row of one token
+    (100, [1, 5, 80, 1, 1030]), (2048, [1] * 66 + [5] + [1] * 70 + [70] + [2] * 3),  # rows beyond the first 64
+    (48, [2]), (100, [32]), (100, [33]), (16, [1025]),
+])  # fmt: skip
+def test_scan_of_many_and_few_rows(width, lens):
+    """Every way in which a step's rows are dealt out, by the numbers of rows that the host knows and without them: rows of one token
+    have the bits that they have alone, the others are the recurrence in 64 bits, nobody else's state changes."""
+    from atomserve_amd.kernels import ops
+
+    R, T = len(lens), sum(lens)
+    gen = torch.Generator().manual_seed(T)
+    a, x = torch.rand(T, width, generator=gen) * 0.2 + 0.8, torch.randn(T, width, generator=gen)
+    proj, state = torch.randn(T, width, generator=gen), torch.randn(R + 2, width, generator=gen)
+    first = [sum(lens[:i]) for i in range(R)]
+    starts, slots = [i % 3 for i in range(R)], torch.randperm(R + 2, generator=gen)[:R].tolist()
+    a, x, proj = (t.to(DEV) for t in (a, x, proj))
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    want, S = torch.empty(T, width, dtype=torch.float64, device=DEV), state.to(DEV).double()
+    for i, n in enumerate(lens):
+        s = S[slots[i]] if starts[i] else torch.zeros(width, dtype=torch.float64, device=DEV)
+        for t in range(first[i], first[i] + n):
+            s = want[t] = a[t].double() * s + x[t].double()
+        S[slots[i]] = s
+    z = proj.double()
+    want = want * 0.5 * z * (1 + torch.tanh(math.sqrt(2 / math.pi) * (z + 0.044715 * z**3)))
+    alone = [i for i, n in enumerate(lens) if n == 1]
+    for kinds in (None, (sum(n > 1 for n in lens), sum(n > 64 for n in lens))):
+        st, out = state.to(DEV), torch.full((T, width + 8), 7.0, device=DEV)
+        ops.rglru_scan(a, x, proj, 0, None, 1.0, st, (None, ints(first), ints(lens), ints(starts), ints(slots)), out, 8, row_kinds=kinds)
+        assert (out[:, :8] == 7).all()
+        # 1 / (1 - a) is 10 on average: some tens of roundings of 2^-24 of values of a few
+        assert (st.double() - S).abs().max() <= 5e-6 * max(1.0, S.abs().max())
+        assert ((out[:, 8:].double() - want).abs() <= 1e-5 * want.abs() + 1e-5).all()
+        if alone:
+            st1, one = state.to(DEV), torch.empty(len(alone), width, device=DEV)
+            at, take = [first[i] for i in alone], lambda v: ints([v[i] for i in alone])
+            ops.rglru_scan(a[at], x[at], proj[at], 0, None, 1.0, st1, (None, ints(range(len(alone))), take(lens), take(starts), take(slots)), one, 0)
+            own = [slots[i] for i in alone]
+            assert torch.equal(out[at, 8:], one) and torch.equal(st[own], st1[own])
+
+
 @pytest.mark.parametrize("N, K", [(16, 128), (80, 384), (272, 256), (48, 1536)])
 @pytest.mark.parametrize("mode", ["gated", "limited", "relu2", "plain", "plain32"])
 def test_experts_products_in_tiles(N, K, mode):
