@@ -966,19 +966,31 @@ def _plain_tile_strips(rows: int, n: int, k: int, dtype) -> int:
     decide.  A trial times candidates on whatever the memory-side cache holds and beside the launches' own time: for qkv of 64 rows
     at Qwen3-8B sizes two processes of five settled on the library's kernel (four steps 6,480 us instead of 6,320).  Weights read
     from memory, replayed, us of the tile kernel with 2 and with 4 strips and of the library's best of 16:
-    N, K             16 rows            32 rows            48 rows            64 rows            96 rows
-    4,096, 1,024    4.4  5.2  6.3     4.8  6.1  6.4     5.4  6.6  8.0     6.1  7.3  8.2     7.4  8.9  9.0
-    4,096, 2,048    6.4  8.3  7.0     7.0  9.6  8.7     8.0 10.8 12.0     8.9 11.6  9.9    11.0 14.1 12.6
-    6,144, 2,560    9.3 12.5 11.1     9.2 12.3 11.6    10.6 13.7 13.3    11.8 15.1 13.8    14.6 17.8 16.0
-    6,144, 4,096   13.7 17.9 14.0    13.7 17.5 15.2    15.3 19.5 17.6    17.0 21.4 18.1    20.9 25.6 20.6
-    7,168, 5,120   16.1 23.1 18.6    18.8 25.8 21.0    18.9 25.0 22.5    20.6 26.8 23.3    25.6 32.1 26.7
-    10,240, 5,120  24.7 23.0 26.7    28.6 27.0 30.9    32.9 26.8 30.1    36.4 28.9 30.1    46.3 33.8 35.1
-    2,560, 9,728   21.4 30.1 18.1    24.2 35.4 20.5    28.2 40.0 20.8    31.8 44.1 25.4    40.1 53.5 25.5
-    so up to 64 rows it runs where K is short enough for a workgroup to walk whole and there are strips for half of the compute
-    units, with tiles of 2 strips while one round of workgroups holds them."""
-    if dtype != BF16 or not SKINNY_MAX_ROWS < rows <= PLAIN_TILE_MAX_ROWS or k > 5120 or n < 16 * compute_units():
+    N, K             20 rows            32 rows            48 rows            64 rows
+    4,096, 1,024    4.8  6.0  6.3     5.0  6.3  5.5     5.6  6.8  6.4     6.2  7.5  6.8
+    4,096, 2,048    7.1  9.7  8.8     7.1  9.7  8.9     8.2 10.8 12.0     9.3 11.7  9.9
+    4,096, 2,560    7.9 11.1 10.1     8.6 11.7  9.5    10.1 13.1 10.5    11.1 14.4 10.6
+    4,096, 4,096   11.0 15.9 13.3    12.3 16.6 11.9    14.2 18.6 14.0    15.9 20.4 14.1
+    5,120, 1,024    4.9  6.4  6.5     5.2  6.5  5.9     5.8  7.0  6.8     6.4  7.7  6.9
+    5,120, 5,120   13.8 19.9 17.5    15.4 21.5 18.0    17.8 23.8 20.8    19.8 25.9 21.7
+    6,144, 2,560    8.4 11.7 11.4     9.3 12.4 11.7    10.7 13.9 13.4    11.9 15.2 13.7
+    6,144, 4,096   12.2 16.6 15.0    13.4 17.5 15.4    15.4 19.7 17.7    17.0 21.6 18.1
+    8,192, 2,048    7.9 11.8 13.3     8.3 12.3 10.5     9.2 13.0 13.7    10.3 13.8 12.3
+    8,192, 5,120   17.2 25.6 19.8    17.2 23.2 20.2    19.7 25.7 22.9    21.4 28.2 24.9
+    10,240, 2,560  14.7 14.5 16.8    15.5 13.6 16.1    18.4 15.2 18.0    20.7 16.7 18.2
+    12,288, 4,096  24.8 21.9 26.1    24.9 21.2 25.3    28.5 22.9 26.2    31.5 24.8 26.7
+    16,384, 1,024   8.8  9.0 14.0     9.1  8.9  9.9    10.1  9.6 13.9    10.9 10.3 11.0
+    16,384, 5,120  31.2 31.3 35.1    34.1 31.4 35.1    37.3 31.7 35.9    41.2 33.8 37.5
+    24,576, 2,048  19.7 25.8 25.3    21.0 26.5 24.9    22.8 26.5 25.4    25.8 28.2 25.2
+    2,560, 9,728 (32, 48, 64 rows)   24.2 35.4 20.5    28.2 40.0 20.8    31.8 44.1 25.4
+    so up to 64 rows it runs where K is short enough for a workgroup to walk whole and one round of workgroups holds the outputs, with tiles
+    of 2 strips up to 32 outputs a compute unit and of 4 up to 64; below 20 outputs a compute unit only while K is short."""
+    units = compute_units()
+    if dtype != BF16 or not SKINNY_MAX_ROWS < rows <= PLAIN_TILE_MAX_ROWS or k > 5120 or not 16 * units <= n <= 64 * units:
         return 0
-    return 2 if n <= 32 * compute_units() else 4
+    if n < 20 * units and k > 2048:
+        return 0  # o of Qwen3-8B sizes: the library's from 32 rows on
+    return 2 if n <= 32 * units else 4
 
 
 def _gated_tile_strips(rows: int, outputs: int) -> int:

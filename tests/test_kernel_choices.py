@@ -130,6 +130,15 @@ def test_which_plain_products_take_the_tile_kernel_without_trials(monkeypatch):
     assert strips(16, 6144, 4096, ops.BF16) == strips(65, 6144, 4096, ops.BF16) == 0
 
 
+def test_plain_products_that_trials_decide(monkeypatch):
+    """Where the library wins at some of 17 to 64 rows: few outputs of a longer K, and more outputs than one round of workgroups holds."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    for rows in (17, 32, 64):
+        for n, k in ((4096, 2560), (4096, 4096), (5104, 4096), (16400, 1024), (24576, 2048), (32768, 4096)):
+            assert ops._plain_tile_strips(rows, n, k, ops.BF16) == 0
+        assert [ops._plain_tile_strips(rows, n, k, ops.BF16) for n, k in ((4096, 2048), (5120, 4096), (16384, 5120))] == [2, 2, 4]
+
+
 def test_how_rows_of_a_state_space_are_cut_into_segments():
     """One long row fills the GPU in segments, whatever short rows stand beside it; many rows of its length stay whole."""
     choose = ops._state_space_segments
