@@ -139,6 +139,39 @@ def test_plain_products_that_trials_decide(monkeypatch):
         assert [ops._plain_tile_strips(rows, n, k, ops.BF16) for n, k in ((4096, 2048), (5120, 4096), (16384, 5120))] == [2, 2, 4]
 
 
+class Mark:  # an event of a timed run
+    def __init__(self, ms=None):
+        self.ms = ms
+
+    def query(self):
+        return True
+
+    def elapsed_time(self, end):
+        return end.ms
+
+
+def test_the_middle_run_of_a_trial_decides():
+    """Neither a run that the host lengthened nor one whose weights the caches still held."""
+    runs = lambda *times: {"runs": [(c, Mark(), Mark(ms)) for n in range(4) for c, ms in enumerate(t[n] for t in times)]}  # noqa: E731
+    assert ops._fastest_of(runs((9.0, 5.0, 5.1, 5.0), (9.0, 4.0, 6.0, 6.0))) == 0
+    assert ops._fastest_of(runs((9.0, 6.0, 6.0, 6.0), (9.0, 5.0, 40.0, 5.0))) == 1
+    assert ops._fastest_of({"runs": [(3, None, None)]}) == 0
+
+
+def test_the_rest_of_a_trial_runs_on_all_weights_in_turn(monkeypatch):
+    choices, met = ops.ProductChoices(), []
+
+    def run(trial, a, w, out, M, N, K):
+        met.append(w)
+        trial["runs"].append((trial["ids"][len(trial["runs"]) % trial["count"]], Mark(), Mark(1.0)))
+
+    monkeypatch.setattr(ops, "_trial_run", run)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"synchronize": lambda self: None})())
+    choices.trials[(32, 64, 64, BF16)] = {"count": 2, "ids": [0, 1], "runs": [], "weights": ["a", "b", "c"], "last": (None, "c", None)}
+    choices.settle()
+    assert met == ["a", "b", "c", "a", "b", "c", "a", "b"] and choices.chosen() == {(32, 64, 64, BF16): 0}
+
+
 def test_how_rows_of_a_state_space_are_cut_into_segments():
     """One long row fills the GPU in segments, whatever short rows stand beside it; many rows of its length stay whole."""
     choose = ops._state_space_segments
