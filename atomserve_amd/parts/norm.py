@@ -117,8 +117,10 @@ register("norm", "rmsnorm", RMSNorm)
 
 class LastNorm:
     """The norm before the head, as the last layer's part sees it: it selects rows, so nothing is left pending in a product for
-    it, but where the tile kernel makes the product whole sums in parts spare it a long walk over K (four steps of 64 requests at
-    Qwen3-8B sizes 6,303 -> 6,252 us, of 13 at -4B sizes 3,915 -> 3,875: a product of 34 us, of 16, and the norm after it)."""
+    it, but where the tile kernel makes the product whole sums in parts spare it a long walk over K.  Down product and norm, the
+    best kernel of the whole product and sums in parts, us: Qwen3-4B sizes 13 rows 19.5 14.7, -8B 64 rows 37.0 28.3, 128 rows 48.0 38.0,
+    -1.7B 48 rows 15.7 13.0; -0.6B (1,024 wide) 48 rows 9.3 9.8, 128 rows 10.7 13.6, so bf16 streams from LAST_IN_PARTS on.  Four decode steps
+    of 64 requests at -8B sizes, the same kernels otherwise: 6,304 and 6,266 us, of 13 at -4B sizes 3,891 and 3,872."""
 
     takes_split_sums = False
 
@@ -126,8 +128,12 @@ class LastNorm:
         self.norm = norm
 
     def absorb(self, a, w, x):
-        self.takes_split_sums = self.norm.takes_split_sums and not ops.few_rows_product(a, w)
+        in_parts = a.dtype == torch.float32 or (x.shape[1] >= LAST_IN_PARTS and not ops.few_rows_product(a, w))
+        self.takes_split_sums = self.norm.takes_split_sums and in_parts
         return None
+
+
+LAST_IN_PARTS = 2048
 
 
 class LayerNorm(Norm):

@@ -186,6 +186,52 @@ def test_decoding_across_the_context_bound_of_a_captured_graph(dtype, tmp_path):
     assert len(replay.runner.decode_graphs.graphs) == 2
 
 
+@pytest.mark.parametrize("hidden, dtype, rows, parts", [(2048, "bfloat16", 40, True), (2048, "bfloat16", 128, True), (2048, "bfloat16", 9, False),
+                                                        (1024, "bfloat16", 40, False), (2048, "float32", 20, True), (1024, "float32", 200, True),
+                                                        (2048, "float32", 5, False)])  # fmt: skip
+def test_the_last_layers_product_in_parts(hidden, dtype, rows, parts, tmp_path, monkeypatch):
+    """The last layer's down product as partial sums that the norm before the head adds up for the rows that it selects, all of them
+    and two of a prompt, against the product made whole: the same bits in 32 bits; in bfloat16 the sums differ by their order
+    before they are rounded, 2^-8 of what is added to the stream, and the norm's result is rounded again."""
+    from atomserve_amd.cache.manager import CacheManager
+    from atomserve_amd.engine.batch import Row
+    from atomserve_amd.engine.runner import ModelRunner
+    from atomserve_amd.kernels import ops
+    from atomserve_amd.models import decoder
+    from atomserve_amd.parts.norm import LastNorm
+    from atomserve_amd.weights.loader import load_model
+
+    raw = dict(TINY["A"], hidden_size=hidden, intermediate_size=512, num_hidden_layers=1)
+    path = write_model_dir(str(tmp_path / "wide"), raw, plain_random_weights(raw, seed=53, std=0.05, gain_std=0.2), torch.bfloat16)
+    model, _, _ = load_model(path, getattr(torch, dtype), "cuda:0")
+    made = []
+
+    class Whole(LastNorm):
+        def absorb(self, a, w, x):
+            return None
+
+    class Watched(LastNorm):
+        def absorb(self, a, w, x):
+            super().absorb(a, w, x)
+            made.append(self.takes_split_sums and ops.gemm_split_sums(a, w) is not None)
+
+    def steps(norm):
+        monkeypatch.setattr(decoder, "LastNorm", norm)
+        manager = CacheManager(model.cache_requests(), 16, 2 * rows + 40, rows + 2)
+        runner = ModelRunner(model, manager, use_graphs=False)
+        out, ids = [], rc.random_ids(raw["vocab_size"], rows, seed=9)
+        decoding, prompt = [manager.new_request() for _ in range(rows)], manager.new_request()
+        assert all(manager.reserve(state, 0, 1) for state in decoding) and manager.reserve(prompt, 0, rows)
+        out.append(runner.step([Row([t], 0, state.tables, [0], state.state_slot) for t, state in zip(ids, decoding)]).double())
+        out.append(runner.step([Row(ids, 0, prompt.tables, [rows - 1, 2], prompt.state_slot)]).double())
+        return out
+
+    whole = steps(Whole)
+    for a, b in zip(steps(Watched), whole):
+        assert torch.equal(a, b) if dtype == "float32" else (a - b).norm() <= 2.0**-6 * b.norm()
+    assert made == [parts, parts]
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("num_requests", [3, 13, 21, 40, 100])
 def test_decode_graphs_replay_what_eager_steps_give(setup, dtype, num_requests):
