@@ -101,9 +101,10 @@ class DecodeGraphs:
     kernel is this package's; above, the matrix products are the library's, which replay
     correctly (checked against eager steps in the tests, several replays with eager work between).
 
-    The first context bucket of few rows comes in two forms: one for contexts of up to `SHORT_CONTEXT` tokens, whose
-    attention walks them whole, beside the one that cuts them into partitions which another kernel merges (one request
-    of 100 tokens at Qwen3-0.6B sizes: 936 us a step with the merge, 837 without; at 400 tokens both take as long).
+    The first context bucket of few rows comes in two forms where the model's attention cuts contexts of 1,024 tokens into
+    partitions, which another kernel merges, and walks contexts of `SHORT_CONTEXT` whole: one for those, one for the longer
+    ones (one request of 100 tokens at Qwen3-0.6B sizes: 936 us a step with the merge, 837 without; at 400 tokens both
+    take as long).  Each is captured when it is first needed, or ahead.
 
     A step is captured on rows that pad only (they store nothing and use the state slot that belongs
     to nobody), so capturing, and the runs that warm it up, touch no request's cache or state; the
@@ -118,7 +119,7 @@ class DecodeGraphs:
 
     ROW_BUCKETS = (1, 2, 4, 8, 16, 32, 48, 64, 96, 128, 192, 256)
     CONTEXT_STEP = 1024
-    SHORT_CONTEXT, SHORT_ROWS = 256, 32  # with more rows the requests themselves fill the GPU and no context is cut
+    SHORT_CONTEXT, SHORT_ROWS = 256, 32  # with more rows 8 kv heads' contexts fill the GPU and are not cut
     MAX_GRAPHS = 64
 
     def __init__(self, runner):
@@ -129,6 +130,7 @@ class DecodeGraphs:
         self.logits = None  # [most_rows, vocab] fp32, shared by all captured steps
         self.most_rows = _bucket(min(self.ROW_BUCKETS[-1], runner.manager.max_num_seqs), self.ROW_BUCKETS)
         self.bytes_held = 0
+        self.two_forms = {}  # rows -> whether the first context bucket is captured in two forms
 
     def filler(self) -> Row:
         """A row that pads a step: one token at position 0 that stores nothing; if the model keeps
@@ -153,7 +155,7 @@ class DecodeGraphs:
         n = _bucket(len(rows), self.ROW_BUCKETS)
         longest = max(row.start + 1 for row in rows)
         context = -(-longest // self.CONTEXT_STEP) * self.CONTEXT_STEP
-        bound = next(b for b in self._bounds(n, context) if longest <= b)
+        bound = next(b for b in self._forms(n, context) if longest <= b)
         width = -(-bound // bs)
         # every row of the captured step yields logits; rows that want none are dropped after the replay
         padded = [row if row.want else Row(row.tokens, row.start, row.tables, [0], row.state_slot) for row in rows]
@@ -163,13 +165,14 @@ class DecodeGraphs:
         if forms is None:
             while len(self.graphs) >= self.MAX_GRAPHS:
                 self.graphs.popitem(last=False)
-            forms = self.graphs[key] = {}
+            forms = {}
         else:
             self.graphs.move_to_end(key)
         entry = forms.get(bound)
         fresh = entry is None
         if fresh:
             entry = forms[bound] = self._capture(n, width, bound)
+            self.graphs[key] = forms
         if fresh or not entry[1].advance(padded):
             # other requests than last time, or a window moved: pack anew into the captured buffer
             batch = r.prepare(padded, table_width=width, max_context=bound, into=entry[1])
@@ -189,6 +192,15 @@ class DecodeGraphs:
     def _bounds(self, n: int, context: int) -> tuple:
         """The longest contexts of the forms in which the bucket (n rows, contexts up to `context`) is captured."""
         return (self.SHORT_CONTEXT, context) if context == self.CONTEXT_STEP and n <= self.SHORT_ROWS else (context,)
+
+    def _forms(self, n: int, context: int) -> tuple:
+        """Those of `_bounds` whose captures differ: without a cut at the longer one, or with one at both, one form serves all."""
+        bounds, r = self._bounds(n, context), self.runner
+        if len(bounds) == 1:
+            return bounds
+        if n not in self.two_forms:
+            self.two_forms[n] = [r.model.contexts_cut(n, bound, r.manager.block_size) for bound in bounds] == [False, True]
+        return bounds if self.two_forms[n] else bounds[-1:]
 
     def _capture(self, n: int, width: int, context: int):
         """Captures the decode step of `n` rows and contexts up to `context`, on padding rows."""
@@ -257,10 +269,11 @@ class DecodeGraphs:
         bs = self.runner.manager.block_size
         for context in contexts:
             for n in row_buckets:
-                forms = self.graphs.setdefault((n, context), {})
-                for bound in self._bounds(n, context):
+                forms = self.graphs.get((n, context), {})
+                for bound in self._forms(n, context):
                     if bound not in forms:
                         forms[bound] = self._capture(n, -(-bound // bs), bound)
+                        self.graphs[(n, context)] = forms
         return len(self.graphs) - before
 
 

@@ -264,11 +264,9 @@ def attn_single_query(q, k_pages, v_pages, items, positions, tok_row, block_tabl
                           f"(needs a multiple of {piece}, at most {SINGLE_QUERY_MAX_HEAD_DIM})")  # fmt: skip
     if max_context > block_tables.shape[1] * bs:
         raise KernelError("attention: block tables are shorter than the longest context")
-    G = H // KV
-    # a group of more query heads than the matrix-core kernel's workgroup takes is cut into equal smaller ones
-    share = next((G // g for g in range(min(G, 16), 0, -1) if G % g == 0 and _decode_mfma_fits(D, g)), 0)
-    mfma = q.dtype == BF16 and D % 32 == 0 and bs % 16 == 0 and share > 0 and not force_generic
-    if mfma and share > 1:
+    share = 0 if force_generic else _decode_mfma_share(q.dtype, H, KV, D, bs)
+    mfma = share > 0
+    if share > 1:
         part_size, P, part_m, part_l, part_acc = _partitions(N, H, KV * share, D, max_context, window or chunk, True, part_size, q.device, sight[1])
         call("as_attn_decode_mfma_shared", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(items), N, _ptr(positions),
              _ptr(tok_row), _ptr(block_tables), block_tables.shape[1], _ptr(out), _ptr(part_m), _ptr(part_l),
@@ -289,6 +287,23 @@ def attn_single_query(q, k_pages, v_pages, items, positions, tok_row, block_tabl
     call("as_attn_single_query", _ptr(q), _ptr(k_pages), _ptr(v_pages), _DT[q.dtype], _ptr(items), N,
          _ptr(positions), _ptr(tok_row), _ptr(block_tables), block_tables.shape[1], _ptr(out), _ptr(part_m),
          _ptr(part_l), _ptr(part_acc), H, KV, D, bs, float(scale), *sight, part_size, P, _stream())  # fmt: skip
+
+
+def _decode_mfma_share(dtype, H: int, KV: int, D: int, bs: int) -> int:
+    """Into how many equal groups the query heads of a kv head are cut for the bf16 matrix-core kernel of single queries (whose
+    workgroup holds a group of up to 16); 0 where another kernel runs."""
+    if dtype != BF16 or D % 32 or bs % 16:
+        return 0
+    G = H // KV
+    return next((G // g for g in range(min(G, 16), 0, -1) if G % g == 0 and _decode_mfma_fits(D, g)), 0)
+
+
+def contexts_cut(rows: int, H: int, KV: int, D: int, dtype, bs: int, context: int, window: int = 0, keep_first: int = 0) -> bool:
+    """Whether `attn_single_query` (and `attn_decode_fresh`) cuts contexts of up to `context` keys into partitions that another
+    kernel merges, for a decode step of `rows` rows."""
+    share = _decode_mfma_share(dtype, H, KV, D, bs)
+    matrix = share > 0 or attn_f32_supported(dtype, H, KV, D, bs, keep_first)
+    return _partitions(rows, H, KV * max(1, share), D, context, window, matrix, None, "meta", keep_first)[1] > 1
 
 
 def attn_f32_supported(dtype, num_heads: int, num_kv_heads: int, head_dim: int, block_size: int, keep_first: int = 0) -> bool:

@@ -136,6 +136,11 @@ class DecoderModel:
         return tuple(sorted({split for block in self.blocks for split in [block.parts()["mixer"].row_split()]
                              if split is not None}))  # fmt: skip
 
+    def contexts_cut(self, rows: int, context: int, block_size: int) -> bool:
+        """Whether a decode step of `rows` rows and contexts of up to `context` tokens cuts some layer's contexts into partitions."""
+        return any(ops.contexts_cut(rows, H, KV, D, self.env.dtype, block_size, context, window, keep)
+                   for H, KV, D, window, keep in {q for block in self.blocks for q in block.parts()["mixer"].single_queries()})  # fmt: skip
+
     def forward(self, step, logits: torch.Tensor = None) -> torch.Tensor:
         """Run this step's tokens through every run of the plan; returns fp32 logits
         [len(step.logits_rows), vocab] for the wanted rows (written into `logits` if given)."""

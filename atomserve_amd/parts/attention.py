@@ -86,6 +86,10 @@ class Attention(Mixer):
     def row_split(self):
         return (SHORT_ROW, TILE_Q)
 
+    def single_queries(self):
+        s = self.spec
+        return ((s.num_heads, s.num_kv_heads, s.head_dim, s.window, 0),)
+
     def forward(self, h, step, cache, residual=None, next_norm=None):
         """h [T, hidden] compute dtype (or the norm left pending on the stream) -> [T, hidden], or the
         pending `next_norm` after adding the output into `residual`.  cache: a PagedLayerView (pages

@@ -208,6 +208,11 @@ class Mixer(Part):
         they come (`step.row_first`, `step.row_len`)."""
         return None
 
+    def single_queries(self) -> tuple:
+        """(query heads, kv heads, head width, window, kept first keys) of every attention over pages that a decode step runs as
+        `ops.attn_single_query` or `ops.attn_decode_fresh`."""
+        return ()
+
     def forward(self, h: torch.Tensor, step: Any, cache: Any) -> torch.Tensor:
         raise NotImplementedError
 

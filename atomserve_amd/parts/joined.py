@@ -370,6 +370,11 @@ class JoinedMixer(Mixer):
     def row_split(self):
         return (SHORT_ROW, TILE_Q) if any(isinstance(core, SoftmaxCore) and not core.wide for core in self.cores) else None
 
+    def single_queries(self):
+        return tuple((c.spec.num_heads * c.spec.maps, c.spec.num_kv_heads, c.head_width, c.spec.window or c.spec.chunk,
+                      c.spec.keep_first if c.spec.window > 0 else 0)
+                     for c in self.cores if isinstance(c, SoftmaxCore) and not c.wide)  # fmt: skip
+
     def forward(self, h, step, cache):
         s, env = self.spec, self.env
         T, dev = h.shape[0], h.device

@@ -115,6 +115,10 @@ class LatentAttention(Mixer):
     def row_split(self):
         return None if self.wide else (SHORT_ROW, TILE_Q)
 
+    def single_queries(self):
+        s = self.spec
+        return () if self.wide else ((s.num_heads, 1, self.width, s.window, s.keep_first if s.window > 0 else 0),)
+
     def forward(self, h, step, cache):
         s, env = self.spec, self.env
         T, dev = h.shape[0], h.device

@@ -190,6 +190,10 @@ class SideBySide(Mixer):
     def row_split(self):
         return (SHORT_ROW, TILE_Q)
 
+    def single_queries(self):
+        a = self.spec.left
+        return ((a.num_heads, a.num_kv_heads, self.head_width, a.window, 0),)
+
     def forward(self, h, step, cache):
         s, a, r, env = self.spec, self.spec.left, self.spec.right, self.env
         T, dev = h.shape[0], h.device

@@ -81,6 +81,34 @@ def test_short_contexts_are_walked_whole():
     assert bounds(1, 1024) == bounds(32, 1024) == (256, 1024) and bounds(48, 1024) == (1024,) and bounds(1, 2048) == (2048,)
 
 
+def test_forms_of_a_captured_bucket():
+    """A bucket is captured in two forms only where the attention of some layer cuts its longer contexts and not the short ones."""
+    from types import SimpleNamespace
+
+    from atomserve_amd.engine.runner import DecodeGraphs
+    from atomserve_amd.models.decoder import DecoderModel
+    from atomserve_amd.parts.attention import Attention
+    from atomserve_amd.parts.base import Mixer
+
+    def graphs(*heads, dtype=BF16):
+        mixer = SimpleNamespace(single_queries=lambda: heads)
+        model = SimpleNamespace(env=SimpleNamespace(dtype=dtype), blocks=[SimpleNamespace(parts=lambda: {"mixer": mixer})])
+        model.contexts_cut = lambda *how: DecoderModel.contexts_cut(model, *how)
+        made = DecodeGraphs.__new__(DecodeGraphs)
+        made.runner, made.two_forms = SimpleNamespace(model=model, manager=SimpleNamespace(block_size=16)), {}
+        return made
+
+    two, one = (256, 1024), (1024,)
+    g = graphs((16, 8, 128, 0, 0))
+    assert [g._forms(n, 1024) for n in (1, 32, 48)] == [two, two, one] and g._forms(1, 2048) == (2048,) and g.two_forms == {1: True, 32: True}
+    assert graphs()._forms(1, 1024) == one  # no paged attention of this kind
+    assert [graphs((32, 16, 128, 0, 0))._forms(n, 1024) for n in (16, 32)] == [two, one]  # 32 x 16 workgroups fill the GPU
+    assert graphs((16, 8, 128, 200, 0))._forms(1, 1024) == one  # a window that both contexts fill
+    assert graphs((16, 8, 128, 0, 0), (16, 8, 128, 200, 0), dtype=F32)._forms(4, 1024) == two
+    spec = SimpleNamespace(num_heads=16, num_kv_heads=8, head_dim=128, window=64)
+    assert Attention.single_queries(SimpleNamespace(spec=spec)) == ((16, 8, 128, 64, 0),) and Mixer.single_queries(None) == ()
+
+
 def test_how_products_of_17_to_128_rows_are_tiled():
     """Tiles of 64 weight rows, K cut into as many ranges of whole chunks as fill the compute units; the gated
     product's tile width by what the longest path loads."""

@@ -186,6 +186,33 @@ def test_decoding_across_the_context_bound_of_a_captured_graph(dtype, tmp_path):
     assert len(replay.runner.decode_graphs.graphs) == 2
 
 
+@pytest.mark.parametrize("head_dim", [16, 64])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_the_two_forms_of_a_captured_bucket(dtype, head_dim, tmp_path):
+    """Decode steps of contexts up to 256 tokens and of longer ones in the same bucket: a request that passes the bound, requests on
+    either side of it one after the other and together, so that either form finds rows that the other has moved on."""
+    raw = dict(TINY["A"], max_position_embeddings=2048, head_dim=head_dim)
+    weights = plain_random_weights(raw, seed=59, std=0.2, gain_std=0.2)
+    path = write_model_dir(str(tmp_path / "forms"), raw, weights, torch.bfloat16)
+    heads = {"a": 246, "b": 300, "c": 20}
+    requests = {rid: rc.random_ids(raw["vocab_size"], n + 40, seed=60 + n) for rid, n in heads.items()}
+    at, steps = dict(heads), []
+    for rid, n in heads.items():
+        steps.append({"step": len(steps), "entries": [{"id": rid, "tokens": requests[rid][:n], "want": [n - 1]}], "end": []})
+    for together in ["a", "b"] * 7 + ["ab", "ac", "ab", "cb", "ac", "c", "a", "ca", "ca", "bc", "c", "c", "b", "c"]:
+        entries = []
+        for rid in together:
+            entries.append({"id": rid, "tokens": [requests[rid][at[rid]]], "want": [0]})
+            at[rid] += 1
+        steps.append({"step": len(steps), "entries": entries, "end": []})
+    steps[-1]["end"] = list(heads)
+    requests = {rid: ids[: at[rid]] for rid, ids in requests.items()}
+    replay = make_replay(path, dtype, rc.live_token_bound(steps) + 64)
+    assert compare(replay, steps, requests, raw, weights, {}, dtype).rows == 3 + sum(len(s["entries"]) for s in steps[3:])
+    graphs = replay.runner.decode_graphs.graphs
+    assert {key: sorted(forms) for key, forms in graphs.items()} == {(1, 1024): [256, 1024], (2, 1024): [256, 1024]}
+
+
 @pytest.mark.parametrize("hidden, dtype, rows, parts", [(2048, "bfloat16", 40, True), (2048, "bfloat16", 128, True), (2048, "bfloat16", 9, False),
                                                         (1024, "bfloat16", 40, False), (2048, "float32", 20, True), (1024, "float32", 200, True),
                                                         (2048, "float32", 5, False)])  # fmt: skip
