@@ -27,17 +27,26 @@ __device__ __forceinline__ void store4(float* p, floatx4 v, int valid) {
   for (int i = 0; i < valid; ++i) p[i] = v[i];
 }
 
-// Columns k .. k+3 of a row, those from K on as zeros.  VEC: rows start on 16 bytes and K % 4 == 0.
+// Columns k .. k+3 of a row, those from K on as zeros.  VEC: rows start on 16 bytes and K % 4 == 0.  Else the load, which needs no
+// more than a float's alignment, ends where the row ends, and `ragged` moves what belongs elsewhere when the columns are used: a
+// test here would make every load wait for the one before.
+typedef float floatx4_anywhere __attribute__((ext_vector_type(4), aligned(4)));
+
 template <bool VEC> __device__ __forceinline__ floatx4 fetch(const float* row, int k, int K) {
   if constexpr (VEC) {
     const floatx4 v = *reinterpret_cast<const floatx4*>(row + (k < K ? k : 0));
     return k < K ? v : floatx4{0.f, 0.f, 0.f, 0.f};
   } else {
-    floatx4 v;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = k + i < K ? row[k + i] : 0.f;
-    return v;
+    return *reinterpret_cast<const floatx4_anywhere*>(row + min(k, K - 4));  // K > F32_NARROW
   }
+}
+
+template <bool VEC> __device__ __forceinline__ floatx4 ragged(floatx4 v, int k, int K) {  // v: what `fetch` gave for k
+  if constexpr (VEC) return v;
+  const int by = k - min(k, K - 4);
+  if (by & 1) v = floatx4{v[1], v[2], v[3], 0.f};
+  if (by & 2) v = floatx4{v[2], v[3], 0.f, 0.f};
+  return by >= 4 ? floatx4{0.f, 0.f, 0.f, 0.f} : v;
 }
 
 // `v`, where it is not finite, again by the fp32 instruction over the steps st0 .. st1 - 1: 16 rows of w (this lane's `wrow`)
@@ -49,7 +58,7 @@ template <bool VEC> __device__ __forceinline__ floatx4 again_f32(floatx4 v, cons
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int k = st * 32 + lg * 8 + half * 4;
-      const floatx4 wv = fetch<VEC>(wrow, k, K), av = fetch<VEC>(arow, k, K);
+      const floatx4 wv = ragged<VEC>(fetch<VEC>(wrow, k, K), k, K), av = ragged<VEC>(fetch<VEC>(arow, k, K), k, K);
 #pragma unroll
       for (int x = 0; x < 4; ++x) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[x], av[x], acc, 0, 0, 0);
     }
@@ -177,6 +186,18 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
     for (int u = 0; u < DEPTH; ++u) {
       if (st + u < st1) {
         Parts as[MT], ws[NT];
+        if (!VEC && st + u + SHARE >= steps) {  // K may end among these steps' columns
+          const int k = (st + u) * 32 + lg * 8, ka = SHARE == 1 ? k : min(st + u + lr / ROWS, steps - 1) * 32 + lg * 8;
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) wv[u][i][half] = ragged<VEC>(wv[u][i][half], k + 4 * half, K);
+            if (u % SHARE == 0) {
+#pragma unroll
+              for (int j = 0; j < MT; ++j) av[u / SHARE][j][half] = ragged<VEC>(av[u / SHARE][j][half], ka + 4 * half, K);
+            }
+          }
+        }
         if (u % SHARE == 0) {
 #pragma unroll
           for (int j = 0; j < MT; ++j) shared[j] = parts(av[u / SHARE][j][0], av[u / SHARE][j][1]);
@@ -281,6 +302,7 @@ __global__ __launch_bounds__(16 / SIDE * 64) void gemm_f32_side_kernel(const flo
   const int n0 = blockIdx.x * R;
   const int steps = (K + 31) / 32, per = (steps + F32_SLICES - 1) / F32_SLICES;
   const int first = (wave * SIDE + lr / R) * per;  // this lane's slice
+  const bool cut = (wave * SIDE + SIDE) * per * 32 > K;  // K ends in the wave's slices
   const float* wrow = w + (size_t)min(n0 + lr % R, N - 1) * K;
   const float* arow = a + (size_t)min(lr % R, M - 1) * K;
   floatx4 wv[DEPTH][2], av[DEPTH][2], acc = {0.f, 0.f, 0.f, 0.f}, low = acc;
@@ -306,6 +328,14 @@ __global__ __launch_bounds__(16 / SIDE * 64) void gemm_f32_side_kernel(const flo
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) {
       if (st + u < per) {
+        if (!VEC && cut) {
+          const int k = (first + st + u) * 32 + lg * 8;
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            wv[u][half] = ragged<VEC>(wv[u][half], k + 4 * half, K);
+            av[u][half] = ragged<VEC>(av[u][half], k + 4 * half, K);
+          }
+        }
         const Parts ws = parts(wv[u][0], wv[u][1]), as = parts(av[u][0], av[u][1]);
         if (st + u + DEPTH < per) load(u, st + u + DEPTH);
 #pragma unroll
@@ -360,8 +390,7 @@ __global__ __launch_bounds__(16 / SIDE * 64) void gemm_f32_side_kernel(const flo
 // same above 32, which so touch every bank once.
 // GATED: half of a tile's rows of w are gate rows, half the up rows of the same outputs.
 // SPLIT: blockIdx.y names a group of four slices, whose sums go to out[group][m][n] for whoever adds the groups up in order.
-// VEC only: rows start on 16 bytes and K % 4 == 0.
-template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT>
+template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT, bool VEC>
 __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
                                                              float* __restrict__ out, int M, int N, int K, int tiles_m, int tiles,
                                                              int per_xcd) {
@@ -400,12 +429,15 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __re
 #pragma unroll
       for (int p = 0; p < PIECES; ++p)
 #pragma unroll
-        for (int half = 0; half < 2; ++half) ahead[u][p][half] = *reinterpret_cast<const floatx4*>(src[p] + k + 4 * half);
+        for (int half = 0; half < 2; ++half) {
+          if constexpr (VEC) ahead[u][p][half] = *reinterpret_cast<const floatx4*>(src[p] + k + 4 * half);
+          else ahead[u][p][half] = *reinterpret_cast<const floatx4_anywhere*>(src[p] + k + 4 * half);
+        }
     } else {
 #pragma unroll
       for (int p = 0; p < PIECES; ++p)
 #pragma unroll
-        for (int half = 0; half < 2; ++half) ahead[u][p][half] = fetch<true>(src[p], k + 4 * half, K);
+        for (int half = 0; half < 2; ++half) ahead[u][p][half] = ragged<VEC>(fetch<VEC>(src[p], k + 4 * half, K), k + 4 * half, K);
     }
   };
   auto place = [&](int u, int buf) {
@@ -483,7 +515,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __re
       v[i] = total[i][j] + (group[i][j] + (acc[i][j] + low[i][j]));
       const int r = (wn * NTW + i) * 16;
       const bool mine = m < M && (IS_GATED ? n0 + wn * 16 : n0 + r) + lg * 4 < N;
-      if (__any(mine && !finite(v[i]))) v[i] = again_f32<true>(v[i], weight(r + lr), a + (size_t)min(m, M - 1) * K, K, st0, st1);
+      if (__any(mine && !finite(v[i]))) v[i] = again_f32<VEC>(v[i], weight(r + lr), a + (size_t)min(m, M - 1) * K, K, st0, st1);
     }
     if constexpr (IS_GATED) {
       const int n = n0 + wn * 16 + lg * 4;
@@ -571,7 +603,7 @@ static int launch_rows(const float* a, const float* w, float* out, int M, int N,
     gemm_f32_rows_kernel<MT, NT, WAVES, DEPTH, SHARE, true, MODE><<<per_xcd * 8, WAVES * 64, lds, stream>>>(a, w, out, M, N, K, tiles_m,
                                                                                                          (int)tiles, per_xcd, link);
   else
-    gemm_f32_rows_kernel<MT, NT, WAVES, SHARE, SHARE, false, MODE><<<per_xcd * 8, WAVES * 64, lds, stream>>>(a, w, out, M, N, K, tiles_m,
+    gemm_f32_rows_kernel<MT, NT, WAVES, DEPTH, SHARE, false, MODE><<<per_xcd * 8, WAVES * 64, lds, stream>>>(a, w, out, M, N, K, tiles_m,
                                                                                                          (int)tiles, per_xcd, link);
   return launch_status();
 }
@@ -584,13 +616,27 @@ static int launch_few(const float* a, const float* w, float* out, int M, int N, 
   return launch_rows<1, NT, WAVES, DEPTH, 1, MODE>(a, w, out, M, N, K, link, stream);
 }
 
+// Strips of 16 rows of w, one to a workgroup.  A long K goes to sixteen waves while a wave's steps are mostly its loads (N, K at 1, 4, 8
+// and 16 rows, eight waves and sixteen, us: 3,072, 8,192 33 27, 33 30, 35 34, 39 43; 4,096, 12,288 50 46, 48 47, 52 52, 57 64; 4,096, 4,096 18 19).
+template <int MODE> static int launch_strips(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
+  if (M <= 8 && K >= 8192 && f32_tiles(M, N, 16, 16) <= compute_units()) return launch_few<1, 16, 4, MODE>(a, w, out, M, N, K, link, stream);
+  return launch_few<1, 8, 4, MODE>(a, w, out, M, N, K, link, stream);
+}
+
+// Two strips a workgroup: on eight waves while that is one round (8,192, 4,096 at 1 / 16 rows 30 / 31 us, on four 39 / 36; 6,144, 1,024 9.7 / 11.5
+// and 10.7 / 11.6), else on four, of which more fit a compute unit (12,288, 2,048 25 / 29, on eight 28 / 33).
+template <int MODE> static int launch_pairs(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
+  if (f32_tiles(M, N, 16, MODE == GATED ? 16 : 32) <= compute_units()) return launch_rows<1, 2, 8, 2, 1, MODE>(a, w, out, M, N, K, link, stream);
+  return launch_rows<1, 2, 4, 2, 1, MODE>(a, w, out, M, N, K, link, stream);
+}
+
 template <int MODE> static int launch_side(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
   const bool vec = (K & 3) == 0 && aligned16(a, w);
 #define SIDE_GO(SIDE)                                                                                                            \
   do {                                                                                                                           \
     const int blocks = (N + 16 / SIDE - 1) / (16 / SIDE);                                                                        \
     if (vec) gemm_f32_side_kernel<SIDE, 6, true, MODE><<<blocks, 16 / SIDE * 64, 0, stream>>>(a, w, out, M, N, K, link);         \
-    else gemm_f32_side_kernel<SIDE, 2, false, MODE><<<blocks, 16 / SIDE * 64, 0, stream>>>(a, w, out, M, N, K, link);            \
+    else gemm_f32_side_kernel<SIDE, 6, false, MODE><<<blocks, 16 / SIDE * 64, 0, stream>>>(a, w, out, M, N, K, link);            \
   } while (0)
   if (M <= 4) SIDE_GO(4);
   else SIDE_GO(2);
@@ -606,19 +652,24 @@ template <int MODE> static int launch_side(const float* a, const float* w, float
 // 1,024, 3,072   12.0  6.6    13.0  7.4    14.4 10.0         3,072, 1,024    6.9  8.8     7.4 11.6     8.3 16.0
 static bool side_by_side(int M, int N, int K) { return N <= 8 * compute_units() && (M <= 4 || (M <= 8 && K >= 2048)); }
 
-template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT>
-static int launch_tile(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT, bool VEC>
+static int launch_tile_of(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
   constexpr int TM = 16 * WM * MTW, TN = 16 * WN * NTW;
   constexpr int lds = 2 * 3 * (TM + TN) * 64;
-  if ((K & 3) != 0 || !aligned16(a, w)) return AS_BAD_SHAPE;
   const long tiles = f32_tiles(M, N, TM, IS_GATED ? TN / 2 : TN);
   if (tiles > 0x3fffffff) return AS_BAD_SHAPE;
-  const auto kernel = gemm_f32_tile_kernel<WM, WN, MTW, NTW, IS_GATED, SPLIT>;
+  const auto kernel = gemm_f32_tile_kernel<WM, WN, MTW, NTW, IS_GATED, SPLIT, VEC>;
   if (lds > 65536 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
     return AS_LAUNCH_FAILED;
   const int per_xcd = (int)((tiles + 7) / 8), tiles_m = (M + TM - 1) / TM;
   kernel<<<dim3(per_xcd * 8, SPLIT ? F32_GROUPS : 1), 512, lds, stream>>>(a, w, out, M, N, K, tiles_m, (int)tiles, per_xcd);
   return launch_status();
+}
+
+template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT>
+static int launch_tile(const float* a, const float* w, float* out, int M, int N, int K, hipStream_t stream) {
+  if ((K & 3) == 0 && aligned16(a, w)) return launch_tile_of<WM, WN, MTW, NTW, IS_GATED, SPLIT, true>(a, w, out, M, N, K, stream);
+  return launch_tile_of<WM, WN, MTW, NTW, IS_GATED, SPLIT, false>(a, w, out, M, N, K, stream);
 }
 
 // Which kernel: the tile of rows of a by rows of w, and what a workgroup on every compute unit takes per 1,024 of K
@@ -630,7 +681,6 @@ struct F32Tile { int rows, columns; float alone_us, round_us; };
 static const F32Tile f32_forms[] = {{16, 16, 3.4f, 4.5f},   {16, 16, 4.5f, 3.6f},   {16, 32, 6.2f, 5.6f},    {32, 16, 5.5f, 7.4f},
                                     {32, 32, 7.8f, 9.f},    {64, 32, 12.f, 13.f},   {64, 64, 18.f, 14.5f},   {128, 128, 48.f, 48.f}};
 #define F32_FORMS 8
-#define F32_TILE_FORMS 6    // the first through LDS
 #define F32_ONE_ROW_TILE 3  // so many of one row tile
 
 static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
@@ -642,23 +692,20 @@ static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
 // form: 0: chosen here; else 1 + the index of a kernel, or after them the one of slices side by side (tests).
 template <int MODE> static int gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, const LinkF32& link,
                                         hipStream_t stream) {
-  const bool vec = (K & 3) == 0 && aligned16(a, w);
   if constexpr (MODE == PLAIN) {
     if (form == F32_FORMS + 1 ? M <= 8 : form == 0 && side_by_side(M, N, K)) return launch_side<PLAIN>(a, w, out, M, N, K, link, stream);
   }
   if (form == 0) {
     float best = 0.f;
     for (int i = MODE == GATED ? 2 : 0; i < (link.ssq_in ? F32_ONE_ROW_TILE : F32_FORMS); ++i) {
-      if ((MODE == GATED && i == 3) || (i >= F32_TILE_FORMS && !vec)) continue;
+      if (MODE == GATED && i == 3) continue;
       const float cost = f32_cost(f32_forms[i], M, MODE == GATED ? 2 * N : N, K, 1);
       if (form == 0 || cost < best) { best = cost; form = i + 1; }
     }
   }
   if constexpr (MODE == GATED) {
     switch (form) {
-      case 3:
-        if (f32_tiles(M, N, 16, 16) <= compute_units()) return launch_rows<1, 2, 8, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
-        return launch_rows<1, 2, 4, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
+      case 3: return launch_pairs<GATED>(a, w, out, M, N, K, link, stream);
       case 5: return launch_rows<2, 2, 4, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
       case 6: return launch_rows<4, 2, 4, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
       case 7: return launch_tile<4, 2, 1, 2, true, false>(a, w, out, M, N, K, stream);
@@ -667,12 +714,12 @@ template <int MODE> static int gemm_f32(const float* a, const float* w, float* o
   } else {
     switch (form) {
       case 1:
-        if (M <= 16) return launch_few<1, 8, 4, PLAIN>(a, w, out, M, N, K, link, stream);
+        if (M <= 16) return launch_strips<PLAIN>(a, w, out, M, N, K, link, stream);
         return launch_rows<1, 1, 8, 4, 1, PLAIN>(a, w, out, M, N, K, link, stream);
       case 2:
         if (M <= 16) return launch_few<1, 4, 4, PLAIN>(a, w, out, M, N, K, link, stream);
         return launch_rows<1, 1, 4, 4, 1, PLAIN>(a, w, out, M, N, K, link, stream);
-      case 3: return launch_rows<1, 2, 4, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
+      case 3: return launch_pairs<PLAIN>(a, w, out, M, N, K, link, stream);
       case 4: return launch_rows<2, 1, 8, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
       case 5: return launch_rows<2, 2, 4, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
       case 6: return launch_rows<4, 2, 4, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
@@ -711,7 +758,7 @@ extern "C" int as_gemm_f32_link(const float* a, const float* w, float* x, const 
   if (M > 16 || N <= 0 || (N & 3) || K <= F32_NARROW || !gain || !scaled || !ssq || !aligned16(x, scaled)) return AS_BAD_SHAPE;
   const LinkF32 link{nullptr, 0, 0.f, gain, scaled, ssq};
   if (side_by_side(M, N, K)) return launch_side<LINK>(a, w, x, M, N, K, link, stream);
-  return launch_few<1, 8, 4, LINK>(a, w, x, M, N, K, link, stream);
+  return launch_strips<LINK>(a, w, x, M, N, K, link, stream);
 }
 
 // The consumer of a LinkF32: out[M, N] = (scaled @ w^T) / rms(x) with rms from ssq[M, strips_in] (strips_in = K / 4) and eps;
@@ -726,19 +773,10 @@ extern "C" int as_gemm_f32_scaled(const float* scaled, const float* ssq, int str
 
 // sums[4][M, N]: the product's sums over the four quarters of K's slices; added up in order they are the product, bit for bit.  For
 // products of too few outputs to fill the GPU: N = 1,024, K = 2,048 at 333 rows 17.7 us, whole 28.5.  K > F32_NARROW, K % 4 == 0,
-// N % 4 == 0.  Rows that do not start on 16 bytes: the product is made whole, three of the sums are zeros.
-__global__ __launch_bounds__(256) void zeros_kernel(float* __restrict__ out, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) out[i] = 0.f;
-}
-
+// N % 4 == 0.
 extern "C" int as_gemm_f32_split(const float* a, const float* w, float* sums, int M, int N, int K, int form, hipStream_t stream) {
   if (M <= 0) return AS_OK;
   if (N <= 0 || (N & 3) || K <= F32_NARROW || (K & 3) || form < 0 || form > 2) return AS_BAD_SHAPE;
-  if (!aligned16(a, w)) {
-    zeros_kernel<<<compute_units() * 4, 256, 0, stream>>>(sums + (size_t)M * N, (size_t)(F32_GROUPS - 1) * M * N);
-    const int rc = launch_status();
-    return rc != AS_OK ? rc : gemm_f32<PLAIN>(a, w, sums, M, N, K, 0, LinkF32{}, stream);
-  }
   if (form == 0) form = f32_cost(f32_forms[6], M, N, K, F32_GROUPS) <= f32_cost(f32_forms[7], M, N, K, F32_GROUPS) ? 1 : 2;
   if (form == 1) return launch_tile<4, 2, 1, 2, false, true>(a, w, sums, M, N, K, stream);
   return launch_tile<2, 4, 4, 2, false, true>(a, w, sums, M, N, K, stream);

@@ -1481,6 +1481,51 @@ def test_gemm_f32_slices_side_by_side(ops, M, N, K, shift):
             assert bool(((got.double() - ref).abs() <= size * (K / 512 + 16) * 2.0**-24).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 40, 257), (3, 2050, 515), (4, 37, 1030), (7, 64, 287), (8, 2100, 1026), (12, 70, 2049), (16, 33, 319), (40, 90, 515),
+                                   (70, 130, 257), (131, 140, 1025), (130, 70, 290)])  # fmt: skip
+@pytest.mark.parametrize("shift", [0, 1])
+def test_gemm_f32_rows_that_start_anywhere(ops, M, N, K, shift):
+    """Widths that are no multiple of 4 and matrices that do not start on 16 bytes, whose last columns are loaded from where the row ends: every
+    kernel has the bits of the product of the rows with zeros up to whole steps of 32 behind them, numbers that are not finite included."""
+    torch.manual_seed(K)
+    a, w = (torch.randn(rows * K + shift, device=DEV)[shift:].view(rows, K) for rows in (M, N))
+    pad = -K % 32
+    blank = lambda *shape: torch.full(shape, float("nan"), device=DEV)  # noqa: E731
+    for spoil in (False, True):
+        if spoil:
+            a[0, K - 1], w[N - 1, K - 2], w[N // 2, 0] = float("inf"), float("nan"), float("-inf")
+        wide = [torch.cat([t, torch.zeros(t.shape[0], pad, device=DEV)], 1).contiguous() for t in (a, w)]
+        want = f32_product("as_gemm_f32", *wide, blank(M, N), 1)
+        if spoil:  # an infinity times the zeros behind a row is none of the row's own products
+            want = torch.where(torch.isfinite(want), want, f32_product("as_gemm_f32", a, w, blank(M, N), 1))
+        same = lambda x, y: torch.equal(x.nan_to_num(3.0), y.nan_to_num(3.0)) and torch.equal(x.isnan(), y.isnan())  # noqa: E731
+        for form in (0, 1, 2, 3, 4, 5, 6, 7, 8) + ((9,) if M <= 8 else ()):
+            assert same(f32_product("as_gemm_f32", a, w, blank(M, N), form), want)
+        if N % 2 == 0:
+            act = blank(M, N // 2)
+            ops.silu_mul(want, act)
+            for form in (0, 3, 5, 6, 7, 8):
+                assert same(f32_product("as_gemm_f32_gated", a, w, blank(M, N // 2), form), act)
+        if not spoil:
+            ref, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+            assert bool(((want.double() - ref).abs() <= size * (6 * (K / 512 + 1) + 22) * 2.0**-24).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 260, 8192), (4, 2308, 8196), (8, 272, 9728), (9, 264, 8192), (5, 4096, 1024), (12, 8192, 512), (16, 8240, 300)])
+def test_gemm_f32_waves_of_a_strip(ops, M, N, K):
+    """Long widths on sixteen waves, and two strips a workgroup on eight waves and on four: the bits of the tiles through LDS.  (More than
+    256 outputs, which a link takes.)"""
+    torch.manual_seed(N)
+    a, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV) * 0.05
+    want = f32_product("as_gemm_f32", a, w, torch.empty(M, N, device=DEV), 7)
+    for form in (0, 1, 3):
+        assert torch.equal(f32_product("as_gemm_f32", a, w, torch.full((M, N), float("nan"), device=DEV), form), want)
+    x, gain = torch.randn(M, N, device=DEV), torch.rand(N, device=DEV)
+    summed, scaled, ssq = x + want, torch.empty(M, N, device=DEV), torch.empty(M, ops.link_strips(N, F32), device=DEV)
+    ops.gemm_link(a, w, x, gain, scaled, ssq)
+    assert torch.equal(x, summed) and torch.equal(scaled, x * gain)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 260, 1024), (4, 1024, 2048), (5, 272, 300), (8, 1024, 3072), (9, 516, 288), (16, 2048, 6144)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_gemm_link_and_scaled_f32(ops, M, N, K, shift):
