@@ -7,8 +7,9 @@
 // off downwards, and that error has one sign.  Against 64 bits (K = 1,024 / 2,048 / 3,072, normal values) the error is 0.76e-7 /
 // 0.87e-7 / 0.98e-7 of the result (in one chain 1.15e-7 / 1.7e-7 / 2.1e-7), with the cores' fp32 instruction in the same order
 // 1.55e-7 / 2.1e-7 / 2.6e-7; heavy tails, outliers and one sign alike: at most 0.9 of that instruction's error.
-// Numbers below 2^-110 keep an absolute error of 2^-134 instead.  Values that are not finite (or that round to infinity in bf16)
-// would become NaN in the parts: a result that is not finite is computed again with the fp32 instruction.
+// Beside those distributions: numbers below 2^-110 keep an absolute error of 2^-134 instead, and a sum of one product that is not zero
+// is not rounded correctly, as the fp32 instruction would (the error is below 2^-23 of it).  Values that are not finite (or that round to
+// infinity in bf16) would become NaN in the parts: a result that is not finite is computed again with the fp32 instruction.
 //
 // The order of every output's sum depends on K alone, so a row's result does not depend on which other rows share the launch,
 // nor on the kernel or the tile that the launch chose: K is cut into 16 slices of whole steps of 32 columns, each slice is one
@@ -771,7 +772,9 @@ extern "C" int as_gemm_f32_scaled(const float* scaled, const float* ssq, int str
   return gated ? gemm_f32<GATED>(scaled, w, out, M, N, K, 0, link, stream) : gemm_f32<PLAIN>(scaled, w, out, M, N, K, 0, link, stream);
 }
 
-// sums[4][M, N]: the product's sums over the four quarters of K's slices; added up in order they are the product, bit for bit.  For
+// sums[4][M, N]: the product's sums over the four quarters of K's slices; added up in order they are the product, bit for bit where
+// every sum is finite.  (Of an output with a sum that is not, the product made whole computes all of K again with the fp32 instruction and
+// this one that quarter: an operand between bf16's largest number, 3.39e38, and fp32's makes them differ by rounding.)  For
 // products of too few outputs to fill the GPU: N = 1,024, K = 2,048 at 333 rows 17.7 us, whole 28.5.  K > F32_NARROW, K % 4 == 0,
 // N % 4 == 0.
 extern "C" int as_gemm_f32_split(const float* a, const float* w, float* sums, int M, int N, int K, int form, hipStream_t stream) {

@@ -673,7 +673,8 @@ def few_rows_product(a, w) -> bool:
 
 
 def gemm(a, w, out, choices=None) -> None:
-    """out[M, N] = a[M, K] @ w[N, K]^T.  fp32: own kernel (true fp32).  bf16: own kernel for few
+    """out[M, N] = a[M, K] @ w[N, K]^T.  fp32: own kernel (32-bit operands and sums; above 256 columns every float as three bf16
+    parts, six products of parts for one, with an error no larger than the fp32 instruction's).  bf16: own kernel for few
     rows, the library's matrix product otherwise; `out` may be bf16 or (few rows) fp32.
     w: a tensor, or a `Streamed`.  choices: the `ProductChoices` that says which of the library's kernels
     runs (a model's own; None: the one the process shares)."""
@@ -1067,7 +1068,8 @@ def gemm_f32_split_preferred(rows: int, n: int, k: int) -> bool:
 
 
 def gemm_f32_split(a, w):
-    """The partial sums [4, M, N] of the 32-bit a[M, K] @ w[N, K]^T: added up in order they are `gemm`'s result."""
+    """The partial sums [4, M, N] of the 32-bit a[M, K] @ w[N, K]^T: added up in order they are `gemm`'s result (bit for bit while no
+    operand exceeds bfloat16's largest number, 3.39e38; such outputs agree within rounding)."""
     _check(a, "a", F32, (None, None))
     M, K = a.shape
     rows = _rows(w)

@@ -1481,6 +1481,26 @@ def test_gemm_f32_slices_side_by_side(ops, M, N, K, shift):
             assert bool(((got.double() - ref).abs() <= size * (K / 512 + 16) * 2.0**-24).all())
 
 
+def test_gemm_f32_split_of_numbers_beyond_bf16(ops):
+    """Operands that are finite and round to infinity in bf16: a quarter that holds one is computed again with the fp32 instruction, in the
+    product made whole all of K.  Bound: a chain of K multiply-adds or the sums of a slice, each rounding 2^-24 of the sums of absolute values."""
+    torch.manual_seed(65)
+    M, N, K = 70, 64, 1024
+    a, w = torch.randn(M, K, device=DEV), torch.randn(N, K, device=DEV)
+    a[3, 700], w[:, 700] = 3.4e38, torch.rand(N, device=DEV) * 1e-38  # their product is of the size of the others
+    a[5, 9], w[7, 9] = float("inf"), 1.0
+    whole = f32_product("as_gemm_f32", a, w, torch.empty(M, N, device=DEV), 0)
+    s = f32_product("as_gemm_f32_split", a, w, torch.empty(4, M, N, device=DEV), 0)
+    parts = ((s[0] + s[1]) + s[2]) + s[3]
+    kind = lambda t: (torch.isnan(t), torch.isposinf(t), torch.isneginf(t))  # noqa: E731
+    assert all(torch.equal(x, y) for x, y in zip(kind(whole), kind(parts))) and bool(torch.isfinite(whole[3]).all())
+    others = [m for m in range(M) if m not in (3, 5)]
+    assert torch.equal(whole[others], parts[others])
+    ref, size = a[3].double() @ w.double().T, a[3].double().abs() @ w.double().abs().T
+    for got in (whole[3], parts[3]):
+        assert bool(((got.double() - ref).abs() <= size * K * 2.0**-24).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 40, 257), (3, 2050, 515), (4, 37, 1030), (7, 64, 287), (8, 2100, 1026), (12, 70, 2049), (16, 33, 319), (40, 90, 515),
                                    (70, 130, 257), (131, 140, 1025), (130, 70, 290)])  # fmt: skip
 @pytest.mark.parametrize("shift", [0, 1])
