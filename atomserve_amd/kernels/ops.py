@@ -718,6 +718,7 @@ def gemm(a, w, out, choices=None) -> None:
 LIBRARY_WORKSPACE_BYTES = 64 << 20
 LIBRARY_DECODE_ROWS = 64  # row counts up to here are decode steps' (padded to 32, 48 and 64)
 LIBRARY_TRIALS_EACH = 4
+SETTLE_EACH = 3  # runs of every candidate behind the fills that let the host get ahead, before a capture
 _workspace = {}  # device index -> the library's scratch memory, one for the process (its calls follow one another)
 
 # Beside the library's candidates a trial may time this package's plain tile product (9 to 128 rows, K in
@@ -873,13 +874,22 @@ class ProductChoices:
 
     def settle(self) -> None:
         """Ends every trial that is under way.  Called before a capture begins, so that the captured
-        launches are the ones later replays should make.  A shape that a pass meets once (the head)
-        has not come round often enough by then: the rest of its runs are made here, on the rows of its
-        last call and in turn all the weights that it has met, which the caches keep the less of the more they are."""
+        launches are the ones later replays should make.  In a pass the host is often the slower one, and a run's
+        time then is the host's between its two events (a kernel of 9 us came out at 10 to 28).  So each candidate runs
+        again here, the rest of its runs or SETTLE_EACH, behind fills of the library's scratch memory that let the host get
+        ahead and that push the weights out of the caches: on the rows of the last call and in turn all the
+        weights that the trial has met.  Large products, which the host does not hold up, run only what is left."""
         for key in list(self.trials):
             trial = self.trials.pop(key)
             a, _, out = trial["last"]
-            while not _tried_enough(trial):
+            runs = max(LIBRARY_TRIALS_EACH * trial["count"] - len(trial["runs"]),
+                       SETTLE_EACH * trial["count"] if key[0] <= LIBRARY_DECODE_ROWS else 0)  # fmt: skip
+            trial["ahead"] = len(trial["runs"])
+            space = _library_workspace(a.device)
+            for _ in range(2 * runs):
+                space.zero_()
+            for _ in range(runs):
+                space.zero_()
                 _trial_run(trial, a, trial["weights"][len(trial["runs"]) % len(trial["weights"])], out, *key[:3])
             torch.cuda.current_stream().synchronize()
             self.choice[key] = _fastest_of(trial)
@@ -909,21 +919,19 @@ def _trial_run(trial, a, w, out, M, N, K) -> None:
 
 
 def _fastest_of(trial) -> int:
-    """The candidate whose middle run took least, among the runs that were timed and have finished and leaving out each
-    candidate's first (which loads the kernel); 0 if none.  (A run is lengthened by whatever the host does between its two
-    events: on averages qkv of 16 rows at Qwen3-4B sizes went to 12.5 us instead of 9.3 in one process of three.  It is shortened
-    where the caches still hold its weights, which a replay reads from memory: the shortest run may be such a one.)"""
-    times = {}
-    for candidate, start, end in trial["runs"]:
+    """The candidate whose shortest run took least, among the runs that were timed and have finished: those with the host ahead
+    (`settle`) where every candidate has one, else all but each candidate's first (which loads the kernel); 0 if none.  (The host
+    between a run's two events lengthens it; the caches, which could shorten it, do not hold its weights: a pass comes back to
+    them after all others.  On averages qkv of 16 rows at Qwen3-4B sizes went to 12.5 us instead of 9.3 in one process of three.)"""
+    times, ahead = {}, {}
+    for n, (candidate, start, end) in enumerate(trial["runs"]):
         if start is not None and end.query():
             times.setdefault(candidate, []).append(start.elapsed_time(end))
-    best, best_time = 0, float("inf")
-    for candidate, took in times.items():
-        rest = sorted(took[1:] or took)
-        middle = rest[(len(rest) - 1) // 2]
-        if middle < best_time:
-            best, best_time = candidate, middle
-    return best
+            if n >= trial.get("ahead", n + 1):
+                ahead.setdefault(candidate, []).append(times[candidate][-1])
+    if ahead.keys() != times.keys():
+        ahead = {candidate: took[1:] or took for candidate, took in times.items()}
+    return min(ahead, key=lambda candidate: min(ahead[candidate]), default=0)
 
 
 # ---- 17 to 128 rows: tiles of weight rows with the activations staged in LDS --------------------

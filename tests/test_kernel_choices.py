@@ -178,26 +178,34 @@ class Mark:  # an event of a timed run
         return end.ms
 
 
-def test_the_middle_run_of_a_trial_decides():
-    """Neither a run that the host lengthened nor one whose weights the caches still held."""
-    runs = lambda *times: {"runs": [(c, Mark(), Mark(ms)) for n in range(4) for c, ms in enumerate(t[n] for t in times)]}  # noqa: E731
-    assert ops._fastest_of(runs((9.0, 5.0, 5.1, 5.0), (9.0, 4.0, 6.0, 6.0))) == 0
-    assert ops._fastest_of(runs((9.0, 6.0, 6.0, 6.0), (9.0, 5.0, 40.0, 5.0))) == 1
-    assert ops._fastest_of({"runs": [(3, None, None)]}) == 0
+def test_the_shortest_run_of_a_trial_decides():
+    """Of the runs with the host ahead where every candidate has one; else of all but each candidate's first."""
+    runs = lambda *times: [(c, Mark(), Mark(ms)) for n in range(len(times[0])) for c, ms in enumerate(t[n] for t in times)]  # noqa: E731
+    assert ops._fastest_of({"runs": runs((1.0, 5.0, 5.1, 50.0), (9.0, 6.0, 6.0, 6.0))}) == 0
+    assert ops._fastest_of({"runs": runs((9.0, 6.0, 6.0, 6.0), (9.0, 7.0, 40.0, 5.0))}) == 1
+    assert ops._fastest_of({"runs": runs((9.0, 3.0, 6.0, 6.0), (9.0, 40.0, 5.0, 5.5)), "ahead": 4}) == 1  # the last two runs of both
+    assert ops._fastest_of({"runs": runs((9.0, 3.0, 6.0), (9.0, 4.0, 5.0))[:5], "ahead": 4}) == 0  # only one candidate ran ahead
+    assert ops._fastest_of({"runs": [(3, None, None)]}) == 0 and ops._fastest_of({"runs": []}) == 0
 
 
 def test_the_rest_of_a_trial_runs_on_all_weights_in_turn(monkeypatch):
-    choices, met = ops.ProductChoices(), []
+    met, fills = [], []
 
     def run(trial, a, w, out, M, N, K):
         met.append(w)
         trial["runs"].append((trial["ids"][len(trial["runs"]) % trial["count"]], Mark(), Mark(1.0)))
 
     monkeypatch.setattr(ops, "_trial_run", run)
+    monkeypatch.setattr(ops, "_library_workspace", lambda device: type("W", (), {"zero_": lambda self: fills.append(len(met))})())
     monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"synchronize": lambda self: None})())
-    choices.trials[(32, 64, 64, BF16)] = {"count": 2, "ids": [0, 1], "runs": [], "weights": ["a", "b", "c"], "last": (None, "c", None)}
-    choices.settle()
-    assert met == ["a", "b", "c", "a", "b", "c", "a", "b"] and choices.chosen() == {(32, 64, 64, BF16): 0}
+    rows = torch.empty(1)
+    for M, done, more in ((32, 0, 8), (32, 8, 6), (2048, 6, 2), (2048, 8, 0)):
+        choices, before = ops.ProductChoices(), [(n % 2, Mark(), Mark(2.0)) for n in range(done)]
+        choices.trials[(M, 64, 64, BF16)] = {"count": 2, "ids": [0, 1], "runs": before, "weights": ["a", "b", "c"], "last": (rows, "c", None)}
+        met.clear(), fills.clear()
+        choices.settle()
+        assert met == [("a", "b", "c")[(done + n) % 3] for n in range(more)] and choices.chosen() == {(M, 64, 64, BF16): 0}
+        assert fills == [0] * 2 * more + list(range(more))  # the queue is filled before the first run and between the runs
 
 
 def test_how_rows_of_a_state_space_are_cut_into_segments():
