@@ -718,7 +718,7 @@ def gemm(a, w, out, choices=None) -> None:
 LIBRARY_WORKSPACE_BYTES = 64 << 20
 LIBRARY_DECODE_ROWS = 64  # row counts up to here are decode steps' (padded to 32, 48 and 64)
 LIBRARY_TRIALS_EACH = 4
-SETTLE_EACH = 3  # runs of every candidate behind the fills that let the host get ahead, before a capture
+SETTLE_EACH = 2  # runs of every candidate behind the fills that let the host get ahead, before a capture
 _workspace = {}  # device index -> the library's scratch memory, one for the process (its calls follow one another)
 
 # Beside the library's candidates a trial may time this package's plain tile product (9 to 128 rows, K in
@@ -876,20 +876,21 @@ class ProductChoices:
         """Ends every trial that is under way.  Called before a capture begins, so that the captured
         launches are the ones later replays should make.  In a pass the host is often the slower one, and a run's
         time then is the host's between its two events (a kernel of 9 us came out at 10 to 28).  So each candidate runs
-        again here, the rest of its runs or SETTLE_EACH, behind fills of the library's scratch memory that let the host get
-        ahead and that push the weights out of the caches: on the rows of the last call and in turn all the
-        weights that the trial has met.  Large products, which the host does not hold up, run only what is left."""
+        again here, SETTLE_EACH times behind fills of the library's scratch memory that let the host get
+        ahead and, between the runs, push the weights out of the caches: on the rows of the last call and in turn all
+        the weights that the trial has met.  Large products, which the host does not hold up, run what is left of their runs."""
         for key in list(self.trials):
             trial = self.trials.pop(key)
             a, _, out = trial["last"]
-            runs = max(LIBRARY_TRIALS_EACH * trial["count"] - len(trial["runs"]),
-                       SETTLE_EACH * trial["count"] if key[0] <= LIBRARY_DECODE_ROWS else 0)  # fmt: skip
-            trial["ahead"] = len(trial["runs"])
-            space = _library_workspace(a.device)
-            for _ in range(2 * runs):
-                space.zero_()
+            small = key[0] <= LIBRARY_DECODE_ROWS
+            runs = SETTLE_EACH * trial["count"] if small else LIBRARY_TRIALS_EACH * trial["count"] - len(trial["runs"])
+            if small:
+                trial["ahead"], space = len(trial["runs"]), _library_workspace(a.device)
+                for _ in range(runs):
+                    space.zero_()
             for _ in range(runs):
-                space.zero_()
+                if small:
+                    space[: LIBRARY_WORKSPACE_BYTES // 4].zero_()
                 _trial_run(trial, a, trial["weights"][len(trial["runs"]) % len(trial["weights"])], out, *key[:3])
             torch.cuda.current_stream().synchronize()
             self.choice[key] = _fastest_of(trial)
