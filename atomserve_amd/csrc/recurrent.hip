@@ -1404,7 +1404,8 @@ extern "C" int as_rglru_gates(const float* u, int width, int blocks, const void*
 //   composes them, the stretches are chained (four of a wave by lane moves, the waves' through LDS), and the thread runs its
 //   tokens again, out of its registers.  Every input is read once and the chain of dependent steps is 16 + 2 + 16 a thousand tokens, but it
 //   takes four times the workgroups, of which a compute unit holds one and of the middle way's two: only while the step's rows of more
-//   than SCAN_LONG tokens fit two rounds of them (every other row stays with the middle way), in a kernel of its own.
+//   than SCAN_LONG tokens fit two rounds of them (every other row stays with the middle way, or goes along where all rows of more than
+//   one token fit four: 32, 100 and 168 tokens at 4,096 channels in two kernels 14.7 us, in one 10), in a kernel of its own.
 // The rows of a way are dealt to lines of workgroups by their place among them, so that no row costs workgroups that find
 // nothing to do.  Neighbouring workgroups of an XCD take neighbouring channels, so that a 128-byte line of two workgroups'
 // channels enters one L2.
@@ -1588,9 +1589,9 @@ template <typename T, typename W> __device__ __forceinline__ void scan_ones(cons
   const Scan<T, W> p = {a, x, proj, y_bias, state, row_first, row_len, row_start, row_slots, out, width, ld, y_off, ld_out, out_off,     \
                         writes, num_rows, scale}
 
-// blockIdx.y < lines: long rows; beyond: rows of one token
+// blockIdx.y < lines: rows of more than `low` tokens; beyond: rows of one token
 template <typename T, typename W>
-__global__ __launch_bounds__(SCAN_THREADS) void rglru_long_kernel(SCAN_PARAMS, int lines, int per_xcd) {
+__global__ __launch_bounds__(SCAN_THREADS) void rglru_long_kernel(SCAN_PARAMS, int lines, int per_xcd, int low) {
   SCAN_STRUCT;
   __shared__ float ends[2][2][SCAN_WAVES][SCAN_CHANNELS];  // [round % 2][decays, ends]
   if ((int)blockIdx.y >= lines) return scan_ones(p, ((int)blockIdx.y - lines) * per_xcd * 8 + (int)blockIdx.x);
@@ -1598,7 +1599,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void rglru_long_kernel(SCAN_PARAMS, i
   if (tile * SCAN_CHANNELS >= width) return;
   int buf = 0;
   if (lines == num_rows) rglru_long(p, ends, buf, scan_row(p, blockIdx.y), tile);  // all of them
-  else scan_rows(p, SCAN_LONG, INT_MAX, blockIdx.y, lines, [&](const ScanRow& row) { rglru_long(p, ends, buf, row, tile); });
+  else scan_rows(p, low, INT_MAX, blockIdx.y, lines, [&](const ScanRow& row) { rglru_long(p, ends, buf, row, tile); });
 }
 
 // BY_ROW: row blockIdx.y, whatever its length.  Else `lines` times the groups of 64 channels workgroups: rows of 2 to `high` tokens; the
@@ -1640,7 +1641,8 @@ extern "C" int as_rglru_scan(const float* a, const float* x, int width, const vo
   // two rounds of workgroups of either way at most; a line a row where few rows or none have one token
   const bool long_way = only ? num_tokens > SCAN_ONLY : many > 0 && many <= std::max(1, 2 * cus / tiles);
   const bool by_row = !long_way && (only || (known && several == num_rows) || (long)num_rows * groups <= 2 * cus);
-  const int longs = only ? 1 : many, middle = only ? 0 : several - (long_way ? many : 0);
+  const int low = several <= std::max(1, 4 * cus / tiles) ? 1 : SCAN_LONG;  // a few middle rows go with the long ones: a launch less
+  const int longs = only ? 1 : low == 1 ? several : many, middle = only ? 0 : several - (long_way ? longs : 0);
   const int lines = by_row ? 0 : std::min(middle, std::max(1, 4 * cus / groups));
   const long ones = by_row || only || (known && several == num_rows) ? 0 : (long)num_rows * chunks;
   const long blocks = (long)lines * groups + (long_way ? 0 : ones);
@@ -1655,7 +1657,7 @@ extern "C" int as_rglru_scan(const float* a, const float* x, int width, const vo
       break;                                                                                                             \
     }                                                                                                                    \
     if (long_way)                                                                                                        \
-      rglru_long_kernel<T, W><<<dim3(all, longs + (int)((ones + all - 1) / all)), SCAN_THREADS, 0, stream>>>(ARGS(T, W), longs, per_xcd); \
+      rglru_long_kernel<T, W><<<dim3(all, longs + (int)((ones + all - 1) / all)), SCAN_THREADS, 0, stream>>>(ARGS(T, W), longs, per_xcd, low); \
     if (by_row)                                                                                                          \
       rglru_scan_kernel<T, W, true><<<dim3(groups, num_rows), SCAN_THREADS, 0, stream>>>(ARGS(T, W), 0, groups, 0);       \
     else if (blocks > 0)                                                                                                 \

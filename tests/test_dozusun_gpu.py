@@ -747,6 +747,7 @@ def test_scan_of_a_linear_recurrence(width, dtype, bias):
     (2048, [1] * 30 + [100] * 5 + [3]),  # more long rows than fit two rounds
     (2048, [9] * 18 + [65]), (1024, [9] * 18),  # no row of one token
     (100, [1, 5, 80, 1, 1030]), (2048, [1] * 66 + [5] + [1] * 70 + [70] + [2] * 3),  # rows beyond the first 64
+    (1024, [32, 100, 168]), (1024, [1] * 70 + [2, 64, 65, 9]),  # middle rows that go with the long ones
     (48, [2]), (100, [32]), (100, [33]), (16, [1025]),
 ])  # fmt: skip
 def test_scan_of_many_and_few_rows(width, lens):
