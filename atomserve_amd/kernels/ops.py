@@ -872,6 +872,7 @@ class ProductChoices:
         place = entry("as_blas_adopt")(M, N, K, _DT[dtype], LIBRARY_WORKSPACE_BYTES, index)
         return place if place >= 0 else 0
 
+    @torch.inference_mode()
     def settle(self) -> None:
         """Ends every trial that is under way.  Called before a capture begins, so that the captured
         launches are the ones later replays should make.  In a pass the host is often the slower one, and a run's

@@ -207,6 +207,12 @@ def test_the_rest_of_a_trial_runs_on_all_weights_in_turn(monkeypatch):
         choices.settle()
         assert met == [("a", "b", "c")[(done + n) % 3] for n in range(more)] and (M, 64, 64, BF16) in choices.chosen()
         assert fills == ([0] * more + list(range(more)) if M == 32 else [])  # the queue is filled before the first run and between the runs
+    with torch.inference_mode():
+        space = torch.ones(8, dtype=torch.uint8)  # what a model's pass has made, cleared by a caller outside of it
+    monkeypatch.setattr(ops, "_library_workspace", lambda device: space)
+    choices.trials[(32, 64, 64, BF16)] = {"count": 1, "ids": [0], "runs": [], "weights": ["a"], "last": (rows, "a", None)}
+    choices.settle()
+    assert int(space.sum()) == 0
 
 
 def test_how_rows_of_a_state_space_are_cut_into_segments():
