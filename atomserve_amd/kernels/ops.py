@@ -1065,6 +1065,80 @@ def gemm_split(a, w, plan=None):
     return sums
 
 
+# ---- more than 128 rows: tiles of up to 256 x 256 outputs, both operands through LDS (`csrc/gemm_wide.hip`) ---------------
+WIDE_MIN_ROWS, WIDE_MAX_ROWS = TILE_MAX_ROWS + 1, 65536
+WIDE_UNIT = 64  # K comes in units of this many columns
+WIDE_PLAIN, WIDE_GATED, WIDE_PARTIAL = 0, 1, 2
+# (rows of a, rows of w, workgroups a compute unit, us a unit of K with all places taken, with few, us a round beside the units),
+# fitted to 2,900 times: 24 products of Qwen3's six sizes, 136 to 2,409 rows, every form and 1 to 12 ranges of K (off by 5 per cent on
+# average, by 25 at most; the form it chooses is within 1 per cent of the best on average)
+WIDE_FORMS = ((256, 256, 1, 1.33, 0.96, 6.6), (256, 192, 1, 1.09, 0.765, 4.5), (256, 128, 1, 0.83, 0.62, 2.4),
+              (192, 256, 1, 1.215, 0.825, 7.6), (128, 128, 1, 0.53, 0.375, 1.0), (128, 128, 2, 1.0, 0.52, 0.5))  # fmt: skip
+WIDE_LAUNCH_US, WIDE_US_A_MB, WIDE_SPLITS = 3.0, 0.2, (2, 3, 4, 6, 8, 12)
+
+
+def _wide_cost(form: int, tiles: int, units: int) -> float:
+    """Microseconds of `tiles` tiles of `units` units of K each: whole rounds of workgroups, and what is left in a round that shares
+    the memory and the power among fewer."""
+    *_, each, full, few, round_us = WIDE_FORMS[form]
+    rounds, rest = divmod(tiles, each * compute_units())
+    share = rest / (each * compute_units())
+    return WIDE_LAUNCH_US + rounds * (units * full + round_us) + ((units * (few + (full - few) * share) + round_us) if rest else 0.0)
+
+
+@functools.lru_cache(maxsize=4096)
+def _wide_plan(rows: int, n: int, k: int, kind: int) -> tuple:
+    """(us, form, splits) of the cheapest tile for a product of these sizes (kind gated: n outputs of 2 n rows of w; partial: with K cut into
+    ranges whose sums are written, and read by whoever adds them up; in one round of workgroups)."""
+    best = None
+    for form, (tm, tn, each, *_) in enumerate(WIDE_FORMS):
+        tiles = -(-rows // tm) * -(-n // (tn // 2 if kind == WIDE_GATED else tn))
+        for splits in WIDE_SPLITS if kind == WIDE_PARTIAL else (1,):
+            units = -(-(k // WIDE_UNIT) // splits)
+            if kind == WIDE_PARTIAL and (tiles * splits > compute_units() or (splits - 1) * units >= k // WIDE_UNIT):
+                continue
+            us = _wide_cost(form, tiles * splits, units)
+            if kind == WIDE_PARTIAL:
+                us += 2 * WIDE_US_A_MB * splits * rows * n * 4e-6
+            if best is None or us < best[0]:
+                best = us, form, splits
+    return best
+
+
+def _library_us(rows: int, n: int, k: int) -> float:
+    """What the library's best kernel of 16 took for the same products (off by 7 per cent on average, by a third at most)."""
+    return 5.8 + 0.66e-9 * 2 * rows * n * k + 0.11 * n * k * 2e-6 + 1.79e-3 * k
+
+
+def _wide_takes(a, w, n: int, rows_of_w: int) -> bool:
+    M, K = a.shape
+    return (a.dtype == BF16 and WIDE_MIN_ROWS <= M <= WIDE_MAX_ROWS and K % WIDE_UNIT == 0 and n % 16 == 0
+            and max(M, rows_of_w) * K * 2 <= 0xF0000000 and a.data_ptr() % 16 == 0 and _rows(w).data_ptr() % 16 == 0)  # fmt: skip
+
+
+@functools.lru_cache(maxsize=4096)
+def wide_gated_form(rows: int, outputs: int, k: int):
+    """The tile of a gated product of more than 128 rows, or None where the library's product with the activation after it is expected
+    to take less: four of the 72 measured products, tall of few rows (333 rows of 12,288 outputs and K = 4,096: 75 us, 83).  Elsewhere, us of
+    the library's best of 16 and the activation, and of this: 3,072 outputs of K = 1,024, 256 / 1,024 / 2,409 rows 19.1 11.5, 24.8 17.6,
+    38.0 32.9; 9,728 of 2,560, 512 / 2,409 rows 61 52, 228 197; 12,288 of 4,096, 512 / 2,048 rows 91 86, 297 300; 25,600 of 5,120, 1,500 rows
+    693 604."""
+    us, form, _ = _wide_plan(rows, outputs, k, WIDE_GATED)
+    return form if us < _library_us(rows, 2 * outputs, k) + 4.0 + 6e-6 * WIDE_US_A_MB * rows * outputs else None
+
+
+@functools.lru_cache(maxsize=4096)
+def wide_split_plan(rows: int, n: int, k: int):
+    """(form, splits) of a product of more than 128 rows cut along K into partial sums, or None where that, the sums' reading counted, is
+    not expected to save 5 per cent of the library's whole product (74 of 144 measured products are cut; none of them was slower):
+    4,096 outputs of K = 12,288, 256 / 512 / 1,024 rows 52 39, 78 56, 106 95; 2,560 of 9,728, 512 / 2,048 rows 52 38, 102 95; 5,120 of
+    17,408, 256 rows 129 58; 1,024 of 3,072, 256 rows 12.5 10.2.  Short products of many rows stay whole (4,096 of 4,096, 700 rows 34 37)."""
+    best = _wide_plan(rows, n, k, WIDE_PARTIAL)
+    if best is None or best[0] >= 0.95 * (_library_us(rows, n, k) + 2e-6 * WIDE_US_A_MB * rows * n):
+        return None
+    return best[1:]
+
+
 F32_NARROW = 256  # up to here a 32-bit sum is one chain, which nothing cuts
 F32_GROUPS = 4  # what a 32-bit sum's order comes in above that, whatever kernel runs
 
@@ -1096,6 +1170,17 @@ def gemm_split_sums(a, w):
     N = _rows(w).shape[0]
     if a.dtype == F32:
         return gemm_f32_split(a, w) if gemm_f32_split_preferred(M, N, K) else None
+    if _wide_takes(a, w, N, N):
+        plan = wide_split_plan(M, N, K)
+        if plan is None:
+            return None
+        form, splits = plan
+        rows = _rows(w)
+        _check(a, "a", BF16, (M, K))
+        _check(rows, "w", BF16, (N, K))
+        sums = torch.empty((splits, M, N), dtype=F32, device=a.device)
+        call("as_gemm_bf16_wide", _ptr(a), _ptr(rows), _ptr(sums), M, N, K, WIDE_PARTIAL, splits, form, _stream())
+        return sums
     plan = gemm_split_plan(M, N, K, a.dtype)
     return None if plan is None else gemm_split(a, w, plan)
 
@@ -1135,6 +1220,11 @@ def gemm_silu_mul(a, w, out, choices=None) -> None:
         call("as_gemm_bf16_tile", _ptr(a), _ptr(rows), _wave_ptr(w), _ptr(out), 0, _DT[BF16], M, inter, K, 1, 0,
              _gated_tile_strips(M, inter), _stream())  # fmt: skip
         return
+    if _wide_takes(a, w, inter, 2 * inter) and out.data_ptr() % 16 == 0:
+        form = wide_gated_form(M, inter, K)
+        if form is not None:
+            call("as_gemm_bf16_wide", _ptr(a), _ptr(rows), _ptr(out), M, inter, K, WIDE_GATED, 1, form, _stream())
+            return
     gate_up = torch.empty((M, 2 * inter), dtype=a.dtype, device=a.device)
     gemm(a, w, gate_up, choices)
     silu_mul(gate_up, out)

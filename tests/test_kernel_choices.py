@@ -253,3 +253,27 @@ def test_the_route_of_a_32_bit_portion(monkeypatch, tokens, start, how):
     step = SimpleNamespace(decode_only=False, all_tokens="all", positions=None, tok_row=None, max_context=start + tokens, split=lambda key: rows)
     attend(torch.empty(tokens, 16, 128), None, step, cache, 1.0, 0, (8, 64))
     assert made == [{"single": ("single", "all"), "tiles": ("tiles", "long"), "short": ("single", "short")}[how]]
+
+
+def test_plans_of_wide_products(monkeypatch):
+    """Products of more than 128 rows: ranges of K that are none of them empty, in one round of workgroups, and no range where
+    the library's whole product takes less."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    for cached in (ops._wide_plan, ops.wide_split_plan, ops.wide_gated_form):
+        cached.cache_clear()
+    try:
+        for rows in (129, 200, 333, 512, 1000, 2409, 65536):
+            for n, k in ((16, 64), (1024, 3072), (2560, 9728), (4096, 12288), (5120, 25600), (4096, 64), (151936, 4096)):
+                plan = ops.wide_split_plan(rows, n, k)
+                if plan is not None:
+                    tm, tn, each, *_ = ops.WIDE_FORMS[plan[0]]
+                    units = -(-(k // 64) // plan[1])
+                    assert plan[1] > 1 and (plan[1] - 1) * units < k // 64
+                    assert -(-rows // tm) * -(-n // tn) * plan[1] <= 256
+                assert ops.wide_gated_form(rows, n, k) in (None, *range(len(ops.WIDE_FORMS)))
+        assert ops.wide_split_plan(512, 4096, 12288) == (2, 4) and ops.wide_split_plan(256, 2560, 9728) == (4, 6)
+        assert ops.wide_split_plan(2048, 4096, 4096) is None and ops.wide_split_plan(1500, 1024, 2048) is None
+        assert ops.wide_gated_form(2048, 12288, 4096) == 0 and ops.wide_gated_form(512, 12288, 4096) == 1
+    finally:
+        for cached in (ops._wide_plan, ops.wide_split_plan, ops.wide_gated_form):
+            cached.cache_clear()

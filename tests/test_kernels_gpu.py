@@ -1579,3 +1579,62 @@ def test_gemm_link_and_scaled_f32(ops, M, N, K, shift):
             bound = 1.1 * bound[:, :L] * u.abs() + (g.abs() + bound[:, :L]) * bound[:, L:] + 8 * 2.0**-24 * ref.abs() + 1e-12
         assert bool(((out.double() - ref).abs() <= bound).all())
     assert not ops.gemm_f32_link_supported(17, N, K) and not ops.gemm_f32_link_supported(M, 256, K)
+
+
+@pytest.mark.parametrize("form", range(6))
+@pytest.mark.parametrize("M,N,K", [(1, 16, 64), (129, 208, 128), (300, 528, 320), (513, 784, 192), (257, 1040, 1024)])
+def test_wide_products(ops, form, M, N, K):
+    """Every tile of the products of many rows, plain, gated and in ranges of K, at the edges of tiles, with one unit of K and with a
+    last range that is shorter.  Operands are whole numbers up to 4, so that every sum of up to 1,024 products is a whole number that
+    32 bits hold: any order of sums gives it, and the results have one right value."""
+    from atomserve_amd.kernels.lib import KernelError, call
+
+    torch.manual_seed(M + N + K)
+    a = torch.randint(-4, 5, (M, K), device=DEV).to(BF16)
+    w = torch.randint(-4, 5, (2 * N, K), device=DEV).to(BF16)
+    exact = a.float() @ w.float().t()
+
+    def run(out, kind, splits):
+        call("as_gemm_bf16_wide", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, kind, splits, form, ops._stream())
+        return out
+
+    out = run(torch.full((M, N), float("nan"), device=DEV, dtype=BF16), ops.WIDE_PLAIN, 1)
+    assert torch.equal(out, exact[:, :N].to(BF16))
+    w.mul_(2.0**-7)  # gates of a few units
+    gate_up = (exact * 2.0**-7).to(BF16)
+    both = torch.empty(M, N, device=DEV, dtype=BF16)
+    ops.silu_mul(gate_up, both)
+    assert torch.equal(run(torch.full((M, N), float("nan"), device=DEV, dtype=BF16), ops.WIDE_GATED, 1), both)
+    units = K // ops.WIDE_UNIT
+    for splits in {1, 2, 3, units}:
+        per = -(-units // splits)
+        sums = torch.full((splits, M, N), float("nan"), device=DEV)
+        if (splits - 1) * per >= units:
+            with pytest.raises(KernelError):
+                run(sums, ops.WIDE_PARTIAL, splits)
+            continue
+        run(sums, ops.WIDE_PARTIAL, splits)
+        for i in range(splits):
+            part = slice(i * per * 64, min(K, (i + 1) * per * 64))
+            assert torch.equal(sums[i], a[:, part].float() @ w[:N, part].float().t())
+
+
+def test_wide_products_are_what_many_rows_take(ops):
+    """`gemm_silu_mul` and `gemm_split_sums` of more than 128 rows: their rules, and the bits of the product and the activation."""
+    torch.manual_seed(3)
+    M, N, K = 300, 3072, 1024
+    a = torch.randint(-4, 5, (M, K), device=DEV).to(BF16)
+    w = torch.randint(-4, 5, (2 * N, K), device=DEV).to(BF16) * 2.0**-7
+    out, two = torch.empty(M, N, device=DEV, dtype=BF16), torch.empty(M, N, device=DEV, dtype=BF16)
+    assert ops.wide_gated_form(M, N, K) is not None
+    ops.gemm_silu_mul(a, w, out)
+    ops.silu_mul((a.float() @ w.float().t()).to(BF16), two)
+    assert torch.equal(out, two)
+    shifted = torch.empty(M * K + 1, device=DEV, dtype=BF16)[1:].view(M, K).copy_(a)  # rows that do not start on 16 bytes: two kernels
+    ops.gemm_silu_mul(shifted, w, out)
+    assert torch.equal(out, two)
+    act, down = out, torch.randint(-4, 5, (K, N), device=DEV).to(BF16)
+    act.copy_(torch.randint(-4, 5, (M, N), device=DEV))
+    sums = ops.gemm_split_sums(act, down)
+    assert sums.shape[0] == ops.wide_split_plan(M, K, N)[1] > 1
+    assert torch.equal(sums.sum(0), act.float() @ down.float().t())
