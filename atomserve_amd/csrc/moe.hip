@@ -8,8 +8,7 @@
 // (so the outputs of a token's experts lie side by side), and `moe_combine` adds them up with their
 // weights.  A pair's result does not depend on what else is in the step: every output is a dot product
 // over the whole width in a fixed order.
-#include "common.h"
-#include <type_traits>
+#include "wide_tile.h"
 
 #define MOE_TILE 128     // pairs of one expert that a tile holds at most (eight column tiles of 16); a route has tiles of 64 or 128
 #define MOE_HALF 64      // four column tiles
@@ -430,44 +429,28 @@ __global__ __launch_bounds__(256) void moe_gemm_bf16_kernel(const bf16* __restri
 // wave's two loads use whole lines.  Weights' loads go through a buffer descriptor of the expert's matrix: those for chunks past
 // the last are sent beyond its end, where they move nothing, and the number of loads in flight is the same everywhere.
 // Workgroups start at different blocks of columns and wrap round, so that they do not all ask for the same memory channels.
-// WIDE: tiles of 128 pairs by 8 waves.  What bounds a prompt's product is what the compute units load, weights and
-//   activations together, most of it from L2: the larger the tile, the less (1,500 tokens of 2 of 16 experts, width 2,048, gate
-//   and up of 1,536: 950 MB in tiles of 64 x 128, 550 in tiles of 128 x 256).  An XCD takes a run of neighbouring (strip,
-//   tile) places, so that the tiles of one expert read a strip from one L2.
-// else: tiles of 64 by 4 waves, weights two chunks of 128 ahead: few pairs, for which the weights are streamed.
-// Both add up an output's products in one order, which depends on the output and its expert alone.
+// An output's products are added up in one order, which depends on the output and its expert alone.
 // Two of 16 experts, both products of a layer, us before (every operand through LDS, tiles of 64 x 64) and now: width 4,096, 8 tokens
-// 155 and 144, 32 255 and 207 (6.0 and 5.5 TB/s of weights), 512 313 and 272, 2,048 752 and 544 (600 TFLOP/s); width 2,048,
-// 1,500 tokens 183 and 126; width 1,024, 300 tokens 32 and 27.
+// 155 and 144, 32 255 and 207 (6.0 and 5.5 TB/s of weights); more pairs: below.
 enum { MOE_PLAIN, MOE_GATED, MOE_RELU2 };
 
-template <int MODE, typename OutT, bool WIDE>
-__global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 4 : 2) void moe_gemm_stream_kernel(
+template <int MODE, typename OutT>
+__global__ __launch_bounds__(256, 2) void moe_gemm_stream_kernel(
     const bf16* __restrict__ a, int a_div, const bf16* __restrict__ w, int N, int K, const int* __restrict__ order,
-    const int* __restrict__ tiles, const int* __restrict__ counts, OutT* __restrict__ out, float limit, int strips) {
+    const int* __restrict__ tiles, const int* __restrict__ counts, OutT* __restrict__ out, float limit) {
   constexpr bool GATED = MODE == MOE_GATED;
-  constexpr int WAVES = WIDE ? 8 : 4, S = GATED || WIDE ? 2 : 1;  // waves, strips of weight rows a wave
-  constexpr int ACROSS = WAVES * 16 * (GATED ? 1 : S);             // outputs a workgroup
-  constexpr int KC = WIDE ? 64 : 128, STEPS = KC / 64, PIECES = KC / 8;
-  constexpr int MOST = WIDE ? MOE_TILE : MOE_TILE / 2, PASS = WAVES * 64 / PIECES;  // pairs; rows the threads bring at once
+  constexpr int WAVES = 4, S = GATED ? 2 : 1;  // waves, strips of weight rows a wave
+  constexpr int ACROSS = WAVES * 16;           // outputs a workgroup
+  constexpr int KC = 128, STEPS = KC / 64, PIECES = KC / 8;
+  constexpr int MOST = MOE_HALF, PASS = WAVES * 64 / PIECES;  // pairs; rows the threads bring at once
   constexpr unsigned BEYOND = 0xfffffff0u;
   __shared__ u32x4 lds[2][MOST * PIECES];
-  int tile, strip;
-  if constexpr (WIDE) {
-    const int live = counts[0], total = live * strips, per_xcd = (total + 7) >> 3;
-    const int place = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || place >= total) return;
-    strip = place / live;
-    tile = place - strip * live;
-  } else {
-    strip = blockIdx.x;
-    tile = blockIdx.y;
-    if (tile >= counts[0]) return;
-  }
+  const int strip = blockIdx.x, tile = blockIdx.y;
+  if (tile >= counts[0]) return;
   const int e = tiles[3 * tile], at = tiles[3 * tile + 1], cnt = min(tiles[3 * tile + 2], MOST);
   const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lr = lane & 15, lg = lane >> 4;
-  const int n0 = strip * ACROSS + wave * (GATED ? 16 : 16 * S);
+  const int n0 = strip * ACROSS + wave * 16;
   const int nchunks = K / KC, turn = (int)((strip * ACROSS / (GATED ? 128 : 256) * 5u + (unsigned)e * 3u) % (unsigned)(K / 128)) * (128 / KC);
   const unsigned NW = GATED ? 2 * N : N;
   const __amdgpu_buffer_rsrc_t w_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(w) + (size_t)e * NW * K, 0,
@@ -481,17 +464,16 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 4 : 2) void moe_gemm_strea
   auto where = [&](int j) { const int c = j + turn; return c >= nchunks ? c - nchunks : c; };
   // LDS place (16 bytes) of block c (8 columns) of pair row r: the hardware reads 16-byte operands in the lane groups
   // {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31} and the same above 32, which so touch every bank once
-  auto place_of = [](int r, int c) { return PIECES == 16 ? r * 16 + (c ^ (r & 15)) : r * 8 + (c ^ (0x32765410 >> ((r & 14) * 2) & 7)); };
+  auto place_of = [](int r, int c) { return r * 16 + (c ^ (r & 15)); };
 
   auto run = [&](auto count) {
     constexpr int CT = decltype(count)::value, TIMES = (CT * 16 + PASS - 1) / PASS;
-    constexpr int AHEAD = WIDE ? 1 : 2;  // chunks of weights in flight
     const int piece = threadIdx.x % PIECES, prow = threadIdx.x / PIECES;  // this thread brings 16 bytes of rows prow + PASS i
     int pair[TIMES];
     const bf16* arow[TIMES];
 #pragma unroll
     for (int i = 0; i < TIMES; ++i) pair[i] = order[at + min(prow + PASS * i, cnt - 1)];
-    u32x4 wa[STEPS][S][2], wb[STEPS][S][2], wc[AHEAD == 2 ? STEPS : 1][S][2], held[TIMES];
+    u32x4 wa[STEPS][S][2], wb[STEPS][S][2], wc[STEPS][S][2], held[TIMES];
     auto fetch = [&](u32x4 (&into)[STEPS][S][2], int j) {
       const unsigned col = (unsigned)where(j) * (KC * 2u);
 #pragma unroll
@@ -518,7 +500,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 4 : 2) void moe_gemm_strea
 #pragma unroll
       for (int i = 0; i < TIMES; ++i) lds[j & 1][place_of(prow + PASS * i, piece)] = held[i];
       request(j + 1);
-      fetch(later, j + AHEAD);
+      fetch(later, j + 2);
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes have landed
       __builtin_amdgcn_s_barrier();
 #pragma unroll
@@ -531,31 +513,22 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 4 : 2) void moe_gemm_strea
 #pragma unroll
             for (int s = 0; s < S; ++s)
               acc[s][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, now[t][s][h]), av, acc[s][i], 0, 0, 0);
-            if (WIDE && CT > 4 && i % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four operands read ahead are what 128 registers hold
           }
     };
     fetch(wa, 0);
-    if constexpr (AHEAD == 2) fetch(wb, 1);
+    fetch(wb, 1);
     __builtin_amdgcn_sched_barrier(0);  // the first weights are asked for before the pairs' numbers are waited for
 #pragma unroll
     for (int i = 0; i < TIMES; ++i) arow[i] = a + (size_t)(pair[i] / a_div) * K + piece * 8;
     request(0);
-    if constexpr (AHEAD == 2) {
-      const int rounds = nchunks / 3;
-      for (int it = 0; it < rounds; ++it) {  // three chunks: the roles of the weights' registers come round
-        chunk(3 * it, wa, wc);
-        chunk(3 * it + 1, wb, wa);
-        chunk(3 * it + 2, wc, wb);
-      }
-      if (nchunks - 3 * rounds >= 1) chunk(3 * rounds, wa, wc);
-      if (nchunks - 3 * rounds == 2) chunk(3 * rounds + 1, wb, wa);
-    } else {
-      for (int j = 0; j + 2 <= nchunks; j += 2) {
-        chunk(j, wa, wb);
-        chunk(j + 1, wb, wa);
-      }
-      if (nchunks & 1) chunk(nchunks - 1, wa, wb);
+    const int rounds = nchunks / 3;
+    for (int it = 0; it < rounds; ++it) {  // three chunks: the roles of the weights' registers come round
+      chunk(3 * it, wa, wc);
+      chunk(3 * it + 1, wb, wa);
+      chunk(3 * it + 2, wc, wb);
     }
+    if (nchunks - 3 * rounds >= 1) chunk(3 * rounds, wa, wc);
+    if (nchunks - 3 * rounds == 2) chunk(3 * rounds + 1, wb, wa);
     // a lane holds outputs n .. n+3 of either strip for the pair in column lr of each column tile
 #pragma unroll
     for (int i = 0; i < CT; ++i) {
@@ -579,14 +552,115 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, WIDE ? 4 : 2) void moe_gemm_strea
     }
   };
   const int col_tiles = (cnt + 15) >> 4;
-  if constexpr (WIDE) {
-    if (col_tiles > 6) return run(std::integral_constant<int, 8>{});
-    if (col_tiles > 4) return run(std::integral_constant<int, 6>{});
-  }
   if (col_tiles == 4) run(std::integral_constant<int, 4>{});
   else if (col_tiles == 3) run(std::integral_constant<int, 3>{});
   else if (col_tiles == 2) run(std::integral_constant<int, 2>{});
   else run(std::integral_constant<int, 1>{});
+}
+
+// Tiles of 128 pairs: the same products, the same bits, with both operands in LDS by copies that pass no register (`wide_tile.h`); the
+// pairs' rows of a are where the copies' lanes find them.  A tile's first 64 pairs are the first four waves', whose neighbours on their
+// SIMDs are the other four: where a tile has no more, those only copy.
+template <int MODE, typename OutT, int FN, int RA, int RW>
+__global__ __launch_bounds__(512, 2) void moe_gemm_tile_kernel(const bf16* __restrict__ a, int a_div, const bf16* __restrict__ w, int N, int K,
+                                                               const int* __restrict__ order, const int* __restrict__ tiles,
+                                                               const int* __restrict__ counts, OutT* __restrict__ out, float limit, int strips) {
+  using T = wide::Tile<2, 4, 4, FN, RA, RW, true>;
+  static_assert(T::TM == MOE_TILE, "a tile's pairs");
+  constexpr bool GATED = MODE == MOE_GATED;
+  constexpr int ACROSS = GATED ? T::TN / 2 : T::TN;  // outputs of a workgroup
+  extern __shared__ __attribute__((aligned(128))) char tile_lds[];
+  const int live = counts[0], total = live * strips, per_xcd = (total + 7) >> 3;
+  const int place = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || place >= total) return;
+  const int strip = place / live, tile = place - strip * live;
+  const int e = tiles[3 * tile], at = tiles[3 * tile + 1], cnt = min(tiles[3 * tile + 2], MOE_TILE);
+  const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lr = lane & 15, lg = lane >> 4, wm = wave >> 2, wn = wave & 3;
+  const int n0 = strip * ACROSS;
+  const int units = K / wide::UNIT, turn = (int)((unsigned)(n0 / (GATED ? 128 : 256) * 5 + e * 3) % (unsigned)(K / 128)) * 2;
+  auto column = [&](int t) { const int u = min(t, units - 1) + turn; return (unsigned)(u >= units ? u - units : u) * wide::ROW_BYTES; };
+
+  const unsigned pitch = (unsigned)K * 2u, NW = GATED ? 2 * N : N;
+  const __amdgpu_buffer_rsrc_t a_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a), 0, (int)0xfffffff0u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t w_buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(w) + (size_t)e * NW * K, 0, (int)(NW * pitch), 0x00020000);
+  unsigned a_at[T::A_COPIES], w_at[T::W_COPIES];
+#pragma unroll
+  for (int i = 0; i < T::A_COPIES; ++i) {  // rows beyond the tile's pairs repeat its last
+    const int row = T::row_of(i, wave, lane);
+    a_at[i] = (unsigned)(order[at + min(row, cnt - 1)] / a_div) * pitch + T::piece_of(row, lane);
+  }
+#pragma unroll
+  for (int i = 0; i < T::W_COPIES; ++i) {  // rows beyond N repeat the last; which row lies where: so that a lane's sums are neighbours
+    const int row = T::row_of(i, wave, lane);
+    const int column_of_waves = row / (16 * FN), q = row % (16 * FN), f = q >> 4, g = (q >> 2) & 3, r = q & 3;
+    int n;
+    if constexpr (GATED) n = min(n0 + column_of_waves * 8 * FN + g * 2 * FN + 2 * f + (r & 1), N - 1) + (r >> 1) * N;
+    else if constexpr (sizeof(OutT) == 4) n = min(n0 + row, N - 1);
+    else n = min(n0 + column_of_waves * 16 * FN + (f & ~1) * 16 + 8 * g + 4 * (f & 1) + r, N - 1);
+    w_at[i] = (unsigned)n * pitch + T::piece_of(row, lane);
+  }
+  floatx4 acc[4][FN];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const bool idle = wm * 64 >= cnt;
+  T::run(tile_lds, a_buf, w_buf, a_at, w_at, wave, wm, wn, lane, units, column, acc, idle);
+  if (idle) return;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = wm * 64 + i * 16 + lr;
+    if (row >= cnt) continue;
+    OutT* to = out + (size_t)order[at + row] * N;
+    if constexpr (GATED) {
+      const int n = n0 + wn * 8 * FN + lg * 2 * FN;
+      alignas(16) bf16 v[2 * FN];
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 2; ++r) v[2 * j + r] = (bf16)gate_times_up(to_f32((bf16)acc[i][j][r]), to_f32((bf16)acc[i][j][2 + r]), limit);
+      if (n >= N) continue;  // N % 16 == 0
+      if constexpr (FN == 4) *reinterpret_cast<u32x4*>(to + n) = *reinterpret_cast<const u32x4*>(v);
+      else *reinterpret_cast<uint2*>(to + n) = *reinterpret_cast<const uint2*>(v);
+    } else if constexpr (sizeof(OutT) == 4) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const int n = n0 + wn * 16 * FN + j * 16 + 4 * lg;
+        if (n < N) *reinterpret_cast<floatx4*>(to + n) = acc[i][j];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < FN; j += 2) {
+        const int n = n0 + wn * 16 * FN + j * 16 + 8 * lg;
+        alignas(16) bf16 v[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          float z = acc[i][j + (r >> 2)][r & 3];
+          if (MODE == MOE_RELU2) { z = fmaxf(to_f32((bf16)z), 0.f); z *= z; }
+          v[r] = (bf16)z;
+        }
+        if (n < N) *reinterpret_cast<u32x4*>(to + n) = *reinterpret_cast<const u32x4*>(v);
+      }
+    }
+  }
+}
+
+template <int MODE, typename OutT, int FN, int RA, int RW>
+static int launch_moe_tile(const void* a, int a_div, const void* w, int N, int K, const int* order, const int* tiles, const int* counts,
+                           int max_tiles, void* out, float limit, hipStream_t stream) {
+  using T = wide::Tile<2, 4, 4, FN, RA, RW, true>;
+  const int across = MODE == MOE_GATED ? T::TN / 2 : T::TN, strips = (N + across - 1) / across;
+  if ((long long)strips * max_tiles > 0x7ffff8ll) return AS_BAD_SHAPE;
+  auto kernel = moe_gemm_tile_kernel<MODE, OutT, FN, RA, RW>;
+  static bool raised = false;
+  if (!raised) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS) != hipSuccess) return AS_LAUNCH_FAILED;
+    raised = true;
+  }
+  kernel<<<(strips * max_tiles + 7) / 8 * 8, 512, T::LDS, stream>>>((const bf16*)a, a_div, (const bf16*)w, N, K, order, tiles, counts, (OutT*)out,
+                                                                    limit, strips);
+  return launch_status();
 }
 
 // fp32: plain multiply-add, every output one chain over k in order.  A thread owns an output and, of every
@@ -641,12 +715,12 @@ __global__ __launch_bounds__(256) void moe_gemm_f32_kernel(const float* __restri
 // are still to be added up); the fp32 product writes fp32.
 // gated: 0: the product; 1: act(gate) * up (limit 0: silu(gate) * up; > 0: the gated activation with limits);
 // 2: relu(product)^2 (an expert without a gate).
-// size: of the route's tiles, 64 or 128.
+// size: of the route's tiles, 64 or 128.  across: weight rows that a tile of 128 pairs is multiplied with in a workgroup, 256 or 128.
 extern "C" int as_moe_gemm(const void* a, int dtype, int a_div, const void* w, int N, int K, int gated, const int* order,
                            const int* tiles, const int* counts, int max_tiles, void* out, int out_dtype, float limit,
-                           int size, hipStream_t stream) {
+                           int size, int across, hipStream_t stream) {
   if (max_tiles <= 0) return AS_OK;
-  if (N <= 0 || K <= 0 || a_div <= 0 || max_tiles > 65535 || (size != MOE_HALF && size != MOE_TILE)) return AS_BAD_SHAPE;
+  if (N <= 0 || K <= 0 || a_div <= 0 || max_tiles > 65535 || (size != MOE_HALF && size != MOE_TILE) || (across != 128 && across != 256)) return AS_BAD_SHAPE;
   dim3 grid((N + MOE_STRIP - 1) / MOE_STRIP, max_tiles);
   if (dtype == DT_F32) {
     if (out_dtype != DT_F32) return AS_BAD_DTYPE;
@@ -659,24 +733,27 @@ extern "C" int as_moe_gemm(const void* a, int dtype, int a_div, const void* w, i
   const unsigned long long expert_bytes = (unsigned long long)(gated == 1 ? 2 : 1) * N * K * 2ull;  // 32-bit offsets within an expert
   if (K % 128 == 0 && N % 16 == 0 && (((uintptr_t)a | (uintptr_t)w | (uintptr_t)out) & 15) == 0 && expert_bytes <= 0xf0000000ull &&
       (gated ? out_dtype == DT_BF16 : out_dtype == DT_BF16 || out_dtype == DT_F32)) {
-    const bool wide = size == MOE_TILE;
-    const int across = (gated == 1 ? 64 : wide ? 128 : 64) * (wide ? 2 : 1), strips = (N + across - 1) / across;
-    if (wide && (long long)strips * max_tiles > 0x3ffffff8ll) return AS_BAD_SHAPE;
-#define STREAM(MODE, T)                                                                                                      \
-  do {                                                                                                                       \
-    if (wide)                                                                                                                \
-      moe_gemm_stream_kernel<MODE, T, true><<<(strips * max_tiles + 7) / 8 * 8, 512, 0, stream>>>(                           \
-          (const bf16*)a, a_div, (const bf16*)w, N, K, order, tiles, counts, (T*)out, limit, strips);                        \
-    else                                                                                                                     \
-      moe_gemm_stream_kernel<MODE, T, false><<<dim3(strips, max_tiles), 256, 0, stream>>>(                                      \
-          (const bf16*)a, a_div, (const bf16*)w, N, K, order, tiles, counts, (T*)out, limit, strips);                        \
-  } while (0)
-    if (gated == 1) STREAM(MOE_GATED, bf16);
-    else if (gated) STREAM(MOE_RELU2, bf16);
-    else if (out_dtype == DT_BF16) STREAM(MOE_PLAIN, bf16);
-    else STREAM(MOE_PLAIN, float);
+    if (size == MOE_TILE && (unsigned long long)max_tiles * MOE_TILE * K * 2 <= 0xf0000000ull) {  // 32-bit offsets among the pairs' rows, too
+#define TILED(MODE, T)                                                                                                                       \
+  return across == 256 ? launch_moe_tile<MODE, T, 4, 3, 3>(a, a_div, w, N, K, order, tiles, counts, max_tiles, out, limit, stream)            \
+                       : launch_moe_tile<MODE, T, 2, 4, 4>(a, a_div, w, N, K, order, tiles, counts, max_tiles, out, limit, stream)
+      if (gated == 1) TILED(MOE_GATED, bf16);
+      if (gated) TILED(MOE_RELU2, bf16);
+      if (out_dtype == DT_BF16) TILED(MOE_PLAIN, bf16);
+      TILED(MOE_PLAIN, float);
+#undef TILED
+    }
+    if (size == MOE_HALF) {
+      const dim3 half_grid((N + 63) / 64, max_tiles);
+#define STREAM(MODE, T) \
+  moe_gemm_stream_kernel<MODE, T><<<half_grid, 256, 0, stream>>>((const bf16*)a, a_div, (const bf16*)w, N, K, order, tiles, counts, (T*)out, limit)
+      if (gated == 1) STREAM(MOE_GATED, bf16);
+      else if (gated) STREAM(MOE_RELU2, bf16);
+      else if (out_dtype == DT_BF16) STREAM(MOE_PLAIN, bf16);
+      else STREAM(MOE_PLAIN, float);
 #undef STREAM
-    return launch_status();
+      return launch_status();
+    }
   }
   grid.z = size / MOE_HALF;
   if (gated == 2) {

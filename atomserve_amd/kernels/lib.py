@@ -51,7 +51,7 @@ SIGNATURES = {
     "as_rglru_gates": ("recurrent", [P, I, I, P, P, P, P, P, I, F, P, P, I, P]),
     "as_rglru_scan": ("recurrent", [P, P, I, P, I, I, I, P, I, F, P, P, P, P, P, I, P, I, I, I, I, I, I, P]),
     "as_moe_route_table": ("moe", [P, P, I, I, I, I, P, P, P, I, I, I, P]),
-    "as_moe_gemm": ("moe", [P, I, I, P, I, I, I, P, P, P, I, P, I, F, I, P]),
+    "as_moe_gemm": ("moe", [P, I, I, P, I, I, I, P, P, P, I, P, I, F, I, I, P]),
     "as_moe_combine": ("moe", [P, I, F, I, P, I, I, P, P, P, P, I, P]),
     "as_moe_route_scores": ("moe", [P, P, P, I, P, I, I, F, I, I, I, I, I, P, P, P]),
     "as_group_norm": ("layer_ops", [P, P, P, P, F, I, P, I, I, I, I, P]),

@@ -2114,7 +2114,7 @@ MOE_TILES = (64, 128)  # pairs of one expert that a tile of the grouped products
 MOE_MAX_EXPERTS = 1024
 
 
-# Pairs an expert from which on tiles of 128 are the faster ones, and the values of all experts' first matrices (gate and up,
+# Pairs an expert from which on tiles of 128 are taken, and the values of all experts' first matrices (gate and up,
 # both in bf16) that the first of the two lines needs (`moe_tile`).
 MOE_MANY, MOE_MANY_SMALL, MOE_LARGE_WEIGHTS = 56, 128, 60 << 20
 
@@ -2129,25 +2129,33 @@ def _moe_streamed(w, gated: bool) -> bool:
 
 def moe_tile(pairs: int, first, second, gated: bool) -> int:
     """Pairs a tile of a route whose grouped products read `first` [experts, N_w, K] and then `second`; decides speed alone.
-    Only the kernel that streams weights gains from tiles of 128, which read every weight once where tiles of 64 read it for every 64
-    pairs, and make a quarter of the workgroups: the LDS kernel takes such a tile as two halves, half of whose workgroups then find
+    Tiles of 128 come with operands that go straight into LDS, tiles of 64 with weights straight into registers.  The LDS kernel of other
+    sizes takes a tile of 128 as two halves, half of whose workgroups then find
     nothing (32 experts of 2,880 at width 2,880, four a token, 1,500 tokens: 892 us in tiles of 64, 973 of 128), and the 32-bit kernel walks
     it in one workgroup (16 experts of 768 at width 1,024, 1,000 tokens of two: 3,944 and 5,852).  Both products of a layer, us in tiles of
-    64 / of 128, by pairs an expert (16 experts, two a token; gate and up, their values in millions):
-                          38        62        75        100       125       162
-    width 1,024,  25 M    27/41     41/44     40/46     41/53     45/53     55/50
-    2,048,        50 M    44/59     51/66     70/67     77/76     79/77     99/74
-    1,024 of 1,536, 50 M  44/57     53/60     64/64     66/72     81/93     86/84
-    2,048,        67 M    51/65     72/70     76/74     78/82     101/83    120/77
-    2,048,       101 M    79/79     97/89     107/96    113/100   134/137   161/127
-    4,096,       101 M    80/100    130/107   136/111   142/122   150/138   187/140
-    4,096,       403 M    257/269   345/289   388/287   405/320   468/392   595/482
-    Up to 64 pairs an expert both read every weight once and small tiles fill more compute units; from 65 to 128 small tiles read it
-    twice, which larger matrices feel; above that three times."""
+    64 / of 128, by pairs an expert (16 experts, two a token where no others are named; gate and up, their values in millions):
+                          16        24        38        62        100       162       256
+    width 1,024,  25 M    26/25     26/25     27/25     37/28     41/32     56/38     73/48
+    1,024 of 1,536, 50 M  37/39     38/35     42/41     51/42     61/47     87/66     112/80
+    2,048,        50 M    36/34     37/35     39/36     47/40     70/48     93/61     123/81
+    2,048,       101 M    65/64     67/58     71/61     95/65     103/75    153/102   204/133
+    4,096,       403 M    217/225   225/229   238/235   341/248   423/303   560/336   791/439
+    2,048, 128 experts, 8 a token, 403 M
+                          227/228   236/235   255/248   332/264   450/321   596/393   840/505
+    (before, weights into registers and pairs through them into LDS: 2,048 and 101 M at 162 pairs 127, 4,096 and 403 M 482).  The lines
+    are where that kernel's lay, 56 pairs and 128 for smaller matrices; they could lie at 32."""
     if not (_moe_streamed(first, gated) and _moe_streamed(second, False)):
         return MOE_TILES[0]
     many = MOE_MANY if first.numel() >= MOE_LARGE_WEIGHTS else MOE_MANY_SMALL
     return MOE_TILES[pairs >= many * first.shape[0]]
+
+
+def moe_across(pairs: int, experts: int, rows: int) -> int:
+    """Weight rows that a workgroup multiplies a tile of 128 pairs with, 256 or, while that leaves half of the compute units idle, 128
+    (a tile more for every second expert than the pairs fill).  One product, us of 256 / of 128, 16 experts, two a token: 1,024 rows
+    of K = 768, 1,000 tokens 19 14.5, 2,048 tokens 20 26; 1,536 of 1,024, 500 tokens 21 16, 1,000 tokens 23 26; 6,144 of 4,096, 1,500 tokens 217 311."""
+    tiles = pairs / MOE_TILES[1] + experts / 2
+    return 128 if 2 * tiles * -(-rows // 256) <= compute_units() else 256
 
 
 class ExpertRoute:
@@ -2254,7 +2262,7 @@ def moe_gemm(a, w, route: ExpertRoute, out, gated: bool, per_token: bool, activa
     call("as_moe_gemm", _ptr(a), _DT[a.dtype], route.top if per_token else 1, _ptr(w), N, K,
          2 if activation else int(bool(gated)),
          _ptr(route.order), _ptr(route.tiles), _ptr(route.counts), route.max_tiles, _ptr(out), _DT[out.dtype], float(limit),
-         route.tile, _stream())  # fmt: skip
+         route.tile, moe_across(pairs, w.shape[0], w.shape[1]), _stream())  # fmt: skip
 
 
 def moe_combine(pair_out, top: int, weight: float, out, pair_weight=None, add=None, same=None, pair_expert=None, experts: int = 0) -> None:

@@ -1638,3 +1638,32 @@ def test_wide_products_are_what_many_rows_take(ops):
     sums = ops.gemm_split_sums(act, down)
     assert sums.shape[0] == ops.wide_split_plan(M, K, N)[1] > 1
     assert torch.equal(sums.sum(0), act.float() @ down.float().t())
+
+
+@pytest.mark.parametrize("across", [128, 256])
+@pytest.mark.parametrize("N,K", [(16, 128), (208, 256), (272, 640)])
+def test_experts_products_in_tiles_of_128_pairs(ops, across, N, K, monkeypatch):
+    """The products of tiles of 128 pairs with either number of weight rows: the bits of the tiles of 64, plain in both widths, gated and
+    squared, for experts of no, one, 64, 65, 128 and 200 pairs, and rows shared by a token's pairs."""
+    torch.manual_seed(N + K)
+    counts = [200, 0, 1, 64, 65, 128]
+    chosen = torch.tensor([e for e, n in enumerate(counts) for _ in range(n)], device=DEV)
+    experts = chosen[torch.randperm(len(chosen), device=DEV)].to(torch.int32).view(-1, 2)  # two a token
+    T = experts.shape[0]
+    ids, P = torch.arange(T, device=DEV, dtype=torch.int32), 2 * T
+    a, each = torch.randn(T, K, device=DEV).to(BF16), torch.randn(P, K, device=DEV).to(BF16)
+    w = (torch.randn(len(counts), 2 * N, K, device=DEV) / math.sqrt(K)).to(BF16)
+    half = w[:, :N].contiguous()
+    monkeypatch.setattr(ops, "moe_across", lambda *sizes: across)
+
+    def results(tile):
+        route = ops.moe_route_table(ids, experts, len(counts), tile=tile)
+        found = []
+        for x, weights, dtype, gated, per_token, activation in ((a, w, BF16, True, True, None), (each, half, F32, False, False, None),
+                                                                (each, half, BF16, False, False, None), (a, half, BF16, False, True, "relu2")):  # fmt: skip
+            found.append(torch.full((P, N), float("nan"), device=DEV, dtype=dtype))
+            ops.moe_gemm(x, weights, route, found[-1], gated, per_token, activation)
+        return found
+
+    for got, want in zip(results(128), results(64)):
+        assert torch.equal(got, want)
