@@ -28,24 +28,28 @@ class CachePools:
         for g in manager.state_groups:
             shape = (len(g.cache_ids), manager.max_num_seqs + 1, *g.request.shape)
             self.state.append(torch.zeros(shape, dtype=g.request.dtype, device=device))
+        # every cache's views of its pool, made once: every layer of every step asks for its own
+        self._views = {}
+        for cache_id, (kind, gi, li) in manager.group_of_cache.items():
+            if kind == "paged":
+                nb, kv, bs, d = self.paged[gi].shape[2:]
+                self._views[cache_id] = gi, self.paged[gi][li, 0], self.paged[gi][li, 1].view(nb, kv, d, bs)
+            elif kind == "state":
+                self._views[cache_id] = gi, self.state[gi][li]
 
     def pages(self, cache_id: int):
         """(group index, k_pages, v_pages) of one cache: k_pages [num_pages, KV, block_size, D];
         v_pages [num_pages, KV, D, block_size], each page of values transposed so that the keys
         of one coordinate are contiguous (what the matrix-core kernels read directly)."""
-        kind, gi, li = self.manager.group_of_cache[cache_id]
-        if kind != "paged":
+        if self.manager.group_of_cache[cache_id][0] != "paged":
             raise KeyError(f"cache {cache_id} is not paged")
-        k = self.paged[gi][li, 0]
-        nb, kv, bs, d = k.shape
-        return gi, k, self.paged[gi][li, 1].view(nb, kv, d, bs)
+        return self._views[cache_id]
 
     def state_of(self, cache_id: int):
         """(group index, state tensor [max_num_seqs + 1, *shape]) of one cache."""
-        kind, gi, li = self.manager.group_of_cache[cache_id]
-        if kind != "state":
+        if self.manager.group_of_cache[cache_id][0] != "state":
             raise KeyError(f"cache {cache_id} holds no fixed-size state")
-        return gi, self.state[gi][li]
+        return self._views[cache_id]
 
     @staticmethod
     def bytes_per_block(requests: dict, block_size: int, dtype: torch.dtype) -> int:

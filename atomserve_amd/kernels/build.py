@@ -22,7 +22,7 @@ FLAGS = ["-O3", "-std=c++17", "-shared", "-fPIC", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]  # fmt: skip
 HEADERS = ["common.h", "float_parts.h", "no_alloc.h", "rows.h", "wide_tile.h"]
 LIBRARIES = ("elementwise", "attention", "attention_mix", "gemm", "gemm_wide", "gemm_f32", "sampling", "blas", "recurrent", "moe", "layer_ops",
-             "linear_attention", "latent", "streams", "sandwich", "state_space")
+             "linear_attention", "latent", "streams", "sandwich", "state_space", "launches")
 LINK = {"blas": ["-lhipblaslt"]}  # what a library links beside the HIP runtime
 
 

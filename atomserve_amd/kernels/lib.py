@@ -7,14 +7,17 @@ library cannot be built or loaded raises.
 """
 
 import ctypes
+import struct
 import threading
-from ctypes import c_double, c_float, c_int, c_longlong, c_size_t, c_void_p
+from ctypes import byref, c_double, c_float, c_int, c_longlong, c_size_t, c_void_p, cast
 
 import torch  # noqa: F401  (loads libamdhip64 first)
 
 from atomserve_amd.kernels import build
 
 P, I, F = c_void_p, c_int, c_float
+_CFuncPtr = ctypes.CDLL(None)._FuncPtr.__base__  # what every C function is that ctypes calls
+_FLOAT, _FLOAT_BITS = struct.Struct("<f"), struct.Struct("<I")
 
 # name -> (library, argument types); every entry point returns an int status.
 SIGNATURES = {
@@ -99,6 +102,7 @@ SIGNATURES = {
     "as_blas_adopt": ("blas", [I, I, I, I, c_size_t, I]),
     "as_blas_prepare_adoption": ("blas", []),
     "as_blas_gemm": ("blas", [P, P, P, I, I, I, I, I, P, c_size_t, P]),
+    "as_launch_list": ("launches", [P, c_longlong, P, I, P]),
     "as_argmax": ("sampling", [P, P, I, I, P]),
     "as_sample": ("sampling", [P, I, I, P, P, P, P, P, P, P]),
     "as_sample_split": ("sampling", [P, I, I, P, P, P, P, P, P, P, P, P]),
@@ -189,12 +193,37 @@ class Launches:
         # sources with the address of one that the calls were given: which of them it was is not known
         self.same = [(i, place[a]) for i, a in enumerate(sources) if a and place[a] in met and place[a] != i]
         self.met = sorted(met.union(i for i, _ in self.same))
+        self.program = self._program() if all(isinstance(fn, _CFuncPtr) for _, fn, _ in self.calls) else None
+
+    def _program(self):
+        """The calls as `csrc/launches.hip` takes them: integers and addresses, 32-bit floats, and where targets go."""
+        words = []
+        for _, fn, args, patches in self.patched:
+            ints, floats, place = [], [], {}
+            for at, (kind, v) in enumerate(zip(fn.argtypes, args, strict=True)):
+                if kind is c_float:
+                    floats.append(_FLOAT_BITS.unpack(_FLOAT.pack(v))[0])
+                else:
+                    place[at] = len(ints)
+                    ints.append(int(v or 0))
+            words += (cast(fn, c_void_p).value, len(ints), len(floats), len(patches), *ints, *floats)
+            for at, i in patches:
+                words += (place[at], i)
+        return (c_longlong * len(words))(*words)
 
     def fits(self, targets: list) -> bool:
         """Whether `targets` (of use: those at the places `met`) can stand for the sources: one address for one address."""
         return all(targets[i] == targets[j] for i, j in self.same)
 
     def again(self, targets: list) -> None:
+        """All calls in one; one by one where an entry point is no C function (something stands in its place)."""
+        if self.program is not None:
+            failed = c_int(-1)
+            status = entry("as_launch_list")(self.program, len(self.program), (c_longlong * len(targets))(*targets), len(targets), byref(failed))
+            if status != 0:
+                name = self.calls[failed.value][0] if failed.value >= 0 else "as_launch_list"
+                raise KernelError(f"{name}: {STATUS.get(status, status)}")
+            return
         for name, fn, args, patches in self.patched:
             for at, i in patches:
                 args[at] = targets[i]

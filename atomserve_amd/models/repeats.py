@@ -153,9 +153,10 @@ class _Own:
             if v is not source:  # what all layers of a step share is itself
                 if v is None or v.dtype is not dtype or v.shape != shape or v.is_contiguous() != contiguous:
                     return None
-                if (v.data_ptr() - address) % 16:  # kernels are chosen by it
+                there = v.data_ptr()
+                if (there - address) & 15:  # kernels are chosen by it
                     return None
-                address = v.data_ptr()
+                address = there
             found[i] = address
         for i, j in self.alike:
             if own[i] is not own[j]:

@@ -228,3 +228,42 @@ def test_a_list_is_made_again_only_for_what_it_fits(gpu):
     finally:
         ops._check = real
     assert listed == alone and few < 0.7 * (len(checked) - few)
+
+
+def test_a_list_of_calls_is_made_again_as_it_was_written_down():
+    """Entry points with few and many integers, floats anywhere among them and none: every argument arrives, the patched ones
+    as the targets say, and a status that is not zero ends the list and names its call."""
+    from ctypes import CFUNCTYPE, c_float, c_int, c_longlong, c_size_t, c_void_p
+
+    from atomserve_amd.kernels.lib import KernelError, Launches
+
+    shapes = [(c_void_p,), (c_float,), (), (c_int, c_float, c_void_p, c_float, c_longlong, c_void_p, c_int, c_int, c_size_t, c_float, c_void_p),
+              (c_void_p, c_int) * 15, (c_int,) * 5 + (c_float,) + (c_void_p,) * 20 + (c_float, c_int)]  # fmt: skip
+    seen, status, made, kept = [], [0], Launches(), []
+    made.calls = []
+    for i, kinds in enumerate(shapes):
+        def entry(*got, i=i):
+            seen.append((i, [0 if v is None else v for v in got]))
+            return status[0] if i == 4 else 0
+
+        kept.append(CFUNCTYPE(c_int, *kinds)(entry))
+        args = [0.5 + n if kind is c_float else None if kind is c_void_p and n % 3 == 2 else (1 << 40) + 8 * n if kind is c_void_p else -3 - n
+                if kind is not c_size_t else 7 for n, kind in enumerate(kinds)]  # fmt: skip
+        made.calls.append((f"call {i}", kept[-1], args))
+    sources = [(1 << 40) + 8 * n for n in (0, 4, 6, 6)]
+    made.aim(sources)
+    assert made.met == [0, 1, 2, 3] and made.fits([1, 2, 3, 3]) and not made.fits([1, 2, 3, 4])
+    targets = [11, 22 << 40, 33, 33]
+    made.again(targets)
+    at = dict(zip(sources, targets))
+    assert seen == [(i, [0 if v is None else at.get(v, v) for v in args]) for i, (_, _, args) in enumerate(made.calls)]
+    seen.clear()
+    status[0] = -2
+    with pytest.raises(KernelError, match="call 4"):
+        made.again(targets)
+    assert [i for i, _ in seen] == [0, 1, 2, 3, 4]
+    made.program[1] = 99  # a call of more integers than the list allows
+    seen.clear()
+    with pytest.raises(KernelError, match="as_launch_list"):
+        made.again(targets)
+    assert not seen
