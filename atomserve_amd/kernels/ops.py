@@ -726,7 +726,11 @@ _workspace = {}  # device index -> the library's scratch memory, one for the pro
 # of Qwen3-8B sizes it takes 12.7 / 14.8 / 16.3 us at 32 / 48 / 64 rows against the library's best 14.7 /
 # 17.3 / 17.6; for the 4,096 columns of o the library wins at 32 to 64 rows.  With 32-bit results (the head) the tile
 # product of 65 to 96 rows is such a candidate too (`_wide_tile_strips`).  Such a candidate's number is OWN_CANDIDATE + its strips.
-OWN_CANDIDATE = 1000
+# Above 128 rows the tile of the large products (`_wide_plan`) is one, WIDE_CANDIDATE, where it may win: 4,096 columns of K = 1,024, 512 rows
+# 10.7 us against the library's best 11.8, 1,024 rows 11.4 against 14.4; 4,096 of 4,096, 1,024 rows 36 against 39; 6,144 of 2,560, 2,048 rows
+# 52 against 55; lost by a tenth and more where there are few outputs and a long K.
+OWN_CANDIDATE, WIDE_CANDIDATE = 1000, 2000
+WIDE_PLAIN_MIN_OUTPUTS = 1024
 
 
 def _library_workspace(device):
@@ -753,6 +757,8 @@ def _own_candidates(M, N, K, dtype, w) -> list:
     if dtype == F32 and (w is None or _wave_ptr(w)):
         strips = _wide_tile_strips(M, N, K)
         return [OWN_CANDIDATE + strips] if strips else []
+    if dtype == BF16 and _wide_sizes(M, N, N, K):
+        return [WIDE_CANDIDATE] if N >= WIDE_PLAIN_MIN_OUTPUTS and _wide_plan(M, N, K, WIDE_PLAIN)[0] <= 1.1 * _library_us(M, N, K) else []
     if dtype != BF16 or not _tile_rows(M, K, BF16, TILE_SPLIT_MAX_ROWS) or N % 16:
         return []
     if w is not None and not _wave_ptr(w):
@@ -760,7 +766,19 @@ def _own_candidates(M, N, K, dtype, w) -> list:
     return [OWN_CANDIDATE + 2, OWN_CANDIDATE + 4]
 
 
+def _own_call_possible(a, w, out, candidate) -> bool:
+    """Whether this package's product `candidate` can run on these matrices (it was chosen for their sizes, on others)."""
+    if candidate >= WIDE_CANDIDATE:
+        return _wide_takes(a, w, out.shape[1], out.shape[1]) and out.data_ptr() % 16 == 0
+    return bool(_wave_ptr(w)) and not (out.dtype == F32 and a.data_ptr() % 16)
+
+
 def _library_call(a, w, out, M, N, K, candidate) -> None:
+    if candidate >= WIDE_CANDIDATE:
+        if not _own_call_possible(a, w, out, candidate):
+            raise KernelError("the large tiles were chosen for matrices that start on 16 bytes")
+        call("as_gemm_bf16_wide", _ptr(a), _ptr(_rows(w)), _ptr(out), M, N, K, WIDE_PLAIN, 1, _wide_plan(M, N, K, WIDE_PLAIN)[1], _stream())
+        return
     if candidate >= OWN_CANDIDATE:
         if not _wave_ptr(w) or (out.dtype == F32 and a.data_ptr() % 16):
             raise KernelError("the tile product was chosen for weights with a copy in wave order and rows that start on 16 bytes")
@@ -801,7 +819,7 @@ class ProductChoices:
 
     def chosen(self) -> dict:
         """(rows, columns, width, output dtype) -> the candidate that runs, for every shape settled so far
-        (-1: torch's own call; OWN_CANDIDATE + strips: this package's tile product); enough to reproduce a
+        (-1: torch's own call; OWN_CANDIDATE + strips, WIDE_CANDIDATE: this package's tile products); enough to reproduce a
         run's products."""
         return dict(self.choice)
 
@@ -849,7 +867,7 @@ class ProductChoices:
                 choice = self.choice[key] = _fastest_of(self.trials.pop(key))
         if choice < 0:
             return _torch_gemm(a, w, out)
-        if choice >= OWN_CANDIDATE and (not _wave_ptr(w) or (out.dtype == F32 and a.data_ptr() % 16)):
+        if choice >= OWN_CANDIDATE and not _own_call_possible(a, w, out, choice):
             choice = 0  # chosen on weights that had a copy in wave order, or on aligned rows; these have none, or are not
         _library_call(a, w, out, M, N, K, choice)
 
@@ -1110,10 +1128,13 @@ def _library_us(rows: int, n: int, k: int) -> float:
     return 5.8 + 0.66e-9 * 2 * rows * n * k + 0.11 * n * k * 2e-6 + 1.79e-3 * k
 
 
+def _wide_sizes(rows: int, n: int, rows_of_w: int, k: int) -> bool:
+    return WIDE_MIN_ROWS <= rows <= WIDE_MAX_ROWS and k % WIDE_UNIT == 0 and n % 16 == 0 and max(rows, rows_of_w) * k * 2 <= 0xF0000000
+
+
 def _wide_takes(a, w, n: int, rows_of_w: int) -> bool:
-    M, K = a.shape
-    return (a.dtype == BF16 and WIDE_MIN_ROWS <= M <= WIDE_MAX_ROWS and K % WIDE_UNIT == 0 and n % 16 == 0
-            and max(M, rows_of_w) * K * 2 <= 0xF0000000 and a.data_ptr() % 16 == 0 and _rows(w).data_ptr() % 16 == 0)  # fmt: skip
+    return (a.dtype == BF16 and _wide_sizes(a.shape[0], n, rows_of_w, a.shape[1]) and a.data_ptr() % 16 == 0
+            and _rows(w).data_ptr() % 16 == 0)  # fmt: skip
 
 
 @functools.lru_cache(maxsize=4096)

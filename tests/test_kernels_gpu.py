@@ -1667,3 +1667,26 @@ def test_experts_products_in_tiles_of_128_pairs(ops, across, N, K, monkeypatch):
 
     for got, want in zip(results(128), results(64)):
         assert torch.equal(got, want)
+
+
+def test_the_large_tile_is_a_candidate_of_many_rows(ops):
+    """Above 128 rows trials of plain products time the large tile too, where it may win; chosen, it gives the product, also for a row
+    count that takes a tuned one's choice, and matrices that do not start on 16 bytes fall back to the library's first."""
+    torch.manual_seed(6)
+    M, N, K = 384, 4096, 512
+    a, w = torch.randint(-4, 5, (M, K), device=DEV).to(BF16), torch.randint(-4, 5, (N, K), device=DEV).to(BF16)
+    shifted = torch.empty(M * K + 1, device=DEV, dtype=BF16)[1:].view(M, K).copy_(a)
+    ref = (a.float() @ w.float().t()).to(BF16)
+    assert ops._own_candidates(M, N, K, BF16, w) == [ops.WIDE_CANDIDATE] and ops._own_candidates(M, 528, K, BF16, w) == []
+    choices = ops.ProductChoices()
+    choices.tune_rows(M)
+    out = torch.empty(M, N, device=DEV, dtype=BF16)
+    choices.gemm(a, w, out, M, N, K)
+    assert choices.trials[(M, N, K, BF16)]["ids"][-1] == ops.WIDE_CANDIDATE
+    choices.trials.clear()
+    choices.choice[(M, N, K, BF16)] = ops.WIDE_CANDIDATE
+    for x, rows in ((a, M), (a, 300), (shifted, M)):
+        out = torch.full((rows, N), float("nan"), device=DEV, dtype=BF16)
+        choices.gemm(x[:rows], w, out, rows, N, K)
+        assert torch.equal(out, ref[:rows])
+    assert choices.chosen()[(300, N, K, BF16)] == ops.WIDE_CANDIDATE
