@@ -1017,6 +1017,20 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
           for (int k = tt * (2 * DC) / 4; k < (tt + 1) * (2 * DC) / 4; ++k) copy(k);
         }
       }
+      // The values are asked for before the softmax, under which they arrive, as far as registers hold them
+      // (512 tokens behind 15,872, 32 heads, 16 queries a wave in two pieces: 222 us with all values asked for behind it, 198 now; 32
+      // queries a wave, 480 behind 7,001 in four pieces: 97, 92).
+      u32x4_t vraw[2][DT];
+      auto read_values = [&](int j, u32x4_t (&into)[DT]) {
+        // this lane's eight weights of step j belong to keys 8 grp .. 8 grp + 7: one 16-byte slot
+        const u32x4_t* values = &lds[(2 * rd + j) % PF_STAGES][2 + (grp >> 1)][(grp & 1) * D + col];
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) into[dt] = values[dt * 16];
+      };
+      constexpr int EARLY = DC <= 5 ? 3 - QT : 2 - QT;  // of a round's two halves
+      if constexpr (EARLY >= 1) read_values(0, vraw[0]);
+      if constexpr (EARLY >= 2) read_values(1, vraw[1]);
+      __builtin_amdgcn_sched_barrier(0);
       // Only rounds that touch the causal diagonal, the window's edge or the end of the context
       // need a mask; the others see all 64 keys (uniform over the wave).
       const bool masked = kb + 63 > my_first_q || (SEE >= 1 ? kb < last_lo : window > 0 && kb < my_last - window + 1);
@@ -1067,7 +1081,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
           }
         const float rs = (part[0] + part[1]) + (part[2] + part[3]);
         m[qt] = mn;
-        l[qt] = l[qt] * alpha[qt] + quad_rows_sum(rs);
+        l[qt] = l[qt] * alpha[qt] + rs;  // of this lane's keys; the four lanes of a query meet at the end
         rescale = rescale || alpha[qt] != 1.f;
       }
       // the accumulated output is rescaled only when some query's maximum moved (rare once the
@@ -1078,15 +1092,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt) o[qt][dt] *= alpha[qt];
       }
-      u32x4_t vraw[2][DT];
-      auto read_values = [&](int j, u32x4_t (&into)[DT]) {
-        // this lane's eight weights of step j belong to keys 8 grp .. 8 grp + 7: one 16-byte slot
-        const u32x4_t* values = &lds[(2 * rd + j) % PF_STAGES][2 + (grp >> 1)][(grp & 1) * D + col];
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) into[dt] = values[dt * 16];
-      };
-      read_values(0, vraw[0]);
-      read_values(1, vraw[1]);
+      if constexpr (EARLY < 1) read_values(0, vraw[0]);
+      if constexpr (EARLY < 2) read_values(1, vraw[1]);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -1100,6 +1107,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
     }
   }
 
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) l[qt] = quad_rows_sum(l[qt]);
   if (partial) {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
