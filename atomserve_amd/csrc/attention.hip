@@ -1460,13 +1460,51 @@ extern "C" int as_attn_single_query(const void* q, const void* k_pages, const vo
 // contexts.  16 heads of 128 on 8 kv heads, in a captured step: 4 requests of 600 tokens 12.2 us, of 2,000 tokens 18.4 (45.2 and 54.4
 // on the general kernel, which reads each value of a transposed page alone); a prompt of 333 tokens 24 (147: a workgroup to
 // every token read all keys before it).
+//
+// FRESH (decode steps whose tokens are their own rows): the kernel takes the projection's output qkv [T, H + 2 KV, D] and does what
+// qk_norm_rope_store does: every workgroup norms and rotates its group's queries in registers (coordinate i's partner i + D/2 lies in
+// the same lane), and the one whose partition holds the token's own position makes the key and value, stores them and takes them
+// from registers where its pages' loads would have found them.  Same arithmetic; the squares are summed in another order.  All that the
+// new key and the queries are made of is asked for before the first keys and values (behind them it waited for those).  In a captured step of 4
+// requests of 500 to 700 tokens, 16 heads of 128 on 8 kv heads: 4.9 us for the kernel before this one and 9.6 for this, 12.1 now.
+struct FreshF32 {
+  const float* qkv;
+  const float* qw;   // gains of the per-head norms, D values each
+  const float* kw;
+  const float2* cs;  // [T, D/2] cos, sin of the whole head's rotation
+  const int* slots;  // [T] page * block_size + offset of the new token, -1: keep it out of the pages
+  float* k_store;    // the pages again, to write through
+  float* v_store;
+  float eps;
+  int store;         // 0: queries only, the pages already hold the token's key and value
+};
+
+// One head's values as attn_f32 has them, normed and rotated: piece i holds coordinates (i / 2) 32 + 8 lg + (i % 2) 4 .. + 3.
 template <int DT>
+__device__ __forceinline__ void norm_rotate_f32(f32x4_t (&v)[DT], const f32x4_t (&gain)[DT], const float4 (&turn)[DT], float eps) {
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < DT; ++i) ss += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
+  const float inv = 1.0f / sqrtf(quad_rows_sum(ss) / (float)(16 * DT) + eps);
+#pragma unroll
+  for (int i = 0; i < DT / 2; ++i)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const float a = v[i][x] * inv * gain[i][x], b = v[i + DT / 2][x] * inv * gain[i + DT / 2][x];
+      const float4 t = turn[2 * i + (x >> 1)];  // two coordinates' cosine and sine
+      const float c = x & 1 ? t.z : t.x, s = x & 1 ? t.w : t.y;
+      v[i][x] = a * c - b * s;
+      v[i + DT / 2][x] = b * c + a * s;
+    }
+}
+
+template <int DT, bool FRESH = false>
 __global__ __launch_bounds__(256) void attn_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
     const int* __restrict__ tiles, const int* __restrict__ items, const int* __restrict__ positions,
     const int* __restrict__ tok_row, const int* __restrict__ block_tables, int table_width, float* __restrict__ out,
     float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int bs,
-    float scale, Sight sight, int subs, int part_size, int P, int N) {
+    float scale, Sight sight, int subs, int part_size, int P, int N, FreshF32 fresh) {
   constexpr int D = 16 * DT, LD = D + 4;
   extern __shared__ float smem[];  // [4][16] m, [4][16] l, [4][16][LD] outputs
   const int G = H / KV;
@@ -1510,10 +1548,12 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   const int* table = block_tables + (size_t)row * table_width;
 
   f32x4_t qf[DT], kf[DT], vf[DT], o[DT];
-  const float* qrow = q + ((size_t)(t0 + (valid ? tok : 0)) * H + (valid ? head : kvh * G)) * D;
+  auto piece_of = [&](int i) { return (i >> 1) * 32 + lg * 8 + (i & 1) * 4; };
+  const float* qrow = FRESH ? fresh.qkv + ((size_t)t0 * (H + 2 * KV) + (valid ? head : kvh * G)) * D
+                            : q + ((size_t)(t0 + (valid ? tok : 0)) * H + (valid ? head : kvh * G)) * D;
 #pragma unroll
   for (int i = 0; i < DT; ++i) {
-    qf[i] = *reinterpret_cast<const f32x4_t*>(qrow + (i >> 1) * 32 + lg * 8 + (i & 1) * 4) * scale;
+    qf[i] = *reinterpret_cast<const f32x4_t*>(qrow + piece_of(i));
     o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   auto page_of = [&](int step) {  // the 16 keys' place: page and offset, as an offset into one head's pages
@@ -1532,11 +1572,79 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   };
   float m = NEG_INF, l = 0.f;
   size_t base = page_of(wave), next = page_of(wave + 4);
+  // FRESH: the new token's key and value, in this partition at key `mine` of step `own_step`, which is one of this wave's, or nowhere.
+  // All that they and the queries are made of is asked for before the keys and values: loads come back in their order.
+  [[maybe_unused]] f32x4_t new_key[FRESH ? DT : 1], q_gain[FRESH ? DT : 1], k_gain[FRESH ? DT : 1];
+  [[maybe_unused]] float new_value[FRESH ? DT : 1];
+  [[maybe_unused]] float4 turn[FRESH ? DT : 1];
+  [[maybe_unused]] int own_step = -1;
+  [[maybe_unused]] const int mine = (pos0 - k0) & 15;
+  if constexpr (FRESH) {
+    if (fresh.store && pos0 < k1 && ((pos0 - k0) >> 4) % 4 == wave) own_step = (pos0 - k0) >> 4;  // k0 <= pos0 where the partition is not empty
+    const float4* angles = reinterpret_cast<const float4*>(fresh.cs + (size_t)t0 * (D / 2));  // two coordinates each
+#pragma unroll
+    for (int i = 0; i < DT; ++i) q_gain[i] = *reinterpret_cast<const f32x4_t*>(fresh.qw + piece_of(i));
+#pragma unroll
+    for (int i = 0; i < DT / 2; ++i) {
+      turn[2 * i] = angles[piece_of(i) / 2];
+      turn[2 * i + 1] = angles[piece_of(i) / 2 + 1];
+    }
+    if (own_step >= 0) {
+      const float* krow = fresh.qkv + ((size_t)t0 * (H + 2 * KV) + H + kvh) * D;
+      const float* vrow = krow + (size_t)KV * D;
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        new_key[i] = *reinterpret_cast<const f32x4_t*>(krow + piece_of(i));
+        k_gain[i] = *reinterpret_cast<const f32x4_t*>(fresh.kw + piece_of(i));
+        new_value[i] = vrow[i * 16 + lr];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if (wave < steps) {
     load_keys(base, wave);
     load_values(base, wave);
   }
+  if constexpr (FRESH) {
+    __builtin_amdgcn_sched_barrier(0);
+    norm_rotate_f32(qf, q_gain, turn, fresh.eps);
+    if (own_step >= 0) {
+      norm_rotate_f32(new_key, k_gain, turn, fresh.eps);
+#pragma unroll
+      for (int i = 0; i < DT; ++i) {
+        new_value[i] = finite_or_zero(new_value[i]);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) new_key[i][x] = finite_or_zero(new_key[i][x]);
+      }
+      const int slot = fresh.slots[t0];
+      if (slot >= 0) {
+        const size_t head_at = ((size_t)(slot / bs) * KV + kvh) * bs * D;
+        if (lr == 0) {
+#pragma unroll
+          for (int i = 0; i < DT; ++i) *reinterpret_cast<f32x4_t*>(fresh.k_store + head_at + (size_t)(slot % bs) * D + piece_of(i)) = new_key[i];
+        }
+        if (lg == 0) {
+#pragma unroll
+          for (int i = 0; i < DT; ++i) fresh.v_store[head_at + (size_t)(i * 16 + lr) * bs + slot % bs] = new_value[i];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < DT; ++i) qf[i] = qf[i] * scale;
   for (int step = wave; step < steps; step += 4) {
+    if constexpr (FRESH) {
+      if (step == own_step) {
+#pragma unroll
+        for (int i = 0; i < DT; ++i) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            kf[i][x] = lr == mine ? new_key[i][x] : kf[i][x];
+            vf[i][x] = lg * 4 + x == mine ? new_value[i] : vf[i][x];
+          }
+        }
+      }
+    }
     f32x4_t s0 = f32x4_t{0.f, 0.f, 0.f, 0.f}, s1 = s0;
 #pragma unroll
     for (int i = 0; i < DT; i += 2)
@@ -1616,7 +1724,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
 
 // Which shapes it takes: heads of 64 or 128, at most 16 query heads to a kv head, pages of whole steps of 16 keys, no
 // kept first keys (a second stretch of keys; the general kernel walks them).
-extern "C" int as_attn_f32(const float* q, const float* k_pages, const float* v_pages, const int* tiles, int num_tiles,
+static int launch_attn_f32(const FreshF32* fresh, const float* q, const float* k_pages, const float* v_pages, const int* tiles, int num_tiles,
                            int most, const int* items, int num_items, const int* positions, const int* tok_row,
                            const int* block_tables, int table_width, float* out, float* part_m, float* part_l,
                            float* part_acc, int H, int KV, int D, int bs, float scale, int window, int keep, int chunk,
@@ -1632,18 +1740,45 @@ extern "C" int as_attn_f32(const float* q, const float* k_pages, const float* v_
   if ((long)blocks_of * subs > 0x7fffffffL) return AS_BAD_SHAPE;
   const dim3 grid(blocks_of * subs, KV, P);
   const size_t lds = (128 + 4 * 16 * (D + 4)) * sizeof(float);
-  if (D == 64)
-    attn_f32_kernel<4><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width,
-                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P, blocks_of * subs);
-  else
-    attn_f32_kernel<8><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width,
-                                                   out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P, blocks_of * subs);
+  const FreshF32 none = {};
+#define GO(DTV, FRESHV)                                                                                                                  \
+  attn_f32_kernel<DTV, FRESHV><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width, \
+                                                           out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P,     \
+                                                           blocks_of * subs, FRESHV ? *fresh : none)
+  if (fresh) {
+    if (D == 64) GO(4, true);
+    else GO(8, true);
+  } else if (D == 64) GO(4, false);
+  else GO(8, false);
+#undef GO
   if (P > 1) {
     const int rc = launch_status();
     if (rc != AS_OK) return rc;
     attn_reduce_kernel<float><<<dim3(num_items, H), D, 0, stream>>>(items, part_m, part_l, part_acc, out, H, D, P, sight.sink, sight.sinks, 0);
   }
   return launch_status();
+}
+
+extern "C" int as_attn_f32(const float* q, const float* k_pages, const float* v_pages, const int* tiles, int num_tiles,
+                           int most, const int* items, int num_items, const int* positions, const int* tok_row,
+                           const int* block_tables, int table_width, float* out, float* part_m, float* part_l,
+                           float* part_acc, int H, int KV, int D, int bs, float scale, int window, int keep, int chunk,
+                           float cap, int sink, const float* sinks, int wide, int part_size, int P, hipStream_t stream) {
+  return launch_attn_f32(nullptr, q, k_pages, v_pages, tiles, num_tiles, most, items, num_items, positions, tok_row, block_tables, table_width, out,
+                         part_m, part_l, part_acc, H, KV, D, bs, scale, window, keep, chunk, cap, sink, sinks, wide, part_size, P, stream);
+}
+
+// The same for a decode step from the projection's output (see FreshF32): q is qkv [T, H + 2 KV, D]; token t is row t.  items
+// [num_items] or null (all in order); slots may be null where store_kv is 0.
+extern "C" int as_attn_f32_fresh(const float* qkv, const float* qw, const float* kw, const float* cs, const int* slots, float eps, int store_kv,
+                                 float* k_pages, float* v_pages, const int* items, int num_items, const int* positions, const int* block_tables,
+                                 int table_width, float* out, float* part_m, float* part_l, float* part_acc, int H, int KV, int D, int bs,
+                                 float scale, int window, int part_size, int P, hipStream_t stream) {
+  if (num_items <= 0) return AS_OK;
+  if (!qkv || !qw || !kw || !cs || (store_kv && !slots) || (((uintptr_t)qkv | (uintptr_t)qw | (uintptr_t)kw | (uintptr_t)cs) & 15)) return AS_BAD_SHAPE;
+  const FreshF32 fresh{qkv, qw, kw, (const float2*)cs, slots, k_pages, v_pages, eps, store_kv};
+  return launch_attn_f32(&fresh, nullptr, k_pages, v_pages, nullptr, 0, 0, items, num_items, positions, nullptr, block_tables, table_width, out,
+                         part_m, part_l, part_acc, H, KV, D, bs, scale, window, 0, 0, 0.f, 0, nullptr, 0, part_size, P, stream);
 }
 
 // ---- the same without scratch buffers from the caller ----------------------------------

@@ -504,6 +504,56 @@ def attn_decode_fresh(qkv, q_weight, k_weight, cos_sin, slots, eps, store_kv, k_
          _ptr(part_acc), H, KV, D, bs, float(scale), int(window), part_size, P, _stream())  # fmt: skip
 
 
+def attn_f32_fresh_supported(dtype, num_heads: int, num_kv_heads: int, head_dim: int, block_size: int, rotary_dim: int, qk_norm: bool) -> bool:
+    """Whether `attn_f32_fresh` takes this case: the 32-bit heads that `attn_f32_supported` names, with a per-head norm and rotated whole."""
+    return attn_f32_supported(dtype, num_heads, num_kv_heads, head_dim, block_size) and rotary_dim == head_dim and qk_norm
+
+
+def attn_f32_fresh_preferred(rows: int, H: int, KV: int, D: int, max_context: int, window: int) -> bool:
+    """Whether a decode step of these sizes is faster through `attn_f32_fresh` than through the two kernels: while its workgroups are one
+    round of the compute units, for the wider kernel leaves room for one to each.  16 heads of 128 on 8 kv heads, us of one / of two: 8
+    requests of 64 tokens 8.9 9.8, 4 of 200 14.3 14.8, 4 of 600 15.4 15.8, 1 of 2,000 17.9 18.5; 8 of 2,000 in 8 parts 36.4 34.8."""
+    return rows * KV * _partitions(rows, H, KV, D, max_context, window, True, None, "meta")[1] <= compute_units()
+
+
+def attn_f32_fresh(qkv, q_weight, k_weight, cos_sin, slots, eps, store_kv, k_pages, v_pages, positions, block_tables, out, num_heads,
+                   scale, window, max_context, part_size=None, order=None) -> None:  # fmt: skip
+    """`attn_decode_fresh` for 32-bit heads, gains, pages and results: what `qk_norm_rope_store` and then `attn_single_query` do."""
+    _check(qkv, "qkv", F32, (None, None, None))
+    T, heads, D = qkv.shape
+    H = num_heads
+    _check(k_pages, "k_pages", F32, (None, None, None, D))
+    _, KV, bs, _ = k_pages.shape
+    if heads != H + 2 * KV:
+        raise KernelError(f"qkv has {heads} heads, expected {H} + 2 x {KV}")
+    _check(v_pages, "v_pages", F32, (k_pages.shape[0], KV, D, bs))
+    _check(out, "out", F32, (T, H, D))
+    _check(positions, "positions", I32, (T,))
+    _check(block_tables, "block_tables", I32, (None, None))
+    if block_tables.shape[0] < T:
+        raise KernelError(f"attention: {T} tokens that are their own rows need as many block tables")
+    R = 2 * cos_sin.shape[1] if cos_sin is not None else 0
+    if not attn_f32_fresh_supported(F32, H, KV, D, bs, R, q_weight is not None and k_weight is not None):
+        raise KernelError(f"attention from fresh projections: unsupported heads {H}/{KV}, head width {D}, "
+                          f"rotary width {R}, page size {bs}, or no per-head norm")  # fmt: skip
+    _check(cos_sin, "cos_sin", F32, (T, D // 2, 2))
+    _check(q_weight, "q_weight", F32, (D,))
+    _check(k_weight, "k_weight", F32, (D,))
+    if store_kv:
+        _check(slots, "slots", I32, (T,))
+    if order is not None:
+        _check(order, "order", I32, (T,))
+    if T == 0:
+        return
+    if max_context > block_tables.shape[1] * bs:
+        raise KernelError("attention: block tables are shorter than the longest context")
+    part_size, P, part_m, part_l, part_acc = _partitions(T, H, KV, D, max_context, window, True, part_size, qkv.device)
+    call("as_attn_f32_fresh", _ptr(qkv), _ptr(q_weight), _ptr(k_weight), _ptr(cos_sin), _ptr(slots) if store_kv else 0, float(eps),
+         int(bool(store_kv)), _ptr(k_pages), _ptr(v_pages), _ptr(order) if order is not None else 0, T, _ptr(positions),
+         _ptr(block_tables), block_tables.shape[1], _ptr(out), _ptr(part_m), _ptr(part_l), _ptr(part_acc), H, KV, D, bs, float(scale),
+         int(window), part_size, P, _stream())  # fmt: skip
+
+
 PREFILL_TILE_QUERIES = 64  # queries of one work item of the prefill kernel
 PREFILL_MAX_HEAD_DIM = 256  # four stages of 32 keys and values of such heads fill 128 KB of LDS
 

@@ -106,11 +106,16 @@ class Attention(Mixer):
         cos_sin = self.position.prepare(step) if self.position is not None else None
         eps = s.qk_norm.eps if s.qk_norm is not None else 0.0
         rotary = 2 * cos_sin.shape[1] if cos_sin is not None else 0
-        if step.decode_only and ops.attn_decode_fresh_supported(env.dtype, H, KV, D, cache.block_size, rotary,
-                                                                s.qk_norm is not None):  # fmt: skip
-            # a decode step: norm, rotation, the cache store and attention in one kernel
+        case = env.dtype, H, KV, D, cache.block_size, rotary, s.qk_norm is not None
+        fresh = None  # a decode step: norm, rotation, the cache store and attention in one kernel
+        if step.decode_only and ops.attn_decode_fresh_supported(*case):
+            fresh = ops.attn_decode_fresh
+        elif (step.decode_only and ops.attn_f32_fresh_supported(*case) and ops.attn_f32_fresh_preferred(T, H, KV, D, step.max_context, s.window)
+              and not (self.q_norm_weight.data_ptr() | self.k_norm_weight.data_ptr()) & 15):  # fmt: skip
+            fresh = ops.attn_f32_fresh
+        if fresh is not None:
             out = torch.empty((T, H, D), dtype=env.dtype, device=device)
-            ops.attn_decode_fresh(
+            fresh(
                 qkv.view(T, H + 2 * KV, D), self.q_norm_weight, self.k_norm_weight, cos_sin, cache.slots, eps,
                 cache.writes, cache.k_pages, cache.v_pages, step.positions, cache.block_tables, out, H, s.scale,
                 s.window, step.max_context, order=step.all_tokens,

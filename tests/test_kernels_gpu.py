@@ -986,6 +986,46 @@ def test_decode_step_from_fresh_projections(ops, H, KV, D, bs, gain, window, par
                                   scale, window, max(lens), part)  # fmt: skip
 
 
+@pytest.mark.parametrize("H,KV,D,bs,window", [(16, 8, 128, 16, 0), (6, 2, 64, 32, 0), (16, 1, 128, 48, 0), (8, 2, 128, 16, 40), (8, 8, 64, 16, 1)])
+@pytest.mark.parametrize("part", [None, 32, 128])
+def test_decode_step_from_fresh_projections_fp32(ops, H, KV, D, bs, window, part):
+    """The same in 32 bits, against the two kernels (sums of squares and of up to 1,000 weighted values in other orders: 2^-24 times
+    their number's root, on results of up to some units); a token that is not a number is stored as zeros and attended as such."""
+    lens = [1, 16, 17, 32, 33, 128, 129, 300, 512, 513, 1000]
+    _, k_pages, v_pages, tables, positions = paged_case(F32, H, KV, D, bs, lens, seed=5, k_scale=3.0 / math.sqrt(D / 16))
+    T, close = len(lens), dict(atol=3e-5, rtol=3e-5)
+    g = torch.Generator().manual_seed(9)
+    qkv = (torch.randn(T, H + 2 * KV, D, generator=g) * 2).to(DEV)
+    qkv[5, H:] = float("nan")
+    qw, kw = (torch.randn(D, generator=g) + 1).to(DEV), (torch.randn(D, generator=g) + 1).to(DEV)
+    cs = torch.empty(T, D // 2, 2, device=DEV)
+    ops.rope_table(positions, (1.0 / (1e4 ** (torch.arange(0, D, 2, dtype=torch.float64) / D))).to(DEV), cs)
+    slot_list = [tables[i, (n - 1) // bs].item() * bs + (n - 1) % bs for i, n in enumerate(lens)]
+    for i, slot in enumerate(slot_list):  # whatever lies where the new token goes
+        k_pages[slot // bs, :, slot % bs], v_pages[slot // bs, :, :, slot % bs] = float("nan"), float("inf")
+    slots, scale = i32([-1 if i == 3 else slot for i, slot in enumerate(slot_list)]), D**-0.5  # row 3 stays out of the pages
+    k2, v2, q2, out2 = k_pages.clone(), v_pages.clone(), torch.empty(T, H, D, device=DEV), torch.zeros(T, H, D, device=DEV)
+    ops.qk_norm_rope_store(qkv, qw, kw, cs, i32(slot_list), q2, k2, v2, H, KV, 1e-6)
+    ops.attn_single_query(q2, k2, v2, None, positions, None, tables, out2, scale, window, max(lens), part)
+    assert not torch.isnan(out2).any()
+    for order in (None, torch.randperm(T, generator=g).to(torch.int32).to(DEV)):
+        k1, v1, out1 = k_pages.clone(), v_pages.clone(), torch.full((T, H, D), float("nan"), device=DEV)
+        ops.attn_f32_fresh(qkv, qw, kw, cs, slots, 1e-6, True, k1, v1, positions, tables, out1, H, scale, window, max(lens), part, order)
+        assert torch.allclose(out1, out2, **close)
+        kept = torch.ones(k_pages.shape[0] * bs, dtype=torch.bool, device=DEV)
+        kept[slot_list[3]] = False
+        kept = kept.view(-1, bs)
+        assert torch.allclose(k1.permute(0, 2, 1, 3)[kept], k2.permute(0, 2, 1, 3)[kept], **close)
+        assert torch.equal(v1.permute(0, 3, 1, 2)[kept], v2.permute(0, 3, 1, 2)[kept])
+        assert torch.isnan(k1.permute(0, 2, 1, 3)[~kept]).all() and torch.isinf(v1.permute(0, 3, 1, 2)[~kept]).all()
+    out3, k3, v3 = torch.zeros(T, H, D, device=DEV), k2.clone(), v2.clone()  # queries only
+    ops.attn_f32_fresh(qkv, qw, kw, cs, None, 1e-6, False, k3, v3, positions, tables, out3, H, scale, window, max(lens), part)
+    assert torch.allclose(out3, out2, **close) and torch.equal(k3, k2) and torch.equal(v3, v2)
+    for weights, angles in ((None, cs), (qw, None), (qw, cs[:, : D // 4].contiguous())):
+        with pytest.raises(ops.KernelError, match="fresh projections"):
+            ops.attn_f32_fresh(qkv, weights, weights, angles, slots, 1e-6, True, k3, v3, positions, tables, out3, H, scale, window, max(lens), part)
+
+
 def test_attention_of_a_batch_that_fills_the_gpu(ops):
     """64 requests of 8 kv heads are 512 workgroups already: the contexts are not partitioned (no
     merge), each workgroup walks its whole context, of very different lengths."""
