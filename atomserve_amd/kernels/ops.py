@@ -856,6 +856,7 @@ class ProductChoices:
     def __init__(self, fixed: bool = False):
         self.fixed = bool(fixed)
         self.choice = {}  # (rows, columns, width, output dtype) -> candidate
+        self.library = {}  # the same key -> the library's fastest candidate of the trial, where a product of this package won it
         self.trials = {}  # the same key -> a trial under way
         self.tuned_rows = {32, 48, 64}
 
@@ -914,17 +915,37 @@ class ProductChoices:
                         trial["weights"].append(w)
                     _trial_run(trial, a, w, out, M, N, K)
                     return
-                choice = self.choice[key] = _fastest_of(self.trials.pop(key))
+                choice = self._end_trial(key, self.trials.pop(key))
         if choice < 0:
             return _torch_gemm(a, w, out)
         if choice >= OWN_CANDIDATE and not _own_call_possible(a, w, out, choice):
-            choice = 0  # chosen on weights that had a copy in wave order, or on aligned rows; these have none, or are not
+            # chosen on weights that had a copy in wave order, or on aligned rows; these have none, or are not
+            choice = self._library_choice(key)
         _library_call(a, w, out, M, N, K, choice)
 
-    def _choice_of_tuned_rows(self, M, N, K, dtype):
+    def _end_trial(self, key, trial) -> int:
+        choice = self.choice[key] = _fastest_of(trial)
+        if choice >= OWN_CANDIDATE:
+            self.library[key] = _fastest_of(trial, OWN_CANDIDATE)
+        return choice
+
+    def _library_choice(self, key) -> int:
+        """The library's candidate for a settled shape on whose matrices this package's product, which was chosen, cannot run: the
+        fastest of the shape's own trial, or of the row count's that this one follows; its first where no trial said."""
+        place = self.library.get(key)
+        if place is None and not self.fixed and key[0] not in self.tuned_rows:
+            place = self._choice_of_tuned_rows(*key, own=False)
+            if place is not None:
+                self.library[key] = place
+        return place or 0
+
+    def _choice_of_tuned_rows(self, M, N, K, dtype, own: bool = True):
         """For a product of a row count that is not tuned itself: the kernel that the nearest tuned row
         count above it (of more than 64 rows: a prompt's, not a decode step's) settled on for the same
-        weights, as a candidate of this shape; None while that one has not settled, or there is none."""
+        weights, as a candidate of this shape; None while that one has not settled, or there is none.
+        Where that is a product of this package which is no candidate here (or `own` is not asked for): the
+        fastest of the library's there (4,096 columns of K = 4,096, 1,300 rows under 1,536, where the large tile had won: 47.7 us with
+        the library's first, 46.4 with that one)."""
         above = [rows for rows in self.tuned_rows if rows >= M and rows > LIBRARY_DECODE_ROWS]
         if not above:
             return None
@@ -934,8 +955,10 @@ class ProductChoices:
             return None
         if settled < 0:
             return 0
-        if settled >= OWN_CANDIDATE:  # this package's tile kernel: for this row count too if it takes it, else the library's first
-            return settled if settled in _own_candidates(M, N, K, dtype, None) else 0
+        if settled >= OWN_CANDIDATE:  # this package's tile kernel: for this row count too if it takes it
+            if own and settled in _own_candidates(M, N, K, dtype, None):
+                return settled
+            settled = self.library.get((tuned, N, K, dtype), 0)
         index = entry("as_blas_candidate_index")(tuned, N, K, _DT[dtype], LIBRARY_WORKSPACE_BYTES, settled)
         place = entry("as_blas_adopt")(M, N, K, _DT[dtype], LIBRARY_WORKSPACE_BYTES, index)
         return place if place >= 0 else 0
@@ -962,7 +985,7 @@ class ProductChoices:
                     space[: LIBRARY_WORKSPACE_BYTES // 4].zero_()
                 _trial_run(trial, a, trial["weights"][len(trial["runs"]) % len(trial["weights"])], out, *key[:3])
             torch.cuda.current_stream().synchronize()
-            self.choice[key] = _fastest_of(trial)
+            self._end_trial(key, trial)
 
 
 SHARED = ProductChoices()  # for products whose caller names no choices of its own (tools, tests, toy parts)
@@ -988,14 +1011,14 @@ def _trial_run(trial, a, w, out, M, N, K) -> None:
     trial["runs"].append((candidate, start, end))
 
 
-def _fastest_of(trial) -> int:
-    """The candidate whose shortest run took least, among the runs that were timed and have finished: those with the host ahead
+def _fastest_of(trial, below=None) -> int:
+    """The candidate (of a number under `below`, if given) whose shortest run took least, among the runs that were timed and have finished: those with the host ahead
     (`settle`) where every candidate has one, else all but each candidate's first (which loads the kernel); 0 if none.  (The host
     between a run's two events lengthens it; the caches, which could shorten it, do not hold its weights: a pass comes back to
     them after all others.  On averages qkv of 16 rows at Qwen3-4B sizes went to 12.5 us instead of 9.3 in one process of three.)"""
     times, ahead = {}, {}
     for n, (candidate, start, end) in enumerate(trial["runs"]):
-        if start is not None and end.query():
+        if start is not None and (below is None or candidate < below) and end.query():
             times.setdefault(candidate, []).append(start.elapsed_time(end))
             if n >= trial.get("ahead", n + 1):
                 ahead.setdefault(candidate, []).append(times[candidate][-1])

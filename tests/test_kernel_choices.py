@@ -277,3 +277,73 @@ def test_plans_of_wide_products(monkeypatch):
     finally:
         for cached in (ops._wide_plan, ops.wide_split_plan, ops.wide_gated_form):
             cached.cache_clear()
+
+
+class Library:
+    """The library's entry points and what runs, without a GPU: every shape has three candidates, whose kernels have the numbers 10 to 12, and
+    takes a fourth one on; times[candidate] is what a run takes (9 where none is given)."""
+
+    def __init__(self, monkeypatch, times=()):
+        self.ran, self.times, self.adopted = [], dict(times), {}
+        doors = {"as_blas_plan": lambda *shape: 3, "as_blas_candidate_index": lambda M, N, K, dtype, size, place: 10 + place,
+                 "as_blas_adopt": self.adopt, "as_gemm_bf16_wide": None}  # fmt: skip
+        monkeypatch.setattr(ops, "entry", doors.__getitem__)
+        monkeypatch.setattr(ops, "_library_workspace", lambda device: torch.empty(1))
+        monkeypatch.setattr(ops, "_library_call", lambda a, w, out, M, N, K, candidate: self.ran.append((M, candidate)))
+        monkeypatch.setattr(ops, "_trial_run", self.trial_run)
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"synchronize": lambda self: None})())
+
+    def adopt(self, M, N, K, dtype, size, index):
+        self.adopted[M] = index
+        return index - 10
+
+    def trial_run(self, trial, a, w, out, M, N, K):
+        candidate = trial["ids"][len(trial["runs"]) % trial["count"]]
+        self.ran.append((M, candidate))
+        trial["runs"].append((candidate, Mark(), Mark(self.times.get(candidate, 9.0))))
+
+
+class Matrix:
+    """A matrix of bf16 as the dispatch looks at it, starting at a place of its choice."""
+
+    def __init__(self, rows, columns, at=0):
+        self.shape, self.dtype, self.at, self.device, self.is_cuda = (rows, columns), BF16, at, "cuda:0", True
+
+    def data_ptr(self):
+        return self.at
+
+
+def settled(choices, M, N, K, run=None):
+    """Runs the product of M rows until its trial has ended."""
+    choices.tune_rows(M)
+    run = run or (lambda: choices.gemm(Matrix(M, K), Matrix(N, K), Matrix(M, N), M, N, K))
+    run()
+    choices.settle()
+
+
+def test_where_the_large_tile_is_no_candidate_the_trials_best_of_the_library_runs(monkeypatch):
+    """A row count that follows a tuned one on which the large tile won takes the tile where it may win there too, and the library's fastest
+    of that trial elsewhere; so do matrices that the tile does not take.  Not the library's first, which no trial has named."""
+    library = Library(monkeypatch, {0: 8.0, 1: 5.0, 2: 4.0, ops.WIDE_CANDIDATE: 3.0})
+    choices, N, K, tuned = ops.ProductChoices(), 4096, 4096, 1536
+    settled(choices, tuned, N, K)
+    assert choices.chosen() == {(tuned, N, K, BF16): ops.WIDE_CANDIDATE}
+    asked = range(1025, tuned)
+    without = [M for M in asked if not ops._own_candidates(M, N, K, BF16, None)]
+    assert 1100 in without and 1520 not in without
+
+    def runs(M, at=0):
+        library.ran.clear()
+        choices.gemm(Matrix(M, K, at), Matrix(N, K), Matrix(M, N), M, N, K)
+        return library.ran
+
+    for M in (1025, 1100, 1504, 1505, 1520):
+        for _ in range(2):
+            assert runs(M) == [(M, 2 if M in without else ops.WIDE_CANDIDATE)]
+        assert library.adopted.get(M) == (12 if M in without else None)
+    assert runs(1520, at=8) == [(1520, 2)] and library.adopted[1520] == 12 and runs(1520) == [(1520, ops.WIDE_CANDIDATE)]
+    assert runs(tuned, at=8) == [(tuned, 2)] and runs(tuned) == [(tuned, ops.WIDE_CANDIDATE)]
+    door = ops.entry
+    monkeypatch.setattr(ops, "entry", lambda name: (lambda *shape: -1) if name == "as_blas_adopt" else door(name))
+    assert runs(1101) == [(1101, 0)]  # a shape that does not take that kernel on: its own first
