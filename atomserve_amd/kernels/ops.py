@@ -879,6 +879,15 @@ class ProductChoices:
         again, like the token budget of the steps that carry a portion of a prompt."""
         self.tuned_rows.add(int(rows))
 
+    def wants_trial(self, M, N, K) -> bool:
+        """Whether the kernels of this product with bf16 results are still to be tried (or are being tried) by calls like this one.  What a
+        rule gives to a kernel beside the trials (a gated product, sums in parts) waits until they have been, though this row count has no use
+        for them then: the row counts that follow it may fall on the library's side of the rule (5,120 outputs of K = 17,408, 800 rows, whole,
+        under 1,024, cut: 234 us with the library's first kernel, 177 with the one that the trial at 1,024 rows names; 2,560 of 9,728, 900
+        rows: 77 and 68; a prompt of 800 tokens through 6 layers of Qwen3-14B sizes 5.04 and 4.38 ms)."""
+        return (M in self.tuned_rows and not self.fixed and (M, N, K, BF16) not in self.choice
+                and not torch.cuda.is_current_stream_capturing())  # fmt: skip
+
     def trials_pending(self) -> bool:
         """Whether some shape is still trying candidates (a warm-up may then run once more)."""
         return bool(self.trials)
@@ -1258,15 +1267,16 @@ def gemm_f32_split(a, w):
     return sums
 
 
-def gemm_split_sums(a, w):
-    """a @ w^T as partial sums for whoever adds them up, or None where the product is better made whole (or has no such kernel)."""
+def gemm_split_sums(a, w, choices=None):
+    """a @ w^T as partial sums for whoever adds them up, or None where the product is better made whole (or has no such kernel, or
+    `choices` want its kernels tried first)."""
     M, K = a.shape
     N = _rows(w).shape[0]
     if a.dtype == F32:
         return gemm_f32_split(a, w) if gemm_f32_split_preferred(M, N, K) else None
     if _wide_takes(a, w, N, N):
         plan = wide_split_plan(M, N, K)
-        if plan is None:
+        if plan is None or (choices or SHARED).wants_trial(M, N, K):
             return None
         form, splits = plan
         rows = _rows(w)
@@ -1314,7 +1324,7 @@ def gemm_silu_mul(a, w, out, choices=None) -> None:
         call("as_gemm_bf16_tile", _ptr(a), _ptr(rows), _wave_ptr(w), _ptr(out), 0, _DT[BF16], M, inter, K, 1, 0,
              _gated_tile_strips(M, inter), _stream())  # fmt: skip
         return
-    if _wide_takes(a, w, inter, 2 * inter) and out.data_ptr() % 16 == 0:
+    if _wide_takes(a, w, inter, 2 * inter) and out.data_ptr() % 16 == 0 and not (choices or SHARED).wants_trial(M, 2 * inter, K):
         form = wide_gated_form(M, inter, K)
         if form is not None:
             call("as_gemm_bf16_wide", _ptr(a), _ptr(rows), _ptr(out), M, inter, K, WIDE_GATED, 1, form, _stream())

@@ -133,7 +133,7 @@ class Attention(Mixer):
             if link is not None:
                 return link
             if next_norm.takes_split_sums:
-                sums = ops.gemm_split_sums(out.view(T, H * D), self.o)
+                sums = ops.gemm_split_sums(out.view(T, H * D), self.o, env.products)
                 if sums is not None:
                     return SplitSums(sums)
         y = torch.empty((T, s.hidden_size), dtype=env.dtype, device=device)

@@ -53,7 +53,7 @@ class GatedMLP(FeedForward):
             if link is not None:
                 return link
             if next_norm.takes_split_sums:
-                sums = ops.gemm_split_sums(act, self.down)
+                sums = ops.gemm_split_sums(act, self.down, env.products)
                 if sums is not None:
                     return SplitSums(sums)
         y = torch.empty((T, s.hidden_size), dtype=env.dtype, device=device)

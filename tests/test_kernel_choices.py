@@ -347,3 +347,56 @@ def test_where_the_large_tile_is_no_candidate_the_trials_best_of_the_library_run
     door = ops.entry
     monkeypatch.setattr(ops, "entry", lambda name: (lambda *shape: -1) if name == "as_blas_adopt" else door(name))
     assert runs(1101) == [(1101, 0)]  # a shape that does not take that kernel on: its own first
+
+
+def user(monkeypatch, library, choices, N, K, gated=False):
+    """One product of M rows as a layer makes it: down in parts where that pays, else whole; or gate and up with their activation."""
+    for name in ("_check", "silu_mul", "_few_rows", "_tile_rows"):
+        monkeypatch.setattr(ops, name, lambda *args, **kw: None)
+    monkeypatch.setattr(ops, "_ptr", lambda t: 0)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "call", lambda name, *args: library.ran.append((args[3], name)))
+    w = Matrix(N, K)
+
+    def product(M):
+        library.ran.clear()
+        a, out = Matrix(M, K), Matrix(M, N // 2 if gated else N)
+        if gated:
+            a.device = "meta"  # gate and up stand there
+            ops.gemm_silu_mul(a, w, out, choices)
+        else:
+            a.device = "meta"  # the sums stand there
+            if ops.gemm_split_sums(a, w, choices) is None:
+                ops.gemm(a, w, out, choices)
+        return library.ran
+
+    return product
+
+
+PROMPT_LENGTHS = [n for p in range(7, 12) for n in (2**p, 3 * 2 ** (p - 1)) if n <= 2048]  # what a warm-up runs up to 2,048 tokens
+
+
+@pytest.mark.parametrize("N,K,gated,away", [(4096, 12288, False, 575), (5120, 17408, False, 418), (34816, 5120, True, 638), (24576, 4096, True, 162)])
+def test_row_counts_on_the_librarys_side_of_a_rule_find_a_settled_one(monkeypatch, N, K, gated, away):
+    """The rules that give a product of many rows to the large tile say yes and no by row count, the warm-up knows a few counts: those that take the
+    tile try the library's candidates too, for the counts below them that do not."""
+    library = Library(monkeypatch, {0: 8.0, 1: 5.0, 2: 4.0})
+    choices = ops.ProductChoices()
+    product = user(monkeypatch, library, choices, N, K, gated)
+    tile = (lambda M: ops.wide_gated_form(M, N // 2, K)) if gated else (lambda M: ops.wide_split_plan(M, N, K))
+    for M in PROMPT_LENGTHS[1:]:
+        choices.tune_rows(M)
+        product(M)
+        assert choices.trials_pending()
+        choices.settle()
+        assert product(M) == [(M, "as_gemm_bf16_wide" if tile(M) is not None else 2)]
+    fell = 0
+    for M in range(129, 2049):
+        if M not in choices.tuned_rows and tile(M) is None:
+            above = min(m for m in PROMPT_LENGTHS if m >= M)
+            fell += tile(above) is not None
+            assert product(M) == [(M, 2)] and library.adopted[M] == 12
+    assert fell == away
+    fixed = ops.ProductChoices(fixed=True)  # no trials: the rule
+    fixed.tune_rows(1024)
+    assert user(monkeypatch, library, fixed, N, K, gated)(1024) == [(1024, "as_gemm_bf16_wide")] and not fixed.trials_pending()
