@@ -29,10 +29,15 @@ typedef __attribute__((address_space(3))) char lds_char;
 constexpr int UNIT = 64, ROW_BYTES = 2 * UNIT;  // columns of K in a unit
 
 // 64 lanes copy 16 bytes each from buf + lane_at + at to lds + 16 lane.  It has no result in registers; the caller waits for it.  (The
-// builtin of this instruction makes every later read of LDS wait for every copy in flight.)
+// builtin of this instruction makes every later read of LDS wait for every copy in flight.)  m0 is named for the compiler's own users of it: a
+// copy by the builtin beside this one is else given the m0 that this one left (the warning says that nobody keeps m0: that is what is wanted).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void copy_to_lds(__amdgpu_buffer_rsrc_t buf, unsigned lane_at, unsigned at, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(lane_at), "s"(buf), "s"(at), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(lane_at), "s"(buf), "s"(at), "s"(lds)
+               : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 template <int WM, int WN, int FM, int FN, int RA, int RW, bool PAIRED = false>
 struct Tile {
