@@ -18,6 +18,8 @@ from atomserve_amd.kernels import build
 P, I, F = c_void_p, c_int, c_float
 _CFuncPtr = ctypes.CDLL(None)._FuncPtr.__base__  # what every C function is that ctypes calls
 _FLOAT, _FLOAT_BITS = struct.Struct("<f"), struct.Struct("<I")
+_WORDS = (c_void_p, c_int, c_longlong, c_size_t)
+LIST_INTEGERS, LIST_FLOATS = 32, 4  # of a call that `csrc/launches.hip` makes (its MOST and FLOATS)
 
 # name -> (library, argument types); every entry point returns an int status.
 SIGNATURES = {
@@ -194,19 +196,26 @@ class Launches:
         # sources with the address of one that the calls were given: which of them it was is not known
         self.same = [(i, place[a]) for i, a in enumerate(sources) if a and place[a] in met and place[a] != i]
         self.met = sorted(met.union(i for i, _ in self.same))
-        self.program = self._program() if all(isinstance(fn, _CFuncPtr) for _, fn, _ in self.calls) else None
+        self.program = self._program()
 
     def _program(self):
-        """The calls as `csrc/launches.hip` takes them: integers and addresses, 32-bit floats, and where targets go."""
+        """The calls as `csrc/launches.hip` takes them: integers and addresses, 32-bit floats, and where targets go; None where one of
+        them is not of that kind: an entry point that is no C function, more arguments than a call of a list has or arguments of other types."""
         words = []
         for _, fn, args, patches in self.patched:
+            if not isinstance(fn, _CFuncPtr):
+                return None
             ints, floats, place = [], [], {}
             for at, (kind, v) in enumerate(zip(fn.argtypes, args, strict=True)):
-                if kind is c_float:
-                    floats.append(_FLOAT_BITS.unpack(_FLOAT.pack(v))[0])
-                else:
+                if kind is c_float and isinstance(v, (int, float)):
+                    floats.append(_FLOAT_BITS.unpack(_FLOAT.pack(c_float(v).value))[0])
+                elif kind in _WORDS and (v is None or isinstance(v, int)):
                     place[at] = len(ints)
                     ints.append(int(v or 0))
+                else:
+                    return None
+            if len(ints) > LIST_INTEGERS or len(floats) > LIST_FLOATS:
+                return None
             words += (cast(fn, c_void_p).value, len(ints), len(floats), len(patches), *ints, *floats)
             for at, i in patches:
                 words += (place[at], i)
@@ -217,7 +226,7 @@ class Launches:
         return all(targets[i] == targets[j] for i, j in self.same)
 
     def again(self, targets: list) -> None:
-        """All calls in one; one by one where an entry point is no C function (something stands in its place)."""
+        """All calls in one; one by one where a call is none that a list can hold (`_program`)."""
         if self.program is not None:
             failed = c_int(-1)
             status = entry("as_launch_list")(self.program, len(self.program), (c_longlong * len(targets))(*targets), len(targets), byref(failed))

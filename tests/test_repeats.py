@@ -267,3 +267,33 @@ def test_a_list_of_calls_is_made_again_as_it_was_written_down():
     with pytest.raises(KernelError, match="as_launch_list"):
         made.again(targets)
     assert not seen
+
+
+@pytest.mark.parametrize("kinds", [("i",) * 33, ("f",) * 5, ("i", "d", "i"), ("p", "f", "d"), ("i",) * 32 + ("f",) * 4])
+def test_calls_that_no_list_holds_are_made_one_by_one(kinds):
+    """More integers or floats than a call of a list has, or floats of 64 bits: every argument arrives all the same, the patched ones as the
+    targets say, and a status that is not zero names its call.  (The last one is as large as a list's calls come.)"""
+    from ctypes import CFUNCTYPE, c_double, c_float, c_int, c_void_p
+
+    from atomserve_amd.kernels.lib import KernelError, Launches
+
+    types = [{"i": c_int, "f": c_float, "d": c_double, "p": c_void_p}[k] for k in kinds]
+    seen, status, made = [], [0], Launches()
+
+    def entry(*got):
+        seen.append(list(got))
+        return status[0]
+
+    function = CFUNCTYPE(c_int, *types)(entry)
+    args = [0.5 + n if k in "fd" else 1000 + n for n, k in enumerate(kinds)]
+    if "d" in kinds:
+        args[kinds.index("d")] = 1.0 + 2.0**-40
+    made.calls = [("the call", function, args)]
+    sources = [args[n] for n, k in enumerate(kinds) if k in "ip"][-1:]
+    made.aim(sources)
+    made.again([7] * len(sources))
+    assert seen == [[7 if v in sources else v for v in args]]
+    status[0] = -2
+    with pytest.raises(KernelError, match="the call"):
+        made.again([7] * len(sources))
+    assert (made.program is None) == (len(kinds) != 36)
