@@ -1211,7 +1211,8 @@ def _library_us(rows: int, n: int, k: int) -> float:
 
 
 def _wide_sizes(rows: int, n: int, rows_of_w: int, k: int) -> bool:
-    return WIDE_MIN_ROWS <= rows <= WIDE_MAX_ROWS and k % WIDE_UNIT == 0 and n % 16 == 0 and max(rows, rows_of_w) * k * 2 <= 0xF0000000
+    return (WIDE_MIN_ROWS <= rows <= WIDE_MAX_ROWS and k > 0 and k % WIDE_UNIT == 0 and n > 0 and n % 16 == 0
+            and max(rows, rows_of_w) * k * 2 <= 0xF0000000)  # fmt: skip
 
 
 def _wide_takes(a, w, n: int, rows_of_w: int) -> bool:

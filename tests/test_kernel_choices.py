@@ -400,3 +400,10 @@ def test_row_counts_on_the_librarys_side_of_a_rule_find_a_settled_one(monkeypatc
     fixed = ops.ProductChoices(fixed=True)  # no trials: the rule
     fixed.tune_rows(1024)
     assert user(monkeypatch, library, fixed, N, K, gated)(1024) == [(1024, "as_gemm_bf16_wide")] and not fixed.trials_pending()
+
+
+@pytest.mark.parametrize("N,K,gated", [(6144, 0, True), (0, 1024, True), (3072, 0, False), (0, 1024, False)])
+def test_products_without_columns_or_outputs_are_not_the_large_tiles(monkeypatch, N, K, gated):
+    """A sum of nothing is zero and no outputs are none, as torch's product gives them; the large tile refuses both."""
+    library = Library(monkeypatch)
+    assert user(monkeypatch, library, ops.ProductChoices(), N, K, gated)(300) == [(300, 0)]
