@@ -407,3 +407,34 @@ def test_products_without_columns_or_outputs_are_not_the_large_tiles(monkeypatch
     """A sum of nothing is zero and no outputs are none, as torch's product gives them; the large tile refuses both."""
     library = Library(monkeypatch)
     assert user(monkeypatch, library, ops.ProductChoices(), N, K, gated)(300) == [(300, 0)]
+
+
+@pytest.mark.parametrize("H,KV,D,rows,context,change,how", [
+    (16, 8, 128, 4, 600, None, "one"), (16, 8, 128, 32, 200, None, "one"), (16, 8, 128, 33, 200, None, "two"),  # 8 workgroups a row
+    (16, 8, 128, 8, 500, None, "one"), (16, 8, 128, 1, 2000, None, "one"), (16, 8, 128, 8, 2000, None, "two"),  # contexts in parts
+    (16, 8, 64, 32, 200, None, "one"), (16, 8, 64, 33, 200, None, "two"), (16, 8, 128, 4, 600, "q gains elsewhere", "two"),
+    (16, 8, 128, 4, 600, "k gains elsewhere", "two"), (16, 8, 128, 4, 600, "no norm", "two"), (16, 8, 128, 4, 600, "no rotation", "two"),
+    (16, 8, 128, 4, 600, "half of a head turned", "two"), (16, 8, 96, 4, 600, None, "two"), (16, 8, 128, 4, 600, "a prompt", "two"),
+    (16, 8, 128, 4, 600, "pages of 8", "two"), (16, 8, 128, 64, 8000, "bf16", "bf16"),
+])  # fmt: skip
+def test_the_route_of_a_32_bit_decode_step(monkeypatch, H, KV, D, rows, context, change, how):
+    """Norm, rotation, store and attention in one kernel while its workgroups are one round of the compute units, for the heads, norms, rotations
+    and pages that it takes and gains that start on 16 bytes; else in two."""
+    from types import SimpleNamespace
+
+    from atomserve_amd.parts.attention import Attention
+
+    made, dtype = [], BF16 if change == "bf16" else F32
+    for name, word in (("attn_f32_fresh", "one"), ("attn_decode_fresh", "bf16"), ("qk_norm_rope_store", "two"), ("gemm", None)):
+        monkeypatch.setattr(ops, name, lambda *args, word=word, **kw: made.append(word))
+    gains = [torch.empty(D + 4)[(1 if change == f"{n} gains elsewhere" else 0) :][:D] for n in "qk"]
+    turned = None if change == "no rotation" else torch.empty(rows, D // (4 if change == "half of a head turned" else 2), 2)
+    mixer = SimpleNamespace(
+        spec=SimpleNamespace(num_heads=H, num_kv_heads=KV, head_dim=D, hidden_size=64, window=0, scale=1.0,
+                             qk_norm=None if change == "no norm" else SimpleNamespace(eps=1e-6)),
+        env=SimpleNamespace(dtype=dtype, products=None), qkv=None, o=None, position=SimpleNamespace(prepare=lambda step: turned),
+        q_norm_weight=gains[0], k_norm_weight=gains[1], attend=lambda *args: None)  # fmt: skip
+    step = SimpleNamespace(decode_only=change != "a prompt", max_context=context, positions=None, all_tokens=None)
+    cache = SimpleNamespace(block_size=8 if change == "pages of 8" else 16, slots=None, writes=True, k_pages=None, v_pages=None, block_tables=None)
+    Attention.forward(mixer, torch.empty(rows, 64, dtype=dtype), step, cache)
+    assert [word for word in made if word] == [how]

@@ -1659,6 +1659,69 @@ def test_wide_products(ops, form, M, N, K):
             assert torch.equal(sums[i], a[:, part].float() @ w[:N, part].float().t())
 
 
+@pytest.mark.parametrize("form", range(6))
+def test_wide_products_of_numbers_that_are_not_finite(ops, form):
+    """An infinity or a NaN in one row of either matrix shows in that row's and that column's results as a plain product has it and nowhere
+    else, also in the last rows, which the tiles' copies repeat beyond the matrices' ends."""
+    from atomserve_amd.kernels.lib import call
+
+    torch.manual_seed(form)
+    M, N, K = 301, 528, 192
+    a, w = torch.randint(-4, 5, (M, K), device=DEV).to(BF16), torch.randint(-4, 5, (2 * N, K), device=DEV).to(BF16)
+    a[0, 7], a[130, 64], a[M - 1, K - 1] = float("inf"), float("nan"), float("-inf")
+    w[3, 9], w[N - 1, 100], w[N + 17, 63], w[2 * N - 1, K - 1] = float("-inf"), float("nan"), float("inf"), float("nan")
+    exact = a.float() @ w.float().t()
+    assert exact.isfinite().sum() > 0.9 * exact.numel()
+
+    def close(out, want):
+        assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.nan_to_num(), want.nan_to_num())
+
+    out = torch.empty(M, N, device=DEV, dtype=BF16)
+    call("as_gemm_bf16_wide", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, ops.WIDE_PLAIN, 1, form, ops._stream())
+    close(out, exact[:, :N].to(BF16))
+    both = torch.empty_like(out)
+    ops.silu_mul(exact.to(BF16), both)
+    call("as_gemm_bf16_wide", a.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, ops.WIDE_GATED, 1, form, ops._stream())
+    close(out, both)
+    sums = torch.empty(3, M, N, device=DEV)
+    call("as_gemm_bf16_wide", a.data_ptr(), w.data_ptr(), sums.data_ptr(), M, N, K, ops.WIDE_PARTIAL, 3, form, ops._stream())
+    for i in range(3):
+        close(sums[i], a[:, 64 * i : 64 * i + 64].float() @ w[:N, 64 * i : 64 * i + 64].float().t())
+
+
+@pytest.mark.parametrize("form", range(6))
+def test_wide_products_of_matrices_beyond_two_gib(ops, form):
+    """Rows of either matrix that start beyond 2^31 bytes, and long sums: whole numbers of up to 1, whose sums 32 bits hold."""
+    from atomserve_amd.kernels.lib import call
+
+    torch.manual_seed(form)
+    K, many, few = 16448, 65536, 144  # 2^31 bytes and 8 MB more
+
+    def whole(rows):
+        return torch.randint(-1, 2, (rows, K), device=DEV, dtype=torch.int8).to(BF16)
+
+    large, small = whole(many), whole(few)
+    picked = torch.tensor([0, 255, 256, 40000, 65279, 65280, many - 17, many - 1], device=DEV)
+    exact = large[picked].float() @ small.float().t()  # [picked, few]
+    out = torch.empty(many, few, device=DEV, dtype=BF16)  # the activations are the large ones
+    call("as_gemm_bf16_wide", large.data_ptr(), small.data_ptr(), out.data_ptr(), many, few, K, ops.WIDE_PLAIN, 1, form, ops._stream())
+    assert torch.equal(out[picked], exact.to(BF16))
+    out = torch.empty(few, many, device=DEV, dtype=BF16)  # the weights are
+    call("as_gemm_bf16_wide", small.data_ptr(), large.data_ptr(), out.data_ptr(), few, many, K, ops.WIDE_PLAIN, 1, form, ops._stream())
+    assert torch.equal(out[:, picked], exact.t().to(BF16))
+    sums = torch.empty(3, few, many, device=DEV)  # 86 units a range, the last one 85
+    call("as_gemm_bf16_wide", small.data_ptr(), large.data_ptr(), sums.data_ptr(), few, many, K, ops.WIDE_PARTIAL, 3, form, ops._stream())
+    assert torch.equal(sums[:, :, picked].sum(0), exact.t())
+    large.mul_(2.0**-7)  # gates of a few units; the second half are the up rows
+    out = torch.empty(few, many // 2, device=DEV, dtype=BF16)
+    call("as_gemm_bf16_wide", small.data_ptr(), large.data_ptr(), out.data_ptr(), few, many // 2, K, ops.WIDE_GATED, 1, form, ops._stream())
+    columns = torch.cat([picked[picked < many // 2], torch.tensor([many // 2 - 1], device=DEV)])
+    gate_up = (small.float() @ large[torch.cat([columns, columns + many // 2])].float().t()).to(BF16)
+    both = torch.empty(few, len(columns), device=DEV, dtype=BF16)
+    ops.silu_mul(gate_up, both)
+    assert torch.equal(out[:, columns], both)
+
+
 def test_wide_products_are_what_many_rows_take(ops):
     """`gemm_silu_mul` and `gemm_split_sums` of more than 128 rows: their rules, and the bits of the product and the activation."""
     torch.manual_seed(3)
