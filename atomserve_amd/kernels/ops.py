@@ -1175,6 +1175,7 @@ WIDE_PLAIN, WIDE_GATED, WIDE_PARTIAL = 0, 1, 2
 WIDE_FORMS = ((256, 256, 1, 1.33, 0.96, 6.6), (256, 192, 1, 1.09, 0.765, 4.5), (256, 128, 1, 0.83, 0.62, 2.4),
               (192, 256, 1, 1.215, 0.825, 7.6), (128, 128, 1, 0.53, 0.375, 1.0), (128, 128, 2, 1.0, 0.52, 0.5))  # fmt: skip
 WIDE_LAUNCH_US, WIDE_US_A_MB, WIDE_SPLITS = 3.0, 0.2, (2, 3, 4, 6, 8, 12)
+WIDE_NO_PARTIAL = 3  # the form whose partial sums are not worth making (`_wide_plan`)
 
 
 def _wide_cost(form: int, tiles: int, units: int) -> float:
@@ -1189,9 +1190,14 @@ def _wide_cost(form: int, tiles: int, units: int) -> float:
 @functools.lru_cache(maxsize=4096)
 def _wide_plan(rows: int, n: int, k: int, kind: int) -> tuple:
     """(us, form, splits) of the cheapest tile for a product of these sizes (kind gated: n outputs of 2 n rows of w; partial: with K cut into
-    ranges whose sums are written, and read by whoever adds them up; in one round of workgroups)."""
+    ranges whose sums are written, and read by whoever adds them up; in one round of workgroups).  Partial sums are not made in tiles of
+    192 x 256: that way out takes 508 registers where the form's others take 396, and inside prompts it lost to 256 x 256 with as many
+    ranges at 58 of 59 sizes measured, by up to 77 us (5,120 outputs of K = 25,600, 1,152 rows in two ranges: 48 us slower than the
+    library's whole product, which they were expected to beat)."""
     best = None
     for form, (tm, tn, each, *_) in enumerate(WIDE_FORMS):
+        if kind == WIDE_PARTIAL and form == WIDE_NO_PARTIAL:
+            continue
         tiles = -(-rows // tm) * -(-n // (tn // 2 if kind == WIDE_GATED else tn))
         for splits in WIDE_SPLITS if kind == WIDE_PARTIAL else (1,):
             units = -(-(k // WIDE_UNIT) // splits)
@@ -1234,11 +1240,13 @@ def wide_gated_form(rows: int, outputs: int, k: int):
 @functools.lru_cache(maxsize=4096)
 def wide_split_plan(rows: int, n: int, k: int):
     """(form, splits) of a product of more than 128 rows cut along K into partial sums, or None where that, the sums' reading counted, is
-    not expected to save 5 per cent of the library's whole product (74 of 144 measured products are cut; none of them was slower):
+    not expected to take less than the library's whole product.  Inside prompts of 47 lengths at six sizes, down is cut in 194 of 282 and saves
+    25 us on average, nowhere less than nothing; o is cut in 100 and saves 6, and loses 5 us once (in a spread of 25) and 2 once (of a layer's
+    242).  (Up to 3 per cent more than the library's was expected to take also pays for down, for o not.)  Alone, us of the two:
     4,096 outputs of K = 12,288, 256 / 512 / 1,024 rows 52 39, 78 56, 106 95; 2,560 of 9,728, 512 / 2,048 rows 52 38, 102 95; 5,120 of
     17,408, 256 rows 129 58; 1,024 of 3,072, 256 rows 12.5 10.2.  Short products of many rows stay whole (4,096 of 4,096, 700 rows 34 37)."""
     best = _wide_plan(rows, n, k, WIDE_PARTIAL)
-    if best is None or best[0] >= 0.95 * (_library_us(rows, n, k) + 2e-6 * WIDE_US_A_MB * rows * n):
+    if best is None or best[0] >= _library_us(rows, n, k) + 2e-6 * WIDE_US_A_MB * rows * n:
         return None
     return best[1:]
 
