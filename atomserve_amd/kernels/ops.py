@@ -1175,6 +1175,7 @@ WIDE_PLAIN, WIDE_GATED, WIDE_PARTIAL = 0, 1, 2
 WIDE_FORMS = ((256, 256, 1, 1.33, 0.96, 6.6), (256, 192, 1, 1.09, 0.765, 4.5), (256, 128, 1, 0.83, 0.62, 2.4),
               (192, 256, 1, 1.215, 0.825, 7.6), (128, 128, 1, 0.53, 0.375, 1.0), (128, 128, 2, 1.0, 0.52, 0.5))  # fmt: skip
 WIDE_LAUNCH_US, WIDE_US_A_MB, WIDE_SPLITS = 3.0, 0.2, (2, 3, 4, 6, 8, 12)
+WIDE_TWO_AT_LEAST = 0.93  # of a full round's time, once a compute unit holds two workgroups (`wide_gated_form`)
 WIDE_NO_PARTIAL = 3  # the form whose partial sums are not worth making (`_wide_plan`)
 
 
@@ -1229,11 +1230,22 @@ def _wide_takes(a, w, n: int, rows_of_w: int) -> bool:
 @functools.lru_cache(maxsize=4096)
 def wide_gated_form(rows: int, outputs: int, k: int):
     """The tile of a gated product of more than 128 rows, or None where the library's product with the activation after it is expected
-    to take less: four of the 72 measured products, tall of few rows (333 rows of 12,288 outputs and K = 4,096: 75 us, 83).  Elsewhere, us of
-    the library's best of 16 and the activation, and of this: 3,072 outputs of K = 1,024, 256 / 1,024 / 2,409 rows 19.1 11.5, 24.8 17.6,
-    38.0 32.9; 9,728 of 2,560, 512 / 2,409 rows 61 52, 228 197; 12,288 of 4,096, 512 / 2,048 rows 91 86, 297 300; 25,600 of 5,120, 1,500 rows
-    693 604."""
+    to take less.  Alone, us of the library's best of 16 and the activation, and of this: 3,072 outputs of K = 1,024, 256 / 1,024 / 2,409 rows
+    19.1 11.5, 24.8 17.6, 38.0 32.9; 9,728 of 2,560, 512 / 2,409 rows 61 52, 228 197; 12,288 of 4,096, 333 / 512 / 2,048 rows 75 83, 91 86,
+    297 300; 25,600 of 5,120, 1,500 rows 693 604.  Inside prompts of 27 lengths at six sizes, the library with the kernel that a trial of the length
+    or of the next tuned one chose: 140 of 162 go to the tile and save 10 us a layer in the middle; 12 lose, 8 us of a layer's 560 once (384 rows of
+    25,600 outputs), 0 to 5 of 270 to 780 else (12,288 outputs, 300, 700 and 1,900 rows); 2,048 rows of 12,288 save 0 to 6.  (Trials of the tuned row
+    counts that time the tile beside the products with their activation decide worse: the least of 16 candidates' runs against that of one gave 44
+    of these to the library, 13 of which lose 9 to 30 us by it and none saves more than 10.)
+    Where a compute unit holds two workgroups of the last round, the round takes as long as a full one, or nearly (tiles in the last round and us a
+    unit of K: 255 0.81, 270 0.99, 303 1.07, 510 1.15): with the mean of few and full, 353 to 384 rows of 17,408 outputs and K = 5,120 went to a
+    tile that took 20 us a layer more than the two kernels (a prompt of 384 tokens through 4 such layers 1,810 us, 1,730 without)."""
     us, form, _ = _wide_plan(rows, outputs, k, WIDE_GATED)
+    tm, tn, each, full, few, _ = WIDE_FORMS[form]
+    places = each * compute_units()
+    rest = -(-rows // tm) * -(-outputs // (tn // 2)) % places
+    if rest > compute_units():
+        us += k // WIDE_UNIT * max(WIDE_TWO_AT_LEAST * full - (few + (full - few) * rest / places), 0.0)
     return form if us < _library_us(rows, 2 * outputs, k) + 4.0 + 6e-6 * WIDE_US_A_MB * rows * outputs else None
 
 
