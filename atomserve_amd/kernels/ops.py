@@ -2271,6 +2271,9 @@ def moe_tile(pairs: int, first, second, gated: bool) -> int:
     are where that kernel's lay, 56 pairs and 128 for smaller matrices; they could lie at 32."""
     if not (_moe_streamed(first, gated) and _moe_streamed(second, False)):
         return MOE_TILES[0]
+    rows = (-(-pairs // MOE_TILES[1]) + first.shape[0]) * MOE_TILES[1]
+    if rows * max(first.shape[2], second.shape[2]) * 2 > 0xF0000000:  # the pairs' rows, too, lie at 32-bit offsets there, at 64-bit ones in tiles of 64
+        return MOE_TILES[0]
     many = MOE_MANY if first.numel() >= MOE_LARGE_WEIGHTS else MOE_MANY_SMALL
     return MOE_TILES[pairs >= many * first.shape[0]]
 

@@ -148,6 +148,22 @@ def test_tiles_of_experts_pairs():
     assert tile(300, weights(1 << 18, 8192, 1), weights(8192, 1 << 17, 1)) == 64  # an expert beyond 32-bit offsets
 
 
+@pytest.mark.parametrize("first,second", [(3072, 4096), (8192, 2048)])  # the wider input: gate and up's, down's
+def test_pairs_whose_rows_pass_4_gib_are_not_in_tiles_of_128(first, second):
+    """The kernel of large tiles finds its pairs' rows at 32-bit offsets and takes tiles of 128 up to 0xf0000000 bytes of them; beyond, such a route
+    would go to the kernel for all sizes, which is slower than tiles of 64."""
+
+    class Weights:
+        def __init__(self, *shape):
+            self.shape, self.dtype, self.numel, self.data_ptr = shape, BF16, lambda: shape[0] * shape[1] * shape[2], lambda: 0
+
+    inner = first // 2
+    up, down = Weights(64, first, second), Weights(64, second, inner)
+    widest = max(second, inner)
+    most = 0xF0000000 // (2 * widest) // 128 - 64  # tiles of pairs: one more for every expert is counted
+    assert ops.moe_tile(128 * most, up, down, True) == 128 and ops.moe_tile(128 * most + 1, up, down, True) == 64
+
+
 def test_which_plain_products_take_the_tile_kernel_without_trials(monkeypatch):
     monkeypatch.setattr(ops, "compute_units", lambda: 256)
     strips = ops._plain_tile_strips
