@@ -2239,9 +2239,7 @@ MOE_TILES = (64, 128)  # pairs of one expert that a tile of the grouped products
 MOE_MAX_EXPERTS = 1024
 
 
-# Pairs an expert from which on tiles of 128 are taken, and the values of all experts' first matrices (gate and up,
-# both in bf16) that the first of the two lines needs (`moe_tile`).
-MOE_MANY, MOE_MANY_SMALL, MOE_LARGE_WEIGHTS = 56, 128, 60 << 20
+MOE_MANY = 32  # pairs an expert from which on tiles of 128 are taken (`moe_tile`)
 
 
 def _moe_streamed(w, gated: bool) -> bool:
@@ -2267,15 +2265,19 @@ def moe_tile(pairs: int, first, second, gated: bool) -> int:
     4,096,       403 M    217/225   225/229   238/235   341/248   423/303   560/336   791/439
     2,048, 128 experts, 8 a token, 403 M
                           227/228   236/235   255/248   332/264   450/321   596/393   840/505
-    (before, weights into registers and pairs through them into LDS: 2,048 and 101 M at 162 pairs 127, 4,096 and 403 M 482).  The lines
-    are where that kernel's lay, 56 pairs and 128 for smaller matrices; they could lie at 32."""
+    (before, weights into registers and pairs through them into LDS: 2,048 and 101 M at 162 pairs 127, 4,096 and 403 M 482).  Inside
+    prompts through 8 layers, 4 of them with such experts, us:
+                          24            32            38            48            56            64            100           128
+    width 1,024,  25 M    1,492/1,495   1,478/1,476   1,517/1,513   1,499/1,496   1,491/1,488   1,503/1,493   1,570/1,567   1,577/1,567
+    2,048,       101 M    1,555/1,550   1,560/1,557   1,578/1,544   1,656/1,616   1,735/1,680   1,850/1,762   2,264/2,188   2,467/2,377
+    4,096,       403 M    2,693/2,688   2,807/2,773   3,078/3,045   3,250/3,153   3,643/3,418   3,818/3,493   5,151/4,665   5,767/5,172
+    From 32 pairs on tiles of 128 lose nowhere; at 20 they lose 6 us at width 4,096."""
     if not (_moe_streamed(first, gated) and _moe_streamed(second, False)):
         return MOE_TILES[0]
     rows = (-(-pairs // MOE_TILES[1]) + first.shape[0]) * MOE_TILES[1]
     if rows * max(first.shape[2], second.shape[2]) * 2 > 0xF0000000:  # the pairs' rows, too, lie at 32-bit offsets there, at 64-bit ones in tiles of 64
         return MOE_TILES[0]
-    many = MOE_MANY if first.numel() >= MOE_LARGE_WEIGHTS else MOE_MANY_SMALL
-    return MOE_TILES[pairs >= many * first.shape[0]]
+    return MOE_TILES[pairs >= MOE_MANY * first.shape[0]]
 
 
 def moe_across(pairs: int, experts: int, rows: int) -> int:
