@@ -510,10 +510,15 @@ def attn_f32_fresh_supported(dtype, num_heads: int, num_kv_heads: int, head_dim:
 
 
 def attn_f32_fresh_preferred(rows: int, H: int, KV: int, D: int, max_context: int, window: int) -> bool:
-    """Whether a decode step of these sizes is faster through `attn_f32_fresh` than through the two kernels: while its workgroups are one
-    round of the compute units, for the wider kernel leaves room for one to each.  16 heads of 128 on 8 kv heads, us of one / of two: 8
-    requests of 64 tokens 8.9 9.8, 4 of 200 14.3 14.8, 4 of 600 15.4 15.8, 1 of 2,000 17.9 18.5; 8 of 2,000 in 8 parts 36.4 34.8."""
-    return rows * KV * _partitions(rows, H, KV, D, max_context, window, True, None, "meta")[1] <= compute_units()
+    """Whether a decode step of these sizes is faster through `attn_f32_fresh` than through the two kernels.  Heads of 128: while its
+    workgroups are one round of the compute units, for it takes 284 registers (32 of them accumulators), which leave room for one workgroup to
+    each where the other kernel has two.  Heads of 64 (152 registers; three workgroups, as without): always.
+    us of one / of two, 16 heads on 8 kv heads, by requests x tokens (heads of 128, then of 64):
+        4 x 200       32 x 200      64 x 200      4 x 600       8 x 600       16 x 600      4 x 2,000     8 x 2,000     32 x 2,000    8 x 6,000
+        14.3/14.6     19.1/20.2     34.7/30.1     15.9/16.4     24.1/22.2     33.5/30.1     22.2/23.8     36.2/34.5     103/102       79/78
+        10.1/11.3     12.1/13.6     16.9/19.3     12.1/13.4     15.0/16.5     18.6/20.1     15.7/17.6     21.2/23.6     55.5/54.8     43/46
+    (heads of 64, 105 sizes with 8 on 2 and 32 on 8 heads too: slower at six, by 1.4 per cent at most)."""
+    return D <= 64 or rows * KV * _partitions(rows, H, KV, D, max_context, window, True, None, "meta")[1] <= compute_units()
 
 
 def attn_f32_fresh(qkv, q_weight, k_weight, cos_sin, slots, eps, store_kv, k_pages, v_pages, positions, block_tables, out, num_heads,
@@ -1324,9 +1329,10 @@ def _gated_two_tiles(rows: int, k: int, w) -> bool:
 
 def gemm_silu_mul(a, w, out, choices=None) -> None:
     """out[M, I] = silu(a @ w[:I]^T) * (a @ w[I:]^T) for w[2 I, K]: the gate and up products and
-    the activation.  bf16 with few rows: one kernel, the products rounded to bf16 before the
-    activation exactly as the two-kernel path does; fp32 of more than 256 columns: one kernel, the same bits as
-    two (333 rows, 1,024 -> 6,144: 51 us, 51 and 5 for two); otherwise the product, then the activation."""
+    the activation.  bf16 of up to 128 rows, and of more where the large tile is expected to be the faster way
+    (`wide_gated_form`): one kernel, the products rounded to bf16 before the activation exactly as the two-kernel path does; fp32 of
+    more than 256 columns: one kernel, the same bits as two (333 rows, 1,024 -> 6,144: 51 us, 51 and 5 for two); otherwise the
+    product, then the activation."""
     _check(a, "a", (F32, BF16), (None, None))
     M, K = a.shape
     _check(out, "out", a.dtype, (M, None))
