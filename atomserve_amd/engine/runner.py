@@ -354,9 +354,11 @@ class ModelRunner:
 
     @torch.inference_mode()
     def tune_prompt_lengths(self, most_tokens: int) -> list:
-        """Runs a prompt that stores nothing at each of a few lengths (128, 192, 256, 384, ... up to `most_tokens`)
+        """Runs a prompt that stores nothing at each of a few lengths (128, 192, 256, 384, ... up to `most_tokens`, and that)
         until the library's candidates for its products have been tried and the fastest chosen; prompts
-        of other lengths then take what the next length above them chose.  Returns the lengths run."""
+        of other lengths then take what the next length above them chose.  Returns the lengths run.  (A step's budget, which is tuned
+        wherever it lies, else has its first eight steps try the candidates: 600 tokens in a budget of 600 at Qwen3-4B sizes 3,300 us
+        for the first two, 2,500 on average of ten, 1,940 later.)"""
         products = self.model.env.products
         if self.device.type != "cuda" or products.fixed:
             return []
@@ -364,6 +366,8 @@ class ModelRunner:
         while n <= most_tokens:
             lengths.extend(m for m in (n, n + n // 2) if m <= most_tokens)
             n *= 2
+        if lengths and lengths[-1] != most_tokens:
+            lengths.append(most_tokens)
         slot = self.pools.scrap_slot if self.manager.state_groups else -1
         for n in lengths:
             products.tune_rows(n)

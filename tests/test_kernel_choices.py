@@ -470,3 +470,19 @@ def test_the_route_of_a_32_bit_decode_step(monkeypatch, H, KV, D, rows, context,
     cache = SimpleNamespace(block_size=8 if change == "pages of 8" else 16, slots=None, writes=True, k_pages=None, v_pages=None, block_tables=None)
     Attention.forward(mixer, torch.empty(rows, 64, dtype=dtype), step, cache)
     assert [word for word in made if word] == [how]
+
+
+@pytest.mark.parametrize("budget,lengths", [(127, []), (128, [128]), (200, [128, 192, 200]), (512, [128, 192, 256, 384, 512]), (600, [128, 192, 256, 384, 512, 600])])
+def test_a_warm_up_tries_the_steps_budget_itself(monkeypatch, budget, lengths):
+    """A budget is a tuned row count wherever it lies: its trials belong to the warm-up, not to the first steps that fill it."""
+    from types import SimpleNamespace
+
+    from atomserve_amd.engine.runner import ModelRunner
+
+    monkeypatch.setattr(ops, "prepare_library_adoption", lambda: True)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    products, ran = ops.ProductChoices(), []
+    runner = SimpleNamespace(model=SimpleNamespace(env=SimpleNamespace(products=products)), device=torch.device("cuda"),
+                             manager=SimpleNamespace(block_size=16, state_groups=[], paged_groups=[0]), step=lambda rows: ran.append(len(rows[0].tokens)))  # fmt: skip
+    assert ModelRunner.tune_prompt_lengths(runner, budget) == lengths == ran
+    assert set(lengths) <= products.tuned_rows
