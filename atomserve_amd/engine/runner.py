@@ -356,7 +356,10 @@ class ModelRunner:
     def tune_prompt_lengths(self, most_tokens: int) -> list:
         """Runs a prompt that stores nothing at each of a few lengths (128, 192, 256, 384, ... up to `most_tokens`, and that)
         until the library's candidates for its products have been tried and the fastest chosen; prompts
-        of other lengths then take what the next length above them chose.  Returns the lengths run.  (A step's budget, which is tuned
+        of other lengths then take what the next length above them chose.  Returns the lengths run.  (Its tokens differ, as a prompt's
+        do: the products of rows that are all alike run at clocks that real ones do not reach, and other kernels win; 2,048 tokens through 8
+        layers of Qwen3-8B sizes 6,152 us with the kernels tried on one token, 6,132 on different ones, 2,409 of -4B sizes 4,391
+        and 4,377, in the middle of six warm-ups each.  A step's budget, which is tuned
         wherever it lies, else has its first eight steps try the candidates: 600 tokens in a budget of 600 at Qwen3-4B sizes 3,300 us
         for the first two, 2,500 on average of ten, 1,940 later.)"""
         products = self.model.env.products
@@ -372,7 +375,7 @@ class ModelRunner:
         for n in lengths:
             products.tune_rows(n)
             tables = [[0] * -(-n // bs) for _ in self.manager.paged_groups]
-            rows = [Row([0] * n, 0, tables, [n - 1], slot, store=False)]
+            rows = [Row([i % self.vocab_size for i in range(n)], 0, tables, [n - 1], slot, store=False)]
             for _ in range(4):
                 self.step(rows)
                 if not products.trials_pending():

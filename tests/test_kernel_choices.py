@@ -483,6 +483,7 @@ def test_a_warm_up_tries_the_steps_budget_itself(monkeypatch, budget, lengths):
     monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
     products, ran = ops.ProductChoices(), []
     runner = SimpleNamespace(model=SimpleNamespace(env=SimpleNamespace(products=products)), device=torch.device("cuda"),
-                             manager=SimpleNamespace(block_size=16, state_groups=[], paged_groups=[0]), step=lambda rows: ran.append(len(rows[0].tokens)))  # fmt: skip
-    assert ModelRunner.tune_prompt_lengths(runner, budget) == lengths == ran
+                             manager=SimpleNamespace(block_size=16, state_groups=[], paged_groups=[0]), vocab_size=150, step=lambda rows: ran.append(rows[0].tokens))  # fmt: skip
+    assert ModelRunner.tune_prompt_lengths(runner, budget) == lengths == [len(tokens) for tokens in ran]
+    assert all(len(set(tokens)) == min(len(tokens), 150) and 0 <= min(tokens) <= max(tokens) < 150 for tokens in ran)  # not one token again and again
     assert set(lengths) <= products.tuned_rows
