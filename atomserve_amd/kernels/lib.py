@@ -7,6 +7,7 @@ library cannot be built or loaded raises.
 """
 
 import ctypes
+import functools
 import struct
 import threading
 from ctypes import byref, c_double, c_float, c_int, c_longlong, c_size_t, c_void_p, cast
@@ -17,7 +18,7 @@ from atomserve_amd.kernels import build
 
 P, I, F = c_void_p, c_int, c_float
 _CFuncPtr = ctypes.CDLL(None)._FuncPtr.__base__  # what every C function is that ctypes calls
-_FLOAT, _FLOAT_BITS = struct.Struct("<f"), struct.Struct("<I")
+_FLOAT_BITS = struct.Struct("<I")
 _WORDS = (c_void_p, c_int, c_longlong, c_size_t)
 LIST_INTEGERS, LIST_FLOATS = 32, 4  # of a call that `csrc/launches.hip` makes (its MOST and FLOATS)
 
@@ -169,6 +170,17 @@ def call(name: str, *args) -> None:
         watch.calls.append((name, fn, args))
 
 
+@functools.lru_cache(maxsize=256)
+def _list_places(argtypes: tuple):
+    """The arguments of such types that are integers or addresses, those that are 32-bit floats, and the integers' places among their
+    like, as `csrc/launches.hip` wants them; None where a list holds no such call."""
+    floats = [at for at, kind in enumerate(argtypes) if kind is c_float]
+    ints = [at for at, kind in enumerate(argtypes) if kind in _WORDS]
+    if len(ints) + len(floats) < len(argtypes) or len(ints) > LIST_INTEGERS or len(floats) > LIST_FLOATS:
+        return None
+    return ints, floats, {at: i for i, at in enumerate(ints)}
+
+
 class Launches:
     """The launches that a piece of code makes (`with Launches() as made:`), to be made again with other
     addresses: `made.aim(sources)`, then `made.again(targets)` for as many lists of targets as there are: wherever a
@@ -203,23 +215,22 @@ class Launches:
         them is not of that kind: an entry point that is no C function, more arguments than a call of a list has or arguments of other types."""
         words = []
         for _, fn, args, patches in self.patched:
-            if not isinstance(fn, _CFuncPtr):
+            known = _list_places(tuple(fn.argtypes)) if isinstance(fn, _CFuncPtr) else None
+            if known is None or len(args) != len(fn.argtypes):
                 return None
-            ints, floats, place = [], [], {}
-            for at, (kind, v) in enumerate(zip(fn.argtypes, args, strict=True)):
-                if kind is c_float and isinstance(v, (int, float)):
-                    floats.append(_FLOAT_BITS.unpack(_FLOAT.pack(c_float(v).value))[0])
-                elif kind in _WORDS and (v is None or isinstance(v, int)):
-                    place[at] = len(ints)
-                    ints.append(int(v or 0))
-                else:
-                    return None
-            if len(ints) > LIST_INTEGERS or len(floats) > LIST_FLOATS:
+            ints, floats, place = known
+            words += (cast(fn, c_void_p).value, len(ints), len(floats), len(patches))
+            words += [0 if args[at] is None else args[at] for at in ints]
+            try:
+                words += [_FLOAT_BITS.unpack(c_float(args[at]))[0] for at in floats]
+            except TypeError:
                 return None
-            words += (cast(fn, c_void_p).value, len(ints), len(floats), len(patches), *ints, *floats)
             for at, i in patches:
                 words += (place[at], i)
-        return (c_longlong * len(words))(*words)
+        try:
+            return (c_longlong * len(words))(*words)
+        except TypeError:  # an argument that is no plain number
+            return None
 
     def fits(self, targets: list) -> bool:
         """Whether `targets` (of use: those at the places `met`) can stand for the sources: one address for one address."""

@@ -285,6 +285,7 @@ def test_calls_that_no_list_holds_are_made_one_by_one(kinds):
         return status[0]
 
     function = CFUNCTYPE(c_int, *types)(entry)
+    function.argtypes = types  # a list, as the entry points' are
     args = [0.5 + n if k in "fd" else 1000 + n for n, k in enumerate(kinds)]
     if "d" in kinds:
         args[kinds.index("d")] = 1.0 + 2.0**-40
@@ -297,3 +298,10 @@ def test_calls_that_no_list_holds_are_made_one_by_one(kinds):
     with pytest.raises(KernelError, match="the call"):
         made.again([7] * len(sources))
     assert (made.program is None) == (len(kinds) != 36)
+    seen.clear()
+    status[0] = 0
+    args[-1] = types[-1](3)  # no plain number
+    made.calls = [("the call", function, args)]
+    made.aim([])
+    made.again([])
+    assert made.program is None and seen == [[*args[:-1], 3]]
