@@ -19,6 +19,10 @@ from atomserve_amd.engine.sequence import StepResult
 from atomserve_amd.kernels import ops
 from atomserve_amd.sampling.sampler import Sampler
 
+# Passes in which the trials of a product that only one layer has come to their end: sixteen candidates of the library and two of this
+# package's, and the call that finds them tried.
+BUDGET_PASSES = 18 * ops.LIBRARY_TRIALS_EACH + 1
+
 
 def rows_for(seqs, num_new_tokens) -> list:
     """The usual rows: each sequence's next uncomputed tokens, logits at its last token only
@@ -361,7 +365,9 @@ class ModelRunner:
         layers of Qwen3-8B sizes 6,152 us with the kernels tried on one token, 6,132 on different ones, 2,409 of -4B sizes 4,391
         and 4,377, in the middle of six warm-ups each.  A step's budget, which is tuned
         wherever it lies, else has its first eight steps try the candidates: 600 tokens in a budget of 600 at Qwen3-4B sizes 3,300 us
-        for the first two, 2,500 on average of ten, 1,940 later.)"""
+        for the first two, 2,500 on average of ten, 1,940 later.  Its trials run inside passes to their end, also where a model has
+        few layers: what `settle` runs by itself, one product after another, has other winners; 1,500 tokens of Dozusun layers of width 2,048,
+        four of a kind, 2,953 us against 2,921 in the middle of nine warm-ups each.)"""
         products = self.model.env.products
         if self.device.type != "cuda" or products.fixed:
             return []
@@ -376,7 +382,7 @@ class ModelRunner:
             products.tune_rows(n)
             tables = [[0] * -(-n // bs) for _ in self.manager.paged_groups]
             rows = [Row([i % self.vocab_size for i in range(n)], 0, tables, [n - 1], slot, store=False)]
-            for _ in range(4):
+            for _ in range(BUDGET_PASSES if n == most_tokens else 4):
                 self.step(rows)
                 if not products.trials_pending():
                     break

@@ -487,3 +487,20 @@ def test_a_warm_up_tries_the_steps_budget_itself(monkeypatch, budget, lengths):
     assert ModelRunner.tune_prompt_lengths(runner, budget) == lengths == [len(tokens) for tokens in ran]
     assert all(len(set(tokens)) == min(len(tokens), 150) and 0 <= min(tokens) <= max(tokens) < 150 for tokens in ran)  # not one token again and again
     assert set(lengths) <= products.tuned_rows
+
+
+@pytest.mark.parametrize("ends_after,passes", [(1, [1, 1, 1]), (3, [3, 3, 3]), (9, [4, 4, 9]), (500, [4, 4, 73])])
+def test_the_budgets_trials_run_inside_passes(monkeypatch, ends_after, passes):
+    """A model of few layers needs many passes until every candidate has run; the other lengths' trials are ended by `settle` after four."""
+    from types import SimpleNamespace
+
+    from atomserve_amd.engine.runner import ModelRunner
+
+    monkeypatch.setattr(ops, "prepare_library_adoption", lambda: True)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    ran, settled_at = [], []
+    products = SimpleNamespace(fixed=False, tune_rows=lambda n: ran.append(0), trials_pending=lambda: ran[-1] < ends_after, settle=lambda: settled_at.append(ran[-1]))
+    runner = SimpleNamespace(model=SimpleNamespace(env=SimpleNamespace(products=products)), device=torch.device("cuda"), vocab_size=150,
+                             manager=SimpleNamespace(block_size=16, state_groups=[], paged_groups=[0]), step=lambda rows: ran.append(ran.pop() + 1))  # fmt: skip
+    ModelRunner.tune_prompt_lengths(runner, 200)
+    assert ran == settled_at == passes
