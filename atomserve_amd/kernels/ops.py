@@ -1239,7 +1239,8 @@ def wide_gated_form(rows: int, outputs: int, k: int):
     19.1 11.5, 24.8 17.6, 38.0 32.9; 9,728 of 2,560, 512 / 2,409 rows 61 52, 228 197; 12,288 of 4,096, 333 / 512 / 2,048 rows 75 83, 91 86,
     297 300; 25,600 of 5,120, 1,500 rows 693 604.  Inside prompts of 27 lengths at six sizes, the library with the kernel that a trial of the length
     or of the next tuned one chose: 140 of 162 go to the tile and save 10 us a layer in the middle; 12 lose, 8 us of a layer's 560 once (384 rows of
-    25,600 outputs), 0 to 5 of 270 to 780 else (12,288 outputs, 300, 700 and 1,900 rows); 2,048 rows of 12,288 save 0 to 6.  (Trials of the tuned row
+    25,600 outputs), 0 to 5 of 270 to 780 else (12,288 outputs, 300, 700 and 1,900 rows).  2,048 rows of 12,288 are even: in a trace of both the tile
+    312 us and the two kernels 278 and 30, a prompt through 8 such layers 6,189 to 6,224 us and 6,223 to 6,237.  (Trials of the tuned row
     counts that time the tile beside the products with their activation decide worse: the least of 16 candidates' runs against that of one gave 44
     of these to the library, 13 of which lose 9 to 30 us by it and none saves more than 10.)
     Where a compute unit holds two workgroups of the last round, the round takes as long as a full one, or nearly (tiles in the last round and us a
