@@ -8,9 +8,12 @@
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx8 __attribute__((ext_vector_type(8)));
 typedef bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
-struct Parts { bf16x8 h, m, l; };  // eight floats as h + m + l
+struct Parts { bf16x8 h, m, l; };   // eight floats as h + m + l
+struct Parts4 { bf16x4 h, m, l; };  // four
 
 __device__ __forceinline__ floatx8 widen(bf16x8 v) {
   const uintx4 u = __builtin_bit_cast(uintx4, v);
@@ -31,6 +34,21 @@ __device__ __forceinline__ Parts parts(floatx4 p, floatx4 q) {
   s.m = __builtin_convertvector(x, bf16x8);
   x -= widen(s.m);
   s.l = __builtin_convertvector(x, bf16x8);
+  return s;
+}
+
+__device__ __forceinline__ floatx4 widen(bf16x4 v) {
+  const uintx2 u = __builtin_bit_cast(uintx2, v);
+  return floatx4{__uint_as_float(u[0] << 16), __uint_as_float(u[0] & 0xffff0000u), __uint_as_float(u[1] << 16), __uint_as_float(u[1] & 0xffff0000u)};
+}
+
+__device__ __forceinline__ Parts4 parts(floatx4 x) {
+  Parts4 s;
+  s.h = __builtin_convertvector(x, bf16x4);  // to nearest
+  x -= widen(s.h);
+  s.m = __builtin_convertvector(x, bf16x4);
+  x -= widen(s.m);
+  s.l = __builtin_convertvector(x, bf16x4);
   return s;
 }
 

@@ -384,8 +384,12 @@ __global__ __launch_bounds__(16 / SIDE * 64) void gemm_f32_side_kernel(const flo
 }
 
 // Operands through LDS, for many rows: 8 waves (WM x WN) make a tile of BM = 16 WM MTW rows of `a` by BN = 16 WN NTW rows of
-// `w` in steps of 32 columns.  Every float is taken apart once a workgroup, on its way from registers (loaded two steps ahead) into
+// `w` in steps of 32 columns.  Every float is taken apart once a workgroup, on its way from registers (asked for a step or two ahead) into
 // LDS, where the parts of the next step are written while those of this one are multiplied: one barrier a step.
+// What bounds it: a step of 128 x 128 takes 1.0 us, its matrix instructions alone 0.77, taking apart 0.16, the writes into LDS 0.08, and the
+// waves of a workgroup do these at the same time; so the vector unit's work is dealt out between the matrix instructions, and every wait for
+// LDS stands behind some of them.  128 x 128 outputs in which every operand was read before the first product, K = 1,024 / 2,048 at
+// up to 256 tiles: 54 / 93 us, now 43 / 75; 64 x 64, one tile a compute unit: 24 / 43, now 19 / 34.
 // A place holds 16 bytes, 8 columns of a row; place (row, column block c) of a part is row * 4 + (c ^ f(row / 4 % 4)), f =
 // 0, 2, 3, 1: the hardware reads 16-byte operands in the lane groups {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31} and the
 // same above 32, which so touch every bank once.
@@ -395,11 +399,13 @@ template <int WM, int WN, int MTW, int NTW, bool IS_GATED, bool SPLIT, bool VEC>
 __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
                                                              float* __restrict__ out, int M, int N, int K, int tiles_m, int tiles,
                                                              int per_xcd) {
-  constexpr int THREADS = 512, AHEAD = 2;
+  constexpr int THREADS = 512;
   constexpr int BM = 16 * WM * MTW, BN = 16 * WN * NTW, ROWS = BM + BN;
-  constexpr int PIECES = ROWS * 4 / THREADS;  // of 8 columns a thread and step
+  constexpr int PIECES = (ROWS * 8 + THREADS - 1) / THREADS;  // of 4 columns a thread and step; where they do not divide, some are brought twice
+  constexpr int AHEAD = MTW > 1 ? 1 : 2;  // steps whose floats wait in registers
   constexpr int PLANE = ROWS * 4;
-  static_assert(WM * WN == 8 && ROWS * 4 % THREADS == 0 && (!IS_GATED || NTW == 2) && !(IS_GATED && SPLIT), "");
+  constexpr int SPREAD = MTW == 1 ? (22 * PIECES + 6 * NTW - 1) / (6 * NTW) : MTW == 2 ? 6 : 4;  // vector instructions a matrix instruction
+  static_assert(WM * WN == 8 && ROWS % 16 == 0 && (!IS_GATED || NTW == 2) && !(IS_GATED && SPLIT), "");
   extern __shared__ bf16x8 lds[];  // [2][3][PLANE]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15, lg = lane >> 4;
@@ -415,41 +421,36 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __re
     const int n = IS_GATED ? n0 + (r >> 5) * 16 + (r & 15) : n0 + r;
     return w + (size_t)(min(n, N - 1) + (IS_GATED && (r & 16) ? N : 0)) * K;
   };
-  const float* src[PIECES];
-  int dst[PIECES];
+  // A thread's pieces: row r of the tile's, columns 4 c .. 4 c + 3 (eight lanes side by side ask for a line).  8 rows are a wave's, of one
+  // matrix: their first one's address is uniform.
+  const float* from[PIECES];
+  unsigned at[PIECES];  // floats from there
+  int dst[PIECES];      // halves of a place
 #pragma unroll
   for (int p = 0; p < PIECES; ++p) {
-    const int x = threadIdx.x + p * THREADS, r = x >> 2, c = x & 3;
-    src[p] = r < BM ? a + (size_t)min(m0 + r, M - 1) * K : weight(r - BM);
-    dst[p] = r * 4 + (c ^ (0x78 >> (r >> 1 & 6) & 3));
+    const int r0 = (wave * 64 + p * THREADS) % (ROWS * 8) >> 3, r = r0 + (lane >> 3), c = lane & 7;
+    const bool of_a = r0 < BM;
+    const int n = n0 + (IS_GATED ? ((r0 - BM) >> 5) * 16 + (r0 & 8) : r0 - BM);
+    from[p] = of_a ? a + (size_t)min(m0 + r0, M - 1) * K : w + (size_t)(min(n, N - 1) + (IS_GATED && ((r0 - BM) & 16) ? N : 0)) * K;
+    at[p] = (unsigned)(of_a ? min(m0 + r, M - 1) - min(m0 + r0, M - 1) : min(n + (lane >> 3), N - 1) - min(n, N - 1)) * K + c * 4;
+    dst[p] = (r * 4 + ((c >> 1) ^ (0x78 >> (r >> 1 & 6) & 3))) * 2 + (c & 1);
   }
-  floatx4 ahead[AHEAD][PIECES][2];
-  auto load = [&](int u, int st) {
-    const int at = min(st, all - 1), k = at * 32 + (threadIdx.x & 3) * 8;
-    if (at * 32 + 32 <= K) {
-#pragma unroll
-      for (int p = 0; p < PIECES; ++p)
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          if constexpr (VEC) ahead[u][p][half] = *reinterpret_cast<const floatx4*>(src[p] + k + 4 * half);
-          else ahead[u][p][half] = *reinterpret_cast<const floatx4_anywhere*>(src[p] + k + 4 * half);
-        }
-    } else {
-#pragma unroll
-      for (int p = 0; p < PIECES; ++p)
-#pragma unroll
-        for (int half = 0; half < 2; ++half) ahead[u][p][half] = ragged<VEC>(fetch<VEC>(src[p], k + 4 * half, K), k + 4 * half, K);
-    }
-  };
-  auto place = [&](int u, int buf) {
-    bf16x8* base = lds + buf * 3 * PLANE;
+  const int last = max(0, K / 32 - 1);
+  floatx4 ahead[AHEAD][PIECES];
+  auto load = [&](int u, int st) {  // whole steps; those past the last one repeat it and are not used
+    const int k = min(st, last) * 32;
 #pragma unroll
     for (int p = 0; p < PIECES; ++p) {
-      const Parts s = parts(ahead[u][p][0], ahead[u][p][1]);
-      base[dst[p]] = s.h;
-      base[PLANE + dst[p]] = s.m;
-      base[2 * PLANE + dst[p]] = s.l;
+      if constexpr (VEC) ahead[u][p] = *reinterpret_cast<const floatx4*>(from[p] + k + at[p]);
+      else ahead[u][p] = *reinterpret_cast<const floatx4_anywhere*>(from[p] + k + at[p]);
     }
+  };
+  auto place = [&](int u, int buf, int p) {
+    bf16x4* base = reinterpret_cast<bf16x4*>(lds + buf * 3 * PLANE) + dst[p];
+    const Parts4 s = parts(ahead[u][p]);
+    base[0] = s.h;
+    base[2 * PLANE] = s.m;
+    base[4 * PLANE] = s.l;
   };
   floatx4 acc[NTW][MTW], low[NTW][MTW], group[NTW][MTW], total[NTW][MTW];
 #pragma unroll
@@ -458,55 +459,168 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __re
     for (int j = 0; j < MTW; ++j) acc[i][j] = low[i][j] = group[i][j] = total[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < AHEAD; ++u) load(u, st0 + u);
-  place(0, 0);
+#pragma unroll
+  for (int p = 0; p < PIECES; ++p) place(0, 0, p);
   load(0, st0 + AHEAD);
-  int left = per, slice = 0;
+  int slice = 0;  // those that are done
   const int ra = (wm * MTW * 16 + lr) * 4 + (lg ^ (0x78 >> (lr >> 1 & 6) & 3));
   const int rw = (BM + wn * NTW * 16 + lr) * 4 + (lg ^ (0x78 >> (lr >> 1 & 6) & 3));
-  auto step = [&](int st, int u, int buf) {  // u: where st + 1 waits in registers; buf: where st lies in LDS
-    __syncthreads();
-    const bf16x8* base = lds + buf * 3 * PLANE;
-    bf16x8 av[MTW][3], wv[NTW][3];
+  bf16x8 av[3], wv[NTW][3];  // the operands of a step's first row tile
+  auto read_a = [&](int j, int buf, bf16x8 (&to)[3]) {
+#pragma unroll
+    for (int x = 0; x < 3; ++x) to[x] = lds[(buf * 3 + x) * PLANE + ra + j * 64];
+  };
+  auto read_first = [&](int buf, bf16x8 (&ws)[NTW][3], bf16x8 (&as)[3]) {  // the largest parts first: their product needs no others
 #pragma unroll
     for (int x = 0; x < 3; ++x) {
 #pragma unroll
-      for (int j = 0; j < MTW; ++j) av[j][x] = base[x * PLANE + ra + j * 64];
-#pragma unroll
-      for (int i = 0; i < NTW; ++i) wv[i][x] = base[x * PLANE + rw + i * 64];
+      for (int i = 0; i < NTW; ++i) ws[i][x] = lds[(buf * 3 + x) * PLANE + rw + i * 64];
+      as[x] = lds[(buf * 3 + x) * PLANE + ra];
     }
-    place(u, buf ^ 1);
-    load(u, st + 1 + AHEAD);
+  };
+  auto add_slice = [&](int j) {
+#pragma unroll
+    for (int i = 0; i < NTW; ++i) group[i][j] += acc[i][j] + low[i][j];
+  };
+  auto products = [&](int j, const bf16x8 (&ws)[NTW][3], const bf16x8 (&as)[3], auto first) {  // first: of a slice
 #pragma unroll
     for (int x = 0; x < 6; ++x)
 #pragma unroll
-      for (int i = 0; i < NTW; ++i)
+      for (int i = 0; i < NTW; ++i) {
+        floatx4& to = x == 0 ? acc[i][j] : low[i][j];  // the largest first, then the five in their order
+        const floatx4 before = first.value && x <= 1 ? floatx4{0.f, 0.f, 0.f, 0.f} : to;
+        to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[i][PART_W[(x + 5) % 6]], as[PART_A[(x + 5) % 6]], before, 0, 0, 0);
+      }
+  };
+  auto spread = [&]() {  // the vector unit's work between a row tile's matrix instructions, whose issue it does not hold up
 #pragma unroll
-        for (int j = 0; j < MTW; ++j) {
-          floatx4& to = x == 5 ? acc[i][j] : low[i][j];
-          to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i][PART_W[x]], av[j][PART_A[x]], to, 0, 0, 0);
-        }
-    if (--left == 0) {
-      left = per;
-      ++slice;
-#pragma unroll
-      for (int i = 0; i < NTW; ++i)
-#pragma unroll
-        for (int j = 0; j < MTW; ++j) {
-          group[i][j] += acc[i][j] + low[i][j];
-          acc[i][j] = low[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-          if (!SPLIT && (slice & 3) == 0) {
-            total[i][j] += group[i][j];
-            group[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-          }
-        }
+    for (int x = 0; x < 6 * NTW; ++x) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, SPREAD, 0);
     }
   };
-  int st = st0;
-  for (; st + 2 <= st1; st += 2) {
-    step(st, 1, 0);
-    step(st + 1, 0, 1);
+  auto group_done = [&]() {
+    if (SPLIT || (slice & 3)) return;
+#pragma unroll
+    for (int i = 0; i < NTW; ++i)
+#pragma unroll
+      for (int j = 0; j < MTW; ++j) {
+        total[i][j] += group[i][j];
+        group[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  auto slice_done = [&]() {  // added up where it ends
+#pragma unroll
+    for (int j = 0; j < MTW; ++j) {
+      add_slice(j);
+#pragma unroll
+      for (int i = 0; i < NTW; ++i) acc[i][j] = low[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    group_done();
+  };
+  constexpr std::true_type begins{};
+  constexpr std::false_type goes_on{};
+  const int whole = min(st1, K / 32);  // steps before one that K ends in
+  int st = st0, buf = 0, left = per;   // buf: where step st lies in LDS; left: steps until the slice ends
+  if constexpr (MTW == 1) {
+    // One row tile a wave: two workgroups on a compute unit fill each other's waits.
+    auto step = [&](int u) {  // u: where st + 1 waits in registers
+      __syncthreads();
+      read_first(buf, wv, av);
+#pragma unroll
+      for (int p = 0; p < PIECES; ++p) place(u, buf ^ 1, p);
+      products(0, wv, av, goes_on);
+      load(u, st + 1 + AHEAD);
+      __builtin_amdgcn_sched_group_barrier(0x100, 3 * NTW + 3, 0);
+      spread();
+      if (--left == 0) {
+        left = per;
+        ++slice;
+        slice_done();
+      }
+      ++st;
+      buf ^= 1;
+    };
+    while (st + 2 <= whole) {
+      buf = 0;
+      step(AHEAD - 1);
+      buf = 1;
+      step(0);
+    }
+    buf = 0;
+    if (st < whole) step(AHEAD - 1);
+  } else {
+    // One workgroup on a compute unit has to fill its own waits: the barrier of a step stands before its last row tile's products, when
+    // every read of this step's operands and every write of the next one's is done, so the next step's first operands are on their way
+    // under those products; a slice's sums are added up under the next slice's first products.
+    auto step = [&](auto first) {
+      bf16x8 as[MTW + 1][3], wn[NTW][3];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) as[0][x] = av[x];
+#pragma unroll
+      for (int j = 0; j < MTW; ++j) {
+        if (j + 1 < MTW) read_a(j + 1, buf, as[j + 1]);
+        else {
+          __syncthreads();
+          read_first(buf ^ 1, wn, av);
+        }
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p)
+          if (p * (MTW - 1) / PIECES == j) place(0, buf ^ 1, p);
+        if ((PIECES - 1) * (MTW - 1) / PIECES == j) load(0, st + 2);
+        if (first.value) add_slice(j);
+        products(j, wv, as[j], first);
+        if (j + 1 < MTW) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+        else __builtin_amdgcn_sched_group_barrier(0x100, 3 * NTW + 3, 0);
+        spread();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < NTW; ++i)
+#pragma unroll
+        for (int x = 0; x < 3; ++x) wv[i][x] = wn[i][x];
+      ++st;
+      buf ^= 1;
+    };
+    __syncthreads();
+    read_first(0, wv, av);
+    if constexpr (SPLIT) {  // a quarter of the slices: added up where they end, which takes fewer registers
+#pragma unroll 1
+      while (st < whole) {
+        step(goes_on);
+        if (--left) continue;
+        left = per;
+        slice_done();
+      }
+    } else {
+#pragma unroll 1
+      while (st < whole) {
+        step(begins);
+        group_done();
+        left = per;
+#pragma unroll 1
+        while (--left && st < whole) step(goes_on);
+        if (left == 0) ++slice;
+      }
+    }
   }
-  if (st < st1) step(st, 1, 0);
+  if (st < st1) {  // columns that are no whole step
+    const int k = st * 32 + (lane & 7) * 4;
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PIECES; ++p) {
+      ahead[0][p] = ragged<VEC>(fetch<VEC>(from[p] + at[p] - (lane & 7) * 4, k, K), k, K);
+      place(0, buf, p);
+    }
+    __syncthreads();
+    if (left == 0) slice_done();
+    read_first(buf, wv, av);
+#pragma unroll
+    for (int j = 0; j < MTW; ++j) {
+      if (j) read_a(j, buf, av);
+      products(j, wv, av, goes_on);
+    }
+  }
 #pragma unroll
   for (int j = 0; j < MTW; ++j) {
     const int m = m0 + (wm * MTW + j) * 16 + lr;
@@ -676,12 +790,16 @@ static int launch_tile(const float* a, const float* w, float* out, int M, int N,
 // Which kernel: the tile of rows of a by rows of w, and what a workgroup on every compute unit takes per 1,024 of K
 // beside the 4.5 us of a launch: the first round, every round.  Measured for N = 1,024 to 12,288 and K = 1,024 to 6,144 at 1 to 512 rows:
 // small tiles where the larger ones would leave compute units idle, large ones where operands would be read over and over
-// (N = 4,096, K = 1,024: 4 rows 8.3 us with the first and 53 with the last; N = 12,288, K = 2,048 at 512 rows 624 and 197,
-// with the fp32 instruction from memory 272).  The results are the same bit for bit.
+// (N = 4,096, K = 1,024: 4 rows 8.3 us with the first and 43 with tiles of 128; N = 12,288, K = 2,048 at 512 rows 624 and 165,
+// with the fp32 instruction from memory 272), and 96 rows where those leave fewer compute units idle (6,144 gated, 1,024 at 333
+// rows: tiles of 64 45.8, of 128 44.0, of 96 41.2; 12,288, 2,048 149.5, 162.8, 146.9).  The results are the same bit for bit.
 struct F32Tile { int rows, columns; float alone_us, round_us; };
 static const F32Tile f32_forms[] = {{16, 16, 3.4f, 4.5f},   {16, 16, 4.5f, 3.6f},   {16, 32, 6.2f, 5.6f},    {32, 16, 5.5f, 7.4f},
-                                    {32, 32, 7.8f, 9.f},    {64, 32, 12.f, 13.f},   {64, 64, 18.f, 14.5f},   {128, 128, 48.f, 48.f}};
-#define F32_FORMS 8
+                                    {32, 32, 7.8f, 9.f},    {64, 32, 12.f, 13.f},   {64, 64, 15.5f, 14.f},   {128, 128, 38.f, 41.f},
+                                    {96, 128, 35.f, 35.f}};
+#define F32_FORMS 9
+#define F32_SIDE 9            // between them
+static int f32_form(int i) { return i < F32_SIDE - 1 ? i + 1 : i + 2; }  // of f32_forms[i]
 #define F32_ONE_ROW_TILE 3  // so many of one row tile
 
 static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
@@ -690,18 +808,18 @@ static float f32_cost(const F32Tile& t, int M, int N, int K, int split) {
   return 4.5f + (float)K / 1024.f / (float)split * crowd * (t.alone_us + t.round_us * (float)(rounds - 1));
 }
 
-// form: 0: chosen here; else 1 + the index of a kernel, or after them the one of slices side by side (tests).
+// form: 0: chosen here; else the kernel `f32_form` numbers, or the one of slices side by side (tests).
 template <int MODE> static int gemm_f32(const float* a, const float* w, float* out, int M, int N, int K, int form, const LinkF32& link,
                                         hipStream_t stream) {
   if constexpr (MODE == PLAIN) {
-    if (form == F32_FORMS + 1 ? M <= 8 : form == 0 && side_by_side(M, N, K)) return launch_side<PLAIN>(a, w, out, M, N, K, link, stream);
+    if (form == F32_SIDE ? M <= 8 : form == 0 && side_by_side(M, N, K)) return launch_side<PLAIN>(a, w, out, M, N, K, link, stream);
   }
   if (form == 0) {
     float best = 0.f;
     for (int i = MODE == GATED ? 2 : 0; i < (link.ssq_in ? F32_ONE_ROW_TILE : F32_FORMS); ++i) {
       if (MODE == GATED && i == 3) continue;
       const float cost = f32_cost(f32_forms[i], M, MODE == GATED ? 2 * N : N, K, 1);
-      if (form == 0 || cost < best) { best = cost; form = i + 1; }
+      if (form == 0 || cost < best) { best = cost; form = f32_form(i); }
     }
   }
   if constexpr (MODE == GATED) {
@@ -711,6 +829,7 @@ template <int MODE> static int gemm_f32(const float* a, const float* w, float* o
       case 6: return launch_rows<4, 2, 4, 2, 1, GATED>(a, w, out, M, N, K, link, stream);
       case 7: return launch_tile<4, 2, 1, 2, true, false>(a, w, out, M, N, K, stream);
       case 8: return launch_tile<2, 4, 4, 2, true, false>(a, w, out, M, N, K, stream);
+      case 10: return launch_tile<2, 4, 3, 2, true, false>(a, w, out, M, N, K, stream);
     }
   } else {
     switch (form) {
@@ -726,6 +845,7 @@ template <int MODE> static int gemm_f32(const float* a, const float* w, float* o
       case 6: return launch_rows<4, 2, 4, 2, 1, PLAIN>(a, w, out, M, N, K, link, stream);
       case 7: return launch_tile<4, 2, 1, 2, false, false>(a, w, out, M, N, K, stream);
       case 8: return launch_tile<2, 4, 4, 2, false, false>(a, w, out, M, N, K, stream);
+      case 10: return launch_tile<2, 4, 3, 2, false, false>(a, w, out, M, N, K, stream);
     }
   }
   return AS_BAD_SHAPE;
@@ -747,7 +867,7 @@ extern "C" int as_gemm_f32(const float* a, const float* w, float* out, int M, in
 // stores: the same bits as the two kernels.
 extern "C" int as_gemm_f32_gated(const float* a, const float* w, float* out, int M, int N, int K, int form, hipStream_t stream) {
   if (M <= 0) return AS_OK;
-  if (N <= 0 || N > 0x3fffffff || K <= F32_NARROW || form < 0 || form > F32_FORMS) return AS_BAD_SHAPE;
+  if (N <= 0 || N > 0x3fffffff || K <= F32_NARROW || form < 0 || form > F32_FORMS + 1) return AS_BAD_SHAPE;
   return gemm_f32<GATED>(a, w, out, M, N, K, form, LinkF32{}, stream);
 }
 
@@ -779,8 +899,15 @@ extern "C" int as_gemm_f32_scaled(const float* scaled, const float* ssq, int str
 // N % 4 == 0.
 extern "C" int as_gemm_f32_split(const float* a, const float* w, float* sums, int M, int N, int K, int form, hipStream_t stream) {
   if (M <= 0) return AS_OK;
-  if (N <= 0 || (N & 3) || K <= F32_NARROW || (K & 3) || form < 0 || form > 2) return AS_BAD_SHAPE;
-  if (form == 0) form = f32_cost(f32_forms[6], M, N, K, F32_GROUPS) <= f32_cost(f32_forms[7], M, N, K, F32_GROUPS) ? 1 : 2;
+  if (N <= 0 || (N & 3) || K <= F32_NARROW || (K & 3) || form < 0 || form > 3) return AS_BAD_SHAPE;
+  if (form == 0) {
+    float best = 0.f;
+    for (int i = 6; i < F32_FORMS; ++i) {
+      const float cost = f32_cost(f32_forms[i], M, N, K, F32_GROUPS);
+      if (form == 0 || cost < best) { best = cost; form = i - 5; }
+    }
+  }
   if (form == 1) return launch_tile<4, 2, 1, 2, false, true>(a, w, sums, M, N, K, stream);
+  if (form == 3) return launch_tile<2, 4, 3, 2, false, true>(a, w, sums, M, N, K, stream);
   return launch_tile<2, 4, 4, 2, false, true>(a, w, sums, M, N, K, stream);
 }

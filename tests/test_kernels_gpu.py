@@ -1472,6 +1472,23 @@ def test_gemm_f32_gated_and_split_are_the_plain_product(ops, M, N, K):
         assert torch.equal(((s[0] + s[1]) + s[2]) + s[3], want)
 
 
+@pytest.mark.parametrize("M,N,K,shift", [(1, 4, 260, 0), (96, 128, 512, 0), (97, 132, 1028, 0), (95, 124, 544, 0), (193, 260, 2080, 0), (98, 70, 1025, 1), (130, 36, 287, 0)])
+def test_gemm_f32_tiles_of_96_rows(ops, M, N, K, shift):
+    """Tiles of 96 x 128 outputs, whole, gated and in four partial sums: the bits of strips straight from memory, where the tile's rows, its
+    columns and the last step of K are whole and where they are not, with slices of one step, of several, short and empty ones."""
+    torch.manual_seed(K + shift)
+    a, w = (torch.randn(rows * K + shift, device=DEV)[shift:].view(rows, K) for rows in (M, N))
+    blank = lambda *shape: torch.full(shape, float("nan"), device=DEV)  # noqa: E731
+    want = f32_product("as_gemm_f32", a, w, blank(M, N), 1)
+    assert torch.equal(f32_product("as_gemm_f32", a, w, blank(M, N), 10), want)
+    act = blank(M, N // 2)
+    ops.silu_mul(want, act)
+    assert torch.equal(f32_product("as_gemm_f32_gated", a, w, blank(M, N // 2), 10), act)
+    if K % 4 == 0 and N % 4 == 0:
+        s = f32_product("as_gemm_f32_split", a, w, blank(4, M, N), 3)
+        assert torch.equal(((s[0] + s[1]) + s[2]) + s[3], want)
+
+
 @pytest.mark.parametrize("M,shift", [(3, 0), (16, 0), (70, 0), (6, 1)])
 def test_gemm_f32_numbers_that_are_not_finite(ops, M, shift):
     """Infinities, NaN, numbers that round to infinity in 16 bits and tiny ones go where plain 32-bit arithmetic takes them, from every
