@@ -35,16 +35,45 @@ __device__ __forceinline__ bf16 finite_or_zero(bf16 v) {
   return (__builtin_bit_cast(unsigned short, v) & 0x7f80u) == 0x7f80u ? (bf16)0.f : v;
 }
 
+// What another lane of the wave holds, without a trip through LDS (a shuffle takes some 100 cycles, these under ten; a sum over
+// a wave is six of them in a row, and the short kernels of a decode step wait for nothing else).  All lanes of the wave take part.
+template <int CONTROL> __device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CONTROL, 0xf, 0xf, true));
+}
+#define DPP_XOR_1 0xb1        // quad_perm [1, 0, 3, 2]
+#define DPP_XOR_2 0x4e        // quad_perm [2, 3, 0, 1]
+#define DPP_HALF_MIRROR 0x141  // lane 7 - i of eight: i ^ 4 where the lanes of a quad hold the same
+#define DPP_MIRROR 0x140       // lane 15 - i of sixteen: i ^ 8 where those of eight hold the same
+#define DPP_ROTATE(N) (0x120 + (N))  // within sixteen; by 8: i ^ 8; by 4: i ^ 4 where lanes eight apart hold the same
+struct TwoHalves { float a, b; };
+__device__ __forceinline__ TwoHalves halves_32(float v) {  // in every lane: its half of the wave and the other one, in one order
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ TwoHalves halves_16(float v) {  // the same for the two sixteens of either half
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ float plus_32(float v) { const TwoHalves h = halves_32(v); return h.a + h.b; }
+__device__ __forceinline__ float plus_16(float v) { const TwoHalves h = halves_16(v); return h.a + h.b; }
+
+// Lane pairs 32 apart first, then 16, 8, 4, 2, 1.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-  return v;
+  v = plus_16(plus_32(v));
+  v += dpp<DPP_ROTATE(8)>(v);
+  v += dpp<DPP_ROTATE(4)>(v);
+  v += dpp<DPP_XOR_2>(v);
+  return v + dpp<DPP_XOR_1>(v);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, WAVE));
-  return v;
+  TwoHalves h = halves_32(v);
+  h = halves_16(fmaxf(h.a, h.b));
+  v = fmaxf(h.a, h.b);
+  v = fmaxf(v, dpp<DPP_ROTATE(8)>(v));
+  v = fmaxf(v, dpp<DPP_ROTATE(4)>(v));
+  v = fmaxf(v, dpp<DPP_XOR_2>(v));
+  return fmaxf(v, dpp<DPP_XOR_1>(v));
 }
 
 // Sum over a block of up to 1024 threads; every thread gets the result.  `red` is a

@@ -133,8 +133,7 @@ __device__ __forceinline__ void link_epilogue(const NormLink& link, float* x, fl
       }
     }
   }
-  ss += __shfl_xor(ss, 16, 64);  // the four lanes that hold the strip's 16 columns of row m
-  ss += __shfl_xor(ss, 32, 64);
+  ss = plus_32(plus_16(ss));  // the four lanes that hold the strip's 16 columns of row m
   if ((threadIdx.x & 63) < 16 && m < M) link.ssq_out[(size_t)m * nstrips + strip] = ss;
 }
 
@@ -364,8 +363,11 @@ __global__ __launch_bounds__(PIPE_WAVES * 64) void gemm_bf16_skinny_pipe_kernel(
       float ss = 0.f;
       if (row < M)
         for (int j = j0; j < link.strips_in; j += 32) ss += link.ssq_in[(size_t)row * link.strips_in + j];
-#pragma unroll
-      for (int off = 1; off < 32; off <<= 1) ss += __shfl_xor(ss, off, 64);
+      ss += dpp<DPP_XOR_1>(ss);
+      ss += dpp<DPP_XOR_2>(ss);
+      ss += dpp<DPP_HALF_MIRROR>(ss);
+      ss += dpp<DPP_MIRROR>(ss);
+      ss = plus_16(ss);
       if (j0 == 0) inv_rms[row] = row < M ? 1.0f / sqrtf(ss / (float)K + link.eps) : 0.f;
     }
   }
