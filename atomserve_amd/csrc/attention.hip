@@ -322,66 +322,65 @@ __device__ __forceinline__ float quad_rows_sum(float v) {
 // The keys and values of one step (32 keys, two 16-key pieces of pages) of one kv head, as the
 // MFMA operands of this lane: keys as rows of A (16 bytes of the head of key KEY_OF_ROW(tile,
 // lane % 16)), values as the transposed page gives them (the lane group's 8 keys of one
-// coordinate: 16 bytes).  A piece that starts at or beyond `end` is not read and counts as zeros.
+// coordinate: 16 bytes).  A second piece that starts at or beyond `end` repeats the first one: finite numbers, whose weights are zero.
 // Loading the next step before computing the current one keeps memory busy while the matrix
-// cores work.
+// cores work.  PAGE: tokens of a page where the compiler knows them (divisions by another number are 30 instructions each), or 0;
+// `kb` and `table` are uniform over the wave, so that pages are found by its scalar unit.
 template <int DC>
 struct KVStep {
   bf16x8_t k[2][DC];
   bf16x8_t v[2 * DC];
 };
 
-template <int DC>
+template <int DC, int PAGE>
 __device__ __forceinline__ void load_kv_step(KVStep<DC>& st, const bf16* __restrict__ k_pages,
                                              const bf16* __restrict__ v_pages, const int* __restrict__ table,
-                                             int kb, int end, int KV, int kvh, int bs, int col, int grp) {
+                                             int kb, int end, int KV, int kvh, int page_size, int col, int grp) {
   constexpr int D = DC * 32, DT = DC * 2;
-  const bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int bs = PAGE ? PAGE : page_size;
   size_t head[2];
   int off0[2];
 #pragma unroll
   for (int pc = 0; pc < 2; ++pc) {  // uniform over the wave
-    const int key0 = kb + 16 * pc;
-    const int page = key0 < end ? table[key0 / bs] : 0;
-    head[pc] = ((size_t)page * KV + kvh) * bs * D;
+    const int key0 = pc == 0 || kb + 16 < end ? kb + 16 * pc : kb;
+    head[pc] = ((size_t)table[key0 / bs] * KV + kvh) * bs * D;
     off0[pc] = key0 % bs;
   }
   {  // keys: rows 0-7 of both tiles lie in the first piece, rows 8-15 in the second
     const int pc = col >> 3;
-    const bool live = kb + 16 * pc < end;
-    const bf16* krow = k_pages + (pc ? head[1] : head[0]) + (size_t)((pc ? off0[1] : off0[0]) + (KEY_OF_ROW(0, col) & 15)) * D + grp * 8;
+    const bf16* krow = k_pages + (pc ? head[1] + (size_t)off0[1] * D : head[0] + (size_t)off0[0] * D) + ((KEY_OF_ROW(0, col) & 15) * D + grp * 8);
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-      for (int c = 0; c < DC; ++c)
-        st.k[tt][c] = live ? *reinterpret_cast<const bf16x8_t*>(krow + (size_t)tt * 4 * D + c * 32) : zero;
+      for (int c = 0; c < DC; ++c) st.k[tt][c] = *reinterpret_cast<const bf16x8_t*>(krow + tt * 4 * D + c * 32);
   }
   {  // values: keys 8 grp .. 8 grp + 7 of coordinates col, col + 16, ...  One instruction of the wave reads two runs of
      // 512 bytes, every 128-byte line whole, and a decode step reads a value once: marked as not to be kept (batch 64
      // of Qwen3-8B sizes 8,542 -> 8,872 tokens/s).  With pages of more than 32 tokens a step's 32 keys are part of a line,
      // which the next step needs again: no mark there.  The keys' loads share their lines in pairs and stay as they are.
-    const int pc = grp >> 1;
-    const bool live = kb + 16 * pc < end;
-    const bf16* vcol = v_pages + (pc ? head[1] : head[0]) + (pc ? off0[1] : off0[0]) + 8 * (grp & 1) + (size_t)col * bs;
+    const bf16* vcol = v_pages + (grp >> 1 ? head[1] + off0[1] : head[0] + off0[0]) + (8 * (grp & 1) + col * bs);
     if (bs <= 32) {  // uniform over the grid: two loops, so that neither holds a choice per load
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
-        st.v[dt] = live ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(vcol + (size_t)dt * 16 * bs)) : zero;
+        st.v[dt] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(vcol + (size_t)dt * 16 * bs));
     } else {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-        st.v[dt] = live ? *reinterpret_cast<const bf16x8_t*>(vcol + (size_t)dt * 16 * bs) : zero;
+      for (int dt = 0; dt < DT; ++dt) st.v[dt] = *reinterpret_cast<const bf16x8_t*>(vcol + (size_t)dt * 16 * bs);
     }
   }
 }
 
 // FRESH: the kernel takes the projection's output qkv [T, H + 2 KV, D] instead of finished queries
 // and does what the norm-rotate-store kernel does before a decode step, for a step whose tokens
-// are their own rows: each workgroup norms and rotates the queries of its group in registers (the
-// partner i + D/2 of coordinate i lies in the same lane when D % 64 == 0), and the workgroup whose
+// are their own rows: each workgroup norms and rotates the queries of its group, and the workgroup whose
 // partition holds the token's own position makes the token's key and value, writes them to the
-// pages and attends them from LDS, so nothing waits for those writes.  Same arithmetic as
+// pages and attends them from LDS, so nothing waits for those writes.  A head is one wave's work (a lane
+// has coordinates i and i + D/2), the waves take the group's heads, the key and the value in turn, and LDS hands the
+// queries to all of them as matrix operands.  Same arithmetic as
 // qk_norm_rope_store_bf16x8_kernel; the squares are summed in another order.
+// What bounds a short context is the instructions of one wave, of which one that is alone on its SIMD issues one in 4 to
+// 8 cycles: with every wave norming all queries as operands (16 columns, most of them empty groups' padding), pages found by divisions in
+// the vector unit and partial outputs merged float by float, one token of Qwen3-0.6B sizes behind 100 took 7.6 us, now 6.2, behind 800 12.0 and 10.4.
 struct FreshQKV {
   const bf16* qkv;
   const void* qw;      // gains of the per-head norms, D values each, bf16 or fp32
@@ -394,31 +393,22 @@ struct FreshQKV {
   int store;           // 0: queries only, the pages already hold the token's key and value
 };
 
-__device__ __forceinline__ void load_gains8(const float* w, float* g) {
-  const float4 a = *reinterpret_cast<const float4*>(w), b = *reinterpret_cast<const float4*>(w + 4);
-  g[0] = a.x; g[1] = a.y; g[2] = a.z; g[3] = a.w; g[4] = b.x; g[5] = b.y; g[6] = b.z; g[7] = b.w;
-}
-__device__ __forceinline__ void load_gains8(const bf16* w, float* g) {
-  const bf16x8_t v = *reinterpret_cast<const bf16x8_t*>(w);
-#pragma unroll
-  for (int j = 0; j < 8; ++j) g[j] = (float)v[j];
-}
-
 // D / 32; FRESH 0: finished queries, 1: qkv with bf16 gains, 2: with fp32 gains; SEE 0: a window at most (nothing of the rest of
-// `sight` is read), 1: kept first tokens, chunks, a sink and fp32 outputs too, 2: also capped scores
-template <int DC, int FRESH, int SEE, bool TURNED = false>
+// `sight` is read), 1: kept first tokens, chunks, a sink and fp32 outputs too, 2: also capped scores; PAGE: tokens of a page, or 0 for any
+template <int DC, int FRESH, int SEE, bool TURNED, int PAGE>
 __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ items, const int* __restrict__ positions, const int* __restrict__ tok_row,
     const int* __restrict__ block_tables, int table_width, bf16* __restrict__ out, float* __restrict__ part_m,
-    float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int bs, float scale, Sight sight,
+    float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int page_size, float scale, Sight sight,
     int part_size, int P, int cus, int share, FreshQKV fresh) {
   // share > 1: every `share` consecutive kv heads named here are one head of the pages (a group of more query heads
   // than a workgroup takes, cut into several); the pages then hold KV / share heads.
   constexpr int D = DC * 32, DT = DC * 2;  // DT: tiles of 16 output coordinates
-  extern __shared__ float smem[];          // [4][16] m, [4][16] l, [4][D][G] acc
+  constexpr int LD = D + 4;                // a partial output's row in LDS
+  extern __shared__ __align__(16) float smem[];  // [4][16] m, [4][16] l, [4][G][LD] acc; FRESH: [G][D + 8] bf16 queries
   __shared__ __align__(16) bf16 fresh_kv[2][256];  // FRESH: the new token's key and value
-  const int G = H / KV;
+  const int G = H / KV, bs = PAGE ? PAGE : page_size;
   int item = blockIdx.x, kvh = blockIdx.y;
   const int part = blockIdx.z;
   if (!TURNED && P == 1) {
@@ -462,7 +452,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   auto first_key = [&](int at) { return SEE >= 1 ? 32 * (at < kept_steps ? at : at - kept_steps + base) : at; };
   const int h0 = kvh * G;
   const int page_heads = KV / share, page_head = kvh / share;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;  // col: head within the group (and key row of A)
 
   if (from >= to) {  // an empty partition (P > 1 only): mark it so for the reduce
@@ -477,122 +467,103 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   }
   const int* table = block_tables + (size_t)(tok_row ? tok_row[t] : t) * table_width;  // null: token t is row t
 
-  // Everything is asked for before anything is waited for: the queries (FRESH: as the projection
-  // left them, with the gains and angles of this lane's coordinates; in the workgroup that holds the
-  // token's own position, wave 0 the new key and wave 1 the new value), then the first keys and values.
-  constexpr int HC = DC / 2, HALF = D / 2, PAIRS = (HALF + WAVE - 1) / WAVE;
+  // Everything is asked for before anything is waited for: the queries (FRESH: this wave's heads as the projection
+  // left them, with their gains and angles), then the first keys and values.
+  constexpr int HALF = D / 2, PAIRS = (HALF + WAVE - 1) / WAVE, TURNS = FRESH ? 5 : 1;  // 16 heads, a key and a value over four waves
   using W = typename std::conditional<FRESH == 2, float, bf16>::type;  // the gains' type
   bf16x8_t qop[DC];
   const bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
   const size_t row = (size_t)t * (H + 2 * KV);  // FRESH: the token's heads in qkv
-  {
-    const bf16* qrow = FRESH ? fresh.qkv + (row + h0 + min(col, G - 1)) * D + grp * 8
-                             : q + ((size_t)t * H + h0 + min(col, G - 1)) * D + grp * 8;
+  [[maybe_unused]] const bool fresh_here = FRESH && fresh.store && pos >= k0 && pos < k1;  // these keys include the token's own
+  [[maybe_unused]] const int jobs = G + (fresh_here ? 2 : 0);  // the group's heads, then the key and the value
+  [[maybe_unused]] bf16 ha[TURNS][PAIRS], hb[TURNS][PAIRS];
+  [[maybe_unused]] float ga[2][PAIRS], gb[2][PAIRS];  // gains of a query and of the key
+  [[maybe_unused]] float2 angle[PAIRS];
+  [[maybe_unused]] int slot = -1;
+  if constexpr (FRESH != 0) {
+#pragma unroll
+    for (int n = 0; n < TURNS; ++n) {
+      const int job = wave + 4 * n;
+      if (job < jobs) {  // uniform over the wave
+        const bf16* src = fresh.qkv + (row + (job < G ? h0 + job : H + kvh + (job - G) * KV)) * D;
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p) {
+          const int i = min(lane + p * WAVE, HALF - 1);
+          ha[n][p] = src[i];
+          hb[n][p] = src[i + HALF];
+        }
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < PAIRS; ++p) {
+      const int i = min(lane + p * WAVE, HALF - 1);
+      ga[0][p] = (float)((const W*)fresh.qw)[i];
+      gb[0][p] = (float)((const W*)fresh.qw)[i + HALF];
+      ga[1][p] = (float)((const W*)fresh.kw)[i];
+      gb[1][p] = (float)((const W*)fresh.kw)[i + HALF];
+      angle[p] = fresh.cs[(size_t)t * HALF + i];
+    }
+    if (fresh_here) slot = fresh.slots[t];
+  } else {
+    const bf16* qrow = q + ((size_t)t * H + h0 + min(col, G - 1)) * D + grp * 8;
 #pragma unroll
     for (int c = 0; c < DC; ++c) qop[c] = col < G ? *reinterpret_cast<const bf16x8_t*>(qrow + c * 32) : zero;
   }
-  [[maybe_unused]] float gain[FRESH ? DC * 8 : 1];
-  [[maybe_unused]] float4 angle[FRESH ? HC * 4 : 1];  // (cos, sin) of two pairs each
-  [[maybe_unused]] bool fresh_here = false;           // this workgroup's keys include the token's own
-  [[maybe_unused]] int slot = -1;
-  [[maybe_unused]] bf16 ka[PAIRS], kb2[PAIRS], vv[2 * PAIRS];
-  [[maybe_unused]] float gka[PAIRS], gkb[PAIRS];
-  [[maybe_unused]] float2 kcs[PAIRS];
-  if constexpr (FRESH != 0) {
-#pragma unroll
-    for (int c = 0; c < HC; ++c) {
-      const int i0 = c * 32 + grp * 8;
-      load_gains8((const W*)fresh.qw + i0, &gain[c * 8]);
-      load_gains8((const W*)fresh.qw + i0 + HALF, &gain[(c + HC) * 8]);
-      const float4* cs4 = reinterpret_cast<const float4*>(fresh.cs + (size_t)t * HALF + i0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) angle[c * 4 + j] = cs4[j];
-    }
-    fresh_here = fresh.store && pos >= k0 && pos < k1;  // the same for the whole workgroup
-    if (fresh_here && wave == 0) {
-      slot = fresh.slots[t];
-      const bf16* src = fresh.qkv + (row + H + kvh) * D;
-#pragma unroll
-      for (int p = 0; p < PAIRS; ++p) {
-        const int i = min(lane + p * WAVE, HALF - 1);
-        ka[p] = src[i];
-        kb2[p] = src[i + HALF];
-        gka[p] = (float)((const W*)fresh.kw)[i];
-        gkb[p] = (float)((const W*)fresh.kw)[i + HALF];
-        kcs[p] = fresh.cs[(size_t)t * HALF + i];
-      }
-    } else if (fresh_here && wave == 1) {
-      slot = fresh.slots[t];
-      const bf16* src = fresh.qkv + (row + H + KV + kvh) * D;
-#pragma unroll
-      for (int p = 0; p < 2 * PAIRS; ++p) vv[p] = src[min(lane + p * WAVE, D - 1)];
-    }
-  }
   KVStep<DC> cur, nxt;
   int at = from + NEXT * wave;
-  if (at < to) load_kv_step<DC>(cur, k_pages, v_pages, table, first_key(at), bound, page_heads, page_head, bs, col, grp);
+  if (at < to) load_kv_step<DC, PAGE>(cur, k_pages, v_pages, table, first_key(at), bound, page_heads, page_head, bs, col, grp);
 
   if constexpr (FRESH != 0) {
-    // the queries of this lane's head: norm over the head (its D values lie in four lanes), rotation
-    float ss = 0.f;
+    bf16* const queries = reinterpret_cast<bf16*>(smem + 128 + 4 * LD * G);
+    const size_t head = slot >= 0 ? ((size_t)(slot / bs) * KV + kvh) * bs * D : 0;
 #pragma unroll
-    for (int c = 0; c < DC; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) ss += (float)qop[c][j] * (float)qop[c][j];
-    ss += __shfl_xor(ss, 16, WAVE);
-    ss += __shfl_xor(ss, 32, WAVE);
-    const float inv = 1.0f / sqrtf(ss / (float)D + fresh.eps);
-#pragma unroll
-    for (int c = 0; c < HC; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float a = (float)qop[c][j] * inv * gain[c * 8 + j];
-        const float b = (float)qop[c + HC][j] * inv * gain[(c + HC) * 8 + j];
-        const float4 cs2 = angle[c * 4 + j / 2];
-        const float cc = (j & 1) ? cs2.z : cs2.x, sn = (j & 1) ? cs2.w : cs2.y;
-        qop[c][j] = (bf16)(a * cc - b * sn);
-        qop[c + HC][j] = (bf16)(b * cc + a * sn);
-      }
-    if (col >= G) {
-#pragma unroll
-      for (int c = 0; c < DC; ++c) qop[c] = zero;
-    }
-    if (fresh_here) {
-      const size_t head = slot >= 0 ? ((size_t)(slot / bs) * KV + kvh) * bs * D : 0;
-      if (wave == 0) {  // the key: norm and rotation as for the queries, one wave over the pairs
-        float ks = 0.f;
-#pragma unroll
-        for (int p = 0; p < PAIRS; ++p)
-          if (lane + p * WAVE < HALF) ks += (float)ka[p] * (float)ka[p] + (float)kb2[p] * (float)kb2[p];
-        ks = wave_sum(ks);
-        const float kinv = 1.0f / sqrtf(ks / (float)D + fresh.eps);
-        bf16* dst = fresh.k_store + head + (size_t)(slot % bs) * D;
+    for (int n = 0; n < TURNS; ++n) {
+      const int job = wave + 4 * n;
+      if (job > G && job < jobs) {  // the value, as it is; its page is stored transposed
+        bf16* vt = fresh.v_store + head + slot % bs;
 #pragma unroll
         for (int p = 0; p < PAIRS; ++p) {
           const int i = lane + p * WAVE;
           if (i < HALF) {
-            const float a = (float)ka[p] * kinv * gka[p], b = (float)kb2[p] * kinv * gkb[p];
-            const bf16 ra = finite_or_zero((bf16)(a * kcs[p].x - b * kcs[p].y));
-            const bf16 rb = finite_or_zero((bf16)(b * kcs[p].x + a * kcs[p].y));
-            fresh_kv[0][i] = ra;
-            fresh_kv[0][i + HALF] = rb;
-            if (slot >= 0) { dst[i] = ra; dst[i + HALF] = rb; }
+            const bf16 ra = finite_or_zero(ha[n][p]), rb = finite_or_zero(hb[n][p]);
+            fresh_kv[1][i] = ra;
+            fresh_kv[1][i + HALF] = rb;
+            if (slot >= 0) { vt[(size_t)i * bs] = ra; vt[(size_t)(i + HALF) * bs] = rb; }
           }
         }
-      } else if (wave == 1) {  // the value, as it is; its page is stored transposed
-        bf16* vt = fresh.v_store + head + slot % bs;
+      } else if (job < jobs) {  // a query or the key: norm and rotation, one wave over the pairs
+        const int is_key = job == G;
+        float ss = 0.f;
 #pragma unroll
-        for (int p = 0; p < 2 * PAIRS; ++p) {
+        for (int p = 0; p < PAIRS; ++p)
+          if (lane + p * WAVE < HALF) ss += (float)ha[n][p] * (float)ha[n][p] + (float)hb[n][p] * (float)hb[n][p];
+        ss = wave_sum(ss);
+        const float inv = 1.0f / sqrtf(ss / (float)D + fresh.eps);
+#pragma unroll
+        for (int p = 0; p < PAIRS; ++p) {
           const int i = lane + p * WAVE;
-          if (i < D) {
-            const bf16 rv = finite_or_zero((bf16)vv[p]);
-            fresh_kv[1][i] = rv;
-            if (slot >= 0) vt[(size_t)i * bs] = rv;
+          if (i < HALF) {
+            const float a = (float)ha[n][p] * inv * (is_key ? ga[1][p] : ga[0][p]), b = (float)hb[n][p] * inv * (is_key ? gb[1][p] : gb[0][p]);
+            bf16 ra = (bf16)(a * angle[p].x - b * angle[p].y), rb = (bf16)(b * angle[p].x + a * angle[p].y);
+            if (is_key) {
+              ra = finite_or_zero(ra);
+              rb = finite_or_zero(rb);
+              fresh_kv[0][i] = ra;
+              fresh_kv[0][i + HALF] = rb;
+              bf16* dst = fresh.k_store + head + (size_t)(slot % bs) * D;
+              if (slot >= 0) { dst[i] = ra; dst[i + HALF] = rb; }
+            } else {
+              queries[job * (D + 8) + i] = ra;
+              queries[job * (D + 8) + i + HALF] = rb;
+            }
           }
         }
       }
-      __syncthreads();
     }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < DC; ++c)
+      qop[c] = col < G ? *reinterpret_cast<const bf16x8_t*>(queries + min(col, G - 1) * (D + 8) + c * 32 + grp * 8) : zero;
   }
   f32x4_t o[DT];
 #pragma unroll
@@ -602,7 +573,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   for (; at < to; at += 4 * NEXT) {
     const int kb = first_key(at);
     const bool more = at + 4 * NEXT < to;
-    if (more) load_kv_step<DC>(nxt, k_pages, v_pages, table, first_key(at + 4 * NEXT), bound, page_heads, page_head, bs, col, grp);
+    if (more) load_kv_step<DC, PAGE>(nxt, k_pages, v_pages, table, first_key(at + 4 * NEXT), bound, page_heads, page_head, bs, col, grp);
     if constexpr (FRESH != 0) {
       if (fresh_here && pos >= kb && pos < kb + 32) {  // this wave's step holds the token itself: take it from LDS
         const int nth = pos - kb;  // = KEY_OF_ROW(tile, row) for
@@ -677,13 +648,11 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   // ---- merge the four waves
   float* sm = smem;
   float* sl = smem + 64;
-  float* so = smem + 128;  // [4][D][G]
+  float* so = smem + 128;  // [4][G][LD]
   if (grp == 0 && col < G) { sm[wave * 16 + col] = m; sl[wave * 16 + col] = l; }
   if (col < G) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) so[((size_t)wave * D + dt * 16 + 4 * grp + r) * G + col] = o[dt][r];
+    for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4_t*>(so + (wave * G + col) * LD + dt * 16 + 4 * grp) = o[dt];
   }
   __syncthreads();
   for (int idx = tid; idx < G * D; idx += 256) {
@@ -696,7 +665,7 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     for (int w = 0; w < 4; ++w) {
       const float mw = sm[w * 16 + g];
       const float e = (mw == NEG_INF) ? 0.f : __expf(mw - mxw);
-      num += so[((size_t)w * D + d) * G + g] * e;
+      num += so[(w * G + g) * LD + d] * e;
       den += sl[w * 16 + g] * e;
     }
     const int h = h0 + g;
@@ -1278,18 +1247,28 @@ static int launch_decode_mfma(const void* q, const void* k_pages, const void* v_
   if (share < 1 || KV % share || (fresh && share != 1)) return AS_BAD_SHAPE;
   const bool turned = P > 1 && num_items > 8 && num_items <= 65535 && needed_sight(sight) == 0;
   const dim3 grid = turned ? dim3(KV, num_items, P) : dim3(num_items, KV, P);
-  const size_t shmem = sizeof(float) * (size_t)(128 + 4 * D * G);
-  if (shmem + 1024 > (64u << 10)) return AS_BAD_SHAPE;  // wide heads in large groups: the general kernel's
+  if (sizeof(float) * (size_t)(128 + 4 * D * G) + 1024 > (64u << 10)) return AS_BAD_SHAPE;  // wide heads in large groups: the general kernel's
+  const size_t shmem = sizeof(float) * (size_t)(128 + 4 * (D + 4) * G) + (fresh ? sizeof(bf16) * (size_t)(D + 8) * G : 0);
   const FreshQKV none = {};
   const int see = needed_sight(sight);
-#define LAUNCH4(DCV, FRESHV, SEEV, TURNEDV)                                                               \
-  attn_decode_mfma_kernel<DCV, FRESHV, SEEV, TURNEDV><<<grid, 256, shmem, stream>>>(                      \
+  // Pages of 16 tokens, the engine's own, have instances of their own (see `load_kv_step`).
+#define LAUNCH5(DCV, FRESHV, SEEV, TURNEDV, PAGEV)                                                        \
+  do {                                                                                                    \
+    const auto kernel = attn_decode_mfma_kernel<DCV, FRESHV, SEEV, TURNEDV, PAGEV>;                       \
+    if (shmem + 1024 > 65536 &&                                                                           \
+        hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) \
+      return AS_LAUNCH_FAILED;                                                                            \
+    kernel<<<grid, 256, shmem, stream>>>(                                                                 \
       (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, items, positions, tok_row, block_tables, \
       table_width, (bf16*)out, part_m, part_l, part_acc, H, KV, bs, scale, sight, part_size, P,           \
-      compute_units(), share, FRESHV ? *fresh : none)
-#define LAUNCH(DCV, FRESHV)                       \
-  if (turned) LAUNCH4(DCV, FRESHV, 0, true);      \
-  else LAUNCH4(DCV, FRESHV, 0, false)
+      compute_units(), share, FRESHV ? *fresh : none);                                                    \
+  } while (0)
+#define LAUNCH4(DCV, FRESHV, SEEV, TURNEDV) LAUNCH5(DCV, FRESHV, SEEV, TURNEDV, 0)
+#define LAUNCH(DCV, FRESHV)                                        \
+  if (turned && bs == 16) LAUNCH5(DCV, FRESHV, 0, true, 16);       \
+  else if (turned) LAUNCH5(DCV, FRESHV, 0, true, 0);               \
+  else if (bs == 16) LAUNCH5(DCV, FRESHV, 0, false, 16);           \
+  else LAUNCH5(DCV, FRESHV, 0, false, 0)
 #define LAUNCH_PLAIN(DCV)                          \
   if (see == 2) LAUNCH4(DCV, 0, 2, false);         \
   else if (see == 1) LAUNCH4(DCV, 0, 1, false);    \
@@ -1321,6 +1300,7 @@ static int launch_decode_mfma(const void* q, const void* k_pages, const void* v_
 #undef LAUNCH_PLAIN
 #undef LAUNCH
 #undef LAUNCH4
+#undef LAUNCH5
   if (hipGetLastError() != hipSuccess) return AS_LAUNCH_FAILED;
   if (P > 1) {
     attn_reduce_kernel<bf16><<<dim3(num_items, H), D <= 64 ? 64 : (D <= 128 ? 128 : 256), 0, stream>>>(

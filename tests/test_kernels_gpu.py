@@ -986,6 +986,37 @@ def test_decode_step_from_fresh_projections(ops, H, KV, D, bs, gain, window, par
                                   scale, window, max(lens), part)  # fmt: skip
 
 
+@pytest.mark.parametrize("G,KV,D", [(1, 3, 128), (3, 2, 64), (5, 2, 128), (7, 1, 192), (15, 1, 256), (16, 2, 128)])
+def test_a_decode_step_gives_the_same_bits_at_every_page_size(ops, G, KV, D):
+    """Pages of 16 tokens, which have kernels of their own, and of other sizes: a group's heads, the key and the value over four waves in
+    one to five turns, partial outputs that need more LDS than a launch gets unasked.  The same keys, values and sums whatever the page size, with
+    contexts whose last 16 keys are whole, begun and absent; against the two kernels with the tolerance of the other cases."""
+    H, lens, scale, T = G * KV, [1, 15, 16, 17, 47, 48, 49, 333], D**-0.5, 8
+    g = torch.Generator().manual_seed(G)
+    keys, values = (torch.randn(T, 336, KV, D, generator=g).to(BF16).to(DEV) for _ in range(2))
+    qkv = (torch.randn(T, H + 2 * KV, D, generator=g) * 2).to(BF16).to(DEV)
+    qw, kw = (torch.randn(D, generator=g) + 1).to(BF16).to(DEV), (torch.randn(D, generator=g) + 1).to(BF16).to(DEV)
+    cs = torch.randn(T, D // 2, 2, generator=g).to(DEV)
+    positions, seen = i32([n - 1 for n in lens]), []
+    for bs in (16, 48, 112):
+        per = 336 // bs
+        tables = torch.randperm(T * per, generator=g).view(T, per).to(torch.int32).to(DEV)
+        k_pages, v_pages = torch.empty(T * per, KV, bs, D, dtype=BF16, device=DEV), torch.empty(T * per, KV, D, bs, dtype=BF16, device=DEV)
+        k_pages[tables.long()] = keys.view(T, per, bs, KV, D).permute(0, 1, 3, 2, 4)
+        v_pages[tables.long()] = values.view(T, per, bs, KV, D).permute(0, 1, 3, 4, 2)
+        slots = i32([int(tables[i, (n - 1) // bs]) * bs + (n - 1) % bs for i, n in enumerate(lens)])
+        q2, out2, k2, v2 = torch.empty(T, H, D, dtype=BF16, device=DEV), torch.empty(T, H, D, dtype=BF16, device=DEV), k_pages.clone(), v_pages.clone()
+        ops.qk_norm_rope_store(qkv, qw, kw, cs, slots, q2, k2, v2, H, KV, 1e-6)
+        ops.attn_single_query(q2, k2, v2, None, positions, None, tables, out2, scale, 0, max(lens))
+        for part in (352, 64):
+            out = torch.full((T, H, D), float("nan"), dtype=BF16, device=DEV)
+            ops.attn_decode_fresh(qkv, qw, kw, cs, slots, 1e-6, True, k_pages, v_pages, positions, tables, out, H, scale, 0, max(lens), part)
+            assert torch.allclose(out.float(), out2.float(), atol=2e-2, rtol=2e-2)
+            seen.append((out, k_pages[tables.long()].permute(0, 1, 3, 2, 4).reshape(T, 336, KV, D), v_pages[tables.long()].permute(0, 1, 4, 2, 3).reshape(T, 336, KV, D)))
+    for n, one in enumerate(seen):
+        assert all(torch.equal(a, b) for a, b in zip(one, seen[n % 2]))
+
+
 @pytest.mark.parametrize("H,KV,D,bs,window", [(16, 8, 128, 16, 0), (6, 2, 64, 32, 0), (16, 1, 128, 48, 0), (8, 2, 128, 16, 40), (8, 8, 64, 16, 1)])
 @pytest.mark.parametrize("part", [None, 32, 128])
 def test_decode_step_from_fresh_projections_fp32(ops, H, KV, D, bs, window, part):
