@@ -245,37 +245,42 @@ __global__ __launch_bounds__(256) void attn_single_query_kernel(
 
 // Merge the partitions of each (item, head): out = sum_p acc_p e^(m_p - M) / sum_p l_p e^(m_p - M).
 // One workgroup per (item, head), one thread per output coordinate; every thread derives the
-// weights itself (P small values, all loads independent), so there is one round of loads for
-// the weights and one for the sums.  Empty partitions carry m = -inf, l = 0 and acc = 0.
-#define REDUCE_MAX_P 64
+// weights itself, a lane a partition, and hands them round by lane reads: one round of loads for the weights and one, which
+// waits for no other, for the sums (a loop over the partitions waited for its loads in each: one request of 800 tokens in 25 partitions,
+// 16 heads of 128, attention and merge 13.2 -> 9.1 us, in 7 partitions 10.1 -> 8.6).  Empty partitions carry m = -inf, l = 0 and acc = 0.
 template <typename T>
 __global__ __launch_bounds__(256) void attn_reduce_kernel(const int* __restrict__ items,
                                                           const float* __restrict__ part_m,
                                                           const float* __restrict__ part_l,
                                                           const float* __restrict__ part_acc, T* __restrict__ out,
                                                           int H, int D, int P, int sink, const float* __restrict__ sinks, int wide) {
-  const int item = blockIdx.x, h = blockIdx.y;
+  const int item = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & (WAVE - 1);
   const size_t base = ((size_t)item * H + h) * P;
   float mx = NEG_INF;
-  for (int p = 0; p < P; ++p) mx = fmaxf(mx, part_m[base + p]);
+  for (int p = lane; p < P; p += WAVE) mx = fmaxf(mx, part_m[base + p]);
+  mx = wave_max(mx);
   const float sk = sink_score(sink, sinks, h);
   if (sink) mx = fmaxf(mx, sk);
-  float den = sink ? fexp<T>(sk - mx) : 0.f;
-  for (int p = 0; p < P; ++p) {
-    const float mp = part_m[base + p];
-    den += (mp == NEG_INF) ? 0.f : part_l[base + p] * fexp<T>(mp - mx);
-  }
-  const float inv = 1.0f / den;
   const int t = items ? items[item] : item;  // null: every token, in order
-  for (int d = threadIdx.x; d < D; d += blockDim.x) {
-    float num = 0.f;
-#pragma unroll 4
-    for (int p = 0; p < P; ++p) {
-      const float mp = part_m[base + p];
-      const float wgt = (mp == NEG_INF) ? 0.f : fexp<T>(mp - mx);
-      num += part_acc[(base + p) * D + d] * wgt;
+  for (int d = threadIdx.x; d < (D + WAVE - 1) / WAVE * WAVE; d += blockDim.x) {  // whole waves: lanes hold the partitions' weights
+    float num = 0.f, den = sink ? fexp<T>(sk - mx) : 0.f;
+    const float* acc = part_acc + base * D + min(d, D - 1);
+    for (int p0 = 0; p0 < P; p0 += WAVE) {
+      const int here = min(WAVE, P - p0);
+      const float mp = lane < here ? part_m[base + p0 + lane] : NEG_INF;
+      const float weight = mp == NEG_INF ? 0.f : fexp<T>(mp - mx), l = weight == 0.f ? 0.f : part_l[base + p0 + lane] * weight;
+      for (int p = 0; p < here; p += 8) {  // eight at a time; those past the end repeat the last with a weight of 0
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = acc[(size_t)(p0 + min(p + j, here - 1)) * D];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          den += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l), p + j));
+          num = fmaf(v[j], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), p + j)), num);
+        }
+      }
     }
-    put(out, ((size_t)t * H + h) * D + d, num * inv, wide);
+    if (d < D) put(out, ((size_t)t * H + h) * D + d, num * (1.0f / den), wide);
   }
 }
 
@@ -294,6 +299,7 @@ __global__ __launch_bounds__(256) void attn_reduce_kernel(const int* __restrict_
 // The softmax weights are rounded to bf16 for the second product; maxima, sums and the
 // output accumulate in fp32.  Needs D % 32 == 0, D <= 256, block_size % 16 == 0.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -380,7 +386,7 @@ __device__ __forceinline__ void load_kv_step(KVStep<DC>& st, const bf16* __restr
 // qk_norm_rope_store_bf16x8_kernel; the squares are summed in another order.
 // What bounds a short context is the instructions of one wave, of which one that is alone on its SIMD issues one in 4 to
 // 8 cycles: with every wave norming all queries as operands (16 columns, most of them empty groups' padding), pages found by divisions in
-// the vector unit and partial outputs merged float by float, one token of Qwen3-0.6B sizes behind 100 took 7.6 us, now 6.2, behind 800 12.0 and 10.4.
+// the vector unit and partial outputs merged float by float, one token of Qwen3-0.6B sizes behind 100 took 7.6 us, now 5.4.
 struct FreshQKV {
   const bf16* qkv;
   const void* qw;      // gains of the per-head norms, D values each, bf16 or fp32
@@ -586,12 +592,16 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
               for (int c = 0; c < DC; ++c) cur.k[tt][c] = *reinterpret_cast<const bf16x8_t*>(&fresh_kv[0][c * 32 + grp * 8]);
             }
         }
-        if (grp == (nth >> 3)) {
+        // the token's half word in the eight keys of its lane group: a mask of bits to take per word, none in other lanes
+        const unsigned half = grp == (nth >> 3) ? (nth & 1 ? 0xffff0000u : 0xffffu) : 0u;
+        u32x4_t take;
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt)
+        for (int w = 0; w < 4; ++w) take[w] = (nth & 7) >> 1 == w ? half : 0u;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-              if (j == (nth & 7)) cur.v[dt][j] = fresh_kv[1][dt * 16 + col];
+        for (int dt = 0; dt < DT; ++dt) {
+          const unsigned value = __builtin_bit_cast(unsigned short, fresh_kv[1][dt * 16 + col]) * 0x10001u;
+          const u32x4_t was = __builtin_bit_cast(u32x4_t, cur.v[dt]);
+          cur.v[dt] = __builtin_bit_cast(bf16x8_t, (was & ~take) | (value & take));
         }
       }
     }
@@ -743,7 +753,6 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
     bf16* __restrict__ out, int H, int KV, int bs, float scale, Sight sight, int units_z, int pass, PrefillSplit split) {
   constexpr int D = DC * 32, DT = DC * 2;
   constexpr int PIECE = 64 * DC;  // 16-byte slots of a 16-key piece: 16 * D / 8
-  typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   typedef const __attribute__((address_space(1))) void* global_ptr_t;
   __shared__ __attribute__((aligned(16))) u32x4_t lds[PF_STAGES][4][PIECE];  // [stage][K0 K1 V0 V1][slot]
@@ -1478,14 +1487,16 @@ __device__ __forceinline__ void norm_rotate_f32(f32x4_t (&v)[DT], const f32x4_t 
     }
 }
 
-template <int DT, bool FRESH = false>
+// PAGE: tokens of a page where the compiler knows them (three divisions a step by another number are some 600 cycles), or 0.
+template <int DT, bool FRESH, int PAGE>
 __global__ __launch_bounds__(256) void attn_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
     const int* __restrict__ tiles, const int* __restrict__ items, const int* __restrict__ positions,
     const int* __restrict__ tok_row, const int* __restrict__ block_tables, int table_width, float* __restrict__ out,
-    float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int bs,
+    float* __restrict__ part_m, float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int page_size,
     float scale, Sight sight, int subs, int part_size, int P, int N, FreshF32 fresh) {
   constexpr int D = 16 * DT, LD = D + 4;
+  const int bs = PAGE ? PAGE : page_size;
   extern __shared__ float smem[];  // [4][16] m, [4][16] l, [4][16][LD] outputs
   const int G = H / KV;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1721,15 +1732,19 @@ static int launch_attn_f32(const FreshF32* fresh, const float* q, const float* k
   const dim3 grid(blocks_of * subs, KV, P);
   const size_t lds = (128 + 4 * 16 * (D + 4)) * sizeof(float);
   const FreshF32 none = {};
-#define GO(DTV, FRESHV)                                                                                                                  \
-  attn_f32_kernel<DTV, FRESHV><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables, table_width, \
-                                                           out, part_m, part_l, part_acc, H, KV, bs, scale, sight, subs, part_size, P,     \
-                                                           blocks_of * subs, FRESHV ? *fresh : none)
+#define GO(DTV, FRESHV, PAGEV)                                                                                                           \
+  attn_f32_kernel<DTV, FRESHV, PAGEV><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables,    \
+                                                                  table_width, out, part_m, part_l, part_acc, H, KV, bs, scale, sight,    \
+                                                                  subs, part_size, P, blocks_of * subs, FRESHV ? *fresh : none)
+#define GO_PAGES(DTV, FRESHV)           \
+  if (bs == 16) GO(DTV, FRESHV, 16);    \
+  else GO(DTV, FRESHV, 0)
   if (fresh) {
-    if (D == 64) GO(4, true);
-    else GO(8, true);
-  } else if (D == 64) GO(4, false);
-  else GO(8, false);
+    if (D == 64) { GO_PAGES(4, true); }
+    else { GO_PAGES(8, true); }
+  } else if (D == 64) { GO_PAGES(4, false); }
+  else { GO_PAGES(8, false); }
+#undef GO_PAGES
 #undef GO
   if (P > 1) {
     const int rc = launch_status();

@@ -986,6 +986,34 @@ def test_decode_step_from_fresh_projections(ops, H, KV, D, bs, gain, window, par
                                   scale, window, max(lens), part)  # fmt: skip
 
 
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_partial_results_of_any_number_merge(ops, dtype):
+    """Contexts in 1 to 79 partitions (a lane holds a partition's weight, 64 at a time, and eight are added up at once), with rows that fill
+    one, some and all of them: the attention of whole contexts.  Pages of 16, which the 32-bit kernel knows, and of 48: the same bits."""
+    H, KV, D, scale, seen = 8, 2, 128, 128**-0.5, []
+    lens = [1, 33, 250, 256, 257, 289, 2048, 2049, 2500]
+    T, g = len(lens), torch.Generator().manual_seed(4)
+    keys, values = (torch.randn(T, 2544, KV, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+    q, positions = torch.randn(T, H, D, generator=g).to(dtype).to(DEV), i32([n - 1 for n in lens])
+    for bs in (16, 48):
+        per = 2544 // bs
+        tables = torch.randperm(T * per, generator=g).view(T, per).to(torch.int32).to(DEV)
+        k_pages, v_pages = torch.empty(T * per, KV, bs, D, dtype=dtype, device=DEV), torch.empty(T * per, KV, D, bs, dtype=dtype, device=DEV)
+        k_pages[tables.long()] = keys.view(T, per, bs, KV, D).permute(0, 1, 3, 2, 4)
+        v_pages[tables.long()] = values.view(T, per, bs, KV, D).permute(0, 1, 3, 4, 2)
+        for part in (2528, 1024, 320, 288, 256, 32):
+            out = torch.full((T, H, D), float("nan"), dtype=dtype, device=DEV)
+            ops.attn_single_query(q, k_pages, v_pages, None, positions, None, tables, out, scale, 0, max(lens), part)
+            seen.append(out)
+    k, v = (t.double().repeat_interleave(H // KV, 2) for t in (keys, values))
+    for i, n in enumerate(lens):
+        p = torch.softmax((k[i, :n] * q[i].double()).sum(-1) * scale, 0)
+        ref = (p.unsqueeze(-1) * v[i, :n]).sum(0)
+        bound = 2e-2 if dtype == BF16 else 2e-6 * float(v[i, :n].abs().max())  # 32 bits: weights and sums of up to 2,500 roundings of 2^-24
+        assert all(bool(((out[i].double() - ref).abs() <= bound).all()) for out in seen)
+    assert all(torch.equal(a, b) for a, b in zip(seen[:6], seen[6:]))
+
+
 @pytest.mark.parametrize("G,KV,D", [(1, 3, 128), (3, 2, 64), (5, 2, 128), (7, 1, 192), (15, 1, 256), (16, 2, 128)])
 def test_a_decode_step_gives_the_same_bits_at_every_page_size(ops, G, KV, D):
     """Pages of 16 tokens, which have kernels of their own, and of other sizes: a group's heads, the key and the value over four waves in
