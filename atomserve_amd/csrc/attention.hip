@@ -399,47 +399,21 @@ struct FreshQKV {
   int store;           // 0: queries only, the pages already hold the token's key and value
 };
 
-// D / 32; FRESH 0: finished queries, 1: qkv with bf16 gains, 2: with fp32 gains; SEE 0: a window at most (nothing of the rest of
-// `sight` is read), 1: kept first tokens, chunks, a sink and fp32 outputs too, 2: also capped scores; PAGE: tokens of a page, or 0 for any
-template <int DC, int FRESH, int SEE, bool TURNED, int PAGE>
-__global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
+// What one workgroup does: partition `part` of item `item` for kv head `kvh`.
+template <int DC, int FRESH, int SEE, int PAGE>
+__device__ __forceinline__ void decode_item(
     const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ items, const int* __restrict__ positions, const int* __restrict__ tok_row,
     const int* __restrict__ block_tables, int table_width, bf16* __restrict__ out, float* __restrict__ part_m,
-    float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int page_size, float scale, Sight sight,
-    int part_size, int P, int cus, int share, FreshQKV fresh) {
+    float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int page_size, float scale, const Sight& sight,
+    int part_size, int P, int share, const FreshQKV& fresh, float* smem, int item, int kvh, int part) {
+  // smem: [4][16] m, [4][16] l, [4][G][LD] acc; FRESH: [G][D + 8] bf16 queries
   // share > 1: every `share` consecutive kv heads named here are one head of the pages (a group of more query heads
   // than a workgroup takes, cut into several); the pages then hold KV / share heads.
   constexpr int D = DC * 32, DT = DC * 2;  // DT: tiles of 16 output coordinates
   constexpr int LD = D + 4;                // a partial output's row in LDS
-  extern __shared__ __align__(16) float smem[];  // [4][16] m, [4][16] l, [4][G][LD] acc; FRESH: [G][D + 8] bf16 queries
   __shared__ __align__(16) bf16 fresh_kv[2][256];  // FRESH: the new token's key and value
   const int G = H / KV, bs = PAGE ? PAGE : page_size;
-  int item = blockIdx.x, kvh = blockIdx.y;
-  const int part = blockIdx.z;
-  if (!TURNED && P == 1) {
-    // Whole contexts, one workgroup each, of unequal length: two workgroups share a compute unit, and
-    // the first two rounds of `cus` workgroups are placed at once, the second on top of the first.
-    // Work is taken eight items at a time, their kv heads one after the other (so neighbours in this
-    // order read different pages at the same time), with the second round backwards: with `items`
-    // sorted longest first a compute unit's first two are a long and a short one, and what follows
-    // goes to whichever compute unit is free, longest first.
-    int s = blockIdx.x + gridDim.x * blockIdx.y;
-    const int total = gridDim.x * gridDim.y;
-    if (s >= cus && s < 2 * cus) s = cus + (min(2 * cus, total) - 1 - s);
-    const int N = gridDim.x, first = s / (8 * KV) * 8, r = s % (8 * KV), here = min(8, N - first);
-    item = first + r % here;
-    kvh = r / here;
-  }
-  if constexpr (TURNED) {
-    // Partitions of many tokens come as a turned grid: workgroups are dealt to the XCDs in turn, and with the tokens changing
-    // fastest an XCD had every eighth context, so that the one with the longest worked alone at the end.  With the kv heads
-    // changing fastest each has its share of every context: 13 requests of 300 to 7,000 keys in a step of 16 rows 67 -> 46 us, 20
-    // of 200 to 3,000 in one of 32 60 -> 41 (equal contexts: within 2 per cent).  Up to eight tokens an XCD has one, and its keys'
-    // pages to itself: left so.  (An instance of its own: the same branch at run time costs whole contexts 3 to 5 per cent.)
-    item = blockIdx.y;
-    kvh = blockIdx.x;
-  }
   const int t = items ? items[item] : item;  // null: every token, in order
   const int pos = positions[t];
   const int ctx = pos + 1;
@@ -694,6 +668,45 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   }
 }
 
+// D / 32; FRESH 0: finished queries, 1: qkv with bf16 gains, 2: with fp32 gains; SEE 0: a window at most (nothing of the rest of
+// `sight` is read), 1: kept first tokens, chunks, a sink and fp32 outputs too, 2: also capped scores; PAGE: tokens of a page, or 0 for any
+template <int DC, int FRESH, int SEE, bool TURNED, int PAGE>
+__global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
+    const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
+    const int* __restrict__ items, const int* __restrict__ positions, const int* __restrict__ tok_row,
+    const int* __restrict__ block_tables, int table_width, bf16* __restrict__ out, float* __restrict__ part_m,
+    float* __restrict__ part_l, float* __restrict__ part_acc, int H, int KV, int page_size, float scale, Sight sight,
+    int part_size, int P, int cus, int share, FreshQKV fresh) {
+  extern __shared__ __align__(16) float smem[];
+  int item = blockIdx.x, kvh = blockIdx.y;
+  const int part = blockIdx.z;
+  if (!TURNED && P == 1) {
+    // Whole contexts, one workgroup each, of unequal length: two workgroups share a compute unit, and
+    // the first two rounds of `cus` workgroups are placed at once, the second on top of the first.
+    // Work is taken eight items at a time, their kv heads one after the other (so neighbours in this
+    // order read different pages at the same time), with the second round backwards: with `items`
+    // sorted longest first a compute unit's first two are a long and a short one, and what follows
+    // goes to whichever compute unit is free, longest first.
+    int s = blockIdx.x + gridDim.x * blockIdx.y;
+    const int total = gridDim.x * gridDim.y;
+    if (s >= cus && s < 2 * cus) s = cus + (min(2 * cus, total) - 1 - s);
+    const int N = gridDim.x, first = s / (8 * KV) * 8, r = s % (8 * KV), here = min(8, N - first);
+    item = first + r % here;
+    kvh = r / here;
+  }
+  if constexpr (TURNED) {
+    // Partitions of many tokens come as a turned grid: workgroups are dealt to the XCDs in turn, and with the tokens changing
+    // fastest an XCD had every eighth context, so that the one with the longest worked alone at the end.  With the kv heads
+    // changing fastest each has its share of every context: 13 requests of 300 to 7,000 keys in a step of 16 rows 67 -> 46 us, 20
+    // of 200 to 3,000 in one of 32 60 -> 41 (equal contexts: within 2 per cent).  Up to eight tokens an XCD has one, and its keys'
+    // pages to itself: left so.  (An instance of its own: the same branch at run time costs whole contexts 3 to 5 per cent.)
+    item = blockIdx.y;
+    kvh = blockIdx.x;
+  }
+  decode_item<DC, FRESH, SEE, PAGE>(q, k_pages, v_pages, items, positions, tok_row, block_tables, table_width, out, part_m, part_l,
+                                    part_acc, H, KV, page_size, scale, sight, part_size, P, share, fresh, smem, item, kvh, part);
+}
+
 // ---- bf16 prefill through the matrix cores ----------------------------------------------
 //
 // Work item: up to 64 consecutive query tokens of one request (`tiles` rows: first flat
@@ -746,16 +759,23 @@ constexpr int PREFILL_MIN_PIECE_ROUNDS = 2;  // an item's last two rounds hold i
 
 // With kept first tokens behind a window the rounds of 64 keys are first those from the sequence's start that hold kept
 // tokens, then those of the window (`first_key`); pieces cut this list.
-template <int DC, int QT, int SEE>  // D / 32; column tiles of 16 queries that a wave owns: 2, or 1 (see the launcher); SEE: see above
-__global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
+// What the workgroup `item` of `blocks` does; lds: a stage's slots are K0 K1 V0 V1.
+template <int DC>
+using PrefillStages = u32x4_t[PF_STAGES][4][64 * DC];  // [stage][K0 K1 V0 V1][slot]
+// BY_HEAD: the kv head changes fastest and a pass is walked backwards by eights.  Workgroups are dealt to the eight XCDs in
+// turn, each with an L2 of its own, so that with eight kv heads an XCD brings one head's keys and values from memory (with four, two share
+// one).  Beside single queries that is what memory is short of (Qwen3-8B sizes, 8 of 500 to 8,192 keys beside 504 tokens 48.3 -> 44.6 us a
+// layer, 2 of 7,000 beside 500 32.9 -> 28.7, 32 of 100 to 2,048 beside 480 behind 7,001 with 64 heads 210 -> 195); portions alone
+// wait for the matrix cores, and several of one request lose (480 tokens behind 7,001 95 -> 97): not there.
+template <int DC, int QT, int SEE, bool BY_HEAD>  // D / 32; column tiles of 16 queries that a wave owns: 2, or 1 (see the launcher); SEE: see above
+__device__ __forceinline__ void prefill_item(
     const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ tiles, const int* __restrict__ block_tables, int table_width,
-    bf16* __restrict__ out, int H, int KV, int bs, float scale, Sight sight, int units_z, int pass, PrefillSplit split) {
+    bf16* __restrict__ out, int H, int KV, int bs, float scale, const Sight& sight, int units_z, int pass, const PrefillSplit& split,
+    PrefillStages<DC>& lds, int item, int blocks) {
   constexpr int D = DC * 32, DT = DC * 2;
-  constexpr int PIECE = 64 * DC;  // 16-byte slots of a 16-key piece: 16 * D / 8
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   typedef const __attribute__((address_space(1))) void* global_ptr_t;
-  __shared__ __attribute__((aligned(16))) u32x4_t lds[PF_STAGES][4][PIECE];  // [stage][K0 K1 V0 V1][slot]
 
   const int G = H / KV;
   // Work items (tile, kv head, group of four waves) in the order of `tiles`, which the caller
@@ -765,18 +785,24 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
   // the next, so that causal prompts, whose items range from one step to hundreds, finish
   // together.
   const int per_tile = KV * units_z;
-  int item = blockIdx.x;
+  int tile, kvh, bz, piece = 0;  // piece: which of an item's workgroups this is
   {
-    const int block = item / pass, first = block * pass;
-    const int size = min(pass, (int)gridDim.x - first);
-    if (block & 1) item = first + size - 1 - (item - first);
+    const int block = item / pass, first = block * pass, size = min(pass, blocks - first), off = item - first;
+    if constexpr (BY_HEAD) {
+      const int eights = size & ~7;
+      if ((block & 1) && off < eights) item = first + eights - 8 - (off & ~7) + (off & 7);
+      const int all = per_tile * split.pieces;
+      tile = item / all, kvh = item % KV, bz = item / KV % units_z, piece = item % all / per_tile;
+      item = (tile * KV + kvh) * units_z + bz;
+    } else {
+      if (block & 1) item = first + size - 1 - off;
+      if (split.pieces > 1) {
+        piece = item % split.pieces;
+        item /= split.pieces;
+      }
+      tile = item / per_tile, kvh = (item % per_tile) / units_z, bz = item % units_z;
+    }
   }
-  int piece = 0;  // which of an item's workgroups this is
-  if (split.pieces > 1) {
-    piece = item % split.pieces;
-    item /= split.pieces;
-  }
-  const int tile = item / per_tile, kvh = (item % per_tile) / units_z, bz = item % units_z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
@@ -1125,6 +1151,46 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
   }
 }
 
+template <int DC, int QT, int SEE>
+__global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
+    const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
+    const int* __restrict__ tiles, const int* __restrict__ block_tables, int table_width,
+    bf16* __restrict__ out, int H, int KV, int bs, float scale, Sight sight, int units_z, int pass, PrefillSplit split) {
+  __shared__ __attribute__((aligned(16))) PrefillStages<DC> lds;
+  prefill_item<DC, QT, SEE, false>(q, k_pages, v_pages, tiles, block_tables, table_width, out, H, KV, bs, scale, sight, units_z, pass, split,
+                            lds, blockIdx.x, gridDim.x);
+}
+
+// A step that has both, portions of prompts and single queries, in one launch: the single queries' workgroups come first, a kv
+// head of every context after the other, and share the compute units with the portions'.  The ones wait for memory most of
+// the time and the others for the matrix cores and the softmax, and the tail of neither leaves compute units idle.
+struct Singles {
+  const int* items;
+  const int* positions;
+  const int* tok_row;
+  float* part_m;
+  float* part_l;
+  float* part_acc;
+  int count, part_size, P;
+};
+
+template <int DC, int QT, int PAGE>
+__global__ __launch_bounds__(256, 2) void attn_mixed_mfma_kernel(
+    const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
+    const int* __restrict__ tiles, const int* __restrict__ block_tables, int table_width,
+    bf16* __restrict__ out, int H, int KV, int bs, float scale, Sight sight, int units_z, int pass, PrefillSplit split, Singles single) {
+  __shared__ __attribute__((aligned(16))) PrefillStages<DC> lds;  // a single query of up to 16 heads needs 256 D + 1,536 of its 512 D bytes
+  const int b = blockIdx.x, singles = single.count * KV * single.P;
+  if (b < singles) {
+    decode_item<DC, 0, 0, PAGE>(q, k_pages, v_pages, single.items, single.positions, single.tok_row, block_tables, table_width, out,
+                                single.part_m, single.part_l, single.part_acc, H, KV, bs, scale, sight, single.part_size, single.P, 1,
+                                FreshQKV{}, reinterpret_cast<float*>(&lds[0][0][0]), b / KV % single.count, b % KV, b / (KV * single.count));
+  } else {
+    prefill_item<DC, QT, 0, true>(q, k_pages, v_pages, tiles, block_tables, table_width, out, H, KV, bs, scale, sight, units_z, pass, split,
+                            lds, b - singles, gridDim.x - singles);
+  }
+}
+
 // The pieces of every cut item, put together: one workgroup per item, its waves and lanes holding the queries and
 // coordinates they hold in the kernel above.  out = sum_j acc_j 2^(m_j - m) / sum_j l_j 2^(m_j - m) with m the
 // largest maximum; a piece that saw no key has m = -inf and l = 0.
@@ -1373,6 +1439,52 @@ extern "C" int as_attn_decode_fresh(const void* qkv, const void* qw, const void*
   return launch_decode_mfma(nullptr, k_pages, v_pages, items, num_tokens, positions, nullptr, block_tables,
                             table_width, out, part_m, part_l, part_acc, H, KV, D, bs, scale, Sight{window, 0, 0, 0.f, 0, nullptr, 0},
                             part_size, P, &fresh, gains_dtype, stream);
+}
+
+// as_attn_prefill_mfma and as_attn_decode_mfma of one step in one launch (with merges behind it where items are cut), for
+// heads of 64 and 128, pages of 16 tokens and no more sight than a window: arguments as there.  The two sets of tokens
+// are apart, and so are the partial results.
+extern "C" int as_attn_mixed_mfma(const void* q, const void* k_pages, const void* v_pages, const int* tiles, int num_tiles,
+                                  const int* items, int num_items, const int* positions, const int* tok_row,
+                                  const int* block_tables, int table_width, void* out, int H, int KV, int D, int bs, float scale,
+                                  int window, int query_tiles, int pieces, int piece_rounds, int* cut, float* piece_ml,
+                                  float* piece_acc, float* part_m, float* part_l, float* part_acc, int part_size, int P,
+                                  hipStream_t stream) {
+  if (num_tiles <= 0 || num_items <= 0) return AS_BAD_SHAPE;
+  const Sight sight{window, 0, 0, 0.f, 0, nullptr, 0};
+  if (!sight_ok(sight)) return AS_BAD_SHAPE;
+  if (H <= 0 || KV <= 0 || H % KV || H / KV > 16 || table_width <= 0 || (D != 64 && D != 128) || bs != 16) return AS_BAD_SHAPE;
+  if (query_tiles != 1 && query_tiles != 2) return AS_BAD_SHAPE;
+  if (pieces < 1) pieces = 1;
+  if (pieces > 1 && (piece_rounds < PREFILL_MIN_PIECE_ROUNDS || !cut || !piece_ml || !piece_acc)) return AS_BAD_SHAPE;
+  if (part_size <= 0 || part_size % 32 || P <= 0 || (P > 1 && (!part_m || !part_l || !part_acc))) return AS_BAD_SHAPE;
+  const int units_z = (64 / (16 * query_tiles) * (H / KV) + 3) / 4;
+  const long tile_items = (long)num_tiles * KV * units_z, blocks = tile_items * pieces + (long)num_items * KV * P;
+  if (blocks > 0x7fffffffL) return AS_BAD_SHAPE;
+  const PrefillSplit split{pieces, piece_rounds, cut, piece_ml, piece_acc};
+  const Singles single{items, positions, tok_row, part_m, part_l, part_acc, num_items, part_size, P};
+#define LAUNCH(DCV, QTV)                                                                                                 \
+  do {                                                                                                                   \
+    attn_mixed_mfma_kernel<DCV, QTV, 16><<<(int)blocks, 256, 0, stream>>>(                                               \
+        (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, tiles, block_tables, table_width, (bf16*)out, H, KV, \
+        bs, scale, sight, units_z, compute_units(), split, single);                                                      \
+    if (hipGetLastError() != hipSuccess) return AS_LAUNCH_FAILED;                                                        \
+    if (pieces > 1)                                                                                                      \
+      attn_prefill_merge_kernel<DCV, QTV><<<(int)tile_items, 256, 0, stream>>>(tiles, (bf16*)out, H, KV, units_z, split, \
+                                                                               0, nullptr, 0);                           \
+  } while (0)
+  if (D == 64) {
+    if (query_tiles == 1) LAUNCH(2, 1);
+    else LAUNCH(2, 2);
+  } else {
+    if (query_tiles == 1) LAUNCH(4, 1);
+    else LAUNCH(4, 2);
+  }
+#undef LAUNCH
+  if (hipGetLastError() != hipSuccess) return AS_LAUNCH_FAILED;
+  if (P > 1)
+    attn_reduce_kernel<bf16><<<dim3(num_items, H), D, 0, stream>>>(items, part_m, part_l, part_acc, (bf16*)out, H, D, P, 0, nullptr, 0);
+  return launch_status();
 }
 
 static int pow2ceil(int v) { int p = 1; while (p < v) p <<= 1; return p; }

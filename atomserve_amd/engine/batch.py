@@ -67,14 +67,14 @@ class RowSplit:
     short_tokens [Ns] int32: the tokens of rows with at most `short` tokens, those that see most keys first;
     long_tiles [Nt, 4] int32: (first flat token, count, row, first position) per `tile` consecutive tokens
     of longer rows, those that see most keys first; max_short_context: host bound on the context of a
-    short token; tile_keys: the keys that the tiles' last tokens see, added up (what the tiles' attention
+    short token; max_tile_context: the keys that the last token of the tile that sees most sees; tile_keys: the keys that the tiles' last tokens see, added up (what the tiles' attention
     has to walk: a kernel may choose by it how to cut its work)."""
 
     def __init__(self, short: int, tile: int):
         if short < 0 or tile < 1:
             raise ValueError(f"a row split is (short >= 0, tile >= 1), not {(short, tile)}")
         self.short, self.tile = short, tile
-        self.tokens, self.tiles, self.max_short_context, self.tile_keys = [], [], 0, 0
+        self.tokens, self.tiles, self.max_short_context, self.max_tile_context, self.tile_keys = [], [], 0, 0, 0
         self.short_tokens = self.long_tiles = None  # on the device once the step is packed
         self.num_short_tokens = self.num_long_tiles = 0
 
@@ -216,6 +216,7 @@ class StepBatch:
         # them out in this order and pairs the longest with the shortest on a compute unit.
         for split in self.splits.values():
             split.tiles.sort(key=lambda t: -(t[3] + t[1]))
+            split.max_tile_context = split.tiles[0][3] + split.tiles[0][1] if split.tiles else 0
             split.tokens.sort(key=lambda t: -int(pos[t]))  # single queries too: the longest contexts first
             split.max_short_context = max(split.max_short_context, max_context if split.tokens else 0)
         self.max_context = max(self.max_context, max_context)

@@ -86,6 +86,7 @@ SIGNATURES = {
     "as_attn_decode_mfma_shared": ("attention", [P, P, P, P, I, P, P, P, I, P, P, P, P, I, I, I, I, F, I, I, I, F, I, P, I, I, I, I, P]),
     "as_attn_decode_fresh": ("attention", [P, P, P, I, P, P, F, I, P, P, P, I, P, P, I, P, P, P, P, I, I, I, I, F, I, I, I, P]),
     "as_attn_prefill_mfma": ("attention", [P, P, P, P, I, P, I, P, I, I, I, I, F, I, I, I, F, I, P, I, I, I, I, P, P, P, P]),
+    "as_attn_mixed_mfma": ("attention", [P, P, P, P, I, P, I, P, P, P, I, P, I, I, I, I, F, I, I, I, I, P, P, P, P, P, P, I, I, P]),
     "as_attn_f32": ("attention", [P, P, P, P, I, I, P, I, P, P, P, I, P, P, P, P, I, I, I, I, F, I, I, I, F, I, P, I, I, I, P]),
     "as_attn_f32_fresh": ("attention", [P, P, P, P, P, F, I, P, P, P, I, P, P, I, P, P, P, P, I, I, I, I, F, I, I, I, P]),
     "as_gemm_f32": ("gemm_f32", [P, P, P, I, I, I, I, P]),

@@ -634,14 +634,18 @@ def _prefill_plan(num_tiles: int, H: int, KV: int, D: int, max_context: int, win
     return _prefill_plan_of(num_tiles, H, KV, D, max_context, window, query_tiles, tile_keys, PREFILL_PIECES, compute_units(), keep_first)
 
 
-@functools.lru_cache(maxsize=1024)
-def _prefill_plan_of(num_tiles, H, KV, D, max_context, window, query_tiles, tile_keys, forced_pieces, units, keep_first=0) -> tuple:
+def _prefill_rounds(num_tiles, max_context, window, tile_keys, keep_first=0) -> tuple:
+    """Rounds of 64 keys of the longest item, and of the items on average."""
     span = min(max_context, window + 64 + keep_first) if window > 0 else max_context  # the keys that the longest item walks
     rounds = max(1, -(-span // 64))
     if tile_keys > 0:
-        mean_rounds = min(rounds, max(1.0, tile_keys / num_tiles / 64))
-    else:
-        mean_rounds = max(rounds - num_tiles / 2, rounds / 2)
+        return rounds, min(rounds, max(1.0, tile_keys / num_tiles / 64))
+    return rounds, max(rounds - num_tiles / 2, rounds / 2)
+
+
+@functools.lru_cache(maxsize=1024)
+def _prefill_plan_of(num_tiles, H, KV, D, max_context, window, query_tiles, tile_keys, forced_pieces, units, keep_first=0) -> tuple:
+    rounds, mean_rounds = _prefill_rounds(num_tiles, max_context, window, tile_keys, keep_first)
     kinds = (2, 1) if query_tiles is None else (int(query_tiles),)
     if forced_pieces is not None:
         cuts = (max(1, min(int(forced_pieces), rounds // 2)),)
@@ -687,6 +691,79 @@ def attn_prefill(q, k_pages, v_pages, tiles, block_tables, out, scale, window, m
     call("as_attn_prefill_mfma", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(tiles), tiles.shape[0],
          _ptr(block_tables), block_tables.shape[1], _ptr(out), H, KV, D, bs, float(scale), *sight,
          int(query_tiles), pieces, piece_rounds, _ptr(cut), _ptr(part_ml), _ptr(part_acc), _stream())  # fmt: skip
+
+
+def attn_mixed_supported(dtype, H: int, KV: int, D: int, block_size: int) -> bool:
+    """Whether `attn_mixed` takes these heads and pages (with a window at most: no kept tokens, caps, sinks or chunks)."""
+    return dtype == BF16 and D in (64, 128) and block_size == 16 and H % KV == 0 and H // KV <= 16
+
+
+# Both kinds of work in one launch, single queries first.  How the portions' items and the singles' contexts are cut is chosen together: the
+# places (two workgroups to a compute unit) are busy for all the work divided by them and for a third of a piece at the end,
+# no less than for the longest piece or partition, and merges cost 10 us and 5 TB/s for what pieces leave, 4 us and 0.6 a
+# partition for what singles leave.  A single costs 4 us and 25 ns a key (contexts: three fifths of the longest on average), alone at the end 18 ns.
+# Pieces of 3 and 6 leave half a round of places idle.  One layer, us, two launches / this (best of all forms): Qwen3-8B sizes, 32 of 100 to
+# 2,048 keys beside 480 tokens behind 7,001 143 / 124 (122), 8 of 2,048 beside 504 33.5 / 27.9 (27.6), 8 of 500 to 8,192 beside 504 60 / 43
+# (42), 96 of 200 to 600 beside 2,000 96 / 92 (87), 20 of 1,000 to 3,000 beside four of 120 behind 6,000 159 / 122 (116); 40 heads, 128 of 32 to
+# 400 beside 384 behind 2,000 83 / 77 (65); 16 heads, 4 of 300 to 900 beside 37 14.2 / 11.1 (11.1).
+MIXED_PIECE_CHOICES = (1, 2, 4, 8)
+
+
+@functools.lru_cache(maxsize=1024)
+def _mixed_plan(num_tiles: int, H: int, KV: int, D: int, tile_context: int, tile_keys: int, singles: int, single_context: int,
+                window: int, units: int) -> tuple:  # fmt: skip
+    """(query tiles of a wave, pieces, rounds of a piece, keys of a single query's partition) for a step of both kinds."""
+    rounds, mean_rounds = _prefill_rounds(num_tiles, tile_context, window, tile_keys)
+    span = _seen_keys(single_context, window, 0, True)
+    places, whole, groups = 2 * units, _up32(span), singles * KV
+
+    def cost(kind, pieces, part):
+        round_time = 2.2 if kind == 2 else 1.4
+        workgroups = num_tiles * KV * _prefill_units(kind, H // KV)
+        piece, parts = -(-rounds // pieces) * round_time, -(-span // part)
+        work = workgroups * mean_rounds * round_time + groups * (4.0 * parts + 0.025 * 0.6 * span)
+        total = max(piece, 4.0 + 0.018 * min(part, span), work / places + 0.35 * piece)
+        if pieces > 1:
+            total += 10.0 + 64 * num_tiles * H * pieces * D * 8 / 5e6
+        return total + (MERGE_LAUNCH + 0.6 * parts if parts > 1 else 0.0)
+
+    kind, pieces, part = min(((k, c, p) for k in (1, 2) for c in MIXED_PIECE_CHOICES if c == 1 or rounds // c >= PREFILL_MIN_PIECE_ROUNDS
+                              for p in (whole, *(n for n in MFMA_PARTITIONS if n < whole))), key=lambda a: cost(*a))  # fmt: skip
+    return kind, pieces, -(-rounds // pieces) if pieces > 1 else 0, part
+
+
+def attn_mixed(q, k_pages, v_pages, items, tiles, positions, tok_row, block_tables, out, scale, window, max_tile, max_single,
+               tile_keys: int = 0) -> None:  # fmt: skip
+    """`attn_single_query` of the tokens `items` and `attn_prefill` of the portions `tiles` in one launch, for steps that
+    `attn_mixed_supported` takes: arguments as there; max_tile, max_single: host bounds on the last position + 1 of a tile and on
+    positions[items] + 1."""
+    _check(q, "q", BF16, (None, None, None))
+    T, H, D = q.shape
+    _check(out, "out", BF16, (T, H, D))
+    _check(k_pages, "k_pages", BF16, (None, None, None, D))
+    _, KV, bs, _ = k_pages.shape
+    _check(v_pages, "v_pages", BF16, (k_pages.shape[0], KV, D, bs))
+    _check(items, "items", I32, (None,))
+    _check(tiles, "tiles", I32, (None, 4))
+    _check(positions, "positions", I32, (T,))
+    _check(tok_row, "tok_row", I32, (T,))
+    _check(block_tables, "block_tables", I32, (None, None))
+    N, tile_count, dev = items.shape[0], tiles.shape[0], q.device
+    if N == 0 or tile_count == 0 or not attn_mixed_supported(q.dtype, H, KV, D, bs):
+        raise KernelError(f"mixed attention: {N} single queries, {tile_count} tiles, heads {H}/{KV} of {D}, pages of {bs}")
+    if max(max_tile, max_single) > block_tables.shape[1] * bs:
+        raise KernelError("attention: block tables are shorter than the longest context")
+    kind, pieces, piece_rounds, part = _mixed_plan(tile_count, H, KV, D, max_tile, tile_keys, N, max_single, window, compute_units())
+    part_size, P, part_m, part_l, part_acc = _partitions(N, H, KV, D, max_single, window, True, part, dev)
+    cut = piece_ml = piece_acc = None
+    if pieces > 1:
+        cut = torch.empty(tile_count * KV * _prefill_units(kind, H // KV), dtype=I32, device=dev)
+        piece_ml = torch.empty((T, H, pieces, 2), dtype=F32, device=dev)
+        piece_acc = torch.empty((T, H, pieces, D), dtype=F32, device=dev)
+    call("as_attn_mixed_mfma", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(tiles), tile_count, _ptr(items), N, _ptr(positions),
+         _ptr(tok_row), _ptr(block_tables), block_tables.shape[1], _ptr(out), H, KV, D, bs, float(scale), window, int(kind),
+         pieces, piece_rounds, _ptr(cut), _ptr(piece_ml), _ptr(piece_acc), _ptr(part_m), _ptr(part_l), _ptr(part_acc),
+         part_size, P, _stream())  # fmt: skip
 
 
 SKINNY_MAX_ROWS = 16  # up to here the bf16 product streams the weights through our own kernel

@@ -167,6 +167,10 @@ def attend(q, out, step, cache, scale: float, window: int, split, wide: bool = F
         ops.attn_single_query(q, cache.k_pages, cache.v_pages, step.all_tokens, step.positions, step.tok_row,
                               cache.block_tables, out, scale, window, step.max_context, **sight)  # fmt: skip
         return
+    if rows.num_short_tokens and rows.num_long_tiles and not sight and ops.attn_mixed_supported(q.dtype, H, KV, D, cache.block_size):
+        ops.attn_mixed(q, cache.k_pages, cache.v_pages, rows.short_tokens, rows.long_tiles, step.positions, step.tok_row,
+                       cache.block_tables, out, scale, window, rows.max_tile_context, rows.max_short_context, rows.tile_keys)  # fmt: skip
+        return
     if rows.num_short_tokens:
         ops.attn_single_query(q, cache.k_pages, cache.v_pages, rows.short_tokens, step.positions, step.tok_row,
                               cache.block_tables, out, scale, window, rows.max_short_context, **sight)  # fmt: skip

@@ -271,6 +271,43 @@ def test_the_route_of_a_32_bit_portion(monkeypatch, tokens, start, how):
     assert made == [{"single": ("single", "all"), "tiles": ("tiles", "long"), "short": ("single", "short")}[how]]
 
 
+def test_plans_of_steps_with_portions_and_single_queries(monkeypatch):
+    """Pieces and partitions cover the longest item and context, and every piece and partition is one that the kernel takes."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    ops._mixed_plan.cache_clear()
+    try:
+        for H, KV, D in ((32, 8, 128), (40, 8, 128), (16, 1, 64), (6, 3, 64)):
+            for tokens, behind, singles, context, window in ((37, 0, 1, 1, 0), (480, 7001, 32, 2049, 0), (2000, 0, 128, 400, 0), (100, 8000, 1, 8193, 0),
+                                                             (300, 5000, 64, 6000, 1024), (9, 31, 3, 40, 1)):  # fmt: skip
+                tiles, most = -(-tokens // 64), behind + tokens
+                keys = sum(behind + min(tokens, 64 * (i + 1)) for i in range(tiles))
+                kind, pieces, piece_rounds, part = ops._mixed_plan(tiles, H, KV, D, most, keys, singles, context, window, 256)
+                span = min(most, window + 64) if window else most
+                assert kind in (1, 2) and part % 32 == 0 and part >= 32
+                assert (pieces, piece_rounds) == (1, 0) or (pieces * piece_rounds * 64 >= span and piece_rounds >= 2)
+        assert ops._mixed_plan(8, 32, 8, 128, 7481, 8 * 7257, 32, 2049, 0, 256) == (2, 4, 30, 2080)
+    finally:
+        ops._mixed_plan.cache_clear()
+
+
+@pytest.mark.parametrize("dtype,D,page,sight,one", [(torch.bfloat16, 128, 16, {}, True), (torch.bfloat16, 64, 16, {}, True), (torch.bfloat16, 96, 16, {}, False),
+                                                    (torch.bfloat16, 128, 32, {}, False), (torch.bfloat16, 128, 16, {"softcap": 5.0}, False)])  # fmt: skip
+def test_the_route_of_a_step_with_portions_and_single_queries(monkeypatch, dtype, D, page, sight, one):
+    from types import SimpleNamespace
+
+    from atomserve_amd.parts.attention import attend
+
+    made = []
+    for name in ("attn_mixed", "attn_single_query", "attn_prefill"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, **kw: made.append(name))
+    pages = torch.empty(1, 8, page, D, dtype=dtype)
+    cache = SimpleNamespace(k_pages=pages, v_pages=pages.view(1, 8, D, page), block_tables=None, block_size=page)
+    rows = SimpleNamespace(num_short_tokens=3, num_long_tiles=2, short_tokens="short", long_tiles="long", max_short_context=90, max_tile_context=100, tile_keys=164)
+    step = SimpleNamespace(decode_only=False, all_tokens="all", positions=None, tok_row=None, max_context=100, split=lambda key: rows)
+    attend(torch.empty(103, 16, D, dtype=dtype), None, step, cache, 1.0, 0, (8, 64), **sight)
+    assert made == (["attn_mixed"] if one else ["attn_single_query", "attn_prefill"])
+
+
 def test_plans_of_wide_products(monkeypatch):
     """Products of more than 128 rows: ranges of K that are none of them empty, in one round of workgroups, and no range where
     the library's whole product takes less."""

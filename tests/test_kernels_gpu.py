@@ -1305,6 +1305,45 @@ def test_long_items_of_a_prompt_step_are_cut_into_pieces_and_merged(ops, H, KV, 
         assert torch.allclose(out.float(), whole.float(), atol=2e-2, rtol=2e-2)  # every token, against the kernel without the cut
 
 
+@pytest.mark.parametrize("H,KV,D,window", [(32, 8, 128, 0), (16, 8, 128, 200), (40, 8, 128, 0), (16, 1, 128, 0), (6, 3, 64, 0), (8, 4, 64, 70)])
+def test_portions_and_single_queries_in_one_launch(ops, monkeypatch, H, KV, D, window):
+    """Prompt portions beside rows of one and of a few tokens, contexts and portions whole and cut, kv heads that do and do
+    not divide the XCDs: plain attention's results for every token, and what the two launches give."""
+    torch.manual_seed(H + D)
+    rows = [(40, 1), (0, 70), (700, 1), (31, 1), (900, 130), (0, 1), (1100, 3), (333, 64), (15, 9)]  # (start, new tokens)
+    lens = [a + n for a, n in rows]
+    _, k_pages, v_pages, tables, _ = paged_case(BF16, H, KV, D, 16, lens, seed=5, k_scale=2.0 / math.sqrt(D / 16))
+    T = sum(n for _, n in rows)
+    q = torch.randn(T, H, D, device=DEV).to(BF16)
+    positions, tok_row, tiles, singles, flat = [], [], [], [], 0
+    for r, (start, n) in enumerate(rows):
+        positions += list(range(start, start + n))
+        tok_row += [r] * n
+        if n <= 8:
+            singles += range(flat, flat + n)
+        else:
+            tiles += [[flat + q0, min(64, n - q0), r, start + q0] for q0 in range(0, n, 64)]
+        flat += n
+    tiles.sort(key=lambda t: -(t[3] + t[1]))
+    singles.sort(key=lambda t: -positions[t])
+    most, keys = tiles[0][3] + tiles[0][1], sum(t[3] + t[1] for t in tiles)
+    ref = pk.paged_attention(q, k_pages, v_pages, i32(list(range(T))), i32(positions), i32(tok_row), tables, D**-0.5, window)
+    where = i32(positions), i32(tok_row), tables
+    two = torch.zeros(T, H, D, dtype=BF16, device=DEV)
+    ops.attn_single_query(q, k_pages, v_pages, i32(singles), *where, two, D**-0.5, window, max(lens))
+    ops.attn_prefill(q, k_pages, v_pages, i32(tiles), tables, two, D**-0.5, window, most, tile_keys=keys)
+    span = min(most, window + 64) if window else most
+    rounds = -(-span // 64)
+    plans = [None] + [(kind, c, -(-rounds // c) if c > 1 else 0, part) for kind, c, part in ((1, 1, 1152), (2, 1, 32), (1, 2, 1152), (2, 2, 128)) if rounds >= 2 * c]
+    for plan in plans:
+        if plan:
+            monkeypatch.setattr(ops, "_mixed_plan", lambda *a: plan)
+        out = torch.full((T, H, D), float("nan"), device=DEV).to(BF16)
+        ops.attn_mixed(q, k_pages, v_pages, i32(singles), i32(tiles), *where, out, D**-0.5, window, most, max(lens), keys)
+        assert torch.allclose(out.float(), ref, atol=2e-2, rtol=2e-2), (plan, (out.float() - ref).abs().max())
+        assert torch.allclose(out.float(), two.float(), atol=2e-2, rtol=2e-2), plan
+
+
 def test_kernels_refuse_what_they_cannot_do(ops):
     from atomserve_amd.kernels.lib import KernelError
 
