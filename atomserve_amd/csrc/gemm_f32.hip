@@ -28,22 +28,21 @@ __device__ __forceinline__ void store4(float* p, floatx4 v, int valid) {
   for (int i = 0; i < valid; ++i) p[i] = v[i];
 }
 
-// Columns k .. k+3 of a row, those from K on as zeros.  VEC: rows start on 16 bytes and K % 4 == 0.  Else the load, which needs no
-// more than a float's alignment, ends where the row ends, and `ragged` moves what belongs elsewhere when the columns are used: a
-// test here would make every load wait for the one before.
+// Columns k .. k+3 of a row, those from K on as zeros.  VEC: rows start on 16 bytes and K % 4 == 0; else the load needs no
+// more than a float's alignment.  It ends where the row ends, and `ragged` puts zeros and moves what belongs elsewhere when the
+// columns are used, where K ends: a test here would make every load wait for the one before, or choose eight times a step of 32 bytes.
 typedef float floatx4_anywhere __attribute__((ext_vector_type(4), aligned(4)));
 
 template <bool VEC> __device__ __forceinline__ floatx4 fetch(const float* row, int k, int K) {
   if constexpr (VEC) {
-    const floatx4 v = *reinterpret_cast<const floatx4*>(row + (k < K ? k : 0));
-    return k < K ? v : floatx4{0.f, 0.f, 0.f, 0.f};
+    return *reinterpret_cast<const floatx4*>(row + min(k, K - 4));
   } else {
     return *reinterpret_cast<const floatx4_anywhere*>(row + min(k, K - 4));  // K > F32_NARROW
   }
 }
 
 template <bool VEC> __device__ __forceinline__ floatx4 ragged(floatx4 v, int k, int K) {  // v: what `fetch` gave for k
-  if constexpr (VEC) return v;
+  if constexpr (VEC) return k < K ? v : floatx4{0.f, 0.f, 0.f, 0.f};
   const int by = k - min(k, K - 4);
   if (by & 1) v = floatx4{v[1], v[2], v[3], 0.f};
   if (by & 2) v = floatx4{v[2], v[3], 0.f, 0.f};
@@ -105,7 +104,7 @@ template <int LANES> __device__ __forceinline__ bf16x8 rotated(bf16x8 v) {  // w
 // SHARE: with at most 16 / SHARE rows the 16 lanes of a row group hold SHARE steps' rows side by side, which are taken apart
 // once for all of them and turned into place by a rotation of the lanes: the vector unit, which takes the floats apart (44
 // instructions for 8 columns of 16 rows), is what a product of few rows is made of beside reading w.
-// GATED: NT = 2, gate rows and the up rows of the same outputs (w has 2 N rows); LINK: MT = NT = 1; ssq_in: MT = 1.
+// GATED: NT = 2, gate rows and the up rows of the same outputs (w has 2 N rows), or NT = MT = 1, eight rows of each in one strip; LINK: MT = NT = 1; ssq_in: MT = 1.
 // VEC: rows start on 16 bytes (K % 4 == 0 and both matrices do).
 template <int MT, int NT, int WAVES, int DEPTH, int SHARE, bool VEC, int MODE>
 __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_rows_kernel(const float* __restrict__ a,
@@ -113,7 +112,8 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
                                                                                        int M, int N, int K, int tiles_m, int tiles,
                                                                                        int per_xcd, LinkF32 link) {
   static_assert(DEPTH % SHARE == 0 && (SHARE == 1 || MT == 1), "whole groups of steps, one row tile");
-  static_assert(MODE != GATED || NT == 2, "a gate strip and its up strip");
+  static_assert(MODE != GATED || NT == 2 || (NT == 1 && MT == 1), "a gate strip and its up strip, or eight rows of both in one");
+  constexpr bool HALVES = MODE == GATED && NT == 1;
   static_assert(MODE != LINK || (NT == 1 && MT == 1), "one strip of the stream");
   constexpr int T = MT * NT, SLICES = F32_SLICES / WAVES;  // slices of a wave
   constexpr int ENTRIES = SLICES == 4 ? 4 : F32_SLICES;    // sums that meet in LDS: of groups or of slices
@@ -126,12 +126,13 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
   // side by side, so that its L2 reads its share of the weights once.
   const int tile = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (tile >= tiles) return;
-  constexpr int ACROSS = MODE == GATED ? 16 : 16 * NT;
+  constexpr int ACROSS = HALVES ? 8 : MODE == GATED ? 16 : 16 * NT;
   const int n0 = tile / tiles_m * ACROSS, m0 = tile % tiles_m * (16 * MT);
   const int steps = (K + 31) / 32, per = (steps + F32_SLICES - 1) / F32_SLICES;
   const int st0 = min(steps, wave * SLICES * per), st1 = min(steps, st0 + SLICES * per);
 
   auto weight = [&](int i) {  // this lane's row of strip i
+    if constexpr (HALVES) return w + ((size_t)min(n0 + (lr & 7), N - 1) + (size_t)(lr >> 3) * N) * K;
     return w + (MODE == GATED ? (size_t)min(n0 + lr, N - 1) + (size_t)i * N : (size_t)min(n0 + i * 16 + lr, N - 1)) * K;
   };
   const float* wrow[NT];
@@ -187,7 +188,7 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
     for (int u = 0; u < DEPTH; ++u) {
       if (st + u < st1) {
         Parts as[MT], ws[NT];
-        if (!VEC && st + u + SHARE >= steps) {  // K may end among these steps' columns
+        if ((K & 31) && st + u + SHARE >= steps) {  // K may end among these steps' columns
           const int k = (st + u) * 32 + lg * 8, ka = SHARE == 1 ? k : min(st + u + lr / ROWS, steps - 1) * 32 + lg * 8;
 #pragma unroll
           for (int half = 0; half < 2; ++half) {
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
       v = g == 0 ? s : v + s;
     }
     const int m = m0 + t % MT * 16 + lr;
-    const bool mine = m < M && n0 + (MODE == GATED ? 0 : t / MT * 16) + lg * 4 < N;
+    const bool mine = m < M && n0 + (MODE == GATED ? 0 : t / MT * 16) + (HALVES ? lg & 1 : lg) * 4 < N;
     if (__any(mine && !finite(v))) v = again_f32<VEC>(v, weight(t / MT), a + (size_t)min(m, M - 1) * K, K, 0, steps);
     return v;
   };
@@ -263,7 +264,13 @@ __global__ __launch_bounds__(WAVES * 64, MT * NT >= 8 ? 2 : 1) void gemm_f32_row
     const int n = n0 + t / MT * 16 + lg * 4, m = m0 + t % MT * 16 + lr;
     floatx4 v = total(t);
     if (link.ssq_in != nullptr) v *= inv_rms[lr];  // MT = 1: rows 0 .. 15 are the launch's
-    if constexpr (MODE == GATED) {
+    if constexpr (HALVES) {  // lanes 32 .. 63 hold the up rows of lanes 0 .. 31
+      floatx4 up;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(v[r], 32);
+      v = silu_times(v, up);
+      if (lg >= 2) continue;
+    } else if constexpr (MODE == GATED) {
       floatx4 up = total(MT + t);
       if (link.ssq_in != nullptr) up *= inv_rms[lr];
       v = silu_times(v, up);
@@ -329,7 +336,7 @@ __global__ __launch_bounds__(16 / SIDE * 64) void gemm_f32_side_kernel(const flo
 #pragma unroll
     for (int u = 0; u < DEPTH; ++u) {
       if (st + u < per) {
-        if (!VEC && cut) {
+        if (cut) {
           const int k = (first + st + u) * 32 + lg * 8;
 #pragma unroll
           for (int half = 0; half < 2; ++half) {
@@ -711,7 +718,7 @@ template <int MT, int NT, int WAVES, int DEPTH, int SHARE, int MODE>
 static int launch_rows(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
   constexpr size_t lds = (size_t)(WAVES == 4 ? F32_GROUPS : F32_SLICES) * MT * NT * 64 * sizeof(floatx4);
   static_assert(lds + 64 <= 65536, "what a launch may ask for without an attribute");
-  const long tiles = f32_tiles(M, N, 16 * MT, MODE == GATED ? 16 : 16 * NT);
+  const long tiles = f32_tiles(M, N, 16 * MT, MODE == GATED ? 8 * NT : 16 * NT);
   if (tiles > 0x3fffffff) return AS_BAD_SHAPE;
   const int per_xcd = (int)((tiles + 7) / 8), tiles_m = (M + 16 * MT - 1) / (16 * MT);
   if ((K & 3) == 0 && aligned16(a, w))
@@ -739,9 +746,25 @@ template <int MODE> static int launch_strips(const float* a, const float* w, flo
 }
 
 // Two strips a workgroup: on eight waves while that is one round (8,192, 4,096 at 1 / 16 rows 30 / 31 us, on four 39 / 36; 6,144, 1,024 9.7 / 11.5
-// and 10.7 / 11.6), else on four, of which more fit a compute unit (12,288, 2,048 25 / 29, on eight 28 / 33).
+// and 10.7 / 11.6), two steps of up to eight rows side by side (gate and up, 3,072 outputs of 1,024 at 4 / 8 rows 9.8 / 10.3 -> 9.35 / 10.0), else on
+// four, of which more fit a compute unit (12,288, 2,048 25 / 29, on eight 28 / 33).  Gate and up of few outputs, or of so many that
+// several workgroups share a compute unit and up to 4 rows, as one strip of eight rows of either: twice the workgroups (2,048 outputs of 1,024
+// at 4 / 16 rows 9.5 / 10.9 -> 7.4 / 8.6, 6,144 of 2,048 at 4 rows 24.5 -> 22.8, at 16 28.2 and 31.0; 9,728 of 2,560 at 4 rows 46 -> 42.8, 12,288 of
+// 1,024 24.6 and 26.9: five strips to a compute unit at most).
 template <int MODE> static int launch_pairs(const float* a, const float* w, float* out, int M, int N, int K, const LinkF32& link, hipStream_t stream) {
-  if (f32_tiles(M, N, 16, MODE == GATED ? 16 : 32) <= compute_units()) return launch_rows<1, 2, 8, 2, 1, MODE>(a, w, out, M, N, K, link, stream);
+  if constexpr (MODE == GATED) {
+    if (f32_tiles(M, N, 16, 8) <= compute_units()) {
+      if (M <= 8) return launch_rows<1, 1, 8, 2, 2, MODE>(a, w, out, M, N, K, link, stream);
+      return launch_rows<1, 1, 8, 2, 1, MODE>(a, w, out, M, N, K, link, stream);
+    }
+  }
+  if (f32_tiles(M, N, 16, MODE == GATED ? 16 : 32) <= compute_units()) {
+    if (M <= 8) return launch_rows<1, 2, 8, 2, 2, MODE>(a, w, out, M, N, K, link, stream);
+    return launch_rows<1, 2, 8, 2, 1, MODE>(a, w, out, M, N, K, link, stream);
+  }
+  if constexpr (MODE == GATED) {
+    if (M <= 4 && f32_tiles(M, N, 16, 8) <= 5 * compute_units()) return launch_rows<1, 1, 4, 4, 4, MODE>(a, w, out, M, N, K, link, stream);
+  }
   return launch_rows<1, 2, 4, 2, 1, MODE>(a, w, out, M, N, K, link, stream);
 }
 

@@ -1570,6 +1570,23 @@ def test_gemm_f32_gated_and_split_are_the_plain_product(ops, M, N, K):
         assert torch.equal(((s[0] + s[1]) + s[2]) + s[3], want)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 300), (5, 13, 257), (4, 2048, 300), (8, 2047, 1023), (16, 2040, 512), (9, 1, 1024), (3, 2056, 260), (8, 4096, 288),
+                                   (9, 4095, 290), (4, 4104, 290), (2, 10240, 260), (2, 10248, 261), (17, 1000, 516)])  # fmt: skip
+def test_gemm_f32_gate_and_up_in_one_strip(ops, M, N, K):
+    """Gate and up of few rows as strips of eight rows of either or as pairs of strips, on both sides of every line between them: the bits
+    of the plain product's strips with the activation after it, numbers that are not finite included."""
+    torch.manual_seed(N)
+    a, w = torch.randn(M, K, device=DEV), torch.randn(2 * N, K, device=DEV)
+    for spoil in (False, True):
+        if spoil:
+            a[M - 1, K - 1], w[N - 1, K - 2], w[2 * N - 1, 0] = float("inf"), float("nan"), float("-inf")
+        act = torch.empty(M, N, device=DEV)
+        ops.silu_mul(f32_product("as_gemm_f32", a, w, torch.empty(M, 2 * N, device=DEV), 1), act)
+        for form in (0, 3):
+            got = f32_product("as_gemm_f32_gated", a, w, torch.full((M, N), float("nan"), device=DEV), form)
+            assert torch.equal(got.nan_to_num(3.0), act.nan_to_num(3.0)) and torch.equal(got.isnan(), act.isnan())
+
+
 @pytest.mark.parametrize("M,N,K,shift", [(1, 4, 260, 0), (96, 128, 512, 0), (97, 132, 1028, 0), (95, 124, 544, 0), (193, 260, 2080, 0), (98, 70, 1025, 1), (130, 36, 287, 0)])
 def test_gemm_f32_tiles_of_96_rows(ops, M, N, K, shift):
     """Tiles of 96 x 128 outputs, whole, gated and in four partial sums: the bits of strips straight from memory, where the tile's rows, its
