@@ -325,6 +325,8 @@ __global__ void qk_norm_rope_store_kernel(const O* __restrict__ qkv, const W* __
 // of two: a group of D / 16 lanes owns one (token, head) and every lane moves 16-byte pieces
 // (coordinates 8l .. 8l+7 and their partners in the other half), so a wave serves several
 // heads at once and a prompt's rows move at memory speed.  Same arithmetic, same order.
+// The heads are columns of rows of `ld` values: queries from q_off on, keys from k_off, values from v_off.  clean: queries that
+// are not finite are written as zeros too.
 template <typename W> struct Gain8;
 template <> struct Gain8<bf16> {
   static __device__ __forceinline__ void load(const bf16* p, float* g) {
@@ -341,26 +343,33 @@ template <> struct Gain8<float> {
   }
 };
 
-template <typename W>
+// U: what counts the units; PAGE: tokens of a page where the compiler knows them, or 0 (a lane has two pieces to load and to store: a
+// 64-bit division and three by the page are as many instructions as all the rest).
+template <typename W, typename U, int PAGE>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
     const bf16* __restrict__ qkv, const W* __restrict__ qw, const W* __restrict__ kw,
     const float2* __restrict__ cs, const int* __restrict__ slots, bf16* __restrict__ q_out,
-    bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int H, int KV, int D, float eps, int block_size,
-    int heads, size_t units) {
+    bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int H, int KV, int D, float eps, int page_size,
+    int heads, U units, int T, int ld, int q_off, int k_off, int v_off, bool clean) {
   typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-  const int lpu = D >> 4, half = D >> 1;  // lanes per (token, head)
-  const size_t unit = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) / lpu;
+  const int lpu = D >> 4, half = D >> 1, block_size = PAGE ? PAGE : page_size;  // lanes per (token, head)
+  const U unit = ((U)blockIdx.x * 256 + threadIdx.x) >> (__ffs(lpu) - 1);
   const int l = threadIdx.x & (lpu - 1);
   if (unit >= units) return;  // whole groups leave: the shuffles below stay inside a group
-  const size_t t = unit / heads;
-  const int hs = (int)(unit % heads);
-  const bf16* src = qkv + (t * (H + 2 * KV) + hs) * D;
+  // Eight tokens' units of a head lie side by side: with heads of 128 they are a wave's, and their values' lines are read once
+  // (with a token's heads side by side a line's eight readers were on as many XCDs: 2,409 tokens of 48 heads 20 us either way; 1,500 of 24 10.0 -> 8.2).
+  const U eight = unit / (8 * heads), rest = unit - eight * (8 * heads);
+  const size_t t = (size_t)eight * 8 + (rest & 7);
+  const int hs = (int)(rest >> 3);
+  if (t >= (size_t)T) return;
   const bool is_q = hs < H, is_k = !is_q && hs < H + KV;
+  const int column = is_q ? q_off + hs * D : is_k ? k_off + (hs - H) * D : v_off + (hs - H - KV) * D;
+  const bf16* src = qkv + t * ld + column;
   bf16* dst;
   if (!is_q && !is_k) {  // values: transposed within the page
     const int slot = slots[t];
     if (slot < 0) return;  // uniform over the group
-    const size_t head = (size_t)(slot / block_size) * KV + (hs - H - KV);
+    const size_t head = (size_t)((unsigned)slot / block_size) * KV + (hs - H - KV);
     // A prompt's tokens fill a page slot after slot.  Where eight tokens in a row go to eight
     // slots in a row that start at a multiple of eight, a coordinate's eight values are 16
     // contiguous bytes of the transposed page, where token by token they would be eight stores
@@ -369,7 +378,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
     // rows and stores two 16-byte pieces.
     const int nth = slot & 7;
     const long lead = (long)t - nth;
-    bool run = (block_size & 7) == 0 && lead >= 0 && lead + 8 <= (long)(units / heads);
+    bool run = (block_size & 7) == 0 && lead >= 0 && lead + 8 <= T;
     if (run) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) run = run && slots[lead + i] == slot - nth + i;
@@ -377,24 +386,24 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
     if (run) {  // uniform over the lanes of this (token, head), and the same for all eight tokens
       typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
       const int d0 = nth * (D >> 3) + 2 * l;
-      const bf16* first = qkv + ((size_t)lead * (H + 2 * KV) + hs) * D + d0;
+      const bf16* first = qkv + (size_t)lead * ld + column + d0;
       bf16x2 pair[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) pair[i] = *reinterpret_cast<const bf16x2*>(first + (size_t)i * (H + 2 * KV) * D);
+      for (int i = 0; i < 8; ++i) pair[i] = *reinterpret_cast<const bf16x2*>(first + (size_t)i * ld);
       bf16x8 oa, ob;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         oa[i] = finite_or_zero((bf16)pair[i][0]);
         ob[i] = finite_or_zero((bf16)pair[i][1]);
       }
-      bf16* vt = v_pages + head * block_size * D + (slot - nth) % block_size;
+      bf16* vt = v_pages + head * block_size * D + (unsigned)(slot - nth) % block_size;
       *reinterpret_cast<bf16x8*>(vt + (size_t)d0 * block_size) = oa;
       *reinterpret_cast<bf16x8*>(vt + (size_t)(d0 + 1) * block_size) = ob;
       return;
     }
     const bf16x8 a8 = *reinterpret_cast<const bf16x8*>(src + 8 * l);
     const bf16x8 b8 = *reinterpret_cast<const bf16x8*>(src + half + 8 * l);
-    bf16* vt = v_pages + head * block_size * D + slot % block_size;
+    bf16* vt = v_pages + head * block_size * D + (unsigned)slot % block_size;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       vt[(size_t)(8 * l + j) * block_size] = finite_or_zero((bf16)a8[j]);
@@ -409,8 +418,8 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
   } else {
     const int slot = slots[t];
     if (slot < 0) return;  // uniform over the group
-    const size_t head = (size_t)(slot / block_size) * KV + (hs - H);
-    dst = k_pages + (head * block_size + slot % block_size) * D;
+    const size_t head = (size_t)((unsigned)slot / block_size) * KV + (hs - H);
+    dst = k_pages + (head * block_size + (unsigned)slot % block_size) * D;
   }
   const W* w = is_q ? qw : kw;
   float inv = 1.0f;
@@ -441,11 +450,15 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
   for (int j = 0; j < 8; ++j) {
     float a = (float)a8[j] * inv, b = (float)b8[j] * inv;
     if (w) { a *= ga[j]; b *= gb[j]; }
-    float c = 1.f, sn = 0.f;
-    if (cs) { c = (j & 1) ? turn[j >> 1].z : turn[j >> 1].x; sn = (j & 1) ? turn[j >> 1].w : turn[j >> 1].y; }
-    oa[j] = (bf16)(a * c - b * sn);
-    ob[j] = (bf16)(b * c + a * sn);
-    if (is_k) { oa[j] = finite_or_zero((bf16)oa[j]); ob[j] = finite_or_zero((bf16)ob[j]); }
+    if (cs) {
+      const float c = (j & 1) ? turn[j >> 1].z : turn[j >> 1].x, sn = (j & 1) ? turn[j >> 1].w : turn[j >> 1].y;
+      oa[j] = (bf16)(a * c - b * sn);
+      ob[j] = (bf16)(b * c + a * sn);
+    } else {
+      oa[j] = (bf16)a;
+      ob[j] = (bf16)b;
+    }
+    if (is_k || clean) { oa[j] = finite_or_zero((bf16)oa[j]); ob[j] = finite_or_zero((bf16)ob[j]); }
   }
   *reinterpret_cast<bf16x8*>(dst + 8 * l) = oa;
   *reinterpret_cast<bf16x8*>(dst + half + 8 * l) = ob;
@@ -461,16 +474,21 @@ extern "C" int as_qk_norm_rope_store(const void* qkv, int dtype, const void* qw,
   const int lpu = D >> 4;
   if (dtype == DT_BF16 && R == D && (D & 15) == 0 && lpu <= WAVE && (lpu & (lpu - 1)) == 0) {
     const int heads = store_kv ? H + 2 * KV : H;
-    const size_t units = (size_t)num_tokens * heads;
+    const size_t units = ((size_t)num_tokens + 7) / 8 * 8 * heads;
     const size_t blocks = (units * lpu + 255) / 256;
     if (blocks > 0x7fffffff) return AS_BAD_SHAPE;
+    const bool known = block_size == 16 && blocks * 256 <= 0xffffffff;
 #define LAUNCH8(W)                                                                                   \
-  qk_norm_rope_store_bf16x8_kernel<W><<<(int)blocks, 256, 0, stream>>>(                              \
+  if (known) LAUNCH9(W, unsigned, 16);                                                               \
+  else LAUNCH9(W, size_t, 0)
+#define LAUNCH9(W, U, PAGE)                                                                          \
+  qk_norm_rope_store_bf16x8_kernel<W, U, PAGE><<<(int)blocks, 256, 0, stream>>>(                     \
       (const bf16*)qkv, (const W*)qw, (const W*)kw, (const float2*)cs, slots, (bf16*)q_out,          \
-      (bf16*)k_pages, (bf16*)v_pages, H, KV, D, eps, block_size, heads, units)
-    if (w_dtype == DT_BF16) LAUNCH8(bf16);
-    else if (w_dtype == DT_F32) LAUNCH8(float);
+      (bf16*)k_pages, (bf16*)v_pages, H, KV, D, eps, block_size, heads, (U)units, num_tokens, (H + 2 * KV) * D, 0, H * D, (H + KV) * D, false)
+    if (w_dtype == DT_BF16) { LAUNCH8(bf16); }
+    else if (w_dtype == DT_F32) { LAUNCH8(float); }
     else return AS_BAD_DTYPE;
+#undef LAUNCH9
 #undef LAUNCH8
     return launch_status();
   }
@@ -729,6 +747,31 @@ extern "C" int as_head_norm_store(const void* proj, int dtype, int ld, int q_off
   if (H <= 0 || KV <= 0 || dim <= 0 || vdim <= 0 || Dp < dim || Dp < vdim || bs <= 0 || ld <= 0 || (!qw) != (!kw))
     return AS_BAD_SHAPE;
   if (H + 2 * KV > 65535) return AS_BAD_SHAPE;
+  // bf16 heads of one width that is 16 times a power of two, turned whole or not at all, in rows and columns on 16 bytes: several heads to a
+  // wave in 16-byte pieces (1,500 tokens of 24 heads of 128 in rows of 7,168, 16.3 us with a wave of 64 threads a head: 10.2, with eight tokens of a head side by side 8.2)
+  const int lpu = dim >> 4;
+  const bool store_kv = store && slots;
+  const uintptr_t bases = (uintptr_t)proj | (uintptr_t)qw | (uintptr_t)kw | (uintptr_t)cs | (uintptr_t)q_out |
+                          (store_kv ? (uintptr_t)k_pages | (uintptr_t)v_pages : 0);
+  if (dtype == DT_BF16 && dim == vdim && dim == Dp && (dim & 15) == 0 && lpu <= WAVE && (lpu & (lpu - 1)) == 0 && (!cs || R == dim) &&
+      ((ld | q_off | k_off | v_off) & 7) == 0 && (bases & 15) == 0 && (!qw || w_dtype == DT_BF16 || w_dtype == DT_F32)) {
+    const int heads = store_kv ? H + 2 * KV : H;
+    const size_t units = ((size_t)num_tokens + 7) / 8 * 8 * heads, blocks = (units * lpu + 255) / 256;
+    if (blocks > 0x7fffffff) return AS_BAD_SHAPE;
+    const bool known = bs == 16 && blocks * 256 <= 0xffffffff;
+#define LAUNCH8(W)                                                                                                       \
+  if (known) LAUNCH9(W, unsigned, 16);                                                                                   \
+  else LAUNCH9(W, size_t, 0)
+#define LAUNCH9(W, U, PAGE)                                                                                              \
+  qk_norm_rope_store_bf16x8_kernel<W, U, PAGE><<<(int)blocks, 256, 0, stream>>>(                                         \
+      (const bf16*)proj, (const W*)qw, (const W*)kw, (const float2*)cs, slots, (bf16*)q_out, (bf16*)k_pages,             \
+      (bf16*)v_pages, H, KV, dim, eps, bs, heads, (U)units, num_tokens, ld, q_off, k_off, v_off, true)
+    if (qw && w_dtype == DT_F32) { LAUNCH8(float); }
+    else { LAUNCH8(bf16); }
+#undef LAUNCH9
+#undef LAUNCH8
+    return launch_status();
+  }
   dim3 grid(num_tokens, H + 2 * KV);
 #define LAUNCH(T, W)                                                                                          \
   head_norm_store_kernel<T, W><<<grid, 64, 0, stream>>>((const T*)proj, ld, q_off, k_off, v_off, H, KV, dim,  \

@@ -49,28 +49,52 @@ __global__ __launch_bounds__(1024) void moe_route_table_kernel(const int* __rest
   __shared__ int hist[MOE_MAX_EXPERTS];
   __shared__ int cursor[MOE_MAX_EXPERTS];
   const int P = num_tokens * top;
+  // A thread's first pairs stay in registers between the two passes: their loads, one behind the other, are asked for together
+  // (3,000 pairs of 16 experts: each pass by itself 11.4 us, now 8.3).
+  constexpr int HELD = 4;
+  int mine[HELD];
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) {
+    const int p = threadIdx.x + i * blockDim.x;
+    mine[i] = p < P ? expert_of_pair(token_ids, table, vocab, top, experts, identity, p) : -1;
+  }
   for (int e = threadIdx.x; e < experts; e += blockDim.x) hist[e] = 0;
   __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
+#pragma unroll
+  for (int i = 0; i < HELD; ++i)
+    if (mine[i] >= 0) atomicAdd(&hist[mine[i]], 1);
+  for (int p = threadIdx.x + HELD * blockDim.x; p < P; p += blockDim.x) {
     const int e = expert_of_pair(token_ids, table, vocab, top, experts, identity, p);
     if (e >= 0) atomicAdd(&hist[e], 1);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < WAVE) {  // a lane an expert, 64 at a time: where its pairs and its tiles start
     int at = 0, n = 0;
-    for (int e = 0; e < experts; ++e) {
-      cursor[e] = at;
-      for (int s = 0; s < hist[e] && n < max_tiles; s += size, ++n) {
-        tiles[3 * n] = e;
-        tiles[3 * n + 1] = at + s;
-        tiles[3 * n + 2] = min(size, hist[e] - s);
+    for (int e0 = 0; e0 < experts; e0 += WAVE) {
+      const int e = e0 + threadIdx.x, pairs = e < experts ? hist[e] : 0, parts = (pairs + size - 1) / size;
+      int pairs_to = pairs, parts_to = parts;  // of the experts up to this one
+#pragma unroll
+      for (int d = 1; d < WAVE; d <<= 1) {
+        const int a = __shfl_up(pairs_to, d), b = __shfl_up(parts_to, d);
+        if ((int)threadIdx.x >= d) { pairs_to += a; parts_to += b; }
       }
-      at += hist[e];
+      const int first = at + pairs_to - pairs, tile = n + parts_to - parts;
+      if (e < experts) cursor[e] = first;
+      for (int i = 0; i < parts && tile + i < max_tiles; ++i) {
+        tiles[3 * (tile + i)] = e;
+        tiles[3 * (tile + i) + 1] = first + i * size;
+        tiles[3 * (tile + i) + 2] = min(size, pairs - i * size);
+      }
+      at += __shfl(pairs_to, WAVE - 1);
+      n += __shfl(parts_to, WAVE - 1);
     }
-    counts[0] = n;
+    if (threadIdx.x == 0) counts[0] = min(n, max_tiles);
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
+#pragma unroll
+  for (int i = 0; i < HELD; ++i)
+    if (mine[i] >= 0) order[atomicAdd(&cursor[mine[i]], 1)] = threadIdx.x + i * blockDim.x;
+  for (int p = threadIdx.x + HELD * blockDim.x; p < P; p += blockDim.x) {
     const int e = expert_of_pair(token_ids, table, vocab, top, experts, identity, p);
     if (e >= 0) order[atomicAdd(&cursor[e], 1)] = p;
   }
@@ -794,6 +818,30 @@ __global__ void moe_combine_kernel(const float* __restrict__ pair_out, int top, 
   }
 }
 
+// The same for rows of whole pieces of four values on 16 (outputs, 8 in bf16) bytes: a workgroup a token and 1,024 of its columns (3,000 pairs of
+// 2,048 for 1,500 tokens, 31 MB: value by value 10.5 us, now 6.6).
+template <typename T>
+__global__ __launch_bounds__(256) void moe_combine_four_kernel(const float* __restrict__ pair_out, int top, float weight, int N,
+                                                               T* __restrict__ out, const float* __restrict__ pair_weight,
+                                                               const T* __restrict__ add, const T* __restrict__ same,
+                                                               const int* __restrict__ pair_expert, int experts) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  typedef T tx4 __attribute__((ext_vector_type(4)));
+  const size_t t = blockIdx.x;
+  const int n = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (n >= N) return;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < top; ++j) {
+    const size_t pair = t * top + j;
+    const bool is_same = same && pair_expert[pair] >= experts;
+    const f32x4 v = is_same ? __builtin_convertvector(*reinterpret_cast<const tx4*>(same + t * N + n), f32x4)
+                            : *reinterpret_cast<const f32x4*>(pair_out + pair * N + n);
+    s += weight * (pair_weight ? pair_weight[pair] : 1.f) * v;
+  }
+  if (add) s += __builtin_convertvector(*reinterpret_cast<const tx4*>(add + t * N + n), f32x4);
+  *reinterpret_cast<tx4*>(out + t * N + n) = __builtin_convertvector(s, tx4);
+}
+
 extern "C" int as_moe_combine(const float* pair_out, int top, float weight, int N, void* out, int out_dtype,
                               int num_tokens, const float* pair_weight, const void* add, const void* same,
                               const int* pair_expert, int experts, hipStream_t stream) {
@@ -801,6 +849,14 @@ extern "C" int as_moe_combine(const float* pair_out, int top, float weight, int 
   if (top <= 0 || N <= 0 || (same && !pair_expert)) return AS_BAD_SHAPE;
   const size_t total = (size_t)num_tokens * N, want = (total + 255) / 256;
   const int blocks = (int)(want > 8192 ? 8192 : want);
+  const uintptr_t typed = (uintptr_t)out | (uintptr_t)add | (uintptr_t)same;
+  if ((N & 3) == 0 && ((uintptr_t)pair_out & 15) == 0 && (typed & (out_dtype == DT_F32 ? 15 : 7)) == 0 && (N + 1023) / 1024 <= 65535 &&
+      (out_dtype == DT_F32 || out_dtype == DT_BF16)) {
+    const dim3 grid(num_tokens, (N + 1023) / 1024);
+    if (out_dtype == DT_F32) moe_combine_four_kernel<float><<<grid, 256, 0, stream>>>(pair_out, top, weight, N, (float*)out, pair_weight, (const float*)add, (const float*)same, pair_expert, experts);
+    else moe_combine_four_kernel<bf16><<<grid, 256, 0, stream>>>(pair_out, top, weight, N, (bf16*)out, pair_weight, (const bf16*)add, (const bf16*)same, pair_expert, experts);
+    return launch_status();
+  }
   if (out_dtype == DT_F32) moe_combine_kernel<float><<<blocks, 256, 0, stream>>>(pair_out, top, weight, N, (float*)out, total, pair_weight, (const float*)add, (const float*)same, pair_expert, experts);
   else if (out_dtype == DT_BF16) moe_combine_kernel<bf16><<<blocks, 256, 0, stream>>>(pair_out, top, weight, N, (bf16*)out, total, pair_weight, (const bf16*)add, (const bf16*)same, pair_expert, experts);
   else return AS_BAD_DTYPE;

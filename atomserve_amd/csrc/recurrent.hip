@@ -240,6 +240,54 @@ __global__ __launch_bounds__(256) void delta_prepare_kernel(float* __restrict__ 
   }
 }
 
+// Sums over neighbouring lanes, 16, 32 or 64, in every one of them.
+template <int LANES> __device__ __forceinline__ float lanes_sum(float v) {
+  if constexpr (LANES == 64) return wave_sum(v);
+  if constexpr (LANES == 32) v = plus_16(v);
+  v += dpp<DPP_ROTATE(8)>(v);
+  v += dpp<DPP_ROTATE(4)>(v);
+  v += dpp<DPP_XOR_2>(v);
+  return v + dpp<DPP_XOR_1>(v);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <typename T> struct Four;  // four neighbouring values
+template <> struct Four<float> {
+  static __device__ __forceinline__ f32x4 load(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+  static __device__ __forceinline__ void store(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+};
+template <> struct Four<bf16> {
+  typedef bf16 V __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ f32x4 load(const bf16* p) { return __builtin_convertvector(*reinterpret_cast<const V*>(p), f32x4); }
+  static __device__ __forceinline__ void store(bf16* p, f32x4 v) { *reinterpret_cast<V*>(p) = __builtin_convertvector(v, V); }
+};
+// Whether p, and what lies `a` and `b` elements further, start on four elements of `size` bytes.
+static bool on_four(const void* p, int size, long a, long b) { return ((uintptr_t)p & (4 * size - 1)) == 0 && ((a | b) & 3) == 0; }
+
+// The same for heads of 64, 128 and 256 in rows on 16 bytes: a head is 16 to 64 lanes' work, four coordinates each, the heads of all tokens
+// one after the other (1,500 tokens of 16 heads of 128, 24 MB: a token to a workgroup, one head of a wave after the other 10.5 us, now 7.3).
+template <typename T, typename W, int LANES>
+__global__ __launch_bounds__(256) void delta_prepare_four_kernel(float* __restrict__ qkv, int C, int G, int H, const T* __restrict__ proj,
+                                                                 int ld, int b_off, int a_off, const W* __restrict__ a_log,
+                                                                 const W* __restrict__ dt_bias, float* __restrict__ beta,
+                                                                 float* __restrict__ decay, size_t units) {
+  const size_t mine = ((size_t)blockIdx.x * 256 + threadIdx.x) / LANES, unit = mine < units ? mine : units - 1;
+  const int l = threadIdx.x % LANES, head = (int)(unit % (2 * G));
+  const size_t t = unit / (2 * G);
+  float* x = qkv + t * C + (size_t)head * (4 * LANES) + 4 * l;
+  const f32x4 v = Four<float>::load(x);
+  const float ss = lanes_sum<LANES>((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]));
+  if (mine >= units) return;
+  float f = 1.0f / sqrtf(ss + 1e-6f);
+  if (head < G) f *= 1.0f / sqrtf((float)(4 * LANES));
+  Four<float>::store(x, v * f);
+  for (int h = head * LANES + l; h < H; h += 2 * G * LANES) {
+    const float b = to_f32(proj[t * ld + b_off + h]), a = to_f32(proj[t * ld + a_off + h]);
+    beta[t * H + h] = sigmoidf_(b);
+    decay[t * H + h] = expf(-expf(to_f32(a_log[h])) * softplusf_(a + to_f32(dt_bias[h])));
+  }
+}
+
 extern "C" int as_delta_prepare(float* qkv, int C, int G, int dim, int H, const void* proj, int dtype, int ld, int b_off,
                                 int a_off, const void* a_log, const void* dt_bias, int w_dtype, float* beta,
                                 float* decay, int num_tokens, hipStream_t stream) {
@@ -247,13 +295,22 @@ extern "C" int as_delta_prepare(float* qkv, int C, int G, int dim, int H, const 
   if (G <= 0 || dim <= 0 || H <= 0 || C < 2 * G * dim) return AS_BAD_SHAPE;
   const int across = num_tokens >= 512 ? 1 : (2 * G + 3) / 4 > 64 ? 64 : (2 * G + 3) / 4;  // many tokens fill the GPU by themselves
   dim3 grid(num_tokens, across);
+  const size_t units = (size_t)num_tokens * 2 * G, blocks = (units * (dim / 4) + 255) / 256;
+  const bool four = (dim == 64 || dim == 128 || dim == 256) && on_four(qkv, 4, C, 0) && blocks <= 0x7fffffff;
+#define FOUR(T, W, LANES)                                                                                          \
+  delta_prepare_four_kernel<T, W, LANES><<<(int)blocks, 256, 0, stream>>>(                                         \
+      qkv, C, G, H, (const T*)proj, ld, b_off, a_off, (const W*)a_log, (const W*)dt_bias, beta, decay, units)
 #define LAUNCH(T, W)                                                                                               \
-  delta_prepare_kernel<T, W><<<grid, 256, 0, stream>>>(qkv, C, G, dim, H, (const T*)proj, ld, b_off, a_off,        \
+  if (four && dim == 64) FOUR(T, W, 16);                                                                           \
+  else if (four && dim == 128) FOUR(T, W, 32);                                                                     \
+  else if (four) FOUR(T, W, 64);                                                                                   \
+  else delta_prepare_kernel<T, W><<<grid, 256, 0, stream>>>(qkv, C, G, dim, H, (const T*)proj, ld, b_off, a_off,        \
                                                        (const W*)a_log, (const W*)dt_bias, beta, decay)
-  if (dtype == DT_F32 && w_dtype == DT_F32) LAUNCH(float, float);
-  else if (dtype == DT_BF16 && w_dtype == DT_BF16) LAUNCH(bf16, bf16);
-  else if (dtype == DT_BF16 && w_dtype == DT_F32) LAUNCH(bf16, float);
+  if (dtype == DT_F32 && w_dtype == DT_F32) { LAUNCH(float, float); }
+  else if (dtype == DT_BF16 && w_dtype == DT_BF16) { LAUNCH(bf16, bf16); }
+  else if (dtype == DT_BF16 && w_dtype == DT_F32) { LAUNCH(bf16, float); }
   else return AS_BAD_DTYPE;
+#undef FOUR
 #undef LAUNCH
   return launch_status();
 }
@@ -964,6 +1021,25 @@ __global__ __launch_bounds__(64) void delta_finish_kernel(const float* __restric
   }
 }
 
+// The same for heads of 64, 128 and 256 on pieces of four values, as in delta_prepare (1,500 tokens of 16 heads of 128, 24 MB: a workgroup of
+// 64 threads a head 10.5 us, now 7.6).
+template <typename T, typename W, int LANES>
+__global__ __launch_bounds__(256) void delta_finish_four_kernel(const float* __restrict__ o, int H, const W* __restrict__ w, int w_stride,
+                                                                float eps, const T* __restrict__ gate, int ld, int g_off, int gate_act,
+                                                                float scale, T* __restrict__ act, int ld_out, int out_off, size_t units) {
+  const size_t mine = ((size_t)blockIdx.x * 256 + threadIdx.x) / LANES, unit = mine < units ? mine : units - 1;
+  const int d = 4 * (threadIdx.x % LANES), h = (int)(unit % H);
+  const size_t t = unit / H;
+  const f32x4 x = Four<float>::load(o + unit * (4 * LANES) + d), z = Four<T>::load(gate + t * ld + g_off + (size_t)h * (4 * LANES) + d),
+              g = Four<W>::load(w + (size_t)h * w_stride + d);
+  const float ss = lanes_sum<LANES>((x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]));
+  const float inv = scale / sqrtf(ss / (float)(4 * LANES) + eps);
+  f32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = x[i] * inv * g[i] * (gate_act == 1 ? sigmoidf_(z[i]) : siluf_(z[i]));
+  if (mine < units) Four<T>::store(act + t * ld_out + out_off + (size_t)h * (4 * LANES) + d, r);
+}
+
 extern "C" int as_delta_finish(const float* o, int H, int vdim, const void* w, int w_dtype, int w_per_head, float eps,
                                const void* gate, int dtype, int ld, int g_off, int gate_act, float scale, void* act,
                                int ld_out, int out_off, int num_tokens, hipStream_t stream) {
@@ -972,14 +1048,25 @@ extern "C" int as_delta_finish(const float* o, int H, int vdim, const void* w, i
       ld_out < out_off + H * vdim)
     return AS_BAD_SHAPE;
   dim3 grid(num_tokens, H);
-  const int w_stride = w_per_head ? vdim : 0;
+  const int w_stride = w_per_head ? vdim : 0, size = dtype == DT_F32 ? 4 : 2;
+  const size_t units = (size_t)num_tokens * H, blocks = (units * (vdim / 4) + 255) / 256;
+  const bool four = (vdim == 64 || vdim == 128 || vdim == 256) && on_four(o, 4, 0, 0) && on_four(gate, size, ld, g_off) &&
+                    on_four(act, size, ld_out, out_off) && on_four(w, w_dtype == DT_F32 ? 4 : 2, 0, 0) && blocks <= 0x7fffffff;
+#define FOUR(T, W, LANES)                                                                                          \
+  delta_finish_four_kernel<T, W, LANES><<<(int)blocks, 256, 0, stream>>>(                                          \
+      o, H, (const W*)w, w_stride, eps, (const T*)gate, ld, g_off, gate_act, scale, (T*)act, ld_out, out_off, units)
 #define LAUNCH(T, W)                                                                                               \
-  delta_finish_kernel<T, W><<<grid, 64, 0, stream>>>(o, H, vdim, (const W*)w, w_stride, eps, (const T*)gate, ld,  \
-                                                     g_off, gate_act, scale, (T*)act, ld_out, out_off)
-  if (dtype == DT_F32 && w_dtype == DT_F32) LAUNCH(float, float);
-  else if (dtype == DT_BF16 && w_dtype == DT_BF16) LAUNCH(bf16, bf16);
-  else if (dtype == DT_BF16 && w_dtype == DT_F32) LAUNCH(bf16, float);
+  if (four && vdim == 64) FOUR(T, W, 16);                                                                          \
+  else if (four && vdim == 128) FOUR(T, W, 32);                                                                    \
+  else if (four) FOUR(T, W, 64);                                                                                   \
+  else delta_finish_kernel<T, W><<<grid, 64, 0, stream>>>((const float*)o, H, vdim, (const W*)w, w_stride, eps,     \
+                                                          (const T*)gate, ld, g_off, gate_act, scale, (T*)act,     \
+                                                          ld_out, out_off)
+  if (dtype == DT_F32 && w_dtype == DT_F32) { LAUNCH(float, float); }
+  else if (dtype == DT_BF16 && w_dtype == DT_BF16) { LAUNCH(bf16, bf16); }
+  else if (dtype == DT_BF16 && w_dtype == DT_F32) { LAUNCH(bf16, float); }
   else return AS_BAD_DTYPE;
+#undef FOUR
 #undef LAUNCH
   return launch_status();
 }

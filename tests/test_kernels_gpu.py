@@ -1344,6 +1344,104 @@ def test_portions_and_single_queries_in_one_launch(ops, monkeypatch, H, KV, D, w
         assert torch.allclose(out.float(), two.float(), atol=2e-2, rtol=2e-2), plan
 
 
+@pytest.mark.parametrize("T,H,KV,D,bs,gain,turned", [(1, 3, 1, 16, 16, None, False), (7, 4, 2, 64, 16, BF16, True), (33, 6, 2, 128, 16, F32, False), (40, 2, 2, 128, 32, BF16, False),
+                                                      (9, 1, 1, 256, 16, None, True), (8, 2, 1, 1024, 16, F32, True)])
+def test_head_norm_store_in_wide_pieces(ops, T, H, KV, D, bs, gain, turned):
+    """Heads whose rows and columns start on 16 bytes, several to a wave, against one that starts one column further, a wave a head: the
+    same within a rounding of bf16 (the squares are summed in another order); numbers that are not finite are zeros in both."""
+    torch.manual_seed(D + T)
+    width = (H + 2 * KV) * D
+    wide = torch.randn(T, width + 16, device=DEV).to(BF16)
+    wide[0, 8], wide[T - 1, 8 + H * D + 3], wide[T // 2, 8 + (H + KV) * D + 1] = float("inf"), float("nan"), float("-inf")
+    odd = torch.zeros(T, width + 17, device=DEV).to(BF16)
+    odd[:, 9 : 9 + width] = wide[:, 8 : 8 + width]
+    gains = [None, None] if gain is None else [(1 + 0.1 * torch.randn(D, device=DEV)).to(gain) for _ in range(2)]
+    cs = torch.randn(T, D // 2, 2, device=DEV) if turned else None
+    pages = -(-T // bs) + 2
+    slots = torch.arange(T) + bs + (3 if T == 9 else 0)  # runs of eight, and (9 tokens) runs that start within one
+    slots[T // 3] = -1 if T > 8 else slots[T // 3]
+    for store in (True, False):
+        got = []
+        for proj, at in ((wide, 8), (odd, 9)):
+            q = torch.full((T, H, D), 7.0, device=DEV).to(BF16)
+            k, v = torch.zeros(pages, KV, bs, D, device=DEV).to(BF16), torch.zeros(pages, KV, D, bs, device=DEV).to(BF16)
+            ops.head_norm_store(proj, at, at + H * D, at + (H + KV) * D, H, KV, D, D, *gains, 1e-6, i32(slots.tolist()), q, k, v, store_kv=store, cos_sin=cs)
+            got.append((q, k, v))
+        for x, y in zip(*got):
+            assert x.isfinite().all() and torch.allclose(x.float(), y.float(), rtol=2.0**-7, atol=1e-6)
+        assert torch.equal(got[0][2], got[1][2])  # values are copied
+
+
+@pytest.mark.parametrize("T,H,D,dtype,w_dtype", [(1, 2, 64, BF16, BF16), (5, 3, 128, BF16, F32), (3, 5, 256, F32, F32), (301, 4, 128, BF16, BF16)])
+def test_delta_heads_in_pieces_of_four(ops, T, H, D, dtype, w_dtype):
+    """What stands before and after the delta rule, for heads that start on four values and for those that do not, against 64 bits: 32-bit
+    sums of up to 256 squares round to 256 * 2^-24, the exponentials' functions to a few units of it; bf16 outputs to 2^-8."""
+    torch.manual_seed(D)
+    o, w = torch.randn(T, H, D, device=DEV), (1 + 0.1 * torch.randn(H, D, device=DEV)).to(w_dtype)
+    z = torch.randn(T, H * D, device=DEV).to(dtype)
+    x, zd = o.double(), z.double().view(T, H, D)
+    want = (0.5 * x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt() * w.double() * zd * torch.sigmoid(zd)).view(T, H * D)
+    for off in (4, 5):
+        proj = torch.cat([torch.zeros(T, off, device=DEV).to(dtype), z, torch.zeros(T, 8 - off, device=DEV).to(dtype)], 1).contiguous()
+        act = torch.zeros(T, H * D + 8, device=DEV).to(dtype)
+        ops.delta_finish(o, w, 1e-5, proj, off, act, scale=0.5, out_off=off)
+        assert torch.allclose(act[:, off : off + H * D].double(), want, rtol=2.0**-8 if dtype == BF16 else 1e-4, atol=1e-6)
+        assert not act[:, :off].any() and not act[:, off + H * D :].any()
+    G = 2
+    heads = torch.randn(T, 2 * G, D, device=DEV)
+    raw = heads.double()
+    unit = raw / (raw.square().sum(-1, keepdim=True) + 1e-6).sqrt()
+    unit[:, :G] *= D**-0.5
+    b, a = torch.randn(T, H, device=DEV).to(dtype), torch.randn(T, H, device=DEV).to(dtype)
+    log, bias = torch.randn(H, device=DEV).to(w_dtype), torch.randn(H, device=DEV).to(w_dtype)
+    for extra in (4, 1):  # channels behind the heads: rows on 16 bytes, and not
+        qkv = torch.cat([heads.view(T, -1), torch.full((T, extra), 3.0, device=DEV)], 1).contiguous()
+        beta, decay = torch.zeros(T, H, device=DEV), torch.zeros(T, H, device=DEV)
+        ops.delta_prepare(qkv, G, D, H, torch.cat([b, a], 1).contiguous(), 0, H, log, bias, beta, decay)
+        assert torch.allclose(qkv[:, : 2 * G * D].double().view(T, 2 * G, D), unit, rtol=1e-4, atol=1e-7) and bool((qkv[:, 2 * G * D :] == 3).all())
+        assert torch.allclose(beta.double(), torch.sigmoid(b.double()), rtol=1e-5)
+        assert torch.allclose(decay.double(), torch.exp(-log.double().exp() * torch.nn.functional.softplus(a.double() + bias.double())), rtol=1e-4, atol=1e-7)
+
+
+@pytest.mark.parametrize("T,top,experts,tile", [(1, 1, 1, 64), (3, 2, 5, 64), (1500, 2, 16, 128), (2100, 2, 200, 64), (5000, 1, 64, 64)])
+def test_pairs_of_more_than_a_threads_registers_are_routed(ops, T, top, experts, tile):
+    """Every pair stands once among its expert's, and the tiles cover each expert's pairs in order, for pairs up to and beyond those that
+    threads hold between the two passes, and more experts than lanes."""
+    torch.manual_seed(experts)
+    table = torch.stack([torch.randperm(max(experts, top))[:top] % experts for _ in range(300)]).int()
+    ids = torch.randint(0, 300, (T,))
+    route = ops.moe_route_table(i32(ids.tolist()), table.to(DEV), experts, tile=tile)
+    chosen = table[ids].reshape(-1)
+    order, n = route.order.cpu()[: T * top], int(route.counts[0])
+    assert sorted(order.tolist()) == list(range(T * top)) and torch.equal(chosen[order.long()], chosen.sort().values)
+    at, want = 0, []
+    for e, pairs in enumerate(torch.bincount(chosen, minlength=experts).tolist()):
+        want += [[e, at + i, min(tile, pairs - i)] for i in range(0, pairs, tile)]
+        at += pairs
+    assert route.tiles.cpu().view(-1, 3)[:n].tolist() == want
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("T,top,N", [(1, 1, 4), (5, 3, 1028), (3, 2, 70)])
+def test_outputs_of_experts_are_added_up_in_pieces_of_four(ops, T, top, N, dtype):
+    """Whole pieces of four and other widths, with everything that a sum may hold: products and additions round to 2^-24 of their sizes."""
+    torch.manual_seed(N)
+    pairs, weights = torch.randn(T * top, N, device=DEV), torch.rand(T * top, device=DEV)
+    add, same = torch.randn(T, N, device=DEV).to(dtype), torch.randn(T, N, device=DEV).to(dtype)
+    chosen = torch.arange(T * top) % 3
+    for kw in ({}, dict(pair_weight=weights), dict(pair_weight=weights, add=add, same=same, pair_expert=i32(chosen.tolist()), experts=2)):
+        out = torch.zeros(T, N, device=DEV).to(dtype)
+        ops.moe_combine(pairs, top, 0.5, out, **kw)
+        terms = pairs.double().view(T, top, N).clone()
+        if "same" in kw:
+            terms = torch.where((chosen >= 2).view(T, top, 1).to(DEV), same.double()[:, None], terms)
+        terms = 0.5 * terms * (weights.double().view(T, top, 1) if "pair_weight" in kw else 1.0)
+        want, size = terms.sum(1), terms.abs().sum(1)
+        if "add" in kw:
+            want, size = want + add.double(), size + add.double().abs()
+        assert bool(((out.double() - want).abs() <= size * (top + 3) * 2.0**-24 + (want.abs() * 2.0**-8 if dtype == BF16 else 0.0)).all())
+
+
 def test_kernels_refuse_what_they_cannot_do(ops):
     from atomserve_amd.kernels.lib import KernelError
 
