@@ -1563,11 +1563,12 @@ extern "C" int as_attn_single_query(const void* q, const void* k_pages, const vo
 // every token read all keys before it).
 //
 // FRESH (decode steps whose tokens are their own rows): the kernel takes the projection's output qkv [T, H + 2 KV, D] and does what
-// qk_norm_rope_store does: every workgroup norms and rotates its group's queries in registers (coordinate i's partner i + D/2 lies in
-// the same lane), and the one whose partition holds the token's own position makes the key and value, stores them and takes them
-// from registers where its pages' loads would have found them.  Same arithmetic; the squares are summed in another order.  All that the
-// new key and the queries are made of is asked for before the first keys and values (behind them it waited for those).  In a captured step of 4
-// requests of 500 to 700 tokens, 16 heads of 128 on 8 kv heads: 4.9 us for the kernel before this one and 9.6 for this, 12.1 now.
+// qk_norm_rope_store does: every workgroup norms and rotates its group's queries, and the one whose partition holds the token's own position
+// makes the key and value, stores them and takes them from LDS where its pages' loads would have found them.  A head is one wave's work
+// (a lane has coordinates i and i + D/2), the waves take the group's heads, the key and the value in turn.  Same
+// arithmetic; the squares are summed in another order.  All that they are made of is asked for before the first keys and values (behind them
+// it waited for those).  In a captured step of 4 requests of 500 to 700 tokens, 16 heads of 128 on 8 kv heads: 4.9 us for the kernel before
+// this one and 9.6 for this, as one 11.8 with every wave norming all queries as operands (284 registers), now 10.6 (222).
 struct FreshF32 {
   const float* qkv;
   const float* qw;   // gains of the per-head norms, D values each
@@ -1579,25 +1580,6 @@ struct FreshF32 {
   float eps;
   int store;         // 0: queries only, the pages already hold the token's key and value
 };
-
-// One head's values as attn_f32 has them, normed and rotated: piece i holds coordinates (i / 2) 32 + 8 lg + (i % 2) 4 .. + 3.
-template <int DT>
-__device__ __forceinline__ void norm_rotate_f32(f32x4_t (&v)[DT], const f32x4_t (&gain)[DT], const float4 (&turn)[DT], float eps) {
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < DT; ++i) ss += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
-  const float inv = 1.0f / sqrtf(quad_rows_sum(ss) / (float)(16 * DT) + eps);
-#pragma unroll
-  for (int i = 0; i < DT / 2; ++i)
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const float a = v[i][x] * inv * gain[i][x], b = v[i + DT / 2][x] * inv * gain[i + DT / 2][x];
-      const float4 t = turn[2 * i + (x >> 1)];  // two coordinates' cosine and sine
-      const float c = x & 1 ? t.z : t.x, s = x & 1 ? t.w : t.y;
-      v[i][x] = a * c - b * s;
-      v[i + DT / 2][x] = b * c + a * s;
-    }
-}
 
 // PAGE: tokens of a page where the compiler knows them (three divisions a step by another number are some 600 cycles), or 0.
 template <int DT, bool FRESH, int PAGE>
@@ -1650,13 +1632,15 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   const int steps = (k1 - k0 + 15) >> 4;
   const int* table = block_tables + (size_t)row * table_width;
 
+  constexpr int HALF = D / 2, TURNS = FRESH ? 5 : 1;  // 16 heads, a key and a value over four waves
+  __shared__ __align__(16) float fresh_kv[2][FRESH ? D : 1];  // the new token's key and value
+  [[maybe_unused]] float* const queries = smem + 128 + 4 * 16 * LD;  // FRESH: [G][LD]
   f32x4_t qf[DT], kf[DT], vf[DT], o[DT];
   auto piece_of = [&](int i) { return (i >> 1) * 32 + lg * 8 + (i & 1) * 4; };
-  const float* qrow = FRESH ? fresh.qkv + ((size_t)t0 * (H + 2 * KV) + (valid ? head : kvh * G)) * D
-                            : q + ((size_t)(t0 + (valid ? tok : 0)) * H + (valid ? head : kvh * G)) * D;
+  const float* qrow = FRESH ? queries + (valid ? lr : 0) * LD : q + ((size_t)(t0 + (valid ? tok : 0)) * H + (valid ? head : kvh * G)) * D;
 #pragma unroll
   for (int i = 0; i < DT; ++i) {
-    qf[i] = *reinterpret_cast<const f32x4_t*>(qrow + piece_of(i));
+    if constexpr (!FRESH) qf[i] = *reinterpret_cast<const f32x4_t*>(qrow + piece_of(i));
     o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
   auto page_of = [&](int step) {  // the 16 keys' place: page and offset, as an offset into one head's pages
@@ -1675,33 +1659,32 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   };
   float m = NEG_INF, l = 0.f;
   size_t base = page_of(wave), next = page_of(wave + 4);
-  // FRESH: the new token's key and value, in this partition at key `mine` of step `own_step`, which is one of this wave's, or nowhere.
-  // All that they and the queries are made of is asked for before the keys and values: loads come back in their order.
-  [[maybe_unused]] f32x4_t new_key[FRESH ? DT : 1], q_gain[FRESH ? DT : 1], k_gain[FRESH ? DT : 1];
-  [[maybe_unused]] float new_value[FRESH ? DT : 1];
-  [[maybe_unused]] float4 turn[FRESH ? DT : 1];
-  [[maybe_unused]] int own_step = -1;
+  // FRESH: the new token's key and value, in this partition at key `mine` of step `own_step`, or nowhere.
+  [[maybe_unused]] int own_step = -1, slot = -1, jobs = G;  // jobs: the group's heads, then the key and the value
   [[maybe_unused]] const int mine = (pos0 - k0) & 15;
+  [[maybe_unused]] float ha[TURNS], hb[TURNS], ga[2], gb[2];
+  [[maybe_unused]] float2 angle;
   if constexpr (FRESH) {
-    if (fresh.store && pos0 < k1 && ((pos0 - k0) >> 4) % 4 == wave) own_step = (pos0 - k0) >> 4;  // k0 <= pos0 where the partition is not empty
-    const float4* angles = reinterpret_cast<const float4*>(fresh.cs + (size_t)t0 * (D / 2));  // two coordinates each
-#pragma unroll
-    for (int i = 0; i < DT; ++i) q_gain[i] = *reinterpret_cast<const f32x4_t*>(fresh.qw + piece_of(i));
-#pragma unroll
-    for (int i = 0; i < DT / 2; ++i) {
-      turn[2 * i] = angles[piece_of(i) / 2];
-      turn[2 * i + 1] = angles[piece_of(i) / 2 + 1];
+    if (fresh.store && pos0 < k1) {  // k0 <= pos0 where the partition is not empty
+      own_step = (pos0 - k0) >> 4;
+      jobs = G + 2;
+      slot = fresh.slots[t0];
     }
-    if (own_step >= 0) {
-      const float* krow = fresh.qkv + ((size_t)t0 * (H + 2 * KV) + H + kvh) * D;
-      const float* vrow = krow + (size_t)KV * D;
+    const int i = min(lane, HALF - 1);
 #pragma unroll
-      for (int i = 0; i < DT; ++i) {
-        new_key[i] = *reinterpret_cast<const f32x4_t*>(krow + piece_of(i));
-        k_gain[i] = *reinterpret_cast<const f32x4_t*>(fresh.kw + piece_of(i));
-        new_value[i] = vrow[i * 16 + lr];
+    for (int n = 0; n < TURNS; ++n) {
+      const int job = wave + 4 * n;
+      if (job < jobs) {  // uniform over the wave
+        const float* src = fresh.qkv + ((size_t)t0 * (H + 2 * KV) + (job < G ? kvh * G + job : H + kvh + (job - G) * KV)) * D;
+        ha[n] = src[i];
+        hb[n] = src[i + HALF];
       }
     }
+    ga[0] = fresh.qw[i];
+    gb[0] = fresh.qw[i + HALF];
+    ga[1] = fresh.kw[i];
+    gb[1] = fresh.kw[i + HALF];
+    angle = fresh.cs[(size_t)t0 * HALF + i];
     __builtin_amdgcn_sched_barrier(0);
   }
   if (wave < steps) {
@@ -1710,28 +1693,39 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   }
   if constexpr (FRESH) {
     __builtin_amdgcn_sched_barrier(0);
-    norm_rotate_f32(qf, q_gain, turn, fresh.eps);
-    if (own_step >= 0) {
-      norm_rotate_f32(new_key, k_gain, turn, fresh.eps);
+    const size_t head_at = slot >= 0 ? ((size_t)(slot / bs) * KV + kvh) * bs * D : 0;
 #pragma unroll
-      for (int i = 0; i < DT; ++i) {
-        new_value[i] = finite_or_zero(new_value[i]);
-#pragma unroll
-        for (int x = 0; x < 4; ++x) new_key[i][x] = finite_or_zero(new_key[i][x]);
-      }
-      const int slot = fresh.slots[t0];
-      if (slot >= 0) {
-        const size_t head_at = ((size_t)(slot / bs) * KV + kvh) * bs * D;
-        if (lr == 0) {
-#pragma unroll
-          for (int i = 0; i < DT; ++i) *reinterpret_cast<f32x4_t*>(fresh.k_store + head_at + (size_t)(slot % bs) * D + piece_of(i)) = new_key[i];
+    for (int n = 0; n < TURNS; ++n) {
+      const int job = wave + 4 * n;
+      if (job > G && job < jobs) {  // the value, as it is; its page is stored transposed
+        const float ra = finite_or_zero(ha[n]), rb = finite_or_zero(hb[n]);
+        if (lane < HALF) {
+          fresh_kv[1][lane] = ra;
+          fresh_kv[1][lane + HALF] = rb;
+          float* vt = fresh.v_store + head_at + slot % bs;
+          if (slot >= 0) { vt[(size_t)lane * bs] = ra; vt[(size_t)(lane + HALF) * bs] = rb; }
         }
-        if (lg == 0) {
-#pragma unroll
-          for (int i = 0; i < DT; ++i) fresh.v_store[head_at + (size_t)(i * 16 + lr) * bs + slot % bs] = new_value[i];
+      } else if (job < jobs) {  // a query or the key
+        const bool is_key = job == G;
+        const float ss = wave_sum(lane < HALF ? ha[n] * ha[n] + hb[n] * hb[n] : 0.f), inv = 1.0f / sqrtf(ss / (float)D + fresh.eps);
+        const float a = ha[n] * inv * (is_key ? ga[1] : ga[0]), b = hb[n] * inv * (is_key ? gb[1] : gb[0]);
+        float ra = a * angle.x - b * angle.y, rb = b * angle.x + a * angle.y;
+        if (is_key) {
+          ra = finite_or_zero(ra);
+          rb = finite_or_zero(rb);
+        }
+        float* to = is_key ? fresh_kv[0] : queries + job * LD;
+        if (lane < HALF) {
+          to[lane] = ra;
+          to[lane + HALF] = rb;
+          float* dst = fresh.k_store + head_at + (size_t)(slot % bs) * D;
+          if (is_key && slot >= 0) { dst[lane] = ra; dst[lane + HALF] = rb; }
         }
       }
     }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < DT; ++i) qf[i] = *reinterpret_cast<const f32x4_t*>(qrow + piece_of(i));
   }
 #pragma unroll
   for (int i = 0; i < DT; ++i) qf[i] = qf[i] * scale;
@@ -1740,11 +1734,10 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
       if (step == own_step) {
 #pragma unroll
         for (int i = 0; i < DT; ++i) {
+          if (lr == mine) kf[i] = *reinterpret_cast<const f32x4_t*>(&fresh_kv[0][piece_of(i)]);
+          const float value = fresh_kv[1][i * 16 + lr];
 #pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            kf[i][x] = lr == mine ? new_key[i][x] : kf[i][x];
-            vf[i][x] = lg * 4 + x == mine ? new_value[i] : vf[i][x];
-          }
+          for (int x = 0; x < 4; ++x) vf[i][x] = lg * 4 + x == mine ? value : vf[i][x];
         }
       }
     }
@@ -1842,7 +1835,7 @@ static int launch_attn_f32(const FreshF32* fresh, const float* q, const float* k
   const int per = tiles ? 16 / (H / KV) : 1, subs = tiles ? (most + per - 1) / per : 1;
   if ((long)blocks_of * subs > 0x7fffffffL) return AS_BAD_SHAPE;
   const dim3 grid(blocks_of * subs, KV, P);
-  const size_t lds = (128 + 4 * 16 * (D + 4)) * sizeof(float);
+  const size_t lds = (128 + (4 * 16 + (fresh ? H / KV : 0)) * (D + 4)) * sizeof(float);
   const FreshF32 none = {};
 #define GO(DTV, FRESHV, PAGEV)                                                                                                           \
   attn_f32_kernel<DTV, FRESHV, PAGEV><<<grid, 256, lds, stream>>>(q, k_pages, v_pages, tiles, items, positions, tok_row, block_tables,    \

@@ -510,14 +510,14 @@ def attn_f32_fresh_supported(dtype, num_heads: int, num_kv_heads: int, head_dim:
 
 
 def attn_f32_fresh_preferred(rows: int, H: int, KV: int, D: int, max_context: int, window: int) -> bool:
-    """Whether a decode step of these sizes is faster through `attn_f32_fresh` than through the two kernels.  Heads of 128: while its
-    workgroups are one round of the compute units, for it takes 284 registers (32 of them accumulators), which leave room for one workgroup to
-    each where the other kernel has two.  Heads of 64 (152 registers; three workgroups, as without): always.
+    """Whether a decode step of these sizes goes through `attn_f32_fresh` or through the two kernels: heads of 64 always, heads of 128 while the
+    workgroups are one round of the compute units.  The line was drawn when the one kernel left room for one workgroup of heads of 128 on a compute
+    unit where the other left room for two; with a head's norm and rotation one wave's work both leave room for two, and it is the faster one on
+    either side.  Steps beyond the line keep the results of the two kernels, whose sums of squares are in another order.
     us of one / of two, 16 heads on 8 kv heads, by requests x tokens (heads of 128, then of 64):
-        4 x 200       32 x 200      64 x 200      4 x 600       8 x 600       16 x 600      4 x 2,000     8 x 2,000     32 x 2,000    8 x 6,000
-        14.3/14.6     19.1/20.2     34.7/30.1     15.9/16.4     24.1/22.2     33.5/30.1     22.2/23.8     36.2/34.5     103/102       79/78
-        10.1/11.3     12.1/13.6     16.9/19.3     12.1/13.4     15.0/16.5     18.6/20.1     15.7/17.6     21.2/23.6     55.5/54.8     43/46
-    (heads of 64, 105 sizes with 8 on 2 and 32 on 8 heads too: slower at six, by 1.4 per cent at most)."""
+        1 x 100       4 x 200       32 x 200      64 x 200      4 x 600       8 x 600       16 x 600      4 x 2,000     32 x 2,000    8 x 6,000
+        9.4/11.1      13.7/15.1     18.9/20.4     29.0/32.2     13.8/15.2     19.6/21.3     28.9/30.7     21.5/23.6     104/106       77/80
+        7.2/8.9       9.6/11.4      11.2/13.1     17.8/20.1     11.5/12.8     13.7/15.5     17.3/19.3     14.2/16.0     55/58         44/46"""
     return D <= 64 or rows * KV * _partitions(rows, H, KV, D, max_context, window, True, None, "meta")[1] <= compute_units()
 
 
