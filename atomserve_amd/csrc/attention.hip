@@ -1568,7 +1568,7 @@ extern "C" int as_attn_single_query(const void* q, const void* k_pages, const vo
 // (a lane has coordinates i and i + D/2), the waves take the group's heads, the key and the value in turn.  Same
 // arithmetic; the squares are summed in another order.  All that they are made of is asked for before the first keys and values (behind them
 // it waited for those).  In a captured step of 4 requests of 500 to 700 tokens, 16 heads of 128 on 8 kv heads: 4.9 us for the kernel before
-// this one and 9.6 for this, as one 11.8 with every wave norming all queries as operands (284 registers), now 10.6 (222).
+// this one and 9.6 for this, as one 11.8 with every wave norming all queries as operands (284 registers), now 10.7 (222).
 struct FreshF32 {
   const float* qkv;
   const float* qw;   // gains of the per-head norms, D values each
