@@ -757,25 +757,52 @@ struct PrefillSplit {
 };
 constexpr int PREFILL_MIN_PIECE_ROUNDS = 2;  // an item's last two rounds hold its own tokens: one piece
 
+// A step that has both, portions of prompts and single queries, in one launch (PAGE != 0): the single queries' workgroups come first, a kv
+// head of every context after the other, and share the compute units with the portions'.  The ones wait for memory most of
+// the time and the others for the matrix cores and the softmax, and the tail of neither leaves compute units idle.
+// One kernel's body, not a function that two kernels call: inlined, the compiler schedules portions alone otherwise (1,500 tokens of 16 heads
+// on 4 kv heads 33.1 and 34.1 us).
+struct Singles {
+  const int* items;
+  const int* positions;
+  const int* tok_row;
+  float* part_m;
+  float* part_l;
+  float* part_acc;
+  int count, part_size, P;
+};
+
 // With kept first tokens behind a window the rounds of 64 keys are first those from the sequence's start that hold kept
 // tokens, then those of the window (`first_key`); pieces cut this list.
-// What the workgroup `item` of `blocks` does; lds: a stage's slots are K0 K1 V0 V1.
-template <int DC>
-using PrefillStages = u32x4_t[PF_STAGES][4][64 * DC];  // [stage][K0 K1 V0 V1][slot]
-// BY_HEAD: the kv head changes fastest and a pass is walked backwards by eights.  Workgroups are dealt to the eight XCDs in
+// With single queries the kv head changes fastest and a pass is walked backwards by eights.  Workgroups are dealt to the eight XCDs in
 // turn, each with an L2 of its own, so that with eight kv heads an XCD brings one head's keys and values from memory (with four, two share
 // one).  Beside single queries that is what memory is short of (Qwen3-8B sizes, 8 of 500 to 8,192 keys beside 504 tokens 48.3 -> 44.6 us a
 // layer, 2 of 7,000 beside 500 32.9 -> 28.7, 32 of 100 to 2,048 beside 480 behind 7,001 with 64 heads 210 -> 195); portions alone
 // wait for the matrix cores, and several of one request lose (480 tokens behind 7,001 95 -> 97): not there.
-template <int DC, int QT, int SEE, bool BY_HEAD>  // D / 32; column tiles of 16 queries that a wave owns: 2, or 1 (see the launcher); SEE: see above
-__device__ __forceinline__ void prefill_item(
+template <int DC, int QT, int SEE, int PAGE>  // D / 32; column tiles of 16 queries that a wave owns: 2, or 1 (see the launcher); SEE: see above;
+                                              // PAGE: 0, or the tokens of a page of the single queries before the portions
+__global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
     const int* __restrict__ tiles, const int* __restrict__ block_tables, int table_width,
-    bf16* __restrict__ out, int H, int KV, int bs, float scale, const Sight& sight, int units_z, int pass, const PrefillSplit& split,
-    PrefillStages<DC>& lds, int item, int blocks) {
+    bf16* __restrict__ out, int H, int KV, int bs, float scale, Sight sight, int units_z, int pass, PrefillSplit split, Singles single) {
   constexpr int D = DC * 32, DT = DC * 2;
+  constexpr int PIECE = 64 * DC;  // 16-byte slots of a 16-key piece: 16 * D / 8
   typedef __attribute__((address_space(3))) void* lds_ptr_t;
   typedef const __attribute__((address_space(1))) void* global_ptr_t;
+  __shared__ __attribute__((aligned(16))) u32x4_t lds[PF_STAGES][4][PIECE];  // [stage][K0 K1 V0 V1][slot]
+  int item = blockIdx.x, blocks = gridDim.x;
+  if constexpr (PAGE != 0) {  // a single query of up to 16 heads needs 256 D + 1,536 of the 512 D bytes
+    const int singles = single.count * KV * single.P;
+    if (item < singles) {
+      decode_item<DC, 0, 0, PAGE>(q, k_pages, v_pages, single.items, single.positions, single.tok_row, block_tables, table_width, out,
+                                  single.part_m, single.part_l, single.part_acc, H, KV, bs, scale, sight, single.part_size, single.P, 1,
+                                  FreshQKV{}, reinterpret_cast<float*>(&lds[0][0][0]), item / KV % single.count, item % KV,
+                                  item / (KV * single.count));
+      return;
+    }
+    item -= singles;
+    blocks -= singles;
+  }
 
   const int G = H / KV;
   // Work items (tile, kv head, group of four waves) in the order of `tiles`, which the caller
@@ -785,24 +812,21 @@ __device__ __forceinline__ void prefill_item(
   // the next, so that causal prompts, whose items range from one step to hundreds, finish
   // together.
   const int per_tile = KV * units_z;
-  int tile, kvh, bz, piece = 0;  // piece: which of an item's workgroups this is
-  {
-    const int block = item / pass, first = block * pass, size = min(pass, blocks - first), off = item - first;
-    if constexpr (BY_HEAD) {
-      const int eights = size & ~7;
-      if ((block & 1) && off < eights) item = first + eights - 8 - (off & ~7) + (off & 7);
-      const int all = per_tile * split.pieces;
-      tile = item / all, kvh = item % KV, bz = item / KV % units_z, piece = item % all / per_tile;
-      item = (tile * KV + kvh) * units_z + bz;
-    } else {
-      if (block & 1) item = first + size - 1 - off;
-      if (split.pieces > 1) {
-        piece = item % split.pieces;
-        item /= split.pieces;
-      }
-      tile = item / per_tile, kvh = (item % per_tile) / units_z, bz = item % units_z;
+  const int block = item / pass, first = block * pass, size = min(pass, blocks - first);
+  int piece = 0;  // which of an item's workgroups this is
+  if constexpr (PAGE != 0) {
+    const int off = item - first, eights = size & ~7, all = per_tile * split.pieces;
+    if ((block & 1) && off < eights) item = first + eights - 8 - (off & ~7) + (off & 7);
+    piece = item % all / per_tile;
+    item = (item / all * KV + item % KV) * units_z + item / KV % units_z;
+  } else {
+    if (block & 1) item = first + size - 1 - (item - first);
+    if (split.pieces > 1) {
+      piece = item % split.pieces;
+      item /= split.pieces;
     }
   }
+  const int tile = item / per_tile, kvh = (item % per_tile) / units_z, bz = item % units_z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
@@ -1151,46 +1175,6 @@ __device__ __forceinline__ void prefill_item(
   }
 }
 
-template <int DC, int QT, int SEE>
-__global__ __launch_bounds__(256, 2) void attn_prefill_mfma_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
-    const int* __restrict__ tiles, const int* __restrict__ block_tables, int table_width,
-    bf16* __restrict__ out, int H, int KV, int bs, float scale, Sight sight, int units_z, int pass, PrefillSplit split) {
-  __shared__ __attribute__((aligned(16))) PrefillStages<DC> lds;
-  prefill_item<DC, QT, SEE, false>(q, k_pages, v_pages, tiles, block_tables, table_width, out, H, KV, bs, scale, sight, units_z, pass, split,
-                            lds, blockIdx.x, gridDim.x);
-}
-
-// A step that has both, portions of prompts and single queries, in one launch: the single queries' workgroups come first, a kv
-// head of every context after the other, and share the compute units with the portions'.  The ones wait for memory most of
-// the time and the others for the matrix cores and the softmax, and the tail of neither leaves compute units idle.
-struct Singles {
-  const int* items;
-  const int* positions;
-  const int* tok_row;
-  float* part_m;
-  float* part_l;
-  float* part_acc;
-  int count, part_size, P;
-};
-
-template <int DC, int QT, int PAGE>
-__global__ __launch_bounds__(256, 2) void attn_mixed_mfma_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ k_pages, const bf16* __restrict__ v_pages,
-    const int* __restrict__ tiles, const int* __restrict__ block_tables, int table_width,
-    bf16* __restrict__ out, int H, int KV, int bs, float scale, Sight sight, int units_z, int pass, PrefillSplit split, Singles single) {
-  __shared__ __attribute__((aligned(16))) PrefillStages<DC> lds;  // a single query of up to 16 heads needs 256 D + 1,536 of its 512 D bytes
-  const int b = blockIdx.x, singles = single.count * KV * single.P;
-  if (b < singles) {
-    decode_item<DC, 0, 0, PAGE>(q, k_pages, v_pages, single.items, single.positions, single.tok_row, block_tables, table_width, out,
-                                single.part_m, single.part_l, single.part_acc, H, KV, bs, scale, sight, single.part_size, single.P, 1,
-                                FreshQKV{}, reinterpret_cast<float*>(&lds[0][0][0]), b / KV % single.count, b % KV, b / (KV * single.count));
-  } else {
-    prefill_item<DC, QT, 0, true>(q, k_pages, v_pages, tiles, block_tables, table_width, out, H, KV, bs, scale, sight, units_z, pass, split,
-                            lds, b - singles, gridDim.x - singles);
-  }
-}
-
 // The pieces of every cut item, put together: one workgroup per item, its waves and lanes holding the queries and
 // coordinates they hold in the kernel above.  out = sum_j acc_j 2^(m_j - m) / sum_j l_j 2^(m_j - m) with m the
 // largest maximum; a piece that saw no key has m = -inf and l = 0.
@@ -1279,9 +1263,9 @@ extern "C" int as_attn_prefill_mfma(const void* q, const void* k_pages, const vo
   const PrefillSplit split{pieces, piece_rounds, cut, part_ml, part_acc};
   const int see = needed_sight(sight);
 #define LAUNCH2(DCV, QTV, SEEV)                                                                       \
-  attn_prefill_mfma_kernel<DCV, QTV, SEEV><<<(int)blocks, 256, 0, stream>>>(                          \
+  attn_prefill_mfma_kernel<DCV, QTV, SEEV, 0><<<(int)blocks, 256, 0, stream>>>(                       \
       (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, tiles, block_tables, table_width,   \
-      (bf16*)out, H, KV, bs, scale, sight, units_z, pass, split)
+      (bf16*)out, H, KV, bs, scale, sight, units_z, pass, split, Singles{})
 #define LAUNCH1(DCV, QTV)                                                                             \
   if (see == 2) LAUNCH2(DCV, QTV, 2);                                                                 \
   else if (see == 1) LAUNCH2(DCV, QTV, 1);                                                            \
@@ -1465,7 +1449,7 @@ extern "C" int as_attn_mixed_mfma(const void* q, const void* k_pages, const void
   const Singles single{items, positions, tok_row, part_m, part_l, part_acc, num_items, part_size, P};
 #define LAUNCH(DCV, QTV)                                                                                                 \
   do {                                                                                                                   \
-    attn_mixed_mfma_kernel<DCV, QTV, 16><<<(int)blocks, 256, 0, stream>>>(                                               \
+    attn_prefill_mfma_kernel<DCV, QTV, 0, 16><<<(int)blocks, 256, 0, stream>>>(                                          \
         (const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, tiles, block_tables, table_width, (bf16*)out, H, KV, \
         bs, scale, sight, units_z, compute_units(), split, single);                                                      \
     if (hipGetLastError() != hipSuccess) return AS_LAUNCH_FAILED;                                                        \
