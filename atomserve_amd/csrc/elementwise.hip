@@ -345,7 +345,15 @@ template <> struct Gain8<float> {
 
 // U: what counts the units; PAGE: tokens of a page where the compiler knows them, or 0 (a lane has two pieces to load and to store: a
 // 64-bit division and three by the page are as many instructions as all the rest).
-template <typename W, typename U, int PAGE>
+// EIGHTS: whose unit is whose neighbour.  Without, a token's heads lie side by side, and its angles are read by one wave: always for
+// qk_norm_rope_store, whose heads are whole waves in every model with eight kv heads of 128.  With, eight tokens of a head do: a wave has one
+// kind of head where a token's would mix queries, keys and values, but eight tokens' angles, and rows of single requests or of a portion that begins within a
+// page cost more.  Us, token by token / in eights: 32 + 8 + 8 heads of 128, 512 rows that begin within
+// a page behind 32 single ones 6.4 / 7.8, in a mixed step 7.5 / 9.0; 2,409 rows of several prompts 17.4 / 17.1; 16 + 4 + 4 heads, 512 rows 5.1 / 4.0
+// of one prompt and 5.5 / 6.0 behind single ones, 1,500 rows 8.7 / 7.0.
+// With the choices below made for each coordinate, sixteen branches, and the slots of a run read one after the other: one row 3.75 us, now
+// 3.2, 2,048 rows of 32 + 8 + 8 heads 16.7 and 15.0.
+template <typename W, typename U, int PAGE, bool EIGHTS>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
     const bf16* __restrict__ qkv, const W* __restrict__ qw, const W* __restrict__ kw,
     const float2* __restrict__ cs, const int* __restrict__ slots, bf16* __restrict__ q_out,
@@ -356,12 +364,17 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
   const U unit = ((U)blockIdx.x * 256 + threadIdx.x) >> (__ffs(lpu) - 1);
   const int l = threadIdx.x & (lpu - 1);
   if (unit >= units) return;  // whole groups leave: the shuffles below stay inside a group
-  // Eight tokens' units of a head lie side by side: with heads of 128 they are a wave's, and their values' lines are read once
-  // (with a token's heads side by side a line's eight readers were on as many XCDs: 2,409 tokens of 48 heads 20 us either way; 1,500 of 24 10.0 -> 8.2).
-  const U eight = unit / (8 * heads), rest = unit - eight * (8 * heads);
-  const size_t t = (size_t)eight * 8 + (rest & 7);
-  const int hs = (int)(rest >> 3);
-  if (t >= (size_t)T) return;
+  size_t t;
+  int hs;
+  if constexpr (EIGHTS) {
+    const U eight = unit / (8 * heads), rest = unit - eight * (8 * heads);
+    t = (size_t)eight * 8 + (rest & 7);
+    hs = (int)(rest >> 3);
+    if (t >= (size_t)T) return;
+  } else {
+    t = unit / heads;
+    hs = (int)(unit - (U)t * heads);
+  }
   const bool is_q = hs < H, is_k = !is_q && hs < H + KV;
   const int column = is_q ? q_off + hs * D : is_k ? k_off + (hs - H) * D : v_off + (hs - H - KV) * D;
   const bf16* src = qkv + t * ld + column;
@@ -379,9 +392,12 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
     const int nth = slot & 7;
     const long lead = (long)t - nth;
     bool run = (block_size & 7) == 0 && lead >= 0 && lead + 8 <= T;
-    if (run) {
+    if (run) {  // all eight asked for before one is looked at
+      int at[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) run = run && slots[lead + i] == slot - nth + i;
+      for (int i = 0; i < 8; ++i) at[i] = slots[lead + i];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) run &= at[i] == slot - nth + i;
     }
     if (run) {  // uniform over the lanes of this (token, head), and the same for all eight tokens
       typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -446,19 +462,33 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_bf16x8_kernel(
     for (int j = 0; j < 4; ++j) turn[j] = cs4[j];
   }
   bf16x8 oa, ob;
+  float a[8], b[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    float a = (float)a8[j] * inv, b = (float)b8[j] * inv;
-    if (w) { a *= ga[j]; b *= gb[j]; }
-    if (cs) {
+    a[j] = (float)a8[j] * inv;
+    b[j] = (float)b8[j] * inv;
+    if (w) { a[j] *= ga[j]; b[j] *= gb[j]; }
+  }
+  if (cs) {  // one choice for all coordinates
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
       const float c = (j & 1) ? turn[j >> 1].z : turn[j >> 1].x, sn = (j & 1) ? turn[j >> 1].w : turn[j >> 1].y;
-      oa[j] = (bf16)(a * c - b * sn);
-      ob[j] = (bf16)(b * c + a * sn);
-    } else {
-      oa[j] = (bf16)a;
-      ob[j] = (bf16)b;
+      oa[j] = (bf16)(a[j] * c - b[j] * sn);
+      ob[j] = (bf16)(b[j] * c + a[j] * sn);
     }
-    if (is_k || clean) { oa[j] = finite_or_zero((bf16)oa[j]); ob[j] = finite_or_zero((bf16)ob[j]); }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      oa[j] = (bf16)a[j];
+      ob[j] = (bf16)b[j];
+    }
+  }
+  if (is_k || clean) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      oa[j] = finite_or_zero((bf16)oa[j]);
+      ob[j] = finite_or_zero((bf16)ob[j]);
+    }
   }
   *reinterpret_cast<bf16x8*>(dst + 8 * l) = oa;
   *reinterpret_cast<bf16x8*>(dst + half + 8 * l) = ob;
@@ -474,7 +504,7 @@ extern "C" int as_qk_norm_rope_store(const void* qkv, int dtype, const void* qw,
   const int lpu = D >> 4;
   if (dtype == DT_BF16 && R == D && (D & 15) == 0 && lpu <= WAVE && (lpu & (lpu - 1)) == 0) {
     const int heads = store_kv ? H + 2 * KV : H;
-    const size_t units = ((size_t)num_tokens + 7) / 8 * 8 * heads;
+    const size_t units = (size_t)num_tokens * heads;
     const size_t blocks = (units * lpu + 255) / 256;
     if (blocks > 0x7fffffff) return AS_BAD_SHAPE;
     const bool known = block_size == 16 && blocks * 256 <= 0xffffffff;
@@ -482,7 +512,7 @@ extern "C" int as_qk_norm_rope_store(const void* qkv, int dtype, const void* qw,
   if (known) LAUNCH9(W, unsigned, 16);                                                               \
   else LAUNCH9(W, size_t, 0)
 #define LAUNCH9(W, U, PAGE)                                                                          \
-  qk_norm_rope_store_bf16x8_kernel<W, U, PAGE><<<(int)blocks, 256, 0, stream>>>(                     \
+  qk_norm_rope_store_bf16x8_kernel<W, U, PAGE, false><<<(int)blocks, 256, 0, stream>>>(              \
       (const bf16*)qkv, (const W*)qw, (const W*)kw, (const float2*)cs, slots, (bf16*)q_out,          \
       (bf16*)k_pages, (bf16*)v_pages, H, KV, D, eps, block_size, heads, (U)units, num_tokens, (H + 2 * KV) * D, 0, H * D, (H + KV) * D, false)
     if (w_dtype == DT_BF16) { LAUNCH8(bf16); }
@@ -748,22 +778,29 @@ extern "C" int as_head_norm_store(const void* proj, int dtype, int ld, int q_off
     return AS_BAD_SHAPE;
   if (H + 2 * KV > 65535) return AS_BAD_SHAPE;
   // bf16 heads of one width that is 16 times a power of two, turned whole or not at all, in rows and columns on 16 bytes: several heads to a
-  // wave in 16-byte pieces (1,500 tokens of 24 heads of 128 in rows of 7,168, 16.3 us with a wave of 64 threads a head: 10.2, with eight tokens of a head side by side 8.2)
+  // wave in 16-byte pieces from 2^19 values on (1,500 tokens of 16 + 4 + 4 heads of 128: 16.7 us with a wave of 64 threads a head, 7.9 in pieces and 6.7 in
+  // eights).  Fewer do not fill the pieces' waves, each of which has eight times the work: 1 / 32 / 128 tokens of a decode step 2.9 / 3.2 / 4.1 and 3.3 / 4.0 / 4.4,
+  // 128 / 256 of a prompt 4.0 / 5.0 and 3.7 / 3.9.  In eights (see the kernel) where a wave of a token's heads would mix kinds, from 512 tokens on: 256 / 512 /
+  // 2,048 of a prompt 3.9 / 4.8 / 8.7 and 3.2 / 3.8 / 7.7, behind single ones 4.3 / 5.3 / 9.0 and 4.8 / 5.8 / 9.5.
   const int lpu = dim >> 4;
   const bool store_kv = store && slots;
   const uintptr_t bases = (uintptr_t)proj | (uintptr_t)qw | (uintptr_t)kw | (uintptr_t)cs | (uintptr_t)q_out |
                           (store_kv ? (uintptr_t)k_pages | (uintptr_t)v_pages : 0);
   if (dtype == DT_BF16 && dim == vdim && dim == Dp && (dim & 15) == 0 && lpu <= WAVE && (lpu & (lpu - 1)) == 0 && (!cs || R == dim) &&
-      ((ld | q_off | k_off | v_off) & 7) == 0 && (bases & 15) == 0 && (!qw || w_dtype == DT_BF16 || w_dtype == DT_F32)) {
+      ((ld | q_off | k_off | v_off) & 7) == 0 && (bases & 15) == 0 && (!qw || w_dtype == DT_BF16 || w_dtype == DT_F32) &&
+      (size_t)num_tokens * (store_kv ? H + 2 * KV : H) * dim >= 1u << 19) {
     const int heads = store_kv ? H + 2 * KV : H;
-    const size_t units = ((size_t)num_tokens + 7) / 8 * 8 * heads, blocks = (units * lpu + 255) / 256;
+    const bool eights = store_kv && num_tokens >= 512 && ((H | KV) & (WAVE / lpu - 1));
+    const size_t units = (eights ? ((size_t)num_tokens + 7) / 8 * 8 : (size_t)num_tokens) * heads, blocks = (units * lpu + 255) / 256;
     if (blocks > 0x7fffffff) return AS_BAD_SHAPE;
     const bool known = bs == 16 && blocks * 256 <= 0xffffffff;
 #define LAUNCH8(W)                                                                                                       \
-  if (known) LAUNCH9(W, unsigned, 16);                                                                                   \
-  else LAUNCH9(W, size_t, 0)
-#define LAUNCH9(W, U, PAGE)                                                                                              \
-  qk_norm_rope_store_bf16x8_kernel<W, U, PAGE><<<(int)blocks, 256, 0, stream>>>(                                         \
+  if (known && eights) LAUNCH9(W, unsigned, 16, true);                                                                   \
+  else if (known) LAUNCH9(W, unsigned, 16, false);                                                                       \
+  else if (eights) LAUNCH9(W, size_t, 0, true);                                                                          \
+  else LAUNCH9(W, size_t, 0, false)
+#define LAUNCH9(W, U, PAGE, EIGHTS)                                                                                      \
+  qk_norm_rope_store_bf16x8_kernel<W, U, PAGE, EIGHTS><<<(int)blocks, 256, 0, stream>>>(                                 \
       (const bf16*)proj, (const W*)qw, (const W*)kw, (const float2*)cs, slots, (bf16*)q_out, (bf16*)k_pages,             \
       (bf16*)v_pages, H, KV, dim, eps, bs, heads, (U)units, num_tokens, ld, q_off, k_off, v_off, true)
     if (qw && w_dtype == DT_F32) { LAUNCH8(float); }

@@ -1344,11 +1344,40 @@ def test_portions_and_single_queries_in_one_launch(ops, monkeypatch, H, KV, D, w
         assert torch.allclose(out.float(), two.float(), atol=2e-2, rtol=2e-2), plan
 
 
+@pytest.mark.parametrize("kind,pieces,tiles", [(2, 1, 61), (1, 1, 50), (2, 2, 37)])
+def test_a_last_pass_of_portions_that_is_no_multiple_of_eight(ops, monkeypatch, kind, pieces, tiles):
+    """Three kv heads and so many tiles that the workgroups of the second pass, which is walked backwards by eights, leave a remainder:
+    every tile is attended once, with the bits that the portions alone get from the same cut."""
+    H, KV, D, per, start = 9, 3, 64, 40, 100
+    units, workgroups = ops.compute_units(), tiles * KV * (-(-(64 // (16 * kind)) * (H // KV) // 4)) * pieces
+    assert workgroups // units == 1 and workgroups % units % 8
+    T = 2 + tiles * per  # two single queries, then a portion behind 100 tokens
+    torch.manual_seed(tiles)
+    _, k_pages, v_pages, tables, _ = paged_case(BF16, H, KV, D, 16, [31, 700, start + tiles * per], seed=6, k_scale=1.0)
+    q = torch.randn(T, H, D, device=DEV).to(BF16)
+    positions, tok_row = i32([30, 699, *range(start, start + tiles * per)]), i32([0, 1] + [2] * (T - 2))
+    items = [[2 + i * per, per, 2, start + i * per] for i in reversed(range(tiles))]
+    most, keys = start + tiles * per, sum(t[3] + t[1] for t in items)
+    rounds = -(-most // 64)
+    monkeypatch.setattr(ops, "PREFILL_PIECES", pieces)
+    two = torch.full((T, H, D), float("nan"), device=DEV).to(BF16)
+    ops.attn_single_query(q, k_pages, v_pages, i32([1, 0]), positions, tok_row, tables, two, D**-0.5, 0, 700, part_size=704)
+    ops.attn_prefill(q, k_pages, v_pages, i32(items), tables, two, D**-0.5, 0, most, query_tiles=kind, tile_keys=keys)
+    monkeypatch.setattr(ops, "_mixed_plan", lambda *a: (kind, pieces, -(-rounds // pieces) if pieces > 1 else 0, 704))
+    out = torch.full((T, H, D), float("nan"), device=DEV).to(BF16)
+    ops.attn_mixed(q, k_pages, v_pages, i32([1, 0]), i32(items), positions, tok_row, tables, out, D**-0.5, 0, most, 700, keys)
+    assert out.isfinite().all() and torch.equal(out, two)
+
+
 @pytest.mark.parametrize("T,H,KV,D,bs,gain,turned", [(1, 3, 1, 16, 16, None, False), (7, 4, 2, 64, 16, BF16, True), (33, 6, 2, 128, 16, F32, False), (40, 2, 2, 128, 32, BF16, False),
-                                                      (9, 1, 1, 256, 16, None, True), (8, 2, 1, 1024, 16, F32, True)])
+                                                      (9, 1, 1, 256, 16, None, True), (8, 2, 1, 1024, 16, F32, True),
+                                                      (128, 16, 8, 128, 16, BF16, True), (129, 16, 8, 128, 48, F32, False), (6600, 3, 1, 16, 16, None, True), (130, 2, 1, 1024, 16, F32, True),
+                                                      (511, 6, 2, 128, 16, BF16, True), (512, 6, 2, 128, 16, F32, False), (519, 6, 2, 128, 32, None, True), (1101, 4, 2, 64, 16, BF16, True),
+                                                      (700, 3, 2, 128, 16, F32, True)])  # fmt: skip
 def test_head_norm_store_in_wide_pieces(ops, T, H, KV, D, bs, gain, turned):
-    """Heads whose rows and columns start on 16 bytes, several to a wave, against one that starts one column further, a wave a head: the
-    same within a rounding of bf16 (the squares are summed in another order); numbers that are not finite are zeros in both."""
+    """Heads whose rows and columns start on 16 bytes, from 2^19 values on several to a wave (a token's side by side, or, from 512 tokens on
+    where a wave would mix their kinds, eight tokens of one), against one that starts one column further, a wave a head: the same
+    within a rounding of bf16 (the squares are summed in another order); numbers that are not finite are zeros in both."""
     torch.manual_seed(D + T)
     width = (H + 2 * KV) * D
     wide = torch.randn(T, width + 16, device=DEV).to(BF16)
@@ -1358,7 +1387,7 @@ def test_head_norm_store_in_wide_pieces(ops, T, H, KV, D, bs, gain, turned):
     gains = [None, None] if gain is None else [(1 + 0.1 * torch.randn(D, device=DEV)).to(gain) for _ in range(2)]
     cs = torch.randn(T, D // 2, 2, device=DEV) if turned else None
     pages = -(-T // bs) + 2
-    slots = torch.arange(T) + bs + (3 if T == 9 else 0)  # runs of eight, and (9 tokens) runs that start within one
+    slots = torch.arange(T) + bs + (3 if T == 9 or (T > 100 and T % 2) else 0)  # runs of eight, and (9 tokens, odd ones of many) runs that start within one
     slots[T // 3] = -1 if T > 8 else slots[T // 3]
     for store in (True, False):
         got = []
