@@ -716,19 +716,24 @@ def _mixed_plan(num_tiles: int, H: int, KV: int, D: int, tile_context: int, tile
     rounds, mean_rounds = _prefill_rounds(num_tiles, tile_context, window, tile_keys)
     span = _seen_keys(single_context, window, 0, True)
     places, whole, groups = 2 * units, _up32(span), singles * KV
-
-    def cost(kind, pieces, part):
-        round_time = 2.2 if kind == 2 else 1.4
-        workgroups = num_tiles * KV * _prefill_units(kind, H // KV)
-        piece, parts = -(-rounds // pieces) * round_time, -(-span // part)
-        work = workgroups * mean_rounds * round_time + groups * (4.0 * parts + 0.025 * 0.6 * span)
-        total = max(piece, 4.0 + 0.018 * min(part, span), work / places + 0.35 * piece)
-        if pieces > 1:
-            total += 10.0 + 64 * num_tiles * H * pieces * D * 8 / 5e6
-        return total + (MERGE_LAUNCH + 0.6 * parts if parts > 1 else 0.0)
-
-    kind, pieces, part = min(((k, c, p) for k in (1, 2) for c in MIXED_PIECE_CHOICES if c == 1 or rounds // c >= PREFILL_MIN_PIECE_ROUNDS
-                              for p in (whole, *(n for n in MFMA_PARTITIONS if n < whole))), key=lambda a: cost(*a))  # fmt: skip
+    # What depends on the singles' cut alone, and on the portions' alone, is worked out once: a step's lengths are new ones, so that a plan is made in each.
+    ways = []
+    for part in (whole, *[n for n in MFMA_PARTITIONS if n < whole]):
+        parts = -(-span // part)
+        ways.append((part, groups * (4.0 * parts + 0.025 * 0.6 * span), 4.0 + 0.018 * min(part, span), MERGE_LAUNCH + 0.6 * parts if parts > 1 else 0.0))
+    best = None
+    for kind, round_time in ((1, 1.4), (2, 2.2)):
+        work = num_tiles * KV * _prefill_units(kind, H // KV) * mean_rounds * round_time
+        for pieces in MIXED_PIECE_CHOICES:
+            if pieces > 1 and rounds // pieces < PREFILL_MIN_PIECE_ROUNDS:
+                continue
+            piece = -(-rounds // pieces) * round_time
+            merge = 10.0 + 64 * num_tiles * H * pieces * D * 8 / 5e6 if pieces > 1 else 0.0
+            for part, single_work, single, single_merge in ways:
+                cost = max(piece, single, (work + single_work) / places + 0.35 * piece) + merge + single_merge
+                if best is None or cost < best[0]:
+                    best = (cost, kind, pieces, part)
+    _, kind, pieces, part = best
     return kind, pieces, -(-rounds // pieces) if pieces > 1 else 0, part
 
 

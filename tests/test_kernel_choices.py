@@ -290,6 +290,21 @@ def test_plans_of_steps_with_portions_and_single_queries(monkeypatch):
         ops._mixed_plan.cache_clear()
 
 
+@pytest.mark.parametrize("behind,context,H", [(7001, 2049, 32), (12000, 8192, 64), (0, 300, 16)])
+def test_a_plan_for_new_lengths_costs_little_on_the_host(behind, context, H):
+    """The lengths of a running server's step are new ones, so a plan is made in each before its first attention is launched: no more than 120
+    Python calls for all ways to cut the step (346 and 57 to 140 us with a cost worked out from the start for each way)."""
+    import sys
+
+    calls = []
+    sys.setprofile(lambda frame, event, arg: calls.append(event) if event in ("call", "c_call") else None)
+    try:
+        ops._mixed_plan.__wrapped__(8, H, 8, 128, behind + 480, 8 * (behind + 250), 32, context, 0, 256)
+    finally:
+        sys.setprofile(None)
+    assert len(calls) <= 120
+
+
 @pytest.mark.parametrize("dtype,D,page,sight,one", [(torch.bfloat16, 128, 16, {}, True), (torch.bfloat16, 64, 16, {}, True), (torch.bfloat16, 96, 16, {}, False),
                                                     (torch.bfloat16, 128, 32, {}, False), (torch.bfloat16, 128, 16, {"softcap": 5.0}, False)])  # fmt: skip
 def test_the_route_of_a_step_with_portions_and_single_queries(monkeypatch, dtype, D, page, sight, one):
