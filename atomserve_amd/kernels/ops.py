@@ -698,39 +698,51 @@ def attn_mixed_supported(dtype, H: int, KV: int, D: int, block_size: int) -> boo
     return dtype == BF16 and D in (64, 128) and block_size == 16 and H % KV == 0 and H // KV <= 16
 
 
-# Both kinds of work in one launch, single queries first.  How the portions' items and the singles' contexts are cut is chosen together: the
-# places (two workgroups to a compute unit) are busy for all the work divided by them and for a third of a piece at the end,
-# no less than for the longest piece or partition, and merges cost 10 us and 5 TB/s for what pieces leave, 4 us and 0.6 a
-# partition for what singles leave.  A single costs 4 us and 25 ns a key (contexts: three fifths of the longest on average), alone at the end 18 ns.
-# Pieces of 3 and 6 leave half a round of places idle.  One layer, us, two launches / this (best of all forms): Qwen3-8B sizes, 32 of 100 to
-# 2,048 keys beside 480 tokens behind 7,001 143 / 124 (122), 8 of 2,048 beside 504 33.5 / 27.9 (27.6), 8 of 500 to 8,192 beside 504 60 / 43
-# (42), 96 of 200 to 600 beside 2,000 96 / 92 (87), 20 of 1,000 to 3,000 beside four of 120 behind 6,000 159 / 122 (116); 40 heads, 128 of 32 to
-# 400 beside 384 behind 2,000 83 / 77 (65); 16 heads, 4 of 300 to 900 beside 37 14.2 / 11.1 (11.1).
-MIXED_PIECE_CHOICES = (1, 2, 4, 8)
-
-
+# Both kinds of work in one launch, single queries first.  How the portions' items and the singles' contexts are cut is chosen together, by a cost in
+# microseconds fitted to 22,000 times of 614 steps (1 to 128 single queries of up to 8,000 keys beside portions of 9 to 4,000 tokens behind up to
+# 14,000; 16 to 64 heads of 128 on 8 kv heads, 1, 2 and 4 kv heads, heads of 64; 256 compute units): a round of 64 keys is 1.4 us of a workgroup
+# of the portions' first kind and 2.05 of the second, with heads of 64 a tenth more; a single query's partition 5 us and 12 ns a key (contexts:
+# three fifths of the longest on average).  Workgroups that all have a place (two to a compute unit, 3.2 with heads of 64) last as long as the longest
+# of them.  More of them last for all the work divided by the places and for a quarter of a piece at the end, and halfway from there to whole
+# turns as far as the items are equally long.  Merges cost 6 us and 2 TB/s for what pieces leave, 4.1 us, 0.3 a partition and 1.5 TB/s for what singles
+# leave.  What it picks takes 1.7 per cent more than the best form on average and 24 at worst, on 160 other steps 1.9 and never more than two
+# launches; two steps of the 614 take 2 to 4 per cent more.  (Without places and turns, pieces by 10 us and 5 TB/s: 4.2 per cent, 40 at worst, and 31
+# steps, of long portions beside few or short contexts, took 2 to 27 per cent more than two launches; one of 1,274 tokens behind 4,530 beside one query, 40 heads,
+# two launches 201, then 237, now 193.)
+# One layer, us, two launches / this (best of all forms): Qwen3-8B sizes, 32 of 100 to 2,048 keys beside 480 tokens behind 7,001 145 / 126 (122), 8 of 2,048
+# beside 504 34 / 27.8 (27.8), 8 of 500 to 8,192 beside 504 60 / 42 (40), 96 of 200 to 600 beside 2,000 100 / 95 (91), 20 of 1,000 to 3,000 beside four of 120 behind
+# 6,000 163 / 126 (117); 40 heads, 128 of 32 to 400 beside 384 behind 2,000 74 / 76 (67); 16 heads, 4 of 300 to 900 beside 37 15.0 / 12.0 (11.1).
 @functools.lru_cache(maxsize=1024)
 def _mixed_plan(num_tiles: int, H: int, KV: int, D: int, tile_context: int, tile_keys: int, singles: int, single_context: int,
                 window: int, units: int) -> tuple:  # fmt: skip
     """(query tiles of a wave, pieces, rounds of a piece, keys of a single query's partition) for a step of both kinds."""
     rounds, mean_rounds = _prefill_rounds(num_tiles, tile_context, window, tile_keys)
     span = _seen_keys(single_context, window, 0, True)
-    places, whole, groups = 2 * units, _up32(span), singles * KV
+    places, whole, groups = (2.0 if D > 64 else 3.2) * units, _up32(span), singles * KV
     # What depends on the singles' cut alone, and on the portions' alone, is worked out once: a step's lengths are new ones, so that a plan is made in each.
     ways = []
     for part in (whole, *[n for n in MFMA_PARTITIONS if n < whole]):
         parts = -(-span // part)
-        ways.append((part, groups * (4.0 * parts + 0.025 * 0.6 * span), 4.0 + 0.018 * min(part, span), MERGE_LAUNCH + 0.6 * parts if parts > 1 else 0.0))
+        merge = MERGE_LAUNCH + 0.3 * parts + singles * H * parts * D * 8 / 1.5e6 if parts > 1 else 0.0
+        ways.append((part, groups * parts, groups * (5.0 * parts + 0.012 * 0.6 * span), 2.75 + 0.0125 * min(part, span), merge))
+    turning = 0.5 * (1.0 - min(1.0, max(0.0, 2.0 * (1.0 - mean_rounds / rounds))))  # 0: items of every length
     best = None
-    for kind, round_time in ((1, 1.4), (2, 2.2)):
-        work = num_tiles * KV * _prefill_units(kind, H // KV) * mean_rounds * round_time
-        for pieces in MIXED_PIECE_CHOICES:
+    for kind, round_time in ((1, 1.4), (2, 2.05)) if D > 64 else ((1, 1.54), (2, 2.255)):
+        workgroups = num_tiles * KV * _prefill_units(kind, H // KV)
+        work = workgroups * mean_rounds * round_time
+        for pieces in PREFILL_PIECE_CHOICES:
             if pieces > 1 and rounds // pieces < PREFILL_MIN_PIECE_ROUNDS:
                 continue
             piece = -(-rounds // pieces) * round_time
-            merge = 10.0 + 64 * num_tiles * H * pieces * D * 8 / 5e6 if pieces > 1 else 0.0
-            for part, single_work, single, single_merge in ways:
-                cost = max(piece, single, (work + single_work) / places + 0.35 * piece) + merge + single_merge
+            turns = -(-workgroups * pieces // places) * piece
+            merge = 6.0 + 64 * num_tiles * H * pieces * D * 8 / 2e6 if pieces > 1 else 0.0
+            for part, single_groups, single_work, single, single_merge in ways:
+                cost = piece if piece > single else single
+                if workgroups * pieces + single_groups > places:
+                    evenly = (work + single_work) / places + 0.25 * piece
+                    busy = evenly + turning * (turns - evenly)
+                    cost = busy if busy > cost else cost
+                cost += merge + single_merge
                 if best is None or cost < best[0]:
                     best = (cost, kind, pieces, part)
     _, kind, pieces, part = best

@@ -290,6 +290,21 @@ def test_plans_of_steps_with_portions_and_single_queries(monkeypatch):
         ops._mixed_plan.cache_clear()
 
 
+@pytest.mark.parametrize("tiles,H,KV,D,most,keys,singles,context,forms", [
+    (10, 16, 8, 128, 5446, 51841, 1, 224, {(1, 3), (1, 6), (2, 3), (2, 6)}), (48, 16, 4, 128, 6207, 226073, 1, 83, {(2, 1), (2, 3)}),
+    (5, 32, 8, 128, 6044, 29716, 7, 59, {(1, 3)}), (51, 32, 8, 64, 3253, 84853, 93, 106, {(1, 1)}), (19, 6, 3, 64, 4043, 66629, 1, 38, {(1, 4), (1, 6)}),
+    (20, 40, 8, 128, 5804, 20 * 5200, 1, 635, {(2, 1)})])  # fmt: skip
+def test_long_portions_beside_few_or_short_contexts_are_not_slower_than_alone(monkeypatch, tiles, H, KV, D, most, keys, singles, context, forms):
+    """Steps that were 14 to 32 per cent slower in one launch than in two where they were cut into eights or halves, or (the last) where portions that
+    all have a place were cut at all; forms: (query tiles, pieces) that took no more than two launches by a hundredth."""
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    ops._mixed_plan.cache_clear()
+    try:
+        assert ops._mixed_plan(tiles, H, KV, D, most, keys, singles, context, 0, 256)[:2] in forms
+    finally:
+        ops._mixed_plan.cache_clear()
+
+
 @pytest.mark.parametrize("behind,context,H", [(7001, 2049, 32), (12000, 8192, 64), (0, 300, 16)])
 def test_a_plan_for_new_lengths_costs_little_on_the_host(behind, context, H):
     """The lengths of a running server's step are new ones, so a plan is made in each before its first attention is launched: no more than 120
