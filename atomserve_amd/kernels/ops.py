@@ -714,8 +714,9 @@ def attn_mixed_supported(dtype, H: int, KV: int, D: int, block_size: int) -> boo
 # 6,000 163 / 126 (117); 40 heads, 128 of 32 to 400 beside 384 behind 2,000 74 / 76 (67); 16 heads, 4 of 300 to 900 beside 37 15.0 / 12.0 (11.1).
 @functools.lru_cache(maxsize=1024)
 def _mixed_plan(num_tiles: int, H: int, KV: int, D: int, tile_context: int, tile_keys: int, singles: int, single_context: int,
-                window: int, units: int) -> tuple:  # fmt: skip
-    """(query tiles of a wave, pieces, rounds of a piece, keys of a single query's partition) for a step of both kinds."""
+                window: int, units: int, query_tiles=None, forced_pieces=None) -> tuple:  # fmt: skip
+    """(query tiles of a wave, pieces, rounds of a piece, keys of a single query's partition) for a step of both kinds; query_tiles,
+    forced_pieces: numbers to force, as PREFILL_QUERY_TILES and PREFILL_PIECES."""
     rounds, mean_rounds = _prefill_rounds(num_tiles, tile_context, window, tile_keys)
     span = _seen_keys(single_context, window, 0, True)
     places, whole, groups = (2.0 if D > 64 else 3.2) * units, _up32(span), singles * KV
@@ -726,13 +727,18 @@ def _mixed_plan(num_tiles: int, H: int, KV: int, D: int, tile_context: int, tile
         merge = MERGE_LAUNCH + 0.3 * parts + singles * H * parts * D * 8 / 1.5e6 if parts > 1 else 0.0
         ways.append((part, groups * parts, groups * (5.0 * parts + 0.012 * 0.6 * span), 2.75 + 0.0125 * min(part, span), merge))
     turning = 0.5 * (1.0 - min(1.0, max(0.0, 2.0 * (1.0 - mean_rounds / rounds))))  # 0: items of every length
+    kinds = ((1, 1.4), (2, 2.05)) if D > 64 else ((1, 1.54), (2, 2.255))
+    if query_tiles is not None:
+        kinds = (kinds[int(query_tiles) - 1],)
+    if forced_pieces is not None:
+        cuts = (max(1, min(int(forced_pieces), rounds // 2)),)
+    else:
+        cuts = [c for c in PREFILL_PIECE_CHOICES if c == 1 or rounds // c >= PREFILL_MIN_PIECE_ROUNDS]
     best = None
-    for kind, round_time in ((1, 1.4), (2, 2.05)) if D > 64 else ((1, 1.54), (2, 2.255)):
+    for kind, round_time in kinds:
         workgroups = num_tiles * KV * _prefill_units(kind, H // KV)
         work = workgroups * mean_rounds * round_time
-        for pieces in PREFILL_PIECE_CHOICES:
-            if pieces > 1 and rounds // pieces < PREFILL_MIN_PIECE_ROUNDS:
-                continue
+        for pieces in cuts:
             piece = -(-rounds // pieces) * round_time
             turns = -(-workgroups * pieces // places) * piece
             merge = 6.0 + 64 * num_tiles * H * pieces * D * 8 / 2e6 if pieces > 1 else 0.0
@@ -770,7 +776,8 @@ def attn_mixed(q, k_pages, v_pages, items, tiles, positions, tok_row, block_tabl
         raise KernelError(f"mixed attention: {N} single queries, {tile_count} tiles, heads {H}/{KV} of {D}, pages of {bs}")
     if max(max_tile, max_single) > block_tables.shape[1] * bs:
         raise KernelError("attention: block tables are shorter than the longest context")
-    kind, pieces, piece_rounds, part = _mixed_plan(tile_count, H, KV, D, max_tile, tile_keys, N, max_single, window, compute_units())
+    kind, pieces, piece_rounds, part = _mixed_plan(tile_count, H, KV, D, max_tile, tile_keys, N, max_single, window, compute_units(),
+                                                   PREFILL_QUERY_TILES, PREFILL_PIECES)  # fmt: skip
     part_size, P, part_m, part_l, part_acc = _partitions(N, H, KV, D, max_single, window, True, part, dev)
     cut = piece_ml = piece_acc = None
     if pieces > 1:

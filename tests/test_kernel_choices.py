@@ -290,6 +290,27 @@ def test_plans_of_steps_with_portions_and_single_queries(monkeypatch):
         ops._mixed_plan.cache_clear()
 
 
+@pytest.mark.parametrize("query_tiles,pieces,want", [(None, None, (2, 4, 30)), (1, None, (1, 2, 59)), (None, 5, (2, 5, 24)), (2, 1, (2, 1, 0)), (1, 99, (1, 58, 3))])
+def test_forced_cuts_of_portions_hold_beside_single_queries(monkeypatch, query_tiles, pieces, want):
+    """What forces a variant and a number of pieces for a step of portions alone forces them where single queries share the launch."""
+    made = []
+    monkeypatch.setattr(ops, "compute_units", lambda: 256)
+    monkeypatch.setattr(ops, "_check", lambda *args: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_partitions", lambda *args: (args[7], 1, None, None, None))
+    monkeypatch.setattr(ops, "call", lambda name, *args: made.append(args[18:21]))
+    monkeypatch.setattr(ops, "PREFILL_QUERY_TILES", query_tiles)
+    monkeypatch.setattr(ops, "PREFILL_PIECES", pieces)
+    ops._mixed_plan.cache_clear()
+    try:
+        q, pages = torch.empty(512, 32, 128, dtype=torch.bfloat16), torch.empty(1, 8, 16, 128, dtype=torch.bfloat16)
+        ops.attn_mixed(q, pages, pages.view(1, 8, 128, 16), torch.empty(32, dtype=torch.int32), torch.empty(8, 4, dtype=torch.int32), None, None,
+                       torch.empty(33, 468, dtype=torch.int32), q, 0.1, 0, 7481, 2049, 8 * 7257)  # fmt: skip
+    finally:
+        ops._mixed_plan.cache_clear()
+    assert made == [want]
+
+
 @pytest.mark.parametrize("tiles,H,KV,D,most,keys,singles,context,forms", [
     (10, 16, 8, 128, 5446, 51841, 1, 224, {(1, 3), (1, 6), (2, 3), (2, 6)}), (48, 16, 4, 128, 6207, 226073, 1, 83, {(2, 1), (2, 3)}),
     (5, 32, 8, 128, 6044, 29716, 7, 59, {(1, 3)}), (51, 32, 8, 64, 3253, 84853, 93, 106, {(1, 1)}), (19, 6, 3, 64, 4043, 66629, 1, 38, {(1, 4), (1, 6)}),
