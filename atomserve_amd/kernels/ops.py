@@ -509,21 +509,14 @@ def attn_f32_fresh_supported(dtype, num_heads: int, num_kv_heads: int, head_dim:
     return attn_f32_supported(dtype, num_heads, num_kv_heads, head_dim, block_size) and rotary_dim == head_dim and qk_norm
 
 
-def attn_f32_fresh_preferred(rows: int, H: int, KV: int, D: int, max_context: int, window: int) -> bool:
-    """Whether a decode step of these sizes goes through `attn_f32_fresh` or through the two kernels: heads of 64 always, heads of 128 while the
-    workgroups are one round of the compute units.  The line was drawn when the one kernel left room for one workgroup of heads of 128 on a compute
-    unit where the other left room for two; with a head's norm and rotation one wave's work both leave room for two, and it is the faster one on
-    either side.  Steps beyond the line keep the results of the two kernels, whose sums of squares are in another order.
-    us of one / of two, 16 heads on 8 kv heads, by requests x tokens (heads of 128, then of 64):
+def attn_f32_fresh(qkv, q_weight, k_weight, cos_sin, slots, eps, store_kv, k_pages, v_pages, positions, block_tables, out, num_heads,
+                   scale, window, max_context, part_size=None, order=None) -> None:  # fmt: skip
+    """`attn_decode_fresh` for 32-bit heads, gains, pages and results: what `qk_norm_rope_store` and then `attn_single_query` do, faster at every size
+    measured and as close to 64 bits.  us of this one / of the two, 16 heads on 8 kv heads, by requests x tokens (heads of 128, then of 64; 8, 32 and 40
+    heads on 8, 8 on 2 and 16 on 1, steps of several workgroups a compute unit: 1.5 to 16 per cent less in each of 65 sizes):
         1 x 100       4 x 200       32 x 200      64 x 200      4 x 600       8 x 600       16 x 600      4 x 2,000     32 x 2,000    8 x 6,000
         9.4/11.1      13.7/15.1     18.9/20.4     29.0/32.2     13.8/15.2     19.6/21.3     28.9/30.7     21.5/23.6     104/106       77/80
         7.2/8.9       9.6/11.4      11.2/13.1     17.8/20.1     11.5/12.8     13.7/15.5     17.3/19.3     14.2/16.0     55/58         44/46"""
-    return D <= 64 or rows * KV * _partitions(rows, H, KV, D, max_context, window, True, None, "meta")[1] <= compute_units()
-
-
-def attn_f32_fresh(qkv, q_weight, k_weight, cos_sin, slots, eps, store_kv, k_pages, v_pages, positions, block_tables, out, num_heads,
-                   scale, window, max_context, part_size=None, order=None) -> None:  # fmt: skip
-    """`attn_decode_fresh` for 32-bit heads, gains, pages and results: what `qk_norm_rope_store` and then `attn_single_query` do."""
     _check(qkv, "qkv", F32, (None, None, None))
     T, heads, D = qkv.shape
     H = num_heads

@@ -110,8 +110,7 @@ class Attention(Mixer):
         fresh = None  # a decode step: norm, rotation, the cache store and attention in one kernel
         if step.decode_only and ops.attn_decode_fresh_supported(*case):
             fresh = ops.attn_decode_fresh
-        elif (step.decode_only and ops.attn_f32_fresh_supported(*case) and ops.attn_f32_fresh_preferred(T, H, KV, D, step.max_context, s.window)
-              and not (self.q_norm_weight.data_ptr() | self.k_norm_weight.data_ptr()) & 15):  # fmt: skip
+        elif step.decode_only and ops.attn_f32_fresh_supported(*case) and not (self.q_norm_weight.data_ptr() | self.k_norm_weight.data_ptr()) & 15:
             fresh = ops.attn_f32_fresh
         if fresh is not None:
             out = torch.empty((T, H, D), dtype=env.dtype, device=device)

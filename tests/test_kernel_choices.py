@@ -530,16 +530,16 @@ def test_products_without_columns_or_outputs_are_not_the_large_tiles(monkeypatch
 
 
 @pytest.mark.parametrize("H,KV,D,rows,context,change,how", [
-    (16, 8, 128, 4, 600, None, "one"), (16, 8, 128, 32, 200, None, "one"), (16, 8, 128, 33, 200, None, "two"),  # 8 workgroups a row
-    (16, 8, 128, 8, 500, None, "one"), (16, 8, 128, 1, 2000, None, "one"), (16, 8, 128, 8, 2000, None, "two"),  # contexts in parts
+    (16, 8, 128, 4, 600, None, "one"), (16, 8, 128, 32, 200, None, "one"), (16, 8, 128, 33, 200, None, "one"),  # 8 workgroups a row
+    (16, 8, 128, 8, 500, None, "one"), (16, 8, 128, 1, 2000, None, "one"), (16, 8, 128, 8, 2000, None, "one"),  # contexts in parts
     (16, 8, 64, 33, 200, None, "one"), (8, 2, 64, 64, 6000, None, "one"), (16, 8, 128, 4, 600, "q gains elsewhere", "two"),
     (16, 8, 128, 4, 600, "k gains elsewhere", "two"), (16, 8, 128, 4, 600, "no norm", "two"), (16, 8, 128, 4, 600, "no rotation", "two"),
     (16, 8, 128, 4, 600, "half of a head turned", "two"), (16, 8, 96, 4, 600, None, "two"), (16, 8, 128, 4, 600, "a prompt", "two"),
     (16, 8, 128, 4, 600, "pages of 8", "two"), (16, 8, 128, 64, 8000, "bf16", "bf16"),
 ])  # fmt: skip
 def test_the_route_of_a_32_bit_decode_step(monkeypatch, H, KV, D, rows, context, change, how):
-    """Norm, rotation, store and attention in one kernel, for heads of 128 while its workgroups are one round of the compute units, for the heads,
-    norms, rotations and pages that it takes and gains that start on 16 bytes; else in two."""
+    """Norm, rotation, store and attention in one kernel at every number of rows and tokens, for the heads, norms, rotations and pages that it
+    takes and gains that start on 16 bytes; else in two."""
     from types import SimpleNamespace
 
     from atomserve_amd.parts.attention import Attention
