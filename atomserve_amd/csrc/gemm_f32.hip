@@ -411,7 +411,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(const float* __re
   constexpr int PIECES = (ROWS * 8 + THREADS - 1) / THREADS;  // of 4 columns a thread and step; where they do not divide, some are brought twice
   constexpr int AHEAD = MTW > 1 ? 1 : 2;  // steps whose floats wait in registers
   constexpr int PLANE = ROWS * 4;
-  constexpr int SPREAD = MTW == 1 ? (22 * PIECES + 6 * NTW - 1) / (6 * NTW) : MTW == 2 ? 6 : 4;  // vector instructions a matrix instruction
+  constexpr int SPREAD = MTW == 1 ? (22 * PIECES + 6 * NTW - 1) / (6 * NTW) : 4;  // vector instructions a matrix instruction
   static_assert(WM * WN == 8 && ROWS % 16 == 0 && (!IS_GATED || NTW == 2) && !(IS_GATED && SPLIT), "");
   extern __shared__ bf16x8 lds[];  // [2][3][PLANE]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
