@@ -43,6 +43,18 @@ def test_rows_are_flattened_with_slots_tables_and_tiles():
         pack([Row([1] * 80 + [-1], 0, [table, table], [])])
 
 
+def test_a_split_names_the_longest_context_of_its_portions_and_of_its_single_queries():
+    """Each by itself: a portion's last token need not be the step's longest context, nor the longest portion the furthest; none without such rows."""
+    pages = [list(range(40))] * 2
+    rows = [Row([1] * 70, 0, pages, []), Row([1] * 9, 64, pages, []), Row([1], 130, pages, [0]), Row([1, 1], 20, pages, [1])]
+    both = pack(rows).split(ATTENTION)
+    assert (both.max_tile_context, both.max_short_context) == (73, 131) and pack(rows).max_context == 131
+    fine = pack(rows, row_splits=[(0, 4)]).split((0, 4))  # every row in tiles
+    assert (fine.max_tile_context, fine.max_short_context) == (131, 0)
+    none = pack(rows[2:]).split(ATTENTION)
+    assert (none.max_tile_context, none.max_short_context, none.tile_keys) == (0, 131, 0)
+
+
 def test_a_repeated_decode_step_is_updated_in_place():
     """Same requests, one position further: `advance` leaves exactly what packing anew gives, also
     when a request has just received a new page; anything else is refused untouched."""
